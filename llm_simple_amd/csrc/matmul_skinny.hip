@@ -1,0 +1,117 @@
+// Projection of few rows (one generated token, a handful of tokens): out[m][n] = lhs[m][k] . W[n][k]^T + bias,
+// fp32 accumulation, one rounding, m <= 16.
+//
+// Bound by reading W once.  W is dealt out in equal shares of whole rows (at most 16) to one workgroup per
+// CU, two or more rounds of them for a wide n: a CU cannot have more than its 32 KiB of first-level cache
+// in flight (about 30 GB/s), so a matrix is only read at full speed if every CU has the same share of it --
+// with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it takes 3.8.
+// The eight waves of a workgroup deal k out among themselves, all loads of a wave are issued before its first
+// MFMA, and the partial sums meet in LDS.
+//
+// mfma_f32_16x16x32 takes 16 rows of 32 k; read that way every load instruction would touch half a
+// cache line of 16 rows.  With at most 8 lhs rows the operand rows are instead 8 rows of W at two
+// neighbouring k slices (KS = 2) and the operand columns the lhs rows at the same two slices: a load covers
+// whole 128-byte lines of 8 rows, of the result the two diagonal blocks are wanted.  3584 x 3584, one
+// row: 6.2 us from HBM (non-temporal loads) against 6.8 with KS = 1; KS = 4 is no better.  For 9..16
+// rows KS = 1, and ordinary loads, because the second half of a line is asked for by the next instruction.
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace llmhip {
+
+namespace {
+
+constexpr int kSkinnyWaves = 8;
+
+struct SkinnyParams {
+  const uint16_t *x;
+  const uint16_t *w;
+  const float *bias;
+  uint16_t *out;
+  int m, n, k;
+  int rows;  // W rows of a workgroup, at most 16
+};
+
+// KS k-slices per MFMA: operand row (column) index i stands for W (lhs) row i % (16/KS) at slice
+// i / (16/KS).  B units of 32*KS k per wave and pass.
+template <typename T, int KS, int B>
+__global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(SkinnyParams p) {
+  using E = Elem<T>;
+  constexpr int NW = kSkinnyWaves, R = 16 / KS, UK = 32 * KS;
+  __shared__ __attribute__((aligned(16))) float red[NW * KS * 256];  // [wave][group of R rows][lane] of f32x4
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int i = lane & 15, cg = lane >> 4, r = i % R;
+  const int n0 = blockIdx.x * p.rows;
+  const int rows = min(p.rows, p.n - n0);
+  const int koff = 32 * (i / R) + 8 * cg;
+  const uint16_t *wp[KS];
+#pragma unroll
+  for (int t = 0; t < KS; ++t) wp[t] = p.w + (size_t)(n0 + min(t * R + r, rows - 1)) * p.k + koff;
+  const bool xv = r < p.m;
+  const uint16_t *xp = p.x + (size_t)(xv ? r : 0) * p.k + koff;
+  f32x4_t acc[KS];
+#pragma unroll
+  for (int t = 0; t < KS; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int units = (p.k + UK - 1) / UK;
+  const u32x4_t zero = {0u, 0u, 0u, 0u};
+  for (int u0 = wave; u0 < units; u0 += NW * B) {
+    u32x4_t wf[B][KS], xf[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int kk = (u0 + b * NW) * UK;
+      const bool in = kk + koff < p.k;  // k is a multiple of 16, a fragment 8 long
+#pragma unroll
+      for (int t = 0; t < KS; ++t) {
+        wf[b][t] = zero;
+        if (in && t * R + r < rows) wf[b][t] = KS > 1 ? global_load_b128_nt(wp[t] + kk) : global_load_b128(wp[t] + kk);
+      }
+      xf[b] = zero;
+      if (in && xv) xf[b] = global_load_b128(xp + kk);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b)
+#pragma unroll
+      for (int t = 0; t < KS; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
+  }
+  f32x4_t *slots = reinterpret_cast<f32x4_t *>(red);
+#pragma unroll
+  for (int t = 0; t < KS; ++t) slots[(wave * KS + t) * 64 + lane] = acc[t];
+  __syncthreads();
+  // thread: feature n0 + f of lhs row `row`
+  const int f = tid & 15, row = tid >> 4;
+  if (f >= rows || row >= p.m) return;
+  float sum = 0.0f;
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const int ar = s * R + f % R, col = s * R + row;
+    const float *src = red + ((f / R) * 64 + (ar >> 2) * 16 + col) * 4 + (ar & 3);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sum += src[w * KS * 256];
+  }
+  if (p.bias) sum += p.bias[n0 + f];
+  p.out[(size_t)row * p.n + n0 + f] = E::round(sum);
+}
+
+}  // namespace
+
+hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, const float *bias, int m, int n,
+                                int k, int dt, hipStream_t stream) {
+  SkinnyParams p;
+  p.x = static_cast<const uint16_t *>(lhs);
+  p.w = static_cast<const uint16_t *>(weight);
+  p.bias = bias;
+  p.out = static_cast<uint16_t *>(out);
+  p.m = m;
+  p.n = n;
+  p.k = k;
+  const int cus = device_compute_units();
+  const int rounds = (n + 16 * cus - 1) / (16 * cus);
+  p.rows = (n + rounds * cus - 1) / (rounds * cus);
+  void (*kern)(SkinnyParams) =
+      m <= 8 ? (dt == kDtFloat16 ? matmul_skinny_kernel<_Float16, 2, 4> : matmul_skinny_kernel<__bf16, 2, 4>)
+             : (dt == kDtFloat16 ? matmul_skinny_kernel<_Float16, 1, 8> : matmul_skinny_kernel<__bf16, 1, 8>);
+  hipLaunchKernelGGL(kern, dim3((n + p.rows - 1) / p.rows), dim3(64 * kSkinnyWaves), 0, stream, p);
+  return hipGetLastError();
+}
+
+}  // namespace llmhip
