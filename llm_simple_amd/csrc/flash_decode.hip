@@ -21,21 +21,32 @@
 // their loads are non-temporal (7.1 TB/s at 2 GiB where ordinary loads give 6.2),
 // and K and V of a step are fetched one after the other so that a CU has 32 KiB
 // in flight, not 64 (see the loop).  Each wave keeps its own running (max, sum,
-// O); the four
-// waves are merged through LDS at the end and the workgroup writes either the
-// final rows (one split) or an fp32 partial (max, sum, unnormalised O) that
-// flash_decode_combine_kernel folds with the log-sum-exp rule.  (Folding inside
-// the last-arriving workgroup instead was measured and rejected: the device-scope
-// release/acquire fences it needs write back and invalidate the XCD's L2 and cost
-// more than the second launch -- 91 us against 33 us at batch 1, 32768 keys.  Without
-// fences, with the partials written through and read back at device scope (sc1 accesses)
-// and one relaxed device-scope atomic, it is correct but still slower -- 35.9 us against
-// 33.4 us, and 15.0 us against 10.6 us at 4096 keys: the chain store-acknowledge, atomic,
-// two dependent rounds of memory-latency loads in ONE workgroup is longer than a launch.
-// Eight-wave workgroups, half as many, merging pairs of splits through LDS: 4.5 TB/s
-// against 6.0 at the time -- a CU draws about 31-35 GB/s however many waves ask, so all of
-// them must stream.)
+// O); the
+// waves are merged through LDS at the end and the workgroup writes the final rows (one split) or an
+// fp32 partial (max, sum, unnormalised O).
+//
+// Up to 16 partials of a (sequence, kv head) are folded (log-sum-exp) by the workgroup that finds them all stored:
+// partials go past the XCD's L2 (sc1 stores), then a flag, then a look at the other flags -- no fence, no atomic.
+// That is three memory round trips, 2.2-2.4 us, against 3.1 us for flash_decode_combine_kernel, whose launch
+// also costs the host 2.4 us.  More partials make more rounds of loads in ONE workgroup (32: 11.2 against 8.8 us at
+// batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses write back
+// and invalidate the XCD's L2: 91 us against 33 at batch 1, 32768 keys.)
+//
+// A short cache is bound by the length of one workgroup's chain, not by bytes: at 32 keys, one sequence, the
+// kernel took 6.3 us, 2.5 us of them the launch.  A wave issues a vector instruction every 4-5 cycles, so the
+// chain is kept short: the query (and table) loads go out before the first keys and are waited for after
+// them, the new K row of a fused step is rotated in a spare query column, bf16 results are rounded by the conversion
+// instruction, K and V rows are read through buffer descriptors (the hardware bounds them, no clamps), integer
+// divisions are prepared by the host, the column maximum goes through permlane swaps, masks and the
+// rescaling of O run only where they change something, and the merge of the waves is free of bank conflicts (it cost
+// 1.4 us).  4.1 us now; 384 keys of 2 kv heads 9.7 -> 6.5 us, 512 keys of 32 kv heads 10.0 -> 7.1, 4096 keys of 8
+// 10.6 -> 8.8, 32768 keys of 8 28.9 -> 25.4 (fused step, back-to-back calls).
+//
+// (Eight-wave workgroups, half as many, merging pairs of splits through LDS: 4.5 TB/s against 6.0 at the time.)
 #include <atomic>
+#include <chrono>
+#include <random>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -44,7 +55,7 @@ namespace llmhip {
 
 constexpr int kDecThreads = 256;
 constexpr int kDecWaveKeys = 32;                  // keys per wave per step
-constexpr int kDecStepKeys = 4 * kDecWaveKeys;    // keys per workgroup per step
+constexpr int kDecStepKeys = 4 * kDecWaveKeys;    // keys per workgroup per step (half of it in short caches)
 constexpr int kDecCols = 16;                      // query rows per kv head (MFMA N)
 constexpr int kDecWaveLds = kDecWaveKeys * kRowBytes;  // 8 KiB of staging per wave, for K and for V
 constexpr int kDecLdsPad = 24 * 1024;             // with the 64 KiB of staging: more than half a CU's LDS
@@ -54,14 +65,18 @@ struct DecodeParams {
   const char *k;
   const char *v;
   char *out;
-  float *ws_o;   // [batch][Hkv][splits][16][128]
-  float *ws_ml;  // [batch][Hkv][splits][16][2]
+  float *ws_o;   // [batch][Hkv][splits][cols][128]
+  float *ws_ml;  // [batch][Hkv][splits][cols][2]; fold: the last column's place is the flag of the split
   int batch, m, n, offset;
   int64_t kv_seq_stride;
   int g, Hkv, H;
   int rows;  // m * g
   int num_splits;
+  int iters_each, iters_rest;  // blocks per split: iters_each, one more for the first iters_rest splits
+  FastDiv g_div;
   float scale_log2e;
+  int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
+  uint64_t fold;  // not 0: the workgroup of a (sequence, kv head) that finds this number in all flags folds
   // Fused decode step (FUSED kernels only): the token at row fused_pos = n - 1 is not in the cache yet.
   // q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
   // q and the new K row are rotated with table row freq_row (64 (cos, sin) pairs) as they are loaded,
@@ -75,43 +90,59 @@ struct DecodeParams {
 // RoPE of the four 16-byte fragments a lane holds of one head row: fragment kk = dims 8*cg + 32*kk .. +7.
 // Arithmetic of the rotary kernel, unfused products and sums (src/llama2_layer_cpu.cpp:835-856):
 // (a*c - b*s, a*s + b*c) rounded once; interleaved pairs (2f, 2f+1), neox pairs (f, f+64).
+// The lane's 16 (cos, sin) pairs are 8 pieces of 16 bytes of the table row.
+__device__ __forceinline__ void load_rotation(f32x4_t (&t)[8], const float *row, int cg, int is_neox) {
+  const float *at = row + (is_neox ? 16 * cg : 8 * cg);
+  const int far = is_neox ? 64 : 32, near = is_neox ? 4 : 2;  // floats between groups, pieces of a group
+#pragma unroll
+  for (int i = 0; i < 8; ++i) t[i] = *reinterpret_cast<const f32x4_t *>(at + far * (is_neox ? i >> 2 : i >> 1) + 4 * (i & (near - 1)));
+}
 template <typename T>
-__device__ __forceinline__ void rotate_frags(u32x4_t (&f)[4], const float *tab, int cg, int is_neox) {
+__device__ __forceinline__ void rotate_frags(u32x4_t (&f)[4], const f32x4_t (&t)[8], int is_neox) {
 #pragma clang fp contract(off)
   using E = Elem<T>;
-  auto get = [](const u32x4_t &w, int e) { return (uint16_t)((w[e >> 1] >> ((e & 1) * 16)) & 0xFFFFu); };
-  auto put = [](u32x4_t &w, int e, uint16_t v) {
-    w[e >> 1] = (w[e >> 1] & ~(0xFFFFu << ((e & 1) * 16))) | ((uint32_t)v << ((e & 1) * 16));
-  };
+  auto lo = [](uint32_t w) { return E::widen((uint16_t)(w & 0xffffu)); };
+  auto hi = [](uint32_t w) { return E::widen((uint16_t)(w >> 16)); };
   if (is_neox) {
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      const int d0 = 8 * cg + 32 * kk;  // pair index of element 0: d0 < 64
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float a = E::widen(get(f[kk], e)), b = E::widen(get(f[kk + 2], e));
-        const float c = tab[2 * (d0 + e)], sn = tab[2 * (d0 + e) + 1];
-        const float ra = a * c - b * sn;
-        const float rb = a * sn + b * c;
-        put(f[kk], e, E::round(ra));
-        put(f[kk + 2], e, E::round(rb));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int f0 = (8 * cg + 32 * kk) / 2;
+    for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float a = E::widen(get(f[kk], 2 * j)), b = E::widen(get(f[kk], 2 * j + 1));
-        const float c = tab[2 * (f0 + j)], sn = tab[2 * (f0 + j) + 1];
-        const float ra = a * c - b * sn;
-        const float rb = a * sn + b * c;
-        put(f[kk], 2 * j, E::round(ra));
-        put(f[kk], 2 * j + 1, E::round(rb));
+        const f32x4_t cs = t[4 * kk + j];
+        const float a0 = lo(f[kk][j]), a1 = hi(f[kk][j]), b0 = lo(f[kk + 2][j]), b1 = hi(f[kk + 2][j]);
+        f[kk][j] = E::pack2(a0 * cs[0] - b0 * cs[1], a1 * cs[2] - b1 * cs[3]);
+        f[kk + 2][j] = E::pack2(a0 * cs[1] + b0 * cs[0], a1 * cs[3] + b1 * cs[2]);
       }
-    }
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float c = t[2 * kk + (j >> 1)][2 * (j & 1)], sn = t[2 * kk + (j >> 1)][2 * (j & 1) + 1];
+        const float x = lo(f[kk][j]), y = hi(f[kk][j]);
+        f[kk][j] = E::pack2(x * c - y * sn, x * sn + y * c);
+      }
   }
+}
+
+// Maximum / sum over the four lanes that hold one column (they differ in bits 4 and 5 of the lane index):
+// v_permlane16_swap and v_permlane32_swap, no LDS crossbar.
+template <typename F> __device__ __forceinline__ float quad_reduce(float x, F f) {
+  typedef __attribute__((ext_vector_type(2))) unsigned u2;
+  unsigned u = __builtin_bit_cast(unsigned, x);
+  u2 r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  unsigned r0 = r[0], r1 = r[1];
+  u = __builtin_bit_cast(unsigned, f(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)));
+  r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  r0 = r[0];
+  r1 = r[1];
+  return f(__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1));
+}
+__device__ __forceinline__ float quad_max(float x) {
+  return quad_reduce(x, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float quad_sum(float x) {
+  return quad_reduce(x, [](float a, float b) { return a + b; });
 }
 
 // V staging swizzle for the 16x16x32 transposed reads: one instruction touches
@@ -121,93 +152,145 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
   return row * kRowBytes + ((((granule >> 1) ^ (row & 7)) << 5) | ((granule & 1) << 4));
 }
 
-template <typename T, bool FUSED>
-__global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams p) {
+constexpr int kMaxFoldSplits = 16;
+constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
+
+__device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
+
+// Buffer descriptor of `bytes` bytes: a load past them returns zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t byte_buffer(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+constexpr int kNonTemporal = 2, kScopeDevice = 16;  // cache policy operand: nt; sc1, past the XCD's own L2
+__device__ __forceinline__ u32x4_t stream_load(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kNonTemporal));
+}
+__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, f32x4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ f32x4_t load_device(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kScopeDevice));
+}
+__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, u32x2_t v) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, r, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
+}
+
+template <typename T, bool FUSED, int NW, bool LONG>
+__global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   using E = Elem<T>;
-  __shared__ __attribute__((aligned(16))) char lds[8 * kDecWaveLds];
+  constexpr int kStepKeys = NW * kDecWaveKeys;
+  __shared__ __attribute__((aligned(16))) char lds[2 * NW * kDecWaveLds];
 
   const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, cg = lane >> 4;
 
-  // A split is not a contiguous key range but every num_splits-th block of kDecStepKeys keys: the
-  // workgroups of one sequence then walk through its cache side by side, which the DRAM channels
-  // serve better than as many far-apart streams (the softmax merge does not care which keys a
-  // partial covers).
-  const int nblocks = (p.n + kDecStepKeys - 1) / kDecStepKeys;
-  const int k_end = p.n;
-  const int iters = (nblocks - split + p.num_splits - 1) / p.num_splits;  // blocks split, split + S, ...
-
-  const size_t kv_row_bytes = (size_t)p.Hkv * kRowBytes;
-  const size_t seq_off = (size_t)b * p.kv_seq_stride * kv_row_bytes + (size_t)kvh * kRowBytes;
-  const char *kbase = p.k + seq_off;
-  const char *vbase = p.v + seq_off;
+  const int iters = p.iters_each + (split < p.iters_rest);  // blocks split, split + S, ...
+  const int row_bytes = p.Hkv * kRowBytes;
+  const size_t seq_off = ((size_t)b * p.kv_seq_stride * p.Hkv + kvh) * kRowBytes;
+  const char *kbase = p.k + seq_off, *vbase = p.v + seq_off;
+  const int stored = FUSED ? p.n - 1 : p.n;  // rows that are in the cache
 
   // query column of this lane
   const bool col_valid = col < p.rows;
-  const int c_row = col_valid ? col / p.g : 0;
-  const int c_head = kvh * p.g + (col_valid ? col % p.g : 0);
+  const int c_row = col_valid ? (int)fast_div(col, p.g_div) : 0;
+  const int c_head = kvh * p.g + (col_valid ? col - c_row * p.g : 0);
   const int c_limit = c_row + p.offset;  // last visible key of this column
+  const bool new_col = FUSED && col == p.rows;  // this column carries the new K row through the rotation
 
   u32x4_t qf[4];
+  f32x4_t tab[8];
+  u32x4_t new_v;
   {
-    const char *qp = p.q + (((size_t)b * p.m + c_row) * p.H + c_head) * kRowBytes + cg * 16;
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      u32x4_t z = {0u, 0u, 0u, 0u};
-      qf[kk] = col_valid ? global_load_b128(qp + kk * 64) : z;
+    const char *qp = p.q + (size_t)b * p.m * p.H * kRowBytes;
+    uint32_t qo = (c_row * p.H + c_head) * kRowBytes + cg * 16;
+    if (new_col) {
+      qp = p.new_k;
+      qo = kvh * kRowBytes + cg * 16;
     }
-    if (FUSED && col_valid) rotate_frags<T>(qf, p.freq_row, cg, p.is_neox);
+    qp += qo;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) qf[kk] = u32x4_t{0u, 0u, 0u, 0u};
+    if (col_valid || new_col) {
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) qf[kk] = global_load_b128(qp + kk * 64);
+    }
+    if (FUSED) {
+      load_rotation(tab, p.freq_row, cg, p.is_neox);
+      new_v = global_load_b128(p.new_v + (size_t)kvh * kRowBytes + col * 16);
+    }
   }
+
+  int voff[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) voff[i] = (wave * kDecWaveKeys + 4 * i + cg) * row_bytes + col * 16;
+  u32x4_t kn[8], vn[8];
+  auto block_buffer = [&](const char *base, int it) {
+    const int first = (it * p.num_splits + split) * kStepKeys;
+    const int have = min(stored - first, kStepKeys);
+    const unsigned records = have > 0 ? (unsigned)(have - 1) * row_bytes + kRowBytes : 0u;
+    return byte_buffer(base + (size_t)first * row_bytes, records);
+  };
+  auto issue_k = [&](int it) {
+    const __amdgpu_buffer_rsrc_t r = block_buffer(kbase, it);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) kn[i] = stream_load(r, voff[i]);
+  };
+  auto issue_v = [&](int it) {
+    const __amdgpu_buffer_rsrc_t r = block_buffer(vbase, it);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) vn[i] = stream_load(r, voff[i]);
+  };
+  // The first step's K and V start together.  From then on they are fetched one after the other, each while the other
+  // half of the step is computed: 32 KiB in flight per CU is where this memory system streams fastest (64 KiB:
+  // every large shape 2-3 % slower; a plain read kernel shows the same optimum).  LONG, a workgroup with many
+  // blocks: V is asked for only after K's MFMAs and the next K after V's, a little less in flight (16 x 32768
+  // keys 303.1 -> 297.2 us, 1 x 32768 keys 25.1 -> 24.8).  With few blocks each goes out as soon as its
+  // registers are free (5 x 2999 keys, 4 blocks each: 15.6 -> 14.9 us).
+  issue_k(0);
+  issue_v(0);
 
   f32x4_t o[8];
 #pragma unroll
   for (int d = 0; d < 8; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;
-
   char *vl = lds + wave * kDecWaveLds;
-  char *kl = lds + (4 + wave) * kDecWaveLds;
-
-  u32x4_t kn[8], vn[8];
-  auto issue_k = [&](int it) {
-    const int kb0 = (it * p.num_splits + split) * kDecStepKeys + wave * kDecWaveKeys;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int key = min(kb0 + 4 * i + cg, p.n - 1);
-      const char *kp = kbase + (size_t)key * kv_row_bytes + col * 16;
-      if (FUSED && key == p.fused_pos) kp = p.new_k + (size_t)kvh * kRowBytes + col * 16;
-      kn[i] = global_load_b128_nt(kp);
-    }
-  };
-  auto issue_v = [&](int it) {
-    const int kb0 = (it * p.num_splits + split) * kDecStepKeys + wave * kDecWaveKeys;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int key = min(kb0 + 4 * i + cg, p.n - 1);
-      const char *vp = vbase + (size_t)key * kv_row_bytes + col * 16;
-      if (FUSED && key == p.fused_pos) vp = p.new_v + (size_t)kvh * kRowBytes + col * 16;
-      vn[i] = global_load_b128_nt(vp);
-    }
-  };
-
-  // K and V of a step are fetched one after the other, each while the other half of the step is
-  // computed: a wave has 8 KiB of loads in flight at any time, the CU 32 KiB.  That is where this
-  // memory system streams fastest -- with both in flight together (64 KiB per CU) every large shape
-  // measured 2-3 % slower, and a plain read kernel shows the same optimum.
-  // (The first step's K and V start together: one memory round trip less for a workgroup with one step.)
-  if (iters > 0) {
-    issue_k(0);
-    issue_v(0);
-  }
+  char *kl = lds + (NW + wave) * kDecWaveLds;
+  if (FUSED) rotate_frags<T>(qf, tab, p.is_neox);
 
   for (int it = 0; it < iters; ++it) {
-    const int kb0 = (it * p.num_splits + split) * kDecStepKeys + wave * kDecWaveKeys;
+    const int kb0 = (it * p.num_splits + split) * kStepKeys + wave * kDecWaveKeys;
+    const int at = p.fused_pos - kb0;               // FUSED: where in the wave's keys the new row is
+    const bool owner = FUSED && at >= 0 && at < kDecWaveKeys;
     u32x4_t kc[2][4];
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int i = 0; i < 8; ++i) lds_write_b128(kl, (4 * i + cg) * kRowBytes + ((col ^ ((4 * i + cg) & 15)) << 4), kn[i]);
+    if (owner) {
+      // the new token's K row takes its place among the staged rows and goes to the cache
+      u32x4_t nk[4] = {qf[0], qf[1], qf[2], qf[3]};
+      bool mine = new_col;
+      if (p.rows == kDecCols) {  // no spare column: one more rotation
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) nk[kk] = global_load_b128(p.new_k + (size_t)kvh * kRowBytes + cg * 16 + kk * 64);
+        load_rotation(tab, p.freq_row, cg, p.is_neox);
+        rotate_frags<T>(nk, tab, p.is_neox);
+        mine = col == 0;
+      }
+      if (mine) {
+        char *dst = const_cast<char *>(kbase) + (size_t)p.fused_pos * row_bytes + cg * 16;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          lds_write_b128(kl, at * kRowBytes + (((4 * kk + cg) ^ (at & 15)) << 4), nk[kk]);
+          *reinterpret_cast<u32x4_t *>(dst + kk * 64) = nk[kk];
+        }
+      }
+    }
     __builtin_amdgcn_wave_barrier();
-    if (it > 0) issue_v(it);
+    if (!LONG && it > 0) issue_v(it);
     // K fragments (A operand): key blk*16+col, dims 32kk + 8cg .. +7
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
@@ -215,21 +298,7 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams 
       for (int kk = 0; kk < 4; ++kk)
         kc[blk][kk] = lds_read_b128(kl, (blk * 16 + col) * kRowBytes + (((4 * kk + cg) ^ col) << 4));
 
-    if (kb0 < k_end) {
-      if (FUSED) {
-        // the new token's row: rotate K in registers and append both rows to the cache (lanes whose
-        // clamped key is the new row all hold and write the same bytes)
-#pragma unroll
-        for (int blk = 0; blk < 2; ++blk) {
-          const int key = min(kb0 + blk * 16 + col, p.n - 1);
-          if (key == p.fused_pos) {
-            rotate_frags<T>(kc[blk], p.freq_row, cg, p.is_neox);
-            char *dst = const_cast<char *>(kbase) + (size_t)key * kv_row_bytes + cg * 16;
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) *reinterpret_cast<u32x4_t *>(dst + kk * 64) = kc[blk][kk];
-          }
-        }
-      }
+    if (kb0 < p.n) {
       // ---- S^T = K Q^T : 2 blocks of 16 keys ----
       f32x4_t s[2];
 #pragma unroll
@@ -238,27 +307,38 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams 
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) s[blk] = E::mfma16(kc[blk][kk], qf[kk], s[blk]);
       }
-      float mloc = -INFINITY;
+      if (LONG && it > 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        issue_v(it);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (kb0 + kDecWaveKeys - 1 > min(p.offset, p.n - 1)) {
 #pragma unroll
-      for (int blk = 0; blk < 2; ++blk)
+        for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = kb0 + blk * 16 + 4 * cg + i;
-          float t = s[blk][i] * p.scale_log2e;
-          if (key >= k_end || key > c_limit) t = -INFINITY;
-          s[blk][i] = t;
-          mloc = fmaxf(mloc, t);
-        }
-      mloc = fmaxf(mloc, xor_lane(mloc, 16));
-      mloc = fmaxf(mloc, xor_lane(mloc, 32));
-      const float m_new = fmaxf(m_run, mloc);
+          for (int i = 0; i < 4; ++i) {
+            const int key = kb0 + blk * 16 + 4 * cg + i;
+            if (key >= p.n || key > c_limit) s[blk][i] = -INFINITY;
+          }
+      }
+      float mloc = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
+                         fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+      mloc = quad_max(mloc);
+      const float m_new = fmaxf(m_run, mloc * p.scale_log2e);
       const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-      const float alpha = fast_exp2(m_run - m_use);
-      m_run = m_new;
+      if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
+        const float alpha = fast_exp2(m_run - m_use);
+        l_run *= alpha;
+#pragma unroll
+        for (int d = 0; d < 8; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[d][i] *= alpha;
+        m_run = m_new;
+      }
 #pragma unroll
       for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[blk][i] = fast_exp2(s[blk][i] - m_use);
+        for (int i = 0; i < 4; ++i) s[blk][i] = fast_exp2(__builtin_fmaf(s[blk][i], p.scale_log2e, -m_use));
       // P^T as B operand: slot e<4 -> block 0 key 4cg+e, e>=4 -> block 1 key 4cg+e-4
       u32x4_t pf;
       pf[0] = E::pack2(s[0][0], s[0][1]);
@@ -271,21 +351,17 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams 
       psum = dot2_ones<T>(pf[1], psum);
       psum = dot2_ones<T>(pf[2], psum);
       psum = dot2_ones<T>(pf[3], psum);
-      l_run = l_run * alpha + psum;
+      l_run += psum;
       // ---- O^T += V^T P^T ----
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int i = 0; i < 8; ++i) lds_write_b128(vl, v_swizzle32_off(4 * i + cg, col), vn[i]);
-      if (FUSED) {  // the new token's V row goes to the cache
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int key = min(kb0 + 4 * i + cg, p.n - 1);
-          if (key == p.fused_pos)
-            *reinterpret_cast<u32x4_t *>(const_cast<char *>(vbase) + (size_t)key * kv_row_bytes + col * 16) = vn[i];
-        }
+      if (owner && cg == (at & 3)) {  // the new token's V row, likewise
+        lds_write_b128(vl, v_swizzle32_off(at, col), new_v);
+        *reinterpret_cast<u32x4_t *>(const_cast<char *>(vbase) + (size_t)p.fused_pos * row_bytes + col * 16) = new_v;
       }
       __builtin_amdgcn_wave_barrier();
-      if (it + 1 < iters) issue_k(it + 1);
+      if (it + 1 < iters && !LONG) issue_k(it + 1);
       const int vr = 4 * cg + (col >> 2);
       const int sub = (col & 1) * 8;
 #pragma unroll
@@ -294,36 +370,42 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams 
         const u32x2_t lo = lds_read_tr16(vl, v_swizzle32_off(vr, gran) + sub);
         const u32x2_t hi = lds_read_tr16(vl, v_swizzle32_off(vr + 16, gran) + sub);
         const u32x4_t vf = {lo[0], lo[1], hi[0], hi[1]};
-        f32x4_t acc = o[d];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] *= alpha;
-        o[d] = E::mfma16(vf, pf, acc);
+        o[d] = E::mfma16(vf, pf, o[d]);
+      }
+      if (it + 1 < iters && LONG) {
+        __builtin_amdgcn_sched_barrier(0);
+        issue_k(it + 1);
       }
     } else if (it + 1 < iters) {
       issue_k(it + 1);
     }
   }
 
-  // ---- merge the four waves ----
-  float l_tot = l_run + xor_lane(l_run, 16);
-  l_tot += xor_lane(l_tot, 32);
+  // ---- merge the waves ----
+  const float l_tot = quad_sum(l_run);
   __syncthreads();
-  float *lo_f = reinterpret_cast<float *>(lds);                      // [wave][col][128]
-  float *lml = reinterpret_cast<float *>(lds + 4 * kDecWaveLds);     // [wave][col][2] (the K staging space)
+  // [wave][col][128]; the 16-byte pieces of a row are XORed with the column, so that neither the columns of a
+  // write nor the pieces of a read meet in one bank
+  float *lo_f = reinterpret_cast<float *>(lds);
+  float *lml = reinterpret_cast<float *>(lds + NW * kDecWaveLds);    // [wave][col][2] (the K staging space)
 #pragma unroll
   for (int d = 0; d < 8; ++d)
-    *reinterpret_cast<f32x4_t *>(lo_f + ((wave * kDecCols + col) * kHeadDim + 16 * d + 4 * cg)) = o[d];
+    *reinterpret_cast<f32x4_t *>(lo_f + (wave * kDecCols + col) * kHeadDim + (((4 * d + cg) ^ col) << 2)) = o[d];
   if (cg == 0) {
     lml[(wave * kDecCols + col) * 2] = m_run;
     lml[(wave * kDecCols + col) * 2 + 1] = l_tot;
   }
   __syncthreads();
 
-  {
-    const int c = tid >> 4, dch = tid & 15;  // column, 8-wide d chunk
-    float mw[4], M = -INFINITY;
+  const size_t pair = (size_t)b * p.Hkv + kvh;
+  const int pair_slots = p.num_splits * p.cols;
+  const __amdgpu_buffer_rsrc_t po = byte_buffer(p.ws_o + pair * pair_slots * kHeadDim, pair_slots * kHeadDim * 4);
+  const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
+  for (int c = tid >> 4; c < p.rows; c += 4 * NW) {
+    const int dch = tid & 15;  // 8-wide d chunk of column c
+    float mw[NW], M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       mw[w] = lml[(w * kDecCols + c) * 2];
       M = fmaxf(M, mw[w]);
     }
@@ -332,32 +414,139 @@ __global__ __launch_bounds__(kDecThreads) void flash_decode_kernel(DecodeParams 
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < NW; ++w) {
       const float wt = fast_exp2(mw[w] - M_use);
       L += wt * lml[(w * kDecCols + c) * 2 + 1];
-      const float *src = lo_f + ((w * kDecCols + c) * kHeadDim + 8 * dch);
+      const float *src = lo_f + (w * kDecCols + c) * kHeadDim;
+      const f32x4_t s0 = *reinterpret_cast<const f32x4_t *>(src + (((2 * dch) ^ c) << 2));
+      const f32x4_t s1 = *reinterpret_cast<const f32x4_t *>(src + (((2 * dch + 1) ^ c) << 2));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] += wt * src[j];
+      for (int j = 0; j < 4; ++j) {
+        acc[j] += wt * s0[j];
+        acc[4 + j] += wt * s1[j];
+      }
     }
-    if (c < p.rows) {
-      if (p.num_splits == 1) {
-        const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-        const int r = c / p.g, hq = c % p.g;
-        char *op = p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + hq) * kRowBytes + dch * 16;
-        u32x4_t w;
+    if (p.num_splits == 1) {
+      const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
+      const int r = (int)fast_div(c, p.g_div), hq = c - r * p.g;
+      char *op = p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + hq) * kRowBytes + dch * 16;
+      u32x4_t w;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) w[j] = E::pack2(acc[2 * j] * inv, acc[2 * j + 1] * inv);
-        *reinterpret_cast<u32x4_t *>(op) = w;
-      } else {
-        const size_t slot = (((size_t)b * p.Hkv + kvh) * p.num_splits + split) * kDecCols + c;
-        float *wo = p.ws_o + slot * kHeadDim + 8 * dch;
-        *reinterpret_cast<f32x4_t *>(wo) = f32x4_t{acc[0], acc[1], acc[2], acc[3]};
-        *reinterpret_cast<f32x4_t *>(wo + 4) = f32x4_t{acc[4], acc[5], acc[6], acc[7]};
-        if (dch == 0) {
-          p.ws_ml[slot * 2] = M;
-          p.ws_ml[slot * 2 + 1] = L;
+      for (int j = 0; j < 4; ++j) w[j] = E::pack2(acc[2 * j] * inv, acc[2 * j + 1] * inv);
+      *reinterpret_cast<u32x4_t *>(op) = w;
+      continue;
+    }
+    const int slot = split * p.cols + c;
+    const f32x4_t a0 = {acc[0], acc[1], acc[2], acc[3]}, a1 = {acc[4], acc[5], acc[6], acc[7]};
+    const u32x2_t ml = {__builtin_bit_cast(uint32_t, M), __builtin_bit_cast(uint32_t, L)};
+    if (p.fold) {
+      store_device(po, slot * kHeadDim * 4 + dch * 32, a0);
+      store_device(po, slot * kHeadDim * 4 + dch * 32 + 16, a1);
+      if (dch == 0) store_device(pml, slot * 8, ml);
+    } else {
+      float *wo = p.ws_o + (pair * pair_slots + slot) * kHeadDim + 8 * dch;
+      *reinterpret_cast<f32x4_t *>(wo) = a0;
+      *reinterpret_cast<f32x4_t *>(wo + 4) = a1;
+      if (dch == 0) *reinterpret_cast<u32x2_t *>(p.ws_ml + (pair * pair_slots + slot) * 2) = ml;
+    }
+  }
+  if (!p.fold) return;
+
+  // ---- fold in the workgroup that finds every partial of its (sequence, kv head) stored ----
+  // Each workgroup raises its flag once its partial has reached the point where all XCDs see it, and looks at the
+  // others' after that: the last one to raise its flag finds all of them up (if two do, both write the
+  // same rows).  A flag is up if it holds this launch's number, whatever the workspace held before; the folding
+  // workgroup takes them down for a replay of the same launch.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  unsigned *all_up = reinterpret_cast<unsigned *>(lds);
+  const u32x2_t up = {(uint32_t)p.fold, (uint32_t)(p.fold >> 32)};
+  if (wave == 0) {
+    const int my_flag = (split * p.cols + p.cols - 1) * 8;
+    if (lane == 0) store_device(pml, my_flag, up);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const u32x2_t f = load_device2(pml, (min(lane, p.num_splits - 1) * p.cols + p.cols - 1) * 8);
+    const bool down = f[0] != up[0] || f[1] != up[1];
+    if (lane == 0) *all_up = 0;
+    if (__builtin_amdgcn_ballot_w64(down) == 0 && lane == 0) *all_up = 1;
+  }
+  __syncthreads();
+  if (*all_up == 0) return;
+  if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
+  // Groups of 32 threads, four dims each: `parts` groups per row deal its splits out among themselves.
+  constexpr int NG = 2 * NW;
+  const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
+  const int at_once = min(p.rows, NG), parts = NG / at_once;
+  const int part = sg / at_once;
+  float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = reinterpret_cast<float *>(lds) + 64;  // per group
+  for (int c0 = 0; c0 < p.rows; c0 += at_once) {
+    const int c = c0 + sg % at_once;
+    const bool mine = part < parts && c < p.rows;
+    float M = -INFINITY, L = 0.0f;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    // every partial of a thread's share is asked for before the first is used
+    auto take = [&](auto depth) {
+      constexpr int D = decltype(depth)::value;
+      const int s0 = part;
+      f32x4_t ov[D];
+      u32x2_t ml[D];
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const int slot = min(s0 + parts * j, S - 1) * p.cols + c;
+        ml[j] = load_device2(pml, slot * 8);
+        ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
+      }
+      float Mn = M;
+#pragma unroll
+      for (int j = 0; j < D; ++j)
+        if (s0 + parts * j < S) Mn = fmaxf(Mn, bits_float(ml[j][0]));
+      const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
+      const float resc = fast_exp2(M - M_use);
+      L *= resc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] *= resc;
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const float wt = (s0 + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
+        L += wt * bits_float(ml[j][1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
+      }
+      M = Mn;
+    };
+    if (mine) {
+      if (S <= kFoldDepth * parts)
+        take(std::integral_constant<int, kFoldDepth>());
+      else
+        take(std::integral_constant<int, kMaxFoldSplits>());
+    }
+    if (parts > 1) {
+      if (d4 == 0) {
+        red_ml[2 * sg] = M;
+        red_ml[2 * sg + 1] = L;
+      }
+      *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
+      __syncthreads();
+      if (part == 0) {
+        for (int g2 = sg + at_once; g2 < parts * at_once; g2 += at_once) {
+          const float m2 = red_ml[2 * g2], Mn = fmaxf(M, m2);
+          const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
+          const float wa = fast_exp2(M - M_use), wb = fast_exp2(m2 - M_use);
+          L = L * wa + red_ml[2 * g2 + 1] * wb;
+          const f32x4_t o2 = *reinterpret_cast<const f32x4_t *>(red_o + g2 * kHeadDim + 4 * d4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] = acc[i] * wa + o2[i] * wb;
+          M = Mn;
         }
       }
+    }
+    if (part == 0 && c < p.rows) {
+      const int r = (int)fast_div(c, p.g_div);
+      const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
+      u32x2_t w;
+      w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
+      w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
+      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + c - r * p.g) * kRowBytes + d4 * 8) = w;
     }
   }
 }
@@ -377,9 +566,9 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(DecodeParams 
   const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
   const int S = p.num_splits;
   const size_t base = ((size_t)b * p.Hkv + kvh) * S;
-  const float *ml = p.ws_ml + (base * kDecCols + c) * 2;
-  const float *src = p.ws_o + (base * kDecCols + c) * kHeadDim + 4 * d4;
-  const size_t ml_stride = (size_t)kDecCols * 2, o_stride = (size_t)kDecCols * kHeadDim;
+  const float *ml = p.ws_ml + (base * p.cols + c) * 2;
+  const float *src = p.ws_o + (base * p.cols + c) * kHeadDim + 4 * d4;
+  const size_t ml_stride = (size_t)p.cols * 2, o_stride = (size_t)p.cols * kHeadDim;
   float M = -INFINITY, L = 0.0f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = sg; s0 < S; s0 += 32) {  // rounds of up to 4 splits per thread
@@ -432,7 +621,7 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(DecodeParams 
     for (int i = 0; i < 4; ++i) tot[i] += wt * o[i];
   }
   const float inv = (Lt > 0.0f) ? 1.0f / Lt : 0.0f;
-  const int r = c / p.g, hq = c % p.g;
+  const int r = (int)fast_div(c, p.g_div), hq = c - r * p.g;
   u32x2_t w;
   w[0] = E::pack2(tot[0] * inv, tot[1] * inv);
   w[1] = E::pack2(tot[2] * inv, tot[3] * inv);
@@ -452,15 +641,16 @@ int flash_decode_max_default_splits(long long pairs) {
 // Split count that a simple model of the launch makes fastest.  Workgroups run one per CU in rounds
 // of as many workgroups as the device has CUs; a CU of a full round streams 27.7 GB/s (all 256 of an
 // MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads), a CU of a thin
-// round at most 32 GB/s (one workgroup keeps 32 KiB of loads in flight); a workgroup costs 3 us beyond
-// its bytes, the combine launch 5 us.  Among the counts within 3 % of the best, one that fills its
+// round the more the fewer they are (32 KiB in flight over a latency that grows with the load: 50 GB/s for a
+// handful, 40 for half the chip); a workgroup costs 3 us beyond its bytes, folding up to 16 partials in the
+// kernel 2.4 us, the combine launch 3.1 us.  Among the counts within 3 % of the best, one that fills its
 // rounds exactly is preferred, else the smallest.  For the common shapes this is about one workgroup
 // per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that do not divide a round
-// it finds the count that fills the rounds.  Model / measured us on 256 CUs, bf16, cold: batch 1,
-// n = 32768, 32 splits 26.9 / 26.2; batch 16, n = 4096, 2 splits 45.9 / 44.6; n = 8192: batch 12,
-// 5 splits 68.6 / 68.6, batch 20, 3 splits 108.5 / 107.6, batch 40, 4 splits 209.3 / 206.8, batch 48,
-// 2 splits 241.1 / 234.4 -- in a sweep of 38 shapes the count chosen is the fastest measured one or
-// within 1.6 % of it.
+// it finds the count that fills the rounds.  Model / measured us on 256 CUs, bf16, cold: batch 1, 8 kv heads,
+// n = 384, 3 splits 6.7 / 6.9, n = 32768, 32 splits 25.0 / 25.4; batch 12, n = 8192, 2 splits 65.1 / 65.4,
+// 5 splits 67.5 / 67.2; batch 40, n = 8192, 4 splits 206.7 / 211; batch 12, 32 kv heads, n = 1000,
+// 1 split 35.4 / 36.3, 2 splits 39.8 / 40.5 -- of 229 shapes measured (batch 1-64, 100-32768 keys, 2-32 kv heads) the
+// count chosen is the fastest measured one or within 3 % of it in all but 6, and there within 8 %.
 static int default_splits_model(long long pairs, int nblocks, int cus) {
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
@@ -473,11 +663,12 @@ static int default_splits_model(long long pairs, int nblocks, int cus) {
     const double wg_bytes = key_bytes * kDecStepKeys * ((nblocks + s - 1) / s);
     double t = full * (wg_bytes / 27.7e9 + 3e-6);
     if (rest > 0) {
-      double rate = all_cus / (double)rest;
-      if (rate > 32e9) rate = 32e9;
+      double rate = 0.95 * all_cus / (double)rest;
+      const double alone = 50e9 - 20e9 * (double)rest / cus;
+      if (rate > alone) rate = alone;
       t += wg_bytes / rate + 3e-6;
     }
-    return s > 1 ? t + 5e-6 : t;
+    return s == 1 ? t : t + (s <= kMaxFoldSplits ? 2.4e-6 : 3.1e-6);
   };
   double t_min = model(1);
   for (int s = 2; s <= smax; ++s) {
@@ -529,41 +720,78 @@ size_t flash_decode_workspace_bytes(int batch, int m, int group_size, int kv_hea
   return slots * (kHeadDim + 2) * sizeof(float);
 }
 
-static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, int batch, int kv_head_num, int num_splits,
-                                     int dt, bool fused, hipStream_t stream) {
-  p.num_splits = flash_decode_effective_splits(num_splits, p.n);
-  p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
-  const size_t slots = (size_t)batch * kv_head_num * p.num_splits * kDecCols;
-  p.ws_o = static_cast<float *>(workspace);
-  p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;
-  dim3 grid(p.num_splits, kv_head_num, batch);
-  void (*kern)(DecodeParams) = (dt == kDtFloat16)
-                                   ? (fused ? flash_decode_kernel<_Float16, true> : flash_decode_kernel<_Float16, false>)
-                                   : (fused ? flash_decode_kernel<__bf16, true> : flash_decode_kernel<__bf16, false>);
+// A number that no workspace holds by chance: the flags of a folding launch (see the kernel).
+static uint64_t launch_number() {
+  static std::atomic<uint64_t> next{[] {
+    std::random_device rd;
+    return ((uint64_t)rd() << 32) ^ rd() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
+  }()};
+  uint64_t n;
+  do n = next.fetch_add(0x9E3779B97F4A7C15ull, std::memory_order_relaxed);
+  while (n == 0);
+  return n;
+}
+
+template <typename T, bool FUSED, int NW, bool LONG>
+static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   // kDecLdsPad bytes of dynamic LDS that nobody touches keep a second workgroup off the CU (two of
   // them would put 64 KiB of loads in flight again).  More than 64 KiB of LDS in total is an opt-in
   // per device and kernel.
-  static std::atomic<uint64_t> attr_done[4] = {};
-  const int which = (dt == kDtFloat16 ? 0 : 2) + (fused ? 1 : 0);
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
-  if (e != hipSuccess) return e;
-  const uint64_t bit = 1ull << (dev & 63);
-  if (!(attr_done[which].load(std::memory_order_acquire) & bit)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                            kDecLdsPad);
+  constexpr int pad = NW == 4 ? kDecLdsPad : 0;
+  void (*kern)(DecodeParams) = flash_decode_kernel<T, FUSED, NW, LONG>;
+  if (pad) {
+    static std::atomic<uint64_t> attr_done{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return e;
-    attr_done[which].fetch_or(bit, std::memory_order_release);
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(attr_done.load(std::memory_order_acquire) & bit)) {
+      e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, pad);
+      if (e != hipSuccess) return e;
+      attr_done.fetch_or(bit, std::memory_order_release);
+    }
   }
-  hipLaunchKernelGGL(kern, grid, dim3(kDecThreads), kDecLdsPad, stream, p);
-  e = hipGetLastError();
-  if (e != hipSuccess || p.num_splits == 1) return e;
-  dim3 cgrid(p.rows, kv_head_num, batch);
-  if (dt == kDtFloat16)
-    hipLaunchKernelGGL(flash_decode_combine_kernel<_Float16>, cgrid, dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL(flash_decode_combine_kernel<__bf16>, cgrid, dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.num_splits, p.Hkv, p.batch), dim3(64 * NW), pad, stream, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.num_splits == 1 || p.fold) return e;
+  hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream, p);
   return hipGetLastError();
+}
+
+template <typename T, bool FUSED>
+static hipError_t launch_decode(const DecodeParams &p, bool half, bool many, hipStream_t stream) {
+  if (half) return launch_decode_t<T, FUSED, 2, false>(p, stream);
+  return many ? launch_decode_t<T, FUSED, 4, true>(p, stream) : launch_decode_t<T, FUSED, 4, false>(p, stream);
+}
+
+static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, int num_splits, int dt, bool fused,
+                                     hipStream_t stream) {
+  p.num_splits = flash_decode_effective_splits(num_splits, p.n);
+  p.cols = kDecCols;
+  int nblocks = (p.n + kDecStepKeys - 1) / kDecStepKeys;
+  // Short caches: where every workgroup has one block of 128 keys and twice as many workgroups still fit the chip at
+  // once, blocks of 64 keys and workgroups of two waves.  Their slots have half the columns, so the
+  // partials take no more room (one column is the flag's: up to 7 query rows).
+  const int half_blocks = (p.n + kDecStepKeys / 2 - 1) / (kDecStepKeys / 2);
+  const bool half = p.num_splits > 1 && p.num_splits == nblocks && p.rows < kDecCols / 2 && half_blocks <= kFoldDepth &&
+                    (long long)p.batch * p.Hkv * half_blocks <= device_compute_units();
+  if (half) {
+    p.num_splits = nblocks = half_blocks;
+    p.cols = kDecCols / 2;
+  }
+  p.iters_each = nblocks / p.num_splits;
+  p.iters_rest = nblocks % p.num_splits;
+  // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
+  p.fold = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? launch_number() : 0;
+  p.g_div = make_fast_div((uint32_t)p.g);
+  p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
+  const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
+  p.ws_o = static_cast<float *>(workspace);
+  p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;
+  const bool many = p.iters_each >= 8;  // long enough to be bound by the stream, see the kernel
+  if (dt == kDtFloat16)
+    return fused ? launch_decode<_Float16, true>(p, half, many, stream) : launch_decode<_Float16, false>(p, half, many, stream);
+  return fused ? launch_decode<__bf16, true>(p, half, many, stream) : launch_decode<__bf16, false>(p, half, many, stream);
 }
 
 hipError_t launch_flash_decode(void *out, const void *q, const void *k, const void *v,
@@ -584,7 +812,7 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
   p.Hkv = kv_head_num;
   p.H = group_size * kv_head_num;
   p.rows = m * group_size;
-  return launch_decode_impl(p, workspace, batch, kv_head_num, num_splits, dt, false, stream);
+  return launch_decode_impl(p, workspace, num_splits, dt, false, stream);
 }
 
 // One decode step of one sequence with the rotary embedding and the cache append inside the decode
@@ -612,7 +840,7 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
   p.freq_row = static_cast<const float *>(freq_cis) + (size_t)pos * kHeadDim;
   p.fused_pos = pos;
   p.is_neox = is_neox ? 1 : 0;
-  return launch_decode_impl(p, workspace, 1, kv_head_num, num_splits, dt, true, stream);
+  return launch_decode_impl(p, workspace, num_splits, dt, true, stream);
 }
 
 // ---------------------------------------------------------------------------
