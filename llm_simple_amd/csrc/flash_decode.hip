@@ -639,37 +639,32 @@ int flash_decode_max_default_splits(long long pairs) {
 }
 
 // Split count that a simple model of the launch makes fastest.  Workgroups run one per CU in rounds
-// of as many workgroups as the device has CUs; a CU of a full round streams 27.7 GB/s (all 256 of an
+// of as many workgroups as the device has CUs; a CU of a full round streams 27.9 GB/s (all 256 of an
 // MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads), a CU of a thin
-// round the more the fewer they are (32 KiB in flight over a latency that grows with the load: 50 GB/s for a
-// handful, 40 for half the chip); a workgroup costs 3 us beyond its bytes, folding up to 16 partials in the
-// kernel 2.4 us, the combine launch 3.1 us.  Among the counts within 3 % of the best, one that fills its
-// rounds exactly is preferred, else the smallest.  For the common shapes this is about one workgroup
-// per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that do not divide a round
-// it finds the count that fills the rounds.  Model / measured us on 256 CUs, bf16, cold: batch 1, 8 kv heads,
-// n = 384, 3 splits 6.7 / 6.9, n = 32768, 32 splits 25.0 / 25.4; batch 12, n = 8192, 2 splits 65.1 / 65.4,
-// 5 splits 67.5 / 67.2; batch 40, n = 8192, 4 splits 206.7 / 211; batch 12, 32 kv heads, n = 1000,
-// 1 split 35.4 / 36.3, 2 splits 39.8 / 40.5 -- of 229 shapes measured (batch 1-64, 100-32768 keys, 2-32 kv heads) the
-// count chosen is the fastest measured one or within 3 % of it in all but 6, and there within 8 %.
+// round the more the fewer they are (32 KiB in flight, a little more in short streams, over a latency that grows with
+// the load); a workgroup costs about 3 us beyond its bytes, folding up to 16 partials in the
+// kernel 3.1 us, 2.3 in blocks of 64 keys, the combine launch 2.3 us.  (Constants fitted over 250 shapes,
+// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %.)  Among the counts within
+// 3 % of the best, one that fills its rounds exactly is preferred, else the smallest.  For the common shapes
+// this is about one workgroup per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that
+// do not divide a round it finds the count that fills the rounds.  Over those shapes the count chosen is the
+// fastest measured one or within 12 % of it, 0.5 % on average.
+static double split_model_us(long long pairs, int nblocks, int s, int cus) {
+  const long long wgs = pairs * s;
+  const long long full = wgs / cus, rest = wgs % cus;
+  const int blocks = (nblocks + s - 1) / s;
+  const double wg_kb = 2.0 * kRowBytes * kDecStepKeys * blocks * 1e-3;  // K and V rows of one kv head
+  double t = full * (wg_kb / 27.9 + 2.7);
+  if (rest > 0) t += wg_kb / ((blocks >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
+  if (s == 1) return t;
+  if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 2.3;
+  return t + (s <= kMaxFoldSplits ? 3.1 : 2.3);
+}
 static int default_splits_model(long long pairs, int nblocks, int cus) {
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
   if (smax < 1) smax = 1;
-  const double key_bytes = 2.0 * kRowBytes;  // K and V row of one kv head
-  const double all_cus = 27.7e9 * cus;       // what the memory system gives all CUs together
-  auto model = [&](int s) {
-    const long long wgs = pairs * s;
-    const long long full = wgs / cus, rest = wgs % cus;
-    const double wg_bytes = key_bytes * kDecStepKeys * ((nblocks + s - 1) / s);
-    double t = full * (wg_bytes / 27.7e9 + 3e-6);
-    if (rest > 0) {
-      double rate = 0.95 * all_cus / (double)rest;
-      const double alone = 50e9 - 20e9 * (double)rest / cus;
-      if (rate > alone) rate = alone;
-      t += wg_bytes / rate + 3e-6;
-    }
-    return s == 1 ? t : t + (s <= kMaxFoldSplits ? 2.4e-6 : 3.1e-6);
-  };
+  auto model = [&](int s) { return split_model_us(pairs, nblocks, s, cus); };
   double t_min = model(1);
   for (int s = 2; s <= smax; ++s) {
     const double t = model(s);
