@@ -19,14 +19,19 @@
 // moves lazily, so O is rarely rescaled.  Accumulation is fp32; out =
 // O / l rounded once; l sums the ROUNDED probabilities (what P.V used).
 //
-// flash_prefill_kernel<T, NW, KB, NT>: NW waves share the K/V tiles of 16*NW*KB query rows.
-// NW = 8, KB = 2 (256 rows, one workgroup per CU) once there are about 1.5 such workgroups per CU;
-// NW = 4, KB = 2 (128 rows, two workgroups per CU) below that; NW = 8, KB = 1 (128 rows, two waves
-// per row block, each taking one 32-key half of every tile) up to two 128-row workgroups per CU;
-// NW = 4, KB = 1 (64 rows, paired waves, two workgroups per CU) up to about 1.2 per CU.  NT: the
-// tile loads are non-temporal (chunks whose K/V tiles only one workgroup reads).
+// flash_prefill_kernel<T, NW, KP, NT>: NW waves share the K/V tiles of 32*NW/KP query rows, KP of them every
+// row block, each on its own 32 keys of every tile (KP = 1: on all 64).  While the chip is not full a launch
+// waits for the serial chain of the waves with the most keys -- a step of a wave takes 1600-1900 cycles
+// where its MFMAs take 512, and nothing else runs on its SIMD -- so that short prompts and chunks want many waves per
+// row (KP = 4: 512 tokens, 28 heads 11.5 -> 9.2 us; 256 tokens, 32 heads 8.7 -> 6.7), long ones the
+// cheapest step (KP = 1, 256 rows).  NT: the tile loads are non-temporal (chunks whose K/V tiles only one
+// workgroup reads).
+// Outside the loop a workgroup costs a short launch 2-3 us: indexes come from divisions prepared by the host, Q
+// of shared rows is fetched once through LDS, and waves that shared rows trade pieces of O^T so that each
+// folds and stores its part (epilogue of a pair 3900 -> 2200 cycles).
 // Tiles travel global -> LDS without VGPR staging (global_load_lds_dwordx4), spread over the MFMA
-// stream in the 8-wave kernels, issued beside the first MFMAs of a phase in the 4-wave ones.  The loop is software pipelined inside a wave: the MFMAs of S(j+1) are issued beside the
+// stream in the 8-wave kernels, issued beside the first MFMAs of a phase in the others.  The loop is
+// software pipelined inside a wave: the MFMAs of S(j+1) are issued beside the
 // softmax of tile j (the first ones beside the row-maximum chain, the rest, together with the
 // MFMAs of P(j).V(j), beside the exponentials), so K is fetched one tile ahead of V.
 // Every LDS fragment address is a loop-invariant register plus an immediate, and a
@@ -36,16 +41,17 @@
 // A chunk of few query rows over a long cache (chunked prefill) has its key range split over
 // workgroups: each leaves an fp32 partial (reference maximum, sum, unnormalised O) and
 // prefill_combine_kernel (or, for few rows and many ranges, prefill_combine_wide_kernel) folds
-// them; a chunk shorter than a tile packs the query heads of a kv head into the rows of one tile.  plan_prefill decides all of this from the shape and the
-// device's CU count.
+// them; the query heads of a kv head can share the rows of a tile.  plan_prefill decides all of this from the
+// shape and the device's CU count.
 #include <atomic>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
 
 namespace LLMHIP_NS {
 
-constexpr int kTileN = 64;                      // keys per LDS tile
+constexpr int kTileN = 64;                      // keys per LDS tile (128 where four waves share the rows)
 constexpr int kTileBytes = kTileN * kRowBytes;  // 16 KiB
 constexpr float kLazyLog2 = 8.0f;                // rescale threshold, log2 units
 constexpr int kMaxPrefillSplits = 128;           // key ranges per call
@@ -59,7 +65,9 @@ struct PrefillParams {
   int H, Hkv, g;
   int num_q_tiles;
   int sched_mode;  // 0: plain, 1: several XCDs per kv head, 2: several kv heads per XCD
-  int sched_a;     // mode 1: XCDs per kv head; mode 2: heads per XCD
+  int sched_a, sched_shift;  // mode 1: XCDs per kv head and its logarithm
+  FastDiv per_split, list_heads;  // of an XCD's work list: items per key range, heads
+  FastDiv g_div;
   float scale_log2e;
   // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers
   // keys [s*chunk, (s+1)*chunk); with more than one split every workgroup leaves an fp32 partial
@@ -84,44 +92,26 @@ struct PrefillParams {
 // list, so that every XCD gets the same number of workgroups whatever the head count.
 __device__ __forceinline__ bool prefill_schedule(const PrefillParams &p, int bid, int &tile,
                                                  int &head, int &split) {
-  const int T = p.num_q_tiles;
-  if (p.pack) {  // packed rows: items are (key range, tile, kv head)
-    const int per = T * p.Hkv;
-    if (bid >= per * p.num_splits) return false;
-    split = bid / per;
-    const int rem = bid % per;
-    tile = T - 1 - rem / p.Hkv;
-    head = (rem % p.Hkv) * p.g;  // first query head of the kv head
-    return true;
+  int idx = bid, xcd = 0;
+  if (p.sched_mode != 0) {
+    xcd = bid & 7;
+    idx = bid >> 3;
+    if (p.sched_mode == 1) {  // sched_a = 2^sched_shift XCDs per kv head
+      idx = (idx << p.sched_shift) + (xcd & (p.sched_a - 1));
+      xcd >>= p.sched_shift;  // the kv head
+    }
   }
-  if (p.sched_mode == 1) {
-    const int X = p.sched_a;
-    const int xcd = bid & 7, slot = bid >> 3;
-    const int kvh = xcd / X, sub = xcd % X;
-    const int idx = slot * X + sub, per = p.g * T;
-    if (idx >= per * p.num_splits) return false;
-    split = idx / per;
-    const int rem = idx % per;
-    tile = T - 1 - rem / p.g;
-    head = kvh * p.g + rem % p.g;
-    return true;
-  }
-  if (p.sched_mode == 2) {
-    const int hp = p.sched_a;
-    const int xcd = bid & 7, slot = bid >> 3, per = hp * T;
-    if (slot >= per * p.num_splits) return false;
-    split = slot / per;
-    const int rem = slot % per;
-    tile = T - 1 - rem / hp;
-    head = xcd * hp + rem % hp;
-    return true;
-  }
-  const int per = T * p.H;
-  if (bid >= per * p.num_splits) return false;
-  split = bid / per;
-  const int rem = bid % per;
-  tile = T - 1 - rem / p.H;
-  head = rem % p.H;
+  // idx: (key range, tile from the last, head among the list's `list_heads`)
+  if (idx >= (int)p.per_split.d * p.num_splits) return false;
+  split = (int)fast_div(idx, p.per_split);
+  const int rem = idx - split * (int)p.per_split.d;
+  const int t = (int)fast_div(rem, p.list_heads);
+  const int h = rem - t * (int)p.list_heads.d;
+  tile = p.num_q_tiles - 1 - t;
+  if (p.pack)
+    head = h * p.g;  // the list holds kv heads: first query head of the kv head
+  else
+    head = xcd * (int)p.list_heads.d + h;
   return true;
 }
 
@@ -200,6 +190,11 @@ template <typename T, int KB = 2> struct WaveAttn {
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qf[kk] = global_load_b128(q_row_head + hh * 16 + kk * 32);
   }
+  // The same fragments of 32 rows in LDS, laid out like a K tile; off: their place less this wave's first tile row
+  __device__ __forceinline__ void load_q_lds(const char *lds, int off) {
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) qf[kk] = lds_read_b128(lds, k_addr[kk] + off);
+  }
   // The Q loads are complete after this: no wait inside the key loop is ever
   // attributed to them.
   __device__ __forceinline__ void pin_q() {
@@ -257,13 +252,12 @@ template <typename T, int KB = 2> struct WaveAttn {
   // Causal / length mask of one tile of scores (only called for tiles that can be cut); key0 =
   // first key of the wave's part of the tile.
   __device__ __forceinline__ void mask(f32x16_t (&s)[KB], int key0, int qrow, int offset, int n) {
+    const int last = min(qrow + offset, n - 1) - key0 - 4 * hh;  // the lane's last key, from its first one
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = key0 + kb * 32 + 8 * (i >> 2) + 4 * hh + (i & 3);
-        if (key > qrow + offset || key >= n) s[kb][i] = -INFINITY;
-      }
+      for (int i = 0; i < 16; ++i)
+        if (kb * 32 + 8 * (i >> 2) + (i & 3) > last) s[kb][i] = -INFINITY;
   }
 
   // P = exp2(s*c + neg_ms) rounded to T and packed as the B operand; returns this lane's sum
@@ -331,90 +325,143 @@ template <typename T, int KB = 2> struct WaveAttn {
     return -((m_run == -INFINITY) ? 0.0f : m_run) * scale_log2e;
   }
 
-  // Two waves that shared the rows (KB == 1): the second writes its state to LDS lane by lane
-  // (66 floats per lane, stride 64 floats between a lane's values: conflict-free), the first folds
-  // it into its own.  The reference maxima are uniform over a lane pair in both waves.
-  __device__ __forceinline__ void export_state(float *lds_pair) const {
+  // KP waves that shared the rows (KB == 1) trade pieces of O^T: wave `part` keeps and will store the
+  // ND = 4 / KP d blocks part*ND .., and hands every other wave the blocks that one keeps, with its maximum and
+  // sum.  All as 16-byte pieces, lane by lane: conflict-free.  The maxima are uniform over a lane pair in
+  // all of them.  lds_rows: trade_bytes(KP) bytes of the row block.
+  static constexpr int kPieceBytes = 4 * 1024;  // one d block of a wave
+  static constexpr int give_bytes(int kp) { return (4 - 4 / kp) * kPieceBytes + 512; }
+  static constexpr int trade_bytes(int kp) { return kp * give_bytes(kp); }
+  template <int KP> __device__ __forceinline__ void give(char *lds_rows, int part) const {
+    constexpr int ND = 4 / KP;
+    char *mine = lds_rows + part * give_bytes(KP);
+    f32x4_t *dst = reinterpret_cast<f32x4_t *>(mine) + lane;
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int d = 0; d < 4; ++d) {
+      if (d / ND == part) continue;  // (wave-uniform)
+      f32x4_t *piece = dst + (d / ND < part ? d : d - ND) * 256;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) lds_pair[(d * 16 + i) * 64 + lane] = o[d][i];
-    lds_pair[64 * 64 + lane] = m_run;
-    lds_pair[65 * 64 + lane] = l_run;
+      for (int i4 = 0; i4 < 4; ++i4)
+        piece[i4 * 64] = f32x4_t{o[d][4 * i4], o[d][4 * i4 + 1], o[d][4 * i4 + 2], o[d][4 * i4 + 3]};
+    }
+    *reinterpret_cast<float2 *>(mine + give_bytes(KP) - 512 + lane * 8) = float2{m_run, l_run};
   }
-  __device__ __forceinline__ void import_state(const float *lds_pair, float scale_log2e) {
-    const float m_b = lds_pair[64 * 64 + lane], l_b = lds_pair[65 * 64 + lane];
-    const float m_new = fmaxf(m_run, m_b);
+  // Folds what the others gave into d blocks PART*ND ..
+  template <int KP, int PART> __device__ __forceinline__ void take(const char *lds_rows, float scale_log2e) {
+    constexpr int ND = 4 / KP;
+    float2 ml[KP];
+    float m_new = m_run;
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+      ml[q] = float2{m_run, l_run};
+      if (q != PART)
+        ml[q] = *reinterpret_cast<const float2 *>(lds_rows + (q + 1) * give_bytes(KP) - 512 + lane * 8);
+    }
+#pragma unroll
+    for (int q = 0; q < KP; ++q) m_new = fmaxf(m_new, ml[q].x);
     const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-    const float fa = fast_exp2((m_run - m_use) * scale_log2e), fb = fast_exp2((m_b - m_use) * scale_log2e);
-    l_run = l_run * fa + l_b * fb;
+    const float f_own = fast_exp2((m_run - m_use) * scale_log2e);
+    float l = 0.0f;  // in the same order in every wave
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int d = PART * ND; d < PART * ND + ND; ++d)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) o[d][i] = o[d][i] * fa + lds_pair[(d * 16 + i) * 64 + lane] * fb;
+      for (int i = 0; i < 16; ++i) o[d][i] *= f_own;
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+      const float f = fast_exp2((ml[q].x - m_use) * scale_log2e);
+      l = __builtin_fmaf(ml[q].y, f, l);
+      if (q == PART) continue;
+      const f32x4_t *src = reinterpret_cast<const f32x4_t *>(lds_rows + q * give_bytes(KP)) + lane;
+#pragma unroll
+      for (int d = PART * ND; d < PART * ND + ND; ++d)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const f32x4_t v = src[((d / ND < q ? d : d - ND) * 4 + i4) * 64];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[d][4 * i4 + i] = __builtin_fmaf(v[i], f, o[d][4 * i4 + i]);
+        }
+    }
     m_run = m_new;
+    l_run = l;
   }
 
-  // out[row][head][0..127] = O^T / l, rounded once.  The lane layout of O^T (a lane holds 4
-  // contiguous dims of one row at 16 places) would make every store instruction touch 32
-  // rows with 16 bytes each; the tile goes through this wave's private 8 KiB of LDS instead
-  // (16-byte granule XOR row%16: conflict-free both ways) and leaves as whole 256-byte rows,
-  // 16 lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the wave][head];
+  // out[row][head][32*D0 .. +32*ND) = O^T / l, rounded once.  The lane layout of O^T (a lane holds 4
+  // contiguous dims of one row at 4*ND places) would make every store instruction touch 32
+  // rows with 16 bytes each; the tile goes through 2*ND KiB of LDS of this wave instead
+  // (16-byte granule XOR row: conflict-free both ways) and leaves as whole pieces of 64*ND bytes,
+  // 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the wave][head];
   // rows_valid: how many of the wave's 32 rows exist.
+  template <int D0 = 0, int ND = 4>
   __device__ __forceinline__ void store(char *lds_wave, char *out_blk, size_t row_bytes, int rows_valid) {
+    constexpr int G = 4 * ND, RB_ = G * 16, RPI = 64 / G;  // granules and bytes of a row, rows per instruction
     const float l_tot = pair_sum(l_run);
     const float inv = (l_tot > 0.0f) ? 1.0f / l_tot : 0.0f;
 #pragma unroll
-    for (int d = 0; d < 4; ++d)
+    for (int d = 0; d < ND; ++d)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
         u32x2_t w;
-        w[0] = E::pack2(o[d][4 * i4] * inv, o[d][4 * i4 + 1] * inv);
-        w[1] = E::pack2(o[d][4 * i4 + 2] * inv, o[d][4 * i4 + 3] * inv);
+        w[0] = E::pack2(o[D0 + d][4 * i4] * inv, o[D0 + d][4 * i4 + 1] * inv);
+        w[1] = E::pack2(o[D0 + d][4 * i4 + 2] * inv, o[D0 + d][4 * i4 + 3] * inv);
         const int gran = 4 * d + i4;  // 16-byte granule of dims 32d + 8*i4 .. +7; hh picks its half
-        *reinterpret_cast<u32x2_t *>(lds_wave + l32 * kRowBytes + ((gran ^ (l32 & 15)) << 4) + hh * 8) = w;
+        *reinterpret_cast<u32x2_t *>(lds_wave + l32 * RB_ + ((gran ^ (l32 & (G - 1))) << 4) + hh * 8) = w;
       }
     __builtin_amdgcn_wave_barrier();  // wave-private region: LDS ops of one wave complete in order
+    const int r0 = lane / G, g0 = lane % G;
+    u32x4_t v[2 * ND];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int r = 4 * t + g16;
-      const u32x4_t v = lds_read_b128(lds_wave, r * kRowBytes + ((li ^ (r & 15)) << 4));
-      if (r < rows_valid) *reinterpret_cast<u32x4_t *>(out_blk + (size_t)r * row_bytes + li * 16) = v;
+    for (int t = 0; t < 2 * ND; ++t) {
+      const int r = RPI * t + r0;
+      v[t] = lds_read_b128(lds_wave, r * RB_ + ((g0 ^ (r & (G - 1))) << 4));
+    }
+    char *dst = out_blk + (size_t)r0 * row_bytes + D0 * 64 + g0 * 16;
+#pragma unroll
+    for (int t = 0; t < 2 * ND; ++t) {
+      if (RPI * t + r0 < rows_valid) *reinterpret_cast<u32x4_t *>(dst) = v[t];
+      dst += RPI * row_bytes;
     }
   }
 };
 
-// Partial result of one key range (see PrefillParams::num_splits): this lane's row gets its
+// Partial result of one key range (see PrefillParams::num_splits): this lane's row gets d blocks D0 .. D0+ND-1 of its
 // unnormalised O^T as fp32, and (reference maximum in raw score units, sum) once per lane pair.
-template <typename T, int KB>
+template <int D0 = 0, int ND = 4, typename T, int KB>
 __device__ __forceinline__ void store_partial(const WaveAttn<T, KB> &w, float *o_row, float *ml_row, bool row_valid) {
   const float l_tot = pair_sum(w.l_run);
   if (!row_valid) return;
 #pragma unroll
-  for (int d = 0; d < 4; ++d)
+  for (int d = D0; d < D0 + ND; ++d)
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
       const f32x4_t v = {w.o[d][4 * i4], w.o[d][4 * i4 + 1], w.o[d][4 * i4 + 2], w.o[d][4 * i4 + 3]};
       *reinterpret_cast<f32x4_t *>(o_row + 32 * d + 8 * i4 + 4 * w.hh) = v;
     }
-  if (w.hh == 0) {
+  if (D0 == 0 && w.hh == 0) {
     ml_row[0] = w.m_run;
     ml_row[1] = l_tot;
   }
+}
+
+// One global_load_lds_dwordx4: lane l's 16 bytes at `src` land at the wave-uniform LDS address lds_addr + 16*l.
+__device__ __forceinline__ void lds_dma(const char *src, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(src), "s"(lds_addr)
+               : "m0");
 }
 
 // Global -> LDS tile loader without VGPR staging (global_load_lds_dwordx4: lane l's 16
 // bytes land at the wave-uniform LDS address in M0 + 16*l).  One wave instruction fills four
 // 256-byte rows; the XOR swizzles are realised on the global side: the lane that owns
 // physical granule pg of row r fetches the logical granule that belongs there.  A tile
-// is 16 instructions, dealt to the NW waves; `slot` s of wave w covers rows
+// of TN keys is TN/4 instructions, dealt to the NW waves; `slot` s of wave w covers rows
 // 4*(s*NW + w) .. +3.  The global address is a scalar tile base plus a per-lane 32-bit
 // offset that never changes (except in a ragged last tile, whose rows are clamped to n-1),
 // so a load costs no vector ALU work.  The loads are issued from inline asm: the compiler
 // would order every later LDS read behind a transfer it knows about (s_waitcnt vmcnt(0)).
 // Completion is waited for explicitly before the barrier that publishes a stage.
-template <int NW, bool NT> struct DirectLoader {
-  static constexpr int kSlots = 16 / NW;  // instructions per wave per tile
+template <int NW, int TN, bool NT> struct DirectLoader {
+  static constexpr int kSlots = TN / 4 / NW;  // instructions per wave per tile
   int n, row_bytes;
   uint32_t lds_row0;          // LDS byte offset of row 4*wave (wave-uniform)
   int row[kSlots];            // tile row this lane fetches in slot s
@@ -452,36 +499,34 @@ template <int NW, bool NT> struct DirectLoader {
   // t: key tile; lds_tile: LDS byte offset of the destination tile
   template <bool IS_V>
   __device__ __forceinline__ void issue(const char *base, int t, uint32_t lds_tile, int s) const {
-    const char *tile_base = base + (size_t)t * kTileN * row_bytes;
+    const char *tile_base = base + (size_t)t * TN * row_bytes;
     const uint32_t dst = lds_tile + lds_row0 + s * NW * 4 * kRowBytes;
     // rows past n-1 (ragged last tile) are clamped to row n-1: nothing beyond the caller's n
     // rows is read and the stale rows hold finite values; branch-free, two VALU instructions
-    const int r = min(row[s], n - 1 - t * kTileN);
+    const int r = min(row[s], n - 1 - t * TN);
     dma(tile_base, r * row_bytes + (IS_V ? lane_v[s] : lane_k[s]), dst);
   }
   static __device__ __forceinline__ void wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 };
 
 // ---------------------------------------------------------------------------
-// NW waves, 32*NW query rows, two LDS stages of SUB 64-key tiles, one barrier per stage.
+// NW waves, 32*NW/KP query rows, two LDS stages of SUB tiles, one barrier per stage.
 // Every wave runs S(j+1) = K Q^T, the softmax of tile j and P(j).V(j) as one instruction
 // stream (the compiler interleaves the softmax VALU work with the MFMAs); the tile loads
-// are spread over that stream.  NW = 4: two workgroups per CU (small problems); NW = 8:
-// one workgroup per CU, K/V tiles shared by 256 rows.  KB = 1: every row block worked on by two
-// waves that each take one 32-key half of every tile and are merged through LDS at the end (NW = 8:
-// 128 rows; NW = 4: 64 rows, two workgroups per CU) -- for sequences so short that there is at most
-// about one 128-row workgroup per CU, where the serial MFMA chain of a wave is what the launch
-// waits for.
+// are spread over that stream.  NW = 4, KP < 4: two workgroups per CU; else one.
+// KP = 2: two waves per row block, each on one 32-key half of every 64-key tile; KP = 4: four waves, tiles of
+// 128 keys; what they have is merged through LDS at the end.
 // ---------------------------------------------------------------------------
-template <typename T, int NW, int KB, bool NT>
+template <typename T, int NW, int KP, bool NT>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(PrefillParams p) {
   // SUB tiles of 64 keys per stage and per barrier: with one workgroup per CU (NW = 8) a stage
   // holds 128 keys, which halves the number of times the waves are forced in step.
   // LDS: K tiles of both stages [2*SUB][16 KiB], then the V tiles likewise; tile t sits in
   // slot t % (2*SUB) of each region, so every fragment address is a per-lane register plus a
   // constant below 64 KiB.
-  constexpr int BM = 16 * NW * KB, RB = BM / 32, PER = 16 / NW, SUB = NW == 8 ? 2 : 1, NSLOT = 2 * SUB;
-  constexpr int kVRegion = NSLOT * kTileBytes;
+  constexpr int KB = KP == 1 ? 2 : 1, TN = KP == 4 ? 2 * kTileN : kTileN, TB = TN * kRowBytes;
+  constexpr int RB = NW / KP, BM = 32 * RB, PER = TN / 4 / NW, SUB = (NW == 8 && KP < 4) ? 2 : 1, NSLOT = 2 * SUB;
+  constexpr int kVRegion = NSLOT * TB;
   constexpr int kWaveKeys = 32 * KB;  // keys of a tile per wave
   constexpr int kSplitKK = 3;  // k-steps of S(j+1) issued beside the row-maximum chain
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -495,41 +540,45 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   }
 #endif
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int kvh = head / p.g;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int kvh = (int)fast_div(head, p.g_div);
   // Rows of the tile.  Unpacked: rows are tokens of one head.  Packed: row index i stands for token
   // i / g of head kvh*g + i % g; `rows` counts them.  Everything below works on tokens: qtok is this
   // lane's token, tok_lo / tok_hi the first / last token of the wave's 32 rows.
   const int rows = p.pack ? p.m * p.g : p.m;
   const int row0 = tile * BM;
   const int rows_end = min(rows, row0 + BM);
-  const int rb = wave % RB, kpar = wave / RB;  // row block; which half of every tile (KB == 1)
-  const int kw0 = (KB == 1) ? 32 * kpar : 0;   // first key of the wave's part of a tile
+  const int rb = wave % RB, kpar = wave / RB;  // row block; which 32 keys of every tile (KP > 1)
+  const int kw0 = (KP > 1) ? 32 * kpar : 0;   // first key of the wave's part of a tile
   const int qblk0 = row0 + rb * 32;
   const int l32_ = lane & 31;
   const int qidx = min(qblk0 + l32_, rows - 1);
   const bool row_valid = qblk0 + l32_ < rows;
-  const int qtok = p.pack ? qidx / p.g : qidx;
-  const int qhead = p.pack ? head + qidx % p.g : head;
-  const int tok_lo = p.pack ? qblk0 / p.g : qblk0;
-  const int tok_hi = p.pack ? (min(qblk0 + 31, rows - 1)) / p.g : min(qblk0 + 31, rows - 1);
-  const int tile_tok_end = p.pack ? (rows_end - 1) / p.g + 1 : rows_end;  // one past the tile's last token
+  int qtok = qidx, qhead = head, tok_lo = qblk0, tok_hi = min(qblk0 + 31, rows - 1);
+  int tile_tok_end = rows_end;  // one past the tile's last token
+  if (p.pack) {
+    qtok = (int)fast_div(qidx, p.g_div);
+    qhead = head + qidx - qtok * p.g;
+    tok_lo = (int)fast_div(qblk0, p.g_div);
+    tok_hi = (int)fast_div(tok_hi, p.g_div);
+    tile_tok_end = (int)fast_div(rows_end - 1, p.g_div) + 1;
+  }
   // This workgroup's key range, seen as a cache of its own: rows [k_lo, k_lo + n_) with the causal
   // offset shifted accordingly (negative when the range starts past a row's last visible key).
   const int k_lo = split * p.chunk;
   const int n_ = min(p.n - k_lo, p.chunk);
   const int offset_ = p.offset - k_lo;
   const int n_vis = min(n_, tile_tok_end + offset_);  // keys any row of this tile can see
-  const int J = (n_vis + kTileN - 1) / kTileN;        // 64-key tiles of the workgroup
+  const int J = (n_vis + TN - 1) / TN;        // tiles of the workgroup
   const size_t q_row_bytes = (size_t)p.H * kRowBytes;
   const int kv_row_bytes = p.Hkv * kRowBytes;
   const char *kbase = p.k + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
   const char *vbase = p.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
 
   WaveAttn<T, KB> w;
-  w.init(lane, kVRegion, (KB == 1) ? kpar : 0);
+  w.init(lane, kVRegion, (KP > 1) ? kpar : 0);
   // tiles in which this wave's keys hold at least one visible key
-  const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + kTileN - 1) / kTileN)) : 0;
+  const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) / TN)) : 0;
   float *part_o = nullptr, *part_ml = nullptr;
   if (p.num_splits > 1) {
     const size_t slot = ((size_t)split * p.m + qtok) * p.H + qhead;
@@ -540,9 +589,29 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       return;
     }
   }
-  w.load_q(p.q + (size_t)qtok * q_row_bytes + (size_t)qhead * kRowBytes);
+  // Q.  A fragment load straight into the operand layout touches 32 rows with 32 bytes each, 256 tag look-ups per
+  // wave; where KP waves share the rows, Q goes through LDS like a K tile instead, fetched once as whole
+  // rows (256 tokens, 32 heads, two waves per 64 rows: 7.4 -> 7.0 us).
+  constexpr int kQRegion = 2 * NSLOT * TB;  // behind the K and V tiles
+  if constexpr (KP > 1) {
+#pragma unroll
+    for (int sl = 0; sl < 8 / KP; ++sl) {
+      const int r = 4 * (sl * NW + wave) + (lane >> 4);
+      const int idx = min(row0 + r, rows - 1);
+      const char *src = p.q + ((lane & 15) ^ (r & 15)) * 16;
+      if (p.pack) {
+        const int tok = (int)fast_div(idx, p.g_div);
+        src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * p.g) * kRowBytes;
+      } else {
+        src += (size_t)idx * q_row_bytes + (size_t)head * kRowBytes;
+      }
+      lds_dma(src, kQRegion + (sl * NW + wave) * 4 * kRowBytes);
+    }
+  } else {
+    w.load_q(p.q + (size_t)qtok * q_row_bytes + (size_t)qhead * kRowBytes);
+  }
 
-  DirectLoader<NW, NT> ld;
+  DirectLoader<NW, TN, NT> ld;
   ld.init(wave, lane, kv_row_bytes, n_);
   // K runs one tile ahead of V: S(j+1) = K(j+1) Q^T is issued together with the softmax of
   // tile j, so K tile t is fetched SUB+1 iterations and V tile t SUB iterations before use.
@@ -550,21 +619,25 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   for (int u = 0; u <= SUB; ++u)
 #pragma unroll
     for (int sl = 0; sl < PER; ++sl) {
-      ld.template issue<false>(kbase, min(u, J - 1), (u % NSLOT) * kTileBytes, sl);
-      if (u < SUB) ld.template issue<true>(vbase, min(u, J - 1), kVRegion + u * kTileBytes, sl);
+      ld.template issue<false>(kbase, min(u, J - 1), (u % NSLOT) * TB, sl);
+      if (u < SUB) ld.template issue<true>(vbase, min(u, J - 1), kVRegion + u * TB, sl);
     }
-  w.pin_q();  // the Q fragments are in registers from here on
+  if (KP == 1) w.pin_q();  // the Q fragments are in registers from here on
   ld.wait_all();
   lds_barrier();
+  if (KP > 1) w.load_q_lds(lds, kQRegion + (rb - kpar) * 32 * kRowBytes);
 
   f32x16_t sa[KB], sb[KB];  // scores of the current / the next tile, roles alternate
   if (Jw > 0) w.qk(lds, 0, sa);
+  // A K load of the first stage lands where tile 0 was just read: no wave may issue it (one without rows would at
+  // once) before all have read.
+  lds_barrier();
 
   auto tile_step = [&](int j, int slot, f32x16_t (&s_cur)[KB], f32x16_t (&s_nxt)[KB]) {
     const int kslot = (slot + SUB + 1) % NSLOT, vslot = (slot + SUB) % NSLOT;  // fetched now
     const int jk = min(j + SUB + 1, J - 1), jv = min(j + SUB, J - 1);
     if (j < Jw) {
-      const int key0 = j * kTileN + kw0;
+      const int key0 = j * TN + kw0;
       if ((key0 + kWaveKeys - 1 > tok_lo + offset_) || (key0 + kWaveKeys > n_))
         w.mask(s_cur, key0, qtok, offset_, n_);
       // In the 8-wave kernel a burst of loads would stall every wave behind the texture addresser's
@@ -577,10 +650,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
 #pragma unroll
         for (int r = 0; r < PER; ++r) {
           if (KB == 1) {
-            if (i == r) ld.template issue<false>(kbase, jk, kslot * kTileBytes, r);
-            if (i == PER + r) ld.template issue<true>(vbase, jv, kVRegion + vslot * kTileBytes, r);
+            if (i == r) ld.template issue<false>(kbase, jk, kslot * TB, r);
+            if (PER < 8 && i == PER + r) ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, r);
           } else if (i == (NW == 4 ? r : (8 * KB / PER) * r + 1)) {
-            ld.template issue<false>(kbase, jk, kslot * kTileBytes, r);
+            ld.template issue<false>(kbase, jk, kslot * TB, r);
           }
         }
       };
@@ -588,22 +661,22 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       // maximum chain, the rest -- and the MFMAs of P.V -- beside the exponentials.  (For the
       // wave's last tile the result is not used: one surplus pass instead of a branch that
       // would separate these MFMAs from the instructions they overlap with.)
-      const int koff = ((slot + 1) % NSLOT) * kTileBytes;
+      const int koff = ((slot + 1) % NSLOT) * TB;
       w.template qk<0, kSplitKK>(lds, koff, s_nxt, k_hook);
       const float neg_ms = w.row_max(s_cur, p.scale_log2e);
       w.template qk<kSplitKK, 8>(lds, koff, s_nxt, k_hook);
       w.l_run += w.probabilities(s_cur, p.scale_log2e, neg_ms);
-      w.pv(lds, slot * kTileBytes, [&](int i) {
+      w.pv(lds, slot * TB, [&](int i) {
 #pragma unroll
         for (int r = 0; r < PER; ++r)
-          if (KB != 1 && i == (NW == 4 ? r : (8 * KB / PER) * r + 1))
-            ld.template issue<true>(vbase, jv, kVRegion + vslot * kTileBytes, r);
+          if (KB == 1 ? (PER == 8 && i == r) : i == (NW == 4 ? r : (8 * KB / PER) * r + 1))
+            ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, r);
       });
     } else {
 #pragma unroll
       for (int sl = 0; sl < PER; ++sl) {
-        ld.template issue<false>(kbase, jk, kslot * kTileBytes, sl);
-        ld.template issue<true>(vbase, jv, kVRegion + vslot * kTileBytes, sl);
+        ld.template issue<false>(kbase, jk, kslot * TB, sl);
+        ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, sl);
       }
     }
   };
@@ -625,20 +698,31 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     }
   }
   // every wave is past the last barrier of the loop: nobody reads the K/V tiles any more
-  if (KB == 1) {
-    // the two waves of a row block: the second hands its state over (behind the RB output
-    // staging regions of 8 KiB), the first folds it in and stores
-    float *pair = reinterpret_cast<float *>(lds + RB * 32 * kRowBytes) + (size_t)rb * 66 * 64;
-    if (kpar == 1) w.export_state(pair);
+  char *out_blk = p.out + (size_t)qblk0 * q_row_bytes + (size_t)head * kRowBytes;
+  if constexpr (KP > 1) {
+    constexpr int kTrade = WaveAttn<T, KB>::trade_bytes(KP), ND = 4 / KP;
+    char *rows_lds = lds + rb * kTrade;
+    w.template give<KP>(rows_lds, kpar);
     __syncthreads();
-    if (kpar == 1) return;
-    w.import_state(pair, p.scale_log2e);
-  }
-  if (p.num_splits > 1)  // (packed rows exist in split mode only)
+    auto finish = [&](auto part) {
+      constexpr int PART = decltype(part)::value;
+      w.template take<KP, PART>(rows_lds, p.scale_log2e);
+      if (p.num_splits > 1)
+        store_partial<PART * ND, ND>(w, part_o, part_ml, row_valid);
+      else
+        w.template store<PART * ND, ND>(lds + RB * kTrade + wave * (32 * 64 * ND), out_blk, q_row_bytes, p.m - qblk0);
+    };
+    if (kpar == 0) finish(std::integral_constant<int, 0>());
+    if (kpar == 1) finish(std::integral_constant<int, 1>());
+    if constexpr (KP == 4) {
+      if (kpar == 2) finish(std::integral_constant<int, 2>());
+      if (kpar == 3) finish(std::integral_constant<int, 3>());
+    }
+  } else if (p.num_splits > 1) {  // (packed rows exist in split mode only)
     store_partial(w, part_o, part_ml, row_valid);
-  else
-    w.store(lds + rb * 32 * kRowBytes, p.out + (size_t)qblk0 * q_row_bytes + (size_t)head * kRowBytes,
-            q_row_bytes, p.m - qblk0);
+  } else {
+    w.store(lds + rb * 32 * kRowBytes, out_blk, q_row_bytes, p.m - qblk0);
+  }
 #ifdef LLMHIP_BENCH
   if (p.clock_probe && blockIdx.x == 0 && tid == 0) {
     p.clock_probe[0] = __builtin_amdgcn_s_memtime() - clk0;
@@ -768,39 +852,45 @@ __global__ __launch_bounds__(256) void prefill_combine_wide_kernel(PrefillParams
   *reinterpret_cast<u32x2_t *>(p.out + slot * kRowBytes + d4 * 8) = w;
 }
 
-template <typename T, int NW, int KB = 2>
+template <typename T, int NW, int KP = 1>
 static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) {
   PrefillParams p = p0;
-  constexpr int BM = 16 * NW * KB;
+  constexpr int BM = 32 * NW / KP;
   constexpr int NT = 64 * NW;
   p.num_q_tiles = (p.m + BM - 1) / BM;
   if (p.pack) p.num_q_tiles = (p.m * p.g + BM - 1) / BM;
   const int T_ = p.num_q_tiles;
-  int grid;
+  int grid, list_heads;
   const int S_ = p.num_splits;
+  p.sched_a = p.sched_shift = 0;
   if (p.pack) {
     p.sched_mode = 0;
-    p.sched_a = 0;
+    list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
   } else if (p.Hkv <= 8 && 8 % p.Hkv == 0) {
     p.sched_mode = 1;
     p.sched_a = 8 / p.Hkv;
+    while ((1 << p.sched_shift) < p.sched_a) ++p.sched_shift;
+    list_heads = p.g;
     const int per_kvh = p.g * T_ * S_;
     grid = 8 * ((per_kvh + p.sched_a - 1) / p.sched_a);
   } else if (p.Hkv % 8 == 0) {
     p.sched_mode = 2;
-    p.sched_a = (p.Hkv / 8) * p.g;
-    grid = 8 * p.sched_a * T_ * S_;
+    list_heads = (p.Hkv / 8) * p.g;
+    grid = 8 * list_heads * T_ * S_;
   } else {
     p.sched_mode = 0;
-    p.sched_a = 0;
+    list_heads = p.H;
     grid = T_ * p.H * S_;
   }
-  const size_t lds_bytes = (NW == 8 ? 2 : 1) * 4 * kTileBytes;
-  // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KB == 2 there)
-  const bool nt = KB == 2 && p.pack && T_ == 1;
-  void (*kern)(PrefillParams) = flash_prefill_kernel<T, NW, KB, false>;
-  if (nt) kern = flash_prefill_kernel<T, NW, KB, (KB == 2)>;
+  p.list_heads = make_fast_div((uint32_t)list_heads);
+  p.per_split = make_fast_div((uint32_t)(list_heads * T_));
+  p.g_div = make_fast_div((uint32_t)p.g);
+  const size_t lds_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes + (KP > 1 ? (size_t)BM * kRowBytes : 0);  // tiles, Q
+  // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KP == 1 there)
+  const bool nt = KP == 1 && p.pack && T_ == 1;
+  void (*kern)(PrefillParams) = flash_prefill_kernel<T, NW, KP, false>;
+  if (nt) kern = flash_prefill_kernel<T, NW, KP, (KP == 1)>;
   // the opt-in for more than 64 KiB of dynamic LDS is per device: once per device and kernel
   static std::atomic<uint64_t> attr_done_both[2];
   std::atomic<uint64_t> &attr_done = attr_done_both[nt ? 1 : 0];
@@ -840,69 +930,117 @@ int device_compute_units() {
   return cus;
 }
 
-// Kernel and key-range split for one call.
-// 256-row workgroups (one per CU) or 128-row ones (two per CU)?  The 256-row kernel has the
-// cheaper step (K/V tiles shared by twice the rows) but coarser work items: with fewer than
-// about one and a half of them per CU the heavy-first list packs badly (the second round is
-// mostly idle) and the 128-row kernel wins.  Measured at H=28, bf16, 256 CUs (128-row / 256-row,
-// us): S=2560 64/73, S=3072 82/88, S=3584 111/107, S=4096 139/131, S=5120 201/194, S=8192 452/438.
-// Key-range split: a chunk of few query rows over a long cache (keys >= 8 x rows) makes too few
-// workgroups to fill the chip; its key range is cut so that about one (256-row kernel) or two
-// (128-row kernel) workgroups per CU exist, each with at least 1024 keys.  Square causal prefill is
-// never split: the fp32 partials would cost more HBM traffic than K and V themselves.
+// ---------------------------------------------------------------------------
+// Kernel and key-range split of a call.
+// ---------------------------------------------------------------------------
+// The workgroup shapes, and what a launch of one costs on this part, in us: `fixed` per workgroup, a step over one
+// tile `step_free` on an otherwise empty chip and `step_full` with every CU busy (fitted over 13000 timed
+// launches: 204 shapes of 2-32 kv heads, 3-8192 tokens, 0-31000 cached keys, every shape and split).
+enum PrefillKind { kPair64, kPair128, kRows128, kRows256, kQuad64, kQuad32, kPrefillKinds };
+struct PrefillShape {
+  int rows, tile, per_cu;  // query rows, keys of a tile, workgroups resident on a CU
+  double fixed, step_free, step_full;
+};
+static const PrefillShape kShapes[kPrefillKinds] = {
+    {64, 64, 2, 2.42, 0.74, 1.05},   // 4 waves, two per row block
+    {128, 64, 1, 3.92, 0.73, 0.85},  // 8 waves, two per row block
+    {128, 64, 2, 2.40, 1.10, 1.55},  // 4 waves
+    {256, 64, 1, 3.61, 1.12, 1.44},  // 8 waves
+    {64, 128, 1, 3.42, 1.03, 1.20},  // 8 waves, four per row block
+    {32, 128, 1, 2.99, 0.81, 1.03},  // 4 waves, four per row block
+};
 struct PrefillPlan {
-  bool rows256, pack;
-  bool pair;  // two waves per row block, each on one 32-key half of every tile (short sequences)
-  bool rows64;  // with pair: 64-row workgroups of 4 waves, two per CU, instead of 128 rows and 8 waves
+  PrefillKind kind;
+  bool pack;
   int num_splits, chunk;
 };
+constexpr int kWholeRange = 0x7fffffc0;
+
+// A prompt (no more cached than new tokens) is never split: the fp32 partials would cost more HBM traffic than K and
+// V.  Which shape: while the chip is not full, the launch waits for the chain of the waves with the most
+// keys, so that as many waves as fit share every row block; once it is, the cheapest step wins.  Lines where the
+// measured times cross (H=32 / 28 / 12, bf16, 256 CUs, us, best / runner-up):
+//   four waves per 32 rows while one such workgroup per CU is enough, from about 100 keys: 256 tokens 6.7 / 7.0
+//   four waves per 64 rows likewise, from about 480 keys: 512 tokens 9.2 / 9.8 (28 heads); with twice as many
+//     workgroups as CUs from 1500 keys on: 2048 tokens 24.6 / 28.8 (12 heads)
+//   two waves per 64 rows up to 1.3 128-row workgroups per CU: 1019 tokens 17.8 / 19.2 (28), 1400 25.6 / 25.8
+//   two waves per 128 rows up to 2 per CU: 1700 tokens 34.0 / 35.3 (28)
+//   256 rows from 1.5 workgroups per CU: 3500 tokens 107.8 / 111 (28); 128 rows of one wave each below: 3000 tokens
+//     81.7 / 85.8
+static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
+  auto per_cu = [&](int rows) { return (double)((m + rows - 1) / rows) * H / cus; };
+  if (n_vis > 96 && per_cu(32) <= 1.05) return kQuad32;
+  if ((n_vis >= 480 && per_cu(64) <= 1.05) || (n_vis >= 1500 && per_cu(64) <= 2.0)) return kQuad64;
+  if (per_cu(128) <= 1.3) return kPair64;
+  if (per_cu(128) <= 2.0) return kPair128;
+  return per_cu(256) >= 1.5 ? kRows256 : kRows128;
+}
+
+// A chunk behind a longer cache makes few workgroups with many keys each: its key range is cut, and with fewer rows than a
+// tile has the g query heads of a kv head share a tile (K and V of the kv head are then read once, not g times).
+// Taken is the combination of shape, packing and cut that the costs above make cheapest: workgroups in rounds of as
+// many as are resident at once, 3 us and the traffic of the partials for the combine launch, K and V at 5.7 TB/s as
+// the floor.  Over the measured shapes that is the fastest combination or within 11 % of it (1 % on
+// average).  Among combinations within 4 % of the cheapest one that reads K and V once and gives every CU the same
+// number of workgroups is preferred.  Some of what it changed (us, before / now): 3 tokens over 3000 keys 29.3 / 10.3, 20 over 600 11.5 / 8.7,
+// 130 over 2000 27.9 / 18.2, 200 over 16001 63.0 / 60.4 (28 heads); 300 over 30000, 40 heads, 232 / 199.
+static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int Hkv, int cus) {
+  PrefillPlan best = {kPair64, false, 1, kWholeRange};
+  double best_us = 1e30;
+  const double floor_us = 2.0 * n_vis * Hkv * kRowBytes / 5.7e6 + 1.8;
+  for (int kind = 0; kind < kPrefillKinds; ++kind)
+    for (int pack = 0; pack < (g > 1 ? 2 : 1); ++pack) {
+      const PrefillShape &sh = kShapes[kind];
+      const long long rows = pack ? (long long)m * g : m, tiles = (rows + sh.rows - 1) / sh.rows;
+      const long long groups = pack ? Hkv : (long long)Hkv * g;
+      const double last_rows = ((double)sh.rows * (tiles - 1) * tiles / 2 + rows) / tiles / (pack ? g : 1);
+      const double keys = past + last_rows;  // that a tile's last row sees, on average
+      for (int s = pack ? 2 : 1; s <= kMaxPrefillSplits; s += s < 16 ? 1 : s < 32 ? 2 : s < 64 ? 4 : 16) {
+        if (s > 1 && n_vis / s < 128) break;
+        const long long chunk = s > 1 ? ((n_vis + s - 1) / s + 127) / 128 * 128 : n_vis;
+        const long long splits = (n_vis + chunk - 1) / chunk;  // no empty trailing range
+        const long long items = tiles * groups * splits, slots = (long long)cus * sh.per_cu;
+        double busy = (double)items / cus;
+        busy = sh.per_cu == 2 ? busy - 1 : busy * busy;
+        busy = busy < 0 ? 0 : busy > 1 ? 1 : busy;
+        const double step = sh.step_free + (sh.step_full - sh.step_free) * busy;
+        const double most = (double)((chunk + sh.tile - 1) / sh.tile);
+        double mean = keys / (splits * sh.tile) + 0.5;
+        if (mean > most) mean = most;
+        double us = sh.fixed + step * most;
+        if (items > slots) {
+          const double rounds = 0.63 * ((items + slots - 1) / slots) + 0.37 * ((double)items / slots);
+          const double all = (sh.fixed + step * mean) * rounds;
+          if (all > us) us = all;
+        }
+        us += 1.8;
+        if (splits > 1) us += 3.0 + (double)splits * m * g * Hkv * (kHeadDim + 2) * sizeof(float) / 1.9e6;
+        if (us < floor_us + sh.fixed) us = floor_us + sh.fixed;
+        if (tiles == 1 && items % cus == 0) us *= 0.96;
+        if (us < best_us) {
+          best_us = us;
+          best = {(PrefillKind)kind, pack != 0, (int)splits, splits > 1 ? (int)chunk : kWholeRange};
+        }
+      }
+    }
+  return best;
+}
+
+// The last answers are kept per thread: every layer of a model asks for the same chunk (several hundred combinations).
 static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cus) {
-  PrefillPlan pl;
-  const int H = g * Hkv;
-  const long long wg256 = (long long)((m + 255) / 256) * H;
-  pl.rows256 = 2 * wg256 >= 3LL * cus;
-  pl.pack = false;
-  // up to two 128-row workgroups per CU: the launch waits for the serial chain of the waves with
-  // the most keys, so two waves share every row block (measured at H=28, bf16, 256 CUs, 4-wave /
-  // paired 8-wave workgroups, us: S=1024 22.6/20.2, S=1536 32.8/27.9, S=2048 45.6/42.1,
-  // S=2560 60.8/64.6, S=3072 76.3/86.0)
-  const long long wg128 = (long long)((m + 127) / 128) * H;
-  pl.pair = !pl.rows256 && wg128 <= 2LL * cus;
-  // Up to about 1.2 such workgroups per CU, halves of them (64 rows, 4 waves, two resident per CU) finish
-  // sooner: the heavy tiles meet less competition for their SIMDs (128-row / 64-row, us: S=256
-  // 10.5/8.6, S=512 13.6/11.5, S=1024 20.2/17.8, S=1280 25.4/23.9, S=1408 27.9/27.5, S=1536 28.0/29.4)
-  pl.rows64 = pl.pair && 5 * wg128 <= 6LL * cus;
-  pl.num_splits = 1;
-  pl.chunk = 0x7fffffc0;
   const long long n_vis = ((long long)m + offset < n) ? (long long)m + offset : n;  // keys the last row sees
-  if (n_vis < 256) pl.pair = pl.rows64 = false;
-  if (pl.rows256 || n_vis < 8LL * m || n_vis < 2048) return pl;
-  pl.pair = pl.rows64 = false;
-  // Split mode.  A chunk shorter than a 128-row tile packs the g query heads of a kv head into the
-  // rows of one tile (K and V of the kv head are then read once, not g times).
-  pl.pack = g > 1 && m < 128;
-  const long long rows = pl.pack ? (long long)m * g : m;  // rows per head (per kv head when packed)
-  const long long groups = pl.pack ? Hkv : H;
-  pl.rows256 = rows >= 192;  // enough rows to use most of a 256-row workgroup
-  const long long wgs = (pl.rows256 ? (rows + 255) / 256 : (rows + 127) / 128) * groups;
-  const long long want_wgs = pl.rows256 ? cus : 2LL * cus;  // one round of workgroups, not one and a bit
-  long long splits = want_wgs / wgs;
-  if (splits > n_vis / 1024) splits = n_vis / 1024;
-  // at most 64 key ranges, 128 where one or two workgroups per range would otherwise leave half the chip
-  // idle (two kv heads, 131072 keys, 16 tokens: 48.6 -> 37.5 us; with four kv heads 128 ranges are slower)
-  const long long max_splits = wgs <= 2 ? kMaxPrefillSplits : kMaxPrefillSplits / 2;
-  if (splits > max_splits) splits = max_splits;
-  if (splits <= 1) {
-    pl.pack = false;
-    pl.rows256 = false;
-    pl.pair = wg128 <= 2LL * cus;
-    pl.rows64 = 5 * wg128 <= 6LL * cus;
-    return pl;
-  }
-  long long chunk = (n_vis + splits - 1) / splits;
-  chunk = (chunk + 127) / 128 * 128;
-  pl.chunk = (int)chunk;
-  pl.num_splits = (int)((n_vis + chunk - 1) / chunk);  // no empty trailing range
+  if (n_vis < 2LL * m) return {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
+  struct Memo {
+    int m, n, offset, g, Hkv, cus;
+    PrefillPlan plan;
+  };
+  constexpr int kMemo = 8;
+  static thread_local Memo memo[kMemo] = {};
+  static thread_local unsigned next = 0;
+  for (const Memo &e : memo)
+    if (e.m == m && e.n == n && e.offset == offset && e.g == g && e.Hkv == Hkv && e.cus == cus) return e.plan;
+  const PrefillPlan pl = chunk_plan(m, n_vis, n_vis - m, g, Hkv, cus);
+  memo[next++ % kMemo] = Memo{m, n, offset, g, Hkv, cus, pl};
   return pl;
 }
 
@@ -911,6 +1049,17 @@ size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, i
   const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units());
   if (pl.num_splits <= 1) return 0;
   return (size_t)pl.num_splits * m * H * (kHeadDim + 2) * sizeof(float);
+}
+
+template <typename T> static hipError_t launch_prefill(const PrefillParams &p, PrefillKind kind, hipStream_t stream) {
+  switch (kind) {
+    case kPair64: return launch_prefill_t<T, 4, 2>(p, stream);
+    case kPair128: return launch_prefill_t<T, 8, 2>(p, stream);
+    case kRows128: return launch_prefill_t<T, 4, 1>(p, stream);
+    case kRows256: return launch_prefill_t<T, 8, 1>(p, stream);
+    case kQuad64: return launch_prefill_t<T, 8, 4>(p, stream);
+    default: return launch_prefill_t<T, 4, 4>(p, stream);
+  }
 }
 
 #ifdef LLMHIP_BENCH
@@ -937,24 +1086,14 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   p.H = group_size * kv_head_num;
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units());
-  if (pl.num_splits > 1 && !workspace) {  // no scratch offered: run unsplit (and unpacked)
-    pl.num_splits = 1;
-    pl.chunk = 0x7fffffc0;
-    pl.pack = false;
-    pl.rows256 = false;
-    pl.rows64 = false;
-  }
+  if (pl.num_splits > 1 && !workspace)  // no scratch offered: run unsplit (and unpacked)
+    pl = {prompt_kind(m, n, p.H, device_compute_units()), false, 1, kWholeRange};
   p.pack = pl.pack ? 1 : 0;
   p.num_splits = pl.num_splits;
   p.chunk = pl.chunk;
   p.ws_o = static_cast<float *>(workspace);
   p.ws_ml = p.ws_o ? p.ws_o + (size_t)pl.num_splits * m * p.H * kHeadDim : nullptr;
-  const bool f16 = dt == kDtFloat16;
-  if (pl.rows256) return f16 ? launch_prefill_t<_Float16, 8>(p, stream) : launch_prefill_t<__bf16, 8>(p, stream);
-  if (pl.pair && pl.rows64)
-    return f16 ? launch_prefill_t<_Float16, 4, 1>(p, stream) : launch_prefill_t<__bf16, 4, 1>(p, stream);
-  if (pl.pair) return f16 ? launch_prefill_t<_Float16, 8, 1>(p, stream) : launch_prefill_t<__bf16, 8, 1>(p, stream);
-  return f16 ? launch_prefill_t<_Float16, 4>(p, stream) : launch_prefill_t<__bf16, 4>(p, stream);
+  return dt == kDtFloat16 ? launch_prefill<_Float16>(p, pl.kind, stream) : launch_prefill<__bf16>(p, pl.kind, stream);
 }
 
 }  // namespace LLMHIP_NS
