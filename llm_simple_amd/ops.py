@@ -1,4 +1,4 @@
-"""ctypes binding of libllmhip.so.
+"""Binding of libllmhip.so: the operators through the extension module ``_operators``, the rest through ctypes.
 
 Function names and argument order follow the reference's operator header
 (prebuild/npu_ops.h:6-18, :39-47) with the ``npu_`` prefix replaced by
@@ -92,67 +92,33 @@ def _check(status, where):
 
 def _ptr(x):
     """Device address of a torch tensor, or an int address passed through."""
-    if x is None:
-        return None
-    if isinstance(x, int):
+    if x is None or isinstance(x, int):
         return x
     return x.data_ptr()
 
 
-def hip_flash_attn_layer(output_dev, q_dev, k_dev, v_dev, m, n, offset, head_num, head_dim, dt,
-                         stream=0):
-    """npu_flash_attn_layer (prebuild/npu_ops.h:6-8)."""
-    _check(lib.llmhip_flash_attn(_ptr(output_dev), _ptr(q_dev), _ptr(k_dev), _ptr(v_dev), m, n,
-                                 offset, head_num, head_dim, dt, stream), "hip_flash_attn_layer")
-
-
-def hip_flash_attn_gqa_layer(output_dev, q_dev, k_dev, v_dev, m, n, offset, group_size,
-                             kv_head_num, head_dim, dt, stream=0):
-    """npu_flash_attn_gqa_layer (prebuild/npu_ops.h:10-13)."""
-    _check(lib.llmhip_flash_attn_gqa(_ptr(output_dev), _ptr(q_dev), _ptr(k_dev), _ptr(v_dev), m,
-                                     n, offset, group_size, kv_head_num, head_dim, dt, stream),
-           "hip_flash_attn_gqa_layer")
-
-
-def hip_flash_attn_opt_prefill_layer(output_dev, q_dev, k_dev, v_dev, m, n, offset, head_num,
-                                     head_dim, dt, stream=0):
-    """npu_flash_attn_opt_prefill_layer (prebuild/npu_ops.h:15-18)."""
-    _check(lib.llmhip_flash_attn_opt_prefill(_ptr(output_dev), _ptr(q_dev), _ptr(k_dev),
-                                             _ptr(v_dev), m, n, offset, head_num, head_dim, dt,
-                                             stream), "hip_flash_attn_opt_prefill_layer")
-
-
-def hip_flash_decode_gqa_layer(output_dev, q_dev, k_cache_dev, v_cache_dev, workspace_dev,
-                               workspace_bytes, batch, n, kv_seq_stride, group_size, kv_head_num,
-                               head_dim, num_splits, dt, stream=0):
-    """Batched split-KV decode (no counterpart in the reference header: decode there
-    is npu_flash_attn_gqa_layer with m = 1, src/llama2_layer_npu.cpp:866-869)."""
-    _check(lib.llmhip_flash_decode_gqa(_ptr(output_dev), _ptr(q_dev), _ptr(k_cache_dev),
-                                       _ptr(v_cache_dev), _ptr(workspace_dev), workspace_bytes,
-                                       batch, n, kv_seq_stride, group_size, kv_head_num, head_dim,
-                                       num_splits, dt, stream), "hip_flash_decode_gqa_layer")
-
-
-def hip_flash_decode_gqa_static_layer(output_dev, q_dev, k_cache_dev, v_cache_dev, batch, n,
-                                      kv_seq_stride, group_size, kv_head_num, head_dim, num_splits, dt,
-                                      stream=0):
-    """hip_flash_decode_gqa_layer without a workspace: the partials live in a fixed 4 MiB array
-    inside the library and the call allocates nothing."""
-    _check(lib.llmhip_flash_decode_gqa_static(_ptr(output_dev), _ptr(q_dev), _ptr(k_cache_dev),
-                                              _ptr(v_cache_dev), batch, n, kv_seq_stride, group_size,
-                                              kv_head_num, head_dim, num_splits, dt, stream),
-           "hip_flash_decode_gqa_static_layer")
-
-
-def hip_decode_step_gqa_layer(output_dev, k_cache_dev, v_cache_dev, freqs_cis_dev, input_q_dev, input_k_dev,
-                              input_v_dev, pos, group_size, kv_head_num, head_dim, is_neox_style, dt, stream=0):
-    """One decode step in one pass over the cache: rope(q), rope(k) -> k_cache[pos], v -> v_cache[pos] and
-    attention over rows [0, pos], fused into the decode kernel (src/llama2_layer_npu.cpp:790-869 does it
-    with four calls)."""
-    _check(lib.llmhip_decode_step_gqa(_ptr(output_dev), _ptr(k_cache_dev), _ptr(v_cache_dev),
-                                      _ptr(freqs_cis_dev), _ptr(input_q_dev), _ptr(input_k_dev),
-                                      _ptr(input_v_dev), pos, group_size, kv_head_num, head_dim,
-                                      int(bool(is_neox_style)), dt, stream), "hip_decode_step_gqa_layer")
+try:
+    from . import _operators
+except ImportError as e:
+    raise ImportError(
+        f"{os.path.join(_HERE, '_operators.so')} is missing or was built for another Python: build it with "
+        "`make -C llm_simple_amd/csrc` (or __graft_entry__.build())") from e
+_operators.set_error(LlmHipError)
+# csrc/py_ops.cpp: argument names, order and documentation of each
+from ._operators import (  # noqa: E402
+    hip_add_layer,
+    hip_decode_step_gqa_layer,
+    hip_flash_attn_gqa_layer,
+    hip_flash_attn_layer,
+    hip_flash_attn_opt_prefill_layer,
+    hip_flash_decode_gqa_layer,
+    hip_flash_decode_gqa_static_layer,
+    hip_matmul_bias_layer,
+    hip_matmul_layer,
+    hip_rope_kv_append_layer,
+    hip_rope_layer,
+    hip_rope_single_layer,
+)
 
 
 def flash_decode_workspace_bytes(batch, group_size, kv_head_num, head_dim, num_splits):
@@ -162,52 +128,6 @@ def flash_decode_workspace_bytes(batch, group_size, kv_head_num, head_dim, num_s
 
 def flash_decode_default_splits(batch, n, kv_head_num):
     return lib.llmhip_flash_decode_default_splits(batch, n, kv_head_num)
-
-
-def hip_matmul_layer(output_dev, lhs_dev, weight_dev, m, n, k, dt, stream=0):
-    """npu_matmul_nz_layer (prebuild/npu_ops.h:87-88) with the weight as W[n][k] row-major."""
-    _check(lib.llmhip_matmul(_ptr(output_dev), _ptr(lhs_dev), _ptr(weight_dev), m, n, k, dt, stream),
-           "hip_matmul_layer")
-
-
-def hip_matmul_bias_layer(output_dev, lhs_dev, weight_dev, bias_dev, m, n, k, dt, stream=0):
-    """npu_matmul_bias_nz_layer (prebuild/npu_ops.h:90-92): fp32 bias added before the rounding."""
-    _check(lib.llmhip_matmul_bias(_ptr(output_dev), _ptr(lhs_dev), _ptr(weight_dev), _ptr(bias_dev),
-                                  m, n, k, dt, stream), "hip_matmul_bias_layer")
-
-
-def hip_add_layer(output_dev, lhs_dev, rhs_dev, total_size, dt, stream=0):
-    """npu_add_layer (prebuild/npu_ops.h:81-82)."""
-    _check(lib.llmhip_add(_ptr(output_dev), _ptr(lhs_dev), _ptr(rhs_dev), total_size, dt, stream),
-           "hip_add_layer")
-
-
-def hip_rope_layer(output_q_dev, output_k_dev, freqs_cis_dev, input_q_dev, input_k_dev, start_pos,
-                   cur_size, n_heads, hidden_dim, is_neox_style, dt, stream=0):
-    """npu_rope_layer (prebuild/npu_ops.h:39-42)."""
-    _check(lib.llmhip_rope(_ptr(output_q_dev), _ptr(output_k_dev), _ptr(freqs_cis_dev),
-                           _ptr(input_q_dev), _ptr(input_k_dev), start_pos, cur_size, n_heads,
-                           hidden_dim, int(bool(is_neox_style)), dt, stream), "hip_rope_layer")
-
-
-def hip_rope_single_layer(output_x_dev, freqs_cis_dev, input_x_dev, start_pos, cur_size, n_heads,
-                          hidden_dim, is_neox_style, dt, stream=0):
-    """npu_rope_single_layer (prebuild/npu_ops.h:44-47)."""
-    _check(lib.llmhip_rope_single(_ptr(output_x_dev), _ptr(freqs_cis_dev), _ptr(input_x_dev),
-                                  start_pos, cur_size, n_heads, hidden_dim,
-                                  int(bool(is_neox_style)), dt, stream), "hip_rope_single_layer")
-
-
-def hip_rope_kv_append_layer(output_q_dev, k_cache_dev, v_cache_dev, freqs_cis_dev, input_q_dev,
-                             input_k_dev, input_v_dev, start_pos, cur_size, n_heads, n_kv_heads,
-                             head_dim, is_neox_style, dt, stream=0):
-    """rope(Q), rope(K) -> k_cache[start_pos:], V -> v_cache[start_pos:] in one launch
-    (src/llama2_layer_npu.cpp:790-798 + :830-844)."""
-    _check(lib.llmhip_rope_kv_append(_ptr(output_q_dev), _ptr(k_cache_dev), _ptr(v_cache_dev),
-                                     _ptr(freqs_cis_dev), _ptr(input_q_dev), _ptr(input_k_dev),
-                                     _ptr(input_v_dev), start_pos, cur_size, n_heads, n_kv_heads,
-                                     head_dim, int(bool(is_neox_style)), dt, stream),
-           "hip_rope_kv_append_layer")
 
 
 def device_props(device=0):
