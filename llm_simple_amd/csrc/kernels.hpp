@@ -62,10 +62,14 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
                                  int k_out_row_offset, int is_neox, int dt, hipStream_t stream);
 
 // Projection out[m][n] = round(lhs[m][k] . weight[n][k]^T + bias), bias fp32 [n] or null; n and k multiples
-// of 16.  matmul_skinny: m <= 16, pointers 16-byte aligned.  matmul_bias: hipBLASLt, whose handle and 64 MiB
+// of 16.  matmul_skinny: m <= 16, pointers 16-byte aligned.  matmul_tile: the sizes that matmul_tile_takes
+// accepts, pointers 16-byte aligned.  matmul_bias: hipBLASLt, whose handle and 64 MiB
 // workspace the first call creates.
 hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, const float *bias,
                                 int m, int n, int k, int dt, hipStream_t stream);
+bool matmul_tile_takes(int m, int n, int k);
+hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias,
+                              int m, int n, int k, int dt, hipStream_t stream);
 hipError_t launch_matmul_bias(void *out, const void *lhs, const void *weight, const float *bias,
                               int m, int n, int k, int dt, hipStream_t stream);
 void release_matmul_resources();

@@ -402,10 +402,14 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
   if (m < 1 || n < 1 || k < 1 || !dtype_ok(dt)) return LLMHIP_ERR_INVALID_ARG;
   if (n % 16 != 0 || k % 16 != 0) return LLMHIP_ERR_UNSUPPORTED;
   // Up to 16 rows one MFMA column block holds every lhs row and the call is a read of W; beyond that lhs, which
-  // every workgroup of that kernel reads whole, outweighs W.  It moves 16-byte pieces; hipBLASLt takes any base.
-  if (m <= 16 && all_aligned16(out, lhs, weight))
-    return from_hip(launch_matmul_skinny(out, lhs, weight, static_cast<const float *>(bias), m, n, k, dt,
-                                         as_stream(stream)));
+  // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  Both kernels move 16-byte
+  // pieces; hipBLASLt takes any base.
+  if (all_aligned16(out, lhs, weight)) {
+    const float *b = static_cast<const float *>(bias);
+    if (m <= 16) return from_hip(launch_matmul_skinny(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
+    if (matmul_tile_takes(m, n, k))
+      return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
+  }
   return from_hip(launch_matmul_bias(out, lhs, weight, static_cast<const float *>(bias), m, n, k, dt,
                                      as_stream(stream)));
 }

@@ -1,0 +1,246 @@
+// Projection of many rows: out[m][n] = lhs[m][k] . W[n][k]^T + bias, fp32 accumulation, one rounding, for calls whose
+// tiles fit the chip in one round (matmul_tile_takes); a launch that needs more is left to hipBLASLt.
+//
+// A workgroup computes one tile of 32*MT lhs rows x 32*NT features over all of k, 64 k (one 128-byte line of every
+// operand row) at a time.  Lines travel global -> LDS without registers, STAGES of them in flight or in use; a
+// fragment load straight into the operand layout, 16 rows by 64 bytes, ran at a third of the rate (512 x
+// 3584, 2048 rows: 29.9 us against 14.3).  Eight waves: four quadrants of the tile, each shared by two waves that take 32 k
+// of every stage, so that a SIMD always has two waves; their sums are traded through LDS at the end.  The fragments of
+// the next stage are read beside the MFMAs of this one, and loads and fragment reads are dealt out among the MFMAs
+// one by one: issued in a burst they held the matrix unit up (128 x 224 tile, k = 3584, 43.4 -> 34.7 us).
+// What bounds a tile now: its MFMAs (28 of 16x16x32 per wave and stage, 0.50 of 0.56 us), for small tiles the
+// barrier and the LDS latency of a stage (32 x 32: 0.09 us where its MFMAs take 0.02).
+//
+// Rows of the operands lie k elements apart, often a multiple of 4 KiB: workgroups that walk k in step would ask few
+// memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
+// (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5).
+//
+// bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 13.2 / 11.0, 128 rows
+// 21.6 / 15.0, 256 rows 19.8 / 18.6, 1019 rows 36.6 / 32.5, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 8.2,
+// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.5; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 72.4 / 65.4.
+#include <atomic>
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace llmhip {
+
+namespace {
+
+constexpr int kTileWaves = 8;
+constexpr int kStageK = 64;               // k of a stage: one 128-byte line of every operand row
+constexpr int kStageRow = 2 * kStageK;    // its bytes
+
+struct TileParams {
+  const char *x, *w;
+  const float *bias;
+  uint16_t *out;
+  int m, n, k;
+  int m_tiles, n_tiles;
+  FastDiv band, band_rows;  // tiles of a band, m tiles of a full band
+};
+
+// LDS offset of logical 16-byte granule g of a staged row
+__device__ __forceinline__ int stage_off(int row, int g) { return row * kStageRow + ((g ^ ((row >> 1) & 7)) << 4); }
+
+template <int N> __device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
+}
+
+template <typename T, int MT, int NT, int STAGES>
+__global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TileParams p) {
+  using E = Elem<T>;
+  constexpr int BM = 32 * MT, BN = 32 * NT, NW = kTileWaves, F = MT * NT, HALF = (F + 1) / 2;
+  constexpr int kStageBytes = (BM + BN) * kStageRow;      // W rows, then lhs rows
+  constexpr int kInstr = (BM + BN) / 8;                   // an instruction fetches 8 rows
+  constexpr int L = (kInstr + NW - 1) / NW;               // of a wave per stage
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int i = lane & 15, cg = lane >> 4;
+
+  // Workgroups are dealt round-robin to the 8 XCDs: each takes a run of tiles, and runs go through bands of up to four
+  // m tiles, so that the tiles of an XCD share rows of both operands in its L2.
+  const int total = p.m_tiles * p.n_tiles, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
+  const int t = xcd * each + min(xcd, rest) + (int)(blockIdx.x >> 3);
+  const int band = (int)fast_div(t, p.band), rem = t - band * (int)p.band.d, gm = (int)p.band_rows.d;
+  const int rows_here = min(gm, p.m_tiles - band * gm);
+  const int tn = rows_here == gm ? (int)fast_div(rem, p.band_rows) : rem / rows_here;
+  const int m0 = (band * gm + rem - tn * rows_here) * BM, n0 = tn * BN;
+
+  const size_t row_bytes = 2 * (size_t)p.k;
+  const char *base[L];
+  uint32_t voff[L], dst[L];
+#pragma unroll
+  for (int s = 0; s < L; ++s) {
+    const int q = min(s * NW + wave, kInstr - 1);  // (a wave without an instruction of its own repeats the last)
+    const int row = 8 * q + (lane >> 3);
+    const bool is_w = 8 * q < BN;
+    const int r = is_w ? min(row, p.n - n0 - 1) : min(row - BN, p.m - m0 - 1);  // rows past the end: the last one
+    base[s] = is_w ? p.w + n0 * row_bytes : p.x + m0 * row_bytes;
+    voff[s] = (uint32_t)r * (uint32_t)row_bytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    dst[s] = __builtin_amdgcn_readfirstlane(q * 8 * kStageRow);
+  }
+  auto issue = [&](int s, int stage, uint32_t slot) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff[s]), "s"(base[s] + (size_t)stage * kStageRow), "s"(slot + dst[s])
+                 : "m0");
+  };
+
+  const int wm = wave & 1, wn = (wave >> 1) & 1, kg = wave >> 2;
+  const int w_addr = stage_off(wn * (BN / 2) + i, 4 * kg + cg), x_addr = stage_off(BN + wm * (BM / 2) + i, 4 * kg + cg);
+  f32x4_t acc[MT][NT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a)
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // The fragments of stage s+1 are read while the MFMAs of stage s run, so that the place of stage s is free for
+  // stage s + STAGES as soon as every wave has come to the barrier.
+  const int stages = p.k / kStageK;
+  int kpos = (int)((unsigned)(xcd * stages / 8 + (t & 3)) % (unsigned)stages);
+  auto advance = [&] { kpos = kpos + 1 == stages ? 0 : kpos + 1; };
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s) {
+#pragma unroll
+    for (int l = 0; l < L; ++l) issue(l, kpos, s * kStageBytes);
+    advance();
+  }
+  uint32_t slot = 0;
+  u32x4_t w0[NT], x0[MT], w1[NT], x1[MT];
+  auto read = [&](u32x4_t (&wf)[NT], u32x4_t (&xf)[MT]) {
+#pragma unroll
+    for (int a = 0; a < MT; ++a) xf[a] = lds_read_b128(lds, x_addr + slot + a * 16 * kStageRow);
+#pragma unroll
+    for (int b = 0; b < NT; ++b) wf[b] = lds_read_b128(lds, w_addr + slot + b * 16 * kStageRow);
+  };
+  auto step = [&](const u32x4_t (&wf)[NT], const u32x4_t (&xf)[MT], u32x4_t (&wnext)[NT], u32x4_t (&xnext)[MT]) {
+    wait_loads<L * (STAGES - 2)>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    const uint32_t fetch = slot;
+    slot = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
+#pragma unroll
+    for (int b = 0; b < (NT > L ? NT : L); ++b) {
+      if (b < L) issue(b, kpos, fetch);
+      if (b < NT) wnext[b] = lds_read_b128(lds, w_addr + slot + b * 16 * kStageRow);
+#pragma unroll
+      for (int a = b; a < MT; a += NT) xnext[a] = lds_read_b128(lds, x_addr + slot + a * 16 * kStageRow);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b < NT) {
+#pragma unroll
+        for (int a = 0; a < MT; ++a) acc[a][b] = E::mfma16(wf[b], xf[a], acc[a][b]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    advance();
+  };
+  wait_loads<L * (STAGES - 1)>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  read(w0, x0);
+  for (int s = 0; s < stages; s += 2) {
+    step(w0, x0, w1, x1);
+    if (s + 1 < stages) step(w1, x1, w0, x0);
+  }
+
+  wait_loads<0>();  // the loads past the last stage (k from its start again) still aim at the places written next
+  // The two waves of a quadrant trade halves of their sums, and each rounds and stores the half it keeps.
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  f32x4_t *pieces = reinterpret_cast<f32x4_t *>(lds) + lane;
+#pragma unroll
+  for (int f = 0; f < F; ++f)
+    if ((f >= HALF) == (kg == 0)) pieces[((wave & 3) * F + f) * 64] = acc[f / NT][f % NT];
+  __syncthreads();
+#pragma unroll
+  for (int f = 0; f < F; ++f) {
+    if ((f >= HALF) == (kg == 0)) continue;  // (wave-uniform)
+    const int row = m0 + wm * (BM / 2) + (f / NT) * 16 + i, col = n0 + wn * (BN / 2) + (f % NT) * 16 + 4 * cg;
+    f32x4_t sum = acc[f / NT][f % NT] + pieces[((wave & 3) * F + f) * 64];
+    if (row >= p.m || col >= p.n) continue;
+    if (p.bias) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum[j] += p.bias[col + j];
+    }
+    *reinterpret_cast<u32x2_t *>(p.out + (size_t)row * p.n + col) = u32x2_t{E::pack2(sum[0], sum[1]), E::pack2(sum[2], sum[3])};
+  }
+}
+
+template <typename T, int MT, int NT, int STAGES> hipError_t launch_tile(TileParams &p, hipStream_t stream) {
+  p.m_tiles = (p.m + 32 * MT - 1) / (32 * MT);
+  p.n_tiles = (p.n + 32 * NT - 1) / (32 * NT);
+  const int gm = p.m_tiles < 4 ? p.m_tiles : 4;
+  p.band = make_fast_div((uint32_t)(gm * p.n_tiles));
+  p.band_rows = make_fast_div((uint32_t)gm);
+  constexpr int stage_bytes = STAGES * 32 * (MT + NT) * kStageRow, piece_bytes = 4 * MT * NT * 1024;
+  constexpr int lds_bytes = stage_bytes > piece_bytes ? stage_bytes : piece_bytes;
+  static_assert(lds_bytes <= 160 * 1024, "");
+  void (*kern)(TileParams) = matmul_tile_kernel<T, MT, NT, STAGES>;
+  if (lds_bytes > 64 * 1024) {  // an opt-in per device and kernel
+    static std::atomic<uint64_t> attr_done{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(attr_done.load(std::memory_order_acquire) & bit)) {
+      e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+      if (e != hipSuccess) return e;
+      attr_done.fetch_or(bit, std::memory_order_release);
+    }
+  }
+  hipLaunchKernelGGL(kern, dim3(p.m_tiles * p.n_tiles), dim3(64 * kTileWaves), lds_bytes, stream, p);
+  return hipGetLastError();
+}
+
+template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_t stream) {
+  switch (kind) {
+    case 0: return launch_tile<T, 1, 1, 6>(p, stream);
+    case 1: return launch_tile<T, 2, 1, 6>(p, stream);
+    case 2: return launch_tile<T, 2, 2, 6>(p, stream);
+    case 3: return launch_tile<T, 4, 2, 4>(p, stream);
+    case 4: return launch_tile<T, 4, 4, 4>(p, stream);
+    case 5: return launch_tile<T, 4, 6, 3>(p, stream);
+    case 6: return launch_tile<T, 4, 7, 3>(p, stream);
+    default: return launch_tile<T, 4, 8, 3>(p, stream);
+  }
+}
+
+// The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
+// From 128 x 64 on hipBLASLt, which cuts k too, is the faster one where that leaves a fifth of the CUs idle: 3584 x
+// 3584, 384 rows (66 % busy) 22.2 us against 26.0, 512 rows (88 %) 25.6 / 25.3, 4096 x 4096, 768 rows (75 %)
+// 33.1 / 36.4, 1019 rows (100 %) 42.1 / 35.7.  Not so up to k = 2048, where the start of a workgroup weighs more: 1536 x
+// 1536, 768 rows (56 %) 12.4 / 11.2.  The 128 x 256 tile, where the MFMAs of either fill the chip, is kept for
+// wide k: 4096 rows of W, 2048 rows, k = 4096 59.5 / 61.3, k = 11008 161 / 147, 5120 x 5120, 1500 rows 77.3 / 72.2.
+int tile_kind(int m, int n, int k) {
+  static const struct { int m, n; } tiles[] = {{32, 32}, {64, 32}, {64, 64}, {128, 64}, {128, 128}, {128, 192}, {128, 224}, {128, 256}};
+  const long long cus = device_compute_units();
+  for (int kind = 0; kind < 8; ++kind) {
+    const long long count = (long long)((m + tiles[kind].m - 1) / tiles[kind].m) * ((n + tiles[kind].n - 1) / tiles[kind].n);
+    if (count > cus) continue;
+    if (kind >= 3 && k > 2048 && 5 * count <= 4 * cus) return -1;
+    if (kind == 7 && k <= 4096) return -1;
+    return kind;
+  }
+  return -1;
+}
+
+}  // namespace
+
+// k in whole stages; offsets inside a tile are 32 bits.
+bool matmul_tile_takes(int m, int n, int k) {
+  return k % kStageK == 0 && k <= 1 << 20 && tile_kind(m, n, k) >= 0;
+}
+
+hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias, int m, int n, int k,
+                              int dt, hipStream_t stream) {
+  TileParams p;
+  p.x = static_cast<const char *>(lhs);
+  p.w = static_cast<const char *>(weight);
+  p.bias = bias;
+  p.out = static_cast<uint16_t *>(out);
+  p.m = m;
+  p.n = n;
+  p.k = k;
+  const int kind = tile_kind(m, n, k);
+  return dt == kDtFloat16 ? launch_kind<_Float16>(p, kind, stream) : launch_kind<__bf16>(p, kind, stream);
+}
+
+}  // namespace llmhip

@@ -1,0 +1,46 @@
+"""The tiled projection kernel against the oracle: every tile shape, with full and ragged tiles in both directions,
+k of one stage, fewer stages than are kept in flight and an odd number of them, tiles in several bands, and the sizes next
+to it (k in part stages, an unaligned base) that take the other path."""
+import numpy as np
+import pytest
+
+from helpers import DT_BFLOAT16, DT_FLOAT16, f32_dev, normal_bits, to_dev, to_host, ulp
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dt", [DT_FLOAT16, DT_BFLOAT16])
+@pytest.mark.parametrize("m,n,k,bias", [
+    (17, 16, 64, True), (32, 8192, 64, False), (200, 272, 832, True),           # 32 x 32
+    (161, 1552, 192, True), (512, 1024, 128, False),                            # 64 x 32
+    (300, 2000, 320, True), (1024, 1024, 64, False),                            # 64 x 64
+    (600, 3088, 192, True),                                                     # 128 x 64
+    (129, 8208, 64, False), (1100, 3088, 128, True), (2048, 2048, 256, False),  # 128 x 128
+    (1500, 3584, 64, True), (130, 24000, 128, False),                           # 128 x 192
+    (2048, 3584, 64, True), (1900, 3600, 128, False),                           # 128 x 224
+    (2000, 4080, 4160, True),                                                   # 128 x 256
+    (64, 512, 80, True)])                                                       # not taken: part stages
+def test_tiles(dt, m, n, k, bias):
+    import torch
+    import llm_simple_amd.ops as ops
+    x = normal_bits(m + k, (m, k), dt)
+    w = orc.round_to(orc.widen(normal_bits(n, (n, k), dt), dt) / np.sqrt(k), dt)
+    b = np.random.default_rng(n).standard_normal(n).astype(np.float32) if bias else None
+    if m * n * k < 1 << 28:
+        ref = orc.widen(orc.matmul_bias(x, w, b, dt), dt)
+    else:  # the oracle's contraction order in fp32, by the host's BLAS
+        ref = orc.widen(x, dt) @ orc.widen(w, dt).T + (0.0 if b is None else b)
+        ref = orc.widen(orc.round_to(ref.astype(np.float32), dt), dt)
+    for shift in (0, 1):  # a base that is not 16-byte aligned takes the other path
+        d_x = torch.empty(m * k + 8, dtype=torch.int16, device="cuda")[shift:shift + m * k]
+        d_x.copy_(to_dev(x).flatten())
+        guard = torch.full((m * n + 16,), 0x55, dtype=torch.int16, device="cuda")
+        args = (guard[8:8 + m * n], d_x, to_dev(w))
+        if bias:
+            ops.hip_matmul_bias_layer(*args, f32_dev(b), m, n, k, dt)
+        else:
+            ops.hip_matmul_layer(*args, m, n, k, dt)
+        got = orc.widen(to_host(guard[8:8 + m * n]), dt).reshape(m, n)
+        assert (np.abs(got - ref) <= np.maximum(1.01 * ulp(ref, dt), 1e-3)).all()
+        assert (guard[:8] == 0x55).all() and (guard[8 + m * n:] == 0x55).all()
