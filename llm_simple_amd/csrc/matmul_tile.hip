@@ -1,23 +1,24 @@
 // Projection of many rows: out[m][n] = lhs[m][k] . W[n][k]^T + bias, fp32 accumulation, one rounding, for calls whose
 // tiles fit the chip in one round (matmul_tile_takes); a launch that needs more is left to hipBLASLt.
 //
-// A workgroup computes one tile of 32*MT lhs rows x 32*NT features over all of k, 64 k (one 128-byte line of every
-// operand row) at a time.  Lines travel global -> LDS without registers, STAGES of them in flight or in use; a
+// A workgroup computes one tile of 32*MT lhs rows x 32*NT features over all of k in stages of KS * 64 k (KS 128-byte
+// lines of every operand row).  Lines travel global -> LDS without registers, STAGES of them in flight or in use; a
 // fragment load straight into the operand layout, 16 rows by 64 bytes, ran at a third of the rate (512 x
 // 3584, 2048 rows: 29.9 us against 14.3).  Eight waves: four quadrants of the tile, each shared by two waves that take 32 k
-// of every stage, so that a SIMD always has two waves; their sums are traded through LDS at the end.  The fragments of
+// of every line, so that a SIMD always has two waves; their sums are traded through LDS at the end.  The fragments of
 // the next stage are read beside the MFMAs of this one, and loads and fragment reads are dealt out among the MFMAs
 // one by one: issued in a burst they held the matrix unit up (128 x 224 tile, k = 3584, 43.4 -> 34.7 us).
 // What bounds a tile now: its MFMAs (28 of 16x16x32 per wave and stage, 0.50 of 0.56 us), for small tiles the
-// barrier and the LDS latency of a stage (32 x 32: 0.09 us where its MFMAs take 0.02).
+// rate at which one CU takes lines in, 60-80 KB/us, and the barrier and LDS latency of a stage (32 x 32: 0.09 us a line where
+// its MFMAs take 0.02; with two lines a stage 0.08, 512 x 3584, 100 rows: 8.0 -> 7.4 us; larger tiles gain nothing by it).
 //
 // Rows of the operands lie k elements apart, often a multiple of 4 KiB: workgroups that walk k in step would ask few
 // memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
 // (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5).
 //
 // bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 13.2 / 11.0, 128 rows
-// 21.6 / 15.0, 256 rows 19.8 / 18.6, 1019 rows 36.6 / 32.5, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 8.2,
-// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.5; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 72.4 / 65.4.
+// 21.6 / 15.0, 256 rows 19.8 / 18.6, 1019 rows 36.6 / 32.5, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 7.5,
+// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.3; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 72.4 / 65.4.
 #include <atomic>
 
 #include "common.hpp"
@@ -28,8 +29,8 @@ namespace llmhip {
 namespace {
 
 constexpr int kTileWaves = 8;
-constexpr int kStageK = 64;               // k of a stage: one 128-byte line of every operand row
-constexpr int kStageRow = 2 * kStageK;    // its bytes
+constexpr int kLineK = 64;             // k of a 128-byte line of an operand row
+constexpr int kStageRow = 2 * kLineK;  // its bytes
 
 struct TileParams {
   const char *x, *w;
@@ -47,13 +48,14 @@ template <int N> __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
 }
 
-template <typename T, int MT, int NT, int STAGES>
+template <typename T, int MT, int NT, int KS, int STAGES>
 __global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TileParams p) {
   using E = Elem<T>;
   constexpr int BM = 32 * MT, BN = 32 * NT, NW = kTileWaves, F = MT * NT, HALF = (F + 1) / 2;
-  constexpr int kStageBytes = (BM + BN) * kStageRow;      // W rows, then lhs rows
+  constexpr int kLineBytes = (BM + BN) * kStageRow;       // one line of every row: W rows, then lhs rows
+  constexpr int kStageBytes = KS * kLineBytes;
   constexpr int kInstr = (BM + BN) / 8;                   // an instruction fetches 8 rows
-  constexpr int L = (kInstr + NW - 1) / NW;               // of a wave per stage
+  constexpr int L = (kInstr + NW - 1) / NW;               // of a wave per line
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i = lane & 15, cg = lane >> 4;
@@ -97,49 +99,55 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TilePar
 
   // The fragments of stage s+1 are read while the MFMAs of stage s run, so that the place of stage s is free for
   // stage s + STAGES as soon as every wave has come to the barrier.
-  const int stages = p.k / kStageK;
-  int kpos = (int)((unsigned)(xcd * stages / 8 + (t & 3)) % (unsigned)stages);
-  auto advance = [&] { kpos = kpos + 1 == stages ? 0 : kpos + 1; };
+  const int lines = p.k / kLineK;
+  int kpos = (int)((unsigned)(xcd * lines / 8 + (t & 3)) % (unsigned)lines);
+  auto issue_line = [&](uint32_t place) {
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s) {
-#pragma unroll
-    for (int l = 0; l < L; ++l) issue(l, kpos, s * kStageBytes);
-    advance();
-  }
-  uint32_t slot = 0;
-  u32x4_t w0[NT], x0[MT], w1[NT], x1[MT];
-  auto read = [&](u32x4_t (&wf)[NT], u32x4_t (&xf)[MT]) {
-#pragma unroll
-    for (int a = 0; a < MT; ++a) xf[a] = lds_read_b128(lds, x_addr + slot + a * 16 * kStageRow);
-#pragma unroll
-    for (int b = 0; b < NT; ++b) wf[b] = lds_read_b128(lds, w_addr + slot + b * 16 * kStageRow);
+    for (int l = 0; l < L; ++l) issue(l, kpos, place);
+    kpos = kpos + 1 == lines ? 0 : kpos + 1;
   };
-  auto step = [&](const u32x4_t (&wf)[NT], const u32x4_t (&xf)[MT], u32x4_t (&wnext)[NT], u32x4_t (&xnext)[MT]) {
-    wait_loads<L * (STAGES - 2)>();
+#pragma unroll
+  for (int s = 0; s < STAGES * KS; ++s) issue_line(s * kLineBytes);
+  uint32_t slot = 0;
+  u32x4_t w0[KS][NT], x0[KS][MT], w1[KS][NT], x1[KS][MT];
+  auto step = [&](int line, const u32x4_t (&wf)[KS][NT], const u32x4_t (&xf)[KS][MT], u32x4_t (&wnext)[KS][NT],
+                  u32x4_t (&xnext)[KS][MT]) {
+    wait_loads<L * KS * (STAGES - 2)>();
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const uint32_t fetch = slot;
     slot = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
 #pragma unroll
-    for (int b = 0; b < (NT > L ? NT : L); ++b) {
-      if (b < L) issue(b, kpos, fetch);
-      if (b < NT) wnext[b] = lds_read_b128(lds, w_addr + slot + b * 16 * kStageRow);
+    for (int u = 0; u < KS; ++u) {
+      const bool have = KS == 1 || line + u < lines;  // (the last stage may hold surplus lines)
 #pragma unroll
-      for (int a = b; a < MT; a += NT) xnext[a] = lds_read_b128(lds, x_addr + slot + a * 16 * kStageRow);
-      __builtin_amdgcn_sched_barrier(0);
-      if (b < NT) {
+      for (int b = 0; b < (NT > L ? NT : L); ++b) {
+        if (b < L) issue(b, kpos, fetch + u * kLineBytes);
+        if (b < NT) wnext[u][b] = lds_read_b128(lds, w_addr + slot + u * kLineBytes + b * 16 * kStageRow);
 #pragma unroll
-        for (int a = 0; a < MT; ++a) acc[a][b] = E::mfma16(wf[b], xf[a], acc[a][b]);
+        for (int a = b; a < MT; a += NT)
+          xnext[u][a] = lds_read_b128(lds, x_addr + slot + u * kLineBytes + a * 16 * kStageRow);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b < NT && have) {
+#pragma unroll
+          for (int a = 0; a < MT; ++a) acc[a][b] = E::mfma16(wf[u][b], xf[u][a], acc[a][b]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+      kpos = kpos + 1 == lines ? 0 : kpos + 1;
     }
-    advance();
   };
-  wait_loads<L * (STAGES - 1)>();
+  wait_loads<L * KS * (STAGES - 1)>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  read(w0, x0);
-  for (int s = 0; s < stages; s += 2) {
-    step(w0, x0, w1, x1);
-    if (s + 1 < stages) step(w1, x1, w0, x0);
+#pragma unroll
+  for (int u = 0; u < KS; ++u) {
+#pragma unroll
+    for (int a = 0; a < MT; ++a) x0[u][a] = lds_read_b128(lds, x_addr + u * kLineBytes + a * 16 * kStageRow);
+#pragma unroll
+    for (int b = 0; b < NT; ++b) w0[u][b] = lds_read_b128(lds, w_addr + u * kLineBytes + b * 16 * kStageRow);
+  }
+  for (int line = 0; line < lines; line += 2 * KS) {
+    step(line, w0, x0, w1, x1);
+    if (line + KS < lines) step(line + KS, w1, x1, w0, x0);
   }
 
   wait_loads<0>();  // the loads past the last stage (k from its start again) still aim at the places written next
@@ -164,16 +172,16 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TilePar
   }
 }
 
-template <typename T, int MT, int NT, int STAGES> hipError_t launch_tile(TileParams &p, hipStream_t stream) {
+template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile(TileParams &p, hipStream_t stream) {
   p.m_tiles = (p.m + 32 * MT - 1) / (32 * MT);
   p.n_tiles = (p.n + 32 * NT - 1) / (32 * NT);
   const int gm = p.m_tiles < 4 ? p.m_tiles : 4;
   p.band = make_fast_div((uint32_t)(gm * p.n_tiles));
   p.band_rows = make_fast_div((uint32_t)gm);
-  constexpr int stage_bytes = STAGES * 32 * (MT + NT) * kStageRow, piece_bytes = 4 * MT * NT * 1024;
+  constexpr int stage_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow, piece_bytes = 4 * MT * NT * 1024;
   constexpr int lds_bytes = stage_bytes > piece_bytes ? stage_bytes : piece_bytes;
   static_assert(lds_bytes <= 160 * 1024, "");
-  void (*kern)(TileParams) = matmul_tile_kernel<T, MT, NT, STAGES>;
+  void (*kern)(TileParams) = matmul_tile_kernel<T, MT, NT, KS, STAGES>;
   if (lds_bytes > 64 * 1024) {  // an opt-in per device and kernel
     static std::atomic<uint64_t> attr_done{0};
     int dev = 0;
@@ -192,14 +200,14 @@ template <typename T, int MT, int NT, int STAGES> hipError_t launch_tile(TilePar
 
 template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_t stream) {
   switch (kind) {
-    case 0: return launch_tile<T, 1, 1, 6>(p, stream);
-    case 1: return launch_tile<T, 2, 1, 6>(p, stream);
-    case 2: return launch_tile<T, 2, 2, 6>(p, stream);
-    case 3: return launch_tile<T, 4, 2, 4>(p, stream);
-    case 4: return launch_tile<T, 4, 4, 4>(p, stream);
-    case 5: return launch_tile<T, 4, 6, 3>(p, stream);
-    case 6: return launch_tile<T, 4, 7, 3>(p, stream);
-    default: return launch_tile<T, 4, 8, 3>(p, stream);
+    case 0: return launch_tile<T, 1, 1, 2, 4>(p, stream);
+    case 1: return launch_tile<T, 2, 1, 1, 6>(p, stream);
+    case 2: return launch_tile<T, 2, 2, 1, 6>(p, stream);
+    case 3: return launch_tile<T, 4, 2, 1, 4>(p, stream);
+    case 4: return launch_tile<T, 4, 4, 1, 4>(p, stream);
+    case 5: return launch_tile<T, 4, 6, 1, 3>(p, stream);
+    case 6: return launch_tile<T, 4, 7, 1, 3>(p, stream);
+    default: return launch_tile<T, 4, 8, 1, 3>(p, stream);
   }
 }
 
@@ -226,7 +234,7 @@ int tile_kind(int m, int n, int k) {
 
 // k in whole stages; offsets inside a tile are 32 bits.
 bool matmul_tile_takes(int m, int n, int k) {
-  return k % kStageK == 0 && k <= 1 << 20 && tile_kind(m, n, k) >= 0;
+  return k % kLineK == 0 && k <= 1 << 20 && tile_kind(m, n, k) >= 0;
 }
 
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias, int m, int n, int k,
