@@ -23,8 +23,9 @@
 // type is rounded by the hardware conversion (equal to round-to-nearest-even on the bit pattern for
 // every non-NaN fp32), the token of a unit comes from a multiply-shift division, the stores are
 // non-temporal.  (Measured at 4096 tokens of Qwen2.5-7B: 12.7 us with the buffers in the last-level
-// cache, 16.5 us from and to HBM; the same kernel without arithmetic and table 12.2 us with ordinary
-// stores, so the rest is the memory path of three separate streams of 256-byte rows.)
+// cache, 15.2 us from and to HBM, where a plain device copy of the same bytes takes 16; the same kernel without
+// arithmetic and table 12.2 us with ordinary stores, so the rest is the memory path of three separate streams
+// of 256-byte rows.  256 tokens, 32 heads 4.1 us, of which the launch is 2.5.)
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -47,14 +48,8 @@ struct RopeParams {
 // = (a[i], b[i]) (dims f, f + 64); interleaved: pair i = elements 2i, 2i+1 of the 16 contiguous ones.
 // Arithmetic of src/llama2_layer_cpu.cpp:835-856: every product and sum rounded on its own.
 template <typename T, bool NEOX>
-__device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const float *tab) {
+__device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t (&cs)[4]) {
   using E = Elem<T>;
-  const f32x4_t t0 = *reinterpret_cast<const f32x4_t *>(tab);
-  const f32x4_t t1 = *reinterpret_cast<const f32x4_t *>(tab + 4);
-  const f32x4_t t2 = *reinterpret_cast<const f32x4_t *>(tab + 8);
-  const f32x4_t t3 = *reinterpret_cast<const f32x4_t *>(tab + 12);
-  const float cs[16] = {t0[0], t0[1], t0[2], t0[3], t1[0], t1[1], t1[2], t1[3],
-                        t2[0], t2[1], t2[2], t2[3], t3[0], t3[1], t3[2], t3[3]};
   float r0[8], r1[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -68,7 +63,7 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const float *t
       xb = (uint16_t)(w >> 16);
     }
     const float a = E::widen(xa), b = E::widen(xb);
-    const float c = cs[2 * i], d = cs[2 * i + 1];
+    const float c = cs[i >> 1][2 * (i & 1)], d = cs[i >> 1][2 * (i & 1) + 1];
     r0[i] = a * c - b * d;
     r1[i] = a * d + b * c;
   }
@@ -93,12 +88,15 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
   const uint32_t stride = gridDim.x * 256u;
   const uint32_t gid0 = blockIdx.x * 256u + threadIdx.x;
   u32x4_t va[U], vb[U];
+  f32x4_t cs[U][4];
   char *outp[U];
-  const float *tabp[U];
   bool rot[U], live[U];
   const uint32_t j = gid0 & 7u;  // stride is a multiple of 8
   const int off_a = NEOX ? (int)j * 16 : (int)j * 32;
   const int off_b = NEOX ? off_a + 128 : off_a + 16;
+  // All loads of a thread go out before anything is waited for, the table's included (a V row's are not used): asked for
+  // when a unit is rotated, the second unit's table was one more memory round trip (from and to HBM 4096 tokens 16.25
+  // -> 15.2 us, 1019 tokens 6.75 -> 5.9; rope and attention of 256 tokens, 32 heads 13.3 -> 13.0).
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t gid = gid0 + u * stride;
@@ -106,29 +104,24 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
     const uint32_t rowid = (live[u] ? gid : 0u) >> 3;
     const uint32_t s = fast_div(rowid, p.rows_per_token);
     const int r = (int)(rowid - s * p.rows_per_token.d);
-    const char *in;
-    rot[u] = true;
-    if (r < p.q_heads) {
-      const size_t row = ((size_t)s * p.q_heads + r) * kRowBytes;
-      in = p.in_q + row;
-      outp[u] = p.out_q + row;
-    } else if (r < p.q_heads + p.k_heads) {
-      const int h = r - p.q_heads;
-      in = p.in_k + ((size_t)s * p.k_heads + h) * kRowBytes;
-      outp[u] = p.out_k + ((size_t)(s + p.k_out_row_offset) * p.k_heads + h) * kRowBytes;
-    } else {
-      const int h = r - p.q_heads - p.k_heads;
-      in = p.in_v + ((size_t)s * p.v_heads + h) * kRowBytes;
-      outp[u] = p.out_v + ((size_t)(s + p.k_out_row_offset) * p.v_heads + h) * kRowBytes;
-      rot[u] = false;
-    }
-    tabp[u] = p.freq_cis + (size_t)(p.start_pos + s) * kHeadDim + 16 * j;
+    const bool is_q = r < p.q_heads;
+    rot[u] = r < p.q_heads + p.k_heads;
+    const int heads = is_q ? p.q_heads : p.k_heads;  // V has as many as K
+    const int h = is_q ? r : rot[u] ? r - p.q_heads : r - p.q_heads - p.k_heads;
+    const char *in = is_q ? p.in_q : rot[u] ? p.in_k : p.in_v;
+    char *out = is_q ? p.out_q : rot[u] ? p.out_k : p.out_v;
+    in += ((size_t)s * heads + h) * kRowBytes;
+    outp[u] = out + ((size_t)(s + (is_q ? 0 : p.k_out_row_offset)) * heads + h) * kRowBytes;
+    const float *tab = p.freq_cis + (size_t)(p.start_pos + s) * kHeadDim + 16 * j;
     va[u] = global_load_b128(in + off_a);
     vb[u] = global_load_b128(in + off_b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cs[u][i] = *reinterpret_cast<const f32x4_t *>(tab + 4 * i);
   }
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (rot[u]) rotate8<T, NEOX>(va[u], vb[u], tabp[u]);
+    if (rot[u]) rotate8<T, NEOX>(va[u], vb[u], cs[u]);
     if (live[u]) {
       // Non-temporal stores for every output row (measured at 4096 tokens, H=28, Hkv=4: from and to HBM
       // 18.2 -> 16.5 us, buffers resident in the last-level cache 13.15 -> 12.70 us; the attention launch
