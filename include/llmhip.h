@@ -216,8 +216,9 @@ int llmhip_release_internal_workspace(void);
  * src/llama2_layer_npu.cpp:1178-1180): out[m][n] = lhs[m][k] . W^T, fp32 accumulation, one
  * rounding to dt.  `weight` is W[n][k] row-major -- the checkpoint layout -- not the
  * reference's Ascend "nz" repacking [n/16][k][16] (tests/gemm_test.cpp:95-101).  n and k
- * must be multiples of 16 (src/llama2_layer_npu.cpp:1211-1218).  Runs on hipBLASLt; the first
- * call allocates the library's handle and a 64 MiB workspace. */
+ * must be multiples of 16 (src/llama2_layer_npu.cpp:1211-1218).  Runs on kernels of this library up to 16 rows, and where its
+ * tiles fit the chip in one round (16-byte aligned pointers; k a multiple of 64 beyond 16 rows); other calls run on
+ * hipBLASLt, the first of which allocates its handle and a 64 MiB workspace. */
 int llmhip_matmul(void *out, const void *lhs, const void *weight, int m, int n, int k, int dt,
                   void *stream);
 
