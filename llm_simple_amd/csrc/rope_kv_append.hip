@@ -21,11 +21,11 @@
 // by the same 8 lanes without the arithmetic.  A thread takes kRopeUnits units a whole grid apart and
 // issues all their loads before it computes.  The pairing style is a template parameter, the storage
 // type is rounded by the hardware conversion (equal to round-to-nearest-even on the bit pattern for
-// every non-NaN fp32), the token of a unit comes from a multiply-shift division, the stores are
-// non-temporal.  (Measured at 4096 tokens of Qwen2.5-7B: 12.7 us with the buffers in the last-level
-// cache, 15.2 us from and to HBM, where a plain device copy of the same bytes takes 16; the same kernel without
-// arithmetic and table 12.2 us with ordinary stores, so the rest is the memory path of three separate streams
-// of 256-byte rows.  256 tokens, 32 heads 4.1 us, of which the launch is 2.5.)
+// every non-NaN fp32), the token of a unit comes from a multiply-shift division.  (Measured at
+// 4096 tokens of Qwen2.5-7B: 13.1 us with the buffers in the last-level cache, 16.4 us from and to HBM, where a
+// plain device copy of the same bytes takes 16; the same kernel without arithmetic and table 12.2 us, so the rest
+// is the memory path of three separate streams of 256-byte rows.  256 tokens, 32 heads 4.1 us, of which the
+// launch is 2.5.)
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -95,8 +95,8 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
   const int off_a = NEOX ? (int)j * 16 : (int)j * 32;
   const int off_b = NEOX ? off_a + 128 : off_a + 16;
   // All loads of a thread go out before anything is waited for, the table's included (a V row's are not used): asked for
-  // when a unit is rotated, the second unit's table was one more memory round trip (from and to HBM 4096 tokens 16.25
-  // -> 15.2 us, 1019 tokens 6.75 -> 5.9; rope and attention of 256 tokens, 32 heads 13.3 -> 13.0).
+  // when a unit is rotated, the second unit's table was one more memory round trip (with non-temporal stores, from and
+  // to HBM, 4096 tokens 16.25 -> 15.2 us, 1019 tokens 6.75 -> 5.9; rope and attention of 256 tokens, 32 heads 13.3 -> 13.0).
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t gid = gid0 + u * stride;
@@ -123,12 +123,11 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
   for (int u = 0; u < U; ++u) {
     if (rot[u]) rotate8<T, NEOX>(va[u], vb[u], cs[u]);
     if (live[u]) {
-      // Non-temporal stores for every output row (measured at 4096 tokens, H=28, Hkv=4: from and to HBM
-      // 18.2 -> 16.5 us, buffers resident in the last-level cache 13.15 -> 12.70 us; the attention launch
-      // that reads the rows next takes the same time either way).  Marking only the cache rows changes
-      // nothing: 7 of 9 written rows are rotated q.
-      __builtin_nontemporal_store(va[u], reinterpret_cast<u32x4_t *>(outp[u] + off_a));
-      __builtin_nontemporal_store(vb[u], reinterpret_cast<u32x4_t *>(outp[u] + off_b));
+      // Ordinary stores: the attention launch reads the rows next.  Non-temporal ones make this launch shorter by itself
+      // (1019 tokens 5.2 -> 4.5 us, 4096 from and to HBM 16.4 -> 15.2) and the pair longer: rope and attention of 256
+      // tokens, 32 heads 12.3 -> 13.05 us, 1019 tokens, 28 heads 22.9 -> 26.5, 4096 131.2 -> 133.0, 8192 446 -> 450.
+      *reinterpret_cast<u32x4_t *>(outp[u] + off_a) = va[u];
+      *reinterpret_cast<u32x4_t *>(outp[u] + off_b) = vb[u];
     }
   }
 }
