@@ -17,8 +17,8 @@
 // (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5).
 //
 // bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 13.2 / 11.0, 128 rows
-// 21.6 / 15.0, 256 rows 19.8 / 18.6, 1019 rows 36.6 / 32.5, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 7.5,
-// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.3; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 72.4 / 65.4.
+// 21.6 / 15.0, 256 rows 19.8 / 18.6, 768 rows 33.1 / 29.4, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 7.5,
+// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.3; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 74.4 / 69.1.
 #include <atomic>
 
 #include "common.hpp"
@@ -203,28 +203,36 @@ template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_
     case 0: return launch_tile<T, 1, 1, 2, 4>(p, stream);
     case 1: return launch_tile<T, 2, 1, 1, 6>(p, stream);
     case 2: return launch_tile<T, 2, 2, 1, 6>(p, stream);
-    case 3: return launch_tile<T, 4, 2, 1, 4>(p, stream);
-    case 4: return launch_tile<T, 4, 4, 1, 4>(p, stream);
-    case 5: return launch_tile<T, 4, 6, 1, 3>(p, stream);
-    case 6: return launch_tile<T, 4, 7, 1, 3>(p, stream);
+    case 3: return launch_tile<T, 3, 2, 1, 5>(p, stream);
+    case 4: return launch_tile<T, 4, 2, 1, 4>(p, stream);
+    case 5: return launch_tile<T, 3, 3, 1, 4>(p, stream);
+    case 6: return launch_tile<T, 3, 4, 1, 4>(p, stream);
+    case 7: return launch_tile<T, 4, 4, 1, 4>(p, stream);
+    case 8: return launch_tile<T, 4, 5, 1, 4>(p, stream);
+    case 9: return launch_tile<T, 4, 6, 1, 3>(p, stream);
+    case 10: return launch_tile<T, 4, 7, 1, 3>(p, stream);
     default: return launch_tile<T, 4, 8, 1, 3>(p, stream);
   }
 }
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
-// From 128 x 64 on hipBLASLt, which cuts k too, is the faster one where that leaves a fifth of the CUs idle: 3584 x
-// 3584, 384 rows (66 % busy) 22.2 us against 26.0, 512 rows (88 %) 25.6 / 25.3, 4096 x 4096, 768 rows (75 %)
-// 33.1 / 36.4, 1019 rows (100 %) 42.1 / 35.7.  Not so up to k = 2048, where the start of a workgroup weighs more: 1536 x
-// 1536, 768 rows (56 %) 12.4 / 11.2.  The 128 x 256 tile, where the MFMAs of either fill the chip, is kept for
-// wide k: 4096 rows of W, 2048 rows, k = 4096 59.5 / 61.3, k = 11008 161 / 147, 5120 x 5120, 1500 rows 77.3 / 72.2.
+// (Twelve tiles rather than eight fill the round better; us, hipBLASLt / here: 3584 x 3584, 320 rows 22.8 / 19.7, 768 rows
+// 33.1 / 29.4, 1280 rows 43.3 / 39.2; 5120 x 5120, 900 rows 62.6 / 56.9.  128 x 96 and 64 x 96 are slower than 96 x 128 and
+// 96 x 64: 640 rows 31.3 / 28.6, 200 rows of 5120 30.4 / 28.2.)
+// From 96 x 64 on hipBLASLt, which cuts k too, is the faster one where that leaves a fifth of the CUs idle: 5120 x 5120, 640
+// rows (78 % busy) 51.5 us against 53.7, 768 rows (94 %) 53.3 / 53.2, 900 rows (100 %) 62.6 / 56.9.  Not so up to k = 2048,
+// where the start of a workgroup weighs more: 1536 x 1536, 768 rows (56 %) 12.4 / 11.2.  And from 128 x 192 on where rows are a
+// multiple of 4 KiB apart: 4096 x 4096, 1280 rows 46.6 / 47.6, 1500 rows 49.7 / 53.7, against 3584 x 3584, 1500 rows 44.2 /
+// 42.7, 2048 rows 52.4 / 50.7.
 int tile_kind(int m, int n, int k) {
-  static const struct { int m, n; } tiles[] = {{32, 32}, {64, 32}, {64, 64}, {128, 64}, {128, 128}, {128, 192}, {128, 224}, {128, 256}};
+  static const struct { int m, n; } tiles[] = {{32, 32},  {64, 32},   {64, 64},   {96, 64},   {128, 64},  {96, 96},
+                                               {96, 128}, {128, 128}, {128, 160}, {128, 192}, {128, 224}, {128, 256}};
   const long long cus = device_compute_units();
-  for (int kind = 0; kind < 8; ++kind) {
+  for (int kind = 0; kind < 12; ++kind) {
     const long long count = (long long)((m + tiles[kind].m - 1) / tiles[kind].m) * ((n + tiles[kind].n - 1) / tiles[kind].n);
     if (count > cus) continue;
     if (kind >= 3 && k > 2048 && 5 * count <= 4 * cus) return -1;
-    if (kind == 7 && k <= 4096) return -1;
+    if (kind >= 9 && k % 2048 == 0) return -1;
     return kind;
   }
   return -1;

@@ -15,8 +15,12 @@ pytestmark = pytest.mark.gpu
     (17, 16, 64, True), (32, 8192, 64, False), (200, 272, 832, True),           # 32 x 32
     (161, 1552, 192, True), (512, 1024, 128, False),                            # 64 x 32
     (300, 2000, 320, True), (1024, 1024, 64, False),                            # 64 x 64
-    (600, 3088, 192, True),                                                     # 128 x 64
-    (129, 8208, 64, False), (1100, 3088, 128, True), (2048, 2048, 256, False),  # 128 x 128
+    (300, 3600, 256, True), (520, 2576, 64, False),                             # 96 x 64
+    (512, 3600, 192, True),                                                     # 128 x 64
+    (570, 3600, 128, True), (700, 2832, 64, False),                             # 96 x 96
+    (640, 4112, 192, False), (129, 15008, 64, True),                            # 96 x 128
+    (1100, 3344, 128, True), (2048, 2048, 256, False),                          # 128 x 128
+    (1280, 3600, 64, True),                                                     # 128 x 160
     (1500, 3584, 64, True), (130, 24000, 128, False),                           # 128 x 192
     (2048, 3584, 64, True), (1900, 3600, 128, False),                           # 128 x 224
     (2000, 4080, 4160, True),                                                   # 128 x 256
