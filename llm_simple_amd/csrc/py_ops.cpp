@@ -2,8 +2,9 @@
 //
 // A decode step of a small model takes the GPU 4-7 us, and a ctypes call with its wrapper took 1.0-1.8 us of the
 // host's 4-5 beside the launch; parsed here it takes 0.3-0.5 us, most of it the data_ptr() of each tensor.
-// Arguments are what the wrappers took: positional or by name; a device buffer is None, an address or anything with
-// data_ptr(); the stream is an address, 0 by default.  A status other than 0 raises LlmHipError(status, name).
+// Arguments are positional or by name; a device buffer is None, an address or anything with data_ptr(); the stream is
+// None, an address (0 by default) or what ctypes takes for a void pointer, as the c_void_p that llmhip_stream_create
+// fills or a torch.cuda.Stream.  A status other than 0 raises LlmHipError(status, name).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -15,8 +16,10 @@ namespace {
 
 PyObject *g_error = nullptr;     // ops.LlmHipError
 PyObject *g_data_ptr = nullptr;  // "data_ptr"
+PyObject *g_cast = nullptr;      // ctypes.cast
+PyObject *g_void_p = nullptr;    // ctypes.c_void_p
 
-enum Kind : char { P = 'p', I = 'i', L = 'l', B = 'b' };  // buffer or stream, int, 64-bit int, truth value
+enum Kind : char { P = 'p', S = 's', I = 'i', L = 'l', B = 'b' };  // buffer, stream, int, 64-bit int, truth value
 
 struct Arg {
   const char *name;
@@ -34,19 +37,21 @@ bool to_value(PyObject *o, Kind kind, Value *out) {
     out->i = t;
     return t >= 0;
   }
-  if (kind == P && o == Py_None) {
+  if (kind == P || kind == S) {
     out->p = nullptr;
-    return true;
-  }
-  if (kind == P && !PyLong_Check(o)) {
-    PyObject *a = PyObject_CallMethodNoArgs(o, g_data_ptr);
-    if (!a) return false;
-    out->p = PyLong_AsVoidPtr(a);
-    Py_DECREF(a);
-    return !PyErr_Occurred();
-  }
-  if (kind == P) {
-    out->p = PyLong_AsVoidPtr(o);
+    if (o == Py_None) return true;
+    PyObject *a = o;
+    if (PyLong_Check(o)) {
+      Py_INCREF(a);
+    } else if (kind == P) {
+      a = PyObject_CallMethodNoArgs(o, g_data_ptr);
+    } else {
+      PyObject *handle = PyObject_CallFunctionObjArgs(g_cast, o, g_void_p, nullptr);
+      a = handle ? PyObject_GetAttrString(handle, "value") : nullptr;  // None for a null pointer
+      Py_XDECREF(handle);
+    }
+    if (a && a != Py_None) out->p = PyLong_AsVoidPtr(a);
+    Py_XDECREF(a);
     return !PyErr_Occurred();
   }
   out->i = PyLong_AsLongLong(o);
@@ -118,19 +123,19 @@ OPERATOR(hip_flash_attn_layer,
          llmhip_flash_attn(v[0].p, v[1].p, v[2].p, v[3].p, as_int(v[4]), as_int(v[5]), as_int(v[6]), as_int(v[7]),
                            as_int(v[8]), as_int(v[9]), v[10].p),
          {"output_dev", P}, {"q_dev", P}, {"k_dev", P}, {"v_dev", P}, {"m", I}, {"n", I}, {"offset", I},
-         {"head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", P})
+         {"head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_flash_attn_gqa_layer,
          llmhip_flash_attn_gqa(v[0].p, v[1].p, v[2].p, v[3].p, as_int(v[4]), as_int(v[5]), as_int(v[6]), as_int(v[7]),
                                as_int(v[8]), as_int(v[9]), as_int(v[10]), v[11].p),
          {"output_dev", P}, {"q_dev", P}, {"k_dev", P}, {"v_dev", P}, {"m", I}, {"n", I}, {"offset", I},
-         {"group_size", I}, {"kv_head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", P})
+         {"group_size", I}, {"kv_head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_flash_attn_opt_prefill_layer,
          llmhip_flash_attn_opt_prefill(v[0].p, v[1].p, v[2].p, v[3].p, as_int(v[4]), as_int(v[5]), as_int(v[6]),
                                        as_int(v[7]), as_int(v[8]), as_int(v[9]), v[10].p),
          {"output_dev", P}, {"q_dev", P}, {"k_dev", P}, {"v_dev", P}, {"m", I}, {"n", I}, {"offset", I},
-         {"head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", P})
+         {"head_num", I}, {"head_dim", I}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_flash_decode_gqa_layer,
          llmhip_flash_decode_gqa(v[0].p, v[1].p, v[2].p, v[3].p, v[4].p, (size_t)v[5].i, as_int(v[6]), as_int(v[7]),
@@ -138,7 +143,7 @@ OPERATOR(hip_flash_decode_gqa_layer,
                                  v[14].p),
          {"output_dev", P}, {"q_dev", P}, {"k_cache_dev", P}, {"v_cache_dev", P}, {"workspace_dev", P},
          {"workspace_bytes", L}, {"batch", I}, {"n", I}, {"kv_seq_stride", L}, {"group_size", I}, {"kv_head_num", I},
-         {"head_dim", I}, {"num_splits", I}, {"dt", I}, {"stream", P})
+         {"head_dim", I}, {"num_splits", I}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_flash_decode_gqa_static_layer,
          llmhip_flash_decode_gqa_static(v[0].p, v[1].p, v[2].p, v[3].p, as_int(v[4]), as_int(v[5]), v[6].i,
@@ -146,47 +151,47 @@ OPERATOR(hip_flash_decode_gqa_static_layer,
                                         v[12].p),
          {"output_dev", P}, {"q_dev", P}, {"k_cache_dev", P}, {"v_cache_dev", P}, {"batch", I}, {"n", I},
          {"kv_seq_stride", L}, {"group_size", I}, {"kv_head_num", I}, {"head_dim", I}, {"num_splits", I}, {"dt", I},
-         {"stream", P})
+         {"stream", S})
 
 OPERATOR(hip_decode_step_gqa_layer,
          llmhip_decode_step_gqa(v[0].p, v[1].p, v[2].p, v[3].p, v[4].p, v[5].p, v[6].p, as_int(v[7]), as_int(v[8]),
                                 as_int(v[9]), as_int(v[10]), as_int(v[11]), as_int(v[12]), v[13].p),
          {"output_dev", P}, {"k_cache_dev", P}, {"v_cache_dev", P}, {"freqs_cis_dev", P}, {"input_q_dev", P},
          {"input_k_dev", P}, {"input_v_dev", P}, {"pos", I}, {"group_size", I}, {"kv_head_num", I}, {"head_dim", I},
-         {"is_neox_style", B}, {"dt", I}, {"stream", P})
+         {"is_neox_style", B}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_matmul_layer,
          llmhip_matmul(v[0].p, v[1].p, v[2].p, as_int(v[3]), as_int(v[4]), as_int(v[5]), as_int(v[6]), v[7].p),
-         {"output_dev", P}, {"lhs_dev", P}, {"weight_dev", P}, {"m", I}, {"n", I}, {"k", I}, {"dt", I}, {"stream", P})
+         {"output_dev", P}, {"lhs_dev", P}, {"weight_dev", P}, {"m", I}, {"n", I}, {"k", I}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_matmul_bias_layer,
          llmhip_matmul_bias(v[0].p, v[1].p, v[2].p, v[3].p, as_int(v[4]), as_int(v[5]), as_int(v[6]), as_int(v[7]),
                             v[8].p),
          {"output_dev", P}, {"lhs_dev", P}, {"weight_dev", P}, {"bias_dev", P}, {"m", I}, {"n", I}, {"k", I},
-         {"dt", I}, {"stream", P})
+         {"dt", I}, {"stream", S})
 
 OPERATOR(hip_add_layer, llmhip_add(v[0].p, v[1].p, v[2].p, v[3].i, as_int(v[4]), v[5].p),
-         {"output_dev", P}, {"lhs_dev", P}, {"rhs_dev", P}, {"total_size", L}, {"dt", I}, {"stream", P})
+         {"output_dev", P}, {"lhs_dev", P}, {"rhs_dev", P}, {"total_size", L}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_rope_layer,
          llmhip_rope(v[0].p, v[1].p, v[2].p, v[3].p, v[4].p, as_int(v[5]), as_int(v[6]), as_int(v[7]), as_int(v[8]),
                      as_int(v[9]), as_int(v[10]), v[11].p),
          {"output_q_dev", P}, {"output_k_dev", P}, {"freqs_cis_dev", P}, {"input_q_dev", P}, {"input_k_dev", P},
          {"start_pos", I}, {"cur_size", I}, {"n_heads", I}, {"hidden_dim", I}, {"is_neox_style", B}, {"dt", I},
-         {"stream", P})
+         {"stream", S})
 
 OPERATOR(hip_rope_single_layer,
          llmhip_rope_single(v[0].p, v[1].p, v[2].p, as_int(v[3]), as_int(v[4]), as_int(v[5]), as_int(v[6]),
                             as_int(v[7]), as_int(v[8]), v[9].p),
          {"output_x_dev", P}, {"freqs_cis_dev", P}, {"input_x_dev", P}, {"start_pos", I}, {"cur_size", I},
-         {"n_heads", I}, {"hidden_dim", I}, {"is_neox_style", B}, {"dt", I}, {"stream", P})
+         {"n_heads", I}, {"hidden_dim", I}, {"is_neox_style", B}, {"dt", I}, {"stream", S})
 
 OPERATOR(hip_rope_kv_append_layer,
          llmhip_rope_kv_append(v[0].p, v[1].p, v[2].p, v[3].p, v[4].p, v[5].p, v[6].p, as_int(v[7]), as_int(v[8]),
                                as_int(v[9]), as_int(v[10]), as_int(v[11]), as_int(v[12]), as_int(v[13]), v[14].p),
          {"output_q_dev", P}, {"k_cache_dev", P}, {"v_cache_dev", P}, {"freqs_cis_dev", P}, {"input_q_dev", P},
          {"input_k_dev", P}, {"input_v_dev", P}, {"start_pos", I}, {"cur_size", I}, {"n_heads", I}, {"n_kv_heads", I},
-         {"head_dim", I}, {"is_neox_style", B}, {"dt", I}, {"stream", P})
+         {"head_dim", I}, {"is_neox_style", B}, {"dt", I}, {"stream", S})
 
 PyObject *set_error(PyObject *, PyObject *cls) {
   Py_INCREF(cls);
@@ -253,7 +258,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_operators", "Operator calls of li
 }  // namespace
 
 PyMODINIT_FUNC PyInit__operators(void) {
+  PyObject *ctypes = PyImport_ImportModule("ctypes");
+  if (ctypes) {
+    g_cast = PyObject_GetAttrString(ctypes, "cast");
+    g_void_p = PyObject_GetAttrString(ctypes, "c_void_p");
+    Py_DECREF(ctypes);
+  }
   g_data_ptr = PyUnicode_InternFromString("data_ptr");
-  if (!g_data_ptr) return nullptr;
+  if (!g_cast || !g_void_p || !g_data_ptr) return nullptr;
   return PyModule_Create(&module);
 }
