@@ -69,13 +69,18 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
 /* How many bytes of the library's per-stream scratch buffer a llmhip_flash_attn* call with these
  * arguments uses (head_num of the MHA entry points = kv_head_num with group_size 1): the fp32
  * partials of the split-KV decode kernel (m * group_size <= 16) or of a key-range split of the
- * prefill kernel (a chunk of few rows over a cache at least 8 times longer); 0 for ordinary
- * prefill shapes.  The buffer is allocated on the first call that needs it on a stream (at least
- * 4 MiB) and replaced by a larger one when a later call needs more; a replaced buffer is kept, not
- * freed, so launches already queued and HIP graphs captured earlier keep a valid pointer.  All of
- * them go with llmhip_stream_destroy or llmhip_release_internal_workspace.  HIP graphs: a call made
- * while its stream is capturing cannot allocate and is refused with LLMHIP_ERR_WORKSPACE when the
- * buffer would have to grow -- warm the stream up with its largest shape before capturing. */
+ * prefill kernel (a chunk behind at least as many cached tokens, wherever the split is faster);
+ * 0 for ordinary prefill shapes.  The buffer is allocated on the first call that
+ * needs it on a stream (at least 4 MiB) and replaced by a larger one when a later
+ * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
+ * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or
+ * llmhip_release_internal_workspace.  HIP graphs: a call made while its stream is capturing cannot
+ * allocate; where the buffer would have to grow it runs with what there is, unsplit if need be, which can
+ * be slower -- warm the stream up with its largest shape before capturing.  Where that would be
+ * much slower it is refused with LLMHIP_ERR_WORKSPACE instead: one token over more than 384 keys
+ * (640 where there are 128 kv heads) and a chunk behind at least 2048 keys and 8 times its own
+ * length whose unsplit form would leave more than half of the device idle.  The same holds when
+ * the device is out of memory (the status is then hipMalloc's). */
 size_t llmhip_flash_attn_scratch_bytes(int m, int n, int offset, int group_size, int kv_head_num);
 
 /* Batched split-KV decode over a contiguous per-sequence KV cache: one query
@@ -87,8 +92,9 @@ size_t llmhip_flash_attn_scratch_bytes(int m, int n, int offset, int group_size,
  * The reference has no batch dimension and no split-KV (decode there is
  * npu_flash_attn_gqa_layer with m = 1, src/llama2_layer_npu.cpp:866-869);
  * for batch == 1 this call returns what llmhip_flash_attn_gqa(m=1,
- * offset=n-1) returns.  num_splits <= 0 picks llmhip_flash_decode_default_splits;
- * values above 256 are treated as 256.
+ * offset=n-1) returns.  num_splits <= 0 picks llmhip_flash_decode_default_splits, or
+ * over a short cache (see llmhip_flash_attn_scratch_bytes) fewer where the workspace holds
+ * fewer; values above 256 are treated as 256.
  * workspace: device memory of at least llmhip_flash_decode_workspace_bytes()
  * bytes, owned by the caller, so that the call allocates nothing. */
 int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,

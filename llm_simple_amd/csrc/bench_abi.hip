@@ -35,7 +35,7 @@ int llmhip_bench_flash_attn_gqa_clocked(void *out, const void *q, const void *k,
   if ((long long)m * group_size <= 16) return LLMHIP_ERR_UNSUPPORTED;  // prefill kernel only
   if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
   return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
-                                       static_cast<hipStream_t>(stream), nullptr, clock_probe));
+                                       static_cast<hipStream_t>(stream), clock_probe));
 }
 
 int llmhip_bench_mfma_ceiling(int mix, double target_ms, double *tflops) {

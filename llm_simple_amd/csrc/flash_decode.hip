@@ -660,11 +660,7 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus) {
   if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 2.3;
   return t + (s <= kMaxFoldSplits ? 3.1 : 2.3);
 }
-static int default_splits_model(long long pairs, int nblocks, int cus) {
-  int smax = flash_decode_max_default_splits(pairs);
-  if (smax > nblocks) smax = nblocks;
-  if (smax < 1) smax = 1;
-  auto model = [&](int s) { return split_model_us(pairs, nblocks, s, cus); };
+template <typename Model> static int best_splits(long long pairs, int smax, int cus, Model model) {
   double t_min = model(1);
   for (int s = 2; s <= smax; ++s) {
     const double t = model(s);
@@ -677,6 +673,12 @@ static int default_splits_model(long long pairs, int nblocks, int cus) {
     if ((pairs * s) % cus == 0) return s;
   }
   return first;
+}
+static int default_splits_model(long long pairs, int nblocks, int cus, int most) {
+  int smax = flash_decode_max_default_splits(pairs);
+  if (smax > nblocks) smax = nblocks;
+  if (smax > most) smax = most;
+  return best_splits(pairs, smax, cus, [&](int s) { return split_model_us(pairs, nblocks, s, cus); });
 }
 
 // The model is evaluated a few hundred times per call; a decode loop asks for the same (pairs, key
@@ -695,9 +697,39 @@ int flash_decode_default_splits(int batch, int n, int kv_head_num) {
   static thread_local unsigned next = 0;
   for (const Memo &e : memo)
     if (e.splits > 0 && e.pairs == pairs && e.nblocks == nblocks && e.cus == cus) return e.splits;
-  const int s = default_splits_model(pairs, nblocks, cus);
+  const int s = default_splits_model(pairs, nblocks, cus, kMaxSplits);
   memo[next++ % kMemo] = Memo{pairs, nblocks, cus, s};
   return s;
+}
+
+int flash_decode_splits_within(int batch, int n, int kv_head_num, size_t bytes) {
+  const int s = flash_decode_default_splits(batch, n, kv_head_num);
+  if (flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, s) <= bytes) return s;
+  int fits = s - 1;
+  while (fits > 1 && flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, fits) > bytes) --fits;
+  return default_splits_model((long long)batch * kv_head_num, (n + kDecStepKeys - 1) / kDecStepKeys,
+                              device_compute_units(), fits);
+}
+
+// What a call may insist on is counted with coarser figures than the default: 27.7 GB/s per CU in a full round and at most
+// 32 in a thin one, 3 us per workgroup, 5 for a fold.  Callers were promised that calls which are not worth a split by
+// these need no room; the promise does not move with the model above.
+size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
+  const long long pairs = (long long)batch * kv_head_num;
+  const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys, cus = device_compute_units();
+  int smax = flash_decode_max_default_splits(pairs);
+  if (smax > nblocks) smax = nblocks;
+  const int s = best_splits(pairs, smax, cus, [&](int splits) {
+    const long long full = pairs * splits / cus, rest = pairs * splits % cus;
+    const double kb = 2.0 * kRowBytes * kDecStepKeys * ((nblocks + splits - 1) / splits) * 1e-3;
+    double t = full * (kb / 27.7 + 3.0);
+    if (rest > 0) {
+      const double rate = 27.7 * cus / (double)rest;
+      t += kb / (rate > 32.0 ? 32.0 : rate) + 3.0;
+    }
+    return splits > 1 ? t + 5.0 : t;
+  });
+  return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, s);
 }
 
 int flash_decode_effective_splits(int num_splits, int n) {

@@ -956,6 +956,10 @@ struct PrefillPlan {
 };
 constexpr int kWholeRange = 0x7fffffc0;
 
+static size_t partial_bytes(long long splits, int m, long long H) {
+  return splits > 1 ? (size_t)splits * m * H * (kHeadDim + 2) * sizeof(float) : 0;
+}
+
 // A prompt (no more cached than new tokens) is never split: the fp32 partials would cost more HBM traffic than K and
 // V.  Which shape: while the chip is not full, the launch waits for the chain of the waves with the most
 // keys, so that as many waves as fit share every row block; once it is, the cheapest step wins.  Lines where the
@@ -982,9 +986,9 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 // many as are resident at once, 3 us and the traffic of the partials for the combine launch, K and V at 5.7 TB/s as
 // the floor.  Over the measured shapes that is the fastest combination or within 11 % of it (1 % on
 // average).  Among combinations within 4 % of the cheapest one that reads K and V once and gives every CU the same
-// number of workgroups is preferred.  Some of what it changed (us, before / now): 3 tokens over 3000 keys 29.3 / 10.3, 20 over 600 11.5 / 8.7,
+// number of workgroups is preferred.  Only those whose partials fit max_bytes are looked at; an unsplit one always does.  Some of what it changed (us, before / now): 3 tokens over 3000 keys 29.3 / 10.3, 20 over 600 11.5 / 8.7,
 // 130 over 2000 27.9 / 18.2, 200 over 16001 63.0 / 60.4 (28 heads); 300 over 30000, 40 heads, 232 / 199.
-static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int Hkv, int cus) {
+static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int Hkv, int cus, size_t max_bytes) {
   PrefillPlan best = {kPair64, false, 1, kWholeRange};
   double best_us = 1e30;
   const double floor_us = 2.0 * n_vis * Hkv * kRowBytes / 5.7e6 + 1.8;
@@ -999,6 +1003,7 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
         if (s > 1 && n_vis / s < 128) break;
         const long long chunk = s > 1 ? ((n_vis + s - 1) / s + 127) / 128 * 128 : n_vis;
         const long long splits = (n_vis + chunk - 1) / chunk;  // no empty trailing range
+        if (partial_bytes(splits, m, (long long)g * Hkv) > max_bytes) continue;
         const long long items = tiles * groups * splits, slots = (long long)cus * sh.per_cu;
         double busy = (double)items / cus;
         busy = sh.per_cu == 2 ? busy - 1 : busy * busy;
@@ -1027,28 +1032,50 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
 }
 
 // The last answers are kept per thread: every layer of a model asks for the same chunk (several hundred combinations).
-static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cus) {
+static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cus, size_t max_bytes) {
   const long long n_vis = ((long long)m + offset < n) ? (long long)m + offset : n;  // keys the last row sees
   if (n_vis < 2LL * m) return {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
   struct Memo {
     int m, n, offset, g, Hkv, cus;
+    size_t bytes, max_bytes;  // what the plan takes, what it was allowed
     PrefillPlan plan;
   };
   constexpr int kMemo = 8;
   static thread_local Memo memo[kMemo] = {};
   static thread_local unsigned next = 0;
-  for (const Memo &e : memo)
-    if (e.m == m && e.n == n && e.offset == offset && e.g == g && e.Hkv == Hkv && e.cus == cus) return e.plan;
-  const PrefillPlan pl = chunk_plan(m, n_vis, n_vis - m, g, Hkv, cus);
-  memo[next++ % kMemo] = Memo{m, n, offset, g, Hkv, cus, pl};
+  for (const Memo &e : memo)  // (the cheapest plan of a larger allowance that fits this one is the cheapest here)
+    if (e.m == m && e.n == n && e.offset == offset && e.g == g && e.Hkv == Hkv && e.cus == cus &&
+        e.bytes <= max_bytes && max_bytes <= e.max_bytes)
+      return e.plan;
+  const PrefillPlan pl = chunk_plan(m, n_vis, n_vis - m, g, Hkv, cus, max_bytes);
+  memo[next++ % kMemo] = Memo{m, n, offset, g, Hkv, cus, partial_bytes(pl.num_splits, m, (long long)g * Hkv), max_bytes, pl};
   return pl;
 }
 
 size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num) {
-  const int H = group_size * kv_head_num;
-  const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units());
-  if (pl.num_splits <= 1) return 0;
-  return (size_t)pl.num_splits * m * H * (kHeadDim + 2) * sizeof(float);
+  const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), ~(size_t)0);
+  return partial_bytes(pl.num_splits, m, (long long)group_size * kv_head_num);
+}
+
+// Where a call may not do with less: a chunk behind at least 2048 keys and 8 times its own length whose unsplit form would
+// leave more than half of the chip idle.  The size is that of one round of workgroups with whole tiles of 128 or 256
+// rows.  This is what callers under graph capture were promised; it does not move with the plan above, so that a
+// better plan never turns a call away that ran before.
+size_t flash_prefill_least_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num) {
+  const long long n_vis = ((long long)m + offset < n) ? (long long)m + offset : n;
+  const long long cus = device_compute_units(), H = (long long)group_size * kv_head_num;
+  if (n_vis < 8LL * m || n_vis < 2048 || 2 * ((m + 255LL) / 256) * H >= 3 * cus) return 0;
+  const bool pack = group_size > 1 && m < 128;
+  const long long rows = pack ? (long long)m * group_size : m, groups = pack ? kv_head_num : H;
+  const int tile = rows >= 192 ? 256 : 128;
+  const long long wgs = (rows + tile - 1) / tile * groups;
+  long long splits = (tile == 256 ? cus : 2 * cus) / wgs;
+  if (splits > n_vis / 1024) splits = n_vis / 1024;
+  const long long most = wgs <= 2 ? kMaxPrefillSplits : kMaxPrefillSplits / 2;
+  if (splits > most) splits = most;
+  if (splits <= 1) return 0;
+  const long long chunk = ((n_vis + splits - 1) / splits + 127) / 128 * 128;
+  return partial_bytes((n_vis + chunk - 1) / chunk, m, H);
 }
 
 template <typename T> static hipError_t launch_prefill(const PrefillParams &p, PrefillKind kind, hipStream_t stream) {
@@ -1065,13 +1092,15 @@ template <typename T> static hipError_t launch_prefill(const PrefillParams &p, P
 #ifdef LLMHIP_BENCH
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *workspace, void *clock_probe) {
+                                hipStream_t stream, void *clock_probe) {
+  void *const workspace = nullptr;
+  size_t workspace_bytes = 0;
   PrefillParams p;
   p.clock_probe = static_cast<unsigned long long *>(clock_probe);
 #else
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *workspace) {
+                                hipStream_t stream, void *workspace, size_t workspace_bytes) {
   PrefillParams p;
 #endif
   p.q = static_cast<const char *>(q);
@@ -1085,9 +1114,8 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   p.Hkv = kv_head_num;
   p.H = group_size * kv_head_num;
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
-  PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units());
-  if (pl.num_splits > 1 && !workspace)  // no scratch offered: run unsplit (and unpacked)
-    pl = {prompt_kind(m, n, p.H, device_compute_units()), false, 1, kWholeRange};
+  const PrefillPlan pl =
+      plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), workspace ? workspace_bytes : 0);
   p.pack = pl.pack ? 1 : 0;
   p.num_splits = pl.num_splits;
   p.chunk = pl.chunk;

@@ -9,19 +9,21 @@
 
 namespace LLMHIP_NS {
 
-// workspace: device memory of flash_prefill_workspace_bytes() bytes (0 = none needed) for the fp32
-// partials of a key-range split; with a null workspace the call runs unsplit.
+// workspace, workspace_bytes: device memory for the fp32 partials of a key-range split; the call takes the fastest
+// plan that fits (null: unsplit).  flash_prefill_workspace_bytes: what the fastest plan of all takes (0: none needed);
+// flash_prefill_least_workspace_bytes: below this a call with no way to get more is to be refused.
 size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num);
+size_t flash_prefill_least_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num);
 #ifdef LLMHIP_BENCH
-// The measurement library's copy: clock_probe is a device pointer to two 64-bit counters that
+// The measurement library's copy, never split: clock_probe is a device pointer to two 64-bit counters that
 // workgroup 0 fills with the shader-clock ticks and the reference-clock ticks of its lifetime.
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *workspace, void *clock_probe);
+                                hipStream_t stream, void *clock_probe);
 #else
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *workspace = nullptr);
+                                hipStream_t stream, void *workspace, size_t workspace_bytes);
 #endif
 
 // Compute units of the current device, cached per device; 256 when no device can be asked.
@@ -32,6 +34,10 @@ size_t flash_decode_workspace_bytes(int batch, int m, int group_size, int kv_hea
                                     int num_splits);
 int flash_decode_default_splits(int batch, int n, int kv_head_num);
 int flash_decode_max_default_splits(long long pairs);
+// The best count whose partials fit `bytes`; the size below which a call that leaves the count to the
+// library and has no way to get more is to be refused.
+int flash_decode_splits_within(int batch, int n, int kv_head_num, size_t bytes);
+size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num);
 // The split count a launch really uses for n keys: at most one split per block of 128 keys.
 int flash_decode_effective_splits(int num_splits, int n);
 hipError_t launch_flash_decode(void *out, const void *q, const void *k, const void *v,

@@ -38,24 +38,45 @@ struct StreamScratch {
 std::mutex g_scratch_mu;
 std::map<void *, StreamScratch> g_scratch;
 
-// Caller holds g_scratch_mu.  Growing allocates, which a stream under capture must not do: such a
-// call is refused with LLMHIP_ERR_WORKSPACE (warm the stream up with its largest shape first).
-int scratch_for_locked(void *stream, size_t need, void **out) {
+// hipMalloc that another stream's capture does not forbid.
+hipError_t scratch_malloc(void **ptr, size_t bytes) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const hipError_t e = hipMalloc(ptr, bytes);
+  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (e != hipSuccess) (void)hipGetLastError();  // handled here: not for the next launch to report
+  return e;
+}
+
+// The stream's scratch for a call whose fastest form takes `need` bytes and that is to run with no less than least().
+// Where the buffer cannot grow -- its stream is under capture, which must not allocate, or the device is full -- the
+// call gets what there is; only if that is less than least() is it refused (LLMHIP_ERR_WORKSPACE under capture:
+// warm the stream up with its largest shape first).  Caller holds g_scratch_mu.
+template <typename Least> int scratch_for_locked(void *stream, size_t need, Least least, StreamScratch **out) {
   StreamScratch &s = g_scratch[stream];
-  if (s.bytes < need) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess) (void)hipGetLastError();
-    if (cap != hipStreamCaptureStatusNone) return LLMHIP_ERR_WORKSPACE;
-    size_t want = need < (size_t)(4u << 20) ? (size_t)(4u << 20) : need;
-    void *fresh = nullptr;
-    hipError_t e = hipMalloc(&fresh, want);
-    if (e != hipSuccess) return (int)e;
-    if (s.ptr) s.retired.push_back(s.ptr);
-    s.ptr = fresh;
-    s.bytes = want;
+  *out = &s;
+  if (s.bytes >= need) return LLMHIP_OK;
+  const size_t fewest = least();
+  int refused = LLMHIP_ERR_WORKSPACE;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess) (void)hipGetLastError();
+  if (cap == hipStreamCaptureStatusNone) {
+    const size_t wanted[] = {need < (size_t)4 << 20 ? (size_t)4 << 20 : need, need, fewest};
+    for (size_t want : wanted) {
+      if (want <= s.bytes) continue;
+      void *fresh = nullptr;
+      const hipError_t e = scratch_malloc(&fresh, want);
+      if (e != hipSuccess) {
+        refused = (int)e;
+        continue;
+      }
+      if (s.ptr) s.retired.push_back(s.ptr);
+      s.ptr = fresh;
+      s.bytes = want;
+      return LLMHIP_OK;
+    }
   }
-  *out = s.ptr;
-  return LLMHIP_OK;
+  return s.bytes >= fewest ? LLMHIP_OK : refused;
 }
 
 int attn_common(void *out, const void *q, const void *k, const void *v, int m, int n,
@@ -72,15 +93,17 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     // few query rows: stream the cache once with the split-KV kernel
     const int n_vis = (n < m + offset) ? n : m + offset;  // keys any row can see
     int splits = flash_decode_default_splits(1, n_vis, kv_head_num);
-    void *ws = nullptr;
     const size_t need = flash_decode_workspace_bytes(1, m, group_size, kv_head_num, splits);
     if (!need)
       return from_hip(launch_flash_decode(out, q, k, v, nullptr, 1, m, n_vis, offset, n_vis, group_size,
                                           kv_head_num, splits, dt, as_stream(stream)));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    int rc = scratch_for_locked(stream, need, &ws);
+    StreamScratch *ws = nullptr;
+    int rc = scratch_for_locked(
+        stream, need, [&] { return flash_decode_least_workspace_bytes(1, n_vis, kv_head_num); }, &ws);
     if (rc != LLMHIP_OK) return rc;
-    return from_hip(launch_flash_decode(out, q, k, v, ws, 1, m, n_vis, offset, n_vis,
+    if (ws->bytes < need) splits = flash_decode_splits_within(1, n_vis, kv_head_num, ws->bytes);
+    return from_hip(launch_flash_decode(out, q, k, v, ws->ptr, 1, m, n_vis, offset, n_vis,
                                         group_size, kv_head_num, splits, dt,
                                         as_stream(stream)));
   }
@@ -89,13 +112,14 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
   const size_t need = flash_prefill_workspace_bytes(m, n, offset, group_size, kv_head_num);
   if (!need)
     return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
-                                         as_stream(stream)));
+                                         as_stream(stream), nullptr, 0));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  void *ws = nullptr;
-  int rc = scratch_for_locked(stream, need, &ws);
+  StreamScratch *ws = nullptr;
+  int rc = scratch_for_locked(
+      stream, need, [&] { return flash_prefill_least_workspace_bytes(m, n, offset, group_size, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
   return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
-                                       as_stream(stream), ws));
+                                       as_stream(stream), ws->ptr, ws->bytes));
 }
 
 }  // namespace
@@ -157,10 +181,17 @@ int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,
   if (!dtype_ok(dt)) return LLMHIP_ERR_INVALID_ARG;
   if (head_dim != 128 || group_size > kMaxDecodeCols) return LLMHIP_ERR_UNSUPPORTED;
   if (batch > 65535 || kv_head_num > 65535) return LLMHIP_ERR_UNSUPPORTED;
-  if (num_splits <= 0) num_splits = flash_decode_default_splits(batch, n, kv_head_num);
+  const size_t room = workspace ? workspace_bytes : 0;
+  if (num_splits <= 0) {
+    // the default count, or the best one the workspace holds, unless that is less than a call may insist on
+    num_splits = flash_decode_default_splits(batch, n, kv_head_num);
+    if (flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits) > room &&
+        flash_decode_least_workspace_bytes(batch, n, kv_head_num) <= room)
+      num_splits = flash_decode_splits_within(batch, n, kv_head_num, room);
+  }
   if (num_splits > kMaxDecodeSplits) num_splits = kMaxDecodeSplits;  // the combine kernel's limit
   const size_t need = flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits);
-  if (need && (!workspace || workspace_bytes < need)) return LLMHIP_ERR_WORKSPACE;
+  if (need > room) return LLMHIP_ERR_WORKSPACE;
   return from_hip(launch_flash_decode(out, q, k_cache, v_cache, workspace, batch, 1, n, n - 1,
                                       kv_seq_stride, group_size, kv_head_num, num_splits, dt,
                                       as_stream(stream)));
@@ -205,17 +236,19 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
   if (head_dim != 128 || group_size > kMaxDecodeCols) return LLMHIP_ERR_UNSUPPORTED;
   if (kv_head_num > 65535) return LLMHIP_ERR_UNSUPPORTED;
   const int n = pos + 1;
-  const int splits = flash_decode_default_splits(1, n, kv_head_num);
+  int splits = flash_decode_default_splits(1, n, kv_head_num);
   const size_t need = flash_decode_workspace_bytes(1, 1, group_size, kv_head_num, splits);
   if (!need)
     return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, nullptr, pos,
                                              group_size, kv_head_num, is_neox_style, splits, dt,
                                              as_stream(stream)));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  void *ws = nullptr;
-  int rc = scratch_for_locked(stream, need, &ws);
+  StreamScratch *ws = nullptr;
+  int rc = scratch_for_locked(
+      stream, need, [&] { return flash_decode_least_workspace_bytes(1, n, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
-  return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, ws, pos, group_size,
+  if (ws->bytes < need) splits = flash_decode_splits_within(1, n, kv_head_num, ws->bytes);
+  return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, ws->ptr, pos, group_size,
                                            kv_head_num, is_neox_style, splits, dt, as_stream(stream)));
 }
 
