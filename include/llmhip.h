@@ -69,9 +69,9 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
 /* How many bytes of the library's per-stream scratch buffer a llmhip_flash_attn* call with these
  * arguments uses (head_num of the MHA entry points = kv_head_num with group_size 1): the fp32
  * partials of the split-KV decode kernel (m * group_size <= 16) or of a key-range split of the
- * prefill kernel (a chunk behind at least as many cached tokens, wherever the split is faster);
- * 0 for ordinary prefill shapes.  The buffer is allocated on the first call that
- * needs it on a stream (at least 4 MiB) and replaced by a larger one when a later
+ * prefill kernel (a chunk behind at least as many cached tokens, wherever the split is faster; at
+ * most 256 MiB); 0 for ordinary prefill shapes.  The buffer is allocated on the first call that
+ * needs it on a stream (a power of two, at least 4 MiB) and replaced by a larger one when a later
  * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
  * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or
  * llmhip_release_internal_workspace.  HIP graphs: a call made while its stream is capturing cannot

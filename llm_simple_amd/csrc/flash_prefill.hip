@@ -956,6 +956,12 @@ struct PrefillPlan {
 };
 constexpr int kWholeRange = 0x7fffffc0;
 
+// The most scratch a plan may ask for.  Without a bound it grows with the chunk (behind 131072
+// keys 7151 tokens of 28 heads 521 MB, 30000 of 40 1248).  By the model below 256 MiB costs at most 2.3 % behind up to 32768 keys and 6 % up to 131072; half of it would be
+// felt: 4885 tokens of 28 heads behind 31258 keys take 2122 us with 213 MB and 2570 within 128 MiB, 4096 of 40 behind
+// 16384 1357 and 1415.
+constexpr size_t kMaxPrefillScratch = (size_t)256 << 20;
+
 static size_t partial_bytes(long long splits, int m, long long H) {
   return splits > 1 ? (size_t)splits * m * H * (kHeadDim + 2) * sizeof(float) : 0;
 }
@@ -1053,7 +1059,7 @@ static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cu
 }
 
 size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num) {
-  const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), ~(size_t)0);
+  const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), kMaxPrefillScratch);
   return partial_bytes(pl.num_splits, m, (long long)group_size * kv_head_num);
 }
 
@@ -1114,6 +1120,7 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   p.Hkv = kv_head_num;
   p.H = group_size * kv_head_num;
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
+  if (workspace_bytes > kMaxPrefillScratch) workspace_bytes = kMaxPrefillScratch;
   const PrefillPlan pl =
       plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), workspace ? workspace_bytes : 0);
   p.pack = pl.pack ? 1 : 0;

@@ -51,7 +51,9 @@ hipError_t scratch_malloc(void **ptr, size_t bytes) {
 // The stream's scratch for a call whose fastest form takes `need` bytes and that is to run with no less than least().
 // Where the buffer cannot grow -- its stream is under capture, which must not allocate, or the device is full -- the
 // call gets what there is; only if that is less than least() is it refused (LLMHIP_ERR_WORKSPACE under capture:
-// warm the stream up with its largest shape first).  Caller holds g_scratch_mu.
+// warm the stream up with its largest shape first).  Sizes are powers of two from 4 MiB on (the exact size where the
+// device has no room for that), so that the replaced buffers together are smaller than the one in use.
+// Caller holds g_scratch_mu.
 template <typename Least> int scratch_for_locked(void *stream, size_t need, Least least, StreamScratch **out) {
   StreamScratch &s = g_scratch[stream];
   *out = &s;
@@ -61,7 +63,9 @@ template <typename Least> int scratch_for_locked(void *stream, size_t need, Leas
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess) (void)hipGetLastError();
   if (cap == hipStreamCaptureStatusNone) {
-    const size_t wanted[] = {need < (size_t)4 << 20 ? (size_t)4 << 20 : need, need, fewest};
+    size_t grown = (size_t)4 << 20;
+    while (grown < need) grown *= 2;
+    const size_t wanted[] = {grown, need, fewest};
     for (size_t want : wanted) {
       if (want <= s.bytes) continue;
       void *fresh = nullptr;

@@ -165,3 +165,25 @@ def test_batched_decode_with_less_workspace_than_the_default_count_takes():
     args = (dq.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), None, 0)
     assert ops.lib.llmhip_flash_decode_gqa(*args, batch, n, n, g, Hkv, 128, 2, DT, None) == -3
     assert ops.lib.llmhip_flash_decode_gqa(*args, 1, 32768, 32768, 5, 8, 128, 0, DT, None) == -3
+
+
+def test_a_growing_buffer_stays_bounded():
+    """Chunks that need more and more: what the stream holds, replaced buffers included, stays under twice the power
+    of two that holds the largest, and goes with the stream."""
+    import torch
+    import llm_simple_amd.ops as ops
+    sizes = [(700, 1900, 12, 2), (700, 4000, 28, 4), (1500, 9000, 28, 4), (3000, 9000, 28, 4), (3000, 16384, 32, 32),
+             (3000, 16384, 28, 4)]
+    needs = [ops.lib.llmhip_flash_attn_scratch_bytes(m, m + p, p, H // Hkv, Hkv) for m, p, H, Hkv in sizes]
+    assert sorted(needs) == needs and sum(needs) > 256 << 20
+    q, k, v = (torch.zeros(r, h, 128, dtype=torch.int16, device="cuda") for r, h in ((3000, 32), (19384, 32), (19384, 32)))
+    out = dev_empty(q.shape)
+    with fresh_stream() as s:
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        for m, past, H, Hkv in sizes:
+            ops.hip_flash_attn_gqa_layer(out, q, k, v, m, m + past, past, H // Hkv, Hkv, 128, DT, s.cuda_stream)
+        s.synchronize()
+        held = free - torch.cuda.mem_get_info()[0]
+        assert max(needs) <= held < 256 << 20  # (128 MiB and the smaller powers of two)
+    assert free - torch.cuda.mem_get_info()[0] < 4 << 20
