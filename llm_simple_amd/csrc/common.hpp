@@ -80,13 +80,10 @@ template <> struct Elem<__bf16> {
   static __device__ __forceinline__ float widen(uint16_t bits) {
     return __builtin_bit_cast(float, ((uint32_t)bits) << 16);
   }
-  // Round to nearest even on the bit pattern; agrees with the reference's
-  // fp32_to_bfloat16 (src/util.cpp:33-72) on every finite input.
-  static __device__ __forceinline__ uint16_t round(float f) {
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-  }
+  // Round to nearest even by the conversion instruction; agrees with the reference's fp32_to_bfloat16
+  // (src/util.cpp:33-72) on every finite input, and a NaN stays one whatever its payload (added to the bit
+  // pattern, the rounding carries 0xFFFFFFFF over to 0).
+  static __device__ __forceinline__ uint16_t round(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 };
 
 // n / d for 32-bit n by multiply and shift (Granlund-Montgomery, round-up variant): exact for every n.
