@@ -6,7 +6,7 @@
 // (src/llama2_layer_cpu.cpp:687-701), scale = 1/sqrt(128) inside
 // (src/llama2_layer_cpu.cpp:177), query head h reading kv head h / group_size.
 //
-// Common to both kernels below.  A wave owns 32 query rows.  The scores are
+// Common to all workgroup shapes.  A wave owns 32 query rows.  The scores are
 // produced transposed, S^T = K Q^T, with mfma_f32_32x32x16: every lane then
 // holds 16 keys of ONE query column per 32-key block, so the softmax row
 // reductions are in-register plus one exchange with lane^32
@@ -482,7 +482,7 @@ template <int NW, int TN, bool NT> struct DirectLoader {
     }
   }
   // NT: the tile is read by this workgroup only (a packed chunk of one tile per kv head over a long
-  // cache): non-temporal, like the decode kernel's loads (4 tokens over 131072 keys: 106 -> 93 us);
+  // cache): non-temporal, like the decode kernel's loads (4 tokens over 131072 keys: 106 -> 91 us);
   // tiles that several workgroups read stay ordinary loads (non-temporal costs those 3-10 %).
   static __device__ __forceinline__ void dma(const char *tile_base, uint32_t lane_off, uint32_t lds_addr) {
     if (NT)
@@ -934,20 +934,22 @@ int device_compute_units() {
 // Kernel and key-range split of a call.
 // ---------------------------------------------------------------------------
 // The workgroup shapes, and what a launch of one costs on this part, in us: `fixed` per workgroup, a step over one
-// tile `step_free` on an otherwise empty chip and `step_full` with every CU busy (fitted over 13000 timed
-// launches: 204 shapes of 2-32 kv heads, 3-8192 tokens, 0-31000 cached keys, every shape and split).
+// tile `step_free` on an otherwise empty chip and `step_full` with every CU busy, up to `past_l2` times that once K and V
+// outgrow the L2s of the 8 XCDs together (32 to 48 MiB; 32 heads, kQuad64: 1.13 us a step at 2450 keys, 1.6 at 2900).  Fitted
+// over 13000 timed launches (204 shapes of 2-32 kv heads, 3-8192 tokens, 0-31000 cached keys, every shape and
+// split), and again over 180000 (1800 shapes of 1-32 kv heads, 2-3000 tokens, 200-131072 cached keys).
 enum PrefillKind { kPair64, kPair128, kRows128, kRows256, kQuad64, kQuad32, kPrefillKinds };
 struct PrefillShape {
   int rows, tile, per_cu;  // query rows, keys of a tile, workgroups resident on a CU
-  double fixed, step_free, step_full;
+  double fixed, step_free, step_full, past_l2;
 };
 static const PrefillShape kShapes[kPrefillKinds] = {
-    {64, 64, 2, 2.42, 0.74, 1.05},   // 4 waves, two per row block
-    {128, 64, 1, 3.92, 0.73, 0.85},  // 8 waves, two per row block
-    {128, 64, 2, 2.40, 1.10, 1.55},  // 4 waves
-    {256, 64, 1, 3.61, 1.12, 1.44},  // 8 waves
-    {64, 128, 1, 3.42, 1.03, 1.20},  // 8 waves, four per row block
-    {32, 128, 1, 2.99, 0.81, 1.03},  // 4 waves, four per row block
+    {64, 64, 2, 2.42, 0.74, 1.10, 1.5},   // 4 waves, two per row block
+    {128, 64, 1, 3.92, 0.73, 0.85, 1.3},  // 8 waves, two per row block
+    {128, 64, 2, 2.50, 1.10, 1.62, 1.3},  // 4 waves
+    {256, 64, 1, 3.00, 1.12, 1.44, 1.3},  // 8 waves
+    {64, 128, 1, 3.25, 1.03, 1.20, 1.5},  // 8 waves, four per row block
+    {32, 128, 1, 2.99, 0.81, 1.03, 1.4},  // 4 waves, four per row block
 };
 struct PrefillPlan {
   PrefillKind kind;
@@ -989,17 +991,27 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 // A chunk behind a longer cache makes few workgroups with many keys each: its key range is cut, and with fewer rows than a
 // tile has the g query heads of a kv head share a tile (K and V of the kv head are then read once, not g times).
 // Taken is the combination of shape, packing and cut that the costs above make cheapest: workgroups in rounds of as
-// many as are resident at once, 3 us and the traffic of the partials for the combine launch, K and V at 5.7 TB/s as
-// the floor.  Over the measured shapes that is the fastest combination or within 11 % of it (1 % on
-// average).  Among combinations within 4 % of the cheapest one that reads K and V once and gives every CU the same
-// number of workgroups is preferred.  Only those whose partials fit max_bytes are looked at; an unsplit one always does.  Some of what it changed (us, before / now): 3 tokens over 3000 keys 29.3 / 10.3, 20 over 600 11.5 / 8.7,
-// 130 over 2000 27.9 / 18.2, 200 over 16001 63.0 / 60.4 (28 heads); 300 over 30000, 40 heads, 232 / 199.
+// many as are resident at once, 2.65 us and the traffic of the partials for the combine launch.  Only combinations whose
+// partials fit max_bytes are looked at; an unsplit one always does.  Over the 1800 measured shapes the choice is 1.1 %
+// slower than the fastest combination on average, 4 % at the 90th percentile.  Among combinations within 4 % of the
+// cheapest one that reads K and V once and gives every CU the same number of workgroups is preferred.
+// Rows that fit one 256-row tile over a cache larger than the last-level cache are a stream from HBM: that tile's loads are
+// non-temporal then, and nothing else was faster (us, it / the best other one: 23 tokens over 68925 keys of 4 kv heads 49.6
+// / 54.3, 7 over 127579 of 8 90.9 / 98.8; below 256 MiB of K and V it no longer holds: 38 over 17018 of 8 36.6 / 31.2).
+// Against fixed rules (a cut for about one round of workgroups of 128 or 256 rows), us: 3 tokens over 3000 keys 28.9 /
+// 9.3, 20 over 600 11.5 / 8.5, 130 over 2000 28.0 / 16.8, 200 over 16001 63.0 / 58.3 (28 heads); 300 over 30000, 40 heads,
+// 227 / 175.  (1800 other shapes: 0.68 of the time of the fixed rules on average, 22 of them more than 2 % slower.)
 static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int Hkv, int cus, size_t max_bytes) {
   PrefillPlan best = {kPair64, false, 1, kWholeRange};
   double best_us = 1e30;
-  const double floor_us = 2.0 * n_vis * Hkv * kRowBytes / 5.7e6 + 1.8;
+  const double kv_bytes = 2.0 * n_vis * Hkv * kRowBytes;
+  double over = (kv_bytes / (1 << 20) - 32.0) / 16.0;  // how far K and V are past the L2s
+  over = over < 0 ? 0 : over > 1 ? 1 : over;
+  const bool streamed = kv_bytes > 256 << 20 && g > 1 && (long long)m * g <= kShapes[kRows256].rows &&
+                        partial_bytes(2, m, (long long)g * Hkv) <= max_bytes;
   for (int kind = 0; kind < kPrefillKinds; ++kind)
     for (int pack = 0; pack < (g > 1 ? 2 : 1); ++pack) {
+      if (streamed && !(kind == kRows256 && pack)) continue;
       const PrefillShape &sh = kShapes[kind];
       const long long rows = pack ? (long long)m * g : m, tiles = (rows + sh.rows - 1) / sh.rows;
       const long long groups = pack ? Hkv : (long long)Hkv * g;
@@ -1014,7 +1026,7 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
         double busy = (double)items / cus;
         busy = sh.per_cu == 2 ? busy - 1 : busy * busy;
         busy = busy < 0 ? 0 : busy > 1 ? 1 : busy;
-        const double step = sh.step_free + (sh.step_full - sh.step_free) * busy;
+        const double step = (sh.step_free + (sh.step_full - sh.step_free) * busy) * (1.0 + over * (sh.past_l2 - 1.0));
         const double most = (double)((chunk + sh.tile - 1) / sh.tile);
         double mean = keys / (splits * sh.tile) + 0.5;
         if (mean > most) mean = most;
@@ -1025,8 +1037,7 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
           if (all > us) us = all;
         }
         us += 1.8;
-        if (splits > 1) us += 3.0 + (double)splits * m * g * Hkv * (kHeadDim + 2) * sizeof(float) / 1.9e6;
-        if (us < floor_us + sh.fixed) us = floor_us + sh.fixed;
+        if (splits > 1) us += 2.65 + (double)splits * m * g * Hkv * (kHeadDim + 2) * sizeof(float) / 1.9e6;
         if (tiles == 1 && items % cus == 0) us *= 0.96;
         if (us < best_us) {
           best_us = us;

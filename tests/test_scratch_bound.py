@@ -12,3 +12,12 @@ def test_no_chunk_takes_more_than_256_mib(H, Hkv):
             assert need <= 256 << 20, (m, past, need)
             most = max(most, need)
     assert most > 16 << 20  # (long chunks still are cut)
+
+
+# 32 MiB of K and V are what the L2s hold: beyond, 64-row workgroups that all read everything take 62.7 us for 440 tokens
+# over 3694 keys of 32 heads, with the key range cut in two 45.5; below, uncut is the fastest (315 over 1615: 23.2 us)
+@pytest.mark.parametrize("m,past,H,Hkv,ranges", [(440, 3694, 32, 32, 2), (315, 1615, 32, 32, 1), (4, 131072, 40, 8, 32)])
+def test_cut_of_a_chunk(m, past, H, Hkv, ranges):
+    import llm_simple_amd.ops as ops
+    need = ops.lib.llmhip_flash_attn_scratch_bytes(m, m + past, past, H // Hkv, Hkv)
+    assert need == (0 if ranges == 1 else ranges * m * H * 130 * 4)
