@@ -1,5 +1,5 @@
 // Shared device helpers for the gfx950 attention kernels: 16-bit storage type
-// traits, MFMA wrappers, LDS swizzles and cross-lane exchanges.
+// traits, MFMA wrappers, LDS swizzles and division by a run-time constant.
 //
 // MFMA operand layouts used throughout (64-lane wavefront, lane l):
 //   32x32x16:  A[row = l%32][k = 8*(l/32) + e],  B[k = 8*(l/32) + e][col = l%32],
@@ -105,9 +105,6 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
   const uint32_t t = (uint32_t)(((uint64_t)n * f.m) >> 32);
   return (t + ((n - t) >> 1)) >> (f.l - 1);
 }
-
-// Exchange with the lane whose index differs in bit 5 / bit 4.
-__device__ __forceinline__ float xor_lane(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 

@@ -53,7 +53,6 @@
 
 namespace llmhip {
 
-constexpr int kDecThreads = 256;
 constexpr int kDecWaveKeys = 32;                  // keys per wave per step
 constexpr int kDecStepKeys = 4 * kDecWaveKeys;    // keys per workgroup per step (half of it in short caches)
 constexpr int kDecCols = 16;                      // query rows per kv head (MFMA N)
