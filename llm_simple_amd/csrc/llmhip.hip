@@ -439,12 +439,16 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
   if (m < 1 || n < 1 || k < 1 || !dtype_ok(dt)) return LLMHIP_ERR_INVALID_ARG;
   if (n % 16 != 0 || k % 16 != 0) return LLMHIP_ERR_UNSUPPORTED;
   // Up to 16 rows one MFMA column block holds every lhs row and the call is a read of W; beyond that lhs, which
-  // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  Both kernels move 16-byte
-  // pieces; hipBLASLt takes any base.
+  // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  From 9 rows on that is so already
+  // where W has more rows than one round of its workgroups takes, 16 per CU (W from HBM, us, few-row kernel /
+  // tiles: 5120 x 5120, 9 rows 17.1 / 15.4, 16 rows 21.0 / 16.0; 11008 x 4096, 16 rows 27.6 / 21.3; not so 4096 x 4096, 9
+  // rows 10.4 / 11.7, nor with 8 rows).  Both kernels move 16-byte pieces; hipBLASLt takes any base.
   if (all_aligned16(out, lhs, weight)) {
     const float *b = static_cast<const float *>(bias);
-    if (m <= 16) return from_hip(launch_matmul_skinny(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
-    if (matmul_tile_takes(m, n, k))
+    const bool tiles = m > 8 && matmul_tile_takes(m, n, k);
+    if (m <= 16 && !(tiles && n > 16LL * device_compute_units()))
+      return from_hip(launch_matmul_skinny(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
+    if (tiles)
       return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
   }
   return from_hip(launch_matmul_bias(out, lhs, weight, static_cast<const float *>(bias), m, n, k, dt,
