@@ -562,7 +562,7 @@ def layer_decode_loop(H=12, Hkv=2, prompt=256, gen=256):
 
 def bench_attention_block(ops, torch, timer, S, steps, warmup, H=28, Hkv=4):
     """The whole attention block of one Qwen2.5-7B layer (src/llama2_layer_npu.cpp:760-901):
-    q/k/v projections with fp32 bias (hipBLASLt), fused RoPE + KV append, causal attention, o_proj,
+    q/k/v projections with fp32 bias (tiles of the library or hipBLASLt, by size), fused RoPE + KV append, causal attention, o_proj,
     residual add -- random weights of that shape, one sequence of S tokens."""
     import numpy as np
     hidden, kvd = H * 128, Hkv * 128

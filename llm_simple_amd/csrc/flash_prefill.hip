@@ -388,8 +388,8 @@ template <typename T, int KB = 2> struct WaveAttn {
   // out[row][head][32*D0 .. +32*ND) = O^T / l, rounded once.  The lane layout of O^T (a lane holds 4
   // contiguous dims of one row at 4*ND places) would make every store instruction touch 32
   // rows with 16 bytes each; the tile goes through 2*ND KiB of LDS of this wave instead
-  // (16-byte granule XOR row: conflict-free both ways) and leaves as whole pieces of 64*ND bytes,
-  // 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the wave][head];
+  // (16-byte granule XOR row: conflict-free both ways with four d blocks; rows of one or two are shorter than the banks, and
+  // up to 8 lanes meet in one, 1-2 % of a launch's cycles) and leaves as whole pieces of 64*ND bytes, 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the wave][head];
   // rows_valid: how many of the wave's 32 rows exist.
   template <int D0 = 0, int ND = 4>
   __device__ __forceinline__ void store(char *lds_wave, char *out_blk, size_t row_bytes, int rows_valid) {

@@ -1,10 +1,11 @@
 // Projection of few rows (one generated token, a handful of tokens): out[m][n] = lhs[m][k] . W[n][k]^T + bias,
-// fp32 accumulation, one rounding, m <= 16.
+// fp32 accumulation, one rounding, m <= 16 (from 9 rows on only where W has at most 16 rows per CU: the tiled kernel is
+// faster beyond).
 //
 // Bound by reading W once.  W is dealt out in equal shares of whole rows (at most 16) to one workgroup per
 // CU, two or more rounds of them for a wide n: a CU cannot have more than its 32 KiB of first-level cache
 // in flight (about 30 GB/s), so a matrix is only read at full speed if every CU has the same share of it --
-// with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it takes 3.8.
+// with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it takes 4.2.
 // The eight waves of a workgroup deal k out among themselves, all loads of a wave are issued before its first
 // MFMA, and the partial sums meet in LDS.
 //

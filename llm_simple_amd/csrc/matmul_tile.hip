@@ -7,10 +7,13 @@
 // 3584, 2048 rows: 29.9 us against 14.3).  Eight waves: four quadrants of the tile, each shared by two waves that take 32 k
 // of every line, so that a SIMD always has two waves; their sums are traded through LDS at the end.  The fragments of
 // the next stage are read beside the MFMAs of this one, and loads and fragment reads are dealt out among the MFMAs
-// one by one: issued in a burst they held the matrix unit up (128 x 224 tile, k = 3584, 43.4 -> 34.7 us).
-// What bounds a tile now: its MFMAs (28 of 16x16x32 per wave and stage, 0.50 of 0.56 us), for small tiles the
-// rate at which one CU takes lines in, 60-80 KB/us, and the barrier and LDS latency of a stage (32 x 32: 0.09 us a line where
-// its MFMAs take 0.02; with two lines a stage 0.08, 512 x 3584, 100 rows: 8.0 -> 7.4 us; larger tiles gain nothing by it).
+// one by one: issued in a burst they held the matrix unit up (3584 x 3584, 2048 rows, W from HBM: 53.2 -> 50.4 us).
+// Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 3.0 until the first
+// lines are in, 56 stages of 0.69, 6.2 for the trade of the sums and the store, the rest launch.  A stage is 28 MFMAs of
+// 16x16x32 for each of a SIMD's two waves, 0.52 at the 1.72 GHz that they leave; with zeros for lhs the clock stays at
+// 2.28 GHz and a stage takes 0.51.  Small tiles are bound by the rate at which one CU takes lines in, 90-120 KB/us, and
+// the barrier and LDS latency of a stage: 64 x 64 1.5, 56 of 0.175, 1.3; 32 x 32 1.1, 56 lines of 0.07 where their MFMAs take
+// 0.02, 0.4 (two lines a stage: 512 x 3584, 100 rows 8.0 -> 7.4; larger tiles gain nothing by it).
 //
 // Rows of the operands lie k elements apart, often a multiple of 4 KiB: workgroups that walk k in step would ask few
 // memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
@@ -223,7 +226,12 @@ template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_
 // rows (78 % busy) 51.5 us against 53.7, 768 rows (94 %) 53.3 / 53.2, 900 rows (100 %) 62.6 / 56.9.  Not so up to k = 2048,
 // where the start of a workgroup weighs more: 1536 x 1536, 768 rows (56 %) 12.4 / 11.2.  And from 128 x 192 on where rows are a
 // multiple of 4 KiB apart: 4096 x 4096, 1280 rows 46.6 / 47.6, 1500 rows 49.7 / 53.7, against 3584 x 3584, 1500 rows 44.2 /
-// 42.7, 2048 rows 52.4 / 50.7.
+// 42.7, 2048 rows 52.4 / 50.7; 8192 x 8192, 2000 rows 175 / 182.
+// hipBLASLt's time is no smooth function of the rows, so that the two cross more often than these lines say.  Left to it
+// though tiles would be faster: 3584 x 3584, 257-288 rows 29.5 / 23.1, 577-672 32.0 / 29.6, 865-896 35.5 / 34.0; 4096 x 4096,
+// 513-576 rows 35.3 / 32.7; 1024 x 5120, 1025-1152 rows 28.3 / 26.6.  Taken though slower: 3584 x 3584, 784-864 rows 29.2 /
+// 31.5; 5120 x 5120, 64-80 rows 21.7 / 24.2, 257-272 30.9 / 33.2, 528-560 41.6 / 45.0; 1024 and 2048 x 8192, 17-32 rows
+// 11.7-16.2 / 18-22 (a quarter of the CUs, rows a multiple of 4 KiB apart).
 int tile_kind(int m, int n, int k) {
   static const struct { int m, n; } tiles[] = {{32, 32},  {64, 32},   {64, 64},   {96, 64},   {128, 64},  {96, 96},
                                                {96, 128}, {128, 128}, {128, 160}, {128, 192}, {128, 224}, {128, 256}};

@@ -14,7 +14,7 @@ CASES = [
     (97, 0, 28, 4), (129, 0, 12, 2), (257, 0, 12, 2),        # four waves per 32 rows
     (481, 0, 28, 4), (705, 0, 12, 2),                        # four waves per 64 rows
     (600, 0, 40, 8), (650, 0, 40, 8), (1100, 0, 40, 8),      # two waves per 64, per 128 rows
-    (1700, 0, 40, 8), (1801, 0, 40, 8),                      # 128 rows of one wave each; 256 rows
+    (1700, 0, 40, 8), (1801, 0, 40, 8), (1281, 0, 64, 2),    # 128 rows of one wave each, twice; 256 rows
     (3, 300, 28, 4), (9, 4000, 40, 8), (20, 1500, 32, 32), (65, 2000, 12, 2), (130, 3001, 28, 4), (150, 151, 12, 2),
     (300, 300, 40, 8), (300, 2500, 28, 4), (2, 10000, 64, 2), (1, 3000, 20, 1),
 ]

@@ -1,6 +1,6 @@
 """GPU parity of the projections either side of the attention block (through the C ABI):
-hipBLASLt GEMM with fp32 bias epilogue and the residual add, against the oracle's
-restatement of tests/gemm_test.cpp:138-149."""
+projection with the fp32 bias added before the rounding, by whichever kernel the sizes lead to (few rows, tiles,
+hipBLASLt for k in part lines), and the residual add, against the oracle's restatement of tests/gemm_test.cpp:138-149."""
 import numpy as np
 import pytest
 
@@ -77,11 +77,12 @@ def test_matmul_rejects_bad_arguments():
         ops.hip_matmul_layer(out, x, w, 0, 16, 32, DT_BFLOAT16)   # m < 1
 
 
-def test_release_then_reuse():
+@pytest.mark.parametrize("m,n,k", [(8, 64, 128), (33, 48, 272)])   # the few-row kernel; hipBLASLt
+def test_release_then_reuse(m, n, k):
     """llmhip_release_internal_workspace() drops the hipBLASLt handle, plans and workspace (and the
     decode scratch); the next call builds them again."""
     ops = _ops()
-    dt, m, n, k = DT_BFLOAT16, 8, 64, 128
+    dt = DT_BFLOAT16
     x = normal_bits(21, (m, k), dt)
     w = orc.round_to(orc.widen(normal_bits(22, (n, k), dt), dt) / np.sqrt(k), dt)
     ref = orc.widen(orc.matmul_bias(x, w, None, dt), dt)

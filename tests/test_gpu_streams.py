@@ -89,12 +89,13 @@ def test_graph_capture_and_replay():
 
 def test_scratch_does_not_grow_under_capture():
     """A reference-signature call whose per-stream scratch would have to grow while its stream is being captured
-    is refused with LLMHIP_ERR_WORKSPACE (growing allocates); after the stream has been warmed up with the shape,
-    the same call is captured, and replays give the eager result."""
+    is refused with LLMHIP_ERR_WORKSPACE (growing allocates), and the capture stays usable: what fits the buffer
+    is captured, and its replay gives the eager result."""
     import torch
     import llm_simple_amd.ops as ops
-    dt, H, Hkv, n = DT_BFLOAT16, 40, 8, 40000   # the default split count for this cache needs more than 4 MiB? no:
-    # 8 kv heads x 32 splits x 8320 bytes = 2.1 MB fits the first 4 MiB buffer, so ask for a chunk whose partials do not
+    dt, H, Hkv, n = DT_BFLOAT16, 40, 8, 40000
+    # a decode over this cache, 8 kv heads x 32 splits x 8320 bytes = 2.1 MB, fits the first 4 MiB buffer; so ask for a
+    # chunk whose partials do not
     m = 24                                        # 24 tokens over 40000 keys: key-range split, fp32 partials
     need = ops.lib.llmhip_flash_attn_scratch_bytes(m, n, n - m, H // Hkv, Hkv)
     assert need > (4 << 20), need
