@@ -388,9 +388,10 @@ template <typename T, int KB = 2> struct WaveAttn {
   // out[row][head][32*D0 .. +32*ND) = O^T / l, rounded once.  The lane layout of O^T (a lane holds 4
   // contiguous dims of one row at 4*ND places) would make every store instruction touch 32
   // rows with 16 bytes each; the tile goes through 2*ND KiB of LDS of this wave instead
-  // (16-byte granule XOR row: conflict-free both ways with four d blocks; rows of one or two are shorter than the banks, and
-  // up to 8 lanes meet in one, 1-2 % of a launch's cycles) and leaves as whole pieces of 64*ND bytes, 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the wave][head];
-  // rows_valid: how many of the wave's 32 rows exist.
+  // (16-byte granule XOR row: conflict-free both ways with four d blocks; rows of one or two are shorter
+  // than the banks, and up to 8 lanes meet in one, 1-2 % of a launch's cycles) and leaves as whole pieces of
+  // 64*ND bytes, 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the
+  // wave][head]; rows_valid: how many of the wave's 32 rows exist.
   template <int D0 = 0, int ND = 4>
   __device__ __forceinline__ void store(char *lds_wave, char *out_blk, size_t row_bytes, int rows_valid) {
     constexpr int G = 4 * ND, RB_ = G * 16, RPI = 64 / G;  // granules and bytes of a row, rows per instruction
@@ -958,10 +959,10 @@ struct PrefillPlan {
 };
 constexpr int kWholeRange = 0x7fffffc0;
 
-// The most scratch a plan may ask for.  Without a bound it grows with the chunk (behind 131072
-// keys 7151 tokens of 28 heads 521 MB, 30000 of 40 1248).  By the model below 256 MiB costs at most 2.3 % behind up to 32768 keys and 6 % up to 131072; half of it would be
-// felt: 4885 tokens of 28 heads behind 31258 keys take 2122 us with 213 MB and 2570 within 128 MiB, 4096 of 40 behind
-// 16384 1357 and 1415.
+// The most scratch a plan may ask for.  Without a bound it grows with the chunk (behind 131072 keys 7151 tokens of 28
+// heads 521 MB, 30000 of 40 1248).  By the model below 256 MiB costs at most 2.3 % behind up to 32768 keys and 6 % up
+// to 131072; half of it would be felt: 4885 tokens of 28 heads behind 31258 keys take 2122 us with 213 MB and 2570
+// within 128 MiB, 4096 of 40 behind 16384 1357 and 1415.
 constexpr size_t kMaxPrefillScratch = (size_t)256 << 20;
 
 static size_t partial_bytes(long long splits, int m, long long H) {
