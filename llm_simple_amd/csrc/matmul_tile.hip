@@ -3,26 +3,37 @@
 //
 // A workgroup computes one tile of 32*MT lhs rows x 32*NT features over all of k in stages of KS * 64 k (KS 128-byte
 // lines of every operand row).  Lines travel global -> LDS without registers, STAGES of them in flight or in use; a
-// fragment load straight into the operand layout, 16 rows by 64 bytes, ran at a third of the rate (512 x
-// 3584, 2048 rows: 29.9 us against 14.3).  Eight waves: four quadrants of the tile, each shared by two waves that take 32 k
-// of every line, so that a SIMD always has two waves; their sums are traded through LDS at the end.  The fragments of
-// the next stage are read beside the MFMAs of this one, and loads and fragment reads are dealt out among the MFMAs
-// one by one: issued in a burst they held the matrix unit up (3584 x 3584, 2048 rows, W from HBM: 53.2 -> 50.4 us).
-// Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 3.0 until the first
-// lines are in, 56 stages of 0.69, 6.2 for the trade of the sums and the store, the rest launch.  A stage is 28 MFMAs of
-// 16x16x32 for each of a SIMD's two waves, 0.52 at the 1.72 GHz that they leave; with zeros for lhs the clock stays at
-// 2.28 GHz and a stage takes 0.51.  Small tiles are bound by the rate at which one CU takes lines in, 90-120 KB/us, and
-// the barrier and LDS latency of a stage: 64 x 64 1.5, 56 of 0.175, 1.3; 32 x 32 1.1, 56 lines of 0.07 where their MFMAs take
-// 0.02, 0.4 (two lines a stage: 512 x 3584, 100 rows 8.0 -> 7.4; larger tiles gain nothing by it).
+// fragment load straight into the operand layout, 16 rows by 64 bytes, ran at a third of the rate.
+// Four waves, one per SIMD, take a quadrant each.  A wave issues one instruction every 4-5 cycles and an MFMA takes
+// 16, so that two others fit between two MFMAs: the loop is written as slots, one MFMA and at most a fragment read
+// and a line load each, and a line load is one instruction (constant lane offsets, the LDS address in M0 for four of
+// them at a time).  The loads of a stage are spread over its whole length: a CU takes in 64 bytes per cycle and no more
+// (128 x 224: 704 cycles of loads beside 896 of MFMAs), and loads issued over half a stage held the wave up for the
+// other half (3584 x 3584, 2048 rows: loop 41.3 -> 39.0 us).  One barrier a stage, where the last fragments of this
+// stage have come back: it frees the stage's place and publishes the next one.
+//   Eight waves, two for each quadrant on alternate halves of k, hide more latency but trade their sums through LDS
+// at the end and issue more: 3584 x 3584, 2048 rows 54.9 us, this kernel 46.2; 4096 x 4096 67.6 / 59.3; 1536 x 1536,
+// 2048 rows 17.5 / 13.7; 512 x 3584, 2048 rows 14.8 / 13.6.  mfma_32x32x16, with half the operand reads, is no
+// faster (4096 x 4096 62.3 / 57.9), the power it saves being small.
+//   Small tiles are bound by the barrier and the LDS latency of a stage, and take several lines per stage (32 x 32, four
+// lines instead of two: 512 x 3584, 400 rows 8.5 -> 7.8 us; 1536 x 1536, 100 rows 5.4 -> 4.9).
+// Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 2.6 until the first
+// lines are in, 56 stages of 0.67, 2.3 for the store (14.7 MB at once), the rest launch.  A stage takes 1120 cycles at
+// 1.68 GHz: the clock is what the power leaves (half of the chip: 1090 cycles at 2.2 GHz; without the line loads 1.9 GHz).
+//
+// A lane's accumulators are four features of one lhs row; W rows are dealt to LDS so that two neighbouring blocks make
+// them eight, and a store 16 bytes.  The bias goes to LDS ahead of the first lines: read from memory at the end it
+// was one round trip more per pair of blocks (epilogue 6.2 us in the kernel of eight waves).
 //
 // Rows of the operands lie k elements apart, often a multiple of 4 KiB: workgroups that walk k in step would ask few
 // memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
-// (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5).
+// (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5, kernel of eight waves).
 //
-// bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 13.2 / 11.0, 128 rows
-// 21.6 / 15.0, 256 rows 19.8 / 18.6, 768 rows 33.1 / 29.4, 2048 rows 52.3 / 49.6; 512 x 3584: 100 rows 11.1 / 7.5,
-// 2048 rows 17.7 / 14.4; 1536 x 1536: 128 rows 7.5 / 5.3; 5120 x 5120: 100 rows 24.3 / 22.1, 1280 rows 74.4 / 69.1.
+// bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 10.9 / 7.9, 128 rows
+// 18.0 / 10.4, 256 rows 16.9 / 13.4, 768 rows 29.1 / 23.4, 2048 rows 54.4 / 46.2; 512 x 3584: 100 rows 11.2 / 7.4,
+// 2048 rows 17.1 / 13.6; 1536 x 1536: 128 rows 7.6 / 5.3; 5120 x 5120: 100 rows 28.6 / 25.8, 1280 rows 77.4 / 61.2.
 #include <atomic>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -31,9 +42,10 @@ namespace llmhip {
 
 namespace {
 
-constexpr int kTileWaves = 8;
+constexpr int kTileThreads = 256;
 constexpr int kLineK = 64;             // k of a 128-byte line of an operand row
 constexpr int kStageRow = 2 * kLineK;  // its bytes
+constexpr int kBiasBytes = 4 * 512;    // LDS: bias of each wave's features
 
 struct TileParams {
   const char *x, *w;
@@ -51,14 +63,26 @@ template <int N> __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
 }
 
+template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>());
+    static_for<I + 1, N>(f);
+  }
+}
+
+// global_load_lds_dwordx4, OFF (0, 1024, 2048 or 3072) added to the global address and to the LDS address in M0, which
+// nothing but the assembly of this kernel writes
+template <int OFF> __device__ __forceinline__ void line_load(uint32_t voff, const char *base) {
+  if constexpr (OFF == 0) asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base));
+  else asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(base), "n"(OFF));
+}
+
 template <typename T, int MT, int NT, int KS, int STAGES>
-__global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TileParams p) {
+__global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams p) {
   using E = Elem<T>;
-  constexpr int BM = 32 * MT, BN = 32 * NT, NW = kTileWaves, F = MT * NT, HALF = (F + 1) / 2;
-  constexpr int kLineBytes = (BM + BN) * kStageRow;       // one line of every row: W rows, then lhs rows
-  constexpr int kStageBytes = KS * kLineBytes;
-  constexpr int kInstr = (BM + BN) / 8;                   // an instruction fetches 8 rows
-  constexpr int L = (kInstr + NW - 1) / NW;               // of a wave per line
+  constexpr int BM = 32 * MT, BN = 32 * NT;
+  constexpr int kLineBytes = (BM + BN) * kStageRow, kStageBytes = KS * kLineBytes;
+  constexpr int L = MT + NT;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i = lane & 15, cg = lane >> 4;
@@ -71,107 +95,145 @@ __global__ __launch_bounds__(64 * kTileWaves, 2) void matmul_tile_kernel(TilePar
   const int rows_here = min(gm, p.m_tiles - band * gm);
   const int tn = rows_here == gm ? (int)fast_div(rem, p.band_rows) : rem / rows_here;
   const int m0 = (band * gm + rem - tn * rows_here) * BM, n0 = tn * BN;
+  const int wm = wave & 1, wn = wave >> 1;
+  const int col0 = n0 + wn * (BN / 2);
 
-  const size_t row_bytes = 2 * (size_t)p.k;
-  const char *base[L];
-  uint32_t voff[L], dst[L];
+  // Bias of the wave's features to LDS of its own (any fp32 address, so four bytes a lane)
+  const uint32_t bias_at = STAGES * kStageBytes + wave * 512;
+  if (p.bias) {
+#pragma unroll
+    for (int h = 0; h < (16 * NT + 63) / 64; ++h) {
+      const float *src = p.bias + min(col0 + 64 * h + lane, p.n - 1);
+      asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(bias_at + 256 * h) : "m0");
+    }
+  }
+
+  // Line loads of a wave: NT of 8 W rows each, then MT of 8 lhs rows, either run contiguous in LDS.  Staged W row
+  // 32b + 16c + 4q + j of a half (c: block of a pair) holds feature 32b + 8q + 4c + j.  Rows past the end: the last one.
+  const uint32_t row_bytes = 2 * (uint32_t)p.k;
+  uint32_t voff[L];
 #pragma unroll
   for (int s = 0; s < L; ++s) {
-    const int q = min(s * NW + wave, kInstr - 1);  // (a wave without an instruction of its own repeats the last)
-    const int row = 8 * q + (lane >> 3);
-    const bool is_w = 8 * q < BN;
-    const int r = is_w ? min(row, p.n - n0 - 1) : min(row - BN, p.m - m0 - 1);  // rows past the end: the last one
-    base[s] = is_w ? p.w + n0 * row_bytes : p.x + m0 * row_bytes;
-    voff[s] = (uint32_t)r * (uint32_t)row_bytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
-    dst[s] = __builtin_amdgcn_readfirstlane(q * 8 * kStageRow);
+    const bool is_w = s < NT;
+    const int nth = is_w ? s : s - NT, row = 8 * (is_w ? wave * NT + nth : wave * MT + nth) + (lane >> 3);
+    int r = row;
+    if (is_w) {
+      const int half = row >= BN / 2 ? BN / 2 : 0, in = row - half, blk = in >> 4;
+      if (blk < (NT & ~1)) r = half + (in & ~31) + 8 * ((in >> 2) & 3) + 4 * (blk & 1) + (in & 3);
+    }
+    r = min(r, is_w ? p.n - n0 - 1 : p.m - m0 - 1);
+    voff[s] = (uint32_t)r * row_bytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4) + 3072 - 1024 * (nth & 3);
   }
-  auto issue = [&](int s, int stage, uint32_t slot) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff[s]), "s"(base[s] + (size_t)stage * kStageRow), "s"(slot + dst[s])
-                 : "m0");
+  const char *wbase = p.w + n0 * (size_t)row_bytes - 3072, *xbase = p.x + m0 * (size_t)row_bytes - 3072;
+  const uint32_t wdst = __builtin_amdgcn_readfirstlane(wave * NT * 1024);
+  const uint32_t xdst = __builtin_amdgcn_readfirstlane(BN * kStageRow + wave * MT * 1024);
+  auto issue = [&](auto s_, const char *wk, const char *xk, uint32_t slot) {
+    constexpr int s = decltype(s_)::value;
+    constexpr bool is_w = s < NT;
+    constexpr int nth = is_w ? s : s - NT;
+    if constexpr (nth % 4 == 0)
+      asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0" : : "s"(slot + (is_w ? wdst : xdst)), "n"(nth * 1024) : "m0", "scc");
+    line_load<1024 * (nth % 4)>(voff[s], is_w ? wk : xk);
   };
+  const int lines = p.k / kLineK, stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
+  uint32_t kpos = (unsigned)(xcd * lines / 8 + (t & 3)) % (unsigned)lines * kStageRow;
+  auto advance = [&]() { kpos = kpos + kStageRow == row_bytes ? 0 : kpos + kStageRow; };
+#pragma unroll
+  for (int s = 0; s < STAGES * KS; ++s) {
+    static_for<0, L>([&](auto l) { issue(l, wbase + kpos, xbase + kpos, s * kLineBytes); });
+    advance();
+  }
 
-  const int wm = wave & 1, wn = (wave >> 1) & 1, kg = wave >> 2;
-  const int w_addr = stage_off(wn * (BN / 2) + i, 4 * kg + cg), x_addr = stage_off(BN + wm * (BM / 2) + i, 4 * kg + cg);
+  int w_addr[2], x_addr[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    w_addr[h] = stage_off(wn * (BN / 2) + i, 4 * h + cg);
+    x_addr[h] = stage_off(BN + wm * (BM / 2) + i, 4 * h + cg);
+  }
   f32x4_t acc[MT][NT];
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
     for (int b = 0; b < NT; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  // The fragments of stage s+1 are read while the MFMAs of stage s run, so that the place of stage s is free for
-  // stage s + STAGES as soon as every wave has come to the barrier.
-  const int lines = p.k / kLineK;
-  int kpos = (int)((unsigned)(xcd * lines / 8 + (t & 3)) % (unsigned)lines);
-  auto issue_line = [&](uint32_t place) {
-#pragma unroll
-    for (int l = 0; l < L; ++l) issue(l, kpos, place);
-    kpos = kpos + 1 == lines ? 0 : kpos + 1;
-  };
-#pragma unroll
-  for (int s = 0; s < STAGES * KS; ++s) issue_line(s * kLineBytes);
   uint32_t slot = 0;
-  u32x4_t w0[KS][NT], x0[KS][MT], w1[KS][NT], x1[KS][MT];
-  auto step = [&](int line, const u32x4_t (&wf)[KS][NT], const u32x4_t (&xf)[KS][MT], u32x4_t (&wnext)[KS][NT],
-                  u32x4_t (&xnext)[KS][MT]) {
-    wait_loads<L * KS * (STAGES - 2)>();
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    const uint32_t fetch = slot;
-    slot = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
-#pragma unroll
-    for (int u = 0; u < KS; ++u) {
-      const bool have = KS == 1 || line + u < lines;  // (the last stage may hold surplus lines)
-#pragma unroll
-      for (int b = 0; b < (NT > L ? NT : L); ++b) {
-        if (b < L) issue(b, kpos, fetch + u * kLineBytes);
-        if (b < NT) wnext[u][b] = lds_read_b128(lds, w_addr + slot + u * kLineBytes + b * 16 * kStageRow);
-#pragma unroll
-        for (int a = b; a < MT; a += NT)
-          xnext[u][a] = lds_read_b128(lds, x_addr + slot + u * kLineBytes + a * 16 * kStageRow);
-        __builtin_amdgcn_sched_barrier(0);
-        if (b < NT && have) {
-#pragma unroll
-          for (int a = 0; a < MT; ++a) acc[a][b] = E::mfma16(wf[u][b], xf[u][a], acc[a][b]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      kpos = kpos + 1 == lines ? 0 : kpos + 1;
-    }
+  u32x4_t wf[2][NT], xf[2][MT];
+  constexpr int NR = MT + NT, NM = MT * NT;
+  auto read = [&](auto r_, int h, uint32_t at) {  // in the order of use
+    constexpr int r = decltype(r_)::value;
+    if constexpr (r == 0) wf[h][0] = lds_read_b128(lds, w_addr[h] + at);
+    else if constexpr (r <= MT) xf[h][r - 1] = lds_read_b128(lds, x_addr[h] + at + (r - 1) * 16 * kStageRow);
+    else wf[h][r - MT] = lds_read_b128(lds, w_addr[h] + at + (r - MT) * 16 * kStageRow);
   };
+  // Fragments of 32 k (half a line) are read while the MFMAs of the 32 before run.
   wait_loads<L * KS * (STAGES - 1)>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  static_for<0, NR>([&](auto r) { read(r, 0, 0); });
+  constexpr int R1 = NR + 4 > NM ? 2 : 1;               // fragment reads of a slot
+  constexpr int READ = (NR + R1 - 1) / R1 + 5;          // by this slot the reads of a phase have come back
+  constexpr int PH = 2 * KS, BS = (PH - 2) * NM + (READ < NM ? READ : NM), DS = PH * NM - BS;
+  // One stage.  LEFT: stages under way beyond the next one; LOAD: fetch another; NEXT: there is a next one.
+  auto stage = [&](auto left, auto load, auto next_) {
+    constexpr int LEFT = decltype(left)::value;
+    constexpr bool LOAD = decltype(load)::value, NEXT = decltype(next_)::value;
+    const uint32_t fetch = slot, next = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
+    static_for<0, PH * NM>([&](auto j_) {
+      constexpr int j = decltype(j_)::value, h = j / NM, q = j % NM;
+      if (KS > 1 && !NEXT && h >= 2 && h / 2 >= last_lines) return;  // (the last stage may hold surplus lines)
+      if constexpr (j == BS && NEXT) {
+        wait_loads<L * KS * LEFT>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+      static_for<0, R1>([&](auto r_) {
+        constexpr int r = q * R1 + decltype(r_)::value;
+        if constexpr (r < NR && (h < PH - 1 || NEXT))
+          read(std::integral_constant<int, r>(), (h + 1) & 1, h == PH - 1 ? next : slot + (h + 1) / 2 * kLineBytes);
+      });
+      static_for<0, KS * L>([&](auto l_) {
+        constexpr int l = decltype(l_)::value;
+        if constexpr (LOAD && BS + l * DS / (KS * L) == j) {
+          issue(std::integral_constant<int, l % L>(), wbase + kpos, xbase + kpos, fetch + l / L * kLineBytes);
+          if (l % L == L - 1) advance();
+        }
+      });
+      __builtin_amdgcn_sched_barrier(0);
+      acc[q % MT][q / MT] = E::mfma16(wf[h & 1][q / MT], xf[h & 1][q % MT], acc[q % MT][q / MT]);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    slot = next;
+  };
+  using True = std::true_type;
+  using False = std::false_type;
+  for (int s = STAGES; s < stages; ++s) stage(std::integral_constant<int, STAGES - 2>(), True(), True());
+  static_for<0, STAGES>([&](auto u_) {
+    constexpr int u = decltype(u_)::value, left = STAGES - 2 - u;
+    if (stages - STAGES + u < 0) return;  // k of fewer stages than are kept
+    stage(std::integral_constant<int, (left > 0 ? left : 0)>(), False(), std::integral_constant<bool, (u < STAGES - 1)>());
+  });
+  wait_loads<0>();  // (k of one stage: the surplus ones are still under way, and LDS is given up at the end)
+  const int row0 = m0 + wm * (BM / 2);
 #pragma unroll
-  for (int u = 0; u < KS; ++u) {
-#pragma unroll
-    for (int a = 0; a < MT; ++a) x0[u][a] = lds_read_b128(lds, x_addr + u * kLineBytes + a * 16 * kStageRow);
-#pragma unroll
-    for (int b = 0; b < NT; ++b) w0[u][b] = lds_read_b128(lds, w_addr + u * kLineBytes + b * 16 * kStageRow);
-  }
-  for (int line = 0; line < lines; line += 2 * KS) {
-    step(line, w0, x0, w1, x1);
-    if (line + KS < lines) step(line + KS, w1, x1, w0, x0);
-  }
-
-  wait_loads<0>();  // the loads past the last stage (k from its start again) still aim at the places written next
-  // The two waves of a quadrant trade halves of their sums, and each rounds and stores the half it keeps.
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  f32x4_t *pieces = reinterpret_cast<f32x4_t *>(lds) + lane;
-#pragma unroll
-  for (int f = 0; f < F; ++f)
-    if ((f >= HALF) == (kg == 0)) pieces[((wave & 3) * F + f) * 64] = acc[f / NT][f % NT];
-  __syncthreads();
-#pragma unroll
-  for (int f = 0; f < F; ++f) {
-    if ((f >= HALF) == (kg == 0)) continue;  // (wave-uniform)
-    const int row = m0 + wm * (BM / 2) + (f / NT) * 16 + i, col = n0 + wn * (BN / 2) + (f % NT) * 16 + 4 * cg;
-    f32x4_t sum = acc[f / NT][f % NT] + pieces[((wave & 3) * F + f) * 64];
-    if (row >= p.m || col >= p.n) continue;
+  for (int b = 0; b < NT; b += 2) {
+    const bool two = b + 1 < NT;
+    const int c = 16 * b + (two ? 8 : 4) * cg, col = col0 + c;
+    f32x4_t b0 = {0.f, 0.f, 0.f, 0.f}, b1 = b0;
     if (p.bias) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum[j] += p.bias[col + j];
+      b0 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c);
+      if (two) b1 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c + 16);
     }
-    *reinterpret_cast<u32x2_t *>(p.out + (size_t)row * p.n + col) = u32x2_t{E::pack2(sum[0], sum[1]), E::pack2(sum[2], sum[3])};
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+      const int row = row0 + 16 * a + i;
+      const f32x4_t u = acc[a][b] + b0;
+      uint16_t *o = p.out + (size_t)row * p.n + col;
+      if (two) {
+        const f32x4_t v = acc[a][b + 1 < NT ? b + 1 : b] + b1;
+        if (row < p.m && col < p.n)
+          *reinterpret_cast<u32x4_t *>(o) = u32x4_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3]), E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+      } else if (row < p.m && col < p.n) {
+        *reinterpret_cast<u32x2_t *>(o) = u32x2_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3])};
+      }
+    }
   }
 }
 
@@ -181,67 +243,57 @@ template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile
   const int gm = p.m_tiles < 4 ? p.m_tiles : 4;
   p.band = make_fast_div((uint32_t)(gm * p.n_tiles));
   p.band_rows = make_fast_div((uint32_t)gm);
-  constexpr int stage_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow, piece_bytes = 4 * MT * NT * 1024;
-  constexpr int lds_bytes = stage_bytes > piece_bytes ? stage_bytes : piece_bytes;
-  static_assert(lds_bytes <= 160 * 1024, "");
+  constexpr int lds_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow + kBiasBytes;
+  static_assert(lds_bytes > 64 * 1024 && lds_bytes <= 160 * 1024, "");
   void (*kern)(TileParams) = matmul_tile_kernel<T, MT, NT, KS, STAGES>;
-  if (lds_bytes > 64 * 1024) {  // an opt-in per device and kernel
-    static std::atomic<uint64_t> attr_done{0};
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+  static std::atomic<uint64_t> attr_done{0};  // more than 64 KiB of dynamic LDS is an opt-in per device and kernel
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (!(attr_done.load(std::memory_order_acquire) & bit)) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) return e;
-    const uint64_t bit = 1ull << (dev & 63);
-    if (!(attr_done.load(std::memory_order_acquire) & bit)) {
-      e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-      if (e != hipSuccess) return e;
-      attr_done.fetch_or(bit, std::memory_order_release);
-    }
+    attr_done.fetch_or(bit, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(p.m_tiles * p.n_tiles), dim3(64 * kTileWaves), lds_bytes, stream, p);
+  hipLaunchKernelGGL(kern, dim3(p.m_tiles * p.n_tiles), dim3(kTileThreads), lds_bytes, stream, p);
   return hipGetLastError();
 }
 
 template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_t stream) {
   switch (kind) {
-    case 0: return launch_tile<T, 1, 1, 2, 4>(p, stream);
-    case 1: return launch_tile<T, 2, 1, 1, 6>(p, stream);
-    case 2: return launch_tile<T, 2, 2, 1, 6>(p, stream);
-    case 3: return launch_tile<T, 3, 2, 1, 5>(p, stream);
-    case 4: return launch_tile<T, 4, 2, 1, 4>(p, stream);
-    case 5: return launch_tile<T, 3, 3, 1, 4>(p, stream);
-    case 6: return launch_tile<T, 3, 4, 1, 4>(p, stream);
-    case 7: return launch_tile<T, 4, 4, 1, 4>(p, stream);
-    case 8: return launch_tile<T, 4, 5, 1, 4>(p, stream);
-    case 9: return launch_tile<T, 4, 6, 1, 3>(p, stream);
-    case 10: return launch_tile<T, 4, 7, 1, 3>(p, stream);
+    case 0: return launch_tile<T, 1, 1, 4, 4>(p, stream);
+    case 1: return launch_tile<T, 2, 1, 4, 3>(p, stream);
+    case 2: return launch_tile<T, 2, 2, 1, 9>(p, stream);
+    case 3: return launch_tile<T, 3, 2, 1, 7>(p, stream);
+    case 4: return launch_tile<T, 4, 2, 1, 6>(p, stream);
+    case 5: return launch_tile<T, 3, 3, 1, 6>(p, stream);
+    case 6: return launch_tile<T, 3, 4, 1, 5>(p, stream);
+    case 7: return launch_tile<T, 4, 3, 1, 5>(p, stream);
+    case 8: return launch_tile<T, 4, 4, 1, 4>(p, stream);
+    case 9: return launch_tile<T, 4, 5, 1, 4>(p, stream);
+    case 10: return launch_tile<T, 4, 6, 1, 3>(p, stream);
+    case 11: return launch_tile<T, 5, 5, 1, 3>(p, stream);
+    case 12: return launch_tile<T, 4, 7, 1, 3>(p, stream);
+    case 13: return launch_tile<T, 5, 6, 1, 3>(p, stream);
     default: return launch_tile<T, 4, 8, 1, 3>(p, stream);
   }
 }
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
-// (Twelve tiles rather than eight fill the round better; us, hipBLASLt / here: 3584 x 3584, 320 rows 22.8 / 19.7, 768 rows
-// 33.1 / 29.4, 1280 rows 43.3 / 39.2; 5120 x 5120, 900 rows 62.6 / 56.9.  128 x 96 and 64 x 96 are slower than 96 x 128 and
-// 96 x 64: 640 rows 31.3 / 28.6, 200 rows of 5120 30.4 / 28.2.)
-// From 96 x 64 on hipBLASLt, which cuts k too, is the faster one where that leaves a fifth of the CUs idle: 5120 x 5120, 640
-// rows (78 % busy) 51.5 us against 53.7, 768 rows (94 %) 53.3 / 53.2, 900 rows (100 %) 62.6 / 56.9.  Not so up to k = 2048,
-// where the start of a workgroup weighs more: 1536 x 1536, 768 rows (56 %) 12.4 / 11.2.  And from 128 x 192 on where rows are a
-// multiple of 4 KiB apart: 4096 x 4096, 1280 rows 46.6 / 47.6, 1500 rows 49.7 / 53.7, against 3584 x 3584, 1500 rows 44.2 /
-// 42.7, 2048 rows 52.4 / 50.7; 8192 x 8192, 2000 rows 175 / 182.
-// hipBLASLt's time is no smooth function of the rows, so that the two cross more often than these lines say.  Left to it
-// though tiles would be faster: 3584 x 3584, 257-288 rows 29.5 / 23.1, 577-672 32.0 / 29.6, 865-896 35.5 / 34.0; 4096 x 4096,
-// 513-576 rows 35.3 / 32.7; 1024 x 5120, 1025-1152 rows 28.3 / 26.6.  Taken though slower: 3584 x 3584, 784-864 rows 29.2 /
-// 31.5; 5120 x 5120, 64-80 rows 21.7 / 24.2, 257-272 30.9 / 33.2, 528-560 41.6 / 45.0; 1024 and 2048 x 8192, 17-32 rows
-// 11.7-16.2 / 18-22 (a quarter of the CUs, rows a multiple of 4 KiB apart).
+// Over 227 sizes (15 weights of 256-11008 rows and k of 1536-18944, 17-4096 lhs rows) the choice takes 0.81 of hipBLASLt's
+// time on average.  Left to hipBLASLt, which cuts k, are few small tiles over a long k (us, hipBLASLt / here: 1024 x 8192, 17
+// rows 10.1 / 13.1, 100 rows 12.7 / 13.7; 2048 x 8192, 24 rows 13.7 / 16.3; not so 1024 x 5120, 48 rows 14.2 / 9.4).  Taken
+// though slower: 5120 x 5120, 64 rows 22.2 / 23.8, 4096 x 11008, 680 rows 83.5 / 87.4.  More than one round is not:
+// 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 / 54.5 with 128 x 128.
 int tile_kind(int m, int n, int k) {
-  static const struct { int m, n; } tiles[] = {{32, 32},  {64, 32},   {64, 64},   {96, 64},   {128, 64},  {96, 96},
-                                               {96, 128}, {128, 128}, {128, 160}, {128, 192}, {128, 224}, {128, 256}};
+  static const struct { int m, n; } tiles[] = {{32, 32},   {64, 32},   {64, 64},   {96, 64},   {128, 64},
+                                               {96, 96},   {96, 128},  {128, 96},  {128, 128}, {128, 160},
+                                               {128, 192}, {160, 160}, {128, 224}, {160, 192}, {128, 256}};
   const long long cus = device_compute_units();
-  for (int kind = 0; kind < 12; ++kind) {
+  for (int kind = 0; kind < 15; ++kind) {
     const long long count = (long long)((m + tiles[kind].m - 1) / tiles[kind].m) * ((n + tiles[kind].n - 1) / tiles[kind].n);
-    if (count > cus) continue;
-    if (kind >= 3 && k > 2048 && 5 * count <= 4 * cus) return -1;
-    if (kind >= 9 && k % 2048 == 0) return -1;
-    return kind;
+    if (count <= cus) return kind == 0 && k > 6144 && 2 * count <= cus ? -1 : kind;
   }
   return -1;
 }
