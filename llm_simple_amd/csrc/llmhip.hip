@@ -440,13 +440,14 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
   if (n % 16 != 0 || k % 16 != 0) return LLMHIP_ERR_UNSUPPORTED;
   // Up to 16 rows one MFMA column block holds every lhs row and the call is a read of W; beyond that lhs, which
   // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  From 9 rows on that is so already
-  // where W has more rows than one round of its workgroups takes, 16 per CU (W from HBM, us, few-row kernel /
-  // tiles: 5120 x 5120, 9 rows 17.1 / 15.4, 16 rows 21.0 / 16.0; 11008 x 4096, 16 rows 27.6 / 21.3; not so 4096 x 4096, 9
-  // rows 10.4 / 11.7, nor with 8 rows).  Both kernels move 16-byte pieces; hipBLASLt takes any base.
+  // where W has more than 8 rows per CU (W from HBM, us, few-row kernel / tiles: 3584 x 3584, 9 rows 7.7 / 7.2, 16 rows 8.9
+  // / 7.2; 4096 x 4096, 9 rows 9.8 / 8.4; 3072 x 8192, 9 rows 16.9 / 15.7; not so 2048 x 2048, 9 rows 4.8 / 5.1, 512 x 3584,
+  // 12 rows 6.1 / 6.7, nor with 8 rows of a long k: 3072 x 8192 13.6 / 18.2).  Both kernels move 16-byte pieces; hipBLASLt
+  // takes any base.
   if (all_aligned16(out, lhs, weight)) {
     const float *b = static_cast<const float *>(bias);
     const bool tiles = m > 8 && matmul_tile_takes(m, n, k);
-    if (m <= 16 && !(tiles && n > 16LL * device_compute_units()))
+    if (m <= 16 && !(tiles && n > 8LL * device_compute_units()))
       return from_hip(launch_matmul_skinny(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
     if (tiles)
       return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));

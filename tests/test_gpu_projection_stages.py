@@ -39,3 +39,18 @@ def test_stages(tile, size, depth, dt):
         assert np.isfinite(got).all(), lines
         # one rounding of an fp32 sum: a step of the storage type, 1e-3 where the sum cancels
         assert (np.abs(got[rows] - ref) <= np.maximum(1.01 * ulp(ref, dt), 1e-3)).all(), lines
+
+
+@pytest.mark.parametrize("dt", [DT_FLOAT16, DT_BFLOAT16])
+@pytest.mark.parametrize("m,n,k", [(9, 2048, 320), (9, 2064, 320), (16, 2064, 64), (8, 2064, 128), (13, 3584, 704)])
+def test_few_rows_line(dt, m, n, k):
+    """Either side of the line (2048 features, 8 rows) from which the tiles take calls of up to 16 rows."""
+    import llm_simple_amd.ops as ops
+    x = normal_bits(m + k, (m, k), dt)
+    w = orc.round_to(orc.widen(normal_bits(n, (n, k), dt), dt) / np.sqrt(k), dt)
+    b = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    ref = orc.widen(orc.matmul_bias(x, w, b, dt), dt)
+    d_out = to_dev(np.zeros((m, n), dtype=np.uint16))
+    ops.hip_matmul_bias_layer(d_out, to_dev(x), to_dev(w), f32_dev(b), m, n, k, dt)
+    got = orc.widen(to_host(d_out), dt)
+    assert (np.abs(got - ref) <= np.maximum(1.01 * ulp(ref, dt), 1e-3)).all()

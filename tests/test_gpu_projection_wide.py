@@ -1,5 +1,5 @@
-"""9 to 16 lhs rows against a weight with more rows than one round of the few-row kernel takes (4096 on 256 compute units)
-go to the tiled kernel: both sides of that line, and k in part stages (which the tiles do not take), against the oracle."""
+"""9 to 16 lhs rows against a wide weight go to the tiled kernel (more than 2048 rows on 256 compute units): 8 and 9 rows,
+both kernels, and k in part stages (which the tiles do not take), against the oracle."""
 import numpy as np
 import pytest
 
