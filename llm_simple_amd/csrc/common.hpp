@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 // The measurement library (libllmhip_bench.so) compiles the prefill kernel a second time with
 // LLMHIP_BENCH defined (a clock stamp in the kernel); its copy lives in a namespace of its own so
 // that the two libraries never share a symbol.
@@ -61,6 +63,8 @@ template <> struct Elem<_Float16> {
   static __device__ __forceinline__ uint16_t round(float f) {
     return __builtin_bit_cast(uint16_t, (_Float16)f);
   }
+  static __device__ __forceinline__ float low(uint32_t pair) { return widen((uint16_t)pair); }
+  static __device__ __forceinline__ float high(uint32_t pair) { return widen((uint16_t)(pair >> 16)); }
 };
 
 template <> struct Elem<__bf16> {
@@ -84,6 +88,8 @@ template <> struct Elem<__bf16> {
   // (src/util.cpp:33-72) on every finite input, and a NaN stays one whatever its payload (added to the bit
   // pattern, the rounding carries 0xFFFFFFFF over to 0).
   static __device__ __forceinline__ uint16_t round(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+  static __device__ __forceinline__ float low(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
+  static __device__ __forceinline__ float high(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
 };
 
 // n / d for 32-bit n by multiply and shift (Granlund-Montgomery, round-up variant): exact for every n.
@@ -107,6 +113,14 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// f(integral_constant<int, I>) ... f(integral_constant<int, N - 1>)
+template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>());
+    static_for<I + 1, N>(f);
+  }
+}
 
 // acc + lo + hi of a packed pair of storage-type values.
 template <typename T> __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc);
@@ -141,6 +155,16 @@ typedef __attribute__((__vector_size__(4 * sizeof(short)))) short lds_s16x4_t;
 __device__ __forceinline__ u32x2_t lds_read_tr16(const char *lds_base, int byte_off) {
   auto p = reinterpret_cast<__attribute__((address_space(3))) lds_s16x4_t *>(
       (__attribute__((address_space(3))) char *)(lds_base) + byte_off);
+  lds_s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(p);
+  return __builtin_bit_cast(u32x2_t, v);
+}
+
+// The same at an LDS address plus a constant that the instruction adds (from a base pointer that is the symbol of the
+// dynamic segment the compiler adds 0 to the address at every use).
+typedef __attribute__((address_space(3))) char lds_char;
+__device__ __forceinline__ uint32_t lds_address(const char *p) { return (uint32_t)(uintptr_t)(lds_char *)p; }
+__device__ __forceinline__ u32x2_t lds_read_tr16(uint32_t address, int constant) {
+  auto p = reinterpret_cast<__attribute__((address_space(3))) lds_s16x4_t *>(reinterpret_cast<lds_char *>(address) + constant);
   lds_s16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(p);
   return __builtin_bit_cast(u32x2_t, v);
 }

@@ -29,14 +29,21 @@
 // Outside the loop a workgroup costs a short launch 2-3 us: indexes come from divisions prepared by the host, Q
 // of shared rows is fetched once through LDS, and waves that shared rows trade pieces of O^T so that each
 // folds and stores its part (epilogue of a pair 3900 -> 2200 cycles).
-// Tiles travel global -> LDS without VGPR staging (global_load_lds_dwordx4), spread over the MFMA
+// Tiles travel global -> LDS without VGPR staging (buffer_load_dwordx4 ... lds), spread over the MFMA
 // stream in the 8-wave kernels, issued beside the first MFMAs of a phase in the others.  The loop is
 // software pipelined inside a wave: the MFMAs of S(j+1) are issued beside the
 // softmax of tile j (the first ones beside the row-maximum chain, the rest, together with the
 // MFMAs of P(j).V(j), beside the exponentials), so K is fetched one tile ahead of V.
 // Every LDS fragment address is a loop-invariant register plus an immediate, and a
-// tile load is a scalar base plus a loop-invariant lane offset: the loop spends its
-// vector ALU instructions on the softmax only.
+// tile load is a descriptor that walks through the cache plus a loop-invariant lane offset: the loop spends its
+// vector ALU instructions on the softmax only.  That counts for more than their order: a full chip runs this loop at
+// 1.6 GHz, what its power allows, and the waves of short prompts issue one instruction in 4-5 cycles.  Clamps
+// and 64-bit address sums of the tile loads, a register for M0 per load, the additive term of the exponent and the
+// line for its move in every tile, an addition of 0 to every V address: without these 40 of 300 instructions of a
+// step (rope not counted, us) 256 tokens of 32 heads 6.6 -> 6.15, 1019 of 28 17.7 -> 16.9, 2048 40.2 -> 39.0, 4096 121.8 ->
+// 118.6, 8192 445 -> 434, 200 past 16001 59.0 -> 56.7.  (The same step written out in slots of one MFMA with every
+// fragment read four slots ahead of its use is not faster: 4096 tokens 115.9 / 115.7, 8192 420 / 418; nor are sums by
+// shifts and additions in place of the dot instructions, which an MFMA cannot overlap: 116.2 / 119.3.)
 //
 // A chunk of few query rows over a long cache (chunked prefill) has its key range split over
 // workgroups: each leaves an fp32 partial (reference maximum, sum, unnormalised O) and
@@ -153,18 +160,21 @@ template <typename T, int KB = 2> struct WaveAttn {
   u32x4_t pf[KB][2];   // P^T packed as B operand: key block x k-step
   u32x4_t qf[8];       // Q^T fragments (B operand), loaded once
   float m_run, l_run;  // running max (raw score units) and sum of this lane's keys
+  float move_above, neg_ms;  // m_run plus the slack of its move; what it adds to the exponent
   int lane, l32, hh, g16, li;
   int k_addr[8];  // LDS byte offset of this lane's K fragment kk in tile slot 0, key block 0
-  int v_addr[4];  // same for the V^T fragment of d block d (k-step 0, low half)
+  uint32_t v_addr[4];  // LDS address of the V^T fragment of d block d (k-step 0, low half)
 
   // kb0: first 32-key block of a tile this wave works on (0, or 1 for the second wave of a pair)
-  __device__ __forceinline__ void init(int lane_, int v_region, int kb0 = 0) {
+  __device__ __forceinline__ void init(const char *lds, int lane_, int v_region, int kb0 = 0) {
     lane = lane_;
     l32 = lane & 31;
     hh = lane >> 5;
     g16 = lane >> 4;
     li = lane & 15;
     m_run = -INFINITY;
+    move_above = -INFINITY;
+    neg_ms = 0.0f;
     l_run = 0.0f;
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -181,7 +191,7 @@ template <typename T, int KB = 2> struct WaveAttn {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       const int gran = d * 4 + (g16 & 1) * 2 + ((li & 3) >> 1);
-      v_addr[d] = v_region + v_swizzle_off(4 * hh + (li >> 2), gran) + (li & 1) * 8 + kb0 * 32 * kRowBytes;
+      v_addr[d] = lds_address(lds) + v_region + v_swizzle_off(4 * hh + (li >> 2), gran) + (li & 1) * 8 + kb0 * 32 * kRowBytes;
       asm volatile("" : "+v"(v_addr[d]));
     }
   }
@@ -203,19 +213,19 @@ template <typename T, int KB = 2> struct WaveAttn {
   }
 
   struct NoHook {
-    __device__ __forceinline__ void operator()(int) const {}
+    template <typename I> __device__ __forceinline__ void operator()(I) const {}
   };
   // S^T = K Q^T for the wave's keys of the K tile at byte offset `koff` of the LDS segment.
   // The fragments of step kk+1 are requested before the MFMAs of step kk.  hook(i) runs
   // after MFMA i (0..8*KB-1): the callers spread their global loads over the MFMA stream with it.
   template <int KK0 = 0, int KK1 = 8, typename Hook = NoHook>
   __device__ __forceinline__ void qk(const char *lds, int koff, f32x16_t (&s)[KB], Hook hook = Hook()) {
-#pragma unroll
-    for (int kk = KK0; kk < KK1; ++kk) {
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
+    static_for<KK0, KK1>([&](auto kk_) {
+      constexpr int kk = decltype(kk_)::value;
+      static_for<0, KB>([&](auto kb_) {
+        constexpr int kb = decltype(kb_)::value;
         const u32x4_t kf = lds_read_b128(lds, k_addr[kk] + koff + kb * 32 * kRowBytes);
-        if (kk == 0) {
+        if constexpr (kk == 0) {
           f32x16_t z;
 #pragma unroll
           for (int i = 0; i < 16; ++i) z[i] = 0.0f;
@@ -223,30 +233,25 @@ template <typename T, int KB = 2> struct WaveAttn {
         } else {
           s[kb] = E::mfma32(kf, qf[kk], s[kb]);
         }
-        hook(kk * KB + kb);
-      }
-    }
+        hook(std::integral_constant<int, kk * KB + kb>());
+      });
+    });
   }
 
   // O^T += V^T P^T over the V tile at byte offset `voff` past the start of the V region.
   // Lane (d = 32*dblk + l32, hh): element e of k-step (kb, ks2) is the key
   // 32*kb + 16*ks2 + 8*(e/4) + 4*hh + e%4 -- the key P's element e carries.
   template <typename Hook = NoHook>
-  __device__ __forceinline__ void pv(const char *lds, int voff, Hook hook = Hook()) {
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-      for (int ks2 = 0; ks2 < 2; ++ks2) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          const int c = voff + (kb * 32 + ks2 * 16) * kRowBytes;
-          const u32x2_t lo = lds_read_tr16(lds, v_addr[d] + c);
-          const u32x2_t hi = lds_read_tr16(lds, v_addr[d] + c + 8 * kRowBytes);
-          const u32x4_t vf = {lo[0], lo[1], hi[0], hi[1]};
-          o[d] = E::mfma32(vf, pf[kb][ks2], o[d]);
-          hook((kb * 2 + ks2) * 4 + d);
-        }
-      }
+  __device__ __forceinline__ void pv(int voff, Hook hook = Hook()) {
+    static_for<0, 8 * KB>([&](auto i_) {
+      constexpr int i = decltype(i_)::value, kb = i / 8, ks2 = i / 4 % 2, d = i % 4;
+      const int c = voff + (kb * 32 + ks2 * 16) * kRowBytes;
+      const u32x2_t lo = lds_read_tr16(v_addr[d], c);
+      const u32x2_t hi = lds_read_tr16(v_addr[d], c + 8 * kRowBytes);
+      const u32x4_t vf = {lo[0], lo[1], hi[0], hi[1]};
+      o[d] = E::mfma32(vf, pf[kb][ks2], o[d]);
+      hook(i_);
+    });
   }
 
   // Causal / length mask of one tile of scores (only called for tiles that can be cut); key0 =
@@ -262,7 +267,7 @@ template <typename T, int KB = 2> struct WaveAttn {
 
   // P = exp2(s*c + neg_ms) rounded to T and packed as the B operand; returns this lane's sum
   // of the rounded values.
-  __device__ __forceinline__ float probabilities(const f32x16_t (&s)[KB], float c, float neg_ms) {
+  __device__ __forceinline__ float probabilities(const f32x16_t (&s)[KB], float c) {
     float ps0 = 0.0f, ps1 = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -295,8 +300,9 @@ template <typename T, int KB = 2> struct WaveAttn {
   // in raw score units.  It moves only when a row maximum exceeds it by more than kLazyLog2
   // in log2 units (probabilities then stay below 2^kLazyLog2, harmless in fp32 sums and in
   // the 16-bit P operand); a -inf reference always moves.  O and l are rescaled only then,
-  // which after the first tiles is rare.  Returns the additive term of the exponent.
-  __device__ __forceinline__ float row_max(const f32x16_t (&s)[KB], float scale_log2e) {
+  // which after the first tiles is rare: what depends on the reference alone (the line `move_above`, the additive term
+  // of the exponent) is computed then too, and a lane pair compares notes only then.
+  __device__ __forceinline__ void row_max(const f32x16_t (&s)[KB], float scale_log2e) {
     float m0 = -INFINITY, m1 = -INFINITY;  // two chains: half the dependent latency
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -309,9 +315,10 @@ template <typename T, int KB = 2> struct WaveAttn {
         m0 = fmaxf(m0, s[0][i]);
       }
     }
-    const float mloc = pair_max(fmaxf(m0, m1));
-    const bool move = mloc > m_run + kLazyLog2 / scale_log2e;
-    if (__builtin_amdgcn_ballot_w64(move) != 0) {
+    float mloc = fmaxf(m0, m1);
+    if (__builtin_amdgcn_ballot_w64(mloc > move_above) != 0) {
+      mloc = pair_max(mloc);
+      const bool move = mloc > move_above;
       const float m_new = move ? mloc : m_run;
       const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
       const float alpha = move ? fast_exp2((m_run - m_use) * scale_log2e) : 1.0f;
@@ -321,8 +328,9 @@ template <typename T, int KB = 2> struct WaveAttn {
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
       m_run = m_new;
+      move_above = m_new + kLazyLog2 / scale_log2e;
+      neg_ms = -m_use * scale_log2e;
     }
-    return -((m_run == -INFINITY) ? 0.0f : m_run) * scale_log2e;
   }
 
   // KP waves that shared the rows (KB == 1) trade pieces of O^T: wave `part` keeps and will store the
@@ -451,61 +459,63 @@ __device__ __forceinline__ void lds_dma(const char *src, uint32_t lds_addr) {
                : "m0");
 }
 
-// Global -> LDS tile loader without VGPR staging (global_load_lds_dwordx4: lane l's 16
-// bytes land at the wave-uniform LDS address in M0 + 16*l).  One wave instruction fills four
-// 256-byte rows; the XOR swizzles are realised on the global side: the lane that owns
-// physical granule pg of row r fetches the logical granule that belongs there.  A tile
-// of TN keys is TN/4 instructions, dealt to the NW waves; `slot` s of wave w covers rows
-// 4*(s*NW + w) .. +3.  The global address is a scalar tile base plus a per-lane 32-bit
-// offset that never changes (except in a ragged last tile, whose rows are clamped to n-1),
-// so a load costs no vector ALU work.  The loads are issued from inline asm: the compiler
-// would order every later LDS read behind a transfer it knows about (s_waitcnt vmcnt(0)).
-// Completion is waited for explicitly before the barrier that publishes a stage.
+// Global -> LDS tile loader without VGPR staging (buffer_load_dwordx4 ... lds: lane l's 16 bytes land at the
+// wave-uniform LDS address in M0 + the instruction's offset + 16*l).  One wave instruction fills four 256-byte rows; the
+// XOR swizzles are realised on the global side: the lane that owns physical granule pg of row r fetches the logical granule
+// that belongs there.  A tile of TN keys is TN/4 instructions; slot s of wave w covers rows 4*(w*kSlots + s) .. +3.
+// The lane offsets never change and rows past the end are cut off by the descriptor (they read as zero), so a load costs no
+// vector ALU work, and M0 is written for every fourth one only: the instruction's offset moves both addresses, and
+// the lane offsets make up for it.  The loads are issued from inline asm: the compiler would order every later LDS
+// read behind a transfer it knows about (s_waitcnt vmcnt(0)).  Completion is waited for explicitly before the barrier that
+// publishes a stage.
+typedef __attribute__((ext_vector_type(4))) uint32_t buffer_t;
 template <int NW, int TN, bool NT> struct DirectLoader {
   static constexpr int kSlots = TN / 4 / NW;  // instructions per wave per tile
+  static constexpr int kLow = 1024 * ((kSlots < 4 ? kSlots : 4) - 1);
   int n, row_bytes;
-  uint32_t lds_row0;          // LDS byte offset of row 4*wave (wave-uniform)
-  int row[kSlots];            // tile row this lane fetches in slot s
-  uint32_t lane_k[kSlots];    // logical granule byte offset within the row, K swizzle
-  uint32_t lane_v[kSlots];    // same, V swizzle
+  uint32_t lds_wave;                          // LDS byte offset of the wave's first row (wave-uniform)
+  uint32_t off_k[kSlots], off_v[kSlots];      // lane offsets within a tile
 
   __device__ __forceinline__ void init(int wave, int lane, int row_bytes_, int n_) {
     n = n_;
     row_bytes = row_bytes_;
-    lds_row0 = __builtin_amdgcn_readfirstlane(4 * wave * kRowBytes);
+    lds_wave = __builtin_amdgcn_readfirstlane(wave * kSlots * 1024);
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
-      const int r = 4 * (s * NW + wave) + (lane >> 4), pg = lane & 15;
-      row[s] = r;
-      lane_k[s] = (pg ^ (r & 15)) << 4;
-      lane_v[s] = ((((pg >> 2) ^ (r & 3)) << 2) | (pg & 3)) << 4;
-      asm volatile("" : "+v"(row[s]), "+v"(lane_k[s]), "+v"(lane_v[s]));
+      const int r = 4 * (wave * kSlots + s) + (lane >> 4), pg = lane & 15;
+      const uint32_t at = r * row_bytes + kLow - 1024 * (s & 3);
+      off_k[s] = at + ((pg ^ (r & 15)) << 4);
+      off_v[s] = at + (((((pg >> 2) ^ (r & 3)) << 2) | (pg & 3)) << 4);
+      asm volatile("" : "+v"(off_k[s]), "+v"(off_v[s]));
     }
   }
+  // Descriptor of a key tile, kLow bytes early, that walks from tile to tile and stays on the last one, J - 1
+  struct Stream {
+    buffer_t d;
+    int left;  // tiles to come
+  };
+  __device__ __forceinline__ uint32_t records(int rows) const { return (uint32_t)(rows - 1) * row_bytes + kRowBytes + kLow; }
+  __device__ __forceinline__ Stream stream(const char *base, int J) const {
+    const uint64_t at = (uint64_t)base - kLow;
+    return Stream{{(uint32_t)at, (uint32_t)(at >> 32), records(min(TN, n)), 0x00020000u}, J - 1};
+  }
+  __device__ __forceinline__ void next(Stream &st, int J) const {
+    const uint64_t at = (((uint64_t)st.d[1] << 32) | st.d[0]) + (st.left > 0 ? (uint32_t)(TN * row_bytes) : 0u);
+    st.left -= st.left > 0 ? 1 : 0;
+    st.d[0] = (uint32_t)at;
+    st.d[1] = (uint32_t)(at >> 32);
+    st.d[2] = st.left > 0 ? records(TN) : records(min(TN, n - (J - 1) * TN));
+  }
+  // Slots 0 .. kSlots-1 of a tile in order, with no other tile's in between; lds_tile: LDS byte offset of the destination.
   // NT: the tile is read by this workgroup only (a packed chunk of one tile per kv head over a long
   // cache): non-temporal, like the decode kernel's loads (4 tokens over 131072 keys: 106 -> 91 us);
   // tiles that several workgroups read stay ordinary loads (non-temporal costs those 3-10 %).
-  static __device__ __forceinline__ void dma(const char *tile_base, uint32_t lane_off, uint32_t lds_addr) {
-    if (NT)
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
-                   :
-                   : "v"(lane_off), "s"(tile_base), "s"(lds_addr)
-                   : "m0");
-    else
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :
-                   : "v"(lane_off), "s"(tile_base), "s"(lds_addr)
-                   : "m0");
-  }
-  // t: key tile; lds_tile: LDS byte offset of the destination tile
-  template <bool IS_V>
-  __device__ __forceinline__ void issue(const char *base, int t, uint32_t lds_tile, int s) const {
-    const char *tile_base = base + (size_t)t * TN * row_bytes;
-    const uint32_t dst = lds_tile + lds_row0 + s * NW * 4 * kRowBytes;
-    // rows past n-1 (ragged last tile) are clamped to row n-1: nothing beyond the caller's n
-    // rows is read and the stale rows hold finite values; branch-free, two VALU instructions
-    const int r = min(row[s], n - 1 - t * TN);
-    dma(tile_base, r * row_bytes + (IS_V ? lane_v[s] : lane_k[s]), dst);
+  template <bool IS_V, int S> __device__ __forceinline__ void issue(const Stream &st, uint32_t lds_tile) const {
+    constexpr int at = 1024 * (S % 4);
+    if constexpr (at == 0) asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0" : : "s"(lds_wave), "s"(lds_tile + S * 1024) : "m0", "scc");
+    const uint32_t off = IS_V ? off_v[S] : off_k[S];
+    if constexpr (NT) asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 nt lds" : : "v"(off), "s"(st.d), "n"(at));
+    else asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(off), "s"(st.d), "n"(at));
   }
   static __device__ __forceinline__ void wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 };
@@ -577,7 +587,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   const char *vbase = p.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
 
   WaveAttn<T, KB> w;
-  w.init(lane, kVRegion, (KP > 1) ? kpar : 0);
+  w.init(lds, lane, kVRegion, (KP > 1) ? kpar : 0);
   // tiles in which this wave's keys hold at least one visible key
   const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) / TN)) : 0;
   float *part_o = nullptr, *part_ml = nullptr;
@@ -616,13 +626,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   ld.init(wave, lane, kv_row_bytes, n_);
   // K runs one tile ahead of V: S(j+1) = K(j+1) Q^T is issued together with the softmax of
   // tile j, so K tile t is fetched SUB+1 iterations and V tile t SUB iterations before use.
-#pragma unroll
-  for (int u = 0; u <= SUB; ++u)
-#pragma unroll
-    for (int sl = 0; sl < PER; ++sl) {
-      ld.template issue<false>(kbase, min(u, J - 1), (u % NSLOT) * TB, sl);
-      if (u < SUB) ld.template issue<true>(vbase, min(u, J - 1), kVRegion + u * TB, sl);
+  using Loader = DirectLoader<NW, TN, NT>;
+  typename Loader::Stream kst = ld.stream(kbase, J), vst = ld.stream(vbase, J);
+  static_for<0, SUB + 1>([&](auto u_) {
+    constexpr int u = decltype(u_)::value;
+    static_for<0, PER>([&](auto r) { ld.template issue<false, decltype(r)::value>(kst, u % NSLOT * TB); });
+    ld.next(kst, J);
+    if constexpr (u < SUB) {
+      static_for<0, PER>([&](auto r) { ld.template issue<true, decltype(r)::value>(vst, kVRegion + u * TB); });
+      ld.next(vst, J);
     }
+  });
   if (KP == 1) w.pin_q();  // the Q fragments are in registers from here on
   ld.wait_all();
   lds_barrier();
@@ -636,7 +650,6 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
 
   auto tile_step = [&](int j, int slot, f32x16_t (&s_cur)[KB], f32x16_t (&s_nxt)[KB]) {
     const int kslot = (slot + SUB + 1) % NSLOT, vslot = (slot + SUB) % NSLOT;  // fetched now
-    const int jk = min(j + SUB + 1, J - 1), jv = min(j + SUB, J - 1);
     if (j < Jw) {
       const int key0 = j * TN + kw0;
       if ((key0 + kWaveKeys - 1 > tok_lo + offset_) || (key0 + kWaveKeys > n_))
@@ -647,16 +660,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       // (S=2560: 61.0 -> 59.1 us, S=3072: 76.3 -> 75.0 us; the 8-wave kernel loses 0.7 % that way).
       // (Paired waves, KB == 1, run short sequences, where a step is shorter than a memory round
       // trip: there all loads of a step go out with its first MFMAs.)
-      auto k_hook = [&](int i) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r) {
-          if (KB == 1) {
-            if (i == r) ld.template issue<false>(kbase, jk, kslot * TB, r);
-            if (PER < 8 && i == PER + r) ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, r);
-          } else if (i == (NW == 4 ? r : (8 * KB / PER) * r + 1)) {
-            ld.template issue<false>(kbase, jk, kslot * TB, r);
+      auto k_hook = [&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        static_for<0, PER>([&](auto r_) {
+          constexpr int r = decltype(r_)::value;
+          if constexpr (KB == 1) {
+            if constexpr (i == r) ld.template issue<false, r>(kst, kslot * TB);
+            if constexpr (PER < 8 && i == PER + r) ld.template issue<true, r>(vst, kVRegion + vslot * TB);
+          } else if constexpr (i == (NW == 4 ? r : (8 * KB / PER) * r + 1)) {
+            ld.template issue<false, r>(kst, kslot * TB);
           }
-        }
+        });
       };
       // The MFMAs of S(j+1) overlap the softmax of tile j: the first ones run beside the row
       // maximum chain, the rest -- and the MFMAs of P.V -- beside the exponentials.  (For the
@@ -664,22 +678,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       // would separate these MFMAs from the instructions they overlap with.)
       const int koff = ((slot + 1) % NSLOT) * TB;
       w.template qk<0, kSplitKK>(lds, koff, s_nxt, k_hook);
-      const float neg_ms = w.row_max(s_cur, p.scale_log2e);
+      w.row_max(s_cur, p.scale_log2e);
       w.template qk<kSplitKK, 8>(lds, koff, s_nxt, k_hook);
-      w.l_run += w.probabilities(s_cur, p.scale_log2e, neg_ms);
-      w.pv(lds, slot * TB, [&](int i) {
-#pragma unroll
-        for (int r = 0; r < PER; ++r)
-          if (KB == 1 ? (PER == 8 && i == r) : i == (NW == 4 ? r : (8 * KB / PER) * r + 1))
-            ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, r);
+      w.l_run += w.probabilities(s_cur, p.scale_log2e);
+      w.pv(slot * TB, [&](auto i_) {
+        constexpr int i = decltype(i_)::value;
+        static_for<0, PER>([&](auto r_) {
+          constexpr int r = decltype(r_)::value;
+          if constexpr (KB == 1 ? (PER == 8 && i == r) : i == (NW == 4 ? r : (8 * KB / PER) * r + 1))
+            ld.template issue<true, r>(vst, kVRegion + vslot * TB);
+        });
       });
     } else {
-#pragma unroll
-      for (int sl = 0; sl < PER; ++sl) {
-        ld.template issue<false>(kbase, jk, kslot * TB, sl);
-        ld.template issue<true>(vbase, jv, kVRegion + vslot * TB, sl);
-      }
+      static_for<0, PER>([&](auto r) { ld.template issue<false, decltype(r)::value>(kst, kslot * TB); });
+      static_for<0, PER>([&](auto r) { ld.template issue<true, decltype(r)::value>(vst, kVRegion + vslot * TB); });
     }
+    ld.next(kst, J);
+    ld.next(vst, J);
   };
 
   for (int jb = 0; jb < J; jb += NSLOT) {

@@ -63,13 +63,6 @@ template <int N> __device__ __forceinline__ void wait_loads() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory");
 }
 
-template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>());
-    static_for<I + 1, N>(f);
-  }
-}
-
 // global_load_lds_dwordx4, OFF (0, 1024, 2048 or 3072) added to the global address and to the LDS address in M0, which
 // nothing but the assembly of this kernel writes
 template <int OFF> __device__ __forceinline__ void line_load(uint32_t voff, const char *base) {
