@@ -25,12 +25,14 @@
 // waves are merged through LDS at the end and the workgroup writes the final rows (one split) or an
 // fp32 partial (max, sum, unnormalised O).
 //
-// Up to 16 partials of a (sequence, kv head) are folded (log-sum-exp) by the workgroup that finds them all stored:
-// partials go past the XCD's L2 (sc1 stores), then a flag, then a look at the other flags -- no fence, no atomic.
-// That is three memory round trips, 2.2-2.4 us, against 3.1 us for flash_decode_combine_kernel, whose launch
-// also costs the host 2.4 us.  More partials make more rounds of loads in ONE workgroup (32: 11.2 against 8.8 us at
-// batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses write back
-// and invalidate the XCD's L2: 91 us against 33 at batch 1, 32768 keys.)
+// Up to 16 partials of a (sequence, kv head) are folded (log-sum-exp) by the workgroup that finds them all stored, with no
+// fence and no atomic.  Up to 8: every word goes past the XCD's L2 (sc1 stores) with the launch's tag beside it, and
+// whoever finds the tag at all of them folds them; that is two memory round trips.  More, or where the tag would be that of
+// a replay: partials, then a flag, then a look at the other flags, then the partials, four round trips.  (The fused step,
+// us, flags / tags: 384 keys of 2 kv heads 6.9 / 5.95, 512 of 32 7.4 / 6.25, 1000 of 8 7.75 / 7.15, 1500 of 32 11.3 / 9.15;
+// the combine launch takes 3.1 us, and 2.4 of the host's.)  More partials make more rounds of loads in ONE workgroup (32:
+// 11.2 against 8.8 us at batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses
+// write back and invalidate the XCD's L2: 91 us against 33 at batch 1, 32768 keys.)
 //
 // A short cache is bound by the length of one workgroup's chain, not by bytes: at 32 keys, one sequence, the
 // kernel took 6.3 us, 2.5 us of them the launch.  A wave issues a vector instruction every 4-5 cycles, so the
@@ -40,7 +42,7 @@
 // divisions are prepared by the host, the column maximum goes through permlane swaps, masks and the
 // rescaling of O run only where they change something, and the merge of the waves is free of bank conflicts (it cost
 // 1.4 us).  4.1 us now; 384 keys of 2 kv heads 9.7 -> 6.9 us, 512 keys of 32 kv heads 9.1 -> 6.6, 4096 keys of 8
-// 10.9 -> 9.2, 32768 keys of 8 28.4 -> 24.8 (fused step, back-to-back calls).
+// 10.9 -> 9.2, 32768 keys of 8 28.4 -> 24.8 (fused step, back-to-back calls, before the tags).
 //
 // (Eight-wave workgroups, half as many, merging pairs of splits through LDS: 4.5 TB/s against 6.0 at the time.)
 #include <atomic>
@@ -76,6 +78,7 @@ struct DecodeParams {
   float scale_log2e;
   int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
   uint64_t fold;  // not 0: the workgroup of a (sequence, kv head) that finds this number in all flags folds
+  uint32_t tag;   // not 0 (fold only): each word of a partial is stored with this one beside it, and there are no flags
   // Fused decode step (FUSED kernels only): the token at row fused_pos = n - 1 is not in the cache yet.
   // q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
   // q and the new K row are rotated with table row freq_row (64 (cos, sin) pairs) as they are loaded,
@@ -152,6 +155,8 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
 }
 
 constexpr int kMaxFoldSplits = 16;
+constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
+constexpr int kTaggedRows = 8;                    // query rows whose words carry a tag, at most
 constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
@@ -177,7 +182,11 @@ __device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int by
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
 }
 
-template <typename T, bool FUSED, int NW, bool LONG>
+// How the partials of a (sequence, kv head) become rows: not here (one split, or the combine launch), by flags, by tags.  A
+// kernel each: the code of the others in the way costs a call of 4 us 0.05.
+enum FoldMode { kNoFold, kFoldByFlags, kFoldByTags };
+
+template <typename T, bool FUSED, int NW, bool LONG, FoldMode FOLD>
 __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   using E = Elem<T>;
   constexpr int kStepKeys = NW * kDecWaveKeys;
@@ -400,6 +409,11 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   const int pair_slots = p.num_splits * p.cols;
   const __amdgpu_buffer_rsrc_t po = byte_buffer(p.ws_o + pair * pair_slots * kHeadDim, pair_slots * kHeadDim * 4);
   const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
+  const int tagged_bytes = p.num_splits * p.rows * kTaggedBytes;
+  const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + pair * tagged_bytes, tagged_bytes);
+  auto tagged = [&](float x, float y) {
+    return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), p.tag, __builtin_bit_cast(uint32_t, y), p.tag});
+  };
   for (int c = tid >> 4; c < p.rows; c += 4 * NW) {
     const int dch = tid & 15;  // 8-wide d chunk of column c
     float mw[NW], M = -INFINITY;
@@ -425,7 +439,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
         acc[4 + j] += wt * s1[j];
       }
     }
-    if (p.num_splits == 1) {
+    if (FOLD == kNoFold && p.num_splits == 1) {
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
       const int r = (int)fast_div(c, p.g_div), hq = c - r * p.g;
       char *op = p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + hq) * kRowBytes + dch * 16;
@@ -438,7 +452,12 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
     const int slot = split * p.cols + c;
     const f32x4_t a0 = {acc[0], acc[1], acc[2], acc[3]}, a1 = {acc[4], acc[5], acc[6], acc[7]};
     const u32x2_t ml = {__builtin_bit_cast(uint32_t, M), __builtin_bit_cast(uint32_t, L)};
-    if (p.fold) {
+    if constexpr (FOLD == kFoldByTags) {
+      const int at = (split * p.rows + c) * kTaggedBytes;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) store_device(pt, at + j * 256 + dch * 16, tagged(acc[2 * j], acc[2 * j + 1]));
+      if (dch == 0) store_device(pt, at + kHeadDim * 8, tagged(M, L));
+    } else if constexpr (FOLD == kFoldByFlags) {
       store_device(po, slot * kHeadDim * 4 + dch * 32, a0);
       store_device(po, slot * kHeadDim * 4 + dch * 32 + 16, a1);
       if (dch == 0) store_device(pml, slot * 8, ml);
@@ -449,7 +468,103 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       if (dch == 0) *reinterpret_cast<u32x2_t *>(p.ws_ml + (pair * pair_slots + slot) * 2) = ml;
     }
   }
-  if (!p.fold) return;
+  if constexpr (FOLD == kNoFold) return;
+
+  // Groups of 32 threads, four dims each: `parts` groups per row deal its splits out among themselves, if they are more
+  // than 8 (fewer: one group takes them all at once; 512 keys of 32 kv heads 6.75 -> 6.55 us, 1500 of 32 10.4 -> 9.45).
+  constexpr int NG = 2 * NW;
+  const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
+  const int at_once = min(p.rows, NG), parts = S <= kFoldDepth ? 1 : NG / at_once, part = sg / at_once;
+  float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = reinterpret_cast<float *>(lds) + 64;  // per group
+  // Folds the partials ml, ov of splits part, part + parts, ... of row c and stores the row, if all of them are `there` (up
+  // to 8 splits: they need not be).
+  auto fold = [&](int c, const auto &ml, const auto &ov, bool there) {
+    constexpr int D = sizeof(ml) / sizeof(ml[0]);
+    const bool mine = part < parts && c < p.rows;
+    float M = -INFINITY, L = 0.0f;
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < D; ++j)
+        if (part + parts * j < S) M = fmaxf(M, bits_float(ml[j][0]));
+      const float M_use = (M == -INFINITY) ? 0.0f : M;
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const float wt = (part + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
+        L += wt * bits_float(ml[j][1]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
+      }
+    }
+    if (parts > 1) {
+      if (d4 == 0) {
+        red_ml[2 * sg] = M;
+        red_ml[2 * sg + 1] = L;
+      }
+      *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
+      __syncthreads();
+      if (part == 0) {
+        for (int g2 = sg + at_once; g2 < parts * at_once; g2 += at_once) {
+          const float m2 = red_ml[2 * g2], Mn = fmaxf(M, m2);
+          const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
+          const float wa = fast_exp2(M - M_use), wb = fast_exp2(m2 - M_use);
+          L = L * wa + red_ml[2 * g2 + 1] * wb;
+          const f32x4_t o2 = *reinterpret_cast<const f32x4_t *>(red_o + g2 * kHeadDim + 4 * d4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] = acc[i] * wa + o2[i] * wb;
+          M = Mn;
+        }
+      }
+    }
+    if (part == 0 && c < p.rows && there) {
+      const int r = (int)fast_div(c, p.g_div);
+      const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
+      u32x2_t w;
+      w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
+      w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
+      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + c - r * p.g) * kRowBytes + d4 * 8) = w;
+    }
+  };
+
+  if constexpr (FOLD == kFoldByTags) {
+    // ---- fold whatever is there with this launch's tag beside every word ----
+    // Words that carry a tag need no flag behind them: two memory round trips (stored here, read all) where
+    // flags take four.  Each workgroup looks once its own words have reached the point where all XCDs see them, so
+    // that the last one to get there finds all of them; another one leaves out what is not there yet.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    constexpr int RI = (kTaggedRows + NG - 1) / NG, D = kFoldDepth;  // rows of a group, splits
+    const int piece = (d4 & 1) * 512 + (d4 >> 1) * 16;                // dims 4*d4 .. +3
+    u32x4_t a[RI][D][2], ml4[RI][D];
+    // (no branches: past the splits and rows the offset is past the buffer, and the load is not made)
+#pragma unroll
+    for (int r = 0; r < RI; ++r)
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const int c = r * at_once + sg;
+        const int at = sg < at_once && c < p.rows && j < S ? (j * p.rows + c) * kTaggedBytes : 0x40000000;
+        a[r][j][0] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece));
+        a[r][j][1] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece + 256));
+        ml4[r][j] = __builtin_bit_cast(u32x4_t, load_device(pt, at + kHeadDim * 8));
+      }
+#pragma unroll
+    for (int r = 0; r < RI; ++r) {
+      const int c = r * at_once + sg;
+      u32x2_t ml[D];
+      f32x4_t ov[D];
+      uint32_t differs = 0;
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const uint32_t d = (a[r][j][0][1] ^ p.tag) | (a[r][j][0][3] ^ p.tag) | (a[r][j][1][1] ^ p.tag) |
+                           (a[r][j][1][3] ^ p.tag) | (ml4[r][j][1] ^ p.tag) | (ml4[r][j][3] ^ p.tag);
+        differs |= j < S ? d : 0u;
+        ml[j] = u32x2_t{ml4[r][j][0], ml4[r][j][2]};
+        ov[j] = f32x4_t{bits_float(a[r][j][0][0]), bits_float(a[r][j][0][2]), bits_float(a[r][j][1][0]), bits_float(a[r][j][1][2])};
+      }
+      fold(c, ml, ov, differs == 0);
+    }
+    return;
+  }
 
   // ---- fold in the workgroup that finds every partial of its (sequence, kv head) stored ----
   // Each workgroup raises its flag once its partial has reached the point where all XCDs see it, and looks at the
@@ -472,81 +587,24 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   __syncthreads();
   if (*all_up == 0) return;
   if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
-  // Groups of 32 threads, four dims each: `parts` groups per row deal its splits out among themselves.
-  constexpr int NG = 2 * NW;
-  const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
-  const int at_once = min(p.rows, NG), parts = NG / at_once;
-  const int part = sg / at_once;
-  float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = reinterpret_cast<float *>(lds) + 64;  // per group
+  // every partial of a thread's share is asked for before the first is used
+  auto take = [&](int c, auto depth) {
+    constexpr int D = decltype(depth)::value;
+    u32x2_t ml[D];
+    f32x4_t ov[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      const int slot = min(part + parts * j, S - 1) * p.cols + min(c, p.rows - 1);
+      ml[j] = load_device2(pml, slot * 8);
+      ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
+    }
+    fold(c, ml, ov, true);
+  };
   for (int c0 = 0; c0 < p.rows; c0 += at_once) {
-    const int c = c0 + sg % at_once;
-    const bool mine = part < parts && c < p.rows;
-    float M = -INFINITY, L = 0.0f;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    // every partial of a thread's share is asked for before the first is used
-    auto take = [&](auto depth) {
-      constexpr int D = decltype(depth)::value;
-      const int s0 = part;
-      f32x4_t ov[D];
-      u32x2_t ml[D];
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const int slot = min(s0 + parts * j, S - 1) * p.cols + c;
-        ml[j] = load_device2(pml, slot * 8);
-        ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
-      }
-      float Mn = M;
-#pragma unroll
-      for (int j = 0; j < D; ++j)
-        if (s0 + parts * j < S) Mn = fmaxf(Mn, bits_float(ml[j][0]));
-      const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
-      const float resc = fast_exp2(M - M_use);
-      L *= resc;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] *= resc;
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const float wt = (s0 + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
-        L += wt * bits_float(ml[j][1]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
-      }
-      M = Mn;
-    };
-    if (mine) {
-      if (S <= kFoldDepth * parts)
-        take(std::integral_constant<int, kFoldDepth>());
-      else
-        take(std::integral_constant<int, kMaxFoldSplits>());
-    }
-    if (parts > 1) {
-      if (d4 == 0) {
-        red_ml[2 * sg] = M;
-        red_ml[2 * sg + 1] = L;
-      }
-      *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
-      __syncthreads();
-      if (part == 0) {
-        for (int g2 = sg + at_once; g2 < parts * at_once; g2 += at_once) {
-          const float m2 = red_ml[2 * g2], Mn = fmaxf(M, m2);
-          const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
-          const float wa = fast_exp2(M - M_use), wb = fast_exp2(m2 - M_use);
-          L = L * wa + red_ml[2 * g2 + 1] * wb;
-          const f32x4_t o2 = *reinterpret_cast<const f32x4_t *>(red_o + g2 * kHeadDim + 4 * d4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = acc[i] * wa + o2[i] * wb;
-          M = Mn;
-        }
-      }
-    }
-    if (part == 0 && c < p.rows) {
-      const int r = (int)fast_div(c, p.g_div);
-      const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-      u32x2_t w;
-      w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
-      w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
-      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + c - r * p.g) * kRowBytes + d4 * 8) = w;
-    }
+    if (S <= kFoldDepth * parts)
+      take(c0 + sg % at_once, std::integral_constant<int, kFoldDepth>());
+    else
+      take(c0 + sg % at_once, std::integral_constant<int, kMaxFoldSplits>());
   }
 }
 
@@ -641,9 +699,10 @@ int flash_decode_max_default_splits(long long pairs) {
 // of as many workgroups as the device has CUs; a CU of a full round streams 27.9 GB/s (all 256 of an
 // MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads), a CU of a thin
 // round the more the fewer they are (32 KiB in flight, a little more in short streams, over a latency that grows with
-// the load); a workgroup costs about 3 us beyond its bytes, folding up to 16 partials in the
-// kernel 3.1 us, 2.3 in blocks of 64 keys, the combine launch 2.3 us.  (Constants fitted over 250 shapes,
-// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %.)  Among the counts within
+// the load); a workgroup costs about 3 us beyond its bytes, folding up to 8 partials in the kernel 2.2 us, 1.2 in blocks of
+// 64 keys, up to 16 3.1 us, the combine launch 2.3 us.  (Constants fitted over 250 shapes,
+// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %; the fold of up to 8 over 180 of 130-4096
+// keys, where the count chosen is 0.35 % slower than the fastest on average: 2 x 384 keys of 32 kv heads 7.8 -> 6.95 us.)  Among the counts within
 // 3 % of the best, one that fills its rounds exactly is preferred, else the smallest.  For the common shapes
 // this is about one workgroup per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that
 // do not divide a round it finds the count that fills the rounds.  Over those shapes the count chosen is the
@@ -656,8 +715,8 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus) {
   double t = full * (wg_kb / 27.9 + 2.7);
   if (rest > 0) t += wg_kb / ((blocks >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
   if (s == 1) return t;
-  if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 2.3;
-  return t + (s <= kMaxFoldSplits ? 3.1 : 2.3);
+  if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 1.2;
+  return t + (s <= kFoldDepth ? 2.2 : s <= kMaxFoldSplits ? 3.1 : 2.3);
 }
 template <typename Model> static int best_splits(long long pairs, int smax, int cus, Model model) {
   double t_min = model(1);
@@ -758,13 +817,28 @@ static uint64_t launch_number() {
   return n;
 }
 
-template <typename T, bool FUSED, int NW, bool LONG>
+// A word that tells this launch's from the words of the 8 million launches before; a NaN, so no finite number that another
+// call left in the workspace has it.
+static uint32_t launch_tag() {
+  static std::atomic<uint32_t> next{std::random_device{}()};
+  const uint32_t n = next.fetch_add(1, std::memory_order_relaxed);
+  return 0x7fc00000u | (n & 0x3fffffu) | (n << 9 & 0x80000000u);
+}
+
+static bool may_be_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+template <typename T, bool FUSED, int NW, bool LONG, FoldMode FOLD>
 static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   // kDecLdsPad bytes of dynamic LDS that nobody touches keep a second workgroup off the CU (two of
   // them would put 64 KiB of loads in flight again).  More than 64 KiB of LDS in total is an opt-in
   // per device and kernel.
   constexpr int pad = NW == 4 ? kDecLdsPad : 0;
-  void (*kern)(DecodeParams) = flash_decode_kernel<T, FUSED, NW, LONG>;
+  void (*kern)(DecodeParams) = flash_decode_kernel<T, FUSED, NW, LONG, FOLD>;
   if (pad) {
     static std::atomic<uint64_t> attr_done{0};
     int dev = 0;
@@ -779,18 +853,29 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   }
   hipLaunchKernelGGL(kern, dim3(p.num_splits, p.Hkv, p.batch), dim3(64 * NW), pad, stream, p);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.num_splits == 1 || p.fold) return e;
+  if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
   hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
+template <typename T, bool FUSED, FoldMode FOLD>
+static hipError_t launch_decode_f(const DecodeParams &p, bool half, bool many, hipStream_t stream) {
+  if constexpr (FOLD != kNoFold) {  // (blocks of 64 keys come in splits of one, and few enough to be folded)
+    if (half) return launch_decode_t<T, FUSED, 2, false, FOLD>(p, stream);
+  }
+  if constexpr (FOLD != kFoldByTags) {
+    if (many) return launch_decode_t<T, FUSED, 4, true, FOLD>(p, stream);
+  }
+  return launch_decode_t<T, FUSED, 4, false, FOLD>(p, stream);
+}
 template <typename T, bool FUSED>
 static hipError_t launch_decode(const DecodeParams &p, bool half, bool many, hipStream_t stream) {
-  if (half) return launch_decode_t<T, FUSED, 2, false>(p, stream);
-  return many ? launch_decode_t<T, FUSED, 4, true>(p, stream) : launch_decode_t<T, FUSED, 4, false>(p, stream);
+  if (p.tag) return launch_decode_f<T, FUSED, kFoldByTags>(p, half, many, stream);
+  return p.fold ? launch_decode_f<T, FUSED, kFoldByFlags>(p, half, many, stream)
+                : launch_decode_f<T, FUSED, kNoFold>(p, half, many, stream);
 }
 
-static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, int num_splits, int dt, bool fused,
+static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t workspace_bytes, int num_splits, int dt, bool fused,
                                      hipStream_t stream) {
   p.num_splits = flash_decode_effective_splits(num_splits, p.n);
   p.cols = kDecCols;
@@ -809,6 +894,14 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, int num_s
   p.iters_rest = nblocks % p.num_splits;
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
   p.fold = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? launch_number() : 0;
+  // Up to 8 partials of up to 8 rows by tags instead of flags, where no workgroup has long to read them and the room is
+  // there (figures at the top; 5 x 2999 keys of 8 kv heads 14.7 / 14.4; 16 partials would be 116 KB to read for each workgroup
+  // of 7 query rows).  A replayed graph launches with the tag of its capture, and words of the replay before would pass for
+  // new ones: taken down by the folder, as flags are, they cost what the tags gain.
+  p.tag = 0;
+  if (p.fold && p.num_splits <= kFoldDepth && p.rows <= kTaggedRows && p.iters_each < 8 &&
+      (size_t)p.batch * p.Hkv * p.num_splits * p.rows * kTaggedBytes <= workspace_bytes && !may_be_capturing(stream))
+    p.tag = launch_tag();
   p.g_div = make_fast_div((uint32_t)p.g);
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
@@ -821,7 +914,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, int num_s
 }
 
 hipError_t launch_flash_decode(void *out, const void *q, const void *k, const void *v,
-                               void *workspace, int batch, int m, int n, int offset,
+                               void *workspace, size_t workspace_bytes, int batch, int m, int n, int offset,
                                int64_t kv_seq_stride, int group_size, int kv_head_num,
                                int num_splits, int dt, hipStream_t stream) {
   DecodeParams p = {};
@@ -838,14 +931,14 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
   p.Hkv = kv_head_num;
   p.H = group_size * kv_head_num;
   p.rows = m * group_size;
-  return launch_decode_impl(p, workspace, num_splits, dt, false, stream);
+  return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, false, stream);
 }
 
 // One decode step of one sequence with the rotary embedding and the cache append inside the decode
 // kernel: rows [0, pos) of the caches are read, row pos is produced from in_k / in_v and written.
 hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, const void *freq_cis,
                                     const void *in_q, const void *in_k, const void *in_v, void *workspace,
-                                    int pos, int group_size, int kv_head_num, int is_neox, int num_splits,
+                                    size_t workspace_bytes, int pos, int group_size, int kv_head_num, int is_neox, int num_splits,
                                     int dt, hipStream_t stream) {
   DecodeParams p = {};
   p.q = static_cast<const char *>(in_q);
@@ -866,7 +959,7 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
   p.freq_row = static_cast<const float *>(freq_cis) + (size_t)pos * kHeadDim;
   p.fused_pos = pos;
   p.is_neox = is_neox ? 1 : 0;
-  return launch_decode_impl(p, workspace, num_splits, dt, true, stream);
+  return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, true, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -901,7 +994,7 @@ hipError_t launch_flash_decode_static(void *out, const void *q, const void *k, c
     if (!ptr) return hipErrorInvalidSymbol;
     g_scratch_ptr[dev].store(ptr, std::memory_order_release);
   }
-  return launch_flash_decode(out, q, k, v, ptr, batch, 1, n, n - 1, kv_seq_stride, group_size,
+  return launch_flash_decode(out, q, k, v, ptr, kStaticDecodeScratchBytes, batch, 1, n, n - 1, kv_seq_stride, group_size,
                              kv_head_num, num_splits, dt, stream);
 }
 

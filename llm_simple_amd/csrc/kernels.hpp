@@ -41,7 +41,7 @@ size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num);
 // The split count a launch really uses for n keys: at most one split per block of 128 keys.
 int flash_decode_effective_splits(int num_splits, int n);
 hipError_t launch_flash_decode(void *out, const void *q, const void *k, const void *v,
-                               void *workspace, int batch, int m, int n, int offset,
+                               void *workspace, size_t workspace_bytes, int batch, int m, int n, int offset,
                                int64_t kv_seq_stride, int group_size, int kv_head_num,
                                int num_splits, int dt, hipStream_t stream);
 
@@ -50,7 +50,7 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
 // the last key range write row pos of both caches, attention runs over rows [0, pos].
 hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, const void *freq_cis,
                                     const void *in_q, const void *in_k, const void *in_v, void *workspace,
-                                    int pos, int group_size, int kv_head_num, int is_neox, int num_splits,
+                                    size_t workspace_bytes, int pos, int group_size, int kv_head_num, int is_neox, int num_splits,
                                     int dt, hipStream_t stream);
 
 // Same decode with the split-KV partials in a fixed device array of kStaticDecodeScratchBytes inside

@@ -99,7 +99,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     int splits = flash_decode_default_splits(1, n_vis, kv_head_num);
     const size_t need = flash_decode_workspace_bytes(1, m, group_size, kv_head_num, splits);
     if (!need)
-      return from_hip(launch_flash_decode(out, q, k, v, nullptr, 1, m, n_vis, offset, n_vis, group_size,
+      return from_hip(launch_flash_decode(out, q, k, v, nullptr, 0, 1, m, n_vis, offset, n_vis, group_size,
                                           kv_head_num, splits, dt, as_stream(stream)));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     StreamScratch *ws = nullptr;
@@ -107,7 +107,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
         stream, need, [&] { return flash_decode_least_workspace_bytes(1, n_vis, kv_head_num); }, &ws);
     if (rc != LLMHIP_OK) return rc;
     if (ws->bytes < need) splits = flash_decode_splits_within(1, n_vis, kv_head_num, ws->bytes);
-    return from_hip(launch_flash_decode(out, q, k, v, ws->ptr, 1, m, n_vis, offset, n_vis,
+    return from_hip(launch_flash_decode(out, q, k, v, ws->ptr, ws->bytes, 1, m, n_vis, offset, n_vis,
                                         group_size, kv_head_num, splits, dt,
                                         as_stream(stream)));
   }
@@ -196,7 +196,7 @@ int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,
   if (num_splits > kMaxDecodeSplits) num_splits = kMaxDecodeSplits;  // the combine kernel's limit
   const size_t need = flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits);
   if (need > room) return LLMHIP_ERR_WORKSPACE;
-  return from_hip(launch_flash_decode(out, q, k_cache, v_cache, workspace, batch, 1, n, n - 1,
+  return from_hip(launch_flash_decode(out, q, k_cache, v_cache, workspace, room, batch, 1, n, n - 1,
                                       kv_seq_stride, group_size, kv_head_num, num_splits, dt,
                                       as_stream(stream)));
 }
@@ -243,7 +243,7 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
   int splits = flash_decode_default_splits(1, n, kv_head_num);
   const size_t need = flash_decode_workspace_bytes(1, 1, group_size, kv_head_num, splits);
   if (!need)
-    return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, nullptr, pos,
+    return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, nullptr, 0, pos,
                                              group_size, kv_head_num, is_neox_style, splits, dt,
                                              as_stream(stream)));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
@@ -252,7 +252,7 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
       stream, need, [&] { return flash_decode_least_workspace_bytes(1, n, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
   if (ws->bytes < need) splits = flash_decode_splits_within(1, n, kv_head_num, ws->bytes);
-  return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, ws->ptr, pos, group_size,
+  return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, ws->ptr, ws->bytes, pos, group_size,
                                            kv_head_num, is_neox_style, splits, dt, as_stream(stream)));
 }
 
