@@ -62,6 +62,7 @@ constexpr int kTileN = 64;                      // keys per LDS tile (128 where 
 constexpr int kTileBytes = kTileN * kRowBytes;  // 16 KiB
 constexpr float kLazyLog2 = 8.0f;                // rescale threshold, log2 units
 constexpr int kMaxPrefillSplits = 128;           // key ranges per call
+constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
 struct PrefillParams {
   const char *q;
@@ -451,6 +452,38 @@ __device__ __forceinline__ void store_partial(const WaveAttn<T, KB> &w, float *o
   }
 }
 
+// The same through LDS: stored straight from the accumulator layout an instruction touches 32 rows with 32 bytes each, this
+// way it writes whole pieces of 128*ND bytes (us: 200 tokens past 16001, 28 heads 55.1 -> 54.6; 64 past 3936, 40 heads 18.7 ->
+// 18.15; 500 past 2500, 32 heads 36.4 -> 35.8; not so where few waves have rows at all, 4 past 5396, 28 heads 9.86 ->
+// 10.0: up to kFewRows rows they go straight).  lds_wave: 4*ND KiB of this
+// wave's own; o_row(r): d block 0 of row r of the wave's 32, of which rows_valid exist.
+template <int D0, int ND, typename T, int KB, typename Row>
+__device__ __forceinline__ void store_partial_rows(const WaveAttn<T, KB> &w, char *lds_wave, Row o_row, float *ml_row, bool row_valid,
+                                                   int rows_valid) {
+  constexpr int G = 8 * ND, RB_ = G * 16, RPI = 64 / G;  // granules and bytes of a row, rows per instruction
+  const float l_tot = pair_sum(w.l_run);
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const f32x4_t v = {w.o[D0 + d][4 * i4], w.o[D0 + d][4 * i4 + 1], w.o[D0 + d][4 * i4 + 2], w.o[D0 + d][4 * i4 + 3]};
+      const int gran = 8 * d + 2 * i4 + w.hh;
+      *reinterpret_cast<f32x4_t *>(lds_wave + w.l32 * RB_ + ((gran ^ (w.l32 & (G - 1))) << 4)) = v;
+    }
+  if (D0 == 0 && w.hh == 0 && row_valid) {
+    ml_row[0] = w.m_run;
+    ml_row[1] = l_tot;
+  }
+  __builtin_amdgcn_wave_barrier();  // wave-private region: LDS ops of one wave complete in order
+  const int r0 = w.lane / G, g0 = w.lane % G;
+#pragma unroll
+  for (int t = 0; t < 32 / RPI; ++t) {
+    const int r = RPI * t + r0;
+    const u32x4_t v = lds_read_b128(lds_wave, r * RB_ + ((g0 ^ (r & (G - 1))) << 4));
+    if (r < rows_valid) *reinterpret_cast<u32x4_t *>(o_row(r) + D0 * 32 + g0 * 4) = v;
+  }
+}
+
 // One global_load_lds_dwordx4: lane l's 16 bytes at `src` land at the wave-uniform LDS address lds_addr + 16*l.
 __device__ __forceinline__ void lds_dma(const char *src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -715,6 +748,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   }
   // every wave is past the last barrier of the loop: nobody reads the K/V tiles any more
   char *out_blk = p.out + (size_t)qblk0 * q_row_bytes + (size_t)head * kRowBytes;
+  auto part_row = [&](int r) {  // where the partial of row r of the wave's goes
+    int tok = qblk0 + r, h = head;
+    if (p.pack) {
+      const int idx = tok;
+      tok = (int)fast_div(idx, p.g_div);
+      h = head + idx - tok * p.g;
+    }
+    return p.ws_o + (((size_t)split * p.m + tok) * p.H + h) * kHeadDim;
+  };
   if constexpr (KP > 1) {
     constexpr int kTrade = WaveAttn<T, KB>::trade_bytes(KP), ND = 4 / KP;
     char *rows_lds = lds + rb * kTrade;
@@ -723,7 +765,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     auto finish = [&](auto part) {
       constexpr int PART = decltype(part)::value;
       w.template take<KP, PART>(rows_lds, p.scale_log2e);
-      if (p.num_splits > 1)
+      if (p.num_splits > 1 && rows > kFewRows)
+        store_partial_rows<PART * ND, ND>(w, lds + RB * kTrade + wave * (32 * 128 * ND), part_row, part_ml, row_valid, rows - qblk0);
+      else if (p.num_splits > 1)
         store_partial<PART * ND, ND>(w, part_o, part_ml, row_valid);
       else
         w.template store<PART * ND, ND>(lds + RB * kTrade + wave * (32 * 64 * ND), out_blk, q_row_bytes, p.m - qblk0);
@@ -735,7 +779,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       if (kpar == 3) finish(std::integral_constant<int, 3>());
     }
   } else if (p.num_splits > 1) {  // (packed rows exist in split mode only)
-    store_partial(w, part_o, part_ml, row_valid);
+    if (rows > kFewRows)
+      store_partial_rows<0, 4>(w, lds + rb * 32 * 512, part_row, part_ml, row_valid, rows - qblk0);
+    else
+      store_partial(w, part_o, part_ml, row_valid);
   } else {
     w.store(lds + rb * 32 * kRowBytes, out_blk, q_row_bytes, p.m - qblk0);
   }
