@@ -1040,15 +1040,15 @@ static size_t partial_bytes(long long splits, int m, long long H) {
 //     workgroups as CUs from 1500 keys on: 2048 tokens 24.6 / 28.8 (12 heads)
 //   two waves per 64 rows up to 1.3 128-row workgroups per CU: 1019 tokens 17.8 / 19.2 (28), 1400 25.6 / 25.8
 //   two waves per 128 rows up to 2 per CU: 1700 tokens 34.0 / 35.3 (28)
-//   256 rows from 1.5 workgroups per CU: 3500 tokens 107.8 / 111 (28); 128 rows of one wave each below: 3000 tokens
-//     81.7 / 85.8
+//   256 rows from more than 1.5 workgroups per CU on: 3500 tokens 107.8 / 111 (28); 128 rows of one wave each up to there:
+//     3000 tokens 81.7 / 85.8, 80.2 / 82.6 (32), 8192 tokens 188 / 202 (12)
 static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
   auto per_cu = [&](int rows) { return (double)((m + rows - 1) / rows) * H / cus; };
   if (n_vis > 96 && per_cu(32) <= 1.05) return kQuad32;
   if ((n_vis >= 480 && per_cu(64) <= 1.05) || (n_vis >= 1500 && per_cu(64) <= 2.0)) return kQuad64;
   if (per_cu(128) <= 1.3) return kPair64;
   if (per_cu(128) <= 2.0) return kPair128;
-  return per_cu(256) >= 1.5 ? kRows256 : kRows128;
+  return per_cu(256) > 1.5 ? kRows256 : kRows128;
 }
 
 // A chunk behind a longer cache makes few workgroups with many keys each: its key range is cut, and with fewer rows than a
