@@ -197,22 +197,11 @@ template <typename T, int KB = 2> struct WaveAttn {
     }
   }
 
-  __device__ __forceinline__ void load_q(const char *q_row_head) {
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) qf[kk] = global_load_b128(q_row_head + hh * 16 + kk * 32);
-  }
-  // The same fragments of 32 rows in LDS, laid out like a K tile; off: their place less this wave's first tile row
+  // Q^T fragments of 32 rows in LDS, laid out like a K tile; off: their place less this wave's first tile row
   __device__ __forceinline__ void load_q_lds(const char *lds, int off) {
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) qf[kk] = lds_read_b128(lds, k_addr[kk] + off);
   }
-  // The Q loads are complete after this: no wait inside the key loop is ever
-  // attributed to them.
-  __device__ __forceinline__ void pin_q() {
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(qf[kk]));
-  }
-
   struct NoHook {
     template <typename I> __device__ __forceinline__ void operator()(I) const {}
   };
@@ -551,6 +540,8 @@ template <int NW, int TN, bool NT> struct DirectLoader {
     else asm volatile("buffer_load_dwordx4 %0, %1, 0 offen offset:%2 lds" : : "v"(off), "s"(st.d), "n"(at));
   }
   static __device__ __forceinline__ void wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+  // All but the last N loads of the wave
+  template <int N> static __device__ __forceinline__ void wait_but() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 };
 
 // ---------------------------------------------------------------------------
@@ -634,25 +625,22 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     }
   }
   // Q.  A fragment load straight into the operand layout touches 32 rows with 32 bytes each, 256 tag look-ups per
-  // wave; where KP waves share the rows, Q goes through LDS like a K tile instead, fetched once as whole
-  // rows (256 tokens, 32 heads, two waves per 64 rows: 7.4 -> 7.0 us).
-  constexpr int kQRegion = 2 * NSLOT * TB;  // behind the K and V tiles
-  if constexpr (KP > 1) {
+  // wave; Q goes through LDS like a K tile instead, fetched once as whole rows, and the first scores wait for it and K
+  // tile 0 only (256 tokens, 32 heads, two waves per 64 rows: 7.4 -> 7.0 us; the wait 6.1 -> 5.9).  Its place is behind the K
+  // and V tiles, or, where every row has one wave, begins with the V slots that the first stage fills.
+  constexpr int kQRegion = KP > 1 ? 2 * NSLOT * TB : kVRegion + SUB * TB;
 #pragma unroll
-    for (int sl = 0; sl < 8 / KP; ++sl) {
-      const int r = 4 * (sl * NW + wave) + (lane >> 4);
-      const int idx = min(row0 + r, rows - 1);
-      const char *src = p.q + ((lane & 15) ^ (r & 15)) * 16;
-      if (p.pack) {
-        const int tok = (int)fast_div(idx, p.g_div);
-        src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * p.g) * kRowBytes;
-      } else {
-        src += (size_t)idx * q_row_bytes + (size_t)head * kRowBytes;
-      }
-      lds_dma(src, kQRegion + (sl * NW + wave) * 4 * kRowBytes);
+  for (int sl = 0; sl < 8 / KP; ++sl) {
+    const int r = 4 * (sl * NW + wave) + (lane >> 4);
+    const int idx = min(row0 + r, rows - 1);
+    const char *src = p.q + ((lane & 15) ^ (r & 15)) * 16;
+    if (p.pack) {
+      const int tok = (int)fast_div(idx, p.g_div);
+      src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * p.g) * kRowBytes;
+    } else {
+      src += (size_t)idx * q_row_bytes + (size_t)head * kRowBytes;
     }
-  } else {
-    w.load_q(p.q + (size_t)qtok * q_row_bytes + (size_t)qhead * kRowBytes);
+    lds_dma(src, kQRegion + (sl * NW + wave) * 4 * kRowBytes);
   }
 
   DirectLoader<NW, TN, NT> ld;
@@ -670,15 +658,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       ld.next(vst, J);
     }
   });
-  if (KP == 1) w.pin_q();  // the Q fragments are in registers from here on
-  ld.wait_all();
+  ld.template wait_but<2 * SUB * PER>();  // Q and K tile 0
   lds_barrier();
-  if (KP > 1) w.load_q_lds(lds, kQRegion + (rb - kpar) * 32 * kRowBytes);
+  w.load_q_lds(lds, kQRegion + (rb - (KP > 1 ? kpar : 0)) * 32 * kRowBytes);
 
   f32x16_t sa[KB], sb[KB];  // scores of the current / the next tile, roles alternate
   if (Jw > 0) w.qk(lds, 0, sa);
   // A K load of the first stage lands where tile 0 was just read: no wave may issue it (one without rows would at
   // once) before all have read.
+  ld.wait_all();
   lds_barrier();
 
   auto tile_step = [&](int j, int slot, f32x16_t (&s_cur)[KB], f32x16_t (&s_nxt)[KB]) {
@@ -949,7 +937,8 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   p.list_heads = make_fast_div((uint32_t)list_heads);
   p.per_split = make_fast_div((uint32_t)(list_heads * T_));
   p.g_div = make_fast_div((uint32_t)p.g);
-  const size_t lds_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes + (KP > 1 ? (size_t)BM * kRowBytes : 0);  // tiles, Q
+  const size_t tile_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes, q_bytes = (size_t)BM * kRowBytes;
+  const size_t lds_bytes = tile_bytes + (KP > 1 ? q_bytes : q_bytes - tile_bytes / 4);  // (half of the V slots are Q's at first)
   // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KP == 1 there)
   const bool nt = KP == 1 && p.pack && T_ == 1;
   void (*kern)(PrefillParams) = flash_prefill_kernel<T, NW, KP, false>;
