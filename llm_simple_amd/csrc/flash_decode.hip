@@ -817,12 +817,12 @@ static uint64_t launch_number() {
   return n;
 }
 
-// A word that tells this launch's from the words of the 8 million launches before; a NaN, so no finite number that another
-// call left in the workspace has it.
+// A word that tells this launch's words from those of the 4 million launches before.  It is a NaN, so that no finite number
+// another call left in the workspace has it, with its last bit set, so that no NaN widened from 16 bits has it either.
 static uint32_t launch_tag() {
   static std::atomic<uint32_t> next{std::random_device{}()};
   const uint32_t n = next.fetch_add(1, std::memory_order_relaxed);
-  return 0x7fc00000u | (n & 0x3fffffu) | (n << 9 & 0x80000000u);
+  return 0x7fc00001u | (n & 0x1fffffu) << 1 | (n << 10 & 0x80000000u);
 }
 
 static bool may_be_capturing(hipStream_t stream) {
