@@ -8,9 +8,10 @@ from helpers import DT_BFLOAT16, DT_FLOAT16, check_attention, dev_empty, normal_
 
 pytestmark = pytest.mark.gpu
 
-# (m, past, H, Hkv): 32 rows x 4 waves, 64 x 4, 64 x 2, 128 x 2, 128 and 256 rows, chunks (cut, packed, whole)
+# (m, past, H, Hkv): 32 rows x 4 waves, 64 x 4, 64 x 2 (two workgroups to a CU: 705 tokens; heads in one list: 1300), 128 x 2,
+# 128 and 256 rows, chunks (cut, packed, whole)
 CASES = [(129, 0, 12, 1), (191, 0, 12, 2), (513, 0, 28, 4), (575, 0, 14, 1), (640, 0, 40, 8), (705, 0, 40, 8), (1089, 0, 40, 8),
-         (1151, 0, 32, 32), (1665, 0, 40, 8), (1983, 0, 40, 8), (2049, 0, 28, 1), (3, 254, 28, 1), (40, 961, 16, 1), (40, 1047, 28, 4),
+         (1151, 0, 32, 32), (1300, 0, 20, 5), (1665, 0, 40, 8), (1983, 0, 40, 8), (2049, 0, 28, 1), (3, 254, 28, 1), (40, 961, 16, 1), (40, 1047, 28, 4),
          (2, 4095, 28, 4), (255, 1730, 28, 4)]
 
 
