@@ -63,8 +63,6 @@ template <> struct Elem<_Float16> {
   static __device__ __forceinline__ uint16_t round(float f) {
     return __builtin_bit_cast(uint16_t, (_Float16)f);
   }
-  static __device__ __forceinline__ float low(uint32_t pair) { return widen((uint16_t)pair); }
-  static __device__ __forceinline__ float high(uint32_t pair) { return widen((uint16_t)(pair >> 16)); }
 };
 
 template <> struct Elem<__bf16> {
@@ -88,8 +86,6 @@ template <> struct Elem<__bf16> {
   // (src/util.cpp:33-72) on every finite input, and a NaN stays one whatever its payload (added to the bit
   // pattern, the rounding carries 0xFFFFFFFF over to 0).
   static __device__ __forceinline__ uint16_t round(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
-  static __device__ __forceinline__ float low(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
-  static __device__ __forceinline__ float high(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
 };
 
 // n / d for 32-bit n by multiply and shift (Granlund-Montgomery, round-up variant): exact for every n.

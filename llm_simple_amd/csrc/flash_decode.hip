@@ -699,10 +699,11 @@ int flash_decode_max_default_splits(long long pairs) {
 // of as many workgroups as the device has CUs; a CU of a full round streams 27.9 GB/s (all 256 of an
 // MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads), a CU of a thin
 // round the more the fewer they are (32 KiB in flight, a little more in short streams, over a latency that grows with
-// the load); a workgroup costs about 3 us beyond its bytes, folding up to 8 partials in the kernel 2.2 us, 1.2 in blocks of
-// 64 keys, up to 16 3.1 us, the combine launch 2.3 us.  (Constants fitted over 250 shapes,
-// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %; the fold of up to 8 over 180 of 130-4096
-// keys, where the count chosen is 0.35 % slower than the fastest on average: 2 x 384 keys of 32 kv heads 7.8 -> 6.95 us.)  Among the counts within
+// the load); a workgroup costs about 3 us beyond its bytes, folding up to 8 partials in the kernel 2.0 us, 1.2 in blocks of
+// 64 keys, up to 16 2.6 us, the combine launch 2.1 us.  (Constants of the streams fitted over 250 shapes,
+// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %; those of the folds over 515 of batch 1-16
+// x 2-32 kv heads x 130-7000 keys, where the count chosen is 0.3 % slower than the fastest on average: 2 x 384 keys of 32 kv
+// heads 7.8 -> 6.95 us; 9 x 3943 of 2 kv heads takes 11 or more parts, 11.6 us, where 8 take 11.9.)  Among the counts within
 // 3 % of the best, one that fills its rounds exactly is preferred, else the smallest.  For the common shapes
 // this is about one workgroup per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that
 // do not divide a round it finds the count that fills the rounds.  Over those shapes the count chosen is the
@@ -716,7 +717,7 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus) {
   if (rest > 0) t += wg_kb / ((blocks >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
   if (s == 1) return t;
   if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 1.2;
-  return t + (s <= kFoldDepth ? 2.2 : s <= kMaxFoldSplits ? 3.1 : 2.3);
+  return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
 }
 template <typename Model> static int best_splits(long long pairs, int smax, int cus, Model model) {
   double t_min = model(1);
