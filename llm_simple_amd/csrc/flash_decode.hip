@@ -818,7 +818,8 @@ static uint64_t launch_number() {
   return n;
 }
 
-// A word that tells this launch's words from those of the 4 million launches before.  It is a NaN, so that no finite number
+// A word that tells this launch's words from those of the 4 million launches before (mistaken for its own would be one that was
+// stored exactly 2^22 tagged launches ago, or a multiple, where none has stored since).  It is a NaN, so that no finite number
 // another call left in the workspace has it, with its last bit set, so that no NaN widened from 16 bits has it either.
 static uint32_t launch_tag() {
   static std::atomic<uint32_t> next{std::random_device{}()};
