@@ -26,9 +26,9 @@
 // fp32 partial (max, sum, unnormalised O).
 //
 // Up to 16 partials of a (sequence, kv head) are folded (log-sum-exp) by the workgroup that finds them all stored, with no
-// fence and no atomic.  Up to 8: every word goes past the XCD's L2 (sc1 stores) with the launch's tag beside it, and
-// whoever finds the tag at all of them folds them; that is two memory round trips.  More, or where the tag would be that of
-// a replay: partials, then a flag, then a look at the other flags, then the partials, four round trips.  (The fused step,
+// fence and no atomic.  Up to 8: every word goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it,
+// and whoever finds the number at all of them folds them; that is two memory round trips.  More, or where the number would be
+// that of a replay: partials, then a flag, then a look at the other flags, then the partials, four round trips.  (The fused step,
 // us, flags / tags: 384 keys of 2 kv heads 6.9 / 5.95, 512 of 32 7.4 / 6.25, 1000 of 8 7.75 / 7.15, 1500 of 32 11.3 / 9.15;
 // the combine launch takes 3.1 us, and 2.4 of the host's.)  More partials make more rounds of loads in ONE workgroup (32:
 // 11.2 against 8.8 us at batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses
@@ -52,6 +52,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "launch_number.hpp"
 
 namespace llmhip {
 
@@ -77,8 +78,7 @@ struct DecodeParams {
   FastDiv g_div;
   float scale_log2e;
   int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
-  uint64_t fold;  // not 0: the workgroup of a (sequence, kv head) that finds this number in all flags folds
-  uint32_t tag;   // not 0 (fold only): each word of a partial is stored with this one beside it, and there are no flags
+  uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial (see FoldMode)
   // Fused decode step (FUSED kernels only): the token at row fused_pos = n - 1 is not in the cache yet.
   // q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
   // q and the new K row are rotated with table row freq_row (64 (cos, sin) pairs) as they are loaded,
@@ -411,8 +411,9 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
   const int tagged_bytes = p.num_splits * p.rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + pair * tagged_bytes, tagged_bytes);
+  const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
   auto tagged = [&](float x, float y) {
-    return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), p.tag, __builtin_bit_cast(uint32_t, y), p.tag});
+    return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), tag0, __builtin_bit_cast(uint32_t, y), tag1});
   };
   for (int c = tid >> 4; c < p.rows; c += 4 * NW) {
     const int dch = tid & 15;  // 8-wide d chunk of column c
@@ -527,9 +528,10 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   };
 
   if constexpr (FOLD == kFoldByTags) {
-    // ---- fold whatever is there with this launch's tag beside every word ----
+    // ---- fold whatever is there with this launch's number beside its words ----
     // Words that carry a tag need no flag behind them: two memory round trips (stored here, read all) where
-    // flags take four.  Each workgroup looks once its own words have reached the point where all XCDs see them, so
+    // flags take four.  The two words of a 16-byte piece carry a half each: a piece that an earlier launch stored differs in
+    // both, whenever that was (one half repeats after 2.97e9 launches, both after 2^64).  Each workgroup looks once its own words have reached the point where all XCDs see them, so
     // that the last one to get there finds all of them; another one leaves out what is not there yet.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
@@ -555,8 +557,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       uint32_t differs = 0;
 #pragma unroll
       for (int j = 0; j < D; ++j) {
-        const uint32_t d = (a[r][j][0][1] ^ p.tag) | (a[r][j][0][3] ^ p.tag) | (a[r][j][1][1] ^ p.tag) |
-                           (a[r][j][1][3] ^ p.tag) | (ml4[r][j][1] ^ p.tag) | (ml4[r][j][3] ^ p.tag);
+        const uint32_t d = (a[r][j][0][1] ^ tag0) | (a[r][j][0][3] ^ tag1) | (a[r][j][1][1] ^ tag0) |
+                           (a[r][j][1][3] ^ tag1) | (ml4[r][j][1] ^ tag0) | (ml4[r][j][3] ^ tag1);
         differs |= j < S ? d : 0u;
         ml[j] = u32x2_t{ml4[r][j][0], ml4[r][j][2]};
         ov[j] = f32x4_t{bits_float(a[r][j][0][0]), bits_float(a[r][j][0][2]), bits_float(a[r][j][1][0]), bits_float(a[r][j][1][2])};
@@ -806,25 +808,16 @@ size_t flash_decode_workspace_bytes(int batch, int m, int group_size, int kv_hea
   return slots * (kHeadDim + 2) * sizeof(float);
 }
 
-// A number that no workspace holds by chance: the flags of a folding launch (see the kernel).
+// A number that no workspace holds: of a launch, see launch_number.hpp.  (By chance 2^-64, from a random start.)
 static uint64_t launch_number() {
-  static std::atomic<uint64_t> next{[] {
+  static std::atomic<uint64_t> last{[] {
     std::random_device rd;
     return ((uint64_t)rd() << 32) ^ rd() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
   }()};
-  uint64_t n;
-  do n = next.fetch_add(0x9E3779B97F4A7C15ull, std::memory_order_relaxed);
-  while (n == 0);
+  uint64_t before = last.load(std::memory_order_relaxed), n;
+  do n = next_launch_number(before);
+  while (!last.compare_exchange_weak(before, n, std::memory_order_relaxed));
   return n;
-}
-
-// A word that tells this launch's words from those of the 4 million launches before (mistaken for its own would be one that was
-// stored exactly 2^22 tagged launches ago, or a multiple, where none has stored since).  It is a NaN, so that no finite number
-// another call left in the workspace has it, with its last bit set, so that no NaN widened from 16 bits has it either.
-static uint32_t launch_tag() {
-  static std::atomic<uint32_t> next{std::random_device{}()};
-  const uint32_t n = next.fetch_add(1, std::memory_order_relaxed);
-  return 0x7fc00001u | (n & 0x1fffffu) << 1 | (n << 10 & 0x80000000u);
 }
 
 static bool may_be_capturing(hipStream_t stream) {
@@ -871,10 +864,10 @@ static hipError_t launch_decode_f(const DecodeParams &p, bool half, bool many, h
   return launch_decode_t<T, FUSED, 4, false, FOLD>(p, stream);
 }
 template <typename T, bool FUSED>
-static hipError_t launch_decode(const DecodeParams &p, bool half, bool many, hipStream_t stream) {
-  if (p.tag) return launch_decode_f<T, FUSED, kFoldByTags>(p, half, many, stream);
-  return p.fold ? launch_decode_f<T, FUSED, kFoldByFlags>(p, half, many, stream)
-                : launch_decode_f<T, FUSED, kNoFold>(p, half, many, stream);
+static hipError_t launch_decode(const DecodeParams &p, FoldMode how, bool half, bool many, hipStream_t stream) {
+  if (how == kFoldByTags) return launch_decode_f<T, FUSED, kFoldByTags>(p, half, many, stream);
+  return how == kFoldByFlags ? launch_decode_f<T, FUSED, kFoldByFlags>(p, half, many, stream)
+                             : launch_decode_f<T, FUSED, kNoFold>(p, half, many, stream);
 }
 
 static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t workspace_bytes, int num_splits, int dt, bool fused,
@@ -895,15 +888,15 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   p.iters_each = nblocks / p.num_splits;
   p.iters_rest = nblocks % p.num_splits;
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
-  p.fold = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? launch_number() : 0;
+  FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
+  p.fold = how != kNoFold ? launch_number() : 0;
   // Up to 8 partials of up to 8 rows by tags instead of flags, where no workgroup has long to read them and the room is
   // there (figures at the top; 5 x 2999 keys of 8 kv heads 14.7 / 14.4; 16 partials would be 116 KB to read for each workgroup
-  // of 7 query rows).  A replayed graph launches with the tag of its capture, and words of the replay before would pass for
-  // new ones: taken down by the folder, as flags are, they cost what the tags gain.
-  p.tag = 0;
-  if (p.fold && p.num_splits <= kFoldDepth && p.rows <= kTaggedRows && p.iters_each < 8 &&
+  // of 7 query rows).  A replayed graph launches with the number of its capture, and words of the replay before would pass
+  // for new ones: taken down by the folder, as flags are, they cost what the tags gain.
+  if (how == kFoldByFlags && p.num_splits <= kFoldDepth && p.rows <= kTaggedRows && p.iters_each < 8 &&
       (size_t)p.batch * p.Hkv * p.num_splits * p.rows * kTaggedBytes <= workspace_bytes && !may_be_capturing(stream))
-    p.tag = launch_tag();
+    how = kFoldByTags;
   p.g_div = make_fast_div((uint32_t)p.g);
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
@@ -911,8 +904,8 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;
   const bool many = p.iters_each >= 8;  // long enough to be bound by the stream, see the kernel
   if (dt == kDtFloat16)
-    return fused ? launch_decode<_Float16, true>(p, half, many, stream) : launch_decode<_Float16, false>(p, half, many, stream);
-  return fused ? launch_decode<__bf16, true>(p, half, many, stream) : launch_decode<__bf16, false>(p, half, many, stream);
+    return fused ? launch_decode<_Float16, true>(p, how, half, many, stream) : launch_decode<_Float16, false>(p, how, half, many, stream);
+  return fused ? launch_decode<__bf16, true>(p, how, half, many, stream) : launch_decode<__bf16, false>(p, how, half, many, stream);
 }
 
 hipError_t launch_flash_decode(void *out, const void *q, const void *k, const void *v,

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../llm_simple_amd/csrc/device_hip.hpp"
+#include "../../llm_simple_amd/csrc/launch_number.hpp"
 
 using namespace llm_simple_amd;
 
@@ -392,7 +393,33 @@ static void test_profiler_file() {
   EXPECT(!mm.Init(nullptr, nullptr, 16, 16, DT_FLOAT16));
 }
 
+// A workspace keeps the words of earlier launches for as long as nothing else is stored there: no launch may carry the
+// number of one before it, nor a half of it beside its words.
+static void test_launch_numbers() {
+  const uint64_t first = llmhip::next_launch_number(0x123456789abcdef1ull);
+  uint64_t n = first, again = 0;
+  for (int i = 0; i < 1 << 24; ++i) {
+    n = llmhip::next_launch_number(n);
+    again += (uint32_t)n == (uint32_t)first || n >> 32 == first >> 32;
+  }
+  EXPECT(again == 0);
+  const uint64_t step = llmhip::next_launch_number(1) - 1;
+  EXPECT(step % 2 == 1);  // (so that 2^64 launches have as many numbers and 2^32 as many lower halves)
+  // upper halves of two numbers differ whatever they are, if the numbers are 2^32 or more apart both ways around
+  uint64_t close = 0;
+  for (uint64_t d = 1; d <= 1ull << 28; ++d) close += (d * step < 1ull << 32) + (0 - d * step < 1ull << 32);
+  EXPECT(close == 0);
+  uint64_t far = 0;
+  for (uint64_t d = 1ull << 22; d < 1ull << 31; d += 1ull << 18) far += (d * step < 1ull << 32) + (0 - d * step < 1ull << 32);
+  EXPECT(far == 0);
+  // a half of zero is what cleared memory holds
+  EXPECT(llmhip::next_launch_number(0 - step) == step);
+  EXPECT(llmhip::next_launch_number((5ull << 32) - step) == (5ull << 32) + step);
+  EXPECT(llmhip::next_launch_number(7 - step) == 7 + step);
+}
+
 int main() {
+  test_launch_numbers();
   test_profiler_file();
   test_sizes();
   test_allocator_pool();

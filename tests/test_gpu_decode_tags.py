@@ -46,3 +46,37 @@ def test_tagged_partials(dt, room):
             replayed.fill_(0x7FFF)
             graph.replay()
             assert np.array_equal(to_host(replayed), want)
+
+
+@pytest.mark.parametrize("halves", [(1, 0), (0, 1), (0, 0)])
+def test_half_a_number_is_not_the_number(halves):
+    """A workspace full of partials with one half of the launch's own number beside every word (the sequence of numbers:
+    tests/cpp/test_device_host.cpp): none of them may be folded."""
+    import torch
+    import llm_simple_amd.ops as ops
+    # 9 blocks in 7 splits, the last workgroups in a second round: some look long before others have stored
+    b, n, H, Hkv, splits, dt = 10, 1100, 16, 4, 7, DT_BFLOAT16
+    q = normal_bits(1, (b, 1, H, 128), dt)
+    k, v = normal_bits(2, (b, n, Hkv, 128), dt), normal_bits(3, (b, n, Hkv, 128), dt)
+    need = ops.flash_decode_workspace_bytes(b, H // Hkv, Hkv, 128, splits)
+    ws = torch.zeros(need // 4, dtype=torch.int32, device="cuda")
+    args = (to_dev(q), to_dev(k), to_dev(v), ws, need, b, n, n, H // Hkv, Hkv, 128, splits, dt)
+    out = dev_empty((b, 1, H, 128))
+    ops.hip_flash_decode_gqa_layer(out, *args)
+    want = to_host(out)
+    check_attention(want, q, k, v, n, n - 1, dt, batch=True)
+
+    def number():  # of the last launch: beside the first two words of the first partial
+        words = ws[:4].cpu().numpy().view(np.uint32)
+        return int(words[1]) | int(words[3]) << 32
+
+    for _ in range(20):
+        due = (number() + 0x9E3779B97F4A7C15) % 2 ** 64
+        piece = np.array([1e3, 0, 1e3, 0], dtype=np.float32).view(np.uint32)
+        piece[1] = (due & 0xffffffff) ^ (0 if halves[0] else 1 << 17)
+        piece[3] = (due >> 32) ^ (0 if halves[1] else 1 << 17)
+        ws.copy_(torch.from_numpy(np.tile(piece, need // 16).view(np.int32)))
+        out.fill_(0x7FFF)
+        ops.hip_flash_decode_gqa_layer(out, *args)
+        assert np.array_equal(to_host(out), want)
+        assert number() == due  # tags, and of the number foreseen
