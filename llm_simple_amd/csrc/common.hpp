@@ -15,6 +15,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 // The measurement library (libllmhip_bench.so) compiles the prefill kernel a second time with
 // LLMHIP_BENCH defined (a clock stamp in the kernel); its copy lives in a namespace of its own so
@@ -111,11 +112,11 @@ __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // f(integral_constant<int, I>) ... f(integral_constant<int, N - 1>)
+template <int I, typename F, int... J> __device__ __forceinline__ void static_for_each(F &f, std::integer_sequence<int, J...>) {
+  (f(std::integral_constant<int, I + J>()), ...);
+}
 template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>());
-    static_for<I + 1, N>(f);
-  }
+  static_for_each<I>(f, std::make_integer_sequence<int, (N > I ? N - I : 0)>());
 }
 
 // acc + lo + hi of a packed pair of storage-type values.

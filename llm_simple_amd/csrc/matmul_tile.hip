@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
   static_for<0, NR>([&](auto r) { read(r, 0, 0); });
   constexpr int R1 = NR + 4 > NM ? 2 : 1;               // fragment reads of a slot
   constexpr int READ = (NR + R1 - 1) / R1 + 5;          // by this slot the reads of a phase have come back
-  constexpr int PH = 2 * KS, BS = (PH - 2) * NM + (READ < NM ? READ : NM), DS = PH * NM - BS;
+  constexpr int PH = 2 * KS, BS = (PH - 2) * NM + (READ < NM ? READ : NM), DS = PH * NM - BS, NL = KS * L;
   // One stage.  LEFT: stages under way beyond the next one; LOAD: fetch another; NEXT: there is a next one.
   auto stage = [&](auto left, auto load, auto next_) {
     constexpr int LEFT = decltype(left)::value;
@@ -182,13 +182,14 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
         if constexpr (r < NR && (h < PH - 1 || NEXT))
           read(std::integral_constant<int, r>(), (h + 1) & 1, h == PH - 1 ? next : slot + (h + 1) / 2 * kLineBytes);
       });
-      static_for<0, KS * L>([&](auto l_) {
-        constexpr int l = decltype(l_)::value;
-        if constexpr (LOAD && BS + l * DS / (KS * L) == j) {
+      if constexpr (LOAD && j >= BS) {  // load l in slot BS + l * DS / NL
+        constexpr int first = ((j - BS) * NL + DS - 1) / DS, end = ((j + 1 - BS) * NL + DS - 1) / DS;
+        static_for<first, end>([&](auto l_) {
+          constexpr int l = decltype(l_)::value;
           issue(std::integral_constant<int, l % L>(), wbase + kpos, xbase + kpos, fetch + l / L * kLineBytes);
           if (l % L == L - 1) advance();
-        }
-      });
+        });
+      }
       __builtin_amdgcn_sched_barrier(0);
       acc[q % MT][q / MT] = E::mfma16(wf[h & 1][q / MT], xf[h & 1][q % MT], acc[q % MT][q / MT]);
       __builtin_amdgcn_sched_barrier(0);
