@@ -275,11 +275,13 @@ template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_
 }
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
-// Over 227 sizes (15 weights of 256-11008 rows and k of 1536-18944, 17-4096 lhs rows) the choice takes 0.81 of hipBLASLt's
-// time on average.  Left to hipBLASLt, which cuts k, are few small tiles over a long k (us, hipBLASLt / here: 1024 x 8192, 17
-// rows 10.1 / 13.1, 100 rows 12.7 / 13.7; 2048 x 8192, 24 rows 13.7 / 16.3; not so 1024 x 5120, 48 rows 14.2 / 9.4).  Taken
-// though slower: 5120 x 5120, 64 rows 22.2 / 23.8, 4096 x 11008, 680 rows 83.5 / 87.4.  More than one round is not:
-// 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 / 54.5 with 128 x 128.
+// Over 270 sizes (16 weights of 256-11008 rows and k of 1536-18944, 17-4096 lhs rows, W from HBM) it takes 0.80 of hipBLASLt's
+// time on average.  Taken though slower, so that no such call needs hipBLASLt's handle and 64 MiB workspace (which a stream under
+// capture cannot create): few rows over k = 8192, which hipBLASLt cuts (us, hipBLASLt / here: 1024 x 8192, 17 rows 11.8 / 15.4,
+// 64 rows 13.8 / 17.5; 2048 x 8192, 24 rows 14.0 / 18.3; 4096 x 8192, 17 rows 17.2 / 17.2, 32 rows 18.3 / 20.3; not so 1536 x
+// 8960, 17 rows 28.2 / 19.0, 3584 x 18944, 32 rows 109.6 / 48.4); 5120 x 5120, 64 rows 21.5 / 22.9; 4096 x 11008, 680 rows 80.5 /
+// 85.0.  More than one round is not: 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 /
+// 54.5 with 128 x 128.
 int tile_kind(int m, int n, int k) {
   static const struct { int m, n; } tiles[] = {{32, 32},   {64, 32},   {64, 64},   {96, 64},   {128, 64},
                                                {96, 96},   {96, 128},  {128, 96},  {128, 128}, {128, 160},
@@ -287,7 +289,7 @@ int tile_kind(int m, int n, int k) {
   const long long cus = device_compute_units();
   for (int kind = 0; kind < 15; ++kind) {
     const long long count = (long long)((m + tiles[kind].m - 1) / tiles[kind].m) * ((n + tiles[kind].n - 1) / tiles[kind].n);
-    if (count <= cus) return kind == 0 && k > 6144 && 2 * count <= cus ? -1 : kind;
+    if (count <= cus) return kind;
   }
   return -1;
 }
