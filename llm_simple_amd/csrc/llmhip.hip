@@ -439,15 +439,21 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
   if (m < 1 || n < 1 || k < 1 || !dtype_ok(dt)) return LLMHIP_ERR_INVALID_ARG;
   if (n % 16 != 0 || k % 16 != 0) return LLMHIP_ERR_UNSUPPORTED;
   // Up to 16 rows one MFMA column block holds every lhs row and the call is a read of W; beyond that lhs, which
-  // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  From 9 rows on that is so already
-  // where W has more than 8 rows per CU (W from HBM, us, few-row kernel / tiles: 3584 x 3584, 9 rows 7.7 / 7.2, 16 rows 8.9
-  // / 7.2; 4096 x 4096, 9 rows 9.8 / 8.4; 3072 x 8192, 9 rows 16.9 / 15.7; not so 2048 x 2048, 9 rows 4.8 / 5.1, 512 x 3584,
-  // 12 rows 6.1 / 6.7, nor with 8 rows of a long k: 3072 x 8192 13.6 / 18.2).  Both kernels move 16-byte pieces; hipBLASLt
-  // takes any base.
+  // every workgroup of that kernel reads whole, outweighs W, and tiles are shared.  From 9 rows on that is so already where W has
+  // more than one round of its workgroups takes, 16 rows per CU, or where rows times W rows per CU, its work beside the stream,
+  // pass a bound, lower over a long k (W from HBM, us, few-row kernel / tiles: 4352 x 5120, 9 rows 15.3 / 12.3; 5120 x 3584 11.6 /
+  // 9.6; 4096 x 4096, 12 rows 10.5 / 9.6; 3584 x 3584, 9 rows 8.2 / 9.0, 16 rows 9.5 / 9.6; 2560 x 3584 7.0 / 8.4, 8.5 / 9.1; long:
+  // 4096 x 11008, 9 rows 28.4 / 22.5, 3584 x 18944, 12 rows 39.1 / 38.0, 2560 x 8192, 9 rows 13.4 / 15.5).  Over 322 sizes of
+  // 512-11008 W rows, k of 1536-18944 and 9-16 rows the kernel chosen is 0.4 % slower than the better one on average, 16 % at most (3072
+  // x 11008, 9 rows); by a line at 16 rows per CU alone 1.8 %, at 8 2.7 %.  With 8 rows neither is ahead by much: 4352 x 5120 13.1
+  // / 12.4, 11008 x 18944 75.4 / 79.4.  (With W in the last-level cache the tiles are ahead earlier, 3584 x 3584, 9 rows 7.3 / 6.8,
+  // but the weights of a model's other layers lie between two calls.)  Both kernels move 16-byte pieces; hipBLASLt takes any
+  // base.
   if (all_aligned16(out, lhs, weight)) {
     const float *b = static_cast<const float *>(bias);
     const bool tiles = m > 8 && matmul_tile_takes(m, n, k);
-    if (m <= 16 && !(tiles && n > 8LL * device_compute_units()))
+    const long long per_cu = (n + device_compute_units() - 1) / device_compute_units();
+    if (m <= 16 && !(tiles && (per_cu > 16 || m * per_cu > (k > 7168 ? 130 : 190))))
       return from_hip(launch_matmul_skinny(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));
     if (tiles)
       return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream)));

@@ -42,9 +42,12 @@ def test_stages(tile, size, depth, dt):
 
 
 @pytest.mark.parametrize("dt", [DT_FLOAT16, DT_BFLOAT16])
-@pytest.mark.parametrize("m,n,k", [(9, 2048, 320), (9, 2064, 320), (16, 2064, 64), (8, 2064, 128), (13, 3584, 704)])
+@pytest.mark.parametrize("m,n,k", [(9, 2048, 320), (9, 2064, 320), (16, 2064, 64), (8, 2064, 128), (13, 3584, 704),
+                                   (11, 4096, 320), (12, 4096, 320), (9, 4112, 320), (8, 4112, 320), (10, 3328, 7232),
+                                   (11, 3328, 7232), (11, 3328, 7168), (16, 2064, 7232), (8, 4112, 7232)])
 def test_few_rows_line(dt, m, n, k):
-    """Either side of the line (2048 features, 8 rows) from which the tiles take calls of up to 16 rows."""
+    """Up to 16 rows, either side of the lines from which the tiles take such calls: 8 rows; 4096 features; rows times features
+    per compute unit of 190, and of 130 where k is beyond 7168."""
     import llm_simple_amd.ops as ops
     x = normal_bits(m + k, (m, k), dt)
     w = orc.round_to(orc.widen(normal_bits(n, (n, k), dt), dt) / np.sqrt(k), dt)

@@ -1,4 +1,4 @@
-"""9 to 16 lhs rows against a wide weight go to the tiled kernel (more than 2048 rows on 256 compute units): 8 and 9 rows,
+"""9 to 16 lhs rows against a wide weight go to the tiled kernel (more than 4096 rows on 256 compute units): 8 and 9 rows,
 both kernels, and k in part stages (which the tiles do not take), against the oracle."""
 import numpy as np
 import pytest
