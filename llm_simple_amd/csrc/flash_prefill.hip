@@ -491,7 +491,7 @@ __device__ __forceinline__ void lds_dma(const char *src, uint32_t lds_addr) {
 // that belongs there.  A tile of TN keys is TN/4 instructions; slot s of wave w covers rows 4*(w*kSlots + s) .. +3.
 // The lane offsets never change and rows past the end are cut off by the descriptor (they read as zero), so a load costs no
 // vector ALU work, and M0 is written for every fourth one only: the instruction's offset moves both addresses, and
-// the lane offsets make up for it.  The loads are issued from inline asm: the compiler would order every later LDS
+// the lane offsets make up for it.  (That nothing else uses M0 in between is checked in the built code, check_m0.py.)  The loads are issued from inline asm: the compiler would order every later LDS
 // read behind a transfer it knows about (s_waitcnt vmcnt(0)).  Completion is waited for explicitly before the barrier that
 // publishes a stage.
 typedef __attribute__((ext_vector_type(4))) uint32_t buffer_t;

@@ -64,7 +64,7 @@ template <int N> __device__ __forceinline__ void wait_loads() {
 }
 
 // global_load_lds_dwordx4, OFF (0, 1024, 2048 or 3072) added to the global address and to the LDS address in M0, which
-// nothing but the assembly of this kernel writes
+// nothing but the assembly of this kernel uses (checked in the built code, check_m0.py)
 template <int OFF> __device__ __forceinline__ void line_load(uint32_t voff, const char *base) {
   if constexpr (OFF == 0) asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base));
   else asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(base), "n"(OFF));
