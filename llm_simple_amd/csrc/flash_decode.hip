@@ -29,8 +29,8 @@
 // fence and no atomic.  Up to 8: every word goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it,
 // and whoever finds the number at all of them folds them; that is two memory round trips.  More, or where the number would be
 // that of a replay: partials, then a flag, then a look at the other flags, then the partials, four round trips.  (The fused step,
-// us, flags / tags: 384 keys of 2 kv heads 6.9 / 5.95, 512 of 32 7.4 / 6.25, 1000 of 8 7.75 / 7.15, 1500 of 32 11.3 / 9.15;
-// the combine launch takes 3.1 us, and 2.4 of the host's.)  More partials make more rounds of loads in ONE workgroup (32:
+// us, flags / tags, cache lines warm: 384 keys of 2 kv heads 6.6 / 5.9, 512 of 32 6.2 / 5.55, 1000 of 8 6.8 / 6.4, 1500 of 32
+// 8.9 / 8.1; the combine launch takes 3.1 us, and 2.4 of the host's.)  More partials make more rounds of loads in ONE workgroup (32:
 // 11.2 against 8.8 us at batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses
 // write back and invalidate the XCD's L2: 91 us against 33 at batch 1, 32768 keys.)
 //
@@ -157,6 +157,7 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
 constexpr int kMaxFoldSplits = 16;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
 constexpr int kTaggedRows = 8;                    // query rows whose words carry a tag, at most
+constexpr size_t kTaggedReads = 7u << 20;         // bytes that the workgroups of a launch read to look for tags, at most
 constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   if constexpr (FOLD == kNoFold) return;
 
   // Groups of 32 threads, four dims each: `parts` groups per row deal its splits out among themselves, if they are more
-  // than 8 (fewer: one group takes them all at once; 512 keys of 32 kv heads 6.75 -> 6.55 us, 1500 of 32 10.4 -> 9.45).
+  // than 8 (fewer: one group takes them all at once; by flags, 512 keys of 32 kv heads 6.65 -> 6.2 us, 1500 of 32 9.9 -> 8.9).
   constexpr int NG = 2 * NW;
   const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
   const int at_once = min(p.rows, NG), parts = S <= kFoldDepth ? 1 : NG / at_once, part = sg / at_once;
@@ -890,12 +891,16 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
   FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
-  // Up to 8 partials of up to 8 rows by tags instead of flags, where no workgroup has long to read them and the room is
-  // there (figures at the top; 5 x 2999 keys of 8 kv heads 14.7 / 14.4; 16 partials would be 116 KB to read for each workgroup
-  // of 7 query rows).  A replayed graph launches with the number of its capture, and words of the replay before would pass
-  // for new ones: taken down by the folder, as flags are, they cost what the tags gain.
+  // Up to 8 partials of up to 8 rows by tags instead of flags, where the room is there and what the workgroups read together,
+  // each the partials of its (sequence, kv head) and that past the L2s, is at most 7 MB: beyond 8 it takes longer than the two
+  // round trips that it saves (us, flags / tags, K and V from HBM; 532 shapes of 1-32 sequences, 1-32 kv heads, 130-8000 keys:
+  // up to 1 MB tags are 6 % faster on average, at 5 MB 3 %; 6 to 8 MB even, 5 x 3000 keys of 8 kv heads 14.6 / 14.4 in one
+  // run, 14.24 / 14.44 in another; 12 MB, 8 x 2000 of 4, 7 query rows 10.7 / 11.8; 17 MB, 16 x 1000 of 2, 8 rows 8.8 / 10.2).
+  // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones: taken
+  // down by the folder, as flags are, they cost what the tags gain.
+  const size_t tagged = (size_t)p.batch * p.Hkv * p.num_splits * p.rows * kTaggedBytes;
   if (how == kFoldByFlags && p.num_splits <= kFoldDepth && p.rows <= kTaggedRows && p.iters_each < 8 &&
-      (size_t)p.batch * p.Hkv * p.num_splits * p.rows * kTaggedBytes <= workspace_bytes && !may_be_capturing(stream))
+      tagged <= workspace_bytes && tagged * p.num_splits <= kTaggedReads && !may_be_capturing(stream))
     how = kFoldByTags;
   p.g_div = make_fast_div((uint32_t)p.g);
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
