@@ -41,8 +41,8 @@
 // instruction, K and V rows are read through buffer descriptors (the hardware bounds them, no clamps), integer
 // divisions are prepared by the host, the column maximum goes through permlane swaps, masks and the
 // rescaling of O run only where they change something, and the merge of the waves is free of bank conflicts (it cost
-// 1.4 us).  4.1 us now; 384 keys of 2 kv heads 9.7 -> 6.9 us, 512 keys of 32 kv heads 9.1 -> 6.6, 4096 keys of 8
-// 10.9 -> 9.2, 32768 keys of 8 28.4 -> 24.8 (fused step, back-to-back calls, before the tags).
+// 1.4 us).  4.1 us now; 384 keys of 2 kv heads 9.7 -> 6.6 us, 512 keys of 32 kv heads 9.1 -> 6.2, 4096 keys of 8
+// 10.9 -> 9.2, 32768 keys of 8 28.4 -> 24.8 (fused step, back-to-back calls, by flags).
 //
 // (Eight-wave workgroups, half as many, merging pairs of splits through LDS: 4.5 TB/s against 6.0 at the time.)
 #include <atomic>

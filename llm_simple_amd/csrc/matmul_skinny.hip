@@ -1,6 +1,6 @@
 // Projection of few rows (one generated token, a handful of tokens): out[m][n] = lhs[m][k] . W[n][k]^T + bias,
-// fp32 accumulation, one rounding, m <= 16 (from 9 rows on only where W has at most 16 rows per CU: the tiled kernel is
-// faster beyond).
+// fp32 accumulation, one rounding, m <= 16 (from 9 rows on only where W has few rows: the tiled kernel is faster
+// beyond, lines and figures in matmul_common).
 //
 // Bound by reading W once.  W is dealt out in equal shares of whole rows (at most 16) to one workgroup per
 // CU, two or more rounds of them for a wide n: a CU cannot have more than its 32 KiB of first-level cache

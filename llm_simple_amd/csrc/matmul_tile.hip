@@ -5,18 +5,20 @@
 // lines of every operand row).  Lines travel global -> LDS without registers, STAGES of them in flight or in use; a
 // fragment load straight into the operand layout, 16 rows by 64 bytes, ran at a third of the rate.
 // Four waves, one per SIMD, take a quadrant each.  A wave issues one instruction every 4-5 cycles and an MFMA takes
-// 16, so that two others fit between two MFMAs: the loop is written as slots, one MFMA and at most a fragment read
-// and a line load each, and a line load is one instruction (constant lane offsets, the LDS address in M0 for four of
-// them at a time).  The loads of a stage are spread over its whole length: a CU takes in 64 bytes per cycle and no more
-// (128 x 224: 704 cycles of loads beside 896 of MFMAs), and loads issued over half a stage held the wave up for the
-// other half (3584 x 3584, 2048 rows: loop 41.3 -> 39.0 us).  One barrier a stage, where the last fragments of this
-// stage have come back: it frees the stage's place and publishes the next one.
+// 16, so that two others fit between two MFMAs: the loop is written as slots, one MFMA each with the fragment reads (one; two
+// in tiles of up to 96 x 96) and line loads that go out before it, and a line load is one instruction (constant lane
+// offsets, the LDS address in M0 for four of them at a time).  One barrier a stage, where the last fragments of this
+// stage have come back: it frees the stage's place and publishes the next one.  The loads of a stage are spread over the slots
+// behind it, at most one to a slot where a stage has one line: the last 40 of 56 of 128 x 224, half of them in tiles of up to 128 x
+// 96.  A CU takes in 64 bytes per cycle and no more (128 x 224: 704 cycles of loads beside 896 of MFMAs), and the fewer slots
+// share them the longer the loads hold the wave up (3584 x 3584, 2048 rows, over 28 and over 40 slots: loop 41.3, 39.0 us).
 //   Eight waves, two for each quadrant on alternate halves of k, hide more latency but trade their sums through LDS
 // at the end and issue more: 3584 x 3584, 2048 rows 54.9 us, this kernel 46.2; 4096 x 4096 67.6 / 59.3; 1536 x 1536,
 // 2048 rows 17.5 / 13.7; 512 x 3584, 2048 rows 14.8 / 13.6.  mfma_32x32x16, with half the operand reads, is no
 // faster (4096 x 4096 62.3 / 57.9), the power it saves being small.
 //   Small tiles are bound by the barrier and the LDS latency of a stage, and take several lines per stage (32 x 32, four
-// lines instead of two: 512 x 3584, 400 rows 8.5 -> 7.8 us; 1536 x 1536, 100 rows 5.4 -> 4.9).
+// lines instead of two: 512 x 3584, 400 rows 8.5 -> 7.8 us; 1536 x 1536, 100 rows 5.4 -> 4.9).  There the barrier comes so late that
+// the loads go out in a burst behind it: 32 x 32 all eight in the last of 8 slots, 64 x 32 twelve in the last two of 16.
 // Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 2.6 until the first
 // lines are in, 56 stages of 0.67, 2.3 for the store (14.7 MB at once), the rest launch.  A stage takes 1120 cycles at
 // 1.68 GHz: the clock is what the power leaves (half of the chip: 1090 cycles at 2.2 GHz; without the line loads 1.9 GHz).
@@ -29,9 +31,10 @@
 // memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
 // (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5, kernel of eight waves).
 //
-// bf16, us, hipBLASLt (without its 10 us of host time) / here, W from HBM: 3584 x 3584: 64 rows 10.9 / 7.9, 128 rows
-// 18.0 / 10.4, 256 rows 16.9 / 13.4, 768 rows 29.1 / 23.4, 2048 rows 54.4 / 46.2; 512 x 3584: 100 rows 11.2 / 7.4,
-// 2048 rows 17.1 / 13.6; 1536 x 1536: 128 rows 7.6 / 5.3; 5120 x 5120: 100 rows 28.6 / 25.8, 1280 rows 77.4 / 61.2.
+// bf16, us, hipBLASLt / here, back-to-back calls, W walked through 800 MB (hipBLASLt takes the host 10-13 us a call, which is
+// what its small sizes show): 3584 x 3584: 64 rows 13.7 / 11.1, 128 rows 22.5 / 14.5, 256 rows 20.1 / 18.8, 768 rows 32.2 / 26.8,
+// 2048 rows 55.9 / 47.0; 512 x 3584: 100 rows 13.4 / 7.1, 2048 rows 19.3 / 13.2; 1536 x 1536: 128 rows 9.7 / 5.7; 5120 x 5120: 100
+// rows 27.6 / 25.2, 1280 rows 76.1 / 59.8.
 #include <atomic>
 #include <type_traits>
 
