@@ -16,22 +16,21 @@
 // separately (this file is compiled with -ffp-contract=off), one rounding to
 // the storage type.  Pairing: interleaved (2f, 2f+1) or neox (f, f + 64).
 //
-// Pure streaming: a unit is 32 bytes of a 256-byte head row (8 units per row; 8 pairs: two 128-bit
-// loads, 64 bytes of the fp32 table, two 128-bit stores), Q, K and V rows alike -- a V row is copied
-// by the same 8 lanes without the arithmetic.  A thread takes kRopeUnits units a whole grid apart and
-// issues all their loads before it computes.  The pairing style is a template parameter, the storage
-// type is rounded by the hardware conversion (equal to round-to-nearest-even on the bit pattern for
-// every non-NaN fp32), the token of a unit comes from a multiply-shift division.  (Measured at
-// 4096 tokens of Qwen2.5-7B: 13.1 us with the buffers in the last-level cache, 16.4 us from and to HBM, where a
-// plain device copy of the same bytes takes 16; the same kernel without arithmetic and table 12.2 us, so the rest
-// is the memory path of three separate streams of 256-byte rows.  256 tokens, 32 heads 4.1 us, of which the
-// launch is 2.5.)
+// Pure streaming: a thread takes 32 bytes of a 256-byte head row, 16 of either half (8 pairs: two 128-bit
+// loads, 64 bytes of the fp32 table, two 128-bit stores; 8 lanes per row, whole lines in either pairing style), Q, K and
+// V rows alike -- a V row is copied by the same 8 lanes without the arithmetic.  The pairing style is a template
+// parameter, the storage type is rounded by the hardware conversion (equal to round-to-nearest-even on the bit pattern for
+// every non-NaN fp32), the token of a row comes from a multiply-shift division.
+//
+// Bound by the memory path of three separate streams of 256-byte rows.  4096 tokens of 28 + 2 x 4 heads (75.5 MB): 11.9 us
+// with the buffers in the last-level cache, 15.2 from and to HBM, where a plain device copy of the same bytes takes
+// 10.4 and 16; 256 tokens of 32 + 2 x 32 heads 3.1 us, of which an empty launch is 1.55.  One piece to a thread: two, a
+// grid apart, kept half as many waves (a layer's rope and attention, us, two / one: 64 tokens of 32 heads 8.29 / 8.02,
+// 256 10.80 / 10.52, 1500 41.9 / 40.9, 256 of 12 9.03 / 8.61).
 #include "common.hpp"
 #include "kernels.hpp"
 
 namespace llmhip {
-
-constexpr int kRopeUnits = 2;  // 32-byte units per thread, a grid apart: twice the loads in flight per wave
 
 struct RopeParams {
   const char *in_q, *in_k, *in_v;
@@ -84,52 +83,32 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t 
 
 template <typename T, bool NEOX>
 __global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
-  constexpr int U = kRopeUnits;
-  const uint32_t stride = gridDim.x * 256u;
-  const uint32_t gid0 = blockIdx.x * 256u + threadIdx.x;
-  u32x4_t va[U], vb[U];
-  f32x4_t cs[U][4];
-  char *outp[U];
-  bool rot[U], live[U];
-  const uint32_t j = gid0 & 7u;  // stride is a multiple of 8
-  const int off_a = NEOX ? (int)j * 16 : (int)j * 32;
-  const int off_b = NEOX ? off_a + 128 : off_a + 16;
-  // All loads of a thread go out before anything is waited for, the table's included (a V row's are not used): asked for
-  // when a unit is rotated, the second unit's table was one more memory round trip (with non-temporal stores, from and
-  // to HBM, 4096 tokens 16.25 -> 15.2 us, 1019 tokens 6.75 -> 5.9; rope and attention of 256 tokens, 32 heads 13.3 -> 13.0).
+  const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
+  if (gid >= p.total) return;
+  const uint32_t j = gid & 7u, rowid = gid >> 3, s = fast_div(rowid, p.rows_per_token);
+  const int r = (int)(rowid - s * p.rows_per_token.d);
+  const bool is_q = r < p.q_heads, rotated = r < p.q_heads + p.k_heads;
+  const int heads = is_q ? p.q_heads : p.k_heads;  // V has as many as K
+  const int h = is_q ? r : rotated ? r - p.q_heads : r - p.q_heads - p.k_heads;
+  const char *in = is_q ? p.in_q : rotated ? p.in_k : p.in_v;
+  char *out = is_q ? p.out_q : rotated ? p.out_k : p.out_v;
+  in += ((size_t)s * heads + h) * kRowBytes + j * 16;
+  out += ((size_t)(s + (is_q ? 0 : p.k_out_row_offset)) * heads + h) * kRowBytes + j * 16;
+  const float *tab = p.freq_cis + (size_t)(p.start_pos + s) * kHeadDim + (NEOX ? 16 : 8) * j;
+  // All loads go out before anything is waited for, the table's included (a V row's are not used)
+  u32x4_t a = global_load_b128(in), b = global_load_b128(in + 128);
+  f32x4_t cs[4];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const uint32_t gid = gid0 + u * stride;
-    live[u] = gid < p.total;
-    const uint32_t rowid = (live[u] ? gid : 0u) >> 3;
-    const uint32_t s = fast_div(rowid, p.rows_per_token);
-    const int r = (int)(rowid - s * p.rows_per_token.d);
-    const bool is_q = r < p.q_heads;
-    rot[u] = r < p.q_heads + p.k_heads;
-    const int heads = is_q ? p.q_heads : p.k_heads;  // V has as many as K
-    const int h = is_q ? r : rot[u] ? r - p.q_heads : r - p.q_heads - p.k_heads;
-    const char *in = is_q ? p.in_q : rot[u] ? p.in_k : p.in_v;
-    char *out = is_q ? p.out_q : rot[u] ? p.out_k : p.out_v;
-    in += ((size_t)s * heads + h) * kRowBytes;
-    outp[u] = out + ((size_t)(s + (is_q ? 0 : p.k_out_row_offset)) * heads + h) * kRowBytes;
-    const float *tab = p.freq_cis + (size_t)(p.start_pos + s) * kHeadDim + 16 * j;
-    va[u] = global_load_b128(in + off_a);
-    vb[u] = global_load_b128(in + off_b);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) cs[u][i] = *reinterpret_cast<const f32x4_t *>(tab + 4 * i);
-  }
+  for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4_t *>(tab + (NEOX ? 4 * i : 64 * (i >> 1) + 4 * (i & 1)));
   __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (rot[u]) rotate8<T, NEOX>(va[u], vb[u], cs[u]);
-    if (live[u]) {
-      // Ordinary stores: the attention launch reads the rows next.  Non-temporal ones make this launch shorter by itself
-      // (1019 tokens 5.2 -> 4.5 us, 4096 from and to HBM 16.4 -> 15.2) and the pair longer: rope and attention of 256
-      // tokens, 32 heads 12.3 -> 13.05 us, 1019 tokens, 28 heads 22.9 -> 26.5, 4096 131.2 -> 133.0, 8192 446 -> 450.
-      *reinterpret_cast<u32x4_t *>(outp[u] + off_a) = va[u];
-      *reinterpret_cast<u32x4_t *>(outp[u] + off_b) = vb[u];
-    }
-  }
+  if (rotated) rotate8<T, NEOX>(a, b, cs);
+  // Past the L2: the attention launch that follows finds nothing to wait for, and every instruction writes whole lines
+  // (interleaved pairs used to be 32 bytes of a lane, stored by halves: 1019 tokens of 32 heads then take 32.8 us this way).
+  // Rope and attention, us, ordinary stores / these: 256 tokens of 28 heads 9.88 / 9.38, 1019 of 28 21.9 / 20.8, 400 of 40
+  // 13.7 / 12.7, 4096 of 28 130.8 / 130.1; whole lines alone 256 tokens of 32 heads, interleaved, 11.7 -> 11.3, both 10.6.
+  // (Non-temporal stores are shorter still by themselves, and the rows then come back from HBM: 1019 tokens 24.3.)
+  store_device_b128(out, a);
+  store_device_b128(out + 128, b);
 }
 
 hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const void *freq_cis,
@@ -156,7 +135,7 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   if (rows > 0x7FFFFFFFLL || total > 0x7FFFFFFFLL) return hipErrorInvalidValue;  // 32-bit thread index
   p.rows_per_token = make_fast_div((uint32_t)rows);
   p.total = (uint32_t)total;
-  const int grid = (int)((total + 256 * kRopeUnits - 1) / (256 * kRopeUnits));
+  const int grid = (int)((total + 255) / 256);
   void (*kern)(RopeParams) =
       (dt == kDtFloat16) ? (is_neox ? rope_kv_append_kernel<_Float16, true> : rope_kv_append_kernel<_Float16, false>)
                          : (is_neox ? rope_kv_append_kernel<__bf16, true> : rope_kv_append_kernel<__bf16, false>);
