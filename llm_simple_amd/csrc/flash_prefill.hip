@@ -392,7 +392,9 @@ template <typename T, int KB = 2> struct WaveAttn {
   // rows with 16 bytes each; the tile goes through 2*ND KiB of LDS of this wave instead
   // (16-byte granule XOR row: conflict-free both ways with four d blocks; rows of one or two are shorter
   // than the banks, and up to 8 lanes meet in one, 1-2 % of a launch's cycles) and leaves as whole pieces of
-  // 64*ND bytes, 4*ND lanes per row.  lds_wave: this wave's region; out_blk: &out[first row of the
+  // 64*ND bytes, 4*ND lanes per row, past the L2: lines that are left there are written back at the end of the launch (rope
+  // and attention, us, ordinary stores / these: 256 tokens of 28 heads 9.39 / 9.20, 600 14.64 / 14.16, 1019 20.5 / 19.7, of
+  // 32 26.3 / 25.7, 2048 of 28 44.5 / 43.8; up to 128 tokens and from 4096 on the same).  lds_wave: this wave's region; out_blk: &out[first row of the
   // wave][head]; rows_valid: how many of the wave's 32 rows exist.
   template <int D0 = 0, int ND = 4>
   __device__ __forceinline__ void store(char *lds_wave, char *out_blk, size_t row_bytes, int rows_valid) {
@@ -420,7 +422,7 @@ template <typename T, int KB = 2> struct WaveAttn {
     char *dst = out_blk + (size_t)r0 * row_bytes + D0 * 64 + g0 * 16;
 #pragma unroll
     for (int t = 0; t < 2 * ND; ++t) {
-      if (RPI * t + r0 < rows_valid) *reinterpret_cast<u32x4_t *>(dst) = v[t];
+      if (RPI * t + r0 < rows_valid) store_device_b128(dst, v[t]);
       dst += RPI * row_bytes;
     }
   }
@@ -448,7 +450,8 @@ __device__ __forceinline__ void store_partial(const WaveAttn<T, KB> &w, float *o
 // The same through LDS: stored straight from the accumulator layout an instruction touches 32 rows with 32 bytes each, this
 // way it writes whole pieces of 128*ND bytes (us: 200 tokens past 16001, 28 heads 55.1 -> 54.6; 64 past 3936, 40 heads 18.7 ->
 // 18.15; 500 past 2500, 32 heads 36.4 -> 35.8; not so where few waves have rows at all, 4 past 5396, 28 heads 9.86 ->
-// 10.0: up to kFewRows rows they go straight).  lds_wave: 4*ND KiB of this
+// 10.0: up to kFewRows rows they go straight), and past the L2 (100 past 8000, 40 heads 29.5 -> 28.7; 200 past 16001, 28 heads
+// 57.8 -> 56.8; 450 past 10000 78.9 -> 78.0; 100 past 8000, 32 heads of one kv head each 43.1 -> 43.8).  lds_wave: 4*ND KiB of this
 // wave's own; o_row(r): d block 0 of row r of the wave's 32, of which rows_valid exist.
 template <int D0, int ND, typename T, int KB, typename Row>
 __device__ __forceinline__ void store_partial_rows(const WaveAttn<T, KB> &w, char *lds_wave, Row o_row, float *ml_row, bool row_valid,
@@ -473,7 +476,7 @@ __device__ __forceinline__ void store_partial_rows(const WaveAttn<T, KB> &w, cha
   for (int t = 0; t < 32 / RPI; ++t) {
     const int r = RPI * t + r0;
     const u32x4_t v = lds_read_b128(lds_wave, r * RB_ + ((g0 ^ (r & (G - 1))) << 4));
-    if (r < rows_valid) *reinterpret_cast<u32x4_t *>(o_row(r) + D0 * 32 + g0 * 4) = v;
+    if (r < rows_valid) store_device_b128(o_row(r) + D0 * 32 + g0 * 4, v);
   }
 }
 
