@@ -6,8 +6,7 @@
 // CU, two or more rounds of them for a wide n: a CU cannot have more than its 32 KiB of first-level cache
 // in flight (about 30 GB/s), so a matrix is only read at full speed if every CU has the same share of it --
 // with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it takes 4.2.
-// The eight waves of a workgroup deal k out among themselves, all loads of a wave are issued before its first
-// MFMA, and the partial sums meet in LDS.
+// The eight waves of a workgroup deal k out among themselves, and the partial sums meet in LDS.
 //
 // mfma_f32_16x16x32 takes 16 rows of 32 k; read that way every load instruction would touch half a
 // cache line of 16 rows.  With at most 8 lhs rows the operand rows are instead 8 rows of W at two
@@ -15,6 +14,12 @@
 // whole 128-byte lines of 8 rows, of the result the two diagonal blocks are wanted.  3584 x 3584, one
 // row: 6.2 us from HBM (non-temporal loads) against 6.8 with KS = 1; KS = 4 is no better.  For 9..16
 // rows KS = 1, and ordinary loads, because the second half of a line is asked for by the next instruction.
+//
+// Where a workgroup has at most 8 W rows (TW = 1; 2 with more) it is not the stream but one wave's chain that counts: all
+// loads of a wave go out before its first MFMA, as many units B as its share of k has, up to 12 (one lhs row, W from HBM, us,
+// four units at a time and a second, empty group of rows / this: 512 x 3584 4.13 / 3.68, 1024 x 5120 5.45 / 4.65, 256 x 1536
+// 2.97 / 2.82, 2048 x 11008, in several rounds of 8, 11.45 / 10.62).  With more rows the stream is what counts, and four units of
+// two groups are what a CU can have under way (3584 x 3584, two / four / six / eight 7.07 / 6.25 / 6.67 / 6.28).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -34,35 +39,35 @@ struct SkinnyParams {
 };
 
 // KS k-slices per MFMA: operand row (column) index i stands for W (lhs) row i % (16/KS) at slice
-// i / (16/KS).  B units of 32*KS k per wave and pass.
-template <typename T, int KS, int B>
+// i / (16/KS).  TW groups of 16/KS W rows; B units of 32*KS k per wave and pass.
+template <typename T, int KS, int TW, int B>
 __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(SkinnyParams p) {
   using E = Elem<T>;
   constexpr int NW = kSkinnyWaves, R = 16 / KS, UK = 32 * KS;
-  __shared__ __attribute__((aligned(16))) float red[NW * KS * 256];  // [wave][group of R rows][lane] of f32x4
+  __shared__ __attribute__((aligned(16))) float red[NW * TW * 256];  // [wave][group of R rows][lane] of f32x4
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int i = lane & 15, cg = lane >> 4, r = i % R;
   const int n0 = blockIdx.x * p.rows;
   const int rows = min(p.rows, p.n - n0);
   const int koff = 32 * (i / R) + 8 * cg;
-  const uint16_t *wp[KS];
+  const uint16_t *wp[TW];
 #pragma unroll
-  for (int t = 0; t < KS; ++t) wp[t] = p.w + (size_t)(n0 + min(t * R + r, rows - 1)) * p.k + koff;
+  for (int t = 0; t < TW; ++t) wp[t] = p.w + (size_t)(n0 + min(t * R + r, rows - 1)) * p.k + koff;
   const bool xv = r < p.m;
   const uint16_t *xp = p.x + (size_t)(xv ? r : 0) * p.k + koff;
-  f32x4_t acc[KS];
+  f32x4_t acc[TW];
 #pragma unroll
-  for (int t = 0; t < KS; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < TW; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   const int units = (p.k + UK - 1) / UK;
   const u32x4_t zero = {0u, 0u, 0u, 0u};
   for (int u0 = wave; u0 < units; u0 += NW * B) {
-    u32x4_t wf[B][KS], xf[B];
+    u32x4_t wf[B][TW], xf[B];
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const int kk = (u0 + b * NW) * UK;
       const bool in = kk + koff < p.k;  // k is a multiple of 16, a fragment 8 long
 #pragma unroll
-      for (int t = 0; t < KS; ++t) {
+      for (int t = 0; t < TW; ++t) {
         wf[b][t] = zero;
         if (in && t * R + r < rows) wf[b][t] = KS > 1 ? global_load_b128_nt(wp[t] + kk) : global_load_b128(wp[t] + kk);
       }
@@ -72,11 +77,11 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(Ski
 #pragma unroll
     for (int b = 0; b < B; ++b)
 #pragma unroll
-      for (int t = 0; t < KS; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
+      for (int t = 0; t < TW; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
   }
   f32x4_t *slots = reinterpret_cast<f32x4_t *>(red);
 #pragma unroll
-  for (int t = 0; t < KS; ++t) slots[(wave * KS + t) * 64 + lane] = acc[t];
+  for (int t = 0; t < TW; ++t) slots[(wave * TW + t) * 64 + lane] = acc[t];
   __syncthreads();
   // thread: feature n0 + f of lhs row `row`
   const int f = tid & 15, row = tid >> 4;
@@ -87,10 +92,18 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(Ski
     const int ar = s * R + f % R, col = s * R + row;
     const float *src = red + ((f / R) * 64 + (ar >> 2) * 16 + col) * 4 + (ar & 3);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) sum += src[w * KS * 256];
+    for (int w = 0; w < NW; ++w) sum += src[w * TW * 256];
   }
   if (p.bias) sum += p.bias[n0 + f];
   p.out[(size_t)row * p.n + n0 + f] = E::round(sum);
+}
+
+template <typename T> void (*kernel_of(const SkinnyParams &p))(SkinnyParams) {
+  if (p.m > 8) return matmul_skinny_kernel<T, 1, 1, 8>;
+  if (p.rows > 8) return matmul_skinny_kernel<T, 2, 2, 4>;
+  const int units = (p.k + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);  // of a wave
+  if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4>;
+  return units > 8 && units <= 12 ? matmul_skinny_kernel<T, 2, 1, 12> : matmul_skinny_kernel<T, 2, 1, 8>;
 }
 
 }  // namespace
@@ -108,9 +121,7 @@ hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, 
   const int cus = device_compute_units();
   const int rounds = (n + 16 * cus - 1) / (16 * cus);
   p.rows = (n + rounds * cus - 1) / (rounds * cus);
-  void (*kern)(SkinnyParams) =
-      m <= 8 ? (dt == kDtFloat16 ? matmul_skinny_kernel<_Float16, 2, 4> : matmul_skinny_kernel<__bf16, 2, 4>)
-             : (dt == kDtFloat16 ? matmul_skinny_kernel<_Float16, 1, 8> : matmul_skinny_kernel<__bf16, 1, 8>);
+  void (*kern)(SkinnyParams) = dt == kDtFloat16 ? kernel_of<_Float16>(p) : kernel_of<__bf16>(p);
   hipLaunchKernelGGL(kern, dim3((n + p.rows - 1) / p.rows), dim3(64 * kSkinnyWaves), 0, stream, p);
   return hipGetLastError();
 }
