@@ -119,6 +119,16 @@ template <int I, int N, typename F> __device__ __forceinline__ void static_for(F
   static_for_each<I>(f, std::make_integer_sequence<int, (N > I ? N - I : 0)>());
 }
 
+// Kernel arguments.  Scalars and vectors among the first 14 words are in a kernel's registers when it starts (Makefile); a
+// struct is fetched from memory, 0.2 us before the first load of a launch can go out (a token's projections, W from HBM, us,
+// struct / registers: 512 x 3584 3.69 / 3.51, 3584 x 3584 6.25 / 6.03; rope and attention of 256 tokens of 32 heads 10.23 / 9.80).
+// So what the first loads need goes there, in few vectors: each argument costs the host too (eleven scalars 0.2 us).
+typedef __attribute__((ext_vector_type(4))) uint64_t addresses_t;
+inline uint64_t address(const void *p) { return reinterpret_cast<uintptr_t>(p); }
+template <typename P> __device__ __forceinline__ P *at_address(uint64_t a) {
+  return (P *)reinterpret_cast<__attribute__((address_space(1))) P *>(a);
+}
+
 // acc + lo + hi of a packed pair of storage-type values.
 template <typename T> __device__ __forceinline__ float dot2_ones(uint32_t packed, float acc);
 template <> __device__ __forceinline__ float dot2_ones<__bf16>(uint32_t packed, float acc) {

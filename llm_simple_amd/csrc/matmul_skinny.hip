@@ -29,43 +29,39 @@ namespace {
 
 constexpr int kSkinnyWaves = 8;
 
-struct SkinnyParams {
-  const uint16_t *x;
-  const uint16_t *w;
-  const float *bias;
-  uint16_t *out;
-  int m, n, k;
-  int rows;  // W rows of a workgroup, at most 16
-};
-
 // KS k-slices per MFMA: operand row (column) index i stands for W (lhs) row i % (16/KS) at slice
-// i / (16/KS).  TW groups of 16/KS W rows; B units of 32*KS k per wave and pass.
+// i / (16/KS).  TW groups of 16/KS W rows; B units of 32*KS k per wave and pass.  rows: W rows of a workgroup, at most 16.
+// a: lhs, W, bias, out; size: m, n, k, rows.
 template <typename T, int KS, int TW, int B>
-__global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(SkinnyParams p) {
+__global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(addresses_t a, u32x4_t size) {
   using E = Elem<T>;
+  const uint16_t *x = at_address<const uint16_t>(a[0]), *w = at_address<const uint16_t>(a[1]);
+  const float *bias = at_address<const float>(a[2]);
+  uint16_t *out = at_address<uint16_t>(a[3]);
+  const int m = size[0], n = size[1], k = size[2], row_share = size[3];
   constexpr int NW = kSkinnyWaves, R = 16 / KS, UK = 32 * KS;
   __shared__ __attribute__((aligned(16))) float red[NW * TW * 256];  // [wave][group of R rows][lane] of f32x4
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int i = lane & 15, cg = lane >> 4, r = i % R;
-  const int n0 = blockIdx.x * p.rows;
-  const int rows = min(p.rows, p.n - n0);
+  const int n0 = blockIdx.x * row_share;
+  const int rows = min(row_share, n - n0);
   const int koff = 32 * (i / R) + 8 * cg;
   const uint16_t *wp[TW];
 #pragma unroll
-  for (int t = 0; t < TW; ++t) wp[t] = p.w + (size_t)(n0 + min(t * R + r, rows - 1)) * p.k + koff;
-  const bool xv = r < p.m;
-  const uint16_t *xp = p.x + (size_t)(xv ? r : 0) * p.k + koff;
+  for (int t = 0; t < TW; ++t) wp[t] = w + (size_t)(n0 + min(t * R + r, rows - 1)) * k + koff;
+  const bool xv = r < m;
+  const uint16_t *xp = x + (size_t)(xv ? r : 0) * k + koff;
   f32x4_t acc[TW];
 #pragma unroll
   for (int t = 0; t < TW; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int units = (p.k + UK - 1) / UK;
+  const int units = (k + UK - 1) / UK;
   const u32x4_t zero = {0u, 0u, 0u, 0u};
   for (int u0 = wave; u0 < units; u0 += NW * B) {
     u32x4_t wf[B][TW], xf[B];
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const int kk = (u0 + b * NW) * UK;
-      const bool in = kk + koff < p.k;  // k is a multiple of 16, a fragment 8 long
+      const bool in = kk + koff < k;  // k is a multiple of 16, a fragment 8 long
 #pragma unroll
       for (int t = 0; t < TW; ++t) {
         wf[b][t] = zero;
@@ -85,23 +81,24 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(Ski
   __syncthreads();
   // thread: feature n0 + f of lhs row `row`
   const int f = tid & 15, row = tid >> 4;
-  if (f >= rows || row >= p.m) return;
+  if (f >= rows || row >= m) return;
   float sum = 0.0f;
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
     const int ar = s * R + f % R, col = s * R + row;
     const float *src = red + ((f / R) * 64 + (ar >> 2) * 16 + col) * 4 + (ar & 3);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) sum += src[w * TW * 256];
+    for (int v = 0; v < NW; ++v) sum += src[v * TW * 256];
   }
-  if (p.bias) sum += p.bias[n0 + f];
-  p.out[(size_t)row * p.n + n0 + f] = E::round(sum);
+  if (bias) sum += bias[n0 + f];
+  out[(size_t)row * n + n0 + f] = E::round(sum);
 }
 
-template <typename T> void (*kernel_of(const SkinnyParams &p))(SkinnyParams) {
-  if (p.m > 8) return matmul_skinny_kernel<T, 1, 1, 8>;
-  if (p.rows > 8) return matmul_skinny_kernel<T, 2, 2, 4>;
-  const int units = (p.k + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);  // of a wave
+using SkinnyKernel = void (*)(addresses_t, u32x4_t);
+template <typename T> SkinnyKernel kernel_of(int m, int k, int rows) {
+  if (m > 8) return matmul_skinny_kernel<T, 1, 1, 8>;
+  if (rows > 8) return matmul_skinny_kernel<T, 2, 2, 4>;
+  const int units = (k + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);  // of a wave
   if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4>;
   return units > 8 && units <= 12 ? matmul_skinny_kernel<T, 2, 1, 12> : matmul_skinny_kernel<T, 2, 1, 8>;
 }
@@ -110,19 +107,13 @@ template <typename T> void (*kernel_of(const SkinnyParams &p))(SkinnyParams) {
 
 hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, const float *bias, int m, int n,
                                 int k, int dt, hipStream_t stream) {
-  SkinnyParams p;
-  p.x = static_cast<const uint16_t *>(lhs);
-  p.w = static_cast<const uint16_t *>(weight);
-  p.bias = bias;
-  p.out = static_cast<uint16_t *>(out);
-  p.m = m;
-  p.n = n;
-  p.k = k;
   const int cus = device_compute_units();
   const int rounds = (n + 16 * cus - 1) / (16 * cus);
-  p.rows = (n + rounds * cus - 1) / (rounds * cus);
-  void (*kern)(SkinnyParams) = dt == kDtFloat16 ? kernel_of<_Float16>(p) : kernel_of<__bf16>(p);
-  hipLaunchKernelGGL(kern, dim3((n + p.rows - 1) / p.rows), dim3(64 * kSkinnyWaves), 0, stream, p);
+  const int rows = (n + rounds * cus - 1) / (rounds * cus);
+  const SkinnyKernel kern = dt == kDtFloat16 ? kernel_of<_Float16>(m, k, rows) : kernel_of<__bf16>(m, k, rows);
+  hipLaunchKernelGGL(kern, dim3((n + rows - 1) / rows), dim3(64 * kSkinnyWaves), 0, stream,
+                     addresses_t{address(lhs), address(weight), address(bias), address(out)},
+                     u32x4_t{(uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)rows});
   return hipGetLastError();
 }
 

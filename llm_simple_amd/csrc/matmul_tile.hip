@@ -49,15 +49,7 @@ constexpr int kTileThreads = 256;
 constexpr int kLineK = 64;             // k of a 128-byte line of an operand row
 constexpr int kStageRow = 2 * kLineK;  // its bytes
 constexpr int kBiasBytes = 4 * 512;    // LDS: bias of each wave's features
-
-struct TileParams {
-  const char *x, *w;
-  const float *bias;
-  uint16_t *out;
-  int m, n, k;
-  int m_tiles, n_tiles;
-  FastDiv band, band_rows;  // tiles of a band, m tiles of a full band
-};
+constexpr int kBandRows = 4;           // m tiles of a band
 
 // LDS offset of logical 16-byte granule g of a staged row
 __device__ __forceinline__ int stage_off(int row, int g) { return row * kStageRow + ((g ^ ((row >> 1) & 7)) << 4); }
@@ -74,8 +66,12 @@ template <int OFF> __device__ __forceinline__ void line_load(uint32_t voff, cons
 }
 
 template <typename T, int MT, int NT, int KS, int STAGES>
-__global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams p) {
+__global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_t a_, u32x4_t size, u32x2_t divisors) {
   using E = Elem<T>;
+  const char *x = at_address<const char>(a_[0]), *w = at_address<const char>(a_[1]);
+  const float *bias = at_address<const float>(a_[2]);
+  uint16_t *out = at_address<uint16_t>(a_[3]);
+  const int m = size[0], n = size[1], k = size[2];
   constexpr int BM = 32 * MT, BN = 32 * NT;
   constexpr int kLineBytes = (BM + BN) * kStageRow, kStageBytes = KS * kLineBytes;
   constexpr int L = MT + NT;
@@ -85,28 +81,31 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
 
   // Workgroups are dealt round-robin to the 8 XCDs: each takes a run of tiles, and runs go through bands of up to four
   // m tiles, so that the tiles of an XCD share rows of both operands in its L2.
-  const int total = p.m_tiles * p.n_tiles, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
+  // (divisors and size[3]: factors and shifts of the divisions by the tiles of a band and by the m tiles of a full band)
+  const int m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN, gm = min(m_tiles, kBandRows);
+  const FastDiv by_band = {(uint32_t)(gm * n_tiles), divisors[0], size[3] & 0xffffu}, by_rows = {(uint32_t)gm, divisors[1], size[3] >> 16};
+  const int total = m_tiles * n_tiles, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
   const int t = xcd * each + min(xcd, rest) + (int)(blockIdx.x >> 3);
-  const int band = (int)fast_div(t, p.band), rem = t - band * (int)p.band.d, gm = (int)p.band_rows.d;
-  const int rows_here = min(gm, p.m_tiles - band * gm);
-  const int tn = rows_here == gm ? (int)fast_div(rem, p.band_rows) : rem / rows_here;
+  const int band = (int)fast_div(t, by_band), rem = t - band * gm * n_tiles;
+  const int rows_here = min(gm, m_tiles - band * gm);
+  const int tn = rows_here == gm ? (int)fast_div(rem, by_rows) : rem / rows_here;
   const int m0 = (band * gm + rem - tn * rows_here) * BM, n0 = tn * BN;
   const int wm = wave & 1, wn = wave >> 1;
   const int col0 = n0 + wn * (BN / 2);
 
   // Bias of the wave's features to LDS of its own (any fp32 address, so four bytes a lane)
   const uint32_t bias_at = STAGES * kStageBytes + wave * 512;
-  if (p.bias) {
+  if (bias) {
 #pragma unroll
     for (int h = 0; h < (16 * NT + 63) / 64; ++h) {
-      const float *src = p.bias + min(col0 + 64 * h + lane, p.n - 1);
+      const float *src = bias + min(col0 + 64 * h + lane, n - 1);
       asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(bias_at + 256 * h) : "m0");
     }
   }
 
   // Line loads of a wave: NT of 8 W rows each, then MT of 8 lhs rows, either run contiguous in LDS.  Staged W row
   // 32b + 16c + 4q + j of a half (c: block of a pair) holds feature 32b + 8q + 4c + j.  Rows past the end: the last one.
-  const uint32_t row_bytes = 2 * (uint32_t)p.k;
+  const uint32_t row_bytes = 2 * (uint32_t)k;
   uint32_t voff[L];
 #pragma unroll
   for (int s = 0; s < L; ++s) {
@@ -117,10 +116,10 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
       const int half = row >= BN / 2 ? BN / 2 : 0, in = row - half, blk = in >> 4;
       if (blk < (NT & ~1)) r = half + (in & ~31) + 8 * ((in >> 2) & 3) + 4 * (blk & 1) + (in & 3);
     }
-    r = min(r, is_w ? p.n - n0 - 1 : p.m - m0 - 1);
+    r = min(r, is_w ? n - n0 - 1 : m - m0 - 1);
     voff[s] = (uint32_t)r * row_bytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4) + 3072 - 1024 * (nth & 3);
   }
-  const char *wbase = p.w + n0 * (size_t)row_bytes - 3072, *xbase = p.x + m0 * (size_t)row_bytes - 3072;
+  const char *wbase = w + n0 * (size_t)row_bytes - 3072, *xbase = x + m0 * (size_t)row_bytes - 3072;
   const uint32_t wdst = __builtin_amdgcn_readfirstlane(wave * NT * 1024);
   const uint32_t xdst = __builtin_amdgcn_readfirstlane(BN * kStageRow + wave * MT * 1024);
   auto issue = [&](auto s_, const char *wk, const char *xk, uint32_t slot) {
@@ -131,7 +130,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
       asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0" : : "s"(slot + (is_w ? wdst : xdst)), "n"(nth * 1024) : "m0", "scc");
     line_load<1024 * (nth % 4)>(voff[s], is_w ? wk : xk);
   };
-  const int lines = p.k / kLineK, stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
+  const int lines = k / kLineK, stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
   uint32_t kpos = (unsigned)(xcd * lines / 8 + (t & 3)) % (unsigned)lines * kStageRow;
   auto advance = [&]() { kpos = kpos + kStageRow == row_bytes ? 0 : kpos + kStageRow; };
 #pragma unroll
@@ -214,7 +213,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
     const bool two = b + 1 < NT;
     const int c = 16 * b + (two ? 8 : 4) * cg, col = col0 + c;
     f32x4_t b0 = {0.f, 0.f, 0.f, 0.f}, b1 = b0;
-    if (p.bias) {
+    if (bias) {
       b0 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c);
       if (two) b1 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c + 16);
     }
@@ -222,27 +221,30 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(TileParams
     for (int a = 0; a < MT; ++a) {
       const int row = row0 + 16 * a + i;
       const f32x4_t u = acc[a][b] + b0;
-      uint16_t *o = p.out + (size_t)row * p.n + col;
+      uint16_t *o = out + (size_t)row * n + col;
       if (two) {
         const f32x4_t v = acc[a][b + 1 < NT ? b + 1 : b] + b1;
-        if (row < p.m && col < p.n)
+        if (row < m && col < n)
           *reinterpret_cast<u32x4_t *>(o) = u32x4_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3]), E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
-      } else if (row < p.m && col < p.n) {
+      } else if (row < m && col < n) {
         *reinterpret_cast<u32x2_t *>(o) = u32x2_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3])};
       }
     }
   }
 }
 
-template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile(TileParams &p, hipStream_t stream) {
-  p.m_tiles = (p.m + 32 * MT - 1) / (32 * MT);
-  p.n_tiles = (p.n + 32 * NT - 1) / (32 * NT);
-  const int gm = p.m_tiles < 4 ? p.m_tiles : 4;
-  p.band = make_fast_div((uint32_t)(gm * p.n_tiles));
-  p.band_rows = make_fast_div((uint32_t)gm);
+struct TileCall {
+  addresses_t a;  // lhs, W, bias, out
+  int m, n, k;
+};
+
+template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile(const TileCall &c, hipStream_t stream) {
+  const int m_tiles = (c.m + 32 * MT - 1) / (32 * MT), n_tiles = (c.n + 32 * NT - 1) / (32 * NT);
+  const int gm = m_tiles < kBandRows ? m_tiles : kBandRows;
+  const FastDiv band = make_fast_div((uint32_t)(gm * n_tiles)), band_rows = make_fast_div((uint32_t)gm);
   constexpr int lds_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow + kBiasBytes;
   static_assert(lds_bytes > 64 * 1024 && lds_bytes <= 160 * 1024, "");
-  void (*kern)(TileParams) = matmul_tile_kernel<T, MT, NT, KS, STAGES>;
+  const auto kern = matmul_tile_kernel<T, MT, NT, KS, STAGES>;
   static std::atomic<uint64_t> attr_done{0};  // more than 64 KiB of dynamic LDS is an opt-in per device and kernel
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -253,27 +255,28 @@ template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile
     if (e != hipSuccess) return e;
     attr_done.fetch_or(bit, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(p.m_tiles * p.n_tiles), dim3(kTileThreads), lds_bytes, stream, p);
+  hipLaunchKernelGGL(kern, dim3(m_tiles * n_tiles), dim3(kTileThreads), lds_bytes, stream, c.a,
+                     u32x4_t{(uint32_t)c.m, (uint32_t)c.n, (uint32_t)c.k, band.l | band_rows.l << 16}, u32x2_t{band.m, band_rows.m});
   return hipGetLastError();
 }
 
-template <typename T> hipError_t launch_kind(TileParams &p, int kind, hipStream_t stream) {
+template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStream_t stream) {
   switch (kind) {
-    case 0: return launch_tile<T, 1, 1, 4, 4>(p, stream);
-    case 1: return launch_tile<T, 2, 1, 4, 3>(p, stream);
-    case 2: return launch_tile<T, 2, 2, 1, 9>(p, stream);
-    case 3: return launch_tile<T, 3, 2, 1, 7>(p, stream);
-    case 4: return launch_tile<T, 4, 2, 1, 6>(p, stream);
-    case 5: return launch_tile<T, 3, 3, 1, 6>(p, stream);
-    case 6: return launch_tile<T, 3, 4, 1, 5>(p, stream);
-    case 7: return launch_tile<T, 4, 3, 1, 5>(p, stream);
-    case 8: return launch_tile<T, 4, 4, 1, 4>(p, stream);
-    case 9: return launch_tile<T, 4, 5, 1, 4>(p, stream);
-    case 10: return launch_tile<T, 4, 6, 1, 3>(p, stream);
-    case 11: return launch_tile<T, 5, 5, 1, 3>(p, stream);
-    case 12: return launch_tile<T, 4, 7, 1, 3>(p, stream);
-    case 13: return launch_tile<T, 5, 6, 1, 3>(p, stream);
-    default: return launch_tile<T, 4, 8, 1, 3>(p, stream);
+    case 0: return launch_tile<T, 1, 1, 4, 4>(c, stream);
+    case 1: return launch_tile<T, 2, 1, 4, 3>(c, stream);
+    case 2: return launch_tile<T, 2, 2, 1, 9>(c, stream);
+    case 3: return launch_tile<T, 3, 2, 1, 7>(c, stream);
+    case 4: return launch_tile<T, 4, 2, 1, 6>(c, stream);
+    case 5: return launch_tile<T, 3, 3, 1, 6>(c, stream);
+    case 6: return launch_tile<T, 3, 4, 1, 5>(c, stream);
+    case 7: return launch_tile<T, 4, 3, 1, 5>(c, stream);
+    case 8: return launch_tile<T, 4, 4, 1, 4>(c, stream);
+    case 9: return launch_tile<T, 4, 5, 1, 4>(c, stream);
+    case 10: return launch_tile<T, 4, 6, 1, 3>(c, stream);
+    case 11: return launch_tile<T, 5, 5, 1, 3>(c, stream);
+    case 12: return launch_tile<T, 4, 7, 1, 3>(c, stream);
+    case 13: return launch_tile<T, 5, 6, 1, 3>(c, stream);
+    default: return launch_tile<T, 4, 8, 1, 3>(c, stream);
   }
 }
 
@@ -306,16 +309,9 @@ bool matmul_tile_takes(int m, int n, int k) {
 
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias, int m, int n, int k,
                               int dt, hipStream_t stream) {
-  TileParams p;
-  p.x = static_cast<const char *>(lhs);
-  p.w = static_cast<const char *>(weight);
-  p.bias = bias;
-  p.out = static_cast<uint16_t *>(out);
-  p.m = m;
-  p.n = n;
-  p.k = k;
+  const TileCall c = {{address(lhs), address(weight), address(bias), address(out)}, m, n, k};
   const int kind = tile_kind(m, n, k);
-  return dt == kDtFloat16 ? launch_kind<_Float16>(p, kind, stream) : launch_kind<__bf16>(p, kind, stream);
+  return dt == kDtFloat16 ? launch_kind<_Float16>(c, kind, stream) : launch_kind<__bf16>(c, kind, stream);
 }
 
 }  // namespace llmhip

@@ -32,15 +32,9 @@
 
 namespace llmhip {
 
-struct RopeParams {
-  const char *in_q, *in_k, *in_v;
-  char *out_q, *out_k, *out_v;
-  const float *freq_cis;
-  int start_pos, cur_size;
-  int q_heads, k_heads, v_heads;  // head rows of a token: q, then k, then v (v_heads = 0 without V)
-  int k_out_row_offset;
-  FastDiv rows_per_token;
-  uint32_t total;  // threads with work: cur_size * rows per token * 8
+// Where the rows of the first token go: fetched from memory while the loads are under way.
+struct RopeOut {
+  char *q, *k, *v;
 };
 
 // The 8 pairs of one thread: a = elements of the first 16-byte chunk, b = of the second.  NEOX: pair i
@@ -82,25 +76,29 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t 
 }
 
 template <typename T, bool NEOX>
-__global__ __launch_bounds__(256) void rope_kv_append_kernel(RopeParams p) {
+__global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u32x4_t size, u32x2_t heads_, RopeOut to) {
+  // in_: q, k, v, the table; size: threads, factor and shift of the division by the rows of a token (bit 8: there is a V), start_pos
+  const uint32_t total = size[0], rows_mul = size[1], rows_shift = size[2];
+  const int start_pos = size[3], q_heads = heads_[0], k_heads = heads_[1];
   const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-  if (gid >= p.total) return;
-  const uint32_t j = gid & 7u, rowid = gid >> 3, s = fast_div(rowid, p.rows_per_token);
-  const int r = (int)(rowid - s * p.rows_per_token.d);
-  const bool is_q = r < p.q_heads, rotated = r < p.q_heads + p.k_heads;
-  const int heads = is_q ? p.q_heads : p.k_heads;  // V has as many as K
-  const int h = is_q ? r : rotated ? r - p.q_heads : r - p.q_heads - p.k_heads;
-  const char *in = is_q ? p.in_q : rotated ? p.in_k : p.in_v;
-  char *out = is_q ? p.out_q : rotated ? p.out_k : p.out_v;
+  if (gid >= total) return;
+  const FastDiv rows_per_token = {(uint32_t)(q_heads + k_heads + (rows_shift & 256u ? k_heads : 0)), rows_mul, rows_shift & 255u};
+  const uint32_t j = gid & 7u, rowid = gid >> 3, s = fast_div(rowid, rows_per_token);
+  const int r = (int)(rowid - s * rows_per_token.d);
+  const bool is_q = r < q_heads, rotated = r < q_heads + k_heads;
+  const int heads = is_q ? q_heads : k_heads;  // V has as many as K
+  const int h = is_q ? r : rotated ? r - q_heads : r - q_heads - k_heads;
+  const char *in = at_address<const char>(is_q ? in_[0] : rotated ? in_[1] : in_[2]);
   in += ((size_t)s * heads + h) * kRowBytes + j * 16;
-  out += ((size_t)(s + (is_q ? 0 : p.k_out_row_offset)) * heads + h) * kRowBytes + j * 16;
-  const float *tab = p.freq_cis + (size_t)(p.start_pos + s) * kHeadDim + (NEOX ? 16 : 8) * j;
+  const float *tab = at_address<const float>(in_[3]) + (size_t)(start_pos + s) * kHeadDim + (NEOX ? 16 : 8) * j;
   // All loads go out before anything is waited for, the table's included (a V row's are not used)
   u32x4_t a = global_load_b128(in), b = global_load_b128(in + 128);
   f32x4_t cs[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4_t *>(tab + (NEOX ? 4 * i : 64 * (i >> 1) + 4 * (i & 1)));
   __builtin_amdgcn_sched_barrier(0);
+  char *out = is_q ? to.q : rotated ? to.k : to.v;
+  out += ((size_t)s * heads + h) * kRowBytes + j * 16;
   if (rotated) rotate8<T, NEOX>(a, b, cs);
   // Past the L2: the attention launch that follows finds nothing to wait for, and every instruction writes whole lines
   // (interleaved pairs used to be 32 bytes of a lane, stored by halves: 1019 tokens of 32 heads then take 32.8 us this way).
@@ -115,31 +113,19 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
                                  const void *in_q, const void *in_k, const void *in_v,
                                  int start_pos, int cur_size, int q_heads, int k_heads,
                                  int k_out_row_offset, int is_neox, int dt, hipStream_t stream) {
-  RopeParams p;
-  p.in_q = static_cast<const char *>(in_q);
-  p.in_k = static_cast<const char *>(in_k);
-  p.in_v = static_cast<const char *>(in_v);
-  p.out_q = static_cast<char *>(out_q);
-  p.out_k = static_cast<char *>(out_k);
-  p.out_v = static_cast<char *>(out_v);
-  p.freq_cis = static_cast<const float *>(freq_cis);
-  p.start_pos = start_pos;
-  p.cur_size = cur_size;
-  p.q_heads = q_heads;
-  p.k_heads = k_heads;
-  p.v_heads = (in_v != nullptr) ? k_heads : 0;
-  p.k_out_row_offset = k_out_row_offset;
-  const long long rows = (long long)q_heads + k_heads + p.v_heads;
+  const long long rows = (long long)q_heads + k_heads + (in_v != nullptr ? k_heads : 0);
   const long long total = (long long)cur_size * rows * 8;
   if (total == 0) return hipSuccess;
   if (rows > 0x7FFFFFFFLL || total > 0x7FFFFFFFLL) return hipErrorInvalidValue;  // 32-bit thread index
-  p.rows_per_token = make_fast_div((uint32_t)rows);
-  p.total = (uint32_t)total;
+  const FastDiv div = make_fast_div((uint32_t)rows);
+  const size_t first = (size_t)k_out_row_offset * k_heads * kRowBytes;
+  const RopeOut to = {static_cast<char *>(out_q), static_cast<char *>(out_k) + first, static_cast<char *>(out_v) + first};
   const int grid = (int)((total + 255) / 256);
-  void (*kern)(RopeParams) =
-      (dt == kDtFloat16) ? (is_neox ? rope_kv_append_kernel<_Float16, true> : rope_kv_append_kernel<_Float16, false>)
-                         : (is_neox ? rope_kv_append_kernel<__bf16, true> : rope_kv_append_kernel<__bf16, false>);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, p);
+  const auto kern = (dt == kDtFloat16) ? (is_neox ? rope_kv_append_kernel<_Float16, true> : rope_kv_append_kernel<_Float16, false>)
+                                       : (is_neox ? rope_kv_append_kernel<__bf16, true> : rope_kv_append_kernel<__bf16, false>);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, addresses_t{address(in_q), address(in_k), address(in_v), address(freq_cis)},
+                     u32x4_t{(uint32_t)total, div.m, div.l | (in_v != nullptr ? 256u : 0u), (uint32_t)start_pos},
+                     u32x2_t{(uint32_t)q_heads, (uint32_t)k_heads}, to);
   return hipGetLastError();
 }
 
