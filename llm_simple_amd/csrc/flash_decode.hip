@@ -62,31 +62,46 @@ constexpr int kDecCols = 16;                      // query rows per kv head (MFM
 constexpr int kDecWaveLds = kDecWaveKeys * kRowBytes;  // 8 KiB of staging per wave, for K and for V
 constexpr int kDecLdsPad = 24 * 1024;             // with the 64 KiB of staging: more than half a CU's LDS
 
-struct DecodeParams {
-  const char *q;
-  const char *k;
-  const char *v;
+// What a launch is told.  What its first loads need is packed into the first 14 words of a kernel's arguments, which are in
+// registers when it starts (DecodeEarly); the rest comes as a struct, fetched while those loads are under way.  (Fused step, us,
+// all in the struct / this: 384 keys of 2 kv heads 5.94 / 5.52, 512 of 32 5.72 / 5.36, 4096 of 8 8.58 / 8.03, 32768 of 8 24.94 /
+// 24.36; 5 x 2999 keys of 8 14.1 / 13.9.)
+struct DecodeLate {
   char *out;
   float *ws_o;   // [batch][Hkv][splits][cols][128]
   float *ws_ml;  // [batch][Hkv][splits][cols][2]; fold: the last column's place is the flag of the split
-  int batch, m, n, offset;
-  int64_t kv_seq_stride;
-  int g, Hkv, H;
-  int rows;  // m * g
   int num_splits;
   int iters_each, iters_rest;  // blocks per split: iters_each, one more for the first iters_rest splits
   FastDiv g_div;
   float scale_log2e;
   int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
   uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial (see FoldMode)
-  // Fused decode step (FUSED kernels only): the token at row fused_pos = n - 1 is not in the cache yet.
-  // q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
-  // q and the new K row are rotated with table row freq_row (64 (cos, sin) pairs) as they are loaded,
-  // and the workgroup that owns the last key range writes the rotated K row and the V row to the cache.
-  const char *new_k;
-  const char *new_v;
-  const float *freq_row;
-  int fused_pos, is_neox;
+};
+// rows = m * g query rows of a kv head, at most 16.  Fused decode step (FUSED kernels only): the token at row n - 1 is not in the
+// cache yet.  q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
+// q and the new K row are rotated with table row freq_row (64 (cos, sin) pairs) as they are loaded,
+// and the workgroup that owns the last key range writes the rotated K row and the V row to the cache.
+struct DecodeParams : DecodeLate {
+  const void *q, *k, *v;
+  const void *freq_row, *new_k, *new_v;
+  int batch, m, n, offset;
+  int64_t kv_seq_stride;
+  int g, Hkv, rows;
+  int is_neox;
+  bool fused;
+};
+// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8, 2^16 / g + 1, offset; c: n, Hkv | g << 16 | is_neox << 31
+struct DecodeEarly {
+  addresses_t a;
+  u32x4_t b;
+  u32x2_t c;
+  explicit DecodeEarly(const DecodeParams &p) {
+    a = addresses_t{address(p.q), address(p.k), address(p.v), p.fused ? address(p.freq_row) : (uint64_t)p.kv_seq_stride};
+    const uint64_t nk = address(p.new_k), nv = address(p.new_v);
+    b = p.fused ? u32x4_t{(uint32_t)nk, (uint32_t)(nk >> 32), (uint32_t)nv, (uint32_t)(nv >> 32)}
+                : u32x4_t{(uint32_t)(p.rows | p.m << 8), 65536u / p.g + 1, (uint32_t)p.offset, 0u};
+    c = u32x2_t{(uint32_t)p.n, (uint32_t)p.Hkv | (uint32_t)p.g << 16 | (uint32_t)p.is_neox << 31};
+  }
 };
 
 // RoPE of the four 16-byte fragments a lane holds of one head row: fragment kk = dims 8*cg + 32*kk .. +7.
@@ -188,37 +203,46 @@ __device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int by
 enum FoldMode { kNoFold, kFoldByFlags, kFoldByTags };
 
 template <typename T, bool FUSED, int NW, bool LONG, FoldMode FOLD>
-__global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
+__global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec, DecodeLate p) {
   using E = Elem<T>;
+  const int n = ec[0], Hkv = ec[1] & 0xffffu, g = ec[1] >> 16 & 0xffu, H = g * Hkv;
+  const bool is_neox = ec[1] >> 31;
+  const int rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8, offset = FUSED ? n - 1 : (int)eb[2];
+  const int fused_pos = n - 1;
   constexpr int kStepKeys = NW * kDecWaveKeys;
   __shared__ __attribute__((aligned(16))) char lds[2 * NW * kDecWaveLds];
 
-  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int split = blockIdx.x, kvh = blockIdx.y, b = FUSED ? 0 : blockIdx.z;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, cg = lane >> 4;
 
-  const int iters = p.iters_each + (split < p.iters_rest);  // blocks split, split + S, ...
-  const int row_bytes = p.Hkv * kRowBytes;
-  const size_t seq_off = ((size_t)b * p.kv_seq_stride * p.Hkv + kvh) * kRowBytes;
-  const char *kbase = p.k + seq_off, *vbase = p.v + seq_off;
-  const int stored = FUSED ? p.n - 1 : p.n;  // rows that are in the cache
+  const int row_bytes = Hkv * kRowBytes;
+  const size_t seq_off = ((FUSED ? 0 : (size_t)b * ea[3] * Hkv) + kvh) * kRowBytes;
+  const char *kbase = at_address<const char>(ea[1]) + seq_off, *vbase = at_address<const char>(ea[2]) + seq_off;
+  const int stored = FUSED ? n - 1 : n;  // rows that are in the cache
 
   // query column of this lane
-  const bool col_valid = col < p.rows;
-  const int c_row = col_valid ? (int)fast_div(col, p.g_div) : 0;
-  const int c_head = kvh * p.g + (col_valid ? col - c_row * p.g : 0);
-  const int c_limit = c_row + p.offset;  // last visible key of this column
-  const bool new_col = FUSED && col == p.rows;  // this column carries the new K row through the rotation
+  const bool col_valid = col < rows;
+  const int c_row = FUSED || !col_valid ? 0 : (int)(col * eb[1] >> 16);  // (col / g)
+  const int c_head = kvh * g + (col_valid ? col - c_row * g : 0);
+  const int c_limit = c_row + offset;  // last visible key of this column
+  const bool new_col = FUSED && col == rows;  // this column carries the new K row through the rotation
+  const char *new_k_row = nullptr;
+  const float *freq_row = nullptr;
 
   u32x4_t qf[4];
   f32x4_t tab[8];
   u32x4_t new_v;
   {
-    const char *qp = p.q + (size_t)b * p.m * p.H * kRowBytes;
-    uint32_t qo = (c_row * p.H + c_head) * kRowBytes + cg * 16;
+    const char *qp = at_address<const char>(ea[0]) + (size_t)b * m * H * kRowBytes;
+    uint32_t qo = (c_row * H + c_head) * kRowBytes + cg * 16;
+    if (FUSED) {
+      new_k_row = at_address<const char>(eb[0] | (uint64_t)eb[1] << 32) + kvh * kRowBytes;
+      freq_row = at_address<const float>(ea[3]);
+    }
     if (new_col) {
-      qp = p.new_k;
-      qo = kvh * kRowBytes + cg * 16;
+      qp = new_k_row;
+      qo = cg * 16;
     }
     qp += qo;
 #pragma unroll
@@ -228,8 +252,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       for (int kk = 0; kk < 4; ++kk) qf[kk] = global_load_b128(qp + kk * 64);
     }
     if (FUSED) {
-      load_rotation(tab, p.freq_row, cg, p.is_neox);
-      new_v = global_load_b128(p.new_v + (size_t)kvh * kRowBytes + col * 16);
+      load_rotation(tab, freq_row, cg, is_neox);
+      new_v = global_load_b128(at_address<const char>(eb[2] | (uint64_t)eb[3] << 32) + kvh * kRowBytes + col * 16);
     }
   }
 
@@ -261,18 +285,18 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   // registers are free (5 x 2999 keys, 4 blocks each: 15.6 -> 14.9 us).
   issue_k(0);
   issue_v(0);
-
   f32x4_t o[8];
 #pragma unroll
   for (int d = 0; d < 8; ++d) o[d] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;
   char *vl = lds + wave * kDecWaveLds;
   char *kl = lds + (NW + wave) * kDecWaveLds;
-  if (FUSED) rotate_frags<T>(qf, tab, p.is_neox);
+  if (FUSED) rotate_frags<T>(qf, tab, is_neox);
 
+  const int iters = p.iters_each + (split < p.iters_rest);  // blocks split, split + S, ...
   for (int it = 0; it < iters; ++it) {
     const int kb0 = (it * p.num_splits + split) * kStepKeys + wave * kDecWaveKeys;
-    const int at = p.fused_pos - kb0;               // FUSED: where in the wave's keys the new row is
+    const int at = fused_pos - kb0;               // FUSED: where in the wave's keys the new row is
     const bool owner = FUSED && at >= 0 && at < kDecWaveKeys;
     u32x4_t kc[2][4];
     __builtin_amdgcn_wave_barrier();
@@ -282,15 +306,15 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       // the new token's K row takes its place among the staged rows and goes to the cache
       u32x4_t nk[4] = {qf[0], qf[1], qf[2], qf[3]};
       bool mine = new_col;
-      if (p.rows == kDecCols) {  // no spare column: one more rotation
+      if (rows == kDecCols) {  // no spare column: one more rotation
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) nk[kk] = global_load_b128(p.new_k + (size_t)kvh * kRowBytes + cg * 16 + kk * 64);
-        load_rotation(tab, p.freq_row, cg, p.is_neox);
-        rotate_frags<T>(nk, tab, p.is_neox);
+        for (int kk = 0; kk < 4; ++kk) nk[kk] = global_load_b128(new_k_row + cg * 16 + kk * 64);
+        load_rotation(tab, freq_row, cg, is_neox);
+        rotate_frags<T>(nk, tab, is_neox);
         mine = col == 0;
       }
       if (mine) {
-        char *dst = const_cast<char *>(kbase) + (size_t)p.fused_pos * row_bytes + cg * 16;
+        char *dst = const_cast<char *>(kbase) + (size_t)fused_pos * row_bytes + cg * 16;
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
           lds_write_b128(kl, at * kRowBytes + (((4 * kk + cg) ^ (at & 15)) << 4), nk[kk]);
@@ -307,7 +331,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       for (int kk = 0; kk < 4; ++kk)
         kc[blk][kk] = lds_read_b128(kl, (blk * 16 + col) * kRowBytes + (((4 * kk + cg) ^ col) << 4));
 
-    if (kb0 < p.n) {
+    if (kb0 < n) {
       // ---- S^T = K Q^T : 2 blocks of 16 keys ----
       f32x4_t s[2];
 #pragma unroll
@@ -321,13 +345,13 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
         issue_v(it);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (kb0 + kDecWaveKeys - 1 > min(p.offset, p.n - 1)) {
+      if (kb0 + kDecWaveKeys - 1 > min(offset, n - 1)) {
 #pragma unroll
         for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int key = kb0 + blk * 16 + 4 * cg + i;
-            if (key >= p.n || key > c_limit) s[blk][i] = -INFINITY;
+            if (key >= n || key > c_limit) s[blk][i] = -INFINITY;
           }
       }
       float mloc = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
@@ -367,7 +391,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
       for (int i = 0; i < 8; ++i) lds_write_b128(vl, v_swizzle32_off(4 * i + cg, col), vn[i]);
       if (owner && cg == (at & 3)) {  // the new token's V row, likewise
         lds_write_b128(vl, v_swizzle32_off(at, col), new_v);
-        *reinterpret_cast<u32x4_t *>(const_cast<char *>(vbase) + (size_t)p.fused_pos * row_bytes + col * 16) = new_v;
+        *reinterpret_cast<u32x4_t *>(const_cast<char *>(vbase) + (size_t)fused_pos * row_bytes + col * 16) = new_v;
       }
       __builtin_amdgcn_wave_barrier();
       if (it + 1 < iters && !LONG) issue_k(it + 1);
@@ -406,17 +430,17 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   }
   __syncthreads();
 
-  const size_t pair = (size_t)b * p.Hkv + kvh;
+  const size_t pair = (size_t)b * Hkv + kvh;
   const int pair_slots = p.num_splits * p.cols;
   const __amdgpu_buffer_rsrc_t po = byte_buffer(p.ws_o + pair * pair_slots * kHeadDim, pair_slots * kHeadDim * 4);
   const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
-  const int tagged_bytes = p.num_splits * p.rows * kTaggedBytes;
+  const int tagged_bytes = p.num_splits * rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + pair * tagged_bytes, tagged_bytes);
   const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
   auto tagged = [&](float x, float y) {
     return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), tag0, __builtin_bit_cast(uint32_t, y), tag1});
   };
-  for (int c = tid >> 4; c < p.rows; c += 4 * NW) {
+  for (int c = tid >> 4; c < rows; c += 4 * NW) {
     const int dch = tid & 15;  // 8-wide d chunk of column c
     float mw[NW], M = -INFINITY;
 #pragma unroll
@@ -443,8 +467,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
     }
     if (FOLD == kNoFold && p.num_splits == 1) {
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-      const int r = (int)fast_div(c, p.g_div), hq = c - r * p.g;
-      char *op = p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + hq) * kRowBytes + dch * 16;
+      const int r = (int)fast_div(c, p.g_div), hq = c - r * g;
+      char *op = p.out + (((size_t)b * m + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
       u32x4_t w;
 #pragma unroll
       for (int j = 0; j < 4; ++j) w[j] = E::pack2(acc[2 * j] * inv, acc[2 * j + 1] * inv);
@@ -455,7 +479,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
     const f32x4_t a0 = {acc[0], acc[1], acc[2], acc[3]}, a1 = {acc[4], acc[5], acc[6], acc[7]};
     const u32x2_t ml = {__builtin_bit_cast(uint32_t, M), __builtin_bit_cast(uint32_t, L)};
     if constexpr (FOLD == kFoldByTags) {
-      const int at = (split * p.rows + c) * kTaggedBytes;
+      const int at = (split * rows + c) * kTaggedBytes;
 #pragma unroll
       for (int j = 0; j < 4; ++j) store_device(pt, at + j * 256 + dch * 16, tagged(acc[2 * j], acc[2 * j + 1]));
       if (dch == 0) store_device(pt, at + kHeadDim * 8, tagged(M, L));
@@ -476,13 +500,13 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
   // than 8 (fewer: one group takes them all at once; by flags, 512 keys of 32 kv heads 6.65 -> 6.2 us, 1500 of 32 9.9 -> 8.9).
   constexpr int NG = 2 * NW;
   const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
-  const int at_once = min(p.rows, NG), parts = S <= kFoldDepth ? 1 : NG / at_once, part = sg / at_once;
+  const int at_once = min(rows, NG), parts = S <= kFoldDepth ? 1 : NG / at_once, part = sg / at_once;
   float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = reinterpret_cast<float *>(lds) + 64;  // per group
   // Folds the partials ml, ov of splits part, part + parts, ... of row c and stores the row, if all of them are `there` (up
   // to 8 splits: they need not be).
   auto fold = [&](int c, const auto &ml, const auto &ov, bool there) {
     constexpr int D = sizeof(ml) / sizeof(ml[0]);
-    const bool mine = part < parts && c < p.rows;
+    const bool mine = part < parts && c < rows;
     float M = -INFINITY, L = 0.0f;
     f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
     if (mine) {
@@ -518,13 +542,13 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
         }
       }
     }
-    if (part == 0 && c < p.rows && there) {
+    if (part == 0 && c < rows && there) {
       const int r = (int)fast_div(c, p.g_div);
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
       u32x2_t w;
       w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
       w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
-      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + c - r * p.g) * kRowBytes + d4 * 8) = w;
+      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * m + r) * H + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
     }
   };
 
@@ -545,7 +569,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
 #pragma unroll
       for (int j = 0; j < D; ++j) {
         const int c = r * at_once + sg;
-        const int at = sg < at_once && c < p.rows && j < S ? (j * p.rows + c) * kTaggedBytes : 0x40000000;
+        const int at = sg < at_once && c < rows && j < S ? (j * rows + c) * kTaggedBytes : 0x40000000;
         a[r][j][0] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece));
         a[r][j][1] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece + 256));
         ml4[r][j] = __builtin_bit_cast(u32x4_t, load_device(pt, at + kHeadDim * 8));
@@ -597,13 +621,13 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
     f32x4_t ov[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      const int slot = min(part + parts * j, S - 1) * p.cols + min(c, p.rows - 1);
+      const int slot = min(part + parts * j, S - 1) * p.cols + min(c, rows - 1);
       ml[j] = load_device2(pml, slot * 8);
       ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
     }
     fold(c, ml, ov, true);
   };
-  for (int c0 = 0; c0 < p.rows; c0 += at_once) {
+  for (int c0 = 0; c0 < rows; c0 += at_once) {
     if (S <= kFoldDepth * parts)
       take(c0 + sg % at_once, std::integral_constant<int, kFoldDepth>());
     else
@@ -618,17 +642,21 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(DecodeParams p) {
 constexpr int kMaxSplits = 256;
 
 template <typename T>
-__global__ __launch_bounds__(256) void flash_decode_combine_kernel(DecodeParams p) {
+__global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a, u32x4_t size, u32x2_t heads) {
+  // a: partials, their maxima and sums, out; size: splits, columns of a slot, Hkv, m; heads: g, 2^16 / g + 1
   using E = Elem<T>;
+  const float *ws_o = at_address<const float>(a[0]), *ws_ml = at_address<const float>(a[1]);
+  char *out = at_address<char>(a[2]);
+  const int cols = size[1], Hkv = size[2], m = size[3], g = heads[0], H = g * Hkv;
   __shared__ float red_m[8], red_l[8];
   __shared__ f32x4_t red_o[8][32];
   const int c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
   const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
-  const int S = p.num_splits;
-  const size_t base = ((size_t)b * p.Hkv + kvh) * S;
-  const float *ml = p.ws_ml + (base * p.cols + c) * 2;
-  const float *src = p.ws_o + (base * p.cols + c) * kHeadDim + 4 * d4;
-  const size_t ml_stride = (size_t)p.cols * 2, o_stride = (size_t)p.cols * kHeadDim;
+  const int S = size[0];
+  const size_t base = ((size_t)b * Hkv + kvh) * S;
+  const float *ml = ws_ml + (base * cols + c) * 2;
+  const float *src = ws_o + (base * cols + c) * kHeadDim + 4 * d4;
+  const size_t ml_stride = (size_t)cols * 2, o_stride = (size_t)cols * kHeadDim;
   float M = -INFINITY, L = 0.0f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = sg; s0 < S; s0 += 32) {  // rounds of up to 4 splits per thread
@@ -681,11 +709,11 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(DecodeParams 
     for (int i = 0; i < 4; ++i) tot[i] += wt * o[i];
   }
   const float inv = (Lt > 0.0f) ? 1.0f / Lt : 0.0f;
-  const int r = (int)fast_div(c, p.g_div), hq = c - r * p.g;
+  const int r = (int)(c * heads[1] >> 16), hq = c - r * g;  // (c / g, c below 16)
   u32x2_t w;
   w[0] = E::pack2(tot[0] * inv, tot[1] * inv);
   w[1] = E::pack2(tot[2] * inv, tot[3] * inv);
-  *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * p.m + r) * p.H + kvh * p.g + hq) * kRowBytes + d4 * 8) = w;
+  *reinterpret_cast<u32x2_t *>(out + (((size_t)b * m + r) * H + kvh * g + hq) * kRowBytes + d4 * 8) = w;
 }
 
 // Largest split count the default rule considers for batch * kv heads = pairs (any KV length): one
@@ -834,7 +862,7 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   // them would put 64 KiB of loads in flight again).  More than 64 KiB of LDS in total is an opt-in
   // per device and kernel.
   constexpr int pad = NW == 4 ? kDecLdsPad : 0;
-  void (*kern)(DecodeParams) = flash_decode_kernel<T, FUSED, NW, LONG, FOLD>;
+  const auto kern = flash_decode_kernel<T, FUSED, NW, LONG, FOLD>;
   if (pad) {
     static std::atomic<uint64_t> attr_done{0};
     int dev = 0;
@@ -847,10 +875,15 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
       attr_done.fetch_or(bit, std::memory_order_release);
     }
   }
-  hipLaunchKernelGGL(kern, dim3(p.num_splits, p.Hkv, p.batch), dim3(64 * NW), pad, stream, p);
+  const DecodeEarly early(p);
+  hipLaunchKernelGGL(kern, dim3(p.num_splits, p.Hkv, p.batch), dim3(64 * NW), pad, stream, early.a, early.b, early.c,
+                     static_cast<const DecodeLate &>(p));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
-  hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream,
+                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), 0},
+                     u32x4_t{(uint32_t)p.num_splits, (uint32_t)p.cols, (uint32_t)p.Hkv, (uint32_t)p.m},
+                     u32x2_t{(uint32_t)p.g, 65536u / p.g + 1});
   return hipGetLastError();
 }
 
@@ -918,9 +951,9 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
                                int64_t kv_seq_stride, int group_size, int kv_head_num,
                                int num_splits, int dt, hipStream_t stream) {
   DecodeParams p = {};
-  p.q = static_cast<const char *>(q);
-  p.k = static_cast<const char *>(k);
-  p.v = static_cast<const char *>(v);
+  p.q = q;
+  p.k = k;
+  p.v = v;
   p.out = static_cast<char *>(out);
   p.batch = batch;
   p.m = m;
@@ -929,7 +962,6 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
   p.kv_seq_stride = kv_seq_stride;
   p.g = group_size;
   p.Hkv = kv_head_num;
-  p.H = group_size * kv_head_num;
   p.rows = m * group_size;
   return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, false, stream);
 }
@@ -941,9 +973,9 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
                                     size_t workspace_bytes, int pos, int group_size, int kv_head_num, int is_neox, int num_splits,
                                     int dt, hipStream_t stream) {
   DecodeParams p = {};
-  p.q = static_cast<const char *>(in_q);
-  p.k = static_cast<const char *>(k_cache);
-  p.v = static_cast<const char *>(v_cache);
+  p.q = in_q;
+  p.k = k_cache;
+  p.v = v_cache;
   p.out = static_cast<char *>(out);
   p.batch = 1;
   p.m = 1;
@@ -952,12 +984,11 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
   p.kv_seq_stride = pos + 1;
   p.g = group_size;
   p.Hkv = kv_head_num;
-  p.H = group_size * kv_head_num;
   p.rows = group_size;
-  p.new_k = static_cast<const char *>(in_k);
-  p.new_v = static_cast<const char *>(in_v);
+  p.new_k = in_k;
+  p.new_v = in_v;
   p.freq_row = static_cast<const float *>(freq_cis) + (size_t)pos * kHeadDim;
-  p.fused_pos = pos;
+  p.fused = true;
   p.is_neox = is_neox ? 1 : 0;
   return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, true, stream);
 }
