@@ -19,13 +19,13 @@
 // moves lazily, so O is rarely rescaled.  Accumulation is fp32; out =
 // O / l rounded once; l sums the ROUNDED probabilities (what P.V used).
 //
-// flash_prefill_kernel<T, NW, KP, NT>: NW waves share the K/V tiles of 32*NW/KP query rows, KP of them every
+// flash_prefill_kernel<T, NW, KP, NT, SPLIT>: NW waves share the K/V tiles of 32*NW/KP query rows, KP of them every
 // row block, each on its own 32 keys of every tile (KP = 1: on all 64).  While the chip is not full a launch
 // waits for the serial chain of the waves with the most keys -- a step of a wave takes 1600-1900 cycles
 // where its MFMAs take 512, and nothing else runs on its SIMD -- so that short prompts and chunks want many waves per
 // row (KP = 4: 512 tokens, 28 heads 11.5 -> 9.2 us; 256 tokens, 32 heads 8.7 -> 6.7), long ones the
 // cheapest step (KP = 1, 256 rows).  NT: the tile loads are non-temporal (chunks whose K/V tiles only one
-// workgroup reads).
+// workgroup reads).  SPLIT: the key range is cut, rows may be packed.
 // Outside the loop a workgroup costs a short launch 2-3 us: indexes come from divisions prepared by the host, Q
 // of shared rows is fetched once through LDS, and waves that shared rows trade pieces of O^T so that each
 // folds and stores its part (epilogue of a pair 3900 -> 2200 cycles).
@@ -64,34 +64,65 @@ constexpr float kLazyLog2 = 8.0f;                // rescale threshold, log2 unit
 constexpr int kMaxPrefillSplits = 128;           // key ranges per call
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
-struct PrefillParams {
-  const char *q;
-  const char *k;
-  const char *v;
+// What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way.
+struct PrefillLate {
   char *out;
-  int m, n, offset;
-  int H, Hkv, g;
-  int num_q_tiles;
-  int sched_mode;  // 0: plain, 1: several XCDs per kv head, 2: several kv heads per XCD
-  int sched_a, sched_shift;  // mode 1: XCDs per kv head and its logarithm
-  int second, second_end;    // places of a list (of the XCD, mode 0: of the launch) that are taken in reverse
-  FastDiv per_split, list_heads;  // of an XCD's work list: items per key range, heads
-  FastDiv g_div;
-  float scale_log2e;
   // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers
   // keys [s*chunk, (s+1)*chunk); with more than one split every workgroup leaves an fp32 partial
   // (reference maximum, sum, unnormalised O) that prefill_combine_kernel folds.
-  int num_splits, chunk;  // chunk: multiple of 64 keys
-  // Split mode only: the rows of a tile are (token, head-in-group) pairs of ONE kv head, packed
-  // token-major (row index = token * g + head % g), so a chunk shorter than a tile reads K and V of
-  // its kv head once for all g query heads.
-  int pack;
   float *ws_o;            // [split][m][H][128]
   float *ws_ml;           // [split][m][H][2]
+  int num_splits, chunk;  // chunk: multiple of 64 keys
+  FastDiv per_split;      // of an XCD's work list: items per key range
+  float scale_log2e;
 #ifdef LLMHIP_BENCH
   // measurement library only: workgroup 0 stores {shader-clock ticks, 100 MHz ticks} of its lifetime
   unsigned long long *clock_probe;
 #endif
+};
+struct PrefillParams : PrefillLate {
+  const void *q, *k, *v;
+  int m, n, offset;
+  int H, Hkv, g;
+  int sched_mode;  // 0: plain, 1: several XCDs per kv head, 2: several kv heads per XCD
+  int sched_shift;           // mode 1: logarithm of the XCDs per kv head
+  int second, second_end;    // places of a list (of the XCD, mode 0: of the launch) that are taken in reverse
+  FastDiv list_heads;        // heads of an XCD's work list
+  FastDiv g_div;
+  // Split mode only: the rows of a tile are (token, head-in-group) pairs of ONE kv head, packed
+  // token-major (row index = token * g + head % g), so a chunk shorter than a tile reads K and V of
+  // its kv head once for all g query heads.
+  int pack;
+};
+// What the index arithmetic and the first loads of a workgroup need, packed into the first 14 words of a kernel's arguments, which
+// are in registers when it starts.  With kernels of their own for key ranges, whose packed rows and partials a prompt need not step
+// over (both together, attention alone, us: 32 tokens of 32 heads 4.65 -> 4.21, 256 5.85 -> 5.50, 512 of 28 8.44 -> 7.94, 1019 14.4 ->
+// 14.05, 2048 35.6 -> 34.8, 4096 113.5 -> 112.8; 200 past 16001 53.1 -> 51.75, 100 past 8000 of 40 25.2 -> 24.1).
+struct PrefillEarly {
+  addresses_t a;  // q, K, V, m | n << 32
+  u32x4_t b;      // offset, Hkv | g << 16, flags, second | second_end << 16
+  u32x2_t c;      // factors of the divisions by g and by the heads of a list
+  // flags: sched_mode, sched_shift << 2, pack << 5, shifts of the divisions << 8 and << 16
+  explicit PrefillEarly(const PrefillParams &p) {
+    a = addresses_t{address(p.q), address(p.k), address(p.v), (uint32_t)p.m | (uint64_t)p.n << 32};
+    b = u32x4_t{(uint32_t)p.offset, (uint32_t)p.Hkv | (uint32_t)p.g << 16,
+                (uint32_t)(p.sched_mode | p.sched_shift << 2 | p.pack << 5) | p.g_div.l << 8 | p.list_heads.l << 16,
+                (uint32_t)p.second | (uint32_t)p.second_end << 16};
+    c = u32x2_t{p.g_div.m, p.list_heads.m};
+  }
+};
+struct PrefillShared {  // the same, unpacked
+  const char *q, *k, *v;
+  int m, n, offset, H, Hkv, g, sched_mode, sched_shift, second, second_end;
+  bool pack;
+  FastDiv g_div, list_heads;
+  __device__ __forceinline__ PrefillShared(addresses_t a, u32x4_t b, u32x2_t c)
+      : q(at_address<const char>(a[0])), k(at_address<const char>(a[1])), v(at_address<const char>(a[2])), m((uint32_t)a[3]),
+        n((uint32_t)(a[3] >> 32)), offset(b[0]), H((b[1] & 0xffffu) * (b[1] >> 16)), Hkv(b[1] & 0xffffu), g(b[1] >> 16),
+        sched_mode(b[2] & 3u), sched_shift(b[2] >> 2 & 7u), second(b[3] & 0xffffu), second_end(b[3] >> 16), pack(b[2] & 32u),
+        g_div{b[1] >> 16, c[0], b[2] >> 8 & 63u} {
+    list_heads = FastDiv{(uint32_t)(sched_mode == 1 ? g : sched_mode == 2 ? (Hkv >> 3) * g : pack ? Hkv : H), c[1], b[2] >> 16 & 63u};
+  }
 };
 
 // blockIdx -> (query tile, head, key range).  Workgroup ids are dealt round-robin to the 8
@@ -99,31 +130,35 @@ struct PrefillParams {
 // so that its K/V stay in that XCD's L2, and within an XCD the heaviest (last)
 // query tiles are issued first.  Key ranges (split mode) are the slowest index of an XCD's
 // list, so that every XCD gets the same number of workgroups whatever the head count.
-__device__ __forceinline__ bool prefill_schedule(const PrefillParams &p, int bid, int &tile,
+template <bool SPLIT>
+__device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const PrefillLate &p, int bid, int num_q_tiles, int &tile,
                                                  int &head, int &split) {
   int idx = bid, xcd = 0;
-  if (p.sched_mode != 0) {
+  if (e.sched_mode != 0) {
     xcd = bid & 7;
     idx = bid >> 3;
   }
-  if (idx >= p.second && idx < p.second_end) idx = p.second + p.second_end - 1 - idx;
-  if (p.sched_mode != 0) {
-    if (p.sched_mode == 1) {  // sched_a = 2^sched_shift XCDs per kv head
-      idx = (idx << p.sched_shift) + (xcd & (p.sched_a - 1));
-      xcd >>= p.sched_shift;  // the kv head
-    }
+  if (idx >= e.second && idx < e.second_end) idx = e.second + e.second_end - 1 - idx;
+  if (e.sched_mode == 1) {  // 2^sched_shift XCDs per kv head
+    idx = (idx << e.sched_shift) + (xcd & ((1 << e.sched_shift) - 1));
+    xcd >>= e.sched_shift;  // the kv head
   }
   // idx: (key range, tile from the last, head among the list's `list_heads`)
-  if (idx >= (int)p.per_split.d * p.num_splits) return false;
-  split = (int)fast_div(idx, p.per_split);
-  const int rem = idx - split * (int)p.per_split.d;
-  const int t = (int)fast_div(rem, p.list_heads);
-  const int h = rem - t * (int)p.list_heads.d;
-  tile = p.num_q_tiles - 1 - t;
-  if (p.pack)
-    head = h * p.g;  // the list holds kv heads: first query head of the kv head
+  int rem = idx;
+  split = 0;
+  if (SPLIT) {
+    if (idx >= (int)p.per_split.d * p.num_splits) return false;
+    split = (int)fast_div(idx, p.per_split);
+    rem = idx - split * (int)p.per_split.d;
+  }
+  const int t = (int)fast_div(rem, e.list_heads);
+  if (t >= num_q_tiles) return false;
+  const int h = rem - t * (int)e.list_heads.d;
+  tile = num_q_tiles - 1 - t;
+  if (SPLIT && e.pack)
+    head = h * e.g;  // the list holds kv heads: first query head of the kv head
   else
-    head = xcd * (int)p.list_heads.d + h;
+    head = xcd * (int)e.list_heads.d + h;
   return true;
 }
 
@@ -561,8 +596,8 @@ template <int NW, int TN, bool NT> struct DirectLoader {
 // KP = 2: two waves per row block, each on one 32-key half of every 64-key tile; KP = 4: four waves, tiles of
 // 128 keys; what they have is merged through LDS at the end.
 // ---------------------------------------------------------------------------
-template <typename T, int NW, int KP, bool NT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(PrefillParams p) {
+template <typename T, int NW, int KP, bool NT, bool SPLIT>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec, PrefillLate p) {
   // SUB tiles of 64 keys per stage and per barrier: with one workgroup per CU (NW = 8) a stage
   // holds 128 keys, which halves the number of times the waves are forced in step.
   // LDS: K tiles of both stages [2*SUB][16 KiB], then the V tiles likewise; tile t sits in
@@ -574,8 +609,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   constexpr int kWaveKeys = 32 * KB;  // keys of a tile per wave
   constexpr int kSplitKK = 3;  // k-steps of S(j+1) issued beside the row-maximum chain
   extern __shared__ __attribute__((aligned(16))) char lds[];
+  const PrefillShared e(ea, eb, ec);
+  const bool pack = SPLIT && e.pack;  // (packed rows exist in split mode only)
+  const int rows = pack ? e.m * e.g : e.m;
   int tile, head, split;
-  if (!prefill_schedule(p, blockIdx.x, tile, head, split)) return;
+  if (!prefill_schedule<SPLIT>(e, p, blockIdx.x, (rows + BM - 1) / BM, tile, head, split)) return;
 #ifdef LLMHIP_BENCH
   unsigned long long clk0 = 0, ref0 = 0;
   if (p.clock_probe) {
@@ -585,11 +623,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
 #endif
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int kvh = (int)fast_div(head, p.g_div);
+  const int kvh = (int)fast_div(head, e.g_div);
   // Rows of the tile.  Unpacked: rows are tokens of one head.  Packed: row index i stands for token
   // i / g of head kvh*g + i % g; `rows` counts them.  Everything below works on tokens: qtok is this
   // lane's token, tok_lo / tok_hi the first / last token of the wave's 32 rows.
-  const int rows = p.pack ? p.m * p.g : p.m;
   const int row0 = tile * BM;
   const int rows_end = min(rows, row0 + BM);
   const int rb = wave % RB, kpar = wave / RB;  // row block; which 32 keys of every tile (KP > 1)
@@ -600,35 +637,35 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   const bool row_valid = qblk0 + l32_ < rows;
   int qtok = qidx, qhead = head, tok_lo = qblk0, tok_hi = min(qblk0 + 31, rows - 1);
   int tile_tok_end = rows_end;  // one past the tile's last token
-  if (p.pack) {
-    qtok = (int)fast_div(qidx, p.g_div);
-    qhead = head + qidx - qtok * p.g;
-    tok_lo = (int)fast_div(qblk0, p.g_div);
-    tok_hi = (int)fast_div(tok_hi, p.g_div);
-    tile_tok_end = (int)fast_div(rows_end - 1, p.g_div) + 1;
+  if (pack) {
+    qtok = (int)fast_div(qidx, e.g_div);
+    qhead = head + qidx - qtok * e.g;
+    tok_lo = (int)fast_div(qblk0, e.g_div);
+    tok_hi = (int)fast_div(tok_hi, e.g_div);
+    tile_tok_end = (int)fast_div(rows_end - 1, e.g_div) + 1;
   }
   // This workgroup's key range, seen as a cache of its own: rows [k_lo, k_lo + n_) with the causal
   // offset shifted accordingly (negative when the range starts past a row's last visible key).
-  const int k_lo = split * p.chunk;
-  const int n_ = min(p.n - k_lo, p.chunk);
-  const int offset_ = p.offset - k_lo;
+  const int k_lo = SPLIT ? split * p.chunk : 0;
+  const int n_ = SPLIT ? min(e.n - k_lo, p.chunk) : e.n;
+  const int offset_ = e.offset - k_lo;
   const int n_vis = min(n_, tile_tok_end + offset_);  // keys any row of this tile can see
   const int J = (n_vis + TN - 1) / TN;        // tiles of the workgroup
-  const size_t q_row_bytes = (size_t)p.H * kRowBytes;
-  const int kv_row_bytes = p.Hkv * kRowBytes;
-  const char *kbase = p.k + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
-  const char *vbase = p.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
+  const size_t q_row_bytes = (size_t)e.H * kRowBytes;
+  const int kv_row_bytes = e.Hkv * kRowBytes;
+  const char *kbase = e.k + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
+  const char *vbase = e.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
 
   WaveAttn<T, KB> w;
-  w.init(lds, lane, kVRegion, (KP > 1) ? kpar : 0);
   // tiles in which this wave's keys hold at least one visible key
   const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) / TN)) : 0;
   float *part_o = nullptr, *part_ml = nullptr;
-  if (p.num_splits > 1) {
-    const size_t slot = ((size_t)split * p.m + qtok) * p.H + qhead;
+  if (SPLIT) {
+    const size_t slot = ((size_t)split * e.m + qtok) * e.H + qhead;
     part_o = p.ws_o + slot * kHeadDim;
     part_ml = p.ws_ml + slot * 2;
     if (J <= 0) {  // workgroup-uniform: no row of this tile sees a key of this range
+      w.init(lds, lane, kVRegion);
       store_partial(w, part_o, part_ml, row_valid);
       return;
     }
@@ -642,10 +679,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   for (int sl = 0; sl < 8 / KP; ++sl) {
     const int r = 4 * (sl * NW + wave) + (lane >> 4);
     const int idx = min(row0 + r, rows - 1);
-    const char *src = p.q + ((lane & 15) ^ (r & 15)) * 16;
-    if (p.pack) {
-      const int tok = (int)fast_div(idx, p.g_div);
-      src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * p.g) * kRowBytes;
+    const char *src = e.q + ((lane & 15) ^ (r & 15)) * 16;
+    if (pack) {
+      const int tok = (int)fast_div(idx, e.g_div);
+      src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * e.g) * kRowBytes;
     } else {
       src += (size_t)idx * q_row_bytes + (size_t)head * kRowBytes;
     }
@@ -667,6 +704,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       ld.next(vst, J);
     }
   });
+  // The late arguments are asked for now, while the loads are under way, not at the place of each one's use
+  asm volatile("" : : "s"(p.out), "s"(p.scale_log2e));
+  if (SPLIT) asm volatile("" : : "s"(p.ws_o), "s"(p.ws_ml));
+  w.init(lds, lane, kVRegion, (KP > 1) ? kpar : 0);
   ld.template wait_but<2 * SUB * PER>();  // Q and K tile 0
   lds_barrier();
   w.load_q_lds(lds, kQRegion + (rb - (KP > 1 ? kpar : 0)) * 32 * kRowBytes);
@@ -747,12 +788,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   char *out_blk = p.out + (size_t)qblk0 * q_row_bytes + (size_t)head * kRowBytes;
   auto part_row = [&](int r) {  // where the partial of row r of the wave's goes
     int tok = qblk0 + r, h = head;
-    if (p.pack) {
+    if (pack) {
       const int idx = tok;
-      tok = (int)fast_div(idx, p.g_div);
-      h = head + idx - tok * p.g;
+      tok = (int)fast_div(idx, e.g_div);
+      h = head + idx - tok * e.g;
     }
-    return p.ws_o + (((size_t)split * p.m + tok) * p.H + h) * kHeadDim;
+    return p.ws_o + (((size_t)split * e.m + tok) * e.H + h) * kHeadDim;
   };
   if constexpr (KP > 1) {
     constexpr int kTrade = WaveAttn<T, KB>::trade_bytes(KP), ND = 4 / KP;
@@ -762,12 +803,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     auto finish = [&](auto part) {
       constexpr int PART = decltype(part)::value;
       w.template take<KP, PART>(rows_lds, p.scale_log2e);
-      if (p.num_splits > 1 && rows > kFewRows)
+      if (SPLIT && rows > kFewRows)
         store_partial_rows<PART * ND, ND>(w, lds + RB * kTrade + wave * (32 * 128 * ND), part_row, part_ml, row_valid, rows - qblk0);
-      else if (p.num_splits > 1)
+      else if (SPLIT)
         store_partial<PART * ND, ND>(w, part_o, part_ml, row_valid);
       else
-        w.template store<PART * ND, ND>(lds + RB * kTrade + wave * (32 * 64 * ND), out_blk, q_row_bytes, p.m - qblk0);
+        w.template store<PART * ND, ND>(lds + RB * kTrade + wave * (32 * 64 * ND), out_blk, q_row_bytes, e.m - qblk0);
     };
     if (kpar == 0) finish(std::integral_constant<int, 0>());
     if (kpar == 1) finish(std::integral_constant<int, 1>());
@@ -775,13 +816,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       if (kpar == 2) finish(std::integral_constant<int, 2>());
       if (kpar == 3) finish(std::integral_constant<int, 3>());
     }
-  } else if (p.num_splits > 1) {  // (packed rows exist in split mode only)
+  } else if (SPLIT) {
     if (rows > kFewRows)
       store_partial_rows<0, 4>(w, lds + rb * 32 * 512, part_row, part_ml, row_valid, rows - qblk0);
     else
       store_partial(w, part_o, part_ml, row_valid);
   } else {
-    w.store(lds + rb * 32 * kRowBytes, out_blk, q_row_bytes, p.m - qblk0);
+    w.store(lds + rb * 32 * kRowBytes, out_blk, q_row_bytes, e.m - qblk0);
   }
 #ifdef LLMHIP_BENCH
   if (p.clock_probe && blockIdx.x == 0 && tid == 0) {
@@ -793,17 +834,21 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
 
 // Folds the key-range partials of the output rows with the log-sum-exp rule.  256 threads handle 8
 // (row, head) slots, 32 threads (4 dims each) per slot; grid = ceil(m * H / 8).
+// a: partials, their maxima and sums, out, slots per split (m * H); c: splits, scale.
 template <typename T>
-__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
+__global__ __launch_bounds__(256) void prefill_combine_kernel(addresses_t a, u32x2_t c) {
   using E = Elem<T>;
-  const size_t stride = (size_t)p.m * p.H;  // slots per split
+  const float *ws_o = at_address<const float>(a[0]), *ws_ml = at_address<const float>(a[1]);
+  char *out = at_address<char>(a[2]);
+  const float scale_log2e = __builtin_bit_cast(float, (uint32_t)c[1]);
+  const size_t stride = a[3];  // slots per split
   const size_t slot = (size_t)blockIdx.x * 8 + (threadIdx.x >> 5);
   const int d4 = threadIdx.x & 31;
   if (slot >= stride) return;
   // One pass, four key ranges per round: all loads of a round are issued before any is used, and the
   // running reference maximum moves between rounds (a pass for the maximum first would be one memory
   // round trip per key range).
-  const int S = p.num_splits;
+  const int S = c[0];
   float M = -INFINITY, L = 0.0f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = 0; s0 < S; s0 += 4) {
@@ -812,23 +857,23 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const size_t at = (size_t)min(s0 + j, S - 1) * stride + slot;
-      mv[j] = p.ws_ml[at * 2];
-      lv[j] = p.ws_ml[at * 2 + 1];
-      ov[j] = *reinterpret_cast<const f32x4_t *>(p.ws_o + at * kHeadDim + 4 * d4);
+      mv[j] = ws_ml[at * 2];
+      lv[j] = ws_ml[at * 2 + 1];
+      ov[j] = *reinterpret_cast<const f32x4_t *>(ws_o + at * kHeadDim + 4 * d4);
     }
     float Mn = M;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (s0 + j < S) Mn = fmaxf(Mn, mv[j]);
     const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
-    const float resc = fast_exp2((M - M_use) * p.scale_log2e);  // 0 on the first round (M = -inf)
+    const float resc = fast_exp2((M - M_use) * scale_log2e);  // 0 on the first round (M = -inf)
     L *= resc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] *= resc;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       // exp2(-inf) = 0 for an empty range
-      const float wt = (s0 + j < S) ? fast_exp2((mv[j] - M_use) * p.scale_log2e) : 0.0f;
+      const float wt = (s0 + j < S) ? fast_exp2((mv[j] - M_use) * scale_log2e) : 0.0f;
       L += wt * lv[j];
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
@@ -839,7 +884,7 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
   u32x2_t w;
   w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
   w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
-  *reinterpret_cast<u32x2_t *>(p.out + slot * kRowBytes + d4 * 8) = w;
+  *reinterpret_cast<u32x2_t *>(out + slot * kRowBytes + d4 * 8) = w;
 }
 
 // The same fold for few output rows and many key ranges (a short chunk over a very long cache): one
@@ -847,13 +892,16 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
 // sg, sg + 8, ..., four per round), the groups merged through LDS -- the slots alone would not fill
 // the chip and every thread would walk all ranges.  grid = m * H.
 template <typename T>
-__global__ __launch_bounds__(256) void prefill_combine_wide_kernel(PrefillParams p) {
+__global__ __launch_bounds__(256) void prefill_combine_wide_kernel(addresses_t a, u32x2_t c) {
   using E = Elem<T>;
+  const float *ws_o = at_address<const float>(a[0]), *ws_ml = at_address<const float>(a[1]);
+  char *out = at_address<char>(a[2]);
+  const float scale_log2e = __builtin_bit_cast(float, (uint32_t)c[1]);
   __shared__ float red_m[8], red_l[8];
   __shared__ f32x4_t red_o[8][32];
-  const size_t stride = (size_t)p.m * p.H, slot = blockIdx.x;
+  const size_t stride = a[3], slot = blockIdx.x;
   const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
-  const int S = p.num_splits;
+  const int S = c[0];
   float M = -INFINITY, L = 0.0f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s0 = sg; s0 < S; s0 += 32) {
@@ -862,22 +910,22 @@ __global__ __launch_bounds__(256) void prefill_combine_wide_kernel(PrefillParams
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const size_t at = (size_t)min(s0 + 8 * j, S - 1) * stride + slot;
-      mv[j] = p.ws_ml[at * 2];
-      lv[j] = p.ws_ml[at * 2 + 1];
-      ov[j] = *reinterpret_cast<const f32x4_t *>(p.ws_o + at * kHeadDim + 4 * d4);
+      mv[j] = ws_ml[at * 2];
+      lv[j] = ws_ml[at * 2 + 1];
+      ov[j] = *reinterpret_cast<const f32x4_t *>(ws_o + at * kHeadDim + 4 * d4);
     }
     float Mn = M;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       if (s0 + 8 * j < S) Mn = fmaxf(Mn, mv[j]);
     const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
-    const float resc = fast_exp2((M - M_use) * p.scale_log2e);
+    const float resc = fast_exp2((M - M_use) * scale_log2e);
     L *= resc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[i] *= resc;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float wt = (s0 + 8 * j < S) ? fast_exp2((mv[j] - M_use) * p.scale_log2e) : 0.0f;
+      const float wt = (s0 + 8 * j < S) ? fast_exp2((mv[j] - M_use) * scale_log2e) : 0.0f;
       L += wt * lv[j];
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
@@ -899,7 +947,7 @@ __global__ __launch_bounds__(256) void prefill_combine_wide_kernel(PrefillParams
   f32x4_t tot = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int g8 = 0; g8 < 8; ++g8) {
-    const float wt = fast_exp2((red_m[g8] - Mt_use) * p.scale_log2e);  // 0 for a group without ranges (-inf)
+    const float wt = fast_exp2((red_m[g8] - Mt_use) * scale_log2e);  // 0 for a group without ranges (-inf)
     Lt += wt * red_l[g8];
     const f32x4_t o = red_o[g8][d4];
 #pragma unroll
@@ -909,7 +957,7 @@ __global__ __launch_bounds__(256) void prefill_combine_wide_kernel(PrefillParams
   u32x2_t w;
   w[0] = E::pack2(tot[0] * inv, tot[1] * inv);
   w[1] = E::pack2(tot[2] * inv, tot[3] * inv);
-  *reinterpret_cast<u32x2_t *>(p.out + slot * kRowBytes + d4 * 8) = w;
+  *reinterpret_cast<u32x2_t *>(out + slot * kRowBytes + d4 * 8) = w;
 }
 
 template <typename T, int NW, int KP = 1>
@@ -917,23 +965,21 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   PrefillParams p = p0;
   constexpr int BM = 32 * NW / KP;
   constexpr int NT = 64 * NW;
-  p.num_q_tiles = (p.m + BM - 1) / BM;
-  if (p.pack) p.num_q_tiles = (p.m * p.g + BM - 1) / BM;
-  const int T_ = p.num_q_tiles;
+  const int T_ = ((p.pack ? p.m * p.g : p.m) + BM - 1) / BM;
   int grid, list_heads;
   const int S_ = p.num_splits;
-  p.sched_a = p.sched_shift = 0;
+  p.sched_shift = 0;
   if (p.pack) {
     p.sched_mode = 0;
     list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
   } else if (p.Hkv <= 8 && 8 % p.Hkv == 0) {
     p.sched_mode = 1;
-    p.sched_a = 8 / p.Hkv;
-    while ((1 << p.sched_shift) < p.sched_a) ++p.sched_shift;
+    const int xcds = 8 / p.Hkv;  // per kv head
+    while ((1 << p.sched_shift) < xcds) ++p.sched_shift;
     list_heads = p.g;
     const int per_kvh = p.g * T_ * S_;
-    grid = 8 * ((per_kvh + p.sched_a - 1) / p.sched_a);
+    grid = 8 * ((per_kvh + xcds - 1) / xcds);
   } else if (p.Hkv % 8 == 0) {
     p.sched_mode = 2;
     list_heads = (p.Hkv / 8) * p.g;
@@ -962,12 +1008,12 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   const size_t tile_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes, q_bytes = (size_t)BM * kRowBytes;
   const size_t lds_bytes = tile_bytes + (KP > 1 ? q_bytes : q_bytes - tile_bytes / 4);  // (half of the V slots are Q's at first)
   // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KP == 1 there)
-  const bool nt = KP == 1 && p.pack && T_ == 1;
-  void (*kern)(PrefillParams) = flash_prefill_kernel<T, NW, KP, false>;
-  if (nt) kern = flash_prefill_kernel<T, NW, KP, (KP == 1)>;
+  const bool nt = KP == 1 && p.pack && T_ == 1, cut = S_ > 1;
+  auto kern = flash_prefill_kernel<T, NW, KP, false, false>;
+  if (cut) kern = nt ? flash_prefill_kernel<T, NW, KP, (KP == 1), true> : flash_prefill_kernel<T, NW, KP, false, true>;
   // the opt-in for more than 64 KiB of dynamic LDS is per device: once per device and kernel
-  static std::atomic<uint64_t> attr_done_both[2];
-  std::atomic<uint64_t> &attr_done = attr_done_both[nt ? 1 : 0];
+  static std::atomic<uint64_t> attr_done_all[3];
+  std::atomic<uint64_t> &attr_done = attr_done_all[nt ? 2 : cut ? 1 : 0];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
@@ -978,14 +1024,17 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
     if (e != hipSuccess) return e;
     attr_done.fetch_or(bit, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds_bytes, stream, p);
+  const PrefillEarly early(p);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
   e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1) return e;
   const size_t slots = (size_t)p.m * p.H;
+  const addresses_t a = {address(p.ws_o), address(p.ws_ml), address(p.out), slots};
+  const u32x2_t c = {(uint32_t)p.num_splits, __builtin_bit_cast(uint32_t, p.scale_log2e)};
   if (slots <= 2048 && p.num_splits >= 8)
-    hipLaunchKernelGGL(prefill_combine_wide_kernel<T>, dim3((unsigned)slots), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(prefill_combine_wide_kernel<T>, dim3((unsigned)slots), dim3(256), 0, stream, a, c);
   else
-    hipLaunchKernelGGL(prefill_combine_kernel<T>, dim3((unsigned)((slots + 7) / 8)), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(prefill_combine_kernel<T>, dim3((unsigned)((slots + 7) / 8)), dim3(256), 0, stream, a, c);
   return hipGetLastError();
 }
 
@@ -1194,9 +1243,9 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
                                 hipStream_t stream, void *workspace, size_t workspace_bytes) {
   PrefillParams p;
 #endif
-  p.q = static_cast<const char *>(q);
-  p.k = static_cast<const char *>(k);
-  p.v = static_cast<const char *>(v);
+  p.q = q;
+  p.k = k;
+  p.v = v;
   p.out = static_cast<char *>(out);
   p.m = m;
   p.n = n;
