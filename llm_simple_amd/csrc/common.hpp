@@ -104,9 +104,8 @@ inline FastDiv make_fast_div(uint32_t d) {
   return f;
 }
 __device__ __forceinline__ uint32_t fast_div(uint32_t n, const FastDiv &f) {
-  if (f.l == 0) return n;  // d == 1
-  const uint32_t t = (uint32_t)(((uint64_t)n * f.m) >> 32);
-  return (t + ((n - t) >> 1)) >> (f.l - 1);
+  const uint32_t t = (uint32_t)(((uint64_t)n * f.m) >> 32), q = (t + ((n - t) >> 1)) >> ((f.l - 1) & 31);
+  return f.l == 0 ? n : q;  // (d == 1; without a branch)
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }

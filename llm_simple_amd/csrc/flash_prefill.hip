@@ -84,8 +84,7 @@ struct PrefillParams : PrefillLate {
   const void *q, *k, *v;
   int m, n, offset;
   int H, Hkv, g;
-  int sched_mode;  // 0: plain, 1: several XCDs per kv head, 2: several kv heads per XCD
-  int sched_shift;           // mode 1: logarithm of the XCDs per kv head
+  int xcd_bits, sched_shift;  // workgroups dealt to XCDs: 3 bits, and the logarithm of the XCDs per kv head; else 0
   int second, second_end;    // places of a list (of the XCD, mode 0: of the launch) that are taken in reverse
   FastDiv list_heads;        // heads of an XCD's work list
   FastDiv g_div;
@@ -97,32 +96,33 @@ struct PrefillParams : PrefillLate {
 // What the index arithmetic and the first loads of a workgroup need, packed into the first 14 words of a kernel's arguments, which
 // are in registers when it starts.  With kernels of their own for key ranges, whose packed rows and partials a prompt need not step
 // over (both together, attention alone, us: 32 tokens of 32 heads 4.65 -> 4.21, 256 5.85 -> 5.50, 512 of 28 8.44 -> 7.94, 1019 14.4 ->
-// 14.05, 2048 35.6 -> 34.8, 4096 113.5 -> 112.8; 200 past 16001 53.1 -> 51.75, 100 past 8000 of 40 25.2 -> 24.1).
+// 14.05, 2048 35.6 -> 34.8, 4096 113.5 -> 112.8; 200 past 16001 53.1 -> 51.75, 100 past 8000 of 40 25.2 -> 24.1).  It counts
+// instructions: one wave issues one in 4-5 cycles, so the lists' forms are one formula, divisions have no branch, tiles are counted by
+// shifts and what a load needs of the last tile is kept (230 instead of 290 of them to the first K line: 32 tokens 4.22 -> 4.00, 256
+// 5.50 -> 5.32, 512 of 28 7.93 -> 7.80; 20 past 600 7.24 -> 7.07).
 struct PrefillEarly {
   addresses_t a;  // q, K, V, m | n << 32
   u32x4_t b;      // offset, Hkv | g << 16, flags, second | second_end << 16
   u32x2_t c;      // factors of the divisions by g and by the heads of a list
-  // flags: sched_mode, sched_shift << 2, pack << 5, shifts of the divisions << 8 and << 16
+  // flags: xcd_bits, sched_shift << 2, pack << 4, shifts of the divisions << 5 and << 10, heads of a list << 16
   explicit PrefillEarly(const PrefillParams &p) {
     a = addresses_t{address(p.q), address(p.k), address(p.v), (uint32_t)p.m | (uint64_t)p.n << 32};
     b = u32x4_t{(uint32_t)p.offset, (uint32_t)p.Hkv | (uint32_t)p.g << 16,
-                (uint32_t)(p.sched_mode | p.sched_shift << 2 | p.pack << 5) | p.g_div.l << 8 | p.list_heads.l << 16,
+                (uint32_t)(p.xcd_bits | p.sched_shift << 2 | p.pack << 4) | p.g_div.l << 5 | p.list_heads.l << 10 | p.list_heads.d << 16,
                 (uint32_t)p.second | (uint32_t)p.second_end << 16};
     c = u32x2_t{p.g_div.m, p.list_heads.m};
   }
 };
 struct PrefillShared {  // the same, unpacked
   const char *q, *k, *v;
-  int m, n, offset, H, Hkv, g, sched_mode, sched_shift, second, second_end;
+  int m, n, offset, H, Hkv, g, xcd_bits, sched_shift, second, second_end;
   bool pack;
   FastDiv g_div, list_heads;
   __device__ __forceinline__ PrefillShared(addresses_t a, u32x4_t b, u32x2_t c)
       : q(at_address<const char>(a[0])), k(at_address<const char>(a[1])), v(at_address<const char>(a[2])), m((uint32_t)a[3]),
         n((uint32_t)(a[3] >> 32)), offset(b[0]), H((b[1] & 0xffffu) * (b[1] >> 16)), Hkv(b[1] & 0xffffu), g(b[1] >> 16),
-        sched_mode(b[2] & 3u), sched_shift(b[2] >> 2 & 7u), second(b[3] & 0xffffu), second_end(b[3] >> 16), pack(b[2] & 32u),
-        g_div{b[1] >> 16, c[0], b[2] >> 8 & 63u} {
-    list_heads = FastDiv{(uint32_t)(sched_mode == 1 ? g : sched_mode == 2 ? (Hkv >> 3) * g : pack ? Hkv : H), c[1], b[2] >> 16 & 63u};
-  }
+        xcd_bits(b[2] & 3u), sched_shift(b[2] >> 2 & 3u), second(b[3] & 0xffffu), second_end(b[3] >> 16), pack(b[2] & 16u),
+        g_div{b[1] >> 16, c[0], b[2] >> 5 & 31u}, list_heads{b[2] >> 16, c[1], b[2] >> 10 & 31u} {}
 };
 
 // blockIdx -> (query tile, head, key range).  Workgroup ids are dealt round-robin to the 8
@@ -133,16 +133,10 @@ struct PrefillShared {  // the same, unpacked
 template <bool SPLIT>
 __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const PrefillLate &p, int bid, int num_q_tiles, int &tile,
                                                  int &head, int &split) {
-  int idx = bid, xcd = 0;
-  if (e.sched_mode != 0) {
-    xcd = bid & 7;
-    idx = bid >> 3;
-  }
+  int idx = bid >> e.xcd_bits, xcd = bid & ((1 << e.xcd_bits) - 1);
   if (idx >= e.second && idx < e.second_end) idx = e.second + e.second_end - 1 - idx;
-  if (e.sched_mode == 1) {  // 2^sched_shift XCDs per kv head
-    idx = (idx << e.sched_shift) + (xcd & ((1 << e.sched_shift) - 1));
-    xcd >>= e.sched_shift;  // the kv head
-  }
+  idx = (idx << e.sched_shift) + (xcd & ((1 << e.sched_shift) - 1));  // 2^sched_shift XCDs per kv head (one: of several heads)
+  xcd >>= e.sched_shift;
   // idx: (key range, tile from the last, head among the list's `list_heads`)
   int rem = idx;
   split = 0;
@@ -536,13 +530,15 @@ typedef __attribute__((ext_vector_type(4))) uint32_t buffer_t;
 template <int NW, int TN, bool NT> struct DirectLoader {
   static constexpr int kSlots = TN / 4 / NW;  // instructions per wave per tile
   static constexpr int kLow = 1024 * ((kSlots < 4 ? kSlots : 4) - 1);
-  int n, row_bytes;
+  uint32_t tile_step, whole, last;            // bytes to the next tile; records of a whole tile and of the last one
   uint32_t lds_wave;                          // LDS byte offset of the wave's first row (wave-uniform)
   uint32_t off_k[kSlots], off_v[kSlots];      // lane offsets within a tile
 
-  __device__ __forceinline__ void init(int wave, int lane, int row_bytes_, int n_) {
-    n = n_;
-    row_bytes = row_bytes_;
+  // n keys in J tiles
+  __device__ __forceinline__ void init(int wave, int lane, int row_bytes, int n, int J) {
+    tile_step = TN * row_bytes;
+    whole = (TN - 1) * row_bytes + kRowBytes + kLow;
+    last = min(TN - 1, n - (J - 1) * TN - 1) * row_bytes + kRowBytes + kLow;
     lds_wave = __builtin_amdgcn_readfirstlane(wave * kSlots * 1024);
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
@@ -560,17 +556,17 @@ template <int NW, int TN, bool NT> struct DirectLoader {
     buffer_t d;
     int left;  // tiles to come
   };
-  __device__ __forceinline__ uint32_t records(int rows) const { return (uint32_t)(rows - 1) * row_bytes + kRowBytes + kLow; }
   __device__ __forceinline__ Stream stream(const char *base, int J) const {
     const uint64_t at = (uint64_t)base - kLow;
-    return Stream{{(uint32_t)at, (uint32_t)(at >> 32), records(min(TN, n)), 0x00020000u}, J - 1};
+    return Stream{{(uint32_t)at, (uint32_t)(at >> 32), J > 1 ? whole : last, 0x00020000u}, J - 1};
   }
-  __device__ __forceinline__ void next(Stream &st, int J) const {
-    const uint64_t at = (((uint64_t)st.d[1] << 32) | st.d[0]) + (st.left > 0 ? (uint32_t)(TN * row_bytes) : 0u);
+  __device__ __forceinline__ void next(Stream &st) const {
+    const uint64_t at = (((uint64_t)st.d[1] << 32) | st.d[0]) + (st.left > 0 ? tile_step : 0u);
     st.left -= 1;
     st.d[0] = (uint32_t)at;
     st.d[1] = (uint32_t)(at >> 32);
-    st.d[2] = st.left > 0 ? records(TN) : st.left == 0 ? records(min(TN, n - (J - 1) * TN)) : 0u;
+    const uint32_t bytes = st.left > 0 ? whole : last;
+    st.d[2] = st.left < 0 ? 0u : bytes;
   }
   // Slots 0 .. kSlots-1 of a tile in order, with no other tile's in between; lds_tile: LDS byte offset of the destination.
   // NT: the tile is read by this workgroup only (a packed chunk of one tile per kv head over a long
@@ -650,15 +646,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   const int n_ = SPLIT ? min(e.n - k_lo, p.chunk) : e.n;
   const int offset_ = e.offset - k_lo;
   const int n_vis = min(n_, tile_tok_end + offset_);  // keys any row of this tile can see
-  const int J = (n_vis + TN - 1) / TN;        // tiles of the workgroup
-  const size_t q_row_bytes = (size_t)e.H * kRowBytes;
+  constexpr int kTileShift = TN == 128 ? 7 : 6;
+  static_assert(1 << kTileShift == TN, "");
+  const int J = (n_vis + TN - 1) >> kTileShift;  // tiles of the workgroup
+  const uint32_t q_row_bytes = (uint32_t)e.H * kRowBytes;
   const int kv_row_bytes = e.Hkv * kRowBytes;
   const char *kbase = e.k + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
   const char *vbase = e.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
 
   WaveAttn<T, KB> w;
   // tiles in which this wave's keys hold at least one visible key
-  const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) / TN)) : 0;
+  const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) >> kTileShift)) : 0;
   float *part_o = nullptr, *part_ml = nullptr;
   if (SPLIT) {
     const size_t slot = ((size_t)split * e.m + qtok) * e.H + qhead;
@@ -682,15 +680,15 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     const char *src = e.q + ((lane & 15) ^ (r & 15)) * 16;
     if (pack) {
       const int tok = (int)fast_div(idx, e.g_div);
-      src += (size_t)tok * q_row_bytes + (size_t)(head + idx - tok * e.g) * kRowBytes;
+      src += (uint64_t)(uint32_t)tok * q_row_bytes + (uint32_t)(head + idx - tok * e.g) * kRowBytes;
     } else {
-      src += (size_t)idx * q_row_bytes + (size_t)head * kRowBytes;
+      src += (uint64_t)(uint32_t)idx * q_row_bytes + (uint32_t)head * kRowBytes;
     }
     lds_dma(src, kQRegion + (sl * NW + wave) * 4 * kRowBytes);
   }
 
   DirectLoader<NW, TN, NT> ld;
-  ld.init(wave, lane, kv_row_bytes, n_);
+  ld.init(wave, lane, kv_row_bytes, n_, J);
   // K runs one tile ahead of V: S(j+1) = K(j+1) Q^T is issued together with the softmax of
   // tile j, so K tile t is fetched SUB+1 iterations and V tile t SUB iterations before use.
   using Loader = DirectLoader<NW, TN, NT>;
@@ -698,10 +696,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   static_for<0, SUB + 1>([&](auto u_) {
     constexpr int u = decltype(u_)::value;
     static_for<0, PER>([&](auto r) { ld.template issue<false, decltype(r)::value>(kst, u % NSLOT * TB); });
-    ld.next(kst, J);
+    ld.next(kst);
     if constexpr (u < SUB) {
       static_for<0, PER>([&](auto r) { ld.template issue<true, decltype(r)::value>(vst, kVRegion + u * TB); });
-      ld.next(vst, J);
+      ld.next(vst);
     }
   });
   // The late arguments are asked for now, while the loads are under way, not at the place of each one's use
@@ -764,8 +762,8 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       static_for<0, PER>([&](auto r) { ld.template issue<false, decltype(r)::value>(kst, kslot * TB); });
       static_for<0, PER>([&](auto r) { ld.template issue<true, decltype(r)::value>(vst, kVRegion + vslot * TB); });
     }
-    ld.next(kst, J);
-    ld.next(vst, J);
+    ld.next(kst);
+    ld.next(vst);
   };
 
   for (int jb = 0; jb < J; jb += NSLOT) {
@@ -968,24 +966,22 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   const int T_ = ((p.pack ? p.m * p.g : p.m) + BM - 1) / BM;
   int grid, list_heads;
   const int S_ = p.num_splits;
-  p.sched_shift = 0;
+  p.xcd_bits = p.sched_shift = 0;
   if (p.pack) {
-    p.sched_mode = 0;
     list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
   } else if (p.Hkv <= 8 && 8 % p.Hkv == 0) {
-    p.sched_mode = 1;
+    p.xcd_bits = 3;
     const int xcds = 8 / p.Hkv;  // per kv head
     while ((1 << p.sched_shift) < xcds) ++p.sched_shift;
     list_heads = p.g;
     const int per_kvh = p.g * T_ * S_;
     grid = 8 * ((per_kvh + xcds - 1) / xcds);
   } else if (p.Hkv % 8 == 0) {
-    p.sched_mode = 2;
+    p.xcd_bits = 3;
     list_heads = (p.Hkv / 8) * p.g;
     grid = 8 * list_heads * T_ * S_;
   } else {
-    p.sched_mode = 0;
     list_heads = p.H;
     grid = T_ * p.H * S_;
   }
@@ -996,7 +992,7 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   // 62.0 -> 60.2).
   p.second = p.second_end = 0;
   if (NW == 4 && KP < 4 && S_ == 1) {
-    const int lists = p.sched_mode == 0 ? 1 : 8, len = grid / lists, first = device_compute_units() / lists;
+    const int lists = 1 << p.xcd_bits, len = grid / lists, first = device_compute_units() / lists;
     if (len > first && (KP == 1 || len <= 2 * first + first / 8)) {
       p.second = first;
       p.second_end = len < 2 * first ? len : 2 * first;
