@@ -75,19 +75,27 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t 
   }
 }
 
-template <typename T, bool NEOX>
+// PLACED: workgroup b works for XCD b % 8, on rows that the attention launch to come reads there (prefill_schedule in
+// flash_prefill.hip): the heads of that XCD's kv heads, or, where two XCDs share one, those of every second token.
+// What these stores leave in an XCD's L2 is valid and clean, and Q, K and V are then read from there.  Which rows go where
+// is nothing but speed.
+template <typename T, bool NEOX, bool PLACED>
 __global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u32x4_t size, u32x2_t heads_, RopeOut to) {
-  // in_: q, k, v, the table; size: threads, factor and shift of the division by the rows of a token (bit 8: there is a V), start_pos
-  const uint32_t total = size[0], rows_mul = size[1], rows_shift = size[2];
+  // in_: q, k, v, the table; size: tokens (PLACED) or threads, factor and shift of the division by a token's rows in a list (bit 8:
+  // there is a V; PLACED, from bit 9 on: logarithm of the XCDs that share a list), start_pos
   const int start_pos = size[3], q_heads = heads_[0], k_heads = heads_[1];
-  const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
-  if (gid >= total) return;
-  const FastDiv rows_per_token = {(uint32_t)(q_heads + k_heads + (rows_shift & 256u ? k_heads : 0)), rows_mul, rows_shift & 255u};
-  const uint32_t j = gid & 7u, rowid = gid >> 3, s = fast_div(rowid, rows_per_token);
-  const int r = (int)(rowid - s * rows_per_token.d);
-  const bool is_q = r < q_heads, rotated = r < q_heads + k_heads;
+  const uint32_t share = PLACED ? size[2] >> 9 : 0, xcd = PLACED ? blockIdx.x & 7u : 0, lists = PLACED ? 3 - share : 0;
+  const uint32_t gid = (PLACED ? blockIdx.x >> 3 : blockIdx.x) * 256u + threadIdx.x;
+  if (!PLACED && gid >= size[0]) return;
+  const int q_list = q_heads >> lists, k_list = k_heads >> lists;
+  const FastDiv rows_per_token = {(uint32_t)(q_list + k_list + (size[2] & 256u ? k_list : 0)), size[1], size[2] & 255u};
+  const uint32_t j = gid & 7u, rowid = gid >> 3, t = fast_div(rowid, rows_per_token);
+  const uint32_t s = PLACED ? (t << share) + (xcd & ((1u << share) - 1)) : t;
+  if (PLACED && s >= size[0]) return;
+  const int r = (int)(rowid - t * rows_per_token.d), list = xcd >> share;
+  const bool is_q = r < q_list, rotated = r < q_list + k_list;
   const int heads = is_q ? q_heads : k_heads;  // V has as many as K
-  const int h = is_q ? r : rotated ? r - q_heads : r - q_heads - k_heads;
+  const int h = is_q ? list * q_list + r : list * k_list + r - q_list - (rotated ? 0 : k_list);
   const char *in = at_address<const char>(is_q ? in_[0] : rotated ? in_[1] : in_[2]);
   in += ((size_t)s * heads + h) * kRowBytes + j * 16;
   const float *tab = at_address<const float>(in_[3]) + (size_t)(start_pos + s) * kHeadDim + (NEOX ? 16 : 8) * j;
@@ -109,6 +117,14 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u3
   store_device_b128(out + 128, b);
 }
 
+constexpr int kPlacedTokens = 64;
+constexpr long long kPlacedBytes = 13 << 19;
+
+template <typename T> static auto kernel_of(bool neox, bool placed) {
+  if (placed) return neox ? rope_kv_append_kernel<T, true, true> : rope_kv_append_kernel<T, false, true>;
+  return neox ? rope_kv_append_kernel<T, true, false> : rope_kv_append_kernel<T, false, false>;
+}
+
 hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const void *freq_cis,
                                  const void *in_q, const void *in_k, const void *in_v,
                                  int start_pos, int cur_size, int q_heads, int k_heads,
@@ -117,14 +133,24 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   const long long total = (long long)cur_size * rows * 8;
   if (total == 0) return hipSuccess;
   if (rows > 0x7FFFFFFFLL || total > 0x7FFFFFFFLL) return hipErrorInvalidValue;  // 32-bit thread index
-  const FastDiv div = make_fast_div((uint32_t)rows);
+  // Rows placed: a prompt (a chunk's workgroups are dealt otherwise) of kv heads that make whole lists, where what is written fits
+  // the L2s beside what is read.  Rope and attention, us, in order / placed: 128 tokens of 32 kv heads 8.27 / 7.07, 256 9.50 / 9.11,
+  // 300 10.42 / 10.42, 512 13.66 / 13.87; 200 of 8 (40 heads) 8.53 / 8.01, 400 11.46 / 11.04, 600 14.07 / 14.17; 200 of 4 (28) 8.01 / 7.84,
+  // 512 11.56 / 11.23, 700 14.01 / 14.02, 1019 18.12 / 18.21; 20 of 4 6.21 / 6.32.  Four XCDs to a kv head: nothing (256 of 2 7.73 / 7.79).
+  int share = -1;  // logarithm of the XCDs of a list
+  if (cur_size >= kPlacedTokens && start_pos < cur_size && total * 32 <= kPlacedBytes && k_heads > 0 && q_heads % k_heads == 0)
+    share = k_heads % 8 == 0 ? 0 : k_heads == 4 ? 1 : -1;
+  const bool placed = share >= 0;
+  const uint32_t list_rows = (uint32_t)(placed ? rows >> (3 - share) : rows);
+  const FastDiv div = make_fast_div(list_rows);
   const size_t first = (size_t)k_out_row_offset * k_heads * kRowBytes;
   const RopeOut to = {static_cast<char *>(out_q), static_cast<char *>(out_k) + first, static_cast<char *>(out_v) + first};
-  const int grid = (int)((total + 255) / 256);
-  const auto kern = (dt == kDtFloat16) ? (is_neox ? rope_kv_append_kernel<_Float16, true> : rope_kv_append_kernel<_Float16, false>)
-                                       : (is_neox ? rope_kv_append_kernel<__bf16, true> : rope_kv_append_kernel<__bf16, false>);
+  const long long threads = placed ? (long long)((cur_size + (1 << share) - 1) >> share) * list_rows * 8 : total;
+  const int grid = (int)((threads + 255) / 256) * (placed ? 8 : 1);
+  const auto kern = (dt == kDtFloat16) ? kernel_of<_Float16>(is_neox, placed) : kernel_of<__bf16>(is_neox, placed);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, addresses_t{address(in_q), address(in_k), address(in_v), address(freq_cis)},
-                     u32x4_t{(uint32_t)total, div.m, div.l | (in_v != nullptr ? 256u : 0u), (uint32_t)start_pos},
+                     u32x4_t{(uint32_t)(placed ? cur_size : total), div.m,
+                             div.l | (in_v != nullptr ? 256u : 0u) | (placed ? (uint32_t)share << 9 : 0u), (uint32_t)start_pos},
                      u32x2_t{(uint32_t)q_heads, (uint32_t)k_heads}, to);
   return hipGetLastError();
 }
