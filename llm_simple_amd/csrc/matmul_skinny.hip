@@ -20,6 +20,13 @@
 // four units at a time and a second, empty group of rows / this: 512 x 3584 4.13 / 3.68, 1024 x 5120 5.45 / 4.65, 256 x 1536
 // 2.97 / 2.82, 2048 x 11008, in several rounds of 8, 11.45 / 10.62).  With more rows the stream is what counts, and four units of
 // two groups are what a CU can have under way (3584 x 3584, two / four / six / eight 7.07 / 6.25 / 6.67 / 6.28).
+//
+// EXACT: k is a multiple of 512, so that every wave has the same units, and nothing is asked for or left out under a mask: a
+// mask and a branch to each load were 190 of the 270 instructions before the first MFMA, and a wave issues one in 4-5 cycles (us, with
+// masks and the bias fetched at the end / this: 512 x 3584 3.50 / 3.35, 3584 x 3584 6.03 / 5.90, 1024 x 5120 4.48 / 4.32, 5120 x 5120, two
+// passes of five units, 11.05 / 10.05, 18944 x 3584 23.0 / 21.2, 1536 x 1536 3.13 / 2.99; eight rows 4096 x 4096 8.16 / 7.93).  Not
+// where it takes more passes than two, nor two of more than five units: they end and begin all at once (1024 x 8192, two of eight
+// 5.68 / 5.90; 4096 x 7168, two of seven 10.87 / 11.45; 4096 x 6144, three of four 9.74 / 9.91; 4096 x 10240, four of five 15.2 / 15.9).
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -32,7 +39,7 @@ constexpr int kSkinnyWaves = 8;
 // KS k-slices per MFMA: operand row (column) index i stands for W (lhs) row i % (16/KS) at slice
 // i / (16/KS).  TW groups of 16/KS W rows; B units of 32*KS k per wave and pass.  rows: W rows of a workgroup, at most 16.
 // a: lhs, W, bias, out; size: m, n, k, rows.
-template <typename T, int KS, int TW, int B>
+template <typename T, int KS, int TW, int B, bool EXACT>
 __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(addresses_t a, u32x4_t size) {
   using E = Elem<T>;
   const uint16_t *x = at_address<const uint16_t>(a[0]), *w = at_address<const uint16_t>(a[1]);
@@ -41,47 +48,77 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(add
   const int m = size[0], n = size[1], k = size[2], row_share = size[3];
   constexpr int NW = kSkinnyWaves, R = 16 / KS, UK = 32 * KS;
   __shared__ __attribute__((aligned(16))) float red[NW * TW * 256];  // [wave][group of R rows][lane] of f32x4
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i = lane & 15, cg = lane >> 4, r = i % R;
   const int n0 = blockIdx.x * row_share;
   const int rows = min(row_share, n - n0);
   const int koff = 32 * (i / R) + 8 * cg;
-  const uint16_t *wp[TW];
-#pragma unroll
-  for (int t = 0; t < TW; ++t) wp[t] = w + (size_t)(n0 + min(t * R + r, rows - 1)) * k + koff;
-  const bool xv = r < m;
-  const uint16_t *xp = x + (size_t)(xv ? r : 0) * k + koff;
   f32x4_t acc[TW];
 #pragma unroll
   for (int t = 0; t < TW; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int units = (k + UK - 1) / UK;
-  const u32x4_t zero = {0u, 0u, 0u, 0u};
-  for (int u0 = wave; u0 < units; u0 += NW * B) {
-    u32x4_t wf[B][TW], xf[B];
+  // The result that this thread will write: feature n0 + f of lhs row `row`.  Its bias is asked for beside the operands, not when the
+  // sum is there.
+  const int f = tid & 15, row = tid >> 4;
+  const bool writes = f < rows && row < m;
+  float bias_here = 0.0f;
+  if constexpr (EXACT) {
+    // What rows past the share or past m hold reaches no result: they read the last (first) one again.
+    const char *wb = reinterpret_cast<const char *>(w + (size_t)n0 * k + wave * UK), *xb = reinterpret_cast<const char *>(x + wave * UK);
+    uint32_t wo[TW];
 #pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const int kk = (u0 + b * NW) * UK;
-      const bool in = kk + koff < k;  // k is a multiple of 16, a fragment 8 long
+    for (int t = 0; t < TW; ++t) wo[t] = 2 * ((uint32_t)min(t * R + r, rows - 1) * k + koff);
+    const uint32_t xo = 2 * ((uint32_t)(r < m ? r : 0) * k + koff);
+    constexpr int kPass = 2 * NW * UK * B;
+    for (int left = 2 * k; left > 0; left -= kPass, wb += kPass, xb += kPass) {
+      u32x4_t wf[B][TW], xf[B];
 #pragma unroll
-      for (int t = 0; t < TW; ++t) {
-        wf[b][t] = zero;
-        if (in && t * R + r < rows) wf[b][t] = KS > 1 ? global_load_b128_nt(wp[t] + kk) : global_load_b128(wp[t] + kk);
+      for (int b = 0; b < B; ++b) {
+#pragma unroll
+        for (int t = 0; t < TW; ++t) wf[b][t] = global_load_b128_nt(wb + b * (2 * NW * UK) + wo[t]);
+        xf[b] = global_load_b128(xb + b * (2 * NW * UK) + xo);
       }
-      xf[b] = zero;
-      if (in && xv) xf[b] = global_load_b128(xp + kk);
+      __builtin_amdgcn_sched_barrier(0);
+      if (bias && writes && left == 2 * k) bias_here = bias[n0 + f];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
     }
+  } else {
+    if (bias && writes) bias_here = bias[n0 + f];
+    const uint16_t *wp[TW];
 #pragma unroll
-    for (int b = 0; b < B; ++b)
+    for (int t = 0; t < TW; ++t) wp[t] = w + (size_t)(n0 + min(t * R + r, rows - 1)) * k + koff;
+    const bool xv = r < m;
+    const uint16_t *xp = x + (size_t)(xv ? r : 0) * k + koff;
+    const int units = (k + UK - 1) / UK;
+    const u32x4_t zero = {0u, 0u, 0u, 0u};
+    for (int u0 = wave; u0 < units; u0 += NW * B) {
+      u32x4_t wf[B][TW], xf[B];
 #pragma unroll
-      for (int t = 0; t < TW; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
+      for (int b = 0; b < B; ++b) {
+        const int kk = (u0 + b * NW) * UK;
+        const bool in = kk + koff < k;  // k is a multiple of 16, a fragment 8 long
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+          wf[b][t] = zero;
+          if (in && t * R + r < rows) wf[b][t] = KS > 1 ? global_load_b128_nt(wp[t] + kk) : global_load_b128(wp[t] + kk);
+        }
+        xf[b] = zero;
+        if (in && xv) xf[b] = global_load_b128(xp + kk);
+      }
+#pragma unroll
+      for (int b = 0; b < B; ++b)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) acc[t] = E::mfma16(wf[b][t], xf[b], acc[t]);
+    }
   }
   f32x4_t *slots = reinterpret_cast<f32x4_t *>(red);
 #pragma unroll
   for (int t = 0; t < TW; ++t) slots[(wave * TW + t) * 64 + lane] = acc[t];
   __syncthreads();
-  // thread: feature n0 + f of lhs row `row`
-  const int f = tid & 15, row = tid >> 4;
-  if (f >= rows || row >= m) return;
+  if (!writes) return;
   float sum = 0.0f;
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -90,17 +127,39 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(add
 #pragma unroll
     for (int v = 0; v < NW; ++v) sum += src[v * TW * 256];
   }
-  if (bias) sum += bias[n0 + f];
+  if (bias) sum += bias_here;
   out[(size_t)row * n + n0 + f] = E::round(sum);
 }
 
 using SkinnyKernel = void (*)(addresses_t, u32x4_t);
+template <typename T, int TW> SkinnyKernel exact_kernel(int units) {
+  constexpr int most = TW == 1 ? 12 : 8;  // (registers)
+  switch (units) {
+    case 1: return matmul_skinny_kernel<T, 2, TW, 1, true>;
+    case 2: return matmul_skinny_kernel<T, 2, TW, 2, true>;
+    case 3: return matmul_skinny_kernel<T, 2, TW, 3, true>;
+    case 4: return matmul_skinny_kernel<T, 2, TW, 4, true>;
+    case 5: return matmul_skinny_kernel<T, 2, TW, 5, true>;
+    case 6: return matmul_skinny_kernel<T, 2, TW, 6, true>;
+    case 7: return matmul_skinny_kernel<T, 2, TW, 7, true>;
+    case 8: return matmul_skinny_kernel<T, 2, TW, 8, true>;
+    case 9: return matmul_skinny_kernel<T, 2, TW, 9 < most ? 9 : most, true>;
+    case 10: return matmul_skinny_kernel<T, 2, TW, 10 < most ? 10 : most, true>;
+    case 11: return matmul_skinny_kernel<T, 2, TW, 11 < most ? 11 : most, true>;
+    default: return matmul_skinny_kernel<T, 2, TW, most, true>;
+  }
+}
 template <typename T> SkinnyKernel kernel_of(int m, int k, int rows) {
-  if (m > 8) return matmul_skinny_kernel<T, 1, 1, 8>;
-  if (rows > 8) return matmul_skinny_kernel<T, 2, 2, 4>;
-  const int units = (k + 64 * kSkinnyWaves - 1) / (64 * kSkinnyWaves);  // of a wave
-  if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4>;
-  return units > 8 && units <= 12 ? matmul_skinny_kernel<T, 2, 1, 12> : matmul_skinny_kernel<T, 2, 1, 8>;
+  if (m > 8) return matmul_skinny_kernel<T, 1, 1, 8, false>;
+  const int round = 64 * kSkinnyWaves, units = (k + round - 1) / round;  // of a wave
+  if (k % round == 0 && rows <= 8 && units <= 12) return exact_kernel<T, 1>(units);
+  if (k % round == 0 && rows > 8) {
+    if (units <= 8) return exact_kernel<T, 2>(units);
+    if (units == 10) return exact_kernel<T, 2>(5);  // two passes; more of them are not faster
+  }
+  if (rows > 8) return matmul_skinny_kernel<T, 2, 2, 4, false>;
+  if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4, false>;
+  return units > 8 && units <= 12 ? matmul_skinny_kernel<T, 2, 1, 12, false> : matmul_skinny_kernel<T, 2, 1, 8, false>;
 }
 
 }  // namespace
