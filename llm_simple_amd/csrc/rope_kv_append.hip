@@ -24,7 +24,7 @@
 //
 // Bound by the memory path of three separate streams of 256-byte rows.  4096 tokens of 28 + 2 x 4 heads (75.5 MB): 11.9 us
 // with the buffers in the last-level cache, 15.2 from and to HBM, where a plain device copy of the same bytes takes
-// 10.4 and 16; 256 tokens of 32 + 2 x 32 heads 3.1 us, of which an empty launch is 1.55.  One piece to a thread: two, a
+// 10.4 and 16; 256 tokens of 32 + 2 x 32 heads 2.85 us, of which an empty launch is 1.55.  One piece to a thread: two, a
 // grid apart, kept half as many waves (a layer's rope and attention, us, two / one: 64 tokens of 32 heads 8.29 / 8.02,
 // 256 10.80 / 10.52, 1500 41.9 / 40.9, 256 of 12 9.03 / 8.61).
 #include "common.hpp"
