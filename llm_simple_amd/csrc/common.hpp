@@ -191,7 +191,8 @@ __device__ __forceinline__ u32x4_t global_load_b128_nt(const void *p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(p));
 }
 // A store that goes past the XCD's own L2 at once (sc1): what an ordinary one leaves there is written back at the end of the
-// launch, before the next one begins.  Wants whole 128-byte lines: a part of one is a write to memory of its own.
+// launch, before the next one begins.  Wants whole 64-byte sectors: a part of one is a write to memory of its own (rope_kv_append.hip
+// has figures of outputs that begin off one).
 __device__ __forceinline__ void store_device_b128(void *p, u32x4_t v) {
   __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4_t *)p, v, "agent");
 }

@@ -75,14 +75,17 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t 
   }
 }
 
-// PLACED: workgroup b works for XCD b % 8, on rows that the attention launch to come reads there (prefill_schedule in
+enum RopeWay { kInOrder, kPlaced, kOrdinaryStores };  // (in order too)
+
+// kPlaced: workgroup b works for XCD b % 8, on rows that the attention launch to come reads there (prefill_schedule in
 // flash_prefill.hip): the heads of that XCD's kv heads, or, where two XCDs share one, those of every second token.
 // What these stores leave in an XCD's L2 is valid and clean, and Q, K and V are then read from there.  Which rows go where
 // is nothing but speed.
-template <typename T, bool NEOX, bool PLACED>
+template <typename T, bool NEOX, RopeWay WAY>
 __global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u32x4_t size, u32x2_t heads_, RopeOut to) {
-  // in_: q, k, v, the table; size: tokens (PLACED) or threads, factor and shift of the division by a token's rows in a list (bit 8:
-  // there is a V; PLACED, from bit 9 on: logarithm of the XCDs that share a list), start_pos
+  // in_: q, k, v, the table; size: tokens (kPlaced) or threads, factor and shift of the division by a token's rows in a list (bit 8:
+  // there is a V; kPlaced, from bit 9 on: logarithm of the XCDs that share a list), start_pos
+  constexpr bool PLACED = WAY == kPlaced;
   const int start_pos = size[3], q_heads = heads_[0], k_heads = heads_[1];
   const uint32_t share = PLACED ? size[2] >> 9 : 0, xcd = PLACED ? blockIdx.x & 7u : 0, lists = PLACED ? 3 - share : 0;
   const uint32_t gid = (PLACED ? blockIdx.x >> 3 : blockIdx.x) * 256u + threadIdx.x;
@@ -113,16 +116,23 @@ __global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u3
   // Rope and attention, us, ordinary stores / these: 256 tokens of 28 heads 9.88 / 9.38, 1019 of 28 21.9 / 20.8, 400 of 40
   // 13.7 / 12.7, 4096 of 28 130.8 / 130.1; whole lines alone 256 tokens of 32 heads, interleaved, 11.7 -> 11.3, both 10.6.
   // (Non-temporal stores are shorter still by themselves, and the rows then come back from HBM: 1019 tokens 24.3.)
-  store_device_b128(out, a);
-  store_device_b128(out + 128, b);
+  if constexpr (WAY == kOrdinaryStores) {
+    *reinterpret_cast<u32x4_t *>(out) = a;
+    *reinterpret_cast<u32x4_t *>(out + 128) = b;
+  } else {
+    store_device_b128(out, a);
+    store_device_b128(out + 128, b);
+  }
 }
 
 constexpr int kPlacedTokens = 64;
 constexpr long long kPlacedBytes = 13 << 19;
+constexpr long long kOffSectorBytes = 11 << 20;
 
-template <typename T> static auto kernel_of(bool neox, bool placed) {
-  if (placed) return neox ? rope_kv_append_kernel<T, true, true> : rope_kv_append_kernel<T, false, true>;
-  return neox ? rope_kv_append_kernel<T, true, false> : rope_kv_append_kernel<T, false, false>;
+template <typename T> static auto kernel_of(bool neox, RopeWay way) {
+  if (way == kPlaced) return neox ? rope_kv_append_kernel<T, true, kPlaced> : rope_kv_append_kernel<T, false, kPlaced>;
+  if (way == kOrdinaryStores) return neox ? rope_kv_append_kernel<T, true, kOrdinaryStores> : rope_kv_append_kernel<T, false, kOrdinaryStores>;
+  return neox ? rope_kv_append_kernel<T, true, kInOrder> : rope_kv_append_kernel<T, false, kInOrder>;
 }
 
 hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const void *freq_cis,
@@ -145,9 +155,17 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   const FastDiv div = make_fast_div(list_rows);
   const size_t first = (size_t)k_out_row_offset * k_heads * kRowBytes;
   const RopeOut to = {static_cast<char *>(out_q), static_cast<char *>(out_k) + first, static_cast<char *>(out_v) + first};
+  // An output that does not begin on a 64-byte sector shares the first and the last one of every 128 bytes with the next store, and
+  // past the L2 both halves are a write to memory of their own; up to some MB that is hidden.  Ordinary stores where more than
+  // 11 MiB go to such outputs (us, past the L2 / ordinary, base 16 bytes off: 1200 tokens of 28 + 2 x 4 heads, 11.1 MB, with attention
+  // 25.9 / 26.2, 1400 30.2 / 30.25, 1700 39.1 / 37.7, 4096 136.5 / 133.9, alone 16.45 / 13.2; 256 of 32 + 2 x 32 10.59 / 10.57, 512, 12.6
+  // MB, 16.2 / 15.1, 1019 30.7 / 28.65; 32 off 512 of them 15.5 / 15.1.  64 off: 512 14.3 / 14.8, 2048 of 28 44.8 / 45.5.)
+  auto off_sector = [&](const void *p, long long heads) { return (address(p) & 63) != 0 ? cur_size * heads * kRowBytes : 0; };
+  const long long off = off_sector(out_q, q_heads) + off_sector(to.k, k_heads) + off_sector(to.v, in_v != nullptr ? k_heads : 0);
+  const RopeWay way = placed ? kPlaced : off > kOffSectorBytes ? kOrdinaryStores : kInOrder;
   const long long threads = placed ? (long long)((cur_size + (1 << share) - 1) >> share) * list_rows * 8 : total;
   const int grid = (int)((threads + 255) / 256) * (placed ? 8 : 1);
-  const auto kern = (dt == kDtFloat16) ? kernel_of<_Float16>(is_neox, placed) : kernel_of<__bf16>(is_neox, placed);
+  const auto kern = (dt == kDtFloat16) ? kernel_of<_Float16>(is_neox, way) : kernel_of<__bf16>(is_neox, way);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, addresses_t{address(in_q), address(in_k), address(in_v), address(freq_cis)},
                      u32x4_t{(uint32_t)(placed ? cur_size : total), div.m,
                              div.l | (in_v != nullptr ? 256u : 0u) | (placed ? (uint32_t)share << 9 : 0u), (uint32_t)start_pos},
