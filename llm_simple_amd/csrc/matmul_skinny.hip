@@ -21,6 +21,12 @@
 // 2.97 / 2.82, 2048 x 11008, in several rounds of 8, 11.45 / 10.62).  With more rows the stream is what counts, and four units of
 // two groups are what a CU can have under way (3584 x 3584, two / four / six / eight 7.07 / 6.25 / 6.67 / 6.28).
 //
+// Over a k of more than 12 units there are several passes, and the lhs, which every workgroup reads whole, comes with each: eight
+// units at a time with few rows, four with many (us, eight / four: one row of 1536 x 8960 6.93 / 7.46, 512 x 18944 9.19 / 10.93; 5 rows of
+// 1024 x 8192 6.78 / 6.94; 4 rows of 2048 x 8960 9.67 / 8.83, 6 of 2048 x 13824 14.46 / 13.00, 8 of 1536 x 8960 9.83 / 9.19).  The line is a
+// product of lhs rows and W rows per workgroup, from 280 sizes of 1-8 rows, 512-2048 W rows, k of 6160-18944: 20, or 32 with 14 to 16
+// units (two passes with little left over: 4 rows of 2048 x 7168 7.35 / 7.57, of 2048 x 6160, 13 units, 7.62 / 7.17).
+//
 // EXACT: k is a multiple of 512, so that every wave has the same units, and nothing is asked for or left out under a mask: a
 // mask and a branch to each load were 190 of the 270 instructions before the first MFMA, and a wave issues one in 4-5 cycles (us, with
 // masks and the bias fetched at the end / this: 512 x 3584 3.50 / 3.35, 3584 x 3584 6.03 / 5.90, 1024 x 5120 4.48 / 4.32, 5120 x 5120, two
@@ -159,7 +165,10 @@ template <typename T> SkinnyKernel kernel_of(int m, int k, int rows) {
   }
   if (rows > 8) return matmul_skinny_kernel<T, 2, 2, 4, false>;
   if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4, false>;
-  return units > 8 && units <= 12 ? matmul_skinny_kernel<T, 2, 1, 12, false> : matmul_skinny_kernel<T, 2, 1, 8, false>;
+  if (units <= 8) return matmul_skinny_kernel<T, 2, 1, 8, false>;
+  if (units <= 12) return matmul_skinny_kernel<T, 2, 1, 12, false>;
+  // Several passes: of eight units while a workgroup has few results, a little longer where two passes hold nearly all of k
+  return m * rows <= (units >= 14 && units <= 16 ? 32 : 20) ? matmul_skinny_kernel<T, 2, 1, 8, false> : matmul_skinny_kernel<T, 2, 1, 4, false>;
 }
 
 }  // namespace
