@@ -5,7 +5,7 @@
 // Bound by reading W once.  W is dealt out in equal shares of whole rows (at most 16) to one workgroup per
 // CU, two or more rounds of them for a wide n: a CU cannot have more than its 32 KiB of first-level cache
 // in flight (about 30 GB/s), so a matrix is only read at full speed if every CU has the same share of it --
-// with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it takes 4.2.
+// with 16 rows per workgroup 512 x 3584 ran on 32 CUs in 6.0 us, with 2 rows on all 256 it took 4.2 (3.35 now).
 // The eight waves of a workgroup deal k out among themselves, and the partial sums meet in LDS.
 //
 // mfma_f32_16x16x32 takes 16 rows of 32 k; read that way every load instruction would touch half a
@@ -32,7 +32,8 @@
 // masks and the bias fetched at the end / this: 512 x 3584 3.50 / 3.35, 3584 x 3584 6.03 / 5.90, 1024 x 5120 4.48 / 4.32, 5120 x 5120, two
 // passes of five units, 11.05 / 10.05, 18944 x 3584 23.0 / 21.2, 1536 x 1536 3.13 / 2.99; eight rows 4096 x 4096 8.16 / 7.93).  Not
 // where it takes more passes than two, nor two of more than five units: they end and begin all at once (1024 x 8192, two of eight
-// 5.68 / 5.90; 4096 x 7168, two of seven 10.87 / 11.45; 4096 x 6144, three of four 9.74 / 9.91; 4096 x 10240, four of five 15.2 / 15.9).
+// 5.68 / 5.90; 4096 x 7168, two of seven 10.87 / 11.45; 4096 x 6144, two of six 9.65 / 10.32, 8 rows 11.39 / 11.53, 8192 x 6144 17.0 / 17.4,
+// three of four 9.74 / 9.91; 4096 x 10240, four of five 15.2 / 15.9).  As one pass takes up to eight units, two passes are a k of 5120.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -138,30 +139,20 @@ __global__ __launch_bounds__(64 * kSkinnyWaves, 4) void matmul_skinny_kernel(add
 }
 
 using SkinnyKernel = void (*)(addresses_t, u32x4_t);
-template <typename T, int TW> SkinnyKernel exact_kernel(int units) {
-  constexpr int most = TW == 1 ? 12 : 8;  // (registers)
-  switch (units) {
-    case 1: return matmul_skinny_kernel<T, 2, TW, 1, true>;
-    case 2: return matmul_skinny_kernel<T, 2, TW, 2, true>;
-    case 3: return matmul_skinny_kernel<T, 2, TW, 3, true>;
-    case 4: return matmul_skinny_kernel<T, 2, TW, 4, true>;
-    case 5: return matmul_skinny_kernel<T, 2, TW, 5, true>;
-    case 6: return matmul_skinny_kernel<T, 2, TW, 6, true>;
-    case 7: return matmul_skinny_kernel<T, 2, TW, 7, true>;
-    case 8: return matmul_skinny_kernel<T, 2, TW, 8, true>;
-    case 9: return matmul_skinny_kernel<T, 2, TW, 9 < most ? 9 : most, true>;
-    case 10: return matmul_skinny_kernel<T, 2, TW, 10 < most ? 10 : most, true>;
-    case 11: return matmul_skinny_kernel<T, 2, TW, 11 < most ? 11 : most, true>;
-    default: return matmul_skinny_kernel<T, 2, TW, most, true>;
-  }
+// The EXACT kernel of so many units a pass; none beyond what a wave has registers for.
+template <typename T, int TW, int B = TW == 1 ? 12 : 8> SkinnyKernel exact_kernel(int units) {
+  if (units == B) return matmul_skinny_kernel<T, 2, TW, B, true>;
+  if constexpr (B > 1) return exact_kernel<T, TW, B - 1>(units);
+  return nullptr;
 }
+constexpr int kTwoPassUnits = 5;  // of a pass, where there are two
+
 template <typename T> SkinnyKernel kernel_of(int m, int k, int rows) {
   if (m > 8) return matmul_skinny_kernel<T, 1, 1, 8, false>;
   const int round = 64 * kSkinnyWaves, units = (k + round - 1) / round;  // of a wave
-  if (k % round == 0 && rows <= 8 && units <= 12) return exact_kernel<T, 1>(units);
-  if (k % round == 0 && rows > 8) {
-    if (units <= 8) return exact_kernel<T, 2>(units);
-    if (units == 10) return exact_kernel<T, 2>(5);  // two passes; more of them are not faster
+  if (k % round == 0) {
+    if (const SkinnyKernel one = rows <= 8 ? exact_kernel<T, 1>(units) : exact_kernel<T, 2>(units)) return one;
+    if (rows > 8 && units % 2 == 0 && units / 2 <= kTwoPassUnits) return exact_kernel<T, 2>(units / 2);
   }
   if (rows > 8) return matmul_skinny_kernel<T, 2, 2, 4, false>;
   if (units <= 4) return matmul_skinny_kernel<T, 2, 1, 4, false>;
