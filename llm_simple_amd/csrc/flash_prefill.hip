@@ -965,22 +965,17 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   constexpr int NT = 64 * NW;
   const int T_ = ((p.pack ? p.m * p.g : p.m) + BM - 1) / BM;
   int grid, list_heads;
-  const int S_ = p.num_splits;
+  const int S_ = p.num_splits, share = prefill_xcd_share_log2(p.Hkv);
   p.xcd_bits = p.sched_shift = 0;
   if (p.pack) {
     list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
-  } else if (p.Hkv <= 8 && 8 % p.Hkv == 0) {
+  } else if (share >= 0) {
     p.xcd_bits = 3;
-    const int xcds = 8 / p.Hkv;  // per kv head
-    while ((1 << p.sched_shift) < xcds) ++p.sched_shift;
-    list_heads = p.g;
-    const int per_kvh = p.g * T_ * S_;
-    grid = 8 * ((per_kvh + xcds - 1) / xcds);
-  } else if (p.Hkv % 8 == 0) {
-    p.xcd_bits = 3;
-    list_heads = (p.Hkv / 8) * p.g;
-    grid = 8 * list_heads * T_ * S_;
+    p.sched_shift = share;
+    list_heads = p.H >> (3 - share);
+    const int xcds = 1 << share;  // per list
+    grid = 8 * ((list_heads * T_ * S_ + xcds - 1) / xcds);
   } else {
     list_heads = p.H;
     grid = T_ * p.H * S_;
@@ -1170,7 +1165,7 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
 // The last answers are kept per thread: every layer of a model asks for the same chunk (several hundred combinations).
 static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cus, size_t max_bytes) {
   const long long n_vis = ((long long)m + offset < n) ? (long long)m + offset : n;  // keys the last row sees
-  if (n_vis < 2LL * m) return {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
+  if (prefill_is_prompt(m, n_vis)) return {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
   struct Memo {
     int m, n, offset, g, Hkv, cus;
     size_t bytes, max_bytes;  // what the plan takes, what it was allowed

@@ -26,6 +26,15 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
                                 hipStream_t stream, void *workspace, size_t workspace_bytes);
 #endif
 
+// What the launch of a prompt does and the rope launch before it counts on.  A call is a prompt if no more tokens are cached than
+// new.  Workgroup b runs on XCD b % 8; the query heads of a kv head are dealt to one XCD (of several kv heads each), or to 2^share_log2 of
+// them, as long as kv heads and XCDs divide; else (share_log2 < 0) workgroups are not dealt at all.
+inline bool prefill_is_prompt(long long new_tokens, long long visible_keys) { return visible_keys < 2 * new_tokens; }
+inline int prefill_xcd_share_log2(int kv_head_num) {
+  if (kv_head_num % 8 == 0) return 0;
+  return kv_head_num == 4 ? 1 : kv_head_num == 2 ? 2 : kv_head_num == 1 ? 3 : -1;
+}
+
 // Compute units of the current device, cached per device; 256 when no device can be asked.
 int device_compute_units();
 

@@ -77,10 +77,10 @@ __device__ __forceinline__ void rotate8(u32x4_t &va, u32x4_t &vb, const f32x4_t 
 
 enum RopeWay { kInOrder, kPlaced, kOrdinaryStores };  // (in order too)
 
-// kPlaced: workgroup b works for XCD b % 8, on rows that the attention launch to come reads there (prefill_schedule in
-// flash_prefill.hip): the heads of that XCD's kv heads, or, where two XCDs share one, those of every second token.
-// What these stores leave in an XCD's L2 is valid and clean, and Q, K and V are then read from there.  Which rows go where
-// is nothing but speed.
+// kPlaced: workgroup b works for XCD b % 8, on rows that the attention launch to come reads there (prefill_xcd_share_log2): the
+// heads of that XCD's kv heads, or, where two XCDs share one, those of every second token.  What these stores leave in an XCD's L2 is
+// valid and clean, and Q, K and V are then read from there; where two XCDs share a kv head, half of what each reads (attention deals
+// tiles and heads to the two, and either reads every K and V row).  Which rows go where is nothing but speed.
 template <typename T, bool NEOX, RopeWay WAY>
 __global__ __launch_bounds__(256) void rope_kv_append_kernel(addresses_t in_, u32x4_t size, u32x2_t heads_, RopeOut to) {
   // in_: q, k, v, the table; size: tokens (kPlaced) or threads, factor and shift of the division by a token's rows in a list (bit 8:
@@ -147,10 +147,9 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   // the L2s beside what is read.  Rope and attention, us, in order / placed: 128 tokens of 32 kv heads 8.27 / 7.07, 256 9.50 / 9.11,
   // 300 10.42 / 10.42, 512 13.66 / 13.87; 200 of 8 (40 heads) 8.53 / 8.01, 400 11.46 / 11.04, 600 14.07 / 14.17; 200 of 4 (28) 8.01 / 7.84,
   // 512 11.56 / 11.23, 700 14.01 / 14.02, 1019 18.12 / 18.21; 20 of 4 6.21 / 6.32.  Four XCDs to a kv head: nothing (256 of 2 7.73 / 7.79).
-  int share = -1;  // logarithm of the XCDs of a list
-  if (cur_size >= kPlacedTokens && start_pos < cur_size && total * 32 <= kPlacedBytes && k_heads > 0 && q_heads % k_heads == 0)
-    share = k_heads % 8 == 0 ? 0 : k_heads == 4 ? 1 : -1;
-  const bool placed = share >= 0;
+  const int share = k_heads > 0 ? prefill_xcd_share_log2(k_heads) : -1;  // logarithm of the XCDs of a list
+  const bool placed = cur_size >= kPlacedTokens && prefill_is_prompt(cur_size, (long long)start_pos + cur_size) &&
+                      total * 32 <= kPlacedBytes && (share == 0 || share == 1) && q_heads % k_heads == 0;
   const uint32_t list_rows = (uint32_t)(placed ? rows >> (3 - share) : rows);
   const FastDiv div = make_fast_div(list_rows);
   const size_t first = (size_t)k_out_row_offset * k_heads * kRowBytes;
