@@ -64,7 +64,8 @@ constexpr float kLazyLog2 = 8.0f;                // rescale threshold, log2 unit
 constexpr int kMaxPrefillSplits = 128;           // key ranges per call
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
-// What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way.
+// What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way -- except with SPLIT, where
+// the key range (per_split, num_splits, chunk) is needed for the first address and waited for.
 struct PrefillLate {
   char *out;
   // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers
@@ -93,8 +94,8 @@ struct PrefillParams : PrefillLate {
   // its kv head once for all g query heads.
   int pack;
 };
-// What the index arithmetic and the first loads of a workgroup need, packed into the first 14 words of a kernel's arguments, which
-// are in registers when it starts.  With kernels of their own for key ranges, whose packed rows and partials a prompt need not step
+// What the index arithmetic and the first loads of a workgroup need (of an unsplit one: see PrefillLate), packed into the first 14
+// words of a kernel's arguments, which are in registers when it starts.  With kernels of their own for key ranges, whose packed rows and partials a prompt need not step
 // over (both together, attention alone, us: 32 tokens of 32 heads 4.65 -> 4.21, 256 5.85 -> 5.50, 512 of 28 8.44 -> 7.94, 1019 14.4 ->
 // 14.05, 2048 35.6 -> 34.8, 4096 113.5 -> 112.8; 200 past 16001 53.1 -> 51.75, 100 past 8000 of 40 25.2 -> 24.1).  It counts
 // instructions: one wave issues one in 4-5 cycles, so the lists' forms are one formula, divisions have no branch, tiles are counted by
@@ -423,7 +424,10 @@ template <typename T, int KB = 2> struct WaveAttn {
   // than the banks, and up to 8 lanes meet in one, 1-2 % of a launch's cycles) and leaves as whole pieces of
   // 64*ND bytes, 4*ND lanes per row, past the L2: lines that are left there are written back at the end of the launch (rope
   // and attention, us, ordinary stores / these: 256 tokens of 28 heads 9.39 / 9.20, 600 14.64 / 14.16, 1019 20.5 / 19.7, of
-  // 32 26.3 / 25.7, 2048 of 28 44.5 / 43.8; up to 128 tokens and from 4096 on the same).  lds_wave: this wave's region; out_blk: &out[first row of the
+  // 32 26.3 / 25.7, 2048 of 28 44.5 / 43.8; up to 128 tokens and from 4096 on the same).  So too with ND = 1, pieces of 64 bytes from
+  // two waves to a line: a sector is enough (attention alone, us: 256 of 32 5.44 / 5.29, 512 of 28 7.98 / 7.78, 2000 of 12 22.7 / 22.4), and
+  // where the output begins off a sector (16 bytes off: 512 of 28 8.80 / 8.60, 1019 18.0 / 17.4, of 32 19.8 / 19.6, 2048 of 28 41.7 / 41.7, 4096
+  // 125.4 / 125.2).  lds_wave: this wave's region; out_blk: &out[first row of the
   // wave][head]; rows_valid: how many of the wave's 32 rows exist.
   template <int D0 = 0, int ND = 4>
   __device__ __forceinline__ void store(char *lds_wave, char *out_blk, size_t row_bytes, int rows_valid) {
@@ -1051,7 +1055,8 @@ int device_compute_units() {
 // tile `step_free` on an otherwise empty chip and `step_full` with every CU busy, up to `past_l2` times that once K and V
 // outgrow the L2s of the 8 XCDs together (32 to 48 MiB; 32 heads, kQuad64: 1.13 us a step at 2450 keys, 1.6 at 2900).  Fitted
 // over 13000 timed launches (204 shapes of 2-32 kv heads, 3-8192 tokens, 0-31000 cached keys, every shape and
-// split), and again over 180000 (1800 shapes of 1-32 kv heads, 2-3000 tokens, 200-131072 cached keys).
+// split), and again over 180000 (1800 shapes of 1-32 kv heads, 2-3000 tokens, 200-131072 cached keys).  Kernels have become faster since,
+// 0.4-0.5 us of `fixed` and part of a step, and the figures were not fitted again: what that costs stands at the two rules below.
 enum PrefillKind { kPair64, kPair128, kRows128, kRows256, kQuad64, kQuad32, kPrefillKinds };
 struct PrefillShape {
   int rows, tile, per_cu;  // query rows, keys of a tile, workgroups resident on a CU
@@ -1093,6 +1098,8 @@ static size_t partial_bytes(long long splits, int m, long long H) {
 //   two waves per 128 rows up to 2 per CU: 1700 tokens 34.0 / 35.3 (28)
 //   256 rows from more than 1.5 workgroups per CU on: 3500 tokens 107.8 / 111 (28); 128 rows of one wave each up to there:
 //     3000 tokens 81.7 / 85.8, 80.2 / 82.6 (32), 8192 tokens 188 / 202 (12)
+// With the kernels of today the choice is 0.6 % slower than the fastest of the six shapes on average over 60 prompts of 24-4096
+// tokens and 1-32 kv heads, 2.8 % at the 90th percentile, 11 % at most (1439 of 12 heads, two kv heads, 17.0 / 15.3, four waves per 64 rows).
 static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
   auto per_cu = [&](int rows) { return (double)((m + rows - 1) / rows) * H / cus; };
   if (n_vis > 96 && per_cu(32) <= 1.05) return kQuad32;
@@ -1106,8 +1113,10 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 // tile has the g query heads of a kv head share a tile (K and V of the kv head are then read once, not g times).
 // Taken is the combination of shape, packing and cut that the costs above make cheapest: workgroups in rounds of as
 // many as are resident at once, 2.65 us and the traffic of the partials for the combine launch.  Only combinations whose
-// partials fit max_bytes are looked at; an unsplit one always does.  Over the 1800 measured shapes the choice is 1.1 %
-// slower than the fastest combination on average, 4 % at the 90th percentile.  Among combinations within 4 % of the
+// partials fit max_bytes are looked at; an unsplit one always does.  Over the 1800 measured shapes the choice was 1.1 %
+// slower than the fastest combination on average, 4 % at the 90th percentile; with the kernels of today, over 110 shapes of 2-512
+// tokens behind 260-29600 keys, 1.9 % and 5.4 %, 22 % at most (19 tokens behind 22155 keys of 20 + 4 heads 20.6 / 16.9 us, 121 behind 1350 of
+// 28 + 4 13.3 / 11.7).  Among combinations within 4 % of the
 // cheapest one that reads K and V once and gives every CU the same number of workgroups is preferred.
 // Rows that fit one 256-row tile over a cache larger than the last-level cache are a stream from HBM: that tile's loads are
 // non-temporal then, and nothing else was faster (us, it / the best other one: 23 tokens over 68925 keys of 4 kv heads 49.6

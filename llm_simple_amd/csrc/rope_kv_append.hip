@@ -22,9 +22,9 @@
 // parameter, the storage type is rounded by the hardware conversion (equal to round-to-nearest-even on the bit pattern for
 // every non-NaN fp32), the token of a row comes from a multiply-shift division.
 //
-// Bound by the memory path of three separate streams of 256-byte rows.  4096 tokens of 28 + 2 x 4 heads (75.5 MB): 11.9 us
-// with the buffers in the last-level cache, 15.2 from and to HBM, where a plain device copy of the same bytes takes
-// 10.4 and 16; 256 tokens of 32 + 2 x 32 heads 2.85 us, of which an empty launch is 1.55.  One piece to a thread: two, a
+// Bound by the memory path of three separate streams of 256-byte rows.  4096 tokens of 28 + 2 x 4 heads (75.5 MB): 11.7 us
+// with the buffers in the last-level cache, 14.4 from and to HBM, where a plain device copy of the same bytes takes
+// 10.2-11.7 and 16-16.6; 256 tokens of 32 + 2 x 32 heads 2.85 us, of which an empty launch is 1.55.  One piece to a thread: two, a
 // grid apart, kept half as many waves (a layer's rope and attention, us, two / one: 64 tokens of 32 heads 8.29 / 8.02,
 // 256 10.80 / 10.52, 1500 41.9 / 40.9, 256 of 12 9.03 / 8.61).
 #include "common.hpp"
@@ -144,9 +144,9 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   if (total == 0) return hipSuccess;
   if (rows > 0x7FFFFFFFLL || total > 0x7FFFFFFFLL) return hipErrorInvalidValue;  // 32-bit thread index
   // Rows placed: a prompt (a chunk's workgroups are dealt otherwise) of kv heads that make whole lists, where what is written fits
-  // the L2s beside what is read.  Rope and attention, us, in order / placed: 128 tokens of 32 kv heads 8.27 / 7.07, 256 9.50 / 9.11,
-  // 300 10.42 / 10.42, 512 13.66 / 13.87; 200 of 8 (40 heads) 8.53 / 8.01, 400 11.46 / 11.04, 600 14.07 / 14.17; 200 of 4 (28) 8.01 / 7.84,
-  // 512 11.56 / 11.23, 700 14.01 / 14.02, 1019 18.12 / 18.21; 20 of 4 6.21 / 6.32.  Four XCDs to a kv head: nothing (256 of 2 7.73 / 7.79).
+  // the L2s beside what is read.  Rope and attention, us, in order / placed: 128 tokens of 32 kv heads 8.19 / 7.15, 256 9.47 / 9.10,
+  // 300 10.42 / 10.42, 512 13.66 / 13.87; 200 of 8 (40 heads) 8.52 / 8.05, 400 11.28 / 11.04, 600 14.07 / 14.17; 200 of 4 (28) 8.00 / 7.76,
+  // 512 11.59 / 11.21, 700 14.01 / 14.06, 1019 18.12 / 18.21; 20 of 4 6.21 / 6.32.  Four XCDs to a kv head: nothing (256 of 2 7.73 / 7.79).
   const int share = k_heads > 0 ? prefill_xcd_share_log2(k_heads) : -1;  // logarithm of the XCDs of a list
   const bool placed = cur_size >= kPlacedTokens && prefill_is_prompt(cur_size, (long long)start_pos + cur_size) &&
                       total * 32 <= kPlacedBytes && (share == 0 || share == 1) && q_heads % k_heads == 0;
