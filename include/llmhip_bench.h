@@ -26,6 +26,18 @@ int llmhip_bench_flash_attn_gqa_clocked(void *out, const void *q, const void *k,
                                         int n, int offset, int group_size, int kv_head_num, int head_dim,
                                         int dt, void *clock_probe, void *stream);
 
+/* llmhip_flash_decode_gqa and llmhip_decode_step_gqa (llmhip.h) on this library's own copy of the decode kernel, in which the
+ * workgroups that fold partials do not wait for them: each computes its rows from the caches by itself, as the product's do
+ * when they have looked for partials in vain for some 50 ms.  num_splits >= 1 and a workspace of
+ * llmhip_flash_decode_workspace_bytes in both. */
+int llmhip_bench_flash_decode_gqa_alone(void *out, const void *q, const void *k_cache, const void *v_cache, void *workspace,
+                                        size_t workspace_bytes, int batch, int n, int64_t kv_seq_stride, int group_size,
+                                        int kv_head_num, int head_dim, int num_splits, int dt, void *stream);
+int llmhip_bench_decode_step_gqa_alone(void *out, void *k_cache, void *v_cache, const void *freq_cis, const void *in_q,
+                                       const void *in_k, const void *in_v, void *workspace, size_t workspace_bytes, int pos,
+                                       int group_size, int kv_head_num, int head_dim, int is_neox_style, int num_splits, int dt,
+                                       void *stream);
+
 /* Runs, for about target_ms (<= 2000), a loop of back-to-back bf16 32x32x16 MFMAs on N(0,1)
  * operands on every CU and returns the sustained TFLOP/s.  mix 0: the MFMAs alone (what the matrix
  * pipe sustains at the clock its own power draw allows); mix 1: the same MFMAs with the LDS

@@ -12,6 +12,8 @@ LIB_PATH = os.path.join(_HERE, "libllmhip_bench.so")
 _vp, _i, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
 SYMBOLS = {
     "llmhip_bench_flash_attn_gqa_clocked": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp]),
+    "llmhip_bench_flash_decode_gqa_alone": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, ctypes.c_int64, _i, _i, _i, _i, _i, _vp]),
+    "llmhip_bench_decode_step_gqa_alone": (_i, [_vp] * 8 + [_sz, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_mfma_ceiling": (_i, [_i, ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
     "llmhip_bench_stream_read": (_i, [_vp, _vp, _sz, _vp, _sz, _i, _vp]),
 }
@@ -45,6 +47,25 @@ def hip_flash_attn_gqa_clocked_layer(output_dev, q_dev, k_dev, v_dev, m, n, offs
     _check(lib.llmhip_bench_flash_attn_gqa_clocked(p(output_dev), p(q_dev), p(k_dev), p(v_dev), m, n, offset,
                                                    group_size, kv_head_num, head_dim, dt, p(clock_probe_dev),
                                                    stream), "hip_flash_attn_gqa_clocked_layer")
+
+
+def hip_flash_decode_gqa_alone_layer(output_dev, q_dev, k_dev, v_dev, ws_dev, ws_bytes, batch, n, kv_seq_stride, group_size,
+                                     kv_head_num, head_dim, num_splits, dt, stream=0):
+    """hip_flash_decode_gqa_layer on the measurement library's copy of the decode kernel, whose folding workgroups compute
+    their rows by themselves."""
+    p = ops._ptr
+    _check(lib.llmhip_bench_flash_decode_gqa_alone(p(output_dev), p(q_dev), p(k_dev), p(v_dev), p(ws_dev), ws_bytes, batch, n,
+                                                   kv_seq_stride, group_size, kv_head_num, head_dim, num_splits, dt, stream),
+           "hip_flash_decode_gqa_alone_layer")
+
+
+def hip_decode_step_gqa_alone_layer(output_dev, k_dev, v_dev, freq_cis_dev, q_dev, new_k_dev, new_v_dev, ws_dev, ws_bytes, pos,
+                                    group_size, kv_head_num, head_dim, is_neox_style, num_splits, dt, stream=0):
+    """hip_decode_step_gqa_layer likewise, with a split count and a workspace of the caller's."""
+    p = ops._ptr
+    _check(lib.llmhip_bench_decode_step_gqa_alone(p(output_dev), p(k_dev), p(v_dev), p(freq_cis_dev), p(q_dev), p(new_k_dev),
+                                                  p(new_v_dev), p(ws_dev), ws_bytes, pos, group_size, kv_head_num, head_dim,
+                                                  is_neox_style, num_splits, dt, stream), "hip_decode_step_gqa_alone_layer")
 
 
 def probe_mfma_ceiling(mix, target_ms=60.0):

@@ -38,6 +38,40 @@ int llmhip_bench_flash_attn_gqa_clocked(void *out, const void *q, const void *k,
                                        static_cast<hipStream_t>(stream), clock_probe));
 }
 
+int llmhip_bench_flash_decode_gqa_alone(void *out, const void *q, const void *k_cache, const void *v_cache, void *workspace,
+                                        size_t workspace_bytes, int batch, int n, int64_t kv_seq_stride, int group_size,
+                                        int kv_head_num, int head_dim, int num_splits, int dt, void *stream) {
+  if (!out || !q || !k_cache || !v_cache || !workspace || !aligned16(out) || !aligned16(q) || !aligned16(k_cache) ||
+      !aligned16(v_cache) || !aligned16(workspace))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (batch < 1 || n < 1 || group_size < 1 || kv_head_num < 1 || kv_seq_stride < n || num_splits < 1 ||
+      (dt != LLMHIP_DT_FLOAT16 && dt != LLMHIP_DT_BFLOAT16))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (head_dim != 128 || group_size > 16 || batch > 65535 || kv_head_num > 65535 || num_splits > 256) return LLMHIP_ERR_UNSUPPORTED;
+  if (flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits) > workspace_bytes) return LLMHIP_ERR_WORKSPACE;
+  if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
+  return from_hip(launch_flash_decode(out, q, k_cache, v_cache, workspace, workspace_bytes, batch, 1, n, n - 1, kv_seq_stride,
+                                      group_size, kv_head_num, num_splits, dt, static_cast<hipStream_t>(stream)));
+}
+
+int llmhip_bench_decode_step_gqa_alone(void *out, void *k_cache, void *v_cache, const void *freq_cis, const void *in_q,
+                                       const void *in_k, const void *in_v, void *workspace, size_t workspace_bytes, int pos,
+                                       int group_size, int kv_head_num, int head_dim, int is_neox_style, int num_splits, int dt,
+                                       void *stream) {
+  if (!out || !k_cache || !v_cache || !freq_cis || !in_q || !in_k || !in_v || !workspace || !aligned16(out) || !aligned16(k_cache) ||
+      !aligned16(v_cache) || !aligned16(freq_cis) || !aligned16(in_q) || !aligned16(in_k) || !aligned16(in_v) || !aligned16(workspace))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (pos < 0 || pos == INT32_MAX || group_size < 1 || kv_head_num < 1 || num_splits < 1 ||
+      (dt != LLMHIP_DT_FLOAT16 && dt != LLMHIP_DT_BFLOAT16))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (head_dim != 128 || group_size > 16 || kv_head_num > 65535 || num_splits > 256) return LLMHIP_ERR_UNSUPPORTED;
+  if (flash_decode_workspace_bytes(1, 1, group_size, kv_head_num, num_splits) > workspace_bytes) return LLMHIP_ERR_WORKSPACE;
+  if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
+  return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, workspace, workspace_bytes, pos,
+                                           group_size, kv_head_num, is_neox_style, num_splits, dt,
+                                           static_cast<hipStream_t>(stream)));
+}
+
 int llmhip_bench_mfma_ceiling(int mix, double target_ms, double *tflops) {
   if (!tflops || (mix != 0 && mix != 1) || target_ms < 0.0 || target_ms > 2000.0) return LLMHIP_ERR_INVALID_ARG;
   if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;

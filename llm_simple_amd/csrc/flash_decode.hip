@@ -25,14 +25,19 @@
 // waves are merged through LDS at the end and the workgroup writes the final rows (one split) or an
 // fp32 partial (max, sum, unnormalised O).
 //
-// Up to 16 partials of a (sequence, kv head) are folded (log-sum-exp) by the workgroup that finds them all stored, with no
-// fence and no atomic.  Up to 8: every word goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it,
-// and whoever finds the number at all of them folds them; that is two memory round trips.  More, or where the number would be
-// that of a replay: partials, then a flag, then a look at the other flags, then the partials, four round trips.  (The fused step,
-// us, flags / tags, cache lines warm: 384 keys of 2 kv heads 6.6 / 5.9, 512 of 32 6.2 / 5.55, 1000 of 8 6.8 / 6.4, 1500 of 32
-// 8.9 / 8.1; the combine launch takes 3.1 us, and 2.4 of the host's.)  More partials make more rounds of loads in ONE workgroup (32:
-// 11.2 against 8.8 us at batch 1, 4096 keys) and keep the second launch.  (Device-scope fences instead of sc1 accesses
-// write back and invalidate the XCD's L2: 91 us against 33 at batch 1, 32768 keys.)
+// Up to 32 partials of a (sequence, kv head) are folded (log-sum-exp) by workgroups of the same launch that do nothing else
+// (folders): every word of a partial goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it, and a folder
+// looks at all of them until it finds the number everywhere.  That is one way to memory and one back; no fence, no flag, no atomic.
+// Folders have the highest workgroup numbers, so that they are dispatched after the workgroups that they wait for, and on
+// idle CUs if there are any; a folder that has looked in vain for some 50 ms computes its rows from the caches by itself, so that nothing
+// depends on the order of dispatch.  A look costs what its loads cost: a wave per row, two dims per lane, the maxima and
+// sums of all partials in one load (two rows per wave with three loads per partial: 1.5 us a look, 0.6 now).
+// (Fused step, us, the last workgroup to store folds / folders: 384 keys of 2 kv heads 5.52 / 4.85, 512 of 32 5.23 / 5.01, 32768 of 8, with
+// a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1.)
+// Where the number would be that of a replay, up to 16 partials are folded by the workgroup that finds them all stored: partials,
+// then a flag, then a look at the other flags, then the partials, four round trips to memory.  Beyond that, for more than 8 rows or
+// 32 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
+// against 33 at batch 1, 32768 keys.)
 //
 // A short cache is bound by the length of one workgroup's chain, not by bytes: at 32 keys, one sequence, the
 // kernel took 6.3 us, 2.5 us of them the launch.  A wave issues a vector instruction every 4-5 cycles, so the
@@ -41,8 +46,7 @@
 // instruction, K and V rows are read through buffer descriptors (the hardware bounds them, no clamps), integer
 // divisions are prepared by the host, the column maximum goes through permlane swaps, masks and the
 // rescaling of O run only where they change something, and the merge of the waves is free of bank conflicts (it cost
-// 1.4 us).  4.1 us now; 384 keys of 2 kv heads 9.7 -> 6.6 us, 512 keys of 32 kv heads 9.1 -> 6.2, 4096 keys of 8
-// 10.9 -> 9.2, 32768 keys of 8 28.4 -> 24.8 (fused step, back-to-back calls, by flags).
+// 1.4 us).  4.1 us now.
 //
 // (Eight-wave workgroups, half as many, merging pairs of splits through LDS: 4.5 TB/s against 6.0 at the time.)
 #include <atomic>
@@ -54,7 +58,7 @@
 #include "kernels.hpp"
 #include "launch_number.hpp"
 
-namespace llmhip {
+namespace LLMHIP_NS {
 
 constexpr int kDecWaveKeys = 32;                  // keys per wave per step
 constexpr int kDecStepKeys = 4 * kDecWaveKeys;    // keys per workgroup per step (half of it in short caches)
@@ -75,7 +79,9 @@ struct DecodeLate {
   FastDiv g_div;
   float scale_log2e;
   int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
-  uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial (see FoldMode)
+  int fold_rows, folders;  // by tags: rows of a folder, folders of a (sequence, kv head)
+  FastDiv folders_div;
+  uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial
 };
 // rows = m * g query rows of a kv head, at most 16.  Fused decode step (FUSED kernels only): the token at row n - 1 is not in the
 // cache yet.  q, new_k and new_v hold the unrotated projections of that token ([H][128], [Hkv][128] twice);
@@ -90,7 +96,8 @@ struct DecodeParams : DecodeLate {
   int is_neox;
   bool fused;
 };
-// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8, 2^16 / g + 1, offset; c: n, Hkv | g << 16 | is_neox << 31
+// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
+// up) << 10 (pairs = batch * Hkv, where the partials are folded by tags: at most kTaggedPairs); c: n, Hkv | g << 16 | is_neox << 31
 struct DecodeEarly {
   addresses_t a;
   u32x4_t b;
@@ -99,7 +106,8 @@ struct DecodeEarly {
     a = addresses_t{address(p.q), address(p.k), address(p.v), p.fused ? address(p.freq_row) : (uint64_t)p.kv_seq_stride};
     const uint64_t nk = address(p.new_k), nv = address(p.new_v);
     b = p.fused ? u32x4_t{(uint32_t)nk, (uint32_t)(nk >> 32), (uint32_t)nv, (uint32_t)(nv >> 32)}
-                : u32x4_t{(uint32_t)(p.rows | p.m << 8), 65536u / p.g + 1, (uint32_t)p.offset, 0u};
+                : u32x4_t{(uint32_t)(p.rows | p.m << 8), 65536u / p.g + 1, (uint32_t)p.offset,
+                          (uint32_t)(p.batch * p.Hkv) | ((1u << 20) + p.Hkv - 1) / p.Hkv << 10};
     c = u32x2_t{(uint32_t)p.n, (uint32_t)p.Hkv | (uint32_t)p.g << 16 | (uint32_t)p.is_neox << 31};
   }
 };
@@ -169,11 +177,19 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
   return row * kRowBytes + ((((granule >> 1) ^ (row & 7)) << 5) | ((granule & 1) << 4));
 }
 
-constexpr int kMaxFoldSplits = 16;
+constexpr int kMaxFoldSplits = 16, kMaxTaggedSplits = 32;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
 constexpr int kTaggedRows = 8;                    // query rows whose words carry a tag, at most
-constexpr size_t kTaggedReads = 7u << 20;         // bytes that the workgroups of a launch read to look for tags, at most
+constexpr int kTaggedPairs = 1023;                // (sequence, kv head) pairs, at most
 constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
+#ifdef LLMHIP_BENCH
+constexpr int kFoldPolls = 0;  // (the measurement library's copy: every folder computes its rows by itself)
+#else
+constexpr int kFoldPolls = 1 << 16;  // looks that a folder takes, 0.6 us each
+#endif
+// Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  (The order of the
+// combine launch where they are more than kMaxFoldSplits.)
+__host__ __device__ constexpr int fold_parts(int splits) { return splits <= kFoldDepth ? 1 : splits <= kMaxFoldSplits ? 2 : 8; }
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
 
@@ -198,12 +214,196 @@ __device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int by
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
 }
 
-// How the partials of a (sequence, kv head) become rows: not here (one split, or the combine launch), by flags, by tags.  A
-// kernel each: the code of the others in the way costs a call of 4 us 0.05.
+// A row from its partials: four dims of it in each thread of a group of 32, the partials dealt to `parts` groups.
+struct RowFold {
+  float M = -INFINITY, L = 0.0f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  // partials part, part + parts, ... of S
+  template <int D>
+  __device__ __forceinline__ void take(const u32x2_t (&ml)[D], const f32x4_t (&ov)[D], int part, int parts, int S) {
+#pragma unroll
+    for (int j = 0; j < D; ++j)
+      if (part + parts * j < S) M = fmaxf(M, bits_float(ml[j][0]));
+    const float M_use = (M == -INFINITY) ? 0.0f : M;
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      const float wt = (part + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
+      L += wt * bits_float(ml[j][1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
+    }
+  }
+  // Part i of a row is in group i * at_once + row; the sum ends up in part 0.  Room: 2 + 128 floats per group, from a
+  // multiple of 16 bytes on.  Every thread of the workgroup calls.
+  template <int GROUPS> __device__ __forceinline__ void merge(float *room, int parts, int at_once) {
+    const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
+    float *red_o = room + 2 * GROUPS;
+    if (d4 == 0) *reinterpret_cast<float2 *>(room + 2 * sg) = float2{M, L};
+    *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
+    __syncthreads();
+    if (sg < at_once) {
+      M = -INFINITY;
+      for (int i = sg; i < parts * at_once; i += at_once) M = fmaxf(M, room[2 * i]);
+      const float M_use = (M == -INFINITY) ? 0.0f : M;
+      L = 0.0f;
+      acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int i = sg; i < parts * at_once; i += at_once) {
+        const float wt = fast_exp2(room[2 * i] - M_use);  // 0 for a group without splits (-inf)
+        L += wt * room[2 * i + 1];
+        const f32x4_t o = *reinterpret_cast<const f32x4_t *>(red_o + i * kHeadDim + 4 * d4);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) acc[d] += wt * o[d];
+      }
+    }
+    __syncthreads();
+  }
+  template <typename T>
+  __device__ __forceinline__ void store(char *out, int b, int m, int c, int kvh, int Hkv, int g, const FastDiv &g_div, int d4) {
+    const int r = (int)fast_div(c, g_div);
+    const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
+    u32x2_t w;
+    w[0] = Elem<T>::pack2(acc[0] * inv, acc[1] * inv);
+    w[1] = Elem<T>::pack2(acc[2] * inv, acc[3] * inv);
+    *reinterpret_cast<u32x2_t *>(out + (((size_t)b * m + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
+  }
+};
+
+// Maximum over each N = 4 or 8 lanes.
+template <int N> __device__ __forceinline__ float max_of_lanes(float x) {
+  auto with = [&](auto control) {
+    const int i = __builtin_bit_cast(int, x);
+    x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, decltype(control)::value, 0xf, 0xf, false)));
+  };
+  with(std::integral_constant<int, 0xB1>());                     // quad_perm: lane ^ 1
+  with(std::integral_constant<int, 0x4E>());                     // quad_perm: lane ^ 2
+  if (N == 8) with(std::integral_constant<int, 0x141>());        // row_half_mirror: the other quad
+  return x;
+}
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return bits_float(__builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+
+// A folder: rows c0 .. c0 + fold_rows - 1 of a pair, from partials whose words carry this launch's tags.  A wave has a row, two
+// dims per lane, and PARTS of the fold_parts() parts of its partials, DEPTH in all.  It looks at all of them until it finds the tags
+// at every word.  False if they were not there after kFoldPolls looks.
+template <typename T, int NW, int DEPTH, int PARTS>
+__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int b, int kvh, int c0, int rows, int m, int Hkv,
+                                            int g) {
+  constexpr int EACH = DEPTH / PARTS;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
+  const int parts = fold_parts(S), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
+  const bool mine = wave % at_once < p.fold_rows && c < rows;  // (of the wave)
+  const int bytes = S * rows * kTaggedBytes;
+  const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + (size_t)pair * bytes, bytes);
+  const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
+  float M[PARTS], L[PARTS], x[PARTS], y[PARTS];
+  bool there = true;
+#pragma unroll
+  for (int i = 0; i < PARTS; ++i) {
+    M[i] = -INFINITY;
+    L[i] = x[i] = y[i] = 0.0f;
+  }
+  if (mine) {
+    // (no branches: past the splits the offset is past the buffer, and the load is not made)
+    auto split_of = [&](int j) { return part + per_row * (j / EACH) + parts * (j % EACH); };
+    int at[DEPTH];
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) at[j] = split_of(j) < S ? (split_of(j) * rows + c) * kTaggedBytes + lane * 16 : 0x40000000;
+    const int my_split = split_of(lane & (DEPTH - 1));
+    const bool have = my_split < S;
+    const int at_ml = have ? (my_split * rows + c) * kTaggedBytes + kHeadDim * 8 : 0x40000000;
+    u32x4_t a[DEPTH] = {}, ml = {};
+    there = false;
+    for (int looks = 0; looks < kFoldPolls; ++looks) {
+      asm volatile("" ::: "memory");  // (the loads are made again)
+      ml = __builtin_bit_cast(u32x4_t, load_device(pt, at_ml));
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) a[j] = __builtin_bit_cast(u32x4_t, load_device(pt, at[j]));
+      uint32_t differs = have ? (ml[1] ^ tag0) | (ml[3] ^ tag1) : 0u;
+#pragma unroll
+      for (int j = 0; j < DEPTH; ++j) differs |= split_of(j) < S ? (a[j][1] ^ tag0) | (a[j][3] ^ tag1) : 0u;
+      there = __builtin_amdgcn_ballot_w64(differs != 0) == 0;
+      if (there) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    const float my_m = have ? bits_float(ml[0]) : -INFINITY, M_lanes = max_of_lanes<EACH>(my_m);
+    const float wt = have ? fast_exp2(my_m - (M_lanes == -INFINITY ? 0.0f : M_lanes)) : 0.0f, my_l = have ? bits_float(ml[2]) : 0.0f;
+#pragma unroll
+    for (int j = 0; j < DEPTH; ++j) {
+      const int i = j / EACH;
+      const float w = lane_value(wt, j);
+      if (j % EACH == 0) M[i] = lane_value(M_lanes, j);
+      L[i] += w * lane_value(my_l, j);
+      x[i] += w * bits_float(a[j][0]);
+      y[i] += w * bits_float(a[j][2]);
+    }
+  }
+  int *failed = reinterpret_cast<int *>(lds);  // per wave
+  if (lane == 0) failed[wave] = !there;
+  if (parts > 1) {
+    // part i of row `wave` is in place wave + i * at_once
+    float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = red_ml + 2 * NW * PARTS;
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) {
+      const int place = wave + i * NW;
+      if (lane == 0) *reinterpret_cast<float2 *>(red_ml + 2 * place) = float2{M[i], L[i]};
+      *reinterpret_cast<float2 *>(red_o + place * kHeadDim + 2 * lane) = float2{x[i], y[i]};
+    }
+    __syncthreads();
+    if (part == 0) {
+      M[0] = -INFINITY;
+      for (int i = wave; i < NW * PARTS; i += at_once) M[0] = fmaxf(M[0], red_ml[2 * i]);
+      const float M_use = (M[0] == -INFINITY) ? 0.0f : M[0];
+      L[0] = x[0] = y[0] = 0.0f;
+      for (int i = wave; i < NW * PARTS; i += at_once) {
+        const float wt = fast_exp2(red_ml[2 * i] - M_use);  // 0 for a part without splits (-inf)
+        L[0] += wt * red_ml[2 * i + 1];
+        const float2 o = *reinterpret_cast<const float2 *>(red_o + i * kHeadDim + 2 * lane);
+        x[0] += wt * o.x;
+        y[0] += wt * o.y;
+      }
+    }
+  }
+  if (mine && part == 0 && there) {
+    const int r = (int)fast_div(c, p.g_div);
+    const float inv = (L[0] > 0.0f) ? 1.0f / L[0] : 0.0f;
+    char *row = p.out + (((size_t)b * m + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes;
+    *reinterpret_cast<uint32_t *>(row + (lane & 15) * 16 + (lane >> 4) * 4) = Elem<T>::pack2(x[0] * inv, y[0] * inv);
+  }
+  __syncthreads();
+  int any = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) any |= failed[w];
+  __syncthreads();
+  return any == 0;
+}
+
+// The argument struct of the running kernel, asked for here (as a parameter that two branches use it is fetched, and waited
+// for, before they part).
+__device__ __forceinline__ DecodeLate fetch_late() {
+  constexpr int at = sizeof(addresses_t) + sizeof(u32x4_t) + sizeof(u32x2_t);
+  static_assert(at % alignof(DecodeLate) == 0);
+  auto arguments = (__attribute__((address_space(4))) const char *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(arguments));
+  struct Words {
+    uint64_t w[sizeof(DecodeLate) / 8];
+  } words;
+#pragma unroll
+  for (size_t i = 0; i < sizeof(DecodeLate) / 8; ++i)
+    words.w[i] = ((__attribute__((address_space(4))) const uint64_t *)(arguments + at))[i];
+  DecodeLate p = __builtin_bit_cast(DecodeLate, words);
+  p.out = at_address<char>((uint64_t)p.out);
+  p.ws_o = at_address<float>((uint64_t)p.ws_o);
+  p.ws_ml = at_address<float>((uint64_t)p.ws_ml);
+  return p;
+}
+
+// How the partials of a (sequence, kv head) become rows: not here (one split, or the combine launch), by the workgroup that
+// finds all flags up, by folders that look for tags.  A kernel each: the code of the others in the way costs a call of 4 us 0.05.
 enum FoldMode { kNoFold, kFoldByFlags, kFoldByTags };
 
 template <typename T, bool FUSED, int NW, bool LONG, FoldMode FOLD>
-__global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec, DecodeLate p) {
+__global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec, DecodeLate late) {
   using E = Elem<T>;
   const int n = ec[0], Hkv = ec[1] & 0xffffu, g = ec[1] >> 16 & 0xffu, H = g * Hkv;
   const bool is_neox = ec[1] >> 31;
@@ -212,9 +412,36 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   constexpr int kStepKeys = NW * kDecWaveKeys;
   __shared__ __attribute__((aligned(16))) char lds[2 * NW * kDecWaveLds];
 
-  const int split = blockIdx.x, kvh = blockIdx.y, b = FUSED ? 0 : blockIdx.z;
+  int split = blockIdx.x, kvh = blockIdx.y, b = FUSED ? 0 : blockIdx.z;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, cg = lane >> 4;
+  bool lone = false;  // a folder that stopped waiting: all keys of its (sequence, kv head), and the rows
+  if constexpr (FOLD == kFoldByTags) {
+    const int pairs = FUSED ? Hkv : eb[3] & 0x3ffu;
+    int pair = blockIdx.y;
+    if (__builtin_expect(pair >= pairs, 0)) {
+      const DecodeLate f = fetch_late();
+      const int e = (pair - pairs) * f.num_splits + split;
+      if (e >= pairs * f.folders) return;
+      pair = (int)fast_div(e, f.folders_div);
+      b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
+      const int c0 = (e - pair * f.folders) * f.fold_rows;
+      auto fold = [&](auto depth, auto parts) {
+        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value>(f, lds, pair, b, pair - b * Hkv, c0, rows, m, Hkv, g);
+      };
+      using std::integral_constant;
+      if (NW == 4 && f.num_splits > kMaxFoldSplits ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 2>())
+          : f.num_splits > 4 ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 1>())
+                             : fold(integral_constant<int, 4>(), integral_constant<int, 1>()))
+        return;
+      lone = true;
+      split = 0;
+    }
+    b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
+    kvh = pair - b * Hkv;
+  }
+  const DecodeLate p = FOLD == kFoldByTags ? fetch_late() : late;
+  const int num_splits = lone ? 1 : p.num_splits;
 
   const int row_bytes = Hkv * kRowBytes;
   const size_t seq_off = ((FUSED ? 0 : (size_t)b * ea[3] * Hkv) + kvh) * kRowBytes;
@@ -262,7 +489,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   for (int i = 0; i < 8; ++i) voff[i] = (wave * kDecWaveKeys + 4 * i + cg) * row_bytes + col * 16;
   u32x4_t kn[8], vn[8];
   auto block_buffer = [&](const char *base, int it) {
-    const int first = (it * p.num_splits + split) * kStepKeys;
+    const int first = (it * num_splits + split) * kStepKeys;
     const int have = min(stored - first, kStepKeys);
     const unsigned records = have > 0 ? (unsigned)(have - 1) * row_bytes + kRowBytes : 0u;
     return byte_buffer(base + (size_t)first * row_bytes, records);
@@ -293,9 +520,10 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   char *kl = lds + (NW + wave) * kDecWaveLds;
   if (FUSED) rotate_frags<T>(qf, tab, is_neox);
 
-  const int iters = p.iters_each + (split < p.iters_rest);  // blocks split, split + S, ...
+  const int iters = lone ? p.iters_each * p.num_splits + p.iters_rest
+                         : p.iters_each + (split < p.iters_rest);  // blocks split, split + S, ...
   for (int it = 0; it < iters; ++it) {
-    const int kb0 = (it * p.num_splits + split) * kStepKeys + wave * kDecWaveKeys;
+    const int kb0 = (it * num_splits + split) * kStepKeys + wave * kDecWaveKeys;
     const int at = fused_pos - kb0;               // FUSED: where in the wave's keys the new row is
     const bool owner = FUSED && at >= 0 && at < kDecWaveKeys;
     u32x4_t kc[2][4];
@@ -465,7 +693,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
         acc[4 + j] += wt * s1[j];
       }
     }
-    if (FOLD == kNoFold && p.num_splits == 1) {
+    if (FOLD == kNoFold ? num_splits == 1 : lone) {
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
       const int r = (int)fast_div(c, p.g_div), hq = c - r * g;
       char *op = p.out + (((size_t)b * m + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
@@ -494,104 +722,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       if (dch == 0) *reinterpret_cast<u32x2_t *>(p.ws_ml + (pair * pair_slots + slot) * 2) = ml;
     }
   }
-  if constexpr (FOLD == kNoFold) return;
-
-  // Groups of 32 threads, four dims each: `parts` groups per row deal its splits out among themselves, if they are more
-  // than 8 (fewer: one group takes them all at once; by flags, 512 keys of 32 kv heads 6.65 -> 6.2 us, 1500 of 32 9.9 -> 8.9).
-  constexpr int NG = 2 * NW;
-  const int S = p.num_splits, sg = tid >> 5, d4 = tid & 31;
-  const int at_once = min(rows, NG), parts = S <= kFoldDepth ? 1 : NG / at_once, part = sg / at_once;
-  float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = reinterpret_cast<float *>(lds) + 64;  // per group
-  // Folds the partials ml, ov of splits part, part + parts, ... of row c and stores the row, if all of them are `there` (up
-  // to 8 splits: they need not be).
-  auto fold = [&](int c, const auto &ml, const auto &ov, bool there) {
-    constexpr int D = sizeof(ml) / sizeof(ml[0]);
-    const bool mine = part < parts && c < rows;
-    float M = -INFINITY, L = 0.0f;
-    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-    if (mine) {
-#pragma unroll
-      for (int j = 0; j < D; ++j)
-        if (part + parts * j < S) M = fmaxf(M, bits_float(ml[j][0]));
-      const float M_use = (M == -INFINITY) ? 0.0f : M;
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const float wt = (part + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
-        L += wt * bits_float(ml[j][1]);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
-      }
-    }
-    if (parts > 1) {
-      if (d4 == 0) {
-        red_ml[2 * sg] = M;
-        red_ml[2 * sg + 1] = L;
-      }
-      *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
-      __syncthreads();
-      if (part == 0) {
-        for (int g2 = sg + at_once; g2 < parts * at_once; g2 += at_once) {
-          const float m2 = red_ml[2 * g2], Mn = fmaxf(M, m2);
-          const float M_use = (Mn == -INFINITY) ? 0.0f : Mn;
-          const float wa = fast_exp2(M - M_use), wb = fast_exp2(m2 - M_use);
-          L = L * wa + red_ml[2 * g2 + 1] * wb;
-          const f32x4_t o2 = *reinterpret_cast<const f32x4_t *>(red_o + g2 * kHeadDim + 4 * d4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] = acc[i] * wa + o2[i] * wb;
-          M = Mn;
-        }
-      }
-    }
-    if (part == 0 && c < rows && there) {
-      const int r = (int)fast_div(c, p.g_div);
-      const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-      u32x2_t w;
-      w[0] = E::pack2(acc[0] * inv, acc[1] * inv);
-      w[1] = E::pack2(acc[2] * inv, acc[3] * inv);
-      *reinterpret_cast<u32x2_t *>(p.out + (((size_t)b * m + r) * H + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
-    }
-  };
-
-  if constexpr (FOLD == kFoldByTags) {
-    // ---- fold whatever is there with this launch's number beside its words ----
-    // Words that carry a tag need no flag behind them: two memory round trips (stored here, read all) where
-    // flags take four.  The two words of a 16-byte piece carry a half each: a piece that an earlier launch stored differs in
-    // both, whenever that was (one half repeats after 2.97e9 launches, both after 2^64).  Each workgroup looks once its own words have reached the point where all XCDs see them, so
-    // that the last one to get there finds all of them; another one leaves out what is not there yet.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    constexpr int RI = (kTaggedRows + NG - 1) / NG, D = kFoldDepth;  // rows of a group, splits
-    const int piece = (d4 & 1) * 512 + (d4 >> 1) * 16;                // dims 4*d4 .. +3
-    u32x4_t a[RI][D][2], ml4[RI][D];
-    // (no branches: past the splits and rows the offset is past the buffer, and the load is not made)
-#pragma unroll
-    for (int r = 0; r < RI; ++r)
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const int c = r * at_once + sg;
-        const int at = sg < at_once && c < rows && j < S ? (j * rows + c) * kTaggedBytes : 0x40000000;
-        a[r][j][0] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece));
-        a[r][j][1] = __builtin_bit_cast(u32x4_t, load_device(pt, at + piece + 256));
-        ml4[r][j] = __builtin_bit_cast(u32x4_t, load_device(pt, at + kHeadDim * 8));
-      }
-#pragma unroll
-    for (int r = 0; r < RI; ++r) {
-      const int c = r * at_once + sg;
-      u32x2_t ml[D];
-      f32x4_t ov[D];
-      uint32_t differs = 0;
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const uint32_t d = (a[r][j][0][1] ^ tag0) | (a[r][j][0][3] ^ tag1) | (a[r][j][1][1] ^ tag0) |
-                           (a[r][j][1][3] ^ tag1) | (ml4[r][j][1] ^ tag0) | (ml4[r][j][3] ^ tag1);
-        differs |= j < S ? d : 0u;
-        ml[j] = u32x2_t{ml4[r][j][0], ml4[r][j][2]};
-        ov[j] = f32x4_t{bits_float(a[r][j][0][0]), bits_float(a[r][j][0][2]), bits_float(a[r][j][1][0]), bits_float(a[r][j][1][2])};
-      }
-      fold(c, ml, ov, differs == 0);
-    }
-    return;
-  }
+  if constexpr (FOLD != kFoldByFlags) return;
 
   // ---- fold in the workgroup that finds every partial of its (sequence, kv head) stored ----
   // Each workgroup raises its flag once its partial has reached the point where all XCDs see it, and looks at the
@@ -615,23 +746,22 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   if (*all_up == 0) return;
   if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
   // every partial of a thread's share is asked for before the first is used
-  auto take = [&](int c, auto depth) {
-    constexpr int D = decltype(depth)::value;
-    u32x2_t ml[D];
-    f32x4_t ov[D];
+  constexpr int NG = 2 * NW;
+  const int parts = fold_parts(p.num_splits), at_once = NG / parts, part = (tid >> 5) / at_once, d4 = tid & 31;
+  for (int c0 = 0; c0 < rows; c0 += at_once) {
+    const int c = c0 + (tid >> 5) % at_once;
+    RowFold f;
+    u32x2_t ml[kFoldDepth];
+    f32x4_t ov[kFoldDepth];
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      const int slot = min(part + parts * j, S - 1) * p.cols + min(c, rows - 1);
+    for (int j = 0; j < kFoldDepth; ++j) {
+      const int slot = min(part + parts * j, p.num_splits - 1) * p.cols + min(c, rows - 1);
       ml[j] = load_device2(pml, slot * 8);
       ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
     }
-    fold(c, ml, ov, true);
-  };
-  for (int c0 = 0; c0 < rows; c0 += at_once) {
-    if (S <= kFoldDepth * parts)
-      take(c0 + sg % at_once, std::integral_constant<int, kFoldDepth>());
-    else
-      take(c0 + sg % at_once, std::integral_constant<int, kMaxFoldSplits>());
+    f.take(ml, ov, part, parts, p.num_splits);
+    if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
+    if (part == 0 && c < rows) f.template store<T>(p.out, b, m, c, kvh, Hkv, g, p.g_div, d4);
   }
 }
 
@@ -846,7 +976,7 @@ static uint64_t launch_number() {
     return ((uint64_t)rd() << 32) ^ rd() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
   }()};
   uint64_t before = last.load(std::memory_order_relaxed), n;
-  do n = next_launch_number(before);
+  do n = llmhip::next_launch_number(before);
   while (!last.compare_exchange_weak(before, n, std::memory_order_relaxed));
   return n;
 }
@@ -878,8 +1008,12 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
     }
   }
   const DecodeEarly early(p);
-  hipLaunchKernelGGL(kern, dim3(p.num_splits, p.Hkv, p.batch), dim3(64 * NW), pad, stream, early.a, early.b, early.c,
-                     static_cast<const DecodeLate &>(p));
+  dim3 grid(p.num_splits, p.Hkv, p.batch);
+  if (FOLD == kFoldByTags) {
+    const int pairs = p.batch * p.Hkv;
+    grid = dim3(p.num_splits, pairs + (pairs * p.folders + p.num_splits - 1) / p.num_splits);
+  }
+  hipLaunchKernelGGL(kern, grid, dim3(64 * NW), pad, stream, early.a, early.b, early.c, static_cast<const DecodeLate &>(p));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
   hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream,
@@ -894,9 +1028,7 @@ static hipError_t launch_decode_f(const DecodeParams &p, bool half, bool many, h
   if constexpr (FOLD != kNoFold) {  // (blocks of 64 keys come in splits of one, and few enough to be folded)
     if (half) return launch_decode_t<T, FUSED, 2, false, FOLD>(p, stream);
   }
-  if constexpr (FOLD != kFoldByTags) {
-    if (many) return launch_decode_t<T, FUSED, 4, true, FOLD>(p, stream);
-  }
+  if (many) return launch_decode_t<T, FUSED, 4, true, FOLD>(p, stream);
   return launch_decode_t<T, FUSED, 4, false, FOLD>(p, stream);
 }
 template <typename T, bool FUSED>
@@ -926,17 +1058,22 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
   FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
-  // Up to 8 partials of up to 8 rows by tags instead of flags, where the room is there and what the workgroups read together,
-  // each the partials of its (sequence, kv head) and that past the L2s, is at most 7 MB: beyond 8 it takes longer than the two
-  // round trips that it saves (us, flags / tags, K and V from HBM; 532 shapes of 1-32 sequences, 1-32 kv heads, 130-8000 keys:
-  // up to 1 MB tags are 6 % faster on average, at 5 MB 3 %; 6 to 8 MB even, 5 x 3000 keys of 8 kv heads 14.6 / 14.4 in one
-  // run, 14.24 / 14.44 in another; 12 MB, 8 x 2000 of 4, 7 query rows 10.7 / 11.8; 17 MB, 16 x 1000 of 2, 8 rows 8.8 / 10.2).
-  // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones: taken
-  // down by the folder, as flags are, they cost what the tags gain.
-  const size_t tagged = (size_t)p.batch * p.Hkv * p.num_splits * p.rows * kTaggedBytes;
-  if (how == kFoldByFlags && p.num_splits <= kFoldDepth && p.rows <= kTaggedRows && p.iters_each < 8 &&
-      tagged <= workspace_bytes && tagged * p.num_splits <= kTaggedReads && !may_be_capturing(stream))
+  // Up to 32 partials of up to 8 rows (as many as the room that a call may insist on holds with tags) by folders, as many of them as
+  // the CUs that the other workgroups leave idle can take, down to one row each.
+  // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones.
+  const long long pairs = (long long)p.batch * p.Hkv;
+  const size_t tagged = (size_t)pairs * p.num_splits * p.rows * kTaggedBytes;
+  if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && p.rows <= kTaggedRows && pairs <= kTaggedPairs &&
+      tagged <= workspace_bytes && !may_be_capturing(stream)) {
     how = kFoldByTags;
+    if (p.fold == 0) p.fold = launch_number();
+    const int parts = fold_parts(p.num_splits);
+    const long long idle = device_compute_units() - pairs * p.num_splits;
+    p.fold_rows = (half ? 2 : 4) / (parts > 4 ? 4 : parts);
+    while (p.fold_rows > 1 && pairs * ((2 * p.rows + p.fold_rows - 1) / p.fold_rows) <= idle) p.fold_rows /= 2;
+    p.folders = (p.rows + p.fold_rows - 1) / p.fold_rows;
+    p.folders_div = make_fast_div((uint32_t)p.folders);
+  }
   p.g_div = make_fast_div((uint32_t)p.g);
   p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
@@ -995,6 +1132,7 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
   return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, true, stream);
 }
 
+#ifndef LLMHIP_BENCH
 // ---------------------------------------------------------------------------
 // Decode without any allocation: the split-KV partials live in a fixed array in device memory
 // that is part of the library's code object (every GPU the library runs on holds its own copy
@@ -1030,5 +1168,6 @@ hipError_t launch_flash_decode_static(void *out, const void *q, const void *k, c
   return launch_flash_decode(out, q, k, v, ptr, kStaticDecodeScratchBytes, batch, 1, n, n - 1, kv_seq_stride, group_size,
                              kv_head_num, num_splits, dt, stream);
 }
+#endif  // !LLMHIP_BENCH
 
-}  // namespace llmhip
+}  // namespace LLMHIP_NS
