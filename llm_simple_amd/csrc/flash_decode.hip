@@ -745,24 +745,33 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   __syncthreads();
   if (*all_up == 0) return;
   if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
-  // every partial of a thread's share is asked for before the first is used
+  // Every partial of a thread's share is asked for before the first is used.  More rows than folders take leave no groups to deal
+  // the partials of a row to: a group has all of them (15 rows of 12 partials, us, in two parts and four rounds / so in two: 12.65 / 11.2).
   constexpr int NG = 2 * NW;
-  const int parts = fold_parts(p.num_splits), at_once = NG / parts, part = (tid >> 5) / at_once, d4 = tid & 31;
-  for (int c0 = 0; c0 < rows; c0 += at_once) {
-    const int c = c0 + (tid >> 5) % at_once;
-    RowFold f;
-    u32x2_t ml[kFoldDepth];
-    f32x4_t ov[kFoldDepth];
+  const int d4 = tid & 31;
+  auto fold = [&](auto depth, int parts) {
+    constexpr int D = decltype(depth)::value;
+    const int at_once = NG / parts, part = (tid >> 5) / at_once;
+    for (int c0 = 0; c0 < rows; c0 += at_once) {
+      const int c = c0 + (tid >> 5) % at_once;
+      RowFold f;
+      u32x2_t ml[D];
+      f32x4_t ov[D];
 #pragma unroll
-    for (int j = 0; j < kFoldDepth; ++j) {
-      const int slot = min(part + parts * j, p.num_splits - 1) * p.cols + min(c, rows - 1);
-      ml[j] = load_device2(pml, slot * 8);
-      ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
+      for (int j = 0; j < D; ++j) {
+        const int slot = min(part + parts * j, p.num_splits - 1) * p.cols + min(c, rows - 1);
+        ml[j] = load_device2(pml, slot * 8);
+        ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
+      }
+      f.take(ml, ov, part, parts, p.num_splits);
+      if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
+      if (part == 0 && c < rows) f.template store<T>(p.out, b, m, c, kvh, Hkv, g, p.g_div, d4);
     }
-    f.take(ml, ov, part, parts, p.num_splits);
-    if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
-    if (part == 0 && c < rows) f.template store<T>(p.out, b, m, c, kvh, Hkv, g, p.g_div, d4);
-  }
+  };
+  if (NW == 4 && rows > kTaggedRows && p.num_splits > kFoldDepth)
+    fold(std::integral_constant<int, kMaxFoldSplits>(), 1);
+  else
+    fold(std::integral_constant<int, kFoldDepth>(), fold_parts(p.num_splits));
 }
 
 // Folds the splits of one output row (one query row of one head) with the log-sum-exp rule.
