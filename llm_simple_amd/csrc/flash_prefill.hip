@@ -65,15 +65,16 @@ constexpr int kMaxPrefillSplits = 128;           // key ranges per call
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
 // What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way -- except with SPLIT, where
-// the key range (per_split, num_splits, chunk) is needed for the first address and waited for.
+// the key range (per_split and what stands before it) is needed for the first address and waited for.
 struct PrefillLate {
   char *out;
-  // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers
-  // keys [s*chunk, (s+1)*chunk); with more than one split every workgroup leaves an fp32 partial
-  // (reference maximum, sum, unnormalised O) that prefill_combine_kernel folds.
+  // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers the key tiles s * first_each,
+  // then every step_div.d-th, up to range_keys keys of them (see launch_prefill_t); with more than one split every workgroup
+  // leaves an fp32 partial (reference maximum, sum, unnormalised O) that prefill_combine_kernel folds.
   float *ws_o;            // [split][m][H][128]
   float *ws_ml;           // [split][m][H][2]
-  int num_splits, chunk;  // chunk: multiple of 64 keys
+  int num_splits, first_each, range_keys;
+  FastDiv step_div;
   FastDiv per_split;      // of an XCD's work list: items per key range
   float scale_log2e;
 #ifdef LLMHIP_BENCH
@@ -93,6 +94,7 @@ struct PrefillParams : PrefillLate {
   // token-major (row index = token * g + head % g), so a chunk shorter than a tile reads K and V of
   // its kv head once for all g query heads.
   int pack;
+  int chunk;  // keys of a range: a multiple of 128
 };
 // What the index arithmetic and the first loads of a workgroup need (of an unsplit one: see PrefillLate), packed into the first 14
 // words of a kernel's arguments, which are in registers when it starts.  With kernels of their own for key ranges, whose packed rows and partials a prompt need not step
@@ -534,15 +536,18 @@ typedef __attribute__((ext_vector_type(4))) uint32_t buffer_t;
 template <int NW, int TN, bool NT> struct DirectLoader {
   static constexpr int kSlots = TN / 4 / NW;  // instructions per wave per tile
   static constexpr int kLow = 1024 * ((kSlots < 4 ? kSlots : 4) - 1);
-  uint32_t tile_step, whole, last;            // bytes to the next tile; records of a whole tile and of the last one
+  uint64_t tile_step;                         // bytes to the next tile
+  uint32_t whole, last;                       // records of a whole tile and of the cache's last one
+  int keys_step;                              // keys to the next tile
   uint32_t lds_wave;                          // LDS byte offset of the wave's first row (wave-uniform)
   uint32_t off_k[kSlots], off_v[kSlots];      // lane offsets within a tile
 
-  // n keys in J tiles
-  __device__ __forceinline__ void init(int wave, int lane, int row_bytes, int n, int J) {
-    tile_step = TN * row_bytes;
+  // Every step-th tile of n keys
+  __device__ __forceinline__ void init(int wave, int lane, int row_bytes, int step, int n) {
+    keys_step = TN * step;
+    tile_step = (uint64_t)(uint32_t)(TN * row_bytes) * (uint32_t)step;
     whole = (TN - 1) * row_bytes + kRowBytes + kLow;
-    last = min(TN - 1, n - (J - 1) * TN - 1) * row_bytes + kRowBytes + kLow;
+    last = ((n - 1) & (TN - 1)) * row_bytes + kRowBytes + kLow;
     lds_wave = __builtin_amdgcn_readfirstlane(wave * kSlots * 1024);
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
@@ -553,24 +558,27 @@ template <int NW, int TN, bool NT> struct DirectLoader {
       asm volatile("" : "+v"(off_k[s]), "+v"(off_v[s]));
     }
   }
-  // Descriptor of a key tile, kLow bytes early, that walks from tile to tile.  Past the last one, J - 1, it has no
+  // Descriptor of a key tile, kLow bytes early, that walks from tile to tile.  Past the last key it has no
   // bytes: the loads that a workgroup makes ahead of its last steps fetch nothing (the last tile again before; us: 256 tokens of 32
   // heads 5.90 -> 5.84, 512 of 28 8.48 -> 8.40, 1400 22.84 -> 22.47, 2048 38.6 -> 38.1, 100 past 8000 of 40 27.0 -> 26.75).
   struct Stream {
     buffer_t d;
-    int left;  // tiles to come
+    int left;  // keys from the tile's first one on
   };
-  __device__ __forceinline__ Stream stream(const char *base, int J) const {
+  __device__ __forceinline__ uint32_t records(int left) const {
+    const uint32_t bytes = left >= TN ? whole : last;
+    return left > 0 ? bytes : 0u;
+  }
+  __device__ __forceinline__ Stream stream(const char *base, int left) const {
     const uint64_t at = (uint64_t)base - kLow;
-    return Stream{{(uint32_t)at, (uint32_t)(at >> 32), J > 1 ? whole : last, 0x00020000u}, J - 1};
+    return Stream{{(uint32_t)at, (uint32_t)(at >> 32), records(left), 0x00020000u}, left};
   }
   __device__ __forceinline__ void next(Stream &st) const {
-    const uint64_t at = (((uint64_t)st.d[1] << 32) | st.d[0]) + (st.left > 0 ? tile_step : 0u);
-    st.left -= 1;
+    const uint64_t at = (((uint64_t)st.d[1] << 32) | st.d[0]) + tile_step;
+    st.left -= keys_step;
     st.d[0] = (uint32_t)at;
     st.d[1] = (uint32_t)(at >> 32);
-    const uint32_t bytes = st.left > 0 ? whole : last;
-    st.d[2] = st.left < 0 ? 0u : bytes;
+    st.d[2] = records(st.left);
   }
   // Slots 0 .. kSlots-1 of a tile in order, with no other tile's in between; lds_tile: LDS byte offset of the destination.
   // NT: the tile is read by this workgroup only (a packed chunk of one tile per kv head over a long
@@ -644,33 +652,34 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     tok_hi = (int)fast_div(tok_hi, e.g_div);
     tile_tok_end = (int)fast_div(rows_end - 1, e.g_div) + 1;
   }
-  // This workgroup's key range, seen as a cache of its own: rows [k_lo, k_lo + n_) with the causal
-  // offset shifted accordingly (negative when the range starts past a row's last visible key).
-  const int k_lo = SPLIT ? split * p.chunk : 0;
-  const int n_ = SPLIT ? min(e.n - k_lo, p.chunk) : e.n;
-  const int offset_ = e.offset - k_lo;
-  const int n_vis = min(n_, tile_tok_end + offset_);  // keys any row of this tile can see
+  const int n_vis = min(e.n, tile_tok_end + e.offset);  // keys any row of this tile can see
   constexpr int kTileShift = TN == 128 ? 7 : 6;
   static_assert(1 << kTileShift == TN, "");
-  const int J = (n_vis + TN - 1) >> kTileShift;  // tiles of the workgroup
+  const int first = SPLIT ? split * p.first_each : 0, step = SPLIT ? (int)p.step_div.d : 1;  // of this workgroup's tiles
+  int first_keys = n_vis - first * TN;  // keys from its first one on, within its range
+  if (SPLIT) first_keys = min(first_keys, p.range_keys);
+  auto mine = [&](int keys) {  // its tiles that hold one of the first `keys` keys
+    int tiles = ((SPLIT ? min(keys - first * TN, p.range_keys) : keys) + TN - 1) >> kTileShift;
+    if (SPLIT && step > 1) tiles = tiles > 0 ? (int)fast_div(tiles + step - 1, p.step_div) : 0;
+    return tiles;
+  };
   const uint32_t q_row_bytes = (uint32_t)e.H * kRowBytes;
   const int kv_row_bytes = e.Hkv * kRowBytes;
-  const char *kbase = e.k + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
-  const char *vbase = e.v + (size_t)k_lo * kv_row_bytes + (size_t)kvh * kRowBytes;
+  const size_t kv_first = (size_t)(uint32_t)(first * TN) * kv_row_bytes + (size_t)kvh * kRowBytes;
+  const char *kbase = e.k + kv_first, *vbase = e.v + kv_first;
 
   WaveAttn<T, KB> w;
-  // tiles in which this wave's keys hold at least one visible key
-  const int Jw = (qblk0 < rows) ? max(0, min(J, (min(n_, tok_hi + offset_ + 1) - kw0 + TN - 1) >> kTileShift)) : 0;
+  const size_t part_slot = SPLIT ? ((size_t)split * e.m + qtok) * e.H + qhead : 0;
   float *part_o = nullptr, *part_ml = nullptr;
-  if (SPLIT) {
-    const size_t slot = ((size_t)split * e.m + qtok) * e.H + qhead;
-    part_o = p.ws_o + slot * kHeadDim;
-    part_ml = p.ws_ml + slot * 2;
-    if (J <= 0) {  // workgroup-uniform: no row of this tile sees a key of this range
-      w.init(lds, lane, kVRegion);
-      store_partial(w, part_o, part_ml, row_valid);
-      return;
-    }
+  auto find_partial = [&] {
+    part_o = p.ws_o + part_slot * kHeadDim;
+    part_ml = p.ws_ml + part_slot * 2;
+  };
+  if (SPLIT && first_keys <= 0) {  // workgroup-uniform: no row of this tile sees a key of this range
+    find_partial();
+    w.init(lds, lane, kVRegion);
+    store_partial(w, part_o, part_ml, row_valid);
+    return;
   }
   // Q.  A fragment load straight into the operand layout touches 32 rows with 32 bytes each, 256 tag look-ups per
   // wave; Q goes through LDS like a K tile instead, fetched once as whole rows, and the first scores wait for it and K
@@ -692,11 +701,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   }
 
   DirectLoader<NW, TN, NT> ld;
-  ld.init(wave, lane, kv_row_bytes, n_, J);
+  ld.init(wave, lane, kv_row_bytes, step, n_vis);
   // K runs one tile ahead of V: S(j+1) = K(j+1) Q^T is issued together with the softmax of
   // tile j, so K tile t is fetched SUB+1 iterations and V tile t SUB iterations before use.
   using Loader = DirectLoader<NW, TN, NT>;
-  typename Loader::Stream kst = ld.stream(kbase, J), vst = ld.stream(vbase, J);
+  typename Loader::Stream kst = ld.stream(kbase, first_keys), vst = ld.stream(vbase, first_keys);
   static_for<0, SUB + 1>([&](auto u_) {
     constexpr int u = decltype(u_)::value;
     static_for<0, PER>([&](auto r) { ld.template issue<false, decltype(r)::value>(kst, u % NSLOT * TB); });
@@ -706,6 +715,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       ld.next(vst);
     }
   });
+  const int J = mine(n_vis);
+  // tiles in which this wave's keys hold at least one visible key
+  const int Jw = (qblk0 < rows) ? max(0, min(J, mine(min(e.n, tok_hi + e.offset + 1) - kw0))) : 0;
   // The late arguments are asked for now, while the loads are under way, not at the place of each one's use
   asm volatile("" : : "s"(p.out), "s"(p.scale_log2e));
   if (SPLIT) asm volatile("" : : "s"(p.ws_o), "s"(p.ws_ml));
@@ -724,9 +736,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   auto tile_step = [&](int j, int slot, f32x16_t (&s_cur)[KB], f32x16_t (&s_nxt)[KB]) {
     const int kslot = (slot + SUB + 1) % NSLOT, vslot = (slot + SUB) % NSLOT;  // fetched now
     if (j < Jw) {
-      const int key0 = j * TN + kw0;
-      if ((key0 + kWaveKeys - 1 > tok_lo + offset_) || (key0 + kWaveKeys > n_))
-        w.mask(s_cur, key0, qtok, offset_, n_);
+      const int key0 = (SPLIT ? j * step + first : j) * TN + kw0;
+      if ((key0 + kWaveKeys - 1 > tok_lo + e.offset) || (key0 + kWaveKeys > e.n))
+        w.mask(s_cur, key0, qtok, e.offset, e.n);
       // In the 8-wave kernel a burst of loads would stall every wave behind the texture addresser's
       // queue: one load every 8 * KB / PER MFMAs instead.  The 4-wave kernels run where a step is
       // short against a memory round trip, and issue a phase's loads beside its first MFMAs
@@ -787,6 +799,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     }
   }
   // every wave is past the last barrier of the loop: nobody reads the K/V tiles any more
+  if (SPLIT) find_partial();
   char *out_blk = p.out + (size_t)qblk0 * q_row_bytes + (size_t)head * kRowBytes;
   auto part_row = [&](int r) {  // where the partial of row r of the wave's goes
     int tok = qblk0 + r, h = head;
@@ -999,6 +1012,15 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   }
   p.list_heads = make_fast_div((uint32_t)list_heads);
   p.per_split = make_fast_div((uint32_t)(list_heads * T_));
+  // Key ranges lie side by side, or, where a key's rows together are long, one tile wide through each other, so that the workgroups
+  // walk through the cache together: ranges that begin a multiple of MiB apart meet the same memory channels (rope and combine included,
+  // us, side by side / through each other: 40 tokens past 16233 keys of 32 kv heads 66.8 / 58.0, past 4013 22.7 / 20.1, 64 past
+  // 32174 119.1 / 108.3, 20 past 32216 of 8 40.2 / 34.7; of 4 and 2, 100 past 3943 19.8 / 20.6, 20 past 16318 18.3 / 18.9).
+  const bool through = p.Hkv >= 8;
+  constexpr int TN = KP == 4 ? 2 * kTileN : kTileN;
+  p.first_each = through ? 1 : p.chunk / TN;
+  p.range_keys = through ? 0x7fffffff : p.chunk;
+  p.step_div = make_fast_div(through ? (uint32_t)S_ : 1u);
   p.g_div = make_fast_div((uint32_t)p.g);
   const size_t tile_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes, q_bytes = (size_t)BM * kRowBytes;
   const size_t lds_bytes = tile_bytes + (KP > 1 ? q_bytes : q_bytes - tile_bytes / 4);  // (half of the V slots are Q's at first)
