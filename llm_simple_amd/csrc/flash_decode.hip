@@ -25,7 +25,7 @@
 // waves are merged through LDS at the end and the workgroup writes the final rows (one split) or an
 // fp32 partial (max, sum, unnormalised O).
 //
-// Up to 32 partials of a (sequence, kv head) are folded (log-sum-exp) by workgroups of the same launch that do nothing else
+// Up to 128 partials of a (sequence, kv head) are folded (log-sum-exp) by workgroups of the same launch that do nothing else
 // (folders): every word of a partial goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it, and a folder
 // looks at all of them until it finds the number everywhere.  That is one way to memory and one back; no fence, no flag, no atomic.
 // Folders have the highest workgroup numbers, so that they are dispatched after the workgroups that they wait for, and on
@@ -33,10 +33,11 @@
 // depends on the order of dispatch.  A look costs what its loads cost: a wave per row, two dims per lane, the maxima and
 // sums of all partials in one load (two rows per wave with three loads per partial: 1.5 us a look, 0.6 now).
 // (Fused step, us, the last workgroup to store folds / folders: 384 keys of 2 kv heads 5.52 / 4.85, 512 of 32 5.23 / 5.01, 32768 of 8, with
-// a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1.)
+// a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1; beyond 32 partials, a combine launch / folders: 4700 keys of
+// 4 kv heads 7.92 / 7.06, 14000 10.45 / 9.62, 31000 15.2 / 14.5, 6000 of 2 7.77 / 6.68, 20000 10.25 / 9.58.)
 // Where the number would be that of a replay, up to 16 partials are folded by the workgroup that finds them all stored: partials,
 // then a flag, then a look at the other flags, then the partials, four round trips to memory.  Beyond that, for more than 8 rows or
-// 32 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
+// 128 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
 // against 33 at batch 1, 32768 keys.)
 //
 // A short cache is bound by the length of one workgroup's chain, not by bytes: at 32 keys, one sequence, the
@@ -177,7 +178,7 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
   return row * kRowBytes + ((((granule >> 1) ^ (row & 7)) << 5) | ((granule & 1) << 4));
 }
 
-constexpr int kMaxFoldSplits = 16, kMaxTaggedSplits = 32;
+constexpr int kMaxFoldSplits = 16, kMaxTaggedSplits = 128;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
 constexpr int kTaggedRows = 8;                    // query rows whose words carry a tag, at most
 constexpr int kTaggedPairs = 1023;                // (sequence, kv head) pairs, at most
@@ -285,11 +286,12 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 
 // A folder: rows c0 .. c0 + fold_rows - 1 of a pair, from partials whose words carry this launch's tags.  A wave has a row, two
 // dims per lane, and PARTS of the fold_parts() parts of its partials, DEPTH in all.  It looks at all of them until it finds the tags
-// at every word.  False if they were not there after kFoldPolls looks.
+// at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  False if they were not there after
+// kFoldPolls looks.
 template <typename T, int NW, int DEPTH, int PARTS>
 __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int b, int kvh, int c0, int rows, int m, int Hkv,
                                             int g) {
-  constexpr int EACH = DEPTH / PARTS;
+  constexpr int EACH = DEPTH / PARTS, ROUND = PARTS > 1 ? 4 : EACH;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
   const int parts = fold_parts(S), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
   const bool mine = wave % at_once < p.fold_rows && c < rows;  // (of the wave)
@@ -326,13 +328,30 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int 
       if (there) break;
       __builtin_amdgcn_s_sleep(1);
     }
-    const float my_m = have ? bits_float(ml[0]) : -INFINITY, M_lanes = max_of_lanes<EACH>(my_m);
-    const float wt = have ? fast_exp2(my_m - (M_lanes == -INFINITY ? 0.0f : M_lanes)) : 0.0f, my_l = have ? bits_float(ml[2]) : 0.0f;
+    // the maximum of each round of partials, then, in the lanes of a round, that of its part up to there
+    const float my_m = have ? bits_float(ml[0]) : -INFINITY, my_l = have ? bits_float(ml[2]) : 0.0f;
+    const float of_round = max_of_lanes<ROUND>(my_m);
+    float upto[DEPTH / ROUND], mine_upto = of_round;
+#pragma unroll
+    for (int r = 0; r < DEPTH / ROUND; ++r) {
+      upto[r] = lane_value(of_round, r * ROUND);
+      if (r * ROUND % EACH != 0) upto[r] = fmaxf(upto[r], upto[r - 1]);
+      if (ROUND < EACH && (lane & (DEPTH - 1)) / ROUND == r) mine_upto = upto[r];
+    }
+    const float wt = have ? fast_exp2(my_m - (mine_upto == -INFINITY ? 0.0f : mine_upto)) : 0.0f;
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) {
-      const int i = j / EACH;
+      const int i = j / EACH, r = j / ROUND;
+      if (j % ROUND == 0) {
+        if (j % EACH != 0) {
+          const float resc = fast_exp2(M[i] - (upto[r] == -INFINITY ? 0.0f : upto[r]));
+          L[i] *= resc;
+          x[i] *= resc;
+          y[i] *= resc;
+        }
+        M[i] = upto[r];
+      }
       const float w = lane_value(wt, j);
-      if (j % EACH == 0) M[i] = lane_value(M_lanes, j);
       L[i] += w * lane_value(my_l, j);
       x[i] += w * bits_float(a[j][0]);
       y[i] += w * bits_float(a[j][2]);
@@ -430,7 +449,9 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
         return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value>(f, lds, pair, b, pair - b * Hkv, c0, rows, m, Hkv, g);
       };
       using std::integral_constant;
-      if (NW == 4 && f.num_splits > kMaxFoldSplits ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 2>())
+      if (NW == 4 && f.num_splits > 64   ? fold(integral_constant<int, 4 * kFoldDepth>(), integral_constant<int, 2>())
+          : NW == 4 && f.num_splits > 32 ? fold(integral_constant<int, 2 * kFoldDepth>(), integral_constant<int, 2>())
+          : NW == 4 && f.num_splits > kMaxFoldSplits ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 2>())
           : f.num_splits > 4 ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 1>())
                              : fold(integral_constant<int, 4>(), integral_constant<int, 1>()))
         return;
@@ -1067,7 +1088,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
   FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
-  // Up to 32 partials of up to 8 rows (as many as the room that a call may insist on holds with tags) by folders, as many of them as
+  // Up to 128 partials of up to 8 rows (as many as the room that a call may insist on holds with tags) by folders, as many of them as
   // the CUs that the other workgroups leave idle can take, down to one row each.
   // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones.
   const long long pairs = (long long)p.batch * p.Hkv;

@@ -1,4 +1,4 @@
-"""Decode partials folded by workgroups of the same launch: the edges of that form (4, 5, 8, 9, 16, 17, 32 splits and 33, 8 query
+"""Decode partials folded by workgroups of the same launch: the edges of that form (4, 5, 8, 9, 16, 17, 32, 33, 64, 65, 128 splits and 129, 8 query
 rows and 9, 1023 (sequence, kv head) pairs and 1024, no CU left idle, more than one round of workgroups), each against the oracle,
 bit for bit the same when repeated over the words of other calls and from a HIP graph, which folds otherwise.  And what a folder does
 that finds no partials in time: its rows from the caches by itself, in the measurement library's copy, where none waits."""
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 # (batch, n, H, Hkv, splits)
 CASES = [(1, 1030, 40, 8, 4), (1, 1030, 7, 1, 5), (1, 2000, 28, 4, 16), (1, 2100, 8, 1, 16), (1, 2177, 5, 1, 17), (2, 4095, 8, 1, 31),
-         (1, 4097, 40, 8, 32), (1, 4300, 40, 8, 33), (1, 2000, 9, 1, 9), (3, 4000, 24, 8, 11), (9, 1500, 14, 2, 12),
+         (1, 4097, 40, 8, 32), (1, 4300, 40, 8, 33), (1, 8200, 7, 1, 64), (1, 8400, 14, 2, 65), (1, 12700, 12, 2, 99), (2, 16500, 8, 1, 128),
+         (1, 17000, 6, 1, 129), (1, 2000, 9, 1, 9), (3, 4000, 24, 8, 11), (9, 1500, 14, 2, 12),
          (1023, 257, 1, 1, 2), (1024, 257, 1, 1, 2), (1, 40000, 4, 4, 32)]
 
 
