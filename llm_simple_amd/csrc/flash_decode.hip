@@ -886,33 +886,35 @@ int flash_decode_max_default_splits(long long pairs) {
   return (int)base;
 }
 
-// Split count that a simple model of the launch makes fastest.  Workgroups run one per CU in rounds
-// of as many workgroups as the device has CUs; a CU of a full round streams 27.9 GB/s (all 256 of an
-// MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads), a CU of a thin
-// round the more the fewer they are (32 KiB in flight, a little more in short streams, over a latency that grows with
-// the load); a workgroup costs about 3 us beyond its bytes, folding up to 8 partials in the kernel 2.0 us, 1.2 in blocks of
-// 64 keys, up to 16 2.6 us, the combine launch 2.1 us.  (Constants of the streams fitted over 250 shapes,
-// batch 1-16 x 2-32 kv heads x 600-32000 keys, every split count: mean error 6 %; those of the folds over 515 of batch 1-16
-// x 2-32 kv heads x 130-7000 keys, where the count chosen is 0.3 % slower than the fastest on average: 2 x 384 keys of 32 kv
-// heads 7.8 -> 6.95 us; 9 x 3943 of 2 kv heads takes 11 or more parts, 11.6 us, where 8 take 11.9.)  Among the counts within
-// 3 % of the best, one that fills its rounds exactly is preferred, else the smallest.  For the common shapes
-// this is about one workgroup per CU (batch 16 x 8 kv heads -> 2 splits, batch 1 -> 32); for pair counts that
-// do not divide a round it finds the count that fills the rounds.  Over those shapes the count chosen is the
-// fastest measured one or within 12 % of it, 0.5 % on average.  (A launch has become 0.3-0.5 us shorter since.  Over 108 other shapes of
-// batch 1-16 x 1-32 kv heads x 130-32000 keys: 0.4 % on average, 1.1 % at the 90th percentile, 18 % at most, 249 keys of 32 kv heads 6.05 us
-// in one part, 5.13 in two.)
-static double split_model_us(long long pairs, int nblocks, int s, int cus) {
+// Split count that a simple model of the launch makes fastest.  Workgroups run one per CU.  While each has a CU of its own, a CU
+// streams the more the fewer they are (32 KiB in flight, over a latency that grows with the load); beyond that a CU streams 27.9
+// GB/s (all 256 of an MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads) and the launch takes
+// something between the rounds that the fullest CU runs and the mean of all.  A fold by folders costs 0.9 us in blocks of 64
+// keys, else 2.0 for up to 8 partials, 1.8 for up to 16 and 1.4 beyond (what more of them cost is in the workgroups); more than 8
+// rows are folded by flags and by a second launch, 2.0, 2.6 and 2.1.  Of counts within 0.5 % of the best one that gives every CU one
+// workgroup is taken, else the smallest.  Fitted over 563 shapes of batch 1-16 x 2-32 kv heads x 130-32000 keys and up to 40 counts each: the
+// count chosen is 0.25 % slower than the fastest on average, 0.7 % at the 90th percentile, 9 % at most, where the model before, which
+// added whole rounds up and took a fold by folders for a second launch, was 1.2, 4.4 and 18 % (us: 250 keys of 4 kv heads
+// 5.47 -> 4.63, 3 x 4200 of 32 38.6 -> 34.2, 11 x 2983 of 8 28.7 -> 25.3, 6 x 4566 of 8 22.6 -> 20.3).
+static double split_model_us(long long pairs, int nblocks, int s, int cus, int rows) {
   const long long wgs = pairs * s;
-  const long long full = wgs / cus, rest = wgs % cus;
   const int blocks = (nblocks + s - 1) / s;
-  const double wg_kb = 2.0 * kRowBytes * kDecStepKeys * blocks * 1e-3;  // K and V rows of one kv head
-  double t = full * (wg_kb / 27.9 + 2.7);
-  if (rest > 0) t += wg_kb / ((blocks >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
+  constexpr double kBlockKb = 2.0 * kRowBytes * kDecStepKeys * 1e-3;  // K and V rows of one kv head
+  double t;
+  if (wgs <= cus) {
+    t = kBlockKb * blocks / ((blocks >= 8 ? 46.8 : 52.4) - 18.5 * (double)wgs / cus) + 2.63;
+  } else {
+    const double rounds = 0.41 * (double)((wgs + cus - 1) / cus) + 0.59 * (double)wgs / cus;
+    t = rounds * (kBlockKb * (0.46 * blocks + 0.54 * nblocks / s) / 27.9 + 0.93) + 1.44;
+  }
   if (s == 1) return t;
-  if (s == nblocks && 2 * s <= kFoldDepth && 2 * wgs <= cus) return t + 1.2;
-  return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
+  if (s == nblocks && 2 * s <= kFoldDepth && pairs * (s == 2 ? 6 : 2 * s) <= cus && rows < kDecCols / 2) return t + 0.9;
+  if (rows > kTaggedRows) return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
+  return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 1.8 : 1.4);
 }
-template <typename Model> static int best_splits(long long pairs, int smax, int cus, Model model) {
+// The smallest count within `tolerance` of the best, or one that fills up to full_rounds rounds exactly.
+template <typename Model>
+static int best_splits(long long pairs, int smax, int cus, double tolerance, long long full_rounds, Model model) {
   double t_min = model(1);
   for (int s = 2; s <= smax; ++s) {
     const double t = model(s);
@@ -920,47 +922,49 @@ template <typename Model> static int best_splits(long long pairs, int smax, int 
   }
   int first = 0;
   for (int s = 1; s <= smax; ++s) {
-    if (model(s) > t_min * 1.03) continue;
+    if (model(s) > t_min * tolerance) continue;
     if (first == 0) first = s;
-    if ((pairs * s) % cus == 0) return s;
+    if ((pairs * s) % cus == 0 && pairs * s / cus <= full_rounds) return s;
   }
   return first;
 }
-static int default_splits_model(long long pairs, int nblocks, int cus, int most) {
+static int default_splits_model(long long pairs, int nblocks, int cus, int most, int rows) {
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
   if (smax > most) smax = most;
-  return best_splits(pairs, smax, cus, [&](int s) { return split_model_us(pairs, nblocks, s, cus); });
+  return best_splits(pairs, smax, cus, 1.005, 1, [&](int s) { return split_model_us(pairs, nblocks, s, cus, rows); });
 }
 
 // The model is evaluated a few hundred times per call; a decode loop asks for the same (pairs, key
 // blocks) at every layer and for the next block count only every 128 tokens, so the last answers are
 // kept per thread.
-int flash_decode_default_splits(int batch, int n, int kv_head_num) {
+int flash_decode_default_splits(int batch, int n, int kv_head_num, int rows) {
+  if (rows > kTaggedRows) rows = kTaggedRows + 1;
   const long long pairs = (long long)batch * kv_head_num;
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys;
   const int cus = device_compute_units();
   struct Memo {
     long long pairs;
     int nblocks, cus, splits;
+    int rows;
   };
   constexpr int kMemo = 8;
   static thread_local Memo memo[kMemo] = {};
   static thread_local unsigned next = 0;
   for (const Memo &e : memo)
-    if (e.splits > 0 && e.pairs == pairs && e.nblocks == nblocks && e.cus == cus) return e.splits;
-  const int s = default_splits_model(pairs, nblocks, cus, kMaxSplits);
-  memo[next++ % kMemo] = Memo{pairs, nblocks, cus, s};
+    if (e.splits > 0 && e.pairs == pairs && e.nblocks == nblocks && e.cus == cus && e.rows == rows) return e.splits;
+  const int s = default_splits_model(pairs, nblocks, cus, kMaxSplits, rows);
+  memo[next++ % kMemo] = Memo{pairs, nblocks, cus, s, rows};
   return s;
 }
 
-int flash_decode_splits_within(int batch, int n, int kv_head_num, size_t bytes) {
-  const int s = flash_decode_default_splits(batch, n, kv_head_num);
+int flash_decode_splits_within(int batch, int n, int kv_head_num, int rows, size_t bytes) {
+  const int s = flash_decode_default_splits(batch, n, kv_head_num, rows);
   if (flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, s) <= bytes) return s;
   int fits = s - 1;
   while (fits > 1 && flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, fits) > bytes) --fits;
   return default_splits_model((long long)batch * kv_head_num, (n + kDecStepKeys - 1) / kDecStepKeys,
-                              device_compute_units(), fits);
+                              device_compute_units(), fits, rows);
 }
 
 // What a call may insist on is counted with coarser figures than the default: 27.7 GB/s per CU in a full round and at most
@@ -971,7 +975,7 @@ size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys, cus = device_compute_units();
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
-  const int s = best_splits(pairs, smax, cus, [&](int splits) {
+  const int s = best_splits(pairs, smax, cus, 1.03, pairs * smax, [&](int splits) {
     const long long full = pairs * splits / cus, rest = pairs * splits % cus;
     const double kb = 2.0 * kRowBytes * kDecStepKeys * ((nblocks + splits - 1) / splits) * 1e-3;
     double t = full * (kb / 27.7 + 3.0);

@@ -41,11 +41,12 @@ int device_compute_units();
 // Split-KV decode.  rows = m * group_size <= 16 query rows per kv head.
 size_t flash_decode_workspace_bytes(int batch, int m, int group_size, int kv_head_num,
                                     int num_splits);
-int flash_decode_default_splits(int batch, int n, int kv_head_num);
+// rows: query rows of a kv head
+int flash_decode_default_splits(int batch, int n, int kv_head_num, int rows);
 int flash_decode_max_default_splits(long long pairs);
 // The best count whose partials fit `bytes`; the size below which a call that leaves the count to the
 // library and has no way to get more is to be refused.
-int flash_decode_splits_within(int batch, int n, int kv_head_num, size_t bytes);
+int flash_decode_splits_within(int batch, int n, int kv_head_num, int rows, size_t bytes);
 size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num);
 // The split count a launch really uses for n keys: at most one split per block of 128 keys.
 int flash_decode_effective_splits(int num_splits, int n);

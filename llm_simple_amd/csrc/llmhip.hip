@@ -96,7 +96,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
   if ((long long)m * group_size <= kMaxDecodeCols) {
     // few query rows: stream the cache once with the split-KV kernel
     const int n_vis = (n < m + offset) ? n : m + offset;  // keys any row can see
-    int splits = flash_decode_default_splits(1, n_vis, kv_head_num);
+    int splits = flash_decode_default_splits(1, n_vis, kv_head_num, m * group_size);
     const size_t need = flash_decode_workspace_bytes(1, m, group_size, kv_head_num, splits);
     if (!need)
       return from_hip(launch_flash_decode(out, q, k, v, nullptr, 0, 1, m, n_vis, offset, n_vis, group_size,
@@ -106,7 +106,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     int rc = scratch_for_locked(
         stream, need, [&] { return flash_decode_least_workspace_bytes(1, n_vis, kv_head_num); }, &ws);
     if (rc != LLMHIP_OK) return rc;
-    if (ws->bytes < need) splits = flash_decode_splits_within(1, n_vis, kv_head_num, ws->bytes);
+    if (ws->bytes < need) splits = flash_decode_splits_within(1, n_vis, kv_head_num, m * group_size, ws->bytes);
     return from_hip(launch_flash_decode(out, q, k, v, ws->ptr, ws->bytes, 1, m, n_vis, offset, n_vis,
                                         group_size, kv_head_num, splits, dt,
                                         as_stream(stream)));
@@ -152,14 +152,14 @@ size_t llmhip_flash_attn_scratch_bytes(int m, int n, int offset, int group_size,
   if ((long long)m * group_size <= kMaxDecodeCols) {
     const int n_vis = (n < m + offset) ? n : m + offset;
     return flash_decode_workspace_bytes(1, m, group_size, kv_head_num,
-                                        flash_decode_default_splits(1, n_vis, kv_head_num));
+                                        flash_decode_default_splits(1, n_vis, kv_head_num, m * group_size));
   }
   return flash_prefill_workspace_bytes(m, n, offset, group_size, kv_head_num);
 }
 
 int llmhip_flash_decode_default_splits(int batch, int n, int kv_head_num) {
   if (batch < 1 || n < 1 || kv_head_num < 1) return LLMHIP_ERR_INVALID_ARG;
-  return flash_decode_default_splits(batch, n, kv_head_num);
+  return flash_decode_default_splits(batch, n, kv_head_num, 1);
 }
 
 size_t llmhip_flash_decode_workspace_bytes(int batch, int group_size, int kv_head_num,
@@ -188,10 +188,10 @@ int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,
   const size_t room = workspace ? workspace_bytes : 0;
   if (num_splits <= 0) {
     // the default count, or the best one the workspace holds, unless that is less than a call may insist on
-    num_splits = flash_decode_default_splits(batch, n, kv_head_num);
+    num_splits = flash_decode_default_splits(batch, n, kv_head_num, group_size);
     if (flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits) > room &&
         flash_decode_least_workspace_bytes(batch, n, kv_head_num) <= room)
-      num_splits = flash_decode_splits_within(batch, n, kv_head_num, room);
+      num_splits = flash_decode_splits_within(batch, n, kv_head_num, group_size, room);
   }
   if (num_splits > kMaxDecodeSplits) num_splits = kMaxDecodeSplits;  // the combine kernel's limit
   const size_t need = flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits);
@@ -213,7 +213,7 @@ int llmhip_flash_decode_gqa_static(void *out, const void *q, const void *k_cache
   if (batch > 65535 || kv_head_num > 65535) return LLMHIP_ERR_UNSUPPORTED;
   if (num_splits <= 0) {
     // the default count, lowered until its partials fit the fixed array (one split needs none)
-    num_splits = flash_decode_default_splits(batch, n, kv_head_num);
+    num_splits = flash_decode_default_splits(batch, n, kv_head_num, group_size);
     while (num_splits > 1 &&
            flash_decode_workspace_bytes(batch, 1, group_size, kv_head_num, num_splits) > kStaticDecodeScratchBytes)
       --num_splits;
@@ -240,7 +240,7 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
   if (head_dim != 128 || group_size > kMaxDecodeCols) return LLMHIP_ERR_UNSUPPORTED;
   if (kv_head_num > 65535) return LLMHIP_ERR_UNSUPPORTED;
   const int n = pos + 1;
-  int splits = flash_decode_default_splits(1, n, kv_head_num);
+  int splits = flash_decode_default_splits(1, n, kv_head_num, group_size);
   const size_t need = flash_decode_workspace_bytes(1, 1, group_size, kv_head_num, splits);
   if (!need)
     return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, nullptr, 0, pos,
@@ -251,7 +251,7 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
   int rc = scratch_for_locked(
       stream, need, [&] { return flash_decode_least_workspace_bytes(1, n, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
-  if (ws->bytes < need) splits = flash_decode_splits_within(1, n, kv_head_num, ws->bytes);
+  if (ws->bytes < need) splits = flash_decode_splits_within(1, n, kv_head_num, group_size, ws->bytes);
   return from_hip(launch_flash_decode_step(out, k_cache, v_cache, freq_cis, in_q, in_k, in_v, ws->ptr, ws->bytes, pos, group_size,
                                            kv_head_num, is_neox_style, splits, dt, as_stream(stream)));
 }
