@@ -288,10 +288,10 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // dims per lane, and PARTS of the fold_parts() parts of its partials, DEPTH in all.  It looks at all of them until it finds the tags
 // at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  False if they were not there after
 // kFoldPolls looks.
-template <typename T, int NW, int DEPTH, int PARTS>
+template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
 __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int b, int kvh, int c0, int rows, int m, int Hkv,
                                             int g) {
-  constexpr int EACH = DEPTH / PARTS, ROUND = PARTS > 1 ? 4 : EACH;
+  constexpr int EACH = DEPTH / PARTS;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
   const int parts = fold_parts(S), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
   const bool mine = wave % at_once < p.fold_rows && c < rows;  // (of the wave)
@@ -445,15 +445,30 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       pair = (int)fast_div(e, f.folders_div);
       b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
       const int c0 = (e - pair * f.folders) * f.fold_rows;
-      auto fold = [&](auto depth, auto parts) {
-        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value>(f, lds, pair, b, pair - b * Hkv, c0, rows, m, Hkv, g);
+      auto fold = [&](auto depth, auto parts, auto round) {
+        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, lds, pair, b, pair - b * Hkv,
+                                                                                                          c0, rows, m, Hkv, g);
       };
       using std::integral_constant;
-      if (NW == 4 && f.num_splits > 64   ? fold(integral_constant<int, 4 * kFoldDepth>(), integral_constant<int, 2>())
-          : NW == 4 && f.num_splits > 32 ? fold(integral_constant<int, 2 * kFoldDepth>(), integral_constant<int, 2>())
-          : NW == 4 && f.num_splits > kMaxFoldSplits ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 2>())
-          : f.num_splits > 4 ? fold(integral_constant<int, kFoldDepth>(), integral_constant<int, 1>())
-                             : fold(integral_constant<int, 4>(), integral_constant<int, 1>()))
+      const integral_constant<int, 1> one;
+      const integral_constant<int, 2> two;
+      const integral_constant<int, 4> four;
+      const integral_constant<int, 8> eight;
+      const integral_constant<int, 16> sixteen;
+      const int S = f.num_splits;
+      bool folded;
+      if constexpr (NW == 4)
+        folded = S > 64                ? fold(integral_constant<int, 32>(), two, four)
+                 : S > 32              ? fold(sixteen, two, four)
+                 : S > kMaxFoldSplits  ? fold(eight, two, four)
+                 : S > 4               ? fold(eight, one, eight)
+                                       : fold(four, one, four);
+      else
+        folded = S > kMaxFoldSplits ? fold(sixteen, four, four)
+                 : S > kFoldDepth   ? fold(sixteen, two, eight)
+                 : S > 4            ? fold(eight, one, eight)
+                                    : fold(four, one, four);
+      if (folded)
         return;
       lone = true;
       split = 0;
@@ -893,7 +908,7 @@ int flash_decode_max_default_splits(long long pairs) {
 // keys, else 2.0 for up to 8 partials, 1.8 for up to 16 and 1.4 beyond (what more of them cost is in the workgroups); more than 8
 // rows are folded by flags and by a second launch, 2.0, 2.6 and 2.1.  Of counts within 0.5 % of the best one that gives every CU one
 // workgroup is taken, else the smallest.  Fitted over 563 shapes of batch 1-16 x 2-32 kv heads x 130-32000 keys and up to 40 counts each: the
-// count chosen is 0.25 % slower than the fastest on average, 0.7 % at the 90th percentile, 9 % at most, where the model before, which
+// count chosen is 0.25 % slower than the fastest on average, 0.7 % at the 90th percentile, 17 % at most (2 x 188 of 32), where the model before, which
 // added whole rounds up and took a fold by folders for a second launch, was 1.2, 4.4 and 18 % (us: 250 keys of 4 kv heads
 // 5.47 -> 4.63, 3 x 4200 of 32 38.6 -> 34.2, 11 x 2983 of 8 28.7 -> 25.3, 6 x 4566 of 8 22.6 -> 20.3).
 static double split_model_us(long long pairs, int nblocks, int s, int cus, int rows) {
@@ -1059,9 +1074,7 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
 
 template <typename T, bool FUSED, FoldMode FOLD>
 static hipError_t launch_decode_f(const DecodeParams &p, bool half, bool many, hipStream_t stream) {
-  if constexpr (FOLD != kNoFold) {  // (blocks of 64 keys come in splits of one, and few enough to be folded)
-    if (half) return launch_decode_t<T, FUSED, 2, false, FOLD>(p, stream);
-  }
+  if (half) return launch_decode_t<T, FUSED, 2, false, FOLD>(p, stream);
   if (many) return launch_decode_t<T, FUSED, 4, true, FOLD>(p, stream);
   return launch_decode_t<T, FUSED, 4, false, FOLD>(p, stream);
 }
@@ -1079,10 +1092,14 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   int nblocks = (p.n + kDecStepKeys - 1) / kDecStepKeys;
   // Short caches: where every workgroup has one block of 128 keys and twice as many workgroups still fit the chip at
   // once, blocks of 64 keys and workgroups of two waves.  Their slots have half the columns, so the
-  // partials take no more room (one column is the flag's: up to 7 query rows).
-  const int half_blocks = (p.n + kDecStepKeys / 2 - 1) / (kDecStepKeys / 2);
-  const bool half = p.num_splits > 1 && p.num_splits == nblocks && p.rows < kDecCols / 2 && half_blocks <= kFoldDepth &&
-                    (long long)p.batch * p.Hkv * half_blocks <= device_compute_units();
+  // partials take no more room (one column is the flag's: up to 7 query rows).  More than 8 such blocks, with some CUs left to
+  // the folders, for the fused step only, where each wave of a CU takes in the query and the table beside its keys (us, blocks of 128 /
+  // 64: 700 keys of 4 kv heads 5.88 / 5.6, 1500 6.28 / 5.83, 1500 of 2 5.95 / 5.54, 1200 of 8 6.21 / 5.91; but unfused 2 x 900 of 4 5.33 /
+  // 5.69, and without CUs for the folders 2000 of 8 6.45 / 6.57).
+  const int half_blocks = (p.n + kDecStepKeys / 2 - 1) / (kDecStepKeys / 2), cus = device_compute_units();
+  const long long half_wgs = (long long)p.batch * p.Hkv * half_blocks;
+  const bool half = p.num_splits > 1 && p.num_splits == nblocks && p.rows < kDecCols / 2 &&
+                    (half_blocks <= kFoldDepth ? half_wgs <= cus : fused && half_blocks <= 2 * kMaxFoldSplits && half_wgs <= cus - cus / 16);
   if (half) {
     p.num_splits = nblocks = half_blocks;
     p.cols = kDecCols / 2;
@@ -1103,7 +1120,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
     if (p.fold == 0) p.fold = launch_number();
     const int parts = fold_parts(p.num_splits);
     const long long idle = device_compute_units() - pairs * p.num_splits;
-    p.fold_rows = (half ? 2 : 4) / (parts > 4 ? 4 : parts);
+    p.fold_rows = half ? (parts > 4 ? 1 : 2) : 4 / (parts > 4 ? 4 : parts);
     while (p.fold_rows > 1 && pairs * ((2 * p.rows + p.fold_rows - 1) / p.fold_rows) <= idle) p.fold_rows /= 2;
     p.folders = (p.rows + p.fold_rows - 1) / p.fold_rows;
     p.folders_div = make_fast_div((uint32_t)p.folders);
