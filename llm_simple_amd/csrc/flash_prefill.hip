@@ -75,7 +75,11 @@ struct PrefillLate {
   float *ws_ml;           // [split][m][H][2]
   int num_splits, first_each, range_keys;
   FastDiv step_div;
-  FastDiv per_split;      // of an XCD's work list: items per key range
+  FastDiv per_split;      // of a work list: items per key range
+  // Packed rows: items, those of an XCD's piece of the list, those of a cluster of tiles of all key ranges and kv heads; tiles of a
+  // cluster and of the last one
+  int items, per_xcd;
+  FastDiv cluster_items, cluster_tiles, last_tiles, splits_div;
   float scale_log2e;
 #ifdef LLMHIP_BENCH
   // measurement library only: workgroup 0 stores {shader-clock ticks, 100 MHz ticks} of its lifetime
@@ -136,6 +140,20 @@ struct PrefillShared {  // the same, unpacked
 template <bool SPLIT>
 __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const PrefillLate &p, int bid, int num_q_tiles, int &tile,
                                                  int &head, int &split) {
+  if (SPLIT && p.per_xcd) {
+    // (cluster of tiles, kv head, key range, tile of the cluster): an XCD has a piece of the list
+    const int i = bid >> 3, idx = (bid & 7) * p.per_xcd + i;
+    if (i >= p.per_xcd || idx >= p.items) return false;
+    const int cluster = (int)fast_div(idx, p.cluster_items), rem = idx - cluster * (int)p.cluster_items.d;
+    const int first = cluster * (int)p.cluster_tiles.d, whole = num_q_tiles - first >= (int)p.cluster_tiles.d;
+    const int size = whole ? (int)p.cluster_tiles.d : (int)p.last_tiles.d;
+    const int group = (int)(whole ? fast_div(rem, p.cluster_tiles) : fast_div(rem, p.last_tiles));
+    const int h = (int)fast_div(group, p.splits_div);
+    split = group - h * p.num_splits;
+    tile = num_q_tiles - 1 - first - (rem - group * size);
+    head = h * e.g;  // first query head of the kv head
+    return true;
+  }
   int idx = bid >> e.xcd_bits, xcd = bid & ((1 << e.xcd_bits) - 1);
   if (idx >= e.second && idx < e.second_end) idx = e.second + e.second_end - 1 - idx;
   idx = (idx << e.sched_shift) + (xcd & ((1 << e.sched_shift) - 1));  // 2^sched_shift XCDs per kv head (one: of several heads)
@@ -975,6 +993,8 @@ __global__ __launch_bounds__(256) void prefill_combine_wide_kernel(addresses_t a
   *reinterpret_cast<u32x2_t *>(out + slot * kRowBytes + d4 * 8) = w;
 }
 
+constexpr int kClusterTiles = 6;
+
 template <typename T, int NW, int KP = 1>
 static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) {
   PrefillParams p = p0;
@@ -984,9 +1004,25 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   int grid, list_heads;
   const int S_ = p.num_splits, share = prefill_xcd_share_log2(p.Hkv);
   p.xcd_bits = p.sched_shift = 0;
+  p.per_xcd = 0;
   if (p.pack) {
     list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
+    // Tiles of a kv head read the same keys.  Dealt one by one, T_ of them meet in 1 / (8 / gcd(kv heads, 8)) of the XCDs; where that puts
+    // no more than two on an XCD, clusters of up to 6 are dealt instead, so that an L2 serves them (attention and combine, us, one by
+    // one / clusters: 14 tokens past 25506 keys of 28 + 4 heads, 2 tiles, 23.9 / 18.5; 17 past 10561 of 12 + 2, 4 tiles, 13.3 / 10.8; 62 past
+    // 30822 of 8 + 1, 16 tiles, 26.5 / 22.9; but 5 tiles of 4 kv heads 15.6 / 16.2, 12 26.5 / 27.9, and with 29 to a cluster 1.25 times).
+    const int heads_xcds = p.Hkv % 8 == 0 ? 8 : p.Hkv % 4 == 0 ? 4 : p.Hkv % 2 == 0 ? 2 : 1;
+    if (T_ > 1 && heads_xcds < 8 && T_ * heads_xcds <= 16) {
+      const int clusters = (T_ + kClusterTiles - 1) / kClusterTiles, each = (T_ + clusters - 1) / clusters;
+      p.items = grid;
+      p.per_xcd = (grid + 7) / 8;
+      grid = 8 * p.per_xcd;
+      p.cluster_items = make_fast_div((uint32_t)(each * p.Hkv * S_));
+      p.cluster_tiles = make_fast_div((uint32_t)each);
+      p.last_tiles = make_fast_div((uint32_t)((T_ - 1) % each + 1));
+      p.splits_div = make_fast_div((uint32_t)S_);
+    }
   } else if (share >= 0) {
     p.xcd_bits = 3;
     p.sched_shift = share;
