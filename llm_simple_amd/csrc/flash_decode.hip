@@ -35,9 +35,12 @@
 // (Fused step, us, the last workgroup to store folds / folders: 384 keys of 2 kv heads 5.52 / 4.85, 512 of 32 5.23 / 5.01, 32768 of 8, with
 // a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1; beyond 32 partials, a combine launch / folders: 4700 keys of
 // 4 kv heads 7.92 / 7.06, 14000 10.45 / 9.62, 31000 15.2 / 14.5, 6000 of 2 7.77 / 6.68, 20000 10.25 / 9.58.)
-// Where the number would be that of a replay, up to 16 partials are folded by the workgroup that finds them all stored: partials,
-// then a flag, then a look at the other flags, then the partials, four round trips to memory.  Beyond that, for more than 8 rows or
-// 128 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
+// More than 8 query rows (a few tokens checked at once) take folders where the room is there, with tags twice that of the partials (rope
+// and attention, us, flags or a combine launch / folders: 2 tokens past 1200 keys of 28 + 4 heads 10.1 / 7.8, past 20000 14.1 / 13.3, 3 past
+// 1500 of 40 + 8 11.1 / 8.4, 12 past 900 of 32 + 32 10.9 / 9.15).
+// Where the number would be that of a replay, or without that room, up to 16 partials are folded by the workgroup that finds them all
+// stored: partials, then a flag, then a look at the other flags, then the partials, four round trips to memory.  Beyond that, or
+// beyond 128 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
 // against 33 at batch 1, 32768 keys.)
 //
 // A short cache is bound by the length of one workgroup's chain, not by bytes: at 32 keys, one sequence, the
@@ -180,7 +183,7 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
 
 constexpr int kMaxFoldSplits = 16, kMaxTaggedSplits = 128;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
-constexpr int kTaggedRows = 8;                    // query rows whose words carry a tag, at most
+constexpr int kFewRows = 8;                       // query rows up to which a row's partials are dealt to parts
 constexpr int kTaggedPairs = 1023;                // (sequence, kv head) pairs, at most
 constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
 #ifdef LLMHIP_BENCH
@@ -189,8 +192,11 @@ constexpr int kFoldPolls = 0;  // (the measurement library's copy: every folder 
 constexpr int kFoldPolls = 1 << 16;  // looks that a folder takes, 0.6 us each
 #endif
 // Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  (The order of the
-// combine launch where they are more than kMaxFoldSplits.)
-__host__ __device__ constexpr int fold_parts(int splits) { return splits <= kFoldDepth ? 1 : splits <= kMaxFoldSplits ? 2 : 8; }
+// combine launch where they are more than kMaxFoldSplits.  More than kFewRows rows leave no groups to deal them to where one
+// workgroup folds by flags.)
+__host__ __device__ constexpr int fold_parts(int splits, int rows) {
+  return splits <= kFoldDepth ? 1 : splits <= kMaxFoldSplits ? (rows > kFewRows ? 1 : 2) : 8;
+}
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
 
@@ -269,7 +275,7 @@ struct RowFold {
   }
 };
 
-// Maximum over each N = 4 or 8 lanes.
+// Maximum over each N = 4, 8 or 16 lanes.
 template <int N> __device__ __forceinline__ float max_of_lanes(float x) {
   auto with = [&](auto control) {
     const int i = __builtin_bit_cast(int, x);
@@ -277,7 +283,8 @@ template <int N> __device__ __forceinline__ float max_of_lanes(float x) {
   };
   with(std::integral_constant<int, 0xB1>());                     // quad_perm: lane ^ 1
   with(std::integral_constant<int, 0x4E>());                     // quad_perm: lane ^ 2
-  if (N == 8) with(std::integral_constant<int, 0x141>());        // row_half_mirror: the other quad
+  if (N >= 8) with(std::integral_constant<int, 0x141>());        // row_half_mirror: the other quad
+  if (N == 16) with(std::integral_constant<int, 0x140>());       // row_mirror: the other half of the row
   return x;
 }
 __device__ __forceinline__ float lane_value(float x, int lane) {
@@ -293,7 +300,7 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int 
                                             int g) {
   constexpr int EACH = DEPTH / PARTS;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
-  const int parts = fold_parts(S), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
+  const int parts = fold_parts(S, rows), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
   const bool mine = wave % at_once < p.fold_rows && c < rows;  // (of the wave)
   const int bytes = S * rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + (size_t)pair * bytes, bytes);
@@ -461,6 +468,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
         folded = S > 64                ? fold(integral_constant<int, 32>(), two, four)
                  : S > 32              ? fold(sixteen, two, four)
                  : S > kMaxFoldSplits  ? fold(eight, two, four)
+                 : S > kFoldDepth && rows > kFewRows ? fold(sixteen, one, sixteen)
                  : S > 4               ? fold(eight, one, eight)
                                        : fold(four, one, four);
       else
@@ -781,11 +789,12 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   __syncthreads();
   if (*all_up == 0) return;
   if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
-  // Every partial of a thread's share is asked for before the first is used.  More rows than folders take leave no groups to deal
-  // the partials of a row to: a group has all of them (15 rows of 12 partials, us, in two parts and four rounds / so in two: 12.65 / 11.2).
+  // Every partial of a thread's share is asked for before the first is used.  More than kFewRows rows have a group each and all their
+  // partials in one round (15 rows of 12 partials, us, in two parts and four rounds / so in two: 12.65 / 11.2).
   constexpr int NG = 2 * NW;
   const int d4 = tid & 31;
-  auto fold = [&](auto depth, int parts) {
+  auto fold = [&](auto depth) {
+    const int parts = fold_parts(p.num_splits, rows);
     constexpr int D = decltype(depth)::value;
     const int at_once = NG / parts, part = (tid >> 5) / at_once;
     for (int c0 = 0; c0 < rows; c0 += at_once) {
@@ -804,10 +813,10 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       if (part == 0 && c < rows) f.template store<T>(p.out, b, m, c, kvh, Hkv, g, p.g_div, d4);
     }
   };
-  if (NW == 4 && rows > kTaggedRows && p.num_splits > kFoldDepth)
-    fold(std::integral_constant<int, kMaxFoldSplits>(), 1);
+  if (NW == 4 && rows > kFewRows && p.num_splits > kFoldDepth)
+    fold(std::integral_constant<int, kMaxFoldSplits>());
   else
-    fold(std::integral_constant<int, kFoldDepth>(), fold_parts(p.num_splits));
+    fold(std::integral_constant<int, kFoldDepth>());
 }
 
 // Folds the splits of one output row (one query row of one head) with the log-sum-exp rule.
@@ -924,7 +933,7 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus, int r
   }
   if (s == 1) return t;
   if (s == nblocks && 2 * s <= kFoldDepth && pairs * (s == 2 ? 6 : 2 * s) <= cus && rows < kDecCols / 2) return t + 0.9;
-  if (rows > kTaggedRows) return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
+  if (rows > kFewRows) return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
   return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 1.8 : 1.4);
 }
 // The smallest count within `tolerance` of the best, or one that fills up to full_rounds rounds exactly.
@@ -954,7 +963,7 @@ static int default_splits_model(long long pairs, int nblocks, int cus, int most,
 // blocks) at every layer and for the next block count only every 128 tokens, so the last answers are
 // kept per thread.
 int flash_decode_default_splits(int batch, int n, int kv_head_num, int rows) {
-  if (rows > kTaggedRows) rows = kTaggedRows + 1;
+  if (rows > kFewRows) rows = kFewRows + 1;
   const long long pairs = (long long)batch * kv_head_num;
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys;
   const int cus = device_compute_units();
@@ -1109,16 +1118,16 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
   FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
-  // Up to 128 partials of up to 8 rows (as many as the room that a call may insist on holds with tags) by folders, as many of them as
+  // Up to 128 partials by folders (more than 8 rows where the room is larger than a call may insist on: with tags they take more), as many of them as
   // the CUs that the other workgroups leave idle can take, down to one row each.
   // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones.
   const long long pairs = (long long)p.batch * p.Hkv;
   const size_t tagged = (size_t)pairs * p.num_splits * p.rows * kTaggedBytes;
-  if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && p.rows <= kTaggedRows && pairs <= kTaggedPairs &&
+  if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && pairs <= kTaggedPairs &&
       tagged <= workspace_bytes && !may_be_capturing(stream)) {
     how = kFoldByTags;
     if (p.fold == 0) p.fold = launch_number();
-    const int parts = fold_parts(p.num_splits);
+    const int parts = fold_parts(p.num_splits, p.rows);
     const long long idle = device_compute_units() - pairs * p.num_splits;
     p.fold_rows = half ? (parts > 4 ? 1 : 2) : 4 / (parts > 4 ? 4 : parts);
     while (p.fold_rows > 1 && pairs * ((2 * p.rows + p.fold_rows - 1) / p.fold_rows) <= idle) p.fold_rows /= 2;
