@@ -192,10 +192,10 @@ constexpr int kFoldPolls = 0;  // (the measurement library's copy: every folder 
 constexpr int kFoldPolls = 1 << 16;  // looks that a folder takes, 0.6 us each
 #endif
 // Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  (The order of the
-// combine launch where they are more than kMaxFoldSplits.  More than kFewRows rows leave no groups to deal them to where one
-// workgroup folds by flags.)
+// combine launch where they are more than kMaxFoldSplits, or there is no column left for a flag.  More than kFewRows rows leave no
+// groups to deal them to where one workgroup folds by flags.)
 __host__ __device__ constexpr int fold_parts(int splits, int rows) {
-  return splits <= kFoldDepth ? 1 : splits <= kMaxFoldSplits ? (rows > kFewRows ? 1 : 2) : 8;
+  return splits <= kFoldDepth ? 1 : splits > kMaxFoldSplits || rows == kDecCols ? 8 : rows > kFewRows ? 1 : 2;
 }
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
@@ -467,8 +467,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       if constexpr (NW == 4)
         folded = S > 64                ? fold(integral_constant<int, 32>(), two, four)
                  : S > 32              ? fold(sixteen, two, four)
-                 : S > kMaxFoldSplits  ? fold(eight, two, four)
-                 : S > kFoldDepth && rows > kFewRows ? fold(sixteen, one, sixteen)
+                 : S > kMaxFoldSplits || (rows == kDecCols && S > kFoldDepth) ? fold(eight, two, four)
+                 : S > kFoldDepth && rows > kFewRows                          ? fold(sixteen, one, sixteen)
                  : S > 4               ? fold(eight, one, eight)
                                        : fold(four, one, four);
       else
