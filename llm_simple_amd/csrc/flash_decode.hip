@@ -914,8 +914,7 @@ int flash_decode_max_default_splits(long long pairs) {
 // streams the more the fewer they are (32 KiB in flight, over a latency that grows with the load); beyond that a CU streams 27.9
 // GB/s (all 256 of an MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads) and the launch takes
 // something between the rounds that the fullest CU runs and the mean of all.  A fold by folders costs 0.9 us in blocks of 64
-// keys, else 2.0 for up to 8 partials, 1.8 for up to 16 and 1.4 beyond (what more of them cost is in the workgroups); more than 8
-// rows are folded by flags and by a second launch, 2.0, 2.6 and 2.1.  Of counts within 0.5 % of the best one that gives every CU one
+// keys, else 2.0 for up to 8 partials, 1.8 for up to 16 and 1.4 beyond (what more of them cost is in the workgroups).  Of counts within 0.5 % of the best one that gives every CU one
 // workgroup is taken, else the smallest.  Fitted over 563 shapes of batch 1-16 x 2-32 kv heads x 130-32000 keys and up to 40 counts each: the
 // count chosen is 0.25 % slower than the fastest on average, 0.7 % at the 90th percentile, 17 % at most (2 x 188 of 32), where the model before, which
 // added whole rounds up and took a fold by folders for a second launch, was 1.2, 4.4 and 18 % (us: 250 keys of 4 kv heads
@@ -933,7 +932,6 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus, int r
   }
   if (s == 1) return t;
   if (s == nblocks && 2 * s <= kFoldDepth && pairs * (s == 2 ? 6 : 2 * s) <= cus && rows < kDecCols / 2) return t + 0.9;
-  if (rows > kFewRows) return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 2.6 : 2.1);
   return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 1.8 : 1.4);
 }
 // The smallest count within `tolerance` of the best, or one that fills up to full_rounds rounds exactly.
@@ -963,7 +961,7 @@ static int default_splits_model(long long pairs, int nblocks, int cus, int most,
 // blocks) at every layer and for the next block count only every 128 tokens, so the last answers are
 // kept per thread.
 int flash_decode_default_splits(int batch, int n, int kv_head_num, int rows) {
-  if (rows > kFewRows) rows = kFewRows + 1;
+  rows = rows < kDecCols / 2 ? 1 : kDecCols;  // (what the model tells apart)
   const long long pairs = (long long)batch * kv_head_num;
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys;
   const int cus = device_compute_units();
