@@ -95,12 +95,13 @@ struct DecodeParams : DecodeLate {
   const void *q, *k, *v;
   const void *freq_row, *new_k, *new_v;
   int batch, m, n, offset;
-  int64_t kv_seq_stride;
+  int64_t kv_seq_stride;  // 0: the sequences are tiles of m tokens of one
+  int last_token;         // where the last sequence or tile begins: a last tile that would be short begins earlier
   int g, Hkv, rows;
   int is_neox;
   bool fused;
 };
-// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
+// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8 | last_token << 16, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
 // up) << 10 (pairs = batch * Hkv, where the partials are folded by tags: at most kTaggedPairs); c: n, Hkv | g << 16 | is_neox << 31
 struct DecodeEarly {
   addresses_t a;
@@ -110,7 +111,7 @@ struct DecodeEarly {
     a = addresses_t{address(p.q), address(p.k), address(p.v), p.fused ? address(p.freq_row) : (uint64_t)p.kv_seq_stride};
     const uint64_t nk = address(p.new_k), nv = address(p.new_v);
     b = p.fused ? u32x4_t{(uint32_t)nk, (uint32_t)(nk >> 32), (uint32_t)nv, (uint32_t)(nv >> 32)}
-                : u32x4_t{(uint32_t)(p.rows | p.m << 8), 65536u / p.g + 1, (uint32_t)p.offset,
+                : u32x4_t{(uint32_t)(p.rows | p.m << 8) | (uint32_t)p.last_token << 16, 65536u / p.g + 1, (uint32_t)p.offset,
                           (uint32_t)(p.batch * p.Hkv) | ((1u << 20) + p.Hkv - 1) / p.Hkv << 10};
     c = u32x2_t{(uint32_t)p.n, (uint32_t)p.Hkv | (uint32_t)p.g << 16 | (uint32_t)p.is_neox << 31};
   }
@@ -265,13 +266,13 @@ struct RowFold {
     __syncthreads();
   }
   template <typename T>
-  __device__ __forceinline__ void store(char *out, int b, int m, int c, int kvh, int Hkv, int g, const FastDiv &g_div, int d4) {
+  __device__ __forceinline__ void store(char *out, int token, int c, int kvh, int Hkv, int g, const FastDiv &g_div, int d4) {
     const int r = (int)fast_div(c, g_div);
     const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
     u32x2_t w;
     w[0] = Elem<T>::pack2(acc[0] * inv, acc[1] * inv);
     w[1] = Elem<T>::pack2(acc[2] * inv, acc[3] * inv);
-    *reinterpret_cast<u32x2_t *>(out + (((size_t)b * m + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
+    *reinterpret_cast<u32x2_t *>(out + (((size_t)token + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
   }
 };
 
@@ -296,7 +297,7 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  False if they were not there after
 // kFoldPolls looks.
 template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
-__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int b, int kvh, int c0, int rows, int m, int Hkv,
+__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int token, int kvh, int c0, int rows, int Hkv,
                                             int g) {
   constexpr int EACH = DEPTH / PARTS;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
@@ -393,7 +394,7 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int 
   if (mine && part == 0 && there) {
     const int r = (int)fast_div(c, p.g_div);
     const float inv = (L[0] > 0.0f) ? 1.0f / L[0] : 0.0f;
-    char *row = p.out + (((size_t)b * m + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes;
+    char *row = p.out + (((size_t)token + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes;
     *reinterpret_cast<uint32_t *>(row + (lane & 15) * 16 + (lane >> 4) * 4) = Elem<T>::pack2(x[0] * inv, y[0] * inv);
   }
   __syncthreads();
@@ -433,7 +434,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   using E = Elem<T>;
   const int n = ec[0], Hkv = ec[1] & 0xffffu, g = ec[1] >> 16 & 0xffu, H = g * Hkv;
   const bool is_neox = ec[1] >> 31;
-  const int rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8, offset = FUSED ? n - 1 : (int)eb[2];
+  const int rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8 & 0xffu;
+  auto token_of = [&](int seq) { return FUSED ? 0 : min(seq * m, (int)(eb[0] >> 16)); };  // first token of a sequence, or of a tile of one
   const int fused_pos = n - 1;
   constexpr int kStepKeys = NW * kDecWaveKeys;
   __shared__ __attribute__((aligned(16))) char lds[2 * NW * kDecWaveLds];
@@ -453,8 +455,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
       const int c0 = (e - pair * f.folders) * f.fold_rows;
       auto fold = [&](auto depth, auto parts, auto round) {
-        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, lds, pair, b, pair - b * Hkv,
-                                                                                                          c0, rows, m, Hkv, g);
+        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, lds, pair, token_of(b), pair - b * Hkv,
+                                                                                                          c0, rows, Hkv, g);
       };
       using std::integral_constant;
       const integral_constant<int, 1> one;
@@ -484,6 +486,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
     b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
     kvh = pair - b * Hkv;
   }
+  const int token = token_of(b);
+  const int offset = FUSED ? n - 1 : (int)eb[2] + (ea[3] == 0 ? token : 0);
   const DecodeLate p = FOLD == kFoldByTags ? fetch_late() : late;
   const int num_splits = lone ? 1 : p.num_splits;
 
@@ -505,7 +509,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   f32x4_t tab[8];
   u32x4_t new_v;
   {
-    const char *qp = at_address<const char>(ea[0]) + (size_t)b * m * H * kRowBytes;
+    const char *qp = at_address<const char>(ea[0]) + (size_t)token * H * kRowBytes;
     uint32_t qo = (c_row * H + c_head) * kRowBytes + cg * 16;
     if (FUSED) {
       new_k_row = at_address<const char>(eb[0] | (uint64_t)eb[1] << 32) + kvh * kRowBytes;
@@ -740,7 +744,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
     if (FOLD == kNoFold ? num_splits == 1 : lone) {
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
       const int r = (int)fast_div(c, p.g_div), hq = c - r * g;
-      char *op = p.out + (((size_t)b * m + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
+      char *op = p.out + (((size_t)token + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
       u32x4_t w;
 #pragma unroll
       for (int j = 0; j < 4; ++j) w[j] = E::pack2(acc[2 * j] * inv, acc[2 * j + 1] * inv);
@@ -810,7 +814,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       }
       f.take(ml, ov, part, parts, p.num_splits);
       if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
-      if (part == 0 && c < rows) f.template store<T>(p.out, b, m, c, kvh, Hkv, g, p.g_div, d4);
+      if (part == 0 && c < rows) f.template store<T>(p.out, token, c, kvh, Hkv, g, p.g_div, d4);
     }
   };
   if (NW == 4 && rows > kFewRows && p.num_splits > kFoldDepth)
@@ -827,7 +831,7 @@ constexpr int kMaxSplits = 256;
 
 template <typename T>
 __global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a, u32x4_t size, u32x2_t heads) {
-  // a: partials, their maxima and sums, out; size: splits, columns of a slot, Hkv, m; heads: g, 2^16 / g + 1
+  // a: partials, their maxima and sums, out, last_token; size: splits, columns of a slot, Hkv, m; heads: g, 2^16 / g + 1
   using E = Elem<T>;
   const float *ws_o = at_address<const float>(a[0]), *ws_ml = at_address<const float>(a[1]);
   char *out = at_address<char>(a[2]);
@@ -897,7 +901,8 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a
   u32x2_t w;
   w[0] = E::pack2(tot[0] * inv, tot[1] * inv);
   w[1] = E::pack2(tot[2] * inv, tot[3] * inv);
-  *reinterpret_cast<u32x2_t *>(out + (((size_t)b * m + r) * H + kvh * g + hq) * kRowBytes + d4 * 8) = w;
+  const size_t token = min((unsigned)(b * m), (unsigned)a[3]);
+  *reinterpret_cast<u32x2_t *>(out + ((token + r) * H + kvh * g + hq) * kRowBytes + d4 * 8) = w;
 }
 
 // Largest split count the default rule considers for batch * kv heads = pairs (any KV length): one
@@ -1073,7 +1078,7 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
   hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream,
-                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), 0},
+                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), (uint64_t)p.last_token},
                      u32x4_t{(uint32_t)p.num_splits, (uint32_t)p.cols, (uint32_t)p.Hkv, (uint32_t)p.m},
                      u32x2_t{(uint32_t)p.g, 65536u / p.g + 1});
   return hipGetLastError();
@@ -1157,9 +1162,46 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
   p.n = n;
   p.offset = offset;
   p.kv_seq_stride = kv_seq_stride;
+  p.last_token = (batch - 1) * m;
   p.g = group_size;
   p.Hkv = kv_head_num;
   p.rows = m * group_size;
+  return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, false, stream);
+}
+
+int flash_decode_tiles(int m, int group_size) {
+  const int most = kDecCols / group_size;
+  return (m + most - 1) / most;
+}
+
+// Tiles read their keys each for itself, so that it is the short calls that they are for, those that wait for one workgroup's chain and
+// the fold: up to 40000 keys of all tiles and kv heads, and from where a chunk's workgroups of all keys take longer (attention, us,
+// key ranges and a combine launch / tiles: 3 tokens past 1000 keys of 28 + 4 heads 8.13 / 5.89, 8 past 2000 8.62 / 7.75, 6 past 1000 of 12 + 2
+// 7.95 / 5.60, 4 past 4000 8.17 / 7.04, 6 past 2000 of 40 + 8 8.69 / 7.84; but 6 past 4000 of 28 + 4 8.92 / 9.50 (49000), 12 past 500 of 40 +
+// 8 6.43 / 6.80, and of 32 heads of one kv head each 32 past 500 7.2 / 8.35).
+bool flash_decode_takes_tiles(int m, int n_vis, int group_size, int kv_head_num) {
+  if (group_size < 2 || group_size > kDecCols || m > 8 * kDecCols || prefill_is_prompt(m, n_vis)) return false;
+  const int tiles = flash_decode_tiles(m, group_size);
+  const long long pairs = (long long)tiles * kv_head_num;
+  return tiles <= 8 && pairs * n_vis <= 40000 && n_vis >= 33 * (pairs - 8);
+}
+
+hipError_t launch_flash_decode_tiles(void *out, const void *q, const void *k, const void *v, void *workspace, size_t workspace_bytes,
+                                     int m, int n, int offset, int group_size, int kv_head_num, int num_splits, int dt,
+                                     hipStream_t stream) {
+  DecodeParams p = {};
+  p.q = q;
+  p.k = k;
+  p.v = v;
+  p.out = static_cast<char *>(out);
+  p.batch = flash_decode_tiles(m, group_size);
+  p.m = (m + p.batch - 1) / p.batch;
+  p.last_token = m - p.m;
+  p.n = n;
+  p.offset = offset;
+  p.g = group_size;
+  p.Hkv = kv_head_num;
+  p.rows = p.m * group_size;
   return launch_decode_impl(p, workspace, workspace_bytes, num_splits, dt, false, stream);
 }
 

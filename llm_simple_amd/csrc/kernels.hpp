@@ -55,6 +55,14 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
                                int64_t kv_seq_stride, int group_size, int kv_head_num,
                                int num_splits, int dt, hipStream_t stream);
 
+// m tokens of one sequence with more query rows than 16: as tiles of up to 16 rows, each with workgroups of its own, over
+// visible keys n.  Partials as of flash_decode_tiles(m, group_size) sequences.
+int flash_decode_tiles(int m, int group_size);
+bool flash_decode_takes_tiles(int m, int n_vis, int group_size, int kv_head_num);
+hipError_t launch_flash_decode_tiles(void *out, const void *q, const void *k, const void *v, void *workspace, size_t workspace_bytes,
+                                     int m, int n, int offset, int group_size, int kv_head_num, int num_splits, int dt,
+                                     hipStream_t stream);
+
 // One decode step of one sequence, rotary embedding and cache append fused into the decode kernel:
 // q and the new K row are rotated with row `pos` of the table as they are loaded, the workgroups that own
 // the last key range write row pos of both caches, attention runs over rows [0, pos].

@@ -111,6 +111,19 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
                                         group_size, kv_head_num, splits, dt,
                                         as_stream(stream)));
   }
+  const int n_vis = (n < m + offset) ? n : m + offset;
+  if (flash_decode_takes_tiles(m, n_vis, group_size, kv_head_num)) {
+    // some more of them over a short cache: the same in tiles of rows, if the scratch is there or can be had
+    const int tiles = flash_decode_tiles(m, group_size);
+    const int splits = flash_decode_default_splits(tiles, n_vis, kv_head_num, kMaxDecodeCols);
+    const size_t need = flash_decode_workspace_bytes(tiles, m, group_size, kv_head_num, splits);
+    std::lock_guard<std::mutex> lk(g_scratch_mu);
+    StreamScratch *ws = nullptr;
+    if (need) (void)scratch_for_locked(stream, need, [] { return (size_t)0; }, &ws);
+    if (!need || ws->bytes >= need)
+      return from_hip(launch_flash_decode_tiles(out, q, k, v, need ? ws->ptr : nullptr, need ? ws->bytes : 0, m, n_vis, offset,
+                                                group_size, kv_head_num, splits, dt, as_stream(stream)));
+  }
   // a chunk of few rows over a long cache is split over the key range: fp32 partials in the
   // per-stream scratch
   const size_t need = flash_prefill_workspace_bytes(m, n, offset, group_size, kv_head_num);
@@ -153,6 +166,12 @@ size_t llmhip_flash_attn_scratch_bytes(int m, int n, int offset, int group_size,
     const int n_vis = (n < m + offset) ? n : m + offset;
     return flash_decode_workspace_bytes(1, m, group_size, kv_head_num,
                                         flash_decode_default_splits(1, n_vis, kv_head_num, m * group_size));
+  }
+  const int n_vis = (n < m + offset) ? n : m + offset;
+  if (flash_decode_takes_tiles(m, n_vis, group_size, kv_head_num)) {
+    const int tiles = flash_decode_tiles(m, group_size);
+    return flash_decode_workspace_bytes(tiles, m, group_size, kv_head_num,
+                                        flash_decode_default_splits(tiles, n_vis, kv_head_num, kMaxDecodeCols));
   }
   return flash_prefill_workspace_bytes(m, n, offset, group_size, kv_head_num);
 }
