@@ -37,6 +37,8 @@ typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
 constexpr int kHeadDim = 128;         // every supported model: hidden / n_heads == 128
 constexpr int kRowBytes = kHeadDim * 2;  // one head row of 16-bit elements
+// 1/sqrt(head dim) of the scores, and the logarithm's base: exponents are of 2
+constexpr float kScaleLog2e = 1.4426950408889634f / 11.3137084989847604f;
 
 // Data type numbering of the reference (prebuild/defs.hpp:8-18).
 constexpr int kDtFloat16 = 4;
@@ -121,7 +123,9 @@ template <int I, int N, typename F> __device__ __forceinline__ void static_for(F
 // Kernel arguments.  Scalars and vectors among the first 14 words are in a kernel's registers when it starts (Makefile); a
 // struct is fetched from memory, 0.2 us before the first load of a launch can go out (a token's projections, W from HBM, us,
 // struct / registers: 512 x 3584 3.69 / 3.51, 3584 x 3584 6.25 / 6.03; rope and attention of 256 tokens of 32 heads 10.23 / 9.80).
-// So what the first loads need goes there, in few vectors: each argument costs the host too (eleven scalars 0.2 us).
+// So what the first loads need goes there, in few vectors: each argument costs the host too (eleven scalars 0.2 us), and so does each
+// 64-byte line of them, by processes 0 or up to 0.5 us a launch (prompts of 40 tokens, two launches: 6.4 us in some processes; in others
+// 7.2 with two lines of arguments to attention, 8.2 with four).
 typedef __attribute__((ext_vector_type(4))) uint64_t addresses_t;
 inline uint64_t address(const void *p) { return reinterpret_cast<uintptr_t>(p); }
 template <typename P> __device__ __forceinline__ P *at_address(uint64_t a) {

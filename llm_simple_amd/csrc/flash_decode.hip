@@ -80,9 +80,6 @@ struct DecodeLate {
   float *ws_ml;  // [batch][Hkv][splits][cols][2]; fold: the last column's place is the flag of the split
   int num_splits;
   int iters_each, iters_rest;  // blocks per split: iters_each, one more for the first iters_rest splits
-  FastDiv g_div;
-  float scale_log2e;
-  int cols;       // columns of a partial's slot: 16, or 8 (see launch_decode_impl)
   int fold_rows, folders;  // by tags: rows of a folder, folders of a (sequence, kv head)
   FastDiv folders_div;
   uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial
@@ -100,6 +97,7 @@ struct DecodeParams : DecodeLate {
   int g, Hkv, rows;
   int is_neox;
   bool fused;
+  int cols;  // columns of a partial's slot: 16, or 8 of workgroups of two waves
 };
 // a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8 | last_token << 16, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
 // up) << 10 (pairs = batch * Hkv, where the partials are folded by tags: at most kTaggedPairs); c: n, Hkv | g << 16 | is_neox << 31
@@ -266,8 +264,7 @@ struct RowFold {
     __syncthreads();
   }
   template <typename T>
-  __device__ __forceinline__ void store(char *out, int token, int c, int kvh, int Hkv, int g, const FastDiv &g_div, int d4) {
-    const int r = (int)fast_div(c, g_div);
+  __device__ __forceinline__ void store(char *out, int token, int c, int kvh, int Hkv, int g, int r, int d4) {
     const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
     u32x2_t w;
     w[0] = Elem<T>::pack2(acc[0] * inv, acc[1] * inv);
@@ -297,7 +294,7 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  False if they were not there after
 // kFoldPolls looks.
 template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
-__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int pair, int token, int kvh, int c0, int rows, int Hkv,
+__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, uint32_t row_part, char *lds, int pair, int token, int kvh, int c0, int rows, int Hkv,
                                             int g) {
   constexpr int EACH = DEPTH / PARTS;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
@@ -392,7 +389,7 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, char *lds, int 
     }
   }
   if (mine && part == 0 && there) {
-    const int r = (int)fast_div(c, p.g_div);
+    const int r = (int)(c * row_part >> 16);  // (c / g)
     const float inv = (L[0] > 0.0f) ? 1.0f / L[0] : 0.0f;
     char *row = p.out + (((size_t)token + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes;
     *reinterpret_cast<uint32_t *>(row + (lane & 15) * 16 + (lane >> 4) * 4) = Elem<T>::pack2(x[0] * inv, y[0] * inv);
@@ -435,6 +432,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   const int n = ec[0], Hkv = ec[1] & 0xffffu, g = ec[1] >> 16 & 0xffu, H = g * Hkv;
   const bool is_neox = ec[1] >> 31;
   const int rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8 & 0xffu;
+  const uint32_t row_part = FUSED ? 0u : eb[1];  // (of a column, 16 bits on: its query row)
+  constexpr int cols = NW == 2 ? kDecCols / 2 : kDecCols;
   auto token_of = [&](int seq) { return FUSED ? 0 : min(seq * m, (int)(eb[0] >> 16)); };  // first token of a sequence, or of a tile of one
   const int fused_pos = n - 1;
   constexpr int kStepKeys = NW * kDecWaveKeys;
@@ -455,7 +454,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
       const int c0 = (e - pair * f.folders) * f.fold_rows;
       auto fold = [&](auto depth, auto parts, auto round) {
-        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, lds, pair, token_of(b), pair - b * Hkv,
+        return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, row_part, lds, pair, token_of(b), pair - b * Hkv,
                                                                                                           c0, rows, Hkv, g);
       };
       using std::integral_constant;
@@ -633,7 +632,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       float mloc = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
                          fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
       mloc = quad_max(mloc);
-      const float m_new = fmaxf(m_run, mloc * p.scale_log2e);
+      const float m_new = fmaxf(m_run, mloc * kScaleLog2e);
       const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
       if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {
         const float alpha = fast_exp2(m_run - m_use);
@@ -647,7 +646,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
 #pragma unroll
       for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[blk][i] = fast_exp2(__builtin_fmaf(s[blk][i], p.scale_log2e, -m_use));
+        for (int i = 0; i < 4; ++i) s[blk][i] = fast_exp2(__builtin_fmaf(s[blk][i], kScaleLog2e, -m_use));
       // P^T as B operand: slot e<4 -> block 0 key 4cg+e, e>=4 -> block 1 key 4cg+e-4
       u32x4_t pf;
       pf[0] = E::pack2(s[0][0], s[0][1]);
@@ -707,7 +706,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   __syncthreads();
 
   const size_t pair = (size_t)b * Hkv + kvh;
-  const int pair_slots = p.num_splits * p.cols;
+  const int pair_slots = p.num_splits * cols;
   const __amdgpu_buffer_rsrc_t po = byte_buffer(p.ws_o + pair * pair_slots * kHeadDim, pair_slots * kHeadDim * 4);
   const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
   const int tagged_bytes = p.num_splits * rows * kTaggedBytes;
@@ -743,7 +742,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
     }
     if (FOLD == kNoFold ? num_splits == 1 : lone) {
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-      const int r = (int)fast_div(c, p.g_div), hq = c - r * g;
+      const int r = (int)(c * row_part >> 16), hq = c - r * g;
       char *op = p.out + (((size_t)token + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
       u32x4_t w;
 #pragma unroll
@@ -751,7 +750,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       *reinterpret_cast<u32x4_t *>(op) = w;
       continue;
     }
-    const int slot = split * p.cols + c;
+    const int slot = split * cols + c;
     const f32x4_t a0 = {acc[0], acc[1], acc[2], acc[3]}, a1 = {acc[4], acc[5], acc[6], acc[7]};
     const u32x2_t ml = {__builtin_bit_cast(uint32_t, M), __builtin_bit_cast(uint32_t, L)};
     if constexpr (FOLD == kFoldByTags) {
@@ -782,17 +781,17 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   unsigned *all_up = reinterpret_cast<unsigned *>(lds);
   const u32x2_t up = {(uint32_t)p.fold, (uint32_t)(p.fold >> 32)};
   if (wave == 0) {
-    const int my_flag = (split * p.cols + p.cols - 1) * 8;
+    const int my_flag = (split * cols + cols - 1) * 8;
     if (lane == 0) store_device(pml, my_flag, up);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const u32x2_t f = load_device2(pml, (min(lane, p.num_splits - 1) * p.cols + p.cols - 1) * 8);
+    const u32x2_t f = load_device2(pml, (min(lane, p.num_splits - 1) * cols + cols - 1) * 8);
     const bool down = f[0] != up[0] || f[1] != up[1];
     if (lane == 0) *all_up = 0;
     if (__builtin_amdgcn_ballot_w64(down) == 0 && lane == 0) *all_up = 1;
   }
   __syncthreads();
   if (*all_up == 0) return;
-  if (tid < p.num_splits) store_device(pml, (tid * p.cols + p.cols - 1) * 8, u32x2_t{0u, 0u});
+  if (tid < p.num_splits) store_device(pml, (tid * cols + cols - 1) * 8, u32x2_t{0u, 0u});
   // Every partial of a thread's share is asked for before the first is used.  More than kFewRows rows have a group each and all their
   // partials in one round (15 rows of 12 partials, us, in two parts and four rounds / so in two: 12.65 / 11.2).
   constexpr int NG = 2 * NW;
@@ -808,13 +807,13 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       f32x4_t ov[D];
 #pragma unroll
       for (int j = 0; j < D; ++j) {
-        const int slot = min(part + parts * j, p.num_splits - 1) * p.cols + min(c, rows - 1);
+        const int slot = min(part + parts * j, p.num_splits - 1) * cols + min(c, rows - 1);
         ml[j] = load_device2(pml, slot * 8);
         ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
       }
       f.take(ml, ov, part, parts, p.num_splits);
       if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
-      if (part == 0 && c < rows) f.template store<T>(p.out, token, c, kvh, Hkv, g, p.g_div, d4);
+      if (part == 0 && c < rows) f.template store<T>(p.out, token, c, kvh, Hkv, g, (int)(c * row_part >> 16), d4);
     }
   };
   if (NW == 4 && rows > kFewRows && p.num_splits > kFoldDepth)
@@ -1137,8 +1136,6 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
     p.folders = (p.rows + p.fold_rows - 1) / p.fold_rows;
     p.folders_div = make_fast_div((uint32_t)p.folders);
   }
-  p.g_div = make_fast_div((uint32_t)p.g);
-  p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
   p.ws_o = static_cast<float *>(workspace);
   p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;

@@ -62,29 +62,45 @@ constexpr int kTileN = 64;                      // keys per LDS tile (128 where 
 constexpr int kTileBytes = kTileN * kRowBytes;  // 16 KiB
 constexpr float kLazyLog2 = 8.0f;                // rescale threshold, log2 units
 constexpr int kMaxPrefillSplits = 128;           // key ranges per call
+constexpr int kWholeRange = 0x7fffffc0;          // keys of a range without an end
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
 // What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way -- except with SPLIT, where
-// the key range (per_split and what stands before it) is needed for the first address and waited for.
+// the key range (num_splits and what stands behind it) is needed for the first address and waited for.
 struct PrefillLate {
   char *out;
-  // Key-range split (chunked prefill: few query rows over a long cache).  Split s covers the key tiles s * first_each,
-  // then every step_div.d-th, up to range_keys keys of them (see launch_prefill_t); with more than one split every workgroup
-  // leaves an fp32 partial (reference maximum, sum, unnormalised O) that prefill_combine_kernel folds.
-  float *ws_o;            // [split][m][H][128]
-  float *ws_ml;           // [split][m][H][2]
+  // Key-range split (chunked prefill: few query rows over a long cache).  Split s of S covers the key tiles s * first_each,
+  // then every following one, up to range_keys keys of them, or, if range_keys is kWholeRange, every S-th (see launch_prefill_t); with more
+  // than one split every workgroup leaves an fp32 partial (reference maximum, sum, unnormalised O) that prefill_combine_kernel folds.
+  float *ws_o;            // [split][m][H][128], then maxima and sums [split][m][H][2]
   int num_splits, first_each, range_keys;
-  FastDiv step_div;
-  FastDiv per_split;      // of a work list: items per key range
-  // Packed rows: items, those of an XCD's piece of the list, those of a cluster of tiles of all key ranges and kv heads; tiles of a
-  // cluster and of the last one
-  int items, per_xcd;
-  FastDiv cluster_items, cluster_tiles, last_tiles, splits_div;
-  float scale_log2e;
+  // Packed rows whose tiles are dealt to XCDs in clusters: items of an XCD's piece of the list (else 0), tiles of a cluster and, 8 bits on, of
+  // the last one, 2^16 over either (rounded up)
+  int per_xcd;
+  uint32_t tiles, each_part, last_part;
+  FastDiv splits_div, per_list;  // items per key range of an XCD's work list, or per cluster of all key ranges and kv heads
 #ifdef LLMHIP_BENCH
   // measurement library only: workgroup 0 stores {shader-clock ticks, 100 MHz ticks} of its lifetime
   unsigned long long *clock_probe;
 #endif
+};
+#ifndef LLMHIP_BENCH
+static_assert(sizeof(PrefillLate) <= 72, "with what stands before it two lines of 64 bytes (common.hpp)");
+#endif
+// What an unsplit launch is told of it.
+struct PrefillBrief {
+  char *out;
+#ifdef LLMHIP_BENCH
+  unsigned long long *clock_probe;
+#endif
+  __host__ __device__ operator PrefillLate() const {
+    PrefillLate p = {};
+    p.out = out;
+#ifdef LLMHIP_BENCH
+    p.clock_probe = clock_probe;
+#endif
+    return p;
+  }
 };
 struct PrefillParams : PrefillLate {
   const void *q, *k, *v;
@@ -143,12 +159,10 @@ __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const P
   if (SPLIT && p.per_xcd) {
     // (cluster of tiles, kv head, key range, tile of the cluster): an XCD has a piece of the list
     const int i = bid >> 3, idx = (bid & 7) * p.per_xcd + i;
-    if (i >= p.per_xcd || idx >= p.items) return false;
-    const int cluster = (int)fast_div(idx, p.cluster_items), rem = idx - cluster * (int)p.cluster_items.d;
-    const int first = cluster * (int)p.cluster_tiles.d, whole = num_q_tiles - first >= (int)p.cluster_tiles.d;
-    const int size = whole ? (int)p.cluster_tiles.d : (int)p.last_tiles.d;
-    const int group = (int)(whole ? fast_div(rem, p.cluster_tiles) : fast_div(rem, p.last_tiles));
-    const int h = (int)fast_div(group, p.splits_div);
+    if (i >= p.per_xcd || idx >= num_q_tiles * e.Hkv * p.num_splits) return false;
+    const int each = p.tiles & 0xffu, cluster = (int)fast_div(idx, p.per_list), rem = idx - cluster * (int)p.per_list.d;
+    const int first = cluster * each, whole = num_q_tiles - first >= each, size = whole ? each : (int)(p.tiles >> 8);
+    const int group = (int)((uint32_t)rem * (whole ? p.each_part : p.last_part) >> 16), h = (int)fast_div(group, p.splits_div);
     split = group - h * p.num_splits;
     tile = num_q_tiles - 1 - first - (rem - group * size);
     head = h * e.g;  // first query head of the kv head
@@ -162,9 +176,9 @@ __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const P
   int rem = idx;
   split = 0;
   if (SPLIT) {
-    if (idx >= (int)p.per_split.d * p.num_splits) return false;
-    split = (int)fast_div(idx, p.per_split);
-    rem = idx - split * (int)p.per_split.d;
+    if (idx >= (int)p.per_list.d * p.num_splits) return false;
+    split = (int)fast_div(idx, p.per_list);
+    rem = idx - split * (int)p.per_list.d;
   }
   const int t = (int)fast_div(rem, e.list_heads);
   if (t >= num_q_tiles) return false;
@@ -623,7 +637,9 @@ template <int NW, int TN, bool NT> struct DirectLoader {
 // 128 keys; what they have is merged through LDS at the end.
 // ---------------------------------------------------------------------------
 template <typename T, int NW, int KP, bool NT, bool SPLIT>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec, PrefillLate p) {
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec,
+                                                                                  std::conditional_t<SPLIT, PrefillLate, PrefillBrief> late) {
+  const PrefillLate p = late;
   // SUB tiles of 64 keys per stage and per barrier: with one workgroup per CU (NW = 8) a stage
   // holds 128 keys, which halves the number of times the waves are forced in step.
   // LDS: K tiles of both stages [2*SUB][16 KiB], then the V tiles likewise; tile t sits in
@@ -673,12 +689,12 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   const int n_vis = min(e.n, tile_tok_end + e.offset);  // keys any row of this tile can see
   constexpr int kTileShift = TN == 128 ? 7 : 6;
   static_assert(1 << kTileShift == TN, "");
-  const int first = SPLIT ? split * p.first_each : 0, step = SPLIT ? (int)p.step_div.d : 1;  // of this workgroup's tiles
+  const int first = SPLIT ? split * p.first_each : 0, step = SPLIT && p.range_keys == kWholeRange ? p.num_splits : 1;  // of this workgroup's tiles
   int first_keys = n_vis - first * TN;  // keys from its first one on, within its range
   if (SPLIT) first_keys = min(first_keys, p.range_keys);
   auto mine = [&](int keys) {  // its tiles that hold one of the first `keys` keys
     int tiles = ((SPLIT ? min(keys - first * TN, p.range_keys) : keys) + TN - 1) >> kTileShift;
-    if (SPLIT && step > 1) tiles = tiles > 0 ? (int)fast_div(tiles + step - 1, p.step_div) : 0;
+    if (SPLIT && step > 1) tiles = tiles > 0 ? (int)fast_div(tiles + step - 1, p.splits_div) : 0;
     return tiles;
   };
   const uint32_t q_row_bytes = (uint32_t)e.H * kRowBytes;
@@ -691,7 +707,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   float *part_o = nullptr, *part_ml = nullptr;
   auto find_partial = [&] {
     part_o = p.ws_o + part_slot * kHeadDim;
-    part_ml = p.ws_ml + part_slot * 2;
+    part_ml = p.ws_o + (size_t)p.num_splits * e.m * e.H * kHeadDim + part_slot * 2;
   };
   if (SPLIT && first_keys <= 0) {  // workgroup-uniform: no row of this tile sees a key of this range
     find_partial();
@@ -737,8 +753,10 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   // tiles in which this wave's keys hold at least one visible key
   const int Jw = (qblk0 < rows) ? max(0, min(J, mine(min(e.n, tok_hi + e.offset + 1) - kw0))) : 0;
   // The late arguments are asked for now, while the loads are under way, not at the place of each one's use
-  asm volatile("" : : "s"(p.out), "s"(p.scale_log2e));
-  if (SPLIT) asm volatile("" : : "s"(p.ws_o), "s"(p.ws_ml));
+  asm volatile("" : : "s"(p.out));
+  float scale = kScaleLog2e;  // (in a register: as a literal 8192 tokens take 0.8 % longer)
+  asm volatile("" : "+s"(scale));
+  if (SPLIT) asm volatile("" : : "s"(p.ws_o));
   w.init(lds, lane, kVRegion, (KP > 1) ? kpar : 0);
   ld.template wait_but<2 * SUB * PER>();  // Q and K tile 0
   lds_barrier();
@@ -781,9 +799,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
       // would separate these MFMAs from the instructions they overlap with.)
       const int koff = ((slot + 1) % NSLOT) * TB;
       w.template qk<0, kSplitKK>(lds, koff, s_nxt, k_hook);
-      w.row_max(s_cur, p.scale_log2e);
+      w.row_max(s_cur, scale);
       w.template qk<kSplitKK, 8>(lds, koff, s_nxt, k_hook);
-      w.l_run += w.probabilities(s_cur, p.scale_log2e);
+      w.l_run += w.probabilities(s_cur, scale);
       w.pv(slot * TB, [&](auto i_) {
         constexpr int i = decltype(i_)::value;
         static_for<0, PER>([&](auto r_) {
@@ -835,7 +853,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     __syncthreads();
     auto finish = [&](auto part) {
       constexpr int PART = decltype(part)::value;
-      w.template take<KP, PART>(rows_lds, p.scale_log2e);
+      w.template take<KP, PART>(rows_lds, scale);
       if (SPLIT && rows > kFewRows)
         store_partial_rows<PART * ND, ND>(w, lds + RB * kTrade + wave * (32 * 128 * ND), part_row, part_ml, row_valid, rows - qblk0);
       else if (SPLIT)
@@ -1015,13 +1033,13 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
     const int heads_xcds = p.Hkv % 8 == 0 ? 8 : p.Hkv % 4 == 0 ? 4 : p.Hkv % 2 == 0 ? 2 : 1;
     if (T_ > 1 && heads_xcds < 8 && T_ * heads_xcds <= 16) {
       const int clusters = (T_ + kClusterTiles - 1) / kClusterTiles, each = (T_ + clusters - 1) / clusters;
-      p.items = grid;
+      const int last = (T_ - 1) % each + 1;
       p.per_xcd = (grid + 7) / 8;
       grid = 8 * p.per_xcd;
-      p.cluster_items = make_fast_div((uint32_t)(each * p.Hkv * S_));
-      p.cluster_tiles = make_fast_div((uint32_t)each);
-      p.last_tiles = make_fast_div((uint32_t)((T_ - 1) % each + 1));
-      p.splits_div = make_fast_div((uint32_t)S_);
+      p.tiles = (uint32_t)(each | last << 8);
+      p.each_part = 65536u / each + 1;  // (exact below 10922 items of a cluster: 6 tiles x 7 kv heads x 128 ranges are 5376)
+      p.last_part = 65536u / last + 1;
+      p.per_list = make_fast_div((uint32_t)(each * p.Hkv * S_));
     }
   } else if (share >= 0) {
     p.xcd_bits = 3;
@@ -1047,7 +1065,8 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
     }
   }
   p.list_heads = make_fast_div((uint32_t)list_heads);
-  p.per_split = make_fast_div((uint32_t)(list_heads * T_));
+  if (!p.per_xcd) p.per_list = make_fast_div((uint32_t)(list_heads * T_));
+  p.splits_div = make_fast_div((uint32_t)S_);
   // Key ranges lie side by side, or, where a key's rows together are long, one tile wide through each other, so that the workgroups
   // walk through the cache together: ranges that begin a multiple of MiB apart meet the same memory channels (rope and combine included,
   // us, side by side / through each other: 40 tokens past 16233 keys of 32 kv heads 66.8 / 58.0, past 4013 22.7 / 20.1, 64 past
@@ -1055,15 +1074,14 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   const bool through = p.Hkv >= 8;
   constexpr int TN = KP == 4 ? 2 * kTileN : kTileN;
   p.first_each = through ? 1 : p.chunk / TN;
-  p.range_keys = through ? 0x7fffffff : p.chunk;
-  p.step_div = make_fast_div(through ? (uint32_t)S_ : 1u);
+  p.range_keys = through ? kWholeRange : p.chunk;
   p.g_div = make_fast_div((uint32_t)p.g);
   const size_t tile_bytes = (NW == 8 || KP == 4 ? 2 : 1) * 4 * kTileBytes, q_bytes = (size_t)BM * kRowBytes;
   const size_t lds_bytes = tile_bytes + (KP > 1 ? q_bytes : q_bytes - tile_bytes / 4);  // (half of the V slots are Q's at first)
   // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KP == 1 there)
   const bool nt = KP == 1 && p.pack && T_ == 1, cut = S_ > 1;
-  auto kern = flash_prefill_kernel<T, NW, KP, false, false>;
-  if (cut) kern = nt ? flash_prefill_kernel<T, NW, KP, (KP == 1), true> : flash_prefill_kernel<T, NW, KP, false, true>;
+  const auto whole = flash_prefill_kernel<T, NW, KP, false, false>;
+  const auto ranges = nt ? flash_prefill_kernel<T, NW, KP, (KP == 1), true> : flash_prefill_kernel<T, NW, KP, false, true>;
   // the opt-in for more than 64 KiB of dynamic LDS is per device: once per device and kernel
   static std::atomic<uint64_t> attr_done_all[3];
   std::atomic<uint64_t> &attr_done = attr_done_all[nt ? 2 : cut ? 1 : 0];
@@ -1072,18 +1090,27 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   if (e != hipSuccess) return e;
   const uint64_t bit = 1ull << (dev & 63);
   if (!(attr_done.load(std::memory_order_acquire) & bit)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+    e = hipFuncSetAttribute(cut ? reinterpret_cast<const void *>(ranges) : reinterpret_cast<const void *>(whole),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (e != hipSuccess) return e;
     attr_done.fetch_or(bit, std::memory_order_release);
   }
   const PrefillEarly early(p);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
+  if (cut) {
+    hipLaunchKernelGGL(ranges, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
+  } else {
+    PrefillBrief brief;
+    brief.out = p.out;
+#ifdef LLMHIP_BENCH
+    brief.clock_probe = p.clock_probe;
+#endif
+    hipLaunchKernelGGL(whole, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, brief);
+  }
   e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1) return e;
   const size_t slots = (size_t)p.m * p.H;
-  const addresses_t a = {address(p.ws_o), address(p.ws_ml), address(p.out), slots};
-  const u32x2_t c = {(uint32_t)p.num_splits, __builtin_bit_cast(uint32_t, p.scale_log2e)};
+  const addresses_t a = {address(p.ws_o), address(p.ws_o + (size_t)p.num_splits * slots * kHeadDim), address(p.out), slots};
+  const u32x2_t c = {(uint32_t)p.num_splits, __builtin_bit_cast(uint32_t, kScaleLog2e)};
   if (slots <= 2048 && p.num_splits >= 8)
     hipLaunchKernelGGL(prefill_combine_wide_kernel<T>, dim3((unsigned)slots), dim3(256), 0, stream, a, c);
   else
@@ -1133,7 +1160,6 @@ struct PrefillPlan {
   bool pack;
   int num_splits, chunk;
 };
-constexpr int kWholeRange = 0x7fffffc0;
 
 // The most scratch a plan may ask for.  Without a bound it grows with the chunk (behind 131072 keys 7151 tokens of 28
 // heads 521 MB, 30000 of 40 1248).  By the model below 256 MiB costs at most 2.3 % behind up to 32768 keys and 6 % up
@@ -1311,7 +1337,6 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   p.g = group_size;
   p.Hkv = kv_head_num;
   p.H = group_size * kv_head_num;
-  p.scale_log2e = 1.4426950408889634f / sqrtf((float)kHeadDim);
   if (workspace_bytes > kMaxPrefillScratch) workspace_bytes = kMaxPrefillScratch;
   const PrefillPlan pl =
       plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), workspace ? workspace_bytes : 0);
@@ -1319,7 +1344,6 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   p.num_splits = pl.num_splits;
   p.chunk = pl.chunk;
   p.ws_o = static_cast<float *>(workspace);
-  p.ws_ml = p.ws_o ? p.ws_o + (size_t)pl.num_splits * m * p.H * kHeadDim : nullptr;
   return dt == kDtFloat16 ? launch_prefill<_Float16>(p, pl.kind, stream) : launch_prefill<__bf16>(p, pl.kind, stream);
 }
 
