@@ -1104,13 +1104,14 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // Short caches: where every workgroup has one block of 128 keys and twice as many workgroups still fit the chip at
   // once, blocks of 64 keys and workgroups of two waves.  Their slots have half the columns, so the
   // partials take no more room (one column is the flag's: up to 7 query rows).  More than 8 such blocks, with some CUs left to
-  // the folders, for the fused step only, where each wave of a CU takes in the query and the table beside its keys (us, blocks of 128 /
-  // 64: 700 keys of 4 kv heads 5.88 / 5.6, 1500 6.28 / 5.83, 1500 of 2 5.95 / 5.54, 1200 of 8 6.21 / 5.91; but unfused 2 x 900 of 4 5.33 /
-  // 5.69, and without CUs for the folders 2000 of 8 6.45 / 6.57).
+  // the folders, for one token of one sequence only: in the fused step each wave of a CU takes in the query and the table beside its keys (us,
+  // blocks of 128 / 64: 700 keys of 4 kv heads 5.88 / 5.6, 1500 6.28 / 5.83, 1500 of 2 5.95 / 5.54, 1200 of 8 6.21 / 5.91; but unfused 2 x 900
+  // of 4 5.33 / 5.69, and without CUs for the folders 2000 of 8 6.45 / 6.57), and the unfused call gives the same bits.
   const int half_blocks = (p.n + kDecStepKeys / 2 - 1) / (kDecStepKeys / 2), cus = device_compute_units();
   const long long half_wgs = (long long)p.batch * p.Hkv * half_blocks;
   const bool half = p.num_splits > 1 && p.num_splits == nblocks && p.rows < kDecCols / 2 &&
-                    (half_blocks <= kFoldDepth ? half_wgs <= cus : fused && half_blocks <= 2 * kMaxFoldSplits && half_wgs <= cus - cus / 16);
+                    (half_blocks <= kFoldDepth ? half_wgs <= cus
+                                               : p.batch == 1 && p.m == 1 && half_blocks <= 2 * kMaxFoldSplits && half_wgs <= cus - cus / 16);
   if (half) {
     p.num_splits = nblocks = half_blocks;
     p.cols = kDecCols / 2;

@@ -1200,7 +1200,8 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 // partials fit max_bytes are looked at; an unsplit one always does.  Over the 1800 measured shapes the choice was 1.1 %
 // slower than the fastest combination on average, 4 % at the 90th percentile; with the kernels of today, over 110 shapes of 2-512
 // tokens behind 260-29600 keys, 1.9 % and 5.4 %, 22 % at most (19 tokens behind 22155 keys of 20 + 4 heads 20.6 / 16.9 us, 121 behind 1350 of
-// 28 + 4 13.3 / 11.7).  Among combinations within 4 % of the
+// 28 + 4 13.3 / 11.7), and since ranges go through each other and tiles in clusters 2.0 % over 761 shapes, which constants fitted again would
+// make 1.3 %.  Among combinations within 4 % of the
 // cheapest one that reads K and V once and gives every CU the same number of workgroups is preferred.
 // Rows that fit one 256-row tile over a cache larger than the last-level cache are a stream from HBM: that tile's loads are
 // non-temporal then, and nothing else was faster (us, it / the best other one: 23 tokens over 68925 keys of 4 kv heads 49.6
