@@ -49,7 +49,7 @@ extern "C" {
  * out[m][head_num*head_dim] = softmax(scale * q k^T + causal(offset)) v with
  * q[m][head_num][head_dim], k and v = cache base pointers of which rows
  * [0, n) are read, key c masked for query r iff c > r + offset, scale =
- * 1/sqrt(head_dim) computed inside. */
+ * 1/sqrt(head_dim) computed inside.  out and q may be one buffer, here and in every other attention call. */
 int llmhip_flash_attn(void *out, const void *q, const void *k, const void *v, int m, int n,
                       int offset, int head_num, int head_dim, int dt, void *stream);
 

@@ -93,13 +93,13 @@ struct DecodeParams : DecodeLate {
   const void *freq_row, *new_k, *new_v;
   int batch, m, n, offset;
   int64_t kv_seq_stride;  // 0: the sequences are tiles of m tokens of one
-  int last_token;         // where the last sequence or tile begins: a last tile that would be short begins earlier
+  int tokens;             // of all sequences or tiles: the last tile may be short
   int g, Hkv, rows;
   int is_neox;
   bool fused;
   int cols;  // columns of a partial's slot: 16, or 8 of workgroups of two waves
 };
-// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8 | last_token << 16, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
+// a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8 | tokens << 16, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
 // up) << 10 (pairs = batch * Hkv, where the partials are folded by tags: at most kTaggedPairs); c: n, Hkv | g << 16 | is_neox << 31
 struct DecodeEarly {
   addresses_t a;
@@ -109,7 +109,7 @@ struct DecodeEarly {
     a = addresses_t{address(p.q), address(p.k), address(p.v), p.fused ? address(p.freq_row) : (uint64_t)p.kv_seq_stride};
     const uint64_t nk = address(p.new_k), nv = address(p.new_v);
     b = p.fused ? u32x4_t{(uint32_t)nk, (uint32_t)(nk >> 32), (uint32_t)nv, (uint32_t)(nv >> 32)}
-                : u32x4_t{(uint32_t)(p.rows | p.m << 8) | (uint32_t)p.last_token << 16, 65536u / p.g + 1, (uint32_t)p.offset,
+                : u32x4_t{(uint32_t)(p.rows | p.m << 8) | (uint32_t)p.tokens << 16, 65536u / p.g + 1, (uint32_t)p.offset,
                           (uint32_t)(p.batch * p.Hkv) | ((1u << 20) + p.Hkv - 1) / p.Hkv << 10};
     c = u32x2_t{(uint32_t)p.n, (uint32_t)p.Hkv | (uint32_t)p.g << 16 | (uint32_t)p.is_neox << 31};
   }
@@ -291,15 +291,15 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 
 // A folder: rows c0 .. c0 + fold_rows - 1 of a pair, from partials whose words carry this launch's tags.  A wave has a row, two
 // dims per lane, and PARTS of the fold_parts() parts of its partials, DEPTH in all.  It looks at all of them until it finds the tags
-// at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  False if they were not there after
-// kFoldPolls looks.
+// at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  have_rows: of the pair's rows, those that
+// are there (a short last tile).  A bit per row c0 + i that was not stored: its partials were not there after kFoldPolls looks.
 template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
-__device__ __forceinline__ bool fold_tagged(const DecodeLate &p, uint32_t row_part, char *lds, int pair, int token, int kvh, int c0, int rows, int Hkv,
-                                            int g) {
+__device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t row_part, char *lds, int pair, int token, int kvh, int c0, int rows,
+                                                int have_rows, int Hkv, int g) {
   constexpr int EACH = DEPTH / PARTS;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
   const int parts = fold_parts(S, rows), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
-  const bool mine = wave % at_once < p.fold_rows && c < rows;  // (of the wave)
+  const bool mine = wave % at_once < p.fold_rows && c < have_rows;  // (of the wave)
   const int bytes = S * rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + (size_t)pair * bytes, bytes);
   const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
@@ -364,6 +364,7 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, uint32_t row_pa
   }
   int *failed = reinterpret_cast<int *>(lds);  // per wave
   if (lane == 0) failed[wave] = !there;
+  bool whole = there;  // of the row's waves
   if (parts > 1) {
     // part i of row `wave` is in place wave + i * at_once
     float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = red_ml + 2 * NW * PARTS;
@@ -386,20 +387,22 @@ __device__ __forceinline__ bool fold_tagged(const DecodeLate &p, uint32_t row_pa
         x[0] += wt * o.x;
         y[0] += wt * o.y;
       }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) whole = whole && !((w & (at_once - 1)) == wave && failed[w]);
     }
   }
-  if (mine && part == 0 && there) {
+  if (mine && part == 0 && whole) {
     const int r = (int)(c * row_part >> 16);  // (c / g)
     const float inv = (L[0] > 0.0f) ? 1.0f / L[0] : 0.0f;
     char *row = p.out + (((size_t)token + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes;
     *reinterpret_cast<uint32_t *>(row + (lane & 15) * 16 + (lane >> 4) * 4) = Elem<T>::pack2(x[0] * inv, y[0] * inv);
   }
   __syncthreads();
-  int any = 0;
+  uint32_t missing = 0;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) any |= failed[w];
+  for (int w = 0; w < NW; ++w) missing |= (uint32_t)failed[w] << (w & (at_once - 1));
   __syncthreads();
-  return any == 0;
+  return __builtin_amdgcn_readfirstlane(missing);
 }
 
 // The argument struct of the running kernel, asked for here (as a parameter that two branches use it is fetched, and waited
@@ -431,10 +434,11 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   using E = Elem<T>;
   const int n = ec[0], Hkv = ec[1] & 0xffffu, g = ec[1] >> 16 & 0xffu, H = g * Hkv;
   const bool is_neox = ec[1] >> 31;
-  const int rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8 & 0xffu;
+  const int all_rows = FUSED ? g : eb[0] & 0xffu, m = FUSED ? 1 : eb[0] >> 8 & 0xffu;
   const uint32_t row_part = FUSED ? 0u : eb[1];  // (of a column, 16 bits on: its query row)
   constexpr int cols = NW == 2 ? kDecCols / 2 : kDecCols;
-  auto token_of = [&](int seq) { return FUSED ? 0 : min(seq * m, (int)(eb[0] >> 16)); };  // first token of a sequence, or of a tile of one
+  auto token_of = [&](int seq) { return FUSED ? 0 : seq * m; };  // first token of a sequence, or of a tile of one
+  auto rows_from = [&](int token) { return FUSED ? g : min(all_rows, ((int)(eb[0] >> 16) - token) * g); };  // (the last tile may be short)
   const int fused_pos = n - 1;
   constexpr int kStepKeys = NW * kDecWaveKeys;
   __shared__ __attribute__((aligned(16))) char lds[2 * NW * kDecWaveLds];
@@ -442,7 +446,8 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   int split = blockIdx.x, kvh = blockIdx.y, b = FUSED ? 0 : blockIdx.z;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int col = lane & 15, cg = lane >> 4;
-  bool lone = false;  // a folder that stopped waiting: all keys of its (sequence, kv head), and the rows
+  bool lone = false;  // a folder that stopped waiting: all keys of its (sequence, kv head)
+  uint32_t lone_rows = 0;  // and its own rows that are not stored yet.  (Not those of other folders, which may be stored: out may be q.)
   if constexpr (FOLD == kFoldByTags) {
     const int pairs = FUSED ? Hkv : eb[3] & 0x3ffu;
     int pair = blockIdx.y;
@@ -455,7 +460,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       const int c0 = (e - pair * f.folders) * f.fold_rows;
       auto fold = [&](auto depth, auto parts, auto round) {
         return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, row_part, lds, pair, token_of(b), pair - b * Hkv,
-                                                                                                          c0, rows, Hkv, g);
+                                                                                                          c0, all_rows, rows_from(token_of(b)), Hkv, g);
       };
       using std::integral_constant;
       const integral_constant<int, 1> one;
@@ -464,28 +469,29 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       const integral_constant<int, 8> eight;
       const integral_constant<int, 16> sixteen;
       const int S = f.num_splits;
-      bool folded;
+      uint32_t missing;
       if constexpr (NW == 4)
-        folded = S > 64                ? fold(integral_constant<int, 32>(), two, four)
+        missing = S > 64                ? fold(integral_constant<int, 32>(), two, four)
                  : S > 32              ? fold(sixteen, two, four)
-                 : S > kMaxFoldSplits || (rows == kDecCols && S > kFoldDepth) ? fold(eight, two, four)
-                 : S > kFoldDepth && rows > kFewRows                          ? fold(sixteen, one, sixteen)
+                 : S > kMaxFoldSplits || (all_rows == kDecCols && S > kFoldDepth) ? fold(eight, two, four)
+                 : S > kFoldDepth && all_rows > kFewRows                          ? fold(sixteen, one, sixteen)
                  : S > 4               ? fold(eight, one, eight)
                                        : fold(four, one, four);
       else
-        folded = S > kMaxFoldSplits ? fold(sixteen, four, four)
+        missing = S > kMaxFoldSplits ? fold(sixteen, four, four)
                  : S > kFoldDepth   ? fold(sixteen, two, eight)
                  : S > 4            ? fold(eight, one, eight)
                                     : fold(four, one, four);
-      if (folded)
+      if (missing == 0)
         return;
       lone = true;
+      lone_rows = missing << c0;
       split = 0;
     }
     b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
     kvh = pair - b * Hkv;
   }
-  const int token = token_of(b);
+  const int token = token_of(b), rows = rows_from(token);
   const int offset = FUSED ? n - 1 : (int)eb[2] + (ea[3] == 0 ? token : 0);
   const DecodeLate p = FOLD == kFoldByTags ? fetch_late() : late;
   const int num_splits = lone ? 1 : p.num_splits;
@@ -709,13 +715,14 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   const int pair_slots = p.num_splits * cols;
   const __amdgpu_buffer_rsrc_t po = byte_buffer(p.ws_o + pair * pair_slots * kHeadDim, pair_slots * kHeadDim * 4);
   const __amdgpu_buffer_rsrc_t pml = byte_buffer(p.ws_ml + pair * pair_slots * 2, pair_slots * 8);
-  const int tagged_bytes = p.num_splits * rows * kTaggedBytes;
+  const int tagged_bytes = p.num_splits * all_rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + pair * tagged_bytes, tagged_bytes);
   const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
   auto tagged = [&](float x, float y) {
     return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), tag0, __builtin_bit_cast(uint32_t, y), tag1});
   };
   for (int c = tid >> 4; c < rows; c += 4 * NW) {
+    if (lone && !(lone_rows >> c & 1)) continue;
     const int dch = tid & 15;  // 8-wide d chunk of column c
     float mw[NW], M = -INFINITY;
 #pragma unroll
@@ -754,7 +761,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
     const f32x4_t a0 = {acc[0], acc[1], acc[2], acc[3]}, a1 = {acc[4], acc[5], acc[6], acc[7]};
     const u32x2_t ml = {__builtin_bit_cast(uint32_t, M), __builtin_bit_cast(uint32_t, L)};
     if constexpr (FOLD == kFoldByTags) {
-      const int at = (split * rows + c) * kTaggedBytes;
+      const int at = (split * all_rows + c) * kTaggedBytes;
 #pragma unroll
       for (int j = 0; j < 4; ++j) store_device(pt, at + j * 256 + dch * 16, tagged(acc[2 * j], acc[2 * j + 1]));
       if (dch == 0) store_device(pt, at + kHeadDim * 8, tagged(M, L));
@@ -797,7 +804,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   constexpr int NG = 2 * NW;
   const int d4 = tid & 31;
   auto fold = [&](auto depth) {
-    const int parts = fold_parts(p.num_splits, rows);
+    const int parts = fold_parts(p.num_splits, all_rows);
     constexpr int D = decltype(depth)::value;
     const int at_once = NG / parts, part = (tid >> 5) / at_once;
     for (int c0 = 0; c0 < rows; c0 += at_once) {
@@ -816,7 +823,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       if (part == 0 && c < rows) f.template store<T>(p.out, token, c, kvh, Hkv, g, (int)(c * row_part >> 16), d4);
     }
   };
-  if (NW == 4 && rows > kFewRows && p.num_splits > kFoldDepth)
+  if (NW == 4 && all_rows > kFewRows && p.num_splits > kFoldDepth)
     fold(std::integral_constant<int, kMaxFoldSplits>());
   else
     fold(std::integral_constant<int, kFoldDepth>());
@@ -830,7 +837,7 @@ constexpr int kMaxSplits = 256;
 
 template <typename T>
 __global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a, u32x4_t size, u32x2_t heads) {
-  // a: partials, their maxima and sums, out, last_token; size: splits, columns of a slot, Hkv, m; heads: g, 2^16 / g + 1
+  // a: partials, their maxima and sums, out, tokens; size: splits, columns of a slot, Hkv, m; heads: g, 2^16 / g + 1
   using E = Elem<T>;
   const float *ws_o = at_address<const float>(a[0]), *ws_ml = at_address<const float>(a[1]);
   char *out = at_address<char>(a[2]);
@@ -838,6 +845,7 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a
   __shared__ float red_m[8], red_l[8];
   __shared__ f32x4_t red_o[8][32];
   const int c = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  if (c >= ((int)a[3] - b * m) * g) return;  // (past a short last tile)
   const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
   const int S = size[0];
   const size_t base = ((size_t)b * Hkv + kvh) * S;
@@ -900,7 +908,7 @@ __global__ __launch_bounds__(256) void flash_decode_combine_kernel(addresses_t a
   u32x2_t w;
   w[0] = E::pack2(tot[0] * inv, tot[1] * inv);
   w[1] = E::pack2(tot[2] * inv, tot[3] * inv);
-  const size_t token = min((unsigned)(b * m), (unsigned)a[3]);
+  const size_t token = (unsigned)(b * m);
   *reinterpret_cast<u32x2_t *>(out + ((token + r) * H + kvh * g + hq) * kRowBytes + d4 * 8) = w;
 }
 
@@ -1077,7 +1085,7 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
   hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream,
-                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), (uint64_t)p.last_token},
+                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), (uint64_t)p.tokens},
                      u32x4_t{(uint32_t)p.num_splits, (uint32_t)p.cols, (uint32_t)p.Hkv, (uint32_t)p.m},
                      u32x2_t{(uint32_t)p.g, 65536u / p.g + 1});
   return hipGetLastError();
@@ -1160,7 +1168,7 @@ hipError_t launch_flash_decode(void *out, const void *q, const void *k, const vo
   p.n = n;
   p.offset = offset;
   p.kv_seq_stride = kv_seq_stride;
-  p.last_token = (batch - 1) * m;
+  p.tokens = batch * m;
   p.g = group_size;
   p.Hkv = kv_head_num;
   p.rows = m * group_size;
@@ -1194,7 +1202,7 @@ hipError_t launch_flash_decode_tiles(void *out, const void *q, const void *k, co
   p.out = static_cast<char *>(out);
   p.batch = flash_decode_tiles(m, group_size);
   p.m = (m + p.batch - 1) / p.batch;
-  p.last_token = m - p.m;
+  p.tokens = m;
   p.n = n;
   p.offset = offset;
   p.g = group_size;
@@ -1216,6 +1224,7 @@ hipError_t launch_flash_decode_step(void *out, void *k_cache, void *v_cache, con
   p.out = static_cast<char *>(out);
   p.batch = 1;
   p.m = 1;
+  p.tokens = 1;
   p.n = pos + 1;
   p.offset = pos;
   p.kv_seq_stride = pos + 1;

@@ -1,4 +1,4 @@
-"""Chunks whose query rows go through the decode kernel in tiles of up to 16: two tiles and eight, a last tile that begins early, whole
+"""Chunks whose query rows go through the decode kernel in tiles of up to 16: two tiles and eight, a short last tile, whole
 tiles of 16 rows, one partial and many, keys behind the last visible one (NaN), the edges of the rule -- against the oracle, the same bits
 when repeated and from a HIP graph, which folds otherwise, and on a stream without scratch under capture, which takes key ranges."""
 import numpy as np
