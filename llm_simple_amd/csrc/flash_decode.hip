@@ -362,8 +362,8 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
       y[i] += w * bits_float(a[j][2]);
     }
   }
-  int *failed = reinterpret_cast<int *>(lds);  // per wave
-  if (lane == 0) failed[wave] = !there;
+  uint32_t *failed = reinterpret_cast<uint32_t *>(lds);  // of each wave, the bit of its row
+  if (lane == 0) failed[wave] = there ? 0u : 1u << (c - c0);
   bool whole = there;  // of the row's waves
   if (parts > 1) {
     // part i of row `wave` is in place wave + i * at_once
@@ -371,7 +371,7 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
 #pragma unroll
     for (int i = 0; i < PARTS; ++i) {
       const int place = wave + i * NW;
-      if (lane == 0) *reinterpret_cast<float2 *>(red_ml + 2 * place) = float2{M[i], L[i]};
+      if (lane == 0) *reinterpret_cast<float2 *>(red_ml + 2 * place) = float2{M[i], there ? L[i] : -1.0f};
       *reinterpret_cast<float2 *>(red_o + place * kHeadDim + 2 * lane) = float2{x[i], y[i]};
     }
     __syncthreads();
@@ -381,14 +381,13 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
       const float M_use = (M[0] == -INFINITY) ? 0.0f : M[0];
       L[0] = x[0] = y[0] = 0.0f;
       for (int i = wave; i < NW * PARTS; i += at_once) {
-        const float wt = fast_exp2(red_ml[2 * i] - M_use);  // 0 for a part without splits (-inf)
-        L[0] += wt * red_ml[2 * i + 1];
+        const float wt = fast_exp2(red_ml[2 * i] - M_use), l = red_ml[2 * i + 1];  // wt: 0 for a part without splits (-inf)
+        if (l < 0.0f) whole = false;
+        L[0] += wt * l;
         const float2 o = *reinterpret_cast<const float2 *>(red_o + i * kHeadDim + 2 * lane);
         x[0] += wt * o.x;
         y[0] += wt * o.y;
       }
-#pragma unroll
-      for (int w = 0; w < NW; ++w) whole = whole && !((w & (at_once - 1)) == wave && failed[w]);
     }
   }
   if (mine && part == 0 && whole) {
@@ -400,7 +399,7 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
   __syncthreads();
   uint32_t missing = 0;
 #pragma unroll
-  for (int w = 0; w < NW; ++w) missing |= (uint32_t)failed[w] << (w & (at_once - 1));
+  for (int w = 0; w < NW; ++w) missing |= failed[w];
   __syncthreads();
   return __builtin_amdgcn_readfirstlane(missing);
 }
@@ -722,7 +721,6 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
     return __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), tag0, __builtin_bit_cast(uint32_t, y), tag1});
   };
   for (int c = tid >> 4; c < rows; c += 4 * NW) {
-    if (lone && !(lone_rows >> c & 1)) continue;
     const int dch = tid & 15;  // 8-wide d chunk of column c
     float mw[NW], M = -INFINITY;
 #pragma unroll
@@ -748,6 +746,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       }
     }
     if (FOLD == kNoFold ? num_splits == 1 : lone) {
+      if (lone && !(lone_rows >> c & 1)) continue;
       const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
       const int r = (int)(c * row_part >> 16), hq = c - r * g;
       char *op = p.out + (((size_t)token + r) * H + kvh * g + hq) * kRowBytes + dch * 16;
