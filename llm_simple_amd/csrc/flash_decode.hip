@@ -1002,15 +1002,18 @@ int flash_decode_splits_within(int batch, int n, int kv_head_num, int rows, size
 
 // What a call may insist on is counted with coarser figures than the default: 27.7 GB/s per CU in a full round and at most
 // 32 in a thin one, 3 us per workgroup, 5 for a fold.  Callers were promised that calls which are not worth a split by
-// these need no room; the promise does not move with the model above.
+// these need no room; the promise does not move with the model above.  Nor does it move for callers whose workspace was sized by the default
+// count of the model before (whole rounds, folds of 1.2 to 2.6 us): the smaller of the two is enough (3 x 3584 keys of 8 kv heads: 10 of
+// now, 7 before, 10 by the coarser figures).
 size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
   const long long pairs = (long long)batch * kv_head_num;
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys, cus = device_compute_units();
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
-  const int s = best_splits(pairs, smax, cus, 1.03, pairs * smax, [&](int splits) {
+  auto kb_of = [&](int splits) { return 2.0 * kRowBytes * kDecStepKeys * ((nblocks + splits - 1) / splits) * 1e-3; };
+  const int coarse = best_splits(pairs, smax, cus, 1.03, pairs * smax, [&](int splits) {
     const long long full = pairs * splits / cus, rest = pairs * splits % cus;
-    const double kb = 2.0 * kRowBytes * kDecStepKeys * ((nblocks + splits - 1) / splits) * 1e-3;
+    const double kb = kb_of(splits);
     double t = full * (kb / 27.7 + 3.0);
     if (rest > 0) {
       const double rate = 27.7 * cus / (double)rest;
@@ -1018,7 +1021,15 @@ size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
     }
     return splits > 1 ? t + 5.0 : t;
   });
-  return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, s);
+  const int before = best_splits(pairs, smax, cus, 1.03, pairs * smax, [&](int splits) {
+    const long long full = pairs * splits / cus, rest = pairs * splits % cus;
+    double t = full * (kb_of(splits) / 27.9 + 2.7);
+    if (rest > 0) t += kb_of(splits) / (((nblocks + splits - 1) / splits >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
+    if (splits == 1) return t;
+    if (splits == nblocks && 2 * splits <= kFoldDepth && 2 * pairs * splits <= cus) return t + 1.2;
+    return t + (splits <= kFoldDepth ? 2.0 : splits <= kMaxFoldSplits ? 2.6 : 2.1);
+  });
+  return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, coarse < before ? coarse : before);
 }
 
 int flash_decode_effective_splits(int num_splits, int n) {

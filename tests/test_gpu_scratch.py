@@ -167,6 +167,20 @@ def test_batched_decode_with_less_workspace_than_the_default_count_takes():
     assert ops.lib.llmhip_flash_decode_gqa(*args, 1, 32768, 32768, 5, 8, 128, 0, DT, None) == -3
 
 
+def test_workspace_of_an_earlier_default_count():
+    """A workspace that held the default count by the model before the present one (7 splits, 10 now) still does."""
+    import torch
+    import llm_simple_amd.ops as ops
+    batch, n, H, Hkv = 3, 3584, 40, 8
+    q = normal_bits(1, (batch, 1, H, 128), DT)
+    k, v = (normal_bits(s, (batch, n, Hkv, 128), DT) for s in (2, 3))
+    seven = ops.flash_decode_workspace_bytes(batch, H // Hkv, Hkv, 128, 7)
+    assert ops.flash_decode_default_splits(batch, n, Hkv) > 7
+    ws, out = torch.empty(seven, dtype=torch.uint8, device="cuda"), dev_empty(q.shape)
+    ops.hip_flash_decode_gqa_layer(out, to_dev(q), to_dev(k), to_dev(v), ws, seven, batch, n, n, H // Hkv, Hkv, 128, 0, DT)
+    check_attention(to_host(out), q, k, v, n, n - 1, DT, batch=True)
+
+
 def test_a_growing_buffer_stays_bounded():
     """Chunks that need more and more: what the stream holds, replaced buffers included, stays under twice the power
     of two that holds the largest, and goes with the stream."""

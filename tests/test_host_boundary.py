@@ -7,6 +7,8 @@ import os
 import re
 import subprocess
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -99,6 +101,20 @@ def test_default_splits_and_workspace_size():
     assert 1 <= s <= 32
     assert ops.flash_decode_workspace_bytes(1, 5, 8, 128, 1) == 0
     assert ops.flash_decode_workspace_bytes(16, 5, 8, 128, 2) == 16 * 8 * 2 * 16 * (128 + 2) * 4
+
+
+# (batch, n, kv heads, splits that a workspace holds): the default count of the model before the present one, and what the coarser figures ask for
+@pytest.mark.parametrize("batch,n,Hkv,splits,taken", [(3, 3584, 8, 7, True), (3, 3584, 8, 6, False), (2, 2688, 32, 3, True), (2, 2688, 32, 2, False),
+                                                      (7, 5248, 4, 7, True), (3, 13568, 32, 2, True), (1, 32768, 8, 32, True), (1, 32768, 8, 31, False)])
+def test_workspace_of_an_earlier_default_count_is_enough(batch, n, Hkv, splits, taken):
+    import llm_simple_amd.ops as ops
+    if ops.lib.llmhip_device_count() > 0:
+        pytest.skip("host pointers: a device would launch (there: test_gpu_scratch.py)")
+    buf = ctypes.create_string_buffer(96)
+    p = (ctypes.addressof(buf) + 15) & ~15
+    room = batch * Hkv * splits * 16 * (128 + 2) * 4
+    rc = ops.lib.llmhip_flash_decode_gqa(p, p, p, p, p, room, batch, n, n, 5, Hkv, 128, 0, 5, None)
+    assert (rc > 0) == taken and (rc == -3) != taken, rc  # (taken: as far as the launch, which finds no device)
 
 
 def test_cpp_device_layer_host_checks():
