@@ -38,7 +38,7 @@
 // More than 8 query rows (a few tokens checked at once) take folders where the room is there, with tags twice that of the partials (rope
 // and attention, us, flags or a combine launch / folders: 2 tokens past 1200 keys of 28 + 4 heads 10.1 / 7.8, past 20000 14.1 / 13.3, 3 past
 // 1500 of 40 + 8 11.1 / 8.4, 12 past 900 of 32 + 32 10.9 / 9.15).
-// Where the number would be that of a replay, or without that room, up to 16 partials are folded by the workgroup that finds them all
+// Where the number would be that of a replay, or without that room, few partials of few rows are folded by the workgroup that finds them all
 // stored: partials, then a flag, then a look at the other flags, then the partials, four round trips to memory.  Beyond that, or
 // beyond 128 partials, there is a second launch.  (Device-scope fences instead of sc1 accesses write back and invalidate the XCD's L2: 91 us
 // against 33 at batch 1, 32768 keys.)
@@ -180,22 +180,19 @@ __device__ __forceinline__ int v_swizzle32_off(int row, int granule) {
   return row * kRowBytes + ((((granule >> 1) ^ (row & 7)) << 5) | ((granule & 1) << 4));
 }
 
-constexpr int kMaxFoldSplits = 16, kMaxTaggedSplits = 128;
+constexpr int kMaxTaggedSplits = 128;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
-constexpr int kFewRows = 8;                       // query rows up to which a row's partials are dealt to parts
 constexpr int kTaggedPairs = 1023;                // (sequence, kv head) pairs, at most
-constexpr int kFoldDepth = 8;  // partials of a row that a thread asks for at once
+constexpr int kFoldDepth = 8;                     // partials that are summed in one part
 #ifdef LLMHIP_BENCH
 constexpr int kFoldPolls = 0;  // (the measurement library's copy: every folder computes its rows by itself)
 #else
 constexpr int kFoldPolls = 1 << 16;  // looks that a folder takes, 0.6 us each
 #endif
-// Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  (The order of the
-// combine launch where they are more than kMaxFoldSplits, or there is no column left for a flag.  More than kFewRows rows leave no
-// groups to deal them to where one workgroup folds by flags.)
-__host__ __device__ constexpr int fold_parts(int splits, int rows) {
-  return splits <= kFoldDepth ? 1 : splits > kMaxFoldSplits || rows == kDecCols ? 8 : rows > kFewRows ? 1 : 2;
-}
+// Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  That is the order of the
+// combine launch, so that all ways to fold give the same bits.
+constexpr int kParts = 8;
+__host__ __device__ constexpr int fold_parts(int splits) { return splits <= kFoldDepth ? 1 : kParts; }
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
 
@@ -220,69 +217,34 @@ __device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int by
   return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
 }
 
-// A row from its partials: four dims of it in each thread of a group of 32, the partials dealt to `parts` groups.
-struct RowFold {
+// The sum of partials, four dims of it per thread.
+struct PartialSum {
   float M = -INFINITY, L = 0.0f;
-  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  // partials part, part + parts, ... of S
-  template <int D>
-  __device__ __forceinline__ void take(const u32x2_t (&ml)[D], const f32x4_t (&ov)[D], int part, int parts, int S) {
+  f32x4_t o = {0.f, 0.f, 0.f, 0.f};
+  template <int D> __device__ __forceinline__ void take(const u32x2_t (&ml)[D], const f32x4_t (&ov)[D], int have) {
 #pragma unroll
     for (int j = 0; j < D; ++j)
-      if (part + parts * j < S) M = fmaxf(M, bits_float(ml[j][0]));
+      if (j < have) M = fmaxf(M, bits_float(ml[j][0]));
     const float M_use = (M == -INFINITY) ? 0.0f : M;
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      const float wt = (part + parts * j < S) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
+      const float wt = (j < have) ? fast_exp2(bits_float(ml[j][0]) - M_use) : 0.0f;
       L += wt * bits_float(ml[j][1]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += wt * ov[j][i];
+      for (int i = 0; i < 4; ++i) o[i] += wt * ov[j][i];
     }
-  }
-  // Part i of a row is in group i * at_once + row; the sum ends up in part 0.  Room: 2 + 128 floats per group, from a
-  // multiple of 16 bytes on.  Every thread of the workgroup calls.
-  template <int GROUPS> __device__ __forceinline__ void merge(float *room, int parts, int at_once) {
-    const int sg = threadIdx.x >> 5, d4 = threadIdx.x & 31;
-    float *red_o = room + 2 * GROUPS;
-    if (d4 == 0) *reinterpret_cast<float2 *>(room + 2 * sg) = float2{M, L};
-    *reinterpret_cast<f32x4_t *>(red_o + sg * kHeadDim + 4 * d4) = acc;
-    __syncthreads();
-    if (sg < at_once) {
-      M = -INFINITY;
-      for (int i = sg; i < parts * at_once; i += at_once) M = fmaxf(M, room[2 * i]);
-      const float M_use = (M == -INFINITY) ? 0.0f : M;
-      L = 0.0f;
-      acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      for (int i = sg; i < parts * at_once; i += at_once) {
-        const float wt = fast_exp2(room[2 * i] - M_use);  // 0 for a group without splits (-inf)
-        L += wt * room[2 * i + 1];
-        const f32x4_t o = *reinterpret_cast<const f32x4_t *>(red_o + i * kHeadDim + 4 * d4);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) acc[d] += wt * o[d];
-      }
-    }
-    __syncthreads();
-  }
-  template <typename T>
-  __device__ __forceinline__ void store(char *out, int token, int c, int kvh, int Hkv, int g, int r, int d4) {
-    const float inv = (L > 0.0f) ? 1.0f / L : 0.0f;
-    u32x2_t w;
-    w[0] = Elem<T>::pack2(acc[0] * inv, acc[1] * inv);
-    w[1] = Elem<T>::pack2(acc[2] * inv, acc[3] * inv);
-    *reinterpret_cast<u32x2_t *>(out + (((size_t)token + r) * Hkv * g + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
   }
 };
 
-// Maximum over each N = 4, 8 or 16 lanes.
+// Maximum over each N = 2, 4 or 8 lanes.
 template <int N> __device__ __forceinline__ float max_of_lanes(float x) {
   auto with = [&](auto control) {
     const int i = __builtin_bit_cast(int, x);
     x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, decltype(control)::value, 0xf, 0xf, false)));
   };
   with(std::integral_constant<int, 0xB1>());                     // quad_perm: lane ^ 1
-  with(std::integral_constant<int, 0x4E>());                     // quad_perm: lane ^ 2
-  if (N >= 8) with(std::integral_constant<int, 0x141>());        // row_half_mirror: the other quad
-  if (N == 16) with(std::integral_constant<int, 0x140>());       // row_mirror: the other half of the row
+  if (N >= 4) with(std::integral_constant<int, 0x4E>());         // quad_perm: lane ^ 2
+  if (N == 8) with(std::integral_constant<int, 0x141>());        // row_half_mirror: the other quad
   return x;
 }
 __device__ __forceinline__ float lane_value(float x, int lane) {
@@ -296,9 +258,10 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
 __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t row_part, char *lds, int pair, int token, int kvh, int c0, int rows,
                                                 int have_rows, int Hkv, int g) {
-  constexpr int EACH = DEPTH / PARTS;
+  constexpr int EACH = DEPTH / PARTS;  // (PARTS 1: of one part, else of kParts)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
-  const int parts = fold_parts(S, rows), per_row = parts / PARTS, at_once = NW / per_row, part = wave / at_once, c = c0 + wave % at_once;
+  constexpr int parts = PARTS > 1 ? kParts : 1, per_row = parts / PARTS, at_once = NW / per_row;
+  const int part = wave / at_once, c = c0 + wave % at_once;
   const bool mine = wave % at_once < p.fold_rows && c < have_rows;  // (of the wave)
   const int bytes = S * rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + (size_t)pair * bytes, bytes);
@@ -365,29 +328,49 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
   uint32_t *failed = reinterpret_cast<uint32_t *>(lds);  // of each wave, the bit of its row
   if (lane == 0) failed[wave] = there ? 0u : 1u << (c - c0);
   bool whole = there;  // of the row's waves
-  if (parts > 1) {
+  if constexpr (PARTS > 1) {
     // part i of row `wave` is in place wave + i * at_once
-    float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = red_ml + 2 * NW * PARTS;
+    float part_m[kParts], part_l[kParts], part_x[kParts], part_y[kParts];
+    if constexpr (PARTS == kParts) {
 #pragma unroll
-    for (int i = 0; i < PARTS; ++i) {
-      const int place = wave + i * NW;
-      if (lane == 0) *reinterpret_cast<float2 *>(red_ml + 2 * place) = float2{M[i], there ? L[i] : -1.0f};
-      *reinterpret_cast<float2 *>(red_o + place * kHeadDim + 2 * lane) = float2{x[i], y[i]};
-    }
-    __syncthreads();
-    if (part == 0) {
-      M[0] = -INFINITY;
-      for (int i = wave; i < NW * PARTS; i += at_once) M[0] = fmaxf(M[0], red_ml[2 * i]);
-      const float M_use = (M[0] == -INFINITY) ? 0.0f : M[0];
-      L[0] = x[0] = y[0] = 0.0f;
-      for (int i = wave; i < NW * PARTS; i += at_once) {
-        const float wt = fast_exp2(red_ml[2 * i] - M_use), l = red_ml[2 * i + 1];  // wt: 0 for a part without splits (-inf)
-        if (l < 0.0f) whole = false;
-        L[0] += wt * l;
-        const float2 o = *reinterpret_cast<const float2 *>(red_o + i * kHeadDim + 2 * lane);
-        x[0] += wt * o.x;
-        y[0] += wt * o.y;
+      for (int i = 0; i < kParts; ++i) {
+        part_m[i] = M[i];
+        part_l[i] = L[i];
+        part_x[i] = x[i];
+        part_y[i] = y[i];
       }
+    } else {
+      float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = red_ml + 2 * NW * PARTS;
+#pragma unroll
+      for (int i = 0; i < PARTS; ++i) {
+        const int place = wave + i * NW;
+        if (lane == 0) *reinterpret_cast<float2 *>(red_ml + 2 * place) = float2{M[i], there ? L[i] : -1.0f};
+        *reinterpret_cast<float2 *>(red_o + place * kHeadDim + 2 * lane) = float2{x[i], y[i]};
+      }
+      __syncthreads();
+      // (all of them read before the first is used: in a loop a turn is a trip to LDS, 32768 keys of 8 kv heads 23.0 us, 22.5 so)
+#pragma unroll
+      for (int i = 0; i < kParts; ++i) {
+        const int place = part == 0 ? wave + i * at_once : 0;
+        const float2 ml_i = *reinterpret_cast<const float2 *>(red_ml + 2 * place), o = *reinterpret_cast<const float2 *>(red_o + place * kHeadDim + 2 * lane);
+        part_m[i] = ml_i.x;
+        part_l[i] = ml_i.y;
+        part_x[i] = o.x;
+        part_y[i] = o.y;
+        if (part_l[i] < 0.0f) whole = false;
+      }
+    }
+    M[0] = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) M[0] = fmaxf(M[0], part_m[i]);
+    const float M_use = (M[0] == -INFINITY) ? 0.0f : M[0];
+    L[0] = x[0] = y[0] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) {
+      const float wt = fast_exp2(part_m[i] - M_use);  // 0 for a part without splits (-inf)
+      L[0] += wt * part_l[i];
+      x[0] += wt * part_x[i];
+      y[0] += wt * part_y[i];
     }
   }
   if (mine && part == 0 && whole) {
@@ -470,17 +453,17 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       const int S = f.num_splits;
       uint32_t missing;
       if constexpr (NW == 4)
-        missing = S > 64                ? fold(integral_constant<int, 32>(), two, four)
-                 : S > 32              ? fold(sixteen, two, four)
-                 : S > kMaxFoldSplits || (all_rows == kDecCols && S > kFoldDepth) ? fold(eight, two, four)
-                 : S > kFoldDepth && all_rows > kFewRows                          ? fold(sixteen, one, sixteen)
-                 : S > 4               ? fold(eight, one, eight)
-                                       : fold(four, one, four);
+        missing = S > 64           ? fold(integral_constant<int, 32>(), two, four)
+                  : S > 32         ? fold(sixteen, two, four)
+                  : S > 16         ? fold(eight, two, four)
+                  : S > kFoldDepth ? fold(sixteen, eight, two)
+                  : S > 4          ? fold(eight, one, eight)
+                                   : fold(four, one, four);
       else
-        missing = S > kMaxFoldSplits ? fold(sixteen, four, four)
-                 : S > kFoldDepth   ? fold(sixteen, two, eight)
-                 : S > 4            ? fold(eight, one, eight)
-                                    : fold(four, one, four);
+        missing = S > 16           ? fold(sixteen, four, four)
+                  : S > kFoldDepth ? fold(sixteen, eight, two)
+                  : S > 4          ? fold(eight, one, eight)
+                                   : fold(four, one, four);
       if (missing == 0)
         return;
       lone = true;
@@ -798,34 +781,56 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
   __syncthreads();
   if (*all_up == 0) return;
   if (tid < p.num_splits) store_device(pml, (tid * cols + cols - 1) * 8, u32x2_t{0u, 0u});
-  // Every partial of a thread's share is asked for before the first is used.  More than kFewRows rows have a group each and all their
-  // partials in one round (15 rows of 12 partials, us, in two parts and four rounds / so in two: 12.65 / 11.2).
-  constexpr int NG = 2 * NW;
-  const int d4 = tid & 31;
-  auto fold = [&](auto depth) {
-    const int parts = fold_parts(p.num_splits, all_rows);
-    constexpr int D = decltype(depth)::value;
-    const int at_once = NG / parts, part = (tid >> 5) / at_once;
-    for (int c0 = 0; c0 < rows; c0 += at_once) {
-      const int c = c0 + (tid >> 5) % at_once;
-      RowFold f;
-      u32x2_t ml[D];
-      f32x4_t ov[D];
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const int slot = min(part + parts * j, p.num_splits - 1) * cols + min(c, rows - 1);
-        ml[j] = load_device2(pml, slot * 8);
-        ov[j] = load_device(po, slot * kHeadDim * 4 + d4 * 16);
-      }
-      f.take(ml, ov, part, parts, p.num_splits);
-      if (parts > 1) f.template merge<2 * NW>(reinterpret_cast<float *>(lds) + 16, parts, at_once);
-      if (part == 0 && c < rows) f.template store<T>(p.out, token, c, kvh, Hkv, g, (int)(c * row_part >> 16), d4);
-    }
+  // Every partial of a thread's share is asked for before the first is used: up to 8 of a row are a group of 32 threads' each, more of up
+  // to 4 rows have a part in each group (NW = 4).
+  const int c = tid >> 5, d4 = tid & 31;
+  auto ask = [&](int s, int row, u32x2_t &ml, f32x4_t &ov) {
+    const int slot = min(s, p.num_splits - 1) * cols + min(row, rows - 1);
+    ml = load_device2(pml, slot * 8);
+    ov = load_device(po, slot * kHeadDim * 4 + d4 * 16);
   };
-  if (NW == 4 && all_rows > kFewRows && p.num_splits > kFoldDepth)
-    fold(std::integral_constant<int, kMaxFoldSplits>());
-  else
-    fold(std::integral_constant<int, kFoldDepth>());
+  PartialSum sum;
+  if (NW == 2 || p.num_splits <= kFoldDepth) {
+    u32x2_t ml[kFoldDepth];
+    f32x4_t ov[kFoldDepth];
+#pragma unroll
+    for (int j = 0; j < kFoldDepth; ++j) ask(j, c, ml[j], ov[j]);
+    sum.take(ml, ov, p.num_splits);
+  } else {
+    constexpr int kRows = 4;
+    static_assert(NW == 2 || kParts == 2 * NW, "a part per group");
+    u32x2_t ml[kRows][2], part_ml[kParts];
+    f32x4_t ov[kRows][2], part_o[kParts];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) ask(c + kParts * j, r, ml[r][j], ov[r][j]);
+    float *red_ml = reinterpret_cast<float *>(lds) + 16, *red_o = red_ml + 2 * kRows * kParts;
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+      PartialSum of_part;
+      of_part.take(ml[r], ov[r], c + kParts < p.num_splits ? 2 : 1);
+      if (d4 == 0) *reinterpret_cast<float2 *>(red_ml + 2 * (r * kParts + c)) = float2{of_part.M, of_part.L};
+      *reinterpret_cast<f32x4_t *>(red_o + (r * kParts + c) * kHeadDim + 4 * d4) = of_part.o;
+    }
+    __syncthreads();
+    if (c < rows) {
+#pragma unroll
+      for (int i = 0; i < kParts; ++i) {
+        part_ml[i] = *reinterpret_cast<const u32x2_t *>(red_ml + 2 * (c * kParts + i));
+        part_o[i] = *reinterpret_cast<const f32x4_t *>(red_o + (c * kParts + i) * kHeadDim + 4 * d4);
+      }
+      sum.take(part_ml, part_o, kParts);
+    }
+  }
+  if (c < rows) {
+    const int r = (int)(c * row_part >> 16);
+    const float inv = (sum.L > 0.0f) ? 1.0f / sum.L : 0.0f;
+    u32x2_t w;
+    w[0] = E::pack2(sum.o[0] * inv, sum.o[1] * inv);
+    w[1] = E::pack2(sum.o[2] * inv, sum.o[3] * inv);
+    *reinterpret_cast<u32x2_t *>(p.out + (((size_t)token + r) * H + kvh * g + c - r * g) * kRowBytes + d4 * 8) = w;
+  }
 }
 
 // Folds the splits of one output row (one query row of one head) with the log-sum-exp rule.
@@ -943,7 +948,7 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus, int r
   }
   if (s == 1) return t;
   if (s == nblocks && 2 * s <= kFoldDepth && pairs * (s == 2 ? 6 : 2 * s) <= cus && rows < kDecCols / 2) return t + 0.9;
-  return t + (s <= kFoldDepth ? 2.0 : s <= kMaxFoldSplits ? 1.8 : 1.4);
+  return t + (s <= kFoldDepth ? 2.0 : s <= 16 ? 1.8 : 1.4);
 }
 // The smallest count within `tolerance` of the best, or one that fills up to full_rounds rounds exactly.
 template <typename Model>
@@ -1027,7 +1032,7 @@ size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
     if (rest > 0) t += kb_of(splits) / (((nblocks + splits - 1) / splits >= 8 ? 47.5 : 49.0) - 18.5 * (double)rest / cus) + 3.05;
     if (splits == 1) return t;
     if (splits == nblocks && 2 * splits <= kFoldDepth && 2 * pairs * splits <= cus) return t + 1.2;
-    return t + (splits <= kFoldDepth ? 2.0 : splits <= kMaxFoldSplits ? 2.6 : 2.1);
+    return t + (splits <= kFoldDepth ? 2.0 : splits <= 16 ? 2.6 : 2.1);
   });
   return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, coarse < before ? coarse : before);
 }
@@ -1124,33 +1129,37 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   // partials take no more room (one column is the flag's: up to 7 query rows).  More than 8 such blocks, with some CUs left to
   // the folders, for one token of one sequence only: in the fused step each wave of a CU takes in the query and the table beside its keys (us,
   // blocks of 128 / 64: 700 keys of 4 kv heads 5.88 / 5.6, 1500 6.28 / 5.83, 1500 of 2 5.95 / 5.54, 1200 of 8 6.21 / 5.91; but unfused 2 x 900
-  // of 4 5.33 / 5.69, and without CUs for the folders 2000 of 8 6.45 / 6.57), and the unfused call gives the same bits.
+  // of 4 5.33 / 5.69, and without CUs for the folders 2000 of 8 6.45 / 6.57), and the unfused call gives the same bits.  They need the room that
+  // folders take: in an exact workspace 5 to 7 rows keep blocks of 128, which folders fit (unfused, 28 + 4 heads, blocks of 64 by flags
+  // or a second launch / so: 1000 keys 8.5 / 5.0, 1030 5.86 / 5.39).
   const int half_blocks = (p.n + kDecStepKeys / 2 - 1) / (kDecStepKeys / 2), cus = device_compute_units();
-  const long long half_wgs = (long long)p.batch * p.Hkv * half_blocks;
+  const long long pairs = (long long)p.batch * p.Hkv, half_wgs = pairs * half_blocks;
+  auto tags_fit = [&](int splits) { return pairs <= kTaggedPairs && (size_t)pairs * splits * p.rows * kTaggedBytes <= workspace_bytes; };
   const bool half = p.num_splits > 1 && p.num_splits == nblocks && p.rows < kDecCols / 2 &&
                     (half_blocks <= kFoldDepth ? half_wgs <= cus
-                                               : p.batch == 1 && p.m == 1 && half_blocks <= 2 * kMaxFoldSplits && half_wgs <= cus - cus / 16);
+                                               : p.batch == 1 && p.m == 1 && half_blocks <= 32 && half_wgs <= cus - cus / 16 &&
+                                                     tags_fit(half_blocks));
   if (half) {
     p.num_splits = nblocks = half_blocks;
     p.cols = kDecCols / 2;
   }
   p.iters_each = nblocks / p.num_splits;
   p.iters_rest = nblocks % p.num_splits;
-  // Up to 16 partials are folded by the decode kernel itself instead of a second launch.
-  FoldMode how = p.num_splits > 1 && p.num_splits <= kMaxFoldSplits && p.rows < p.cols ? kFoldByFlags : kNoFold;
+  // Without folders, few partials of few rows are folded by the workgroup that finds them all stored.  It takes in every one of them, and that is what
+  // more of either wait for (captured calls, us, flags / a second launch, which a graph brings at no cost to the host: the fused step, 1000 keys of 28 +
+  // 4 heads, 16 partials of 7 rows, 9.3 / 6.6, 2048 of 40 + 8, 16 of 5, 9.0 / 7.4, 153 of 28 + 4, 4 of 7, 6.9 / 6.4; 522 of 30 + 2, 5 of 15,
+  // 7.48 / 7.06; but 474 of 32 + 32, 8 of one, 6.24 / 6.57, 496 of 16 + 2, 4 of 8, 6.57 / 6.75, 3 tokens past 3021 of 16 + 16, 16 of 3, 8.68 / 9.18).
+  const int few_rows = p.num_splits <= kFoldDepth ? (half ? 4 : 8) : p.num_splits <= 16 && !half ? 4 : 0;
+  FoldMode how = p.num_splits > 1 && p.rows <= few_rows ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
   // Up to 128 partials by folders (more than 8 rows where the room is larger than a call may insist on: with tags they take more), as many of them as
   // the CUs that the other workgroups leave idle can take, down to one row each.
   // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones.
-  const long long pairs = (long long)p.batch * p.Hkv;
-  const size_t tagged = (size_t)pairs * p.num_splits * p.rows * kTaggedBytes;
-  if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && pairs <= kTaggedPairs &&
-      tagged <= workspace_bytes && !may_be_capturing(stream)) {
+  if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && tags_fit(p.num_splits) && !may_be_capturing(stream)) {
     how = kFoldByTags;
     if (p.fold == 0) p.fold = launch_number();
-    const int parts = fold_parts(p.num_splits, p.rows);
     const long long idle = device_compute_units() - pairs * p.num_splits;
-    p.fold_rows = half ? (parts > 4 ? 1 : 2) : 4 / (parts > 4 ? 4 : parts);
+    p.fold_rows = p.num_splits > 16 ? 1 : half || (p.num_splits > kFoldDepth && p.rows <= 8) ? 2 : 4;
     while (p.fold_rows > 1 && pairs * ((2 * p.rows + p.fold_rows - 1) / p.fold_rows) <= idle) p.fold_rows /= 2;
     p.folders = (p.rows + p.fold_rows - 1) / p.fold_rows;
     p.folders_div = make_fast_div((uint32_t)p.folders);

@@ -1,0 +1,38 @@
+"""Captured decode steps whose partials no folder takes in: 9 to 16 blocks of 64 keys must not take longer than 32 of them (one workgroup that
+takes in every partial of 7 rows took 1.4 times as long), and 16 blocks of 128 not longer than 17."""
+import pytest
+
+from helpers import DT_BFLOAT16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,Hkv,keys,more_keys", [(28, 4, 1000, 2040), (7, 1, 1000, 2040), (40, 8, 2048, 2176)])
+def test_time_of_a_captured_step(H, Hkv, keys, more_keys):
+    import torch
+    import llm_simple_amd.ops as ops
+
+    def microseconds(n):
+        rows = lambda *shape: torch.zeros(*shape, 128, dtype=torch.int16, device="cuda")
+        args = (rows(1, H), rows(n, Hkv), rows(n, Hkv), torch.zeros(n, 64, 2, device="cuda"), rows(1, H), rows(1, Hkv), rows(1, Hkv), n - 1,
+                H // Hkv, Hkv, 128, True, DT_BFLOAT16)
+        side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        ops.hip_decode_step_gqa_layer(*args, side.cuda_stream)
+        side.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            for _ in range(40):
+                ops.hip_decode_step_gqa_layer(*args, torch.cuda.current_stream().cuda_stream)
+        times = []
+        for _ in range(15):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 1e3 / 40)
+        return sorted(times)[len(times) // 2]
+
+    # 64 and 128 keys more are 0.1 us; a tenth is more than the medians of two runs differ
+    few, more = microseconds(keys), microseconds(more_keys)
+    assert few <= 1.1 * more, (few, more)

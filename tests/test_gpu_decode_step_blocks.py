@@ -1,6 +1,6 @@
 """The fused decode step in blocks of 64 keys: 8, 9, 16, 17 and 32 of them, a last block of one key and a whole one, one block more than
 the form takes, no CU left to the workgroups that fold, 7 query rows and 8 -- against the oracle, the same bits when repeated and from a
-HIP graph, which folds by flags (up to 16 blocks) or by a second launch."""
+HIP graph, which folds by flags (up to 8 blocks, 4 rows) or by a second launch."""
 import numpy as np
 import pytest
 
