@@ -28,9 +28,10 @@
 // Up to 128 partials of a (sequence, kv head) are folded (log-sum-exp) by workgroups of the same launch that do nothing else
 // (folders): every word of a partial goes past the XCD's L2 (sc1 stores) with half of the launch's number beside it, and a folder
 // looks at all of them until it finds the number everywhere.  That is one way to memory and one back; no fence, no flag, no atomic.
-// Folders have the highest workgroup numbers, so that they are dispatched after the workgroups that they wait for, and on
-// idle CUs if there are any; a folder that has looked in vain for some 50 ms computes its rows from the caches by itself, so that nothing
-// depends on the order of dispatch.  A look costs what its loads cost: a wave per row, two dims per lane, the maxima and
+// Folders have the highest workgroup numbers, so that an XCD dispatches them after the workgroups of their own launch, and on
+// idle CUs if there are any.  Of launches on two streams one's folders can hold the CUs that the other's workgroups wait for, and the other way
+// round on another XCD: a folder that has looked in vain for long (see fold_looks) computes its rows from the caches by itself, so that nothing
+// depends on the order of dispatch but time, and a row's last bits.  A look costs what its loads cost: a wave per row, two dims per lane, the maxima and
 // sums of all partials in one load (two rows per wave with three loads per partial: 1.5 us a look, 0.6 now).
 // (Fused step, us, the last workgroup to store folds / folders: 384 keys of 2 kv heads 5.52 / 4.85, 512 of 32 5.23 / 5.01, 32768 of 8, with
 // a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1; beyond 32 partials, a combine launch / folders: 4700 keys of
@@ -80,7 +81,7 @@ struct DecodeLate {
   float *ws_ml;  // [batch][Hkv][splits][cols][2]; fold: the last column's place is the flag of the split
   int num_splits;
   int iters_each, iters_rest;  // blocks per split: iters_each, one more for the first iters_rest splits
-  int fold_rows, folders;  // by tags: rows of a folder, folders of a (sequence, kv head)
+  int fold_rows, folders;  // by tags: rows of a folder and, 8 bits on, the looks that it takes; folders of a (sequence, kv head)
   FastDiv folders_div;
   uint64_t fold;  // the launch's number: what the flags hold, or halves of it beside the words of a partial
 };
@@ -184,11 +185,18 @@ constexpr int kMaxTaggedSplits = 128;
 constexpr int kTaggedBytes = (kHeadDim + 2) * 8;  // a row of a partial whose words carry a tag
 constexpr int kTaggedPairs = 1023;                // (sequence, kv head) pairs, at most
 constexpr int kFoldDepth = 8;                     // partials that are summed in one part
+// Looks that a folder takes, 0.6 us each or more: what its whole cache takes one workgroup, eight times over, and 0.3 ms.  It is there for
+// launches on two streams (see above), which a wait of any length only holds up; too short a wait makes work, and rows summed in another order,
+// where other kernels hold the workgroups up that it waits for.
+static int fold_looks(int nblocks) {
 #ifdef LLMHIP_BENCH
-constexpr int kFoldPolls = 0;  // (the measurement library's copy: every folder computes its rows by itself)
+  return 0;  // (the measurement library's copy: every folder computes its rows by itself)
 #else
-constexpr int kFoldPolls = 1 << 16;  // looks that a folder takes, 0.6 us each
+  constexpr double kBlockUs = 2.0 * kRowBytes * kDecStepKeys * 1e-3 / 27.9, kLookUs = 0.6;  // (a CU's share of the memory system, see split_model_us)
+  const double looks = (300.0 + 8.0 * kBlockUs * nblocks) / kLookUs;
+  return looks < 1 << 16 ? (int)looks : 1 << 16;
 #endif
+}
 // Parts that a row's partials are summed in before those sums are: part i has splits i, i + parts, ...  That is the order of the
 // combine launch, so that all ways to fold give the same bits.
 constexpr int kParts = 8;
@@ -254,7 +262,7 @@ __device__ __forceinline__ float lane_value(float x, int lane) {
 // A folder: rows c0 .. c0 + fold_rows - 1 of a pair, from partials whose words carry this launch's tags.  A wave has a row, two
 // dims per lane, and PARTS of the fold_parts() parts of its partials, DEPTH in all.  It looks at all of them until it finds the tags
 // at every word.  A part's partials are summed ROUND at a time, as in the combine launch.  have_rows: of the pair's rows, those that
-// are there (a short last tile).  A bit per row c0 + i that was not stored: its partials were not there after kFoldPolls looks.
+// are there (a short last tile).  A bit per row c0 + i that was not stored: its partials were not there after all looks.
 template <typename T, int NW, int DEPTH, int PARTS, int ROUND>
 __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t row_part, char *lds, int pair, int token, int kvh, int c0, int rows,
                                                 int have_rows, int Hkv, int g) {
@@ -262,7 +270,7 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, S = p.num_splits;
   constexpr int parts = PARTS > 1 ? kParts : 1, per_row = parts / PARTS, at_once = NW / per_row;
   const int part = wave / at_once, c = c0 + wave % at_once;
-  const bool mine = wave % at_once < p.fold_rows && c < have_rows;  // (of the wave)
+  const bool mine = wave % at_once < (p.fold_rows & 0xff) && c < have_rows;  // (of the wave)
   const int bytes = S * rows * kTaggedBytes;
   const __amdgpu_buffer_rsrc_t pt = byte_buffer(reinterpret_cast<char *>(p.ws_o) + (size_t)pair * bytes, bytes);
   const uint32_t tag0 = (uint32_t)p.fold, tag1 = (uint32_t)(p.fold >> 32);
@@ -284,7 +292,7 @@ __device__ __forceinline__ uint32_t fold_tagged(const DecodeLate &p, uint32_t ro
     const int at_ml = have ? (my_split * rows + c) * kTaggedBytes + kHeadDim * 8 : 0x40000000;
     u32x4_t a[DEPTH] = {}, ml = {};
     there = false;
-    for (int looks = 0; looks < kFoldPolls; ++looks) {
+    for (int looks = p.fold_rows >> 8; looks > 0; --looks) {
       asm volatile("" ::: "memory");  // (the loads are made again)
       ml = __builtin_bit_cast(u32x4_t, load_device(pt, at_ml));
 #pragma unroll
@@ -439,7 +447,7 @@ __global__ __launch_bounds__(64 * NW) void flash_decode_kernel(addresses_t ea, u
       if (e >= pairs * f.folders) return;
       pair = (int)fast_div(e, f.folders_div);
       b = FUSED ? 0 : (int)(pair * (eb[3] >> 10) >> 20);
-      const int c0 = (e - pair * f.folders) * f.fold_rows;
+      const int c0 = (e - pair * f.folders) * (f.fold_rows & 0xff);
       auto fold = [&](auto depth, auto parts, auto round) {
         return fold_tagged<T, NW, decltype(depth)::value, decltype(parts)::value, decltype(round)::value>(f, row_part, lds, pair, token_of(b), pair - b * Hkv,
                                                                                                           c0, all_rows, rows_from(token_of(b)), Hkv, g);
@@ -1163,6 +1171,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
     while (p.fold_rows > 1 && pairs * ((2 * p.rows + p.fold_rows - 1) / p.fold_rows) <= idle) p.fold_rows /= 2;
     p.folders = (p.rows + p.fold_rows - 1) / p.fold_rows;
     p.folders_div = make_fast_div((uint32_t)p.folders);
+    p.fold_rows |= fold_looks((p.n + kDecStepKeys - 1) / kDecStepKeys) << 8;
   }
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
   p.ws_o = static_cast<float *>(workspace);

@@ -87,6 +87,34 @@ def test_graph_capture_and_replay():
             assert np.array_equal(a, b), f"replay {rep}"
 
 
+@pytest.mark.parametrize("shapes", [((16, 2000, 40, 8, 2), (16, 2000, 40, 8, 2)), ((16, 1200, 28, 4, 5), (1, 20000, 12, 2, 120)), ((5, 2999, 40, 8, 6), (3, 4000, 32, 32, 9))])
+def test_two_streams_fold_at_once(shapes):
+    """Launches on two streams whose partials are folded by workgroups that wait for them, as many of those as the device has compute units: each
+    result is that of the call alone, up to the order of a sum (a folder that has waited too long sums its row in one part)."""
+    import torch
+    import llm_simple_amd.ops as ops
+    dt, calls = DT_BFLOAT16, []
+    for i, (batch, n, H, Hkv, splits) in enumerate(shapes):
+        q = to_dev(normal_bits(10 * i, (batch, 1, H, 128), dt))
+        k, v = (to_dev(normal_bits(10 * i + s, (batch, n, Hkv, 128), dt)) for s in (1, 2))
+        ws = torch.zeros(2 * ops.flash_decode_workspace_bytes(batch, H // Hkv, Hkv, 128, splits), dtype=torch.uint8, device="cuda")
+        args = (q, k, v, ws, ws.numel(), batch, n, n, H // Hkv, Hkv, 128, splits, dt)
+        alone, outs, stream = dev_empty(q.shape), [dev_empty(q.shape) for _ in range(20)], torch.cuda.Stream()
+        torch.cuda.synchronize()
+        ops.hip_flash_decode_gqa_layer(alone, *args, stream.cuda_stream)
+        stream.synchronize()
+        calls.append((alone, outs, args, stream))
+    for turn in range(20):
+        for _, outs, args, stream in calls:
+            ops.hip_flash_decode_gqa_layer(outs[turn], *args, stream.cuda_stream)
+    torch.cuda.synchronize()
+    for alone, outs, _, _ in calls:
+        want = orc.widen(to_host(alone), dt)
+        for o in outs:
+            # one part or several: sums of at most 20000 products in 32 bits, far below half a step of 2^-8 of bf16, so a step at most
+            assert (np.abs(orc.widen(to_host(o), dt) - want) <= 2.0 ** -7 * np.abs(want) + 1e-6).all()
+
+
 def test_scratch_does_not_grow_under_capture():
     """A reference-signature call whose per-stream scratch would have to grow while its stream is being captured
     is refused with LLMHIP_ERR_WORKSPACE (growing allocates), and the capture stays usable: what fits the buffer
