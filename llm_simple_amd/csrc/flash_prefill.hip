@@ -1031,13 +1031,14 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
     // one / clusters: 14 tokens past 25506 keys of 28 + 4 heads, 2 tiles, 23.9 / 18.5; 17 past 10561 of 12 + 2, 4 tiles, 13.3 / 10.8; 62 past
     // 30822 of 8 + 1, 16 tiles, 26.5 / 22.9; but 5 tiles of 4 kv heads 15.6 / 16.2, 12 26.5 / 27.9, and with 29 to a cluster 1.25 times).
     const int heads_xcds = p.Hkv % 8 == 0 ? 8 : p.Hkv % 4 == 0 ? 4 : p.Hkv % 2 == 0 ? 2 : 1;
-    if (T_ > 1 && heads_xcds < 8 && T_ * heads_xcds <= 16) {
-      const int clusters = (T_ + kClusterTiles - 1) / kClusterTiles, each = (T_ + clusters - 1) / clusters;
+    const int clusters = (T_ + kClusterTiles - 1) / kClusterTiles, each = (T_ + clusters - 1) / clusters;
+    // (16-bit reciprocals of 1 to 6 are exact below 16384 items of a cluster; over 256 compute units plans have up to 5940)
+    if (T_ > 1 && heads_xcds < 8 && T_ * heads_xcds <= 16 && (long long)each * p.Hkv * S_ < 16384) {
       const int last = (T_ - 1) % each + 1;
       p.per_xcd = (grid + 7) / 8;
       grid = 8 * p.per_xcd;
       p.tiles = (uint32_t)(each | last << 8);
-      p.each_part = 65536u / each + 1;  // (exact below 10922 items of a cluster: 6 tiles x 7 kv heads x 128 ranges are 5376)
+      p.each_part = 65536u / each + 1;
       p.last_part = 65536u / last + 1;
       p.per_list = make_fast_div((uint32_t)(each * p.Hkv * S_));
     }
