@@ -68,9 +68,10 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
 
 /* How many bytes of the library's per-stream scratch buffer a llmhip_flash_attn* call with these
  * arguments uses (head_num of the MHA entry points = kv_head_num with group_size 1): the fp32
- * partials of the split-KV decode kernel (m * group_size <= 16) or of a key-range split of the
- * prefill kernel (a chunk behind at least as many cached tokens, wherever the split is faster; at
- * most 256 MiB); 0 for ordinary prefill shapes.  The buffer is allocated on the first call that
+ * partials of the split-KV decode kernel (m * group_size <= 16, and a few tokens more over a short
+ * cache, which it takes in tiles of up to 16 rows) or of a key-range split of the prefill kernel (a
+ * chunk behind at least as many cached tokens, wherever the split is faster; at most 256 MiB); 0 for
+ * ordinary prefill shapes.  The buffer is allocated on the first call that
  * needs it on a stream (a power of two, at least 4 MiB) and replaced by a larger one when a later
  * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
  * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or
@@ -92,9 +93,9 @@ size_t llmhip_flash_attn_scratch_bytes(int m, int n, int offset, int group_size,
  * The reference has no batch dimension and no split-KV (decode there is
  * npu_flash_attn_gqa_layer with m = 1, src/llama2_layer_npu.cpp:866-869);
  * for batch == 1 this call returns what llmhip_flash_attn_gqa(m=1,
- * offset=n-1) returns.  num_splits <= 0 picks llmhip_flash_decode_default_splits, or
- * over a short cache (see llmhip_flash_attn_scratch_bytes) fewer where the workspace holds
- * fewer; values above 256 are treated as 256.
+ * offset=n-1) returns.  num_splits <= 0 picks a count (see llmhip_flash_decode_default_splits), and
+ * a smaller one where the workspace holds no more, unless that is much slower (over a long cache, see
+ * llmhip_flash_attn_scratch_bytes: LLMHIP_ERR_WORKSPACE); values above 256 are treated as 256.
  * workspace: device memory of at least llmhip_flash_decode_workspace_bytes()
  * bytes, owned by the caller, so that the call allocates nothing. */
 int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,
@@ -110,8 +111,10 @@ int llmhip_flash_decode_gqa(void *out, const void *q, const void *k_cache,
 size_t llmhip_flash_decode_workspace_bytes(int batch, int group_size, int kv_head_num,
                                            int head_dim, int num_splits);
 
-/* The split count the decode call uses for num_splits <= 0: about one workgroup per compute unit of the
- * current device, from a small model of the launch (whole rounds of workgroups preferred). */
+/* The split count that the decode calls use for num_splits <= 0 with up to 7 query heads per kv head: about one
+ * workgroup per compute unit of the current device, from a small model of the launch.  With 8 to 16 query heads per
+ * kv head a call over a short cache may use fewer (256 keys of one sequence: one, where this says 2), because their
+ * partials take longer to fold. */
 int llmhip_flash_decode_default_splits(int batch, int n, int kv_head_num);
 
 /* llmhip_flash_decode_gqa for callers that cannot allocate device memory or carry a workspace

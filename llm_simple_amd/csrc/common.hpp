@@ -17,9 +17,9 @@
 #include <type_traits>
 #include <utility>
 
-// The measurement library (libllmhip_bench.so) compiles the prefill kernel a second time with
-// LLMHIP_BENCH defined (a clock stamp in the kernel); its copy lives in a namespace of its own so
-// that the two libraries never share a symbol.
+// The measurement library (libllmhip_bench.so) compiles the prefill and decode kernels a second time with
+// LLMHIP_BENCH defined (a clock stamp in the prefill kernel, folders that do not wait in the decode kernel); its
+// copies live in a namespace of their own so that the two libraries never share a symbol.
 #ifdef LLMHIP_BENCH
 #define LLMHIP_NS llmhip_bench
 #else

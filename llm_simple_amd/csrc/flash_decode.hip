@@ -34,8 +34,9 @@
 // depends on the order of dispatch but time, and a row's last bits.  A look costs what its loads cost: a wave per row, two dims per lane, the maxima and
 // sums of all partials in one load (two rows per wave with three loads per partial: 1.5 us a look, 0.6 now).
 // (Fused step, us, the last workgroup to store folds / folders: 384 keys of 2 kv heads 5.52 / 4.85, 512 of 32 5.23 / 5.01, 32768 of 8, with
-// a combine launch before, 24.2 / 23.6; 5 x 2999 keys of 8 13.9 / 13.1; beyond 32 partials, a combine launch / folders: 4700 keys of
-// 4 kv heads 7.92 / 7.06, 14000 10.45 / 9.62, 31000 15.2 / 14.5, 6000 of 2 7.77 / 6.68, 20000 10.25 / 9.58.)
+// a combine launch before, 24.25 / 23.93; 5 x 2999 keys of 8 13.9 / 13.1; beyond 32 partials, a combine launch / folders: 4700 keys of
+// 4 kv heads 7.92 / 7.06, 14000 10.45 / 9.62, 31000 15.2 / 14.5, 6000 of 2 7.77 / 6.68, 20000 10.25 / 9.58.  Since a folder reads the sums of
+// its parts at once, 32768 of 8 23.9 -> 23.5.)
 // More than 8 query rows (a few tokens checked at once) take folders where the room is there, with tags twice that of the partials (rope
 // and attention, us, flags or a combine launch / folders: 2 tokens past 1200 keys of 28 + 4 heads 10.1 / 7.8, past 20000 14.1 / 13.3, 3 past
 // 1500 of 40 + 8 11.1 / 8.4, 12 past 900 of 32 + 32 10.9 / 9.15).
@@ -1160,7 +1161,8 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   const int few_rows = p.num_splits <= kFoldDepth ? (half ? 4 : 8) : p.num_splits <= 16 && !half ? 4 : 0;
   FoldMode how = p.num_splits > 1 && p.rows <= few_rows ? kFoldByFlags : kNoFold;
   p.fold = how != kNoFold ? launch_number() : 0;
-  // Up to 128 partials by folders (more than 8 rows where the room is larger than a call may insist on: with tags they take more), as many of them as
+  // Up to 128 partials by folders (more than 8 rows where the room is larger than a call may insist on: with tags they take more, and a full round of
+  // 256 workgroups with 16 rows more than a stream's first 4 MiB of scratch: 32 kv heads fold by a second launch until a call has made it grow), as many of them as
   // the CUs that the other workgroups leave idle can take, down to one row each.
   // A replayed graph launches with the number of its capture, and words of the replay before would pass for new ones.
   if (p.num_splits > 1 && p.num_splits <= kMaxTaggedSplits && tags_fit(p.num_splits) && !may_be_capturing(stream)) {
@@ -1209,8 +1211,8 @@ int flash_decode_tiles(int m, int group_size) {
 }
 
 // Tiles read their keys each for itself, so that it is the short calls that they are for, those that wait for one workgroup's chain and
-// the fold: up to 40000 keys of all tiles and kv heads, and from where a chunk's workgroups of all keys take longer (attention, us,
-// key ranges and a combine launch / tiles: 3 tokens past 1000 keys of 28 + 4 heads 8.13 / 5.89, 8 past 2000 8.62 / 7.75, 6 past 1000 of 12 + 2
+// the fold: up to 40000 keys of all tiles and kv heads, and from where a chunk's workgroups of all keys take longer (lines measured with 256
+// compute units; attention, us, key ranges and a combine launch / tiles: 3 tokens past 1000 keys of 28 + 4 heads 8.13 / 5.89, 8 past 2000 8.62 / 7.75, 6 past 1000 of 12 + 2
 // 7.95 / 5.60, 4 past 4000 8.17 / 7.04, 6 past 2000 of 40 + 8 8.69 / 7.84; but 6 past 4000 of 28 + 4 8.92 / 9.50 (49000), 12 past 500 of 40 +
 // 8 6.43 / 6.80, and of 32 heads of one kv head each 32 past 500 7.2 / 8.35).
 bool flash_decode_takes_tiles(int m, int n_vis, int group_size, int kv_head_num) {

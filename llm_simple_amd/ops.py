@@ -127,6 +127,8 @@ def flash_decode_workspace_bytes(batch, group_size, kv_head_num, head_dim, num_s
 
 
 def flash_decode_default_splits(batch, n, kv_head_num):
+    """The split count of a decode call with num_splits <= 0 and up to 7 query heads per kv head (8 to 16: over a short
+    cache perhaps fewer)."""
     return lib.llmhip_flash_decode_default_splits(batch, n, kv_head_num)
 
 

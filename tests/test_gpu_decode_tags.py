@@ -1,7 +1,7 @@
 """Decode partials whose words carry a tag: the edges of that form (8 splits and 9, 8 query rows and 9, one row, a workspace
-that holds no more than the flags need, workgroups that read 6.4 and 7.5 MB together), calls that take turns on one workspace so
+that holds no more than an exact call needs, 96 and 112 partials of 8 rows), calls that take turns on one workspace so
 that each finds the words of another, and a workspace full of numbers that look like tags.  Against the oracle, and bit for bit
-against the same call from a HIP graph, which folds by flags."""
+against the same call from a HIP graph, which folds by flags (up to 8 partials of 8 rows, 16 of 4) or by a second launch."""
 import numpy as np
 import pytest
 

@@ -117,6 +117,18 @@ def test_workspace_of_an_earlier_default_count_is_enough(batch, n, Hkv, splits, 
     assert (rc > 0) == taken and (rc == -3) != taken, rc  # (taken: as far as the launch, which finds no device)
 
 
+def test_default_split_count_is_for_up_to_seven_query_heads():
+    """A call with 8 or more query rows per kv head, whose partials take longer to fold, may use fewer parts than the default count
+    says, which is for fewer."""
+    import llm_simple_amd.ops as ops
+    for n in (129, 200, 256):
+        for Hkv in (1, 2, 5):
+            splits = ops.flash_decode_default_splits(1, n, Hkv)
+            assert splits == 2
+            assert ops.lib.llmhip_flash_attn_scratch_bytes(1, n, n - 1, 7, Hkv) == ops.flash_decode_workspace_bytes(1, 7, Hkv, 128, splits)
+            assert ops.lib.llmhip_flash_attn_scratch_bytes(1, n, n - 1, 8, Hkv) == 0
+
+
 def test_cpp_device_layer_host_checks():
     exe = os.path.join(ROOT, "tests", "cpp", "bin", "test_device_host")
     if not os.path.exists(exe):
