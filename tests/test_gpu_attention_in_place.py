@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 # (m, past, H, Hkv): tiles of rows are those of 3 to 63 tokens; 8 tiles of 4 kv heads in 8 to 11 parts, and of 8 in 9, are two rounds
 @pytest.mark.parametrize("m,past,H,Hkv", [(1, 700, 28, 4), (2, 3000, 28, 4), (4, 1200, 28, 4), (5, 1000, 28, 4), (7, 900, 40, 8), (15, 1100, 28, 4),
                                           (22, 1300, 40, 8), (29, 1200, 16, 4), (57, 1200, 8, 4), (9, 1500, 16, 1), (61, 700, 4, 2), (30, 4130, 40, 8),
-                                          (33, 8160, 28, 4), (200, 0, 12, 2), (1019, 0, 28, 4), (2100, 0, 40, 8)])
+                                          (33, 8160, 28, 4), (200, 0, 12, 2), (512, 0, 28, 4), (1019, 0, 28, 4), (1700, 0, 28, 4),
+                                          (2100, 0, 40, 8), (3500, 0, 28, 4), (400, 1000, 32, 32)])
 @pytest.mark.parametrize("dt", [DT_FLOAT16, DT_BFLOAT16])
 def test_attention(dt, m, past, H, Hkv):
     import llm_simple_amd.ops as ops
