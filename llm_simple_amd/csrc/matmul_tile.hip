@@ -18,7 +18,7 @@
 // faster (4096 x 4096 62.3 / 57.9), the power it saves being small.
 //   Small tiles are bound by the barrier and the LDS latency of a stage, and take several lines per stage (32 x 32, four
 // lines instead of two: 512 x 3584, 400 rows 8.5 -> 7.8 us; 1536 x 1536, 100 rows 5.4 -> 4.9).  There the barrier comes so late that
-// the loads go out in a burst behind it: 32 x 32 all eight in the last of 8 slots, 64 x 32 twelve in the last two of 16.
+// the loads go out in a burst behind it: 32 x 32 all eight in the last of 8 slots, 64 x 32 (two lines) six in the last two of 8.
 // Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 2.6 until the first
 // lines are in, 56 stages of 0.67, 2.3 for the store (14.7 MB at once), the rest launch.  A stage takes 1120 cycles at
 // 1.68 GHz: the clock is what the power leaves (half of the chip: 1090 cycles at 2.2 GHz; without the line loads 1.9 GHz).
@@ -28,13 +28,24 @@
 // was one round trip more per pair of blocks (epilogue 6.2 us in the kernel of eight waves).
 //
 // Rows of the operands lie k elements apart, often a multiple of 4 KiB: workgroups that walk k in step would ask few
-// memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles a stage apart
+// memory channels for everything.  Each XCD starts at another eighth of k, neighbouring tiles of W rows a line apart
 // (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5, kernel of eight waves).
+//   A CU draws no more than 30 to 45 GB/s from beyond its XCD's L2, however much it has under way.  Tiles of the same W rows that
+// take the lines in one order leave all of that to the one that is ahead, and the others wait with it (3584 x 3584, 256 rows: 31 GB/s of
+// W to a tile of 64 rows, and as long with 112 workgroups as with 224).  So lines go in groups of 8, and each of up to 4 such tiles
+// begins at another place of a group: the first to ask for a line is a different one each time, and the rest find it in the L2 a moment later
+// (us, one order / so, W from HBM: 3584 x 3584, 64 rows 10.7 / 9.5, 256 18.5 / 14.6, 512 24.2 / 20.8, 1024 30.9 / 28.3, 2048 48.0 /
+// 46.5; 4096 x 4096, 256 rows 20.3 / 16.5; 5120 x 5120, 384 rows 36.9 / 31.0; 1024 x 5120, 128 rows 13.3 / 11.1).  Half or a quarter of k apart
+// instead, the small ones are as fast, but what the L2 has to keep in between outgrows it (3584 x 3584, 1024 rows 36.0); groups of 4 or 16 lose 1-3 %
+// either at the small or at the large sizes; turns by the tile's W rows too, for those that share lhs rows, change nothing.
+//   Stages under way: as few as hold 64 to 100 KiB, but for 96 x 64.  More of them are no faster anywhere, and begin with a longer burst (5 / 9 stages of a
+// 64 x 64 tile, us: 512 x 3584, 2048 rows 12.6 / 13.1, 3584 x 3584, 256 rows 14.15 / 14.55; 3 / 4 of 32 x 32, 512 x 3584, 512 rows 7.1 / 7.35;
+// 3 / 5 of 96 x 128, 3584 x 3584, 768 rows 24.0 / 24.9; one line to a stage less and four stages of 64 x 32: 256 x 1536, 2048 rows 5.65 / 5.45).
 //
 // bf16, us, hipBLASLt / here, back-to-back calls, W walked through 800 MB (hipBLASLt takes the host 10-13 us a call, which is
 // what its small sizes show): 3584 x 3584: 64 rows 13.7 / 11.1, 128 rows 22.5 / 14.5, 256 rows 20.1 / 18.8, 768 rows 32.2 / 26.8,
 // 2048 rows 55.9 / 47.0; 512 x 3584: 100 rows 13.4 / 7.1, 2048 rows 19.3 / 13.2; 1536 x 1536: 128 rows 9.7 / 5.7; 5120 x 5120: 100
-// rows 27.6 / 25.2, 1280 rows 76.1 / 59.8.
+// rows 27.6 / 25.2, 1280 rows 76.1 / 59.8 (before the order of lines above).
 #include <atomic>
 #include <type_traits>
 
@@ -89,7 +100,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
   const int band = (int)fast_div(t, by_band), rem = t - band * gm * n_tiles;
   const int rows_here = min(gm, m_tiles - band * gm);
   const int tn = rows_here == gm ? (int)fast_div(rem, by_rows) : rem / rows_here;
-  const int m0 = (band * gm + rem - tn * rows_here) * BM, n0 = tn * BN;
+  const int in_band = rem - tn * rows_here, m0 = (band * gm + in_band) * BM, n0 = tn * BN;
   const int wm = wave & 1, wn = wave >> 1;
   const int col0 = n0 + wn * (BN / 2);
 
@@ -131,8 +142,18 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
     line_load<1024 * (nth % 4)>(voff[s], is_w ? wk : xk);
   };
   const int lines = k / kLineK, stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
-  uint32_t kpos = (unsigned)(xcd * lines / 8 + (t & 3)) % (unsigned)lines * kStageRow;
-  auto advance = [&]() { kpos = kpos + kStageRow == row_bytes ? 0 : kpos + kStageRow; };
+  // The order of the lines: each XCD begins at another eighth, and in every group of 8 (4, 2: what divides k) each tile of those that share
+  // W rows at another place.  Not where a quarter of the last one is padding: begun ahead of the others it stays there, and fetches for them.
+  const bool padded = m_tiles <= kBandRows && 4 * (m - (m_tiles - 1) * BM) <= 3 * BM;
+  uint32_t pos = (((uint32_t)(xcd * lines) >> 3) + ((padded ? t : tn) & 3)) * kStageRow;
+  if (pos >= row_bytes) pos = 0;
+  const int group = lines % 8 == 0 ? 8 : lines % 4 == 0 ? 4 : lines % 2 == 0 ? 2 : 1;
+  const uint32_t turn = padded ? 0u : (uint32_t)(in_band * group >> (rows_here == 2 ? 1 : 2)) * kStageRow;
+  uint32_t kpos = pos ^ turn;
+  auto advance = [&]() {
+    pos = pos + kStageRow == row_bytes ? 0 : pos + kStageRow;
+    kpos = pos ^ turn;
+  };
 #pragma unroll
   for (int s = 0; s < STAGES * KS; ++s) {
     static_for<0, L>([&](auto l) { issue(l, wbase + kpos, xbase + kpos, s * kLineBytes); });
@@ -260,24 +281,30 @@ template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile
   return hipGetLastError();
 }
 
+// Lhs rows, features, lines of a stage and stages of the tiles; see tile_kind for their order
+#define LLMHIP_TILES(TILE)                                                                                            \
+  TILE(1, 1, 4, 3) TILE(1, 1, 4, 4) TILE(2, 1, 2, 4) TILE(1, 2, 2, 5) TILE(2, 2, 1, 5) TILE(3, 2, 1, 5) TILE(2, 3, 1, 4) TILE(4, 2, 1, 4) \
+  TILE(3, 3, 1, 4) TILE(3, 4, 1, 3) TILE(4, 3, 1, 4) TILE(4, 4, 1, 4) TILE(4, 5, 1, 4) TILE(4, 6, 1, 3) TILE(5, 5, 1, 3) \
+  TILE(4, 7, 1, 3) TILE(5, 6, 1, 3) TILE(4, 8, 1, 3)
+struct Tile {
+  int m, n;
+};
+constexpr Tile kTiles[] = {
+#define LLMHIP_TILE(MT, NT, KS, STAGES) {32 * MT, 32 * NT},
+    LLMHIP_TILES(LLMHIP_TILE)
+#undef LLMHIP_TILE
+};
+constexpr int kTileKinds = sizeof(kTiles) / sizeof(kTiles[0]), kDeep = 1, kTall = 2, kWide = 3;  // 32 x 32 with more stages, 64 x 32, 32 x 64
+static_assert(kTiles[kTall].m == 2 * kTiles[kTall].n && kTiles[kWide].n == 2 * kTiles[kWide].m, "");
+
 template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStream_t stream) {
-  switch (kind) {
-    case 0: return launch_tile<T, 1, 1, 4, 4>(c, stream);
-    case 1: return launch_tile<T, 2, 1, 4, 3>(c, stream);
-    case 2: return launch_tile<T, 2, 2, 1, 9>(c, stream);
-    case 3: return launch_tile<T, 3, 2, 1, 7>(c, stream);
-    case 4: return launch_tile<T, 4, 2, 1, 6>(c, stream);
-    case 5: return launch_tile<T, 3, 3, 1, 6>(c, stream);
-    case 6: return launch_tile<T, 3, 4, 1, 5>(c, stream);
-    case 7: return launch_tile<T, 4, 3, 1, 5>(c, stream);
-    case 8: return launch_tile<T, 4, 4, 1, 4>(c, stream);
-    case 9: return launch_tile<T, 4, 5, 1, 4>(c, stream);
-    case 10: return launch_tile<T, 4, 6, 1, 3>(c, stream);
-    case 11: return launch_tile<T, 5, 5, 1, 3>(c, stream);
-    case 12: return launch_tile<T, 4, 7, 1, 3>(c, stream);
-    case 13: return launch_tile<T, 5, 6, 1, 3>(c, stream);
-    default: return launch_tile<T, 4, 8, 1, 3>(c, stream);
-  }
+  using Launch = hipError_t (*)(const TileCall &, hipStream_t);
+  static constexpr Launch launch[] = {
+#define LLMHIP_TILE(MT, NT, KS, STAGES) launch_tile<T, MT, NT, KS, STAGES>,
+      LLMHIP_TILES(LLMHIP_TILE)
+#undef LLMHIP_TILE
+  };
+  return launch[kind](c, stream);
 }
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
@@ -288,15 +315,21 @@ template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStr
 // 8960, 17 rows 28.2 / 19.0, 3584 x 18944, 32 rows 109.6 / 48.4); 5120 x 5120, 64 rows 21.5 / 22.9; 4096 x 11008, 680 rows 80.5 /
 // 85.0.  More than one round is not: 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 /
 // 54.5 with 128 x 128.
+//   Of 64 x 32 and 32 x 64 the second where W is much the larger operand and next to nothing is padding: up to 4 tiles then share its rows,
+// and not two (us, 64 x 32 / 32 x 64: 3584 x 3584, 128 rows 12.5 / 11.7, 5120 x 5120, 64 rows 23.1 / 19.0, with 320 workgroups; but
+// 512 x 3584, 768 rows 9.5 / 9.9, 1536 x 1536, 256 rows 5.85 / 6.05, 3584 x 3584, 96 rows 11.4 / 12.5).
+//   32 x 32 with a stage more where W rows are fetched by one tile alone, or by one that is ahead of another, and many CUs do so: the longer way
+// to HBM wants more under way (3 / 4 stages: 3584 x 3584, 17 rows 9.4 / 9.25, 40 9.0 / 8.6; 4096 x 4096, 40 rows 9.55 / 9.1; 512 x 3584, 32 rows 6.3 / 6.5).
 int tile_kind(int m, int n, int k) {
-  static const struct { int m, n; } tiles[] = {{32, 32},   {64, 32},   {64, 64},   {96, 64},   {128, 64},
-                                               {96, 96},   {96, 128},  {128, 96},  {128, 128}, {128, 160},
-                                               {128, 192}, {160, 160}, {128, 224}, {160, 192}, {128, 256}};
   const long long cus = device_compute_units();
-  for (int kind = 0; kind < 15; ++kind) {
-    const long long count = (long long)((m + tiles[kind].m - 1) / tiles[kind].m) * ((n + tiles[kind].n - 1) / tiles[kind].n);
-    if (count <= cus) return kind;
-  }
+  auto count = [&](int kind) {
+    const Tile &t = kTiles[kind];
+    return (long long)((m + t.m - 1) / t.m) * ((n + t.n - 1) / t.n);
+  };
+  if (count(0) <= cus) return m <= 56 && 4 * count(0) >= cus && 4 * ((m - 1) % 32 + 1) <= (m <= 32 ? 128 : 96) ? kDeep : 0;
+  for (int kind = kTall; kind < kTileKinds; ++kind)
+    if (count(kind) <= cus)
+      return kind == kTall && n >= 16LL * m && count(kWide) <= cus && (m - 1) % 64 >= 56 ? kWide : kind;
   return -1;
 }
 
