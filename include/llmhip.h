@@ -71,7 +71,9 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
  * partials of the split-KV decode kernel (m * group_size <= 16, and a few tokens more over a short
  * cache, which it takes in tiles of up to 16 rows) or of a key-range split of the prefill kernel (a
  * chunk behind at least as many cached tokens, wherever the split is faster; at most 256 MiB); 0 for
- * ordinary prefill shapes.  The buffer is allocated on the first call that
+ * ordinary prefill shapes, which need none (prompts of some 900 to 1500 tokens, by the number of
+ * heads, use some MiB of the buffer where it can be had and the stream is not capturing: the longest
+ * rows are then shared by two workgroups each).  The buffer is allocated on the first call that
  * needs it on a stream (a power of two, at least 4 MiB) and replaced by a larger one when a later
  * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
  * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or

@@ -201,4 +201,25 @@ __device__ __forceinline__ void store_device_b128(void *p, u32x4_t v) {
   __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4_t *)p, v, "agent");
 }
 
+// Buffer descriptor of `bytes` bytes: a load past them returns zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t byte_buffer(const void *base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
+}
+constexpr int kNonTemporal = 2, kScopeDevice = 16;  // cache policy operand: nt; sc1, past the XCD's own L2
+__device__ __forceinline__ u32x4_t stream_load(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kNonTemporal));
+}
+__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, f32x4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ f32x4_t load_device(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kScopeDevice));
+}
+__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, u32x2_t v) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, r, byte, 0, kScopeDevice);
+}
+__device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int byte) {
+  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
+}
+
 }  // namespace LLMHIP_NS

@@ -205,27 +205,6 @@ __host__ __device__ constexpr int fold_parts(int splits) { return splits <= kFol
 
 __device__ __forceinline__ float bits_float(uint32_t u) { return __builtin_bit_cast(float, u); }
 
-// Buffer descriptor of `bytes` bytes: a load past them returns zero.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t byte_buffer(const void *base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
-}
-constexpr int kNonTemporal = 2, kScopeDevice = 16;  // cache policy operand: nt; sc1, past the XCD's own L2
-__device__ __forceinline__ u32x4_t stream_load(__amdgpu_buffer_rsrc_t r, int byte) {
-  return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kNonTemporal));
-}
-__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, f32x4_t v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), r, byte, 0, kScopeDevice);
-}
-__device__ __forceinline__ f32x4_t load_device(__amdgpu_buffer_rsrc_t r, int byte) {
-  return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(r, byte, 0, kScopeDevice));
-}
-__device__ __forceinline__ void store_device(__amdgpu_buffer_rsrc_t r, int byte, u32x2_t v) {
-  __builtin_amdgcn_raw_buffer_store_b64(v, r, byte, 0, kScopeDevice);
-}
-__device__ __forceinline__ u32x2_t load_device2(__amdgpu_buffer_rsrc_t r, int byte) {
-  return __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(r, byte, 0, kScopeDevice));
-}
-
 // The sum of partials, four dims of it per thread.
 struct PartialSum {
   float M = -INFINITY, L = 0.0f;
@@ -1062,7 +1041,7 @@ size_t flash_decode_workspace_bytes(int batch, int m, int group_size, int kv_hea
 }
 
 // A number that no workspace holds: of a launch, see launch_number.hpp.  (By chance 2^-64, from a random start.)
-static uint64_t launch_number() {
+uint64_t launch_number() {
   static std::atomic<uint64_t> last{[] {
     std::random_device rd;
     return ((uint64_t)rd() << 32) ^ rd() ^ (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count();
@@ -1073,7 +1052,7 @@ static uint64_t launch_number() {
   return n;
 }
 
-static bool may_be_capturing(hipStream_t stream) {
+bool may_be_capturing(hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
   (void)hipGetLastError();

@@ -19,13 +19,13 @@
 // moves lazily, so O is rarely rescaled.  Accumulation is fp32; out =
 // O / l rounded once; l sums the ROUNDED probabilities (what P.V used).
 //
-// flash_prefill_kernel<T, NW, KP, NT, SPLIT>: NW waves share the K/V tiles of 32*NW/KP query rows, KP of them every
+// flash_prefill_kernel<T, NW, KP, NT, KEYS>: NW waves share the K/V tiles of 32*NW/KP query rows, KP of them every
 // row block, each on its own 32 keys of every tile (KP = 1: on all 64).  While the chip is not full a launch
 // waits for the serial chain of the waves with the most keys -- a step of a wave takes 1600-1900 cycles
 // where its MFMAs take 512, and nothing else runs on its SIMD -- so that short prompts and chunks want many waves per
 // row (KP = 4: 512 tokens, 28 heads 11.5 -> 9.2 us; 256 tokens, 32 heads 8.7 -> 6.7), long ones the
 // cheapest step (KP = 1, 256 rows).  NT: the tile loads are non-temporal (chunks whose K/V tiles only one
-// workgroup reads).  SPLIT: the key range is cut, rows may be packed.
+// workgroup reads).  KEYS: all of them, the key range cut (rows may be packed), or the keys of the longest rows of a prompt in halves.
 // Outside the loop a workgroup costs a short launch 2-3 us: indexes come from divisions prepared by the host, Q
 // of shared rows is fetched once through LDS, and waves that shared rows trade pieces of O^T so that each
 // folds and stores its part (epilogue of a pair 3900 -> 2200 cycles).
@@ -65,6 +65,10 @@ constexpr int kMaxPrefillSplits = 128;           // key ranges per call
 constexpr int kWholeRange = 0x7fffffc0;          // keys of a range without an end
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
+// Keys of a workgroup: all that its rows see; a range of them, its partial to be folded by a launch of its own; all, but a half where
+// two workgroups have the longest rows (see fold_halves)
+enum PrefillKeys { kAllKeys, kRanges, kHalves };
+
 // What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way -- except with SPLIT, where
 // the key range (num_splits and what stands behind it) is needed for the first address and waited for.
 struct PrefillLate {
@@ -102,12 +106,20 @@ struct PrefillBrief {
     return p;
   }
 };
+struct PrefillHalves : PrefillBrief {
+  char *halves;     // of a pair of workgroups a half's O, maxima and sums, words with tags (kHalfBytes), and behind all of them a word each
+  uint64_t number;  // of the launch
+  int pairs;
+};
 struct PrefillParams : PrefillLate {
   const void *q, *k, *v;
   int m, n, offset;
   int H, Hkv, g;
   int xcd_bits, sched_shift;  // workgroups dealt to XCDs: 3 bits, and the logarithm of the XCDs per kv head; else 0
   int second, second_end;    // places of a list (of the XCD, mode 0: of the launch) that are taken in reverse
+  int cut, cut_at;           // query tiles of a head, from the last on, whose keys two workgroups share, and how many others come before them
+  char *halves;
+  uint64_t number;
   FastDiv list_heads;        // heads of an XCD's work list
   FastDiv g_div;
   // Split mode only: the rows of a tile are (token, head-in-group) pairs of ONE kv head, packed
@@ -127,24 +139,27 @@ struct PrefillEarly {
   addresses_t a;  // q, K, V, m | n << 32
   u32x4_t b;      // offset, Hkv | g << 16, flags, second | second_end << 16
   u32x2_t c;      // factors of the divisions by g and by the heads of a list
-  // flags: xcd_bits, sched_shift << 2, pack << 4, shifts of the divisions << 5 and << 10, heads of a list << 16
+  // flags: xcd_bits, sched_shift << 2, pack << 4, shifts of the divisions << 5 and << 10, heads of a list << 16; with halves the places
+  // are second | second_end << 10 | cut << 20 | cut_at << 26
   explicit PrefillEarly(const PrefillParams &p) {
     a = addresses_t{address(p.q), address(p.k), address(p.v), (uint32_t)p.m | (uint64_t)p.n << 32};
     b = u32x4_t{(uint32_t)p.offset, (uint32_t)p.Hkv | (uint32_t)p.g << 16,
                 (uint32_t)(p.xcd_bits | p.sched_shift << 2 | p.pack << 4) | p.g_div.l << 5 | p.list_heads.l << 10 | p.list_heads.d << 16,
-                (uint32_t)p.second | (uint32_t)p.second_end << 16};
+                p.cut ? (uint32_t)p.second | (uint32_t)p.second_end << 10 | (uint32_t)p.cut << 20 | (uint32_t)p.cut_at << 26
+                      : (uint32_t)p.second | (uint32_t)p.second_end << 16};
     c = u32x2_t{p.g_div.m, p.list_heads.m};
   }
 };
 struct PrefillShared {  // the same, unpacked
   const char *q, *k, *v;
-  int m, n, offset, H, Hkv, g, xcd_bits, sched_shift, second, second_end;
+  int m, n, offset, H, Hkv, g, xcd_bits, sched_shift, second, second_end, cut, cut_at;
   bool pack;
   FastDiv g_div, list_heads;
-  __device__ __forceinline__ PrefillShared(addresses_t a, u32x4_t b, u32x2_t c)
+  __device__ __forceinline__ PrefillShared(addresses_t a, u32x4_t b, u32x2_t c, bool halves)
       : q(at_address<const char>(a[0])), k(at_address<const char>(a[1])), v(at_address<const char>(a[2])), m((uint32_t)a[3]),
         n((uint32_t)(a[3] >> 32)), offset(b[0]), H((b[1] & 0xffffu) * (b[1] >> 16)), Hkv(b[1] & 0xffffu), g(b[1] >> 16),
-        xcd_bits(b[2] & 3u), sched_shift(b[2] >> 2 & 3u), second(b[3] & 0xffffu), second_end(b[3] >> 16), pack(b[2] & 16u),
+        xcd_bits(b[2] & 3u), sched_shift(b[2] >> 2 & 3u), second(b[3] & (halves ? 0x3ffu : 0xffffu)),
+        second_end(halves ? b[3] >> 10 & 0x3ffu : b[3] >> 16), cut(b[3] >> 20 & 63u), cut_at(b[3] >> 26), pack(b[2] & 16u),
         g_div{b[1] >> 16, c[0], b[2] >> 5 & 31u}, list_heads{b[2] >> 16, c[1], b[2] >> 10 & 31u} {}
 };
 
@@ -153,9 +168,10 @@ struct PrefillShared {  // the same, unpacked
 // so that its K/V stay in that XCD's L2, and within an XCD the heaviest (last)
 // query tiles are issued first.  Key ranges (split mode) are the slowest index of an XCD's
 // list, so that every XCD gets the same number of workgroups whatever the head count.
-template <bool SPLIT>
+template <PrefillKeys KEYS>
 __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const PrefillLate &p, int bid, int num_q_tiles, int &tile,
                                                  int &head, int &split) {
+  constexpr bool SPLIT = KEYS == kRanges;
   if (SPLIT && p.per_xcd) {
     // (cluster of tiles, kv head, key range, tile of the cluster): an XCD has a piece of the list
     const int i = bid >> 3, idx = (bid & 7) * p.per_xcd + i;
@@ -180,9 +196,15 @@ __device__ __forceinline__ bool prefill_schedule(const PrefillShared &e, const P
     split = (int)fast_div(idx, p.per_list);
     rem = idx - split * (int)p.per_list.d;
   }
-  const int t = (int)fast_div(rem, e.list_heads);
-  if (t >= num_q_tiles) return false;
+  int t = (int)fast_div(rem, e.list_heads);
   const int h = rem - t * (int)e.list_heads.d;
+  if (KEYS == kHalves) {  // split: all keys, the first half, the second
+    const int in = t - e.cut_at;
+    const bool half = (uint32_t)in < 2u * e.cut;
+    split = half ? 1 + (in & 1) : 0;
+    t = half ? in >> 1 : in < 0 ? t + e.cut : t - e.cut;
+  }
+  if (t >= num_q_tiles) return false;
   tile = num_q_tiles - 1 - t;
   if (SPLIT && e.pack)
     head = h * e.g;  // the list holds kv heads: first query head of the kv head
@@ -547,6 +569,60 @@ __device__ __forceinline__ void store_partial_rows(const WaveAttn<T, KB> &w, cha
   }
 }
 
+// The longest rows of a prompt, dealt to two workgroups: each has half of the keys, and the one that began first passes what it has to
+// the other, lane by lane as it lies in registers, every word beside half of the launch's number, past the XCD's L2.  No fence, no flag;
+// the other looks at what is stored last until it finds the number, then at all.  Both in the order of the halves, whoever folds.
+constexpr int kHalfBytes = 4 * 17 * 1024;  // 4 waves of 32 floats, a maximum and a sum to a lane
+template <int D0, int ND, typename T, int KB>
+__device__ __forceinline__ void pass_half(const WaveAttn<T, KB> &w, __amdgpu_buffer_rsrc_t words, int wave, uint64_t number) {
+  const uint32_t tag0 = (uint32_t)number, tag1 = (uint32_t)(number >> 32);
+  const int at = wave * 17 * 1024 + w.lane * 16;
+  auto word = [&](int i, float x, float y) {
+    store_device(words, at + i * 1024, __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, x), tag0, __builtin_bit_cast(uint32_t, y), tag1}));
+  };
+#pragma unroll
+  for (int i = 0; i < 8 * ND; ++i) word(i, w.o[D0 + i / 8][2 * (i % 8)], w.o[D0 + i / 8][2 * (i % 8) + 1]);
+  word(8 * ND, w.m_run, w.l_run);
+}
+template <int D0, int ND, typename T, int KB>
+__device__ __forceinline__ void fold_halves(WaveAttn<T, KB> &w, __amdgpu_buffer_rsrc_t words, int wave, uint64_t number, bool first, float scale_log2e) {
+  const uint32_t tag0 = (uint32_t)number, tag1 = (uint32_t)(number >> 32);
+  const int at = wave * 17 * 1024 + w.lane * 16;
+  u32x4_t v[8 * ND + 1];
+  bool there;
+  int looks = 1 << 17;  // (0.1 s: the other one is under way.  Rows of NaN where the buffer was another launch's too)
+  do {
+    do {
+      asm volatile("" ::: "memory");  // (the load is made again)
+      v[8 * ND] = __builtin_bit_cast(u32x4_t, load_device(words, at + 8 * ND * 1024));
+      there = __builtin_amdgcn_ballot_w64(((v[8 * ND][1] ^ tag0) | (v[8 * ND][3] ^ tag1)) != 0) == 0;
+      if (!there) __builtin_amdgcn_s_sleep(1);
+    } while (!there && --looks > 0);
+    asm volatile("" ::: "memory");
+    uint32_t differs = 0;
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) v[i] = __builtin_bit_cast(u32x4_t, load_device(words, at + i * 1024));
+#pragma unroll
+    for (int i = 0; i < 8 * ND; ++i) differs |= (v[i][1] ^ tag0) | (v[i][3] ^ tag1);
+    there = there && __builtin_amdgcn_ballot_w64(differs != 0) == 0;
+  } while (!there && --looks > 0);
+  if (!there) w.l_run = NAN;
+  const float m = __builtin_bit_cast(float, (uint32_t)v[8 * ND][0]), l = __builtin_bit_cast(float, (uint32_t)v[8 * ND][2]);
+  const float m_new = fmaxf(w.m_run, m), m_use = (m_new == -INFINITY) ? 0.0f : m_new;
+  const float own = fast_exp2((w.m_run - m_use) * scale_log2e), other = fast_exp2((m - m_use) * scale_log2e);
+  // (the first half's product is rounded, whichever it is)
+  auto sum = [&](float mine, float theirs) {
+    return first ? __builtin_fmaf(theirs, other, mine * own) : __builtin_fmaf(mine, own, theirs * other);
+  };
+  w.l_run = sum(w.l_run, l);
+#pragma unroll
+  for (int i = 0; i < 8 * ND; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      w.o[D0 + i / 8][2 * (i % 8) + j] = sum(w.o[D0 + i / 8][2 * (i % 8) + j], __builtin_bit_cast(float, (uint32_t)v[i][2 * j]));
+  w.m_run = m_new;
+}
+
 // One global_load_lds_dwordx4: lane l's 16 bytes at `src` land at the wave-uniform LDS address lds_addr + 16*l.
 __device__ __forceinline__ void lds_dma(const char *src, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -636,9 +712,14 @@ template <int NW, int TN, bool NT> struct DirectLoader {
 // KP = 2: two waves per row block, each on one 32-key half of every 64-key tile; KP = 4: four waves, tiles of
 // 128 keys; what they have is merged through LDS at the end.
 // ---------------------------------------------------------------------------
-template <typename T, int NW, int KP, bool NT, bool SPLIT>
+template <PrefillKeys KEYS> struct LateOf { using type = PrefillBrief; };
+template <> struct LateOf<kRanges> { using type = PrefillLate; };
+template <> struct LateOf<kHalves> { using type = PrefillHalves; };
+
+template <typename T, int NW, int KP, bool NT, PrefillKeys KEYS>
 __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec,
-                                                                                  std::conditional_t<SPLIT, PrefillLate, PrefillBrief> late) {
+                                                                                  typename LateOf<KEYS>::type late) {
+  constexpr bool SPLIT = KEYS == kRanges;
   const PrefillLate p = late;
   // SUB tiles of 64 keys per stage and per barrier: with one workgroup per CU (NW = 8) a stage
   // holds 128 keys, which halves the number of times the waves are forced in step.
@@ -651,11 +732,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   constexpr int kWaveKeys = 32 * KB;  // keys of a tile per wave
   constexpr int kSplitKK = 3;  // k-steps of S(j+1) issued beside the row-maximum chain
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const PrefillShared e(ea, eb, ec);
+  const PrefillShared e(ea, eb, ec, KEYS == kHalves);
   const bool pack = SPLIT && e.pack;  // (packed rows exist in split mode only)
   const int rows = pack ? e.m * e.g : e.m;
   int tile, head, split;
-  if (!prefill_schedule<SPLIT>(e, p, blockIdx.x, (rows + BM - 1) / BM, tile, head, split)) return;
+  if (!prefill_schedule<KEYS>(e, p, blockIdx.x, (rows + BM - 1) / BM, tile, head, split)) return;
 #ifdef LLMHIP_BENCH
   unsigned long long clk0 = 0, ref0 = 0;
   if (p.clock_probe) {
@@ -689,11 +770,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   const int n_vis = min(e.n, tile_tok_end + e.offset);  // keys any row of this tile can see
   constexpr int kTileShift = TN == 128 ? 7 : 6;
   static_assert(1 << kTileShift == TN, "");
-  const int first = SPLIT ? split * p.first_each : 0, step = SPLIT && p.range_keys == kWholeRange ? p.num_splits : 1;  // of this workgroup's tiles
+  const int half = KEYS == kHalves ? ((n_vis + TN - 1) >> kTileShift) >> 1 : 0;  // tiles of the first one
+  const int first = SPLIT ? split * p.first_each : KEYS == kHalves && split == 2 ? half : 0, step = SPLIT && p.range_keys == kWholeRange ? p.num_splits : 1;  // of this workgroup's tiles
   int first_keys = n_vis - first * TN;  // keys from its first one on, within its range
-  if (SPLIT) first_keys = min(first_keys, p.range_keys);
+  const int range_keys = SPLIT ? p.range_keys : KEYS == kHalves && split == 1 ? half * TN : kWholeRange;
+  if (KEYS != kAllKeys) first_keys = min(first_keys, range_keys);
   auto mine = [&](int keys) {  // its tiles that hold one of the first `keys` keys
-    int tiles = ((SPLIT ? min(keys - first * TN, p.range_keys) : keys) + TN - 1) >> kTileShift;
+    int tiles = ((KEYS != kAllKeys ? min(keys - first * TN, range_keys) : keys) + TN - 1) >> kTileShift;
     if (SPLIT && step > 1) tiles = tiles > 0 ? (int)fast_div(tiles + step - 1, p.splits_div) : 0;
     return tiles;
   };
@@ -714,6 +797,17 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     w.init(lds, lane, kVRegion);
     store_partial(w, part_o, part_ml, row_valid);
     return;
+  }
+  // Which of a pair begins first passes its half on: it is under way, and so the other one never waits for a workgroup that is not.
+  [[maybe_unused]] unsigned long long began = 0;
+  [[maybe_unused]] int pair = 0;
+  if constexpr (KEYS == kHalves) {
+    if (split) {
+      pair = ((rows + BM - 1) / BM - 1 - tile) * e.H + head;
+      if (tid == 0)
+        began = __hip_atomic_exchange(reinterpret_cast<unsigned long long *>(late.halves + (size_t)late.pairs * kHalfBytes) + pair,
+                                      (unsigned long long)late.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   // Q.  A fragment load straight into the operand layout touches 32 rows with 32 bytes each, 256 tag look-ups per
   // wave; Q goes through LDS like a K tile instead, fetched once as whole rows, and the first scores wait for it and K
@@ -772,7 +866,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   auto tile_step = [&](int j, int slot, f32x16_t (&s_cur)[KB], f32x16_t (&s_nxt)[KB]) {
     const int kslot = (slot + SUB + 1) % NSLOT, vslot = (slot + SUB) % NSLOT;  // fetched now
     if (j < Jw) {
-      const int key0 = (SPLIT ? j * step + first : j) * TN + kw0;
+      const int key0 = (SPLIT ? j * step + first : KEYS == kHalves ? j + first : j) * TN + kw0;
       if ((key0 + kWaveKeys - 1 > tok_lo + e.offset) || (key0 + kWaveKeys > e.n))
         w.mask(s_cur, key0, qtok, e.offset, e.n);
       // In the 8-wave kernel a burst of loads would stall every wave behind the texture addresser's
@@ -850,10 +944,23 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     constexpr int kTrade = WaveAttn<T, KB>::trade_bytes(KP), ND = 4 / KP;
     char *rows_lds = lds + rb * kTrade;
     w.template give<KP>(rows_lds, kpar);
+    volatile uint32_t *second = reinterpret_cast<volatile uint32_t *>(lds + 2 * NSLOT * TB);  // (Q's place)
+    if constexpr (KEYS == kHalves) {
+      if (split && tid == 0) *second = began == late.number;
+    }
     __syncthreads();
+    bool there = true;  // (all that the rows see)
     auto finish = [&](auto part) {
       constexpr int PART = decltype(part)::value;
       w.template take<KP, PART>(rows_lds, scale);
+      if constexpr (KEYS == kHalves) {
+        if (split) {
+          const __amdgpu_buffer_rsrc_t words = byte_buffer(late.halves + (size_t)pair * kHalfBytes, kHalfBytes);
+          if (__builtin_amdgcn_readfirstlane(*second)) fold_halves<PART * ND, ND>(w, words, wave, late.number, split == 1, scale);
+          else pass_half<PART * ND, ND>(w, words, wave, late.number), there = false;
+        }
+      }
+      if (!there) return;
       if (SPLIT && rows > kFewRows)
         store_partial_rows<PART * ND, ND>(w, lds + RB * kTrade + wave * (32 * 128 * ND), part_row, part_ml, row_valid, rows - qblk0);
       else if (SPLIT)
@@ -1023,6 +1130,7 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   const int S_ = p.num_splits, share = prefill_xcd_share_log2(p.Hkv);
   p.xcd_bits = p.sched_shift = 0;
   p.per_xcd = 0;
+  const int T_cut = T_ + p.cut;  // workgroups of a head
   if (p.pack) {
     list_heads = p.Hkv;
     grid = T_ * p.Hkv * S_;
@@ -1047,10 +1155,10 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
     p.sched_shift = share;
     list_heads = p.H >> (3 - share);
     const int xcds = 1 << share;  // per list
-    grid = 8 * ((list_heads * T_ * S_ + xcds - 1) / xcds);
+    grid = 8 * ((list_heads * T_cut * S_ + xcds - 1) / xcds);
   } else {
     list_heads = p.H;
-    grid = T_ * p.H * S_;
+    grid = T_cut * p.H * S_;
   }
   // Two workgroups to a CU: the second one that a CU gets runs beside its first one, the heaviest ones' too, so that those
   // places are dealt from the lightest on (us: 700 tokens of 40 heads 13.0 -> 12.5, 1019 of 28 16.7 -> 16.1, of 32 18.6 -> 18.0,
@@ -1081,24 +1189,33 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   const size_t lds_bytes = tile_bytes + (KP > 1 ? q_bytes : q_bytes - tile_bytes / 4);  // (half of the V slots are Q's at first)
   // packed rows, one tile per kv head: every K/V tile is read by one workgroup only (KP == 1 there)
   const bool nt = KP == 1 && p.pack && T_ == 1, cut = S_ > 1;
-  const auto whole = flash_prefill_kernel<T, NW, KP, false, false>;
-  const auto ranges = nt ? flash_prefill_kernel<T, NW, KP, (KP == 1), true> : flash_prefill_kernel<T, NW, KP, false, true>;
+  const auto whole = flash_prefill_kernel<T, NW, KP, false, kAllKeys>;
+  const auto ranges = nt ? flash_prefill_kernel<T, NW, KP, (KP == 1), kRanges> : flash_prefill_kernel<T, NW, KP, false, kRanges>;
+  const void *kern = cut ? reinterpret_cast<const void *>(ranges) : reinterpret_cast<const void *>(whole);
+  [[maybe_unused]] const auto halves = flash_prefill_kernel<T, 4, 2, false, kHalves>;
+  if (p.cut) kern = reinterpret_cast<const void *>(halves);
   // the opt-in for more than 64 KiB of dynamic LDS is per device: once per device and kernel
-  static std::atomic<uint64_t> attr_done_all[3];
-  std::atomic<uint64_t> &attr_done = attr_done_all[nt ? 2 : cut ? 1 : 0];
+  static std::atomic<uint64_t> attr_done_all[4];
+  std::atomic<uint64_t> &attr_done = attr_done_all[p.cut ? 3 : nt ? 2 : cut ? 1 : 0];
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   const uint64_t bit = 1ull << (dev & 63);
   if (!(attr_done.load(std::memory_order_acquire) & bit)) {
-    e = hipFuncSetAttribute(cut ? reinterpret_cast<const void *>(ranges) : reinterpret_cast<const void *>(whole),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (e != hipSuccess) return e;
     attr_done.fetch_or(bit, std::memory_order_release);
   }
   const PrefillEarly early(p);
   if (cut) {
     hipLaunchKernelGGL(ranges, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
+  } else if (p.cut) {
+    PrefillHalves late = {};
+    late.out = p.out;
+    late.halves = p.halves;
+    late.number = p.number;
+    late.pairs = p.cut * p.H;
+    hipLaunchKernelGGL(halves, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, late);
   } else {
     PrefillBrief brief;
     brief.out = p.out;
@@ -1160,6 +1277,7 @@ struct PrefillPlan {
   PrefillKind kind;
   bool pack;
   int num_splits, chunk;
+  int cut = 0, cut_at = 0;  // see prompt_cut
 };
 
 // The most scratch a plan may ask for.  Without a bound it grows with the chunk (behind 131072 keys 7151 tokens of 28
@@ -1192,6 +1310,29 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
   if (per_cu(128) <= 1.3) return kPair64;
   if (per_cu(128) <= 2.0) return kPair128;
   return per_cu(256) > 1.5 ? kRows256 : kRows128;
+}
+
+// Where two waves share 64 rows and not every CU has two workgroups, the launch waits for those with the most keys, while others have long
+// ended: the longest rows are dealt to two workgroups each (see fold_halves), as many as leave places for all workgroups at once, and as many
+// as leave those that are not cut longer than a half and what it is passed on in, which takes as long as 6 steps.  Cut ones come behind those that
+// are longer than a half and 4 steps (by 2 to 6 the same; before all others 1.05 to 1.15 times as long: the longest rows then begin later and
+// beside longer ones).  Attention, us, whole / so: 1019 tokens of 28 + 4 heads (of 16 steps 14) 14.9 / 14.1, 930 13.2 / 12.75, 1088 15.9 / 15.4, 930 of 32
+// + 32 15.2 / 13.8, 1480 of 12 + 2 17.2 / 15.0; with 3 steps for passing a half on 700 of 28 + 4 10.35 / 11.1.
+static void prompt_cut(int m, long long n_vis, int g, int Hkv, int cus, int &cut, int &cut_at) {
+  constexpr int kPassSteps = 6, kOrderSteps = 4;
+  const int share = prefill_xcd_share_log2(Hkv), H = g * Hkv;
+  const long long tiles = (m + 63) / 64, longest = (n_vis + kTileN - 1) / kTileN;
+  // (a list has the heads of 2^share XCDs)
+  const long long places = (share >= 0 ? (2LL * cus / 8 << share) / (H >> (3 - share)) : 2LL * cus / H) - tiles;
+  long long most = longest / 2 - kPassSteps;
+  if (places < most) most = places;
+  if (tiles < most) most = tiles;
+  cut = cut_at = 0;
+  if (most < 1 || 2 * cus > 1023) return;  // (places are told in 10 bits)
+  cut = (int)(most < 63 ? most : 63);
+  const long long before = longest - cut - ((longest + 1) / 2 + kOrderSteps) + 1;
+  cut_at = before < 0 ? 0 : (int)(before < tiles - cut ? before : tiles - cut);
+  if (cut_at > 63) cut_at = 63;
 }
 
 // A chunk behind a longer cache makes few workgroups with many keys each: its key range is cut, and with fewer rows than a
@@ -1260,7 +1401,11 @@ static PrefillPlan chunk_plan(int m, long long n_vis, long long past, int g, int
 // The last answers are kept per thread: every layer of a model asks for the same chunk (several hundred combinations).
 static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cus, size_t max_bytes) {
   const long long n_vis = ((long long)m + offset < n) ? (long long)m + offset : n;  // keys the last row sees
-  if (prefill_is_prompt(m, n_vis)) return {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
+  if (prefill_is_prompt(m, n_vis)) {
+    PrefillPlan pl = {prompt_kind(m, n_vis, g * Hkv, cus), false, 1, kWholeRange};
+    if (pl.kind == kPair64) prompt_cut(m, n_vis, g, Hkv, cus, pl.cut, pl.cut_at);
+    return pl;
+  }
   struct Memo {
     int m, n, offset, g, Hkv, cus;
     size_t bytes, max_bytes;  // what the plan takes, what it was allowed
@@ -1281,6 +1426,12 @@ static PrefillPlan plan_prefill(int m, int n, int offset, int g, int Hkv, int cu
 size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num) {
   const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), kMaxPrefillScratch);
   return partial_bytes(pl.num_splits, m, (long long)group_size * kv_head_num);
+}
+
+static size_t halves_bytes(long long pairs) { return pairs * (kHalfBytes + sizeof(uint64_t)); }
+size_t flash_prefill_halves_bytes(int m, int n, int offset, int group_size, int kv_head_num) {
+  const PrefillPlan pl = plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), 0);
+  return halves_bytes((long long)pl.cut * group_size * kv_head_num);
 }
 
 // Where a call may not do with less: a chunk behind at least 2048 keys and 8 times its own length whose unsplit form would
@@ -1342,6 +1493,13 @@ hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const v
   if (workspace_bytes > kMaxPrefillScratch) workspace_bytes = kMaxPrefillScratch;
   const PrefillPlan pl =
       plan_prefill(m, n, offset, group_size, kv_head_num, device_compute_units(), workspace ? workspace_bytes : 0);
+  p.cut = p.cut_at = 0;
+  if (pl.cut && workspace && halves_bytes((long long)pl.cut * p.H) <= workspace_bytes && !may_be_capturing(stream)) {
+    p.cut = pl.cut;
+    p.cut_at = pl.cut_at;
+    p.halves = static_cast<char *>(workspace);
+    p.number = launch_number();
+  }
   p.pack = pl.pack ? 1 : 0;
   p.num_splits = pl.num_splits;
   p.chunk = pl.chunk;

@@ -14,6 +14,9 @@ namespace LLMHIP_NS {
 // flash_prefill_least_workspace_bytes: below this a call with no way to get more is to be refused.
 size_t flash_prefill_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num);
 size_t flash_prefill_least_workspace_bytes(int m, int n, int offset, int group_size, int kv_head_num);
+// What a prompt whose longest rows two workgroups share takes for the halves that are passed on (0: none do).  Without it they are not
+// shared; nor are they on a stream that may be capturing.
+size_t flash_prefill_halves_bytes(int m, int n, int offset, int group_size, int kv_head_num);
 #ifdef LLMHIP_BENCH
 // The measurement library's copy, never split: clock_probe is a device pointer to two 64-bit counters that
 // workgroup 0 fills with the shader-clock ticks and the reference-clock ticks of its lifetime.
@@ -34,6 +37,11 @@ inline int prefill_xcd_share_log2(int kv_head_num) {
   if (kv_head_num % 8 == 0) return 0;
   return kv_head_num == 4 ? 1 : kv_head_num == 2 ? 2 : kv_head_num == 1 ? 3 : -1;
 }
+
+// A number that no workspace holds: of a launch, see launch_number.hpp.  (A replayed graph launches with the number of its
+// capture, and words of the replay before would pass for new ones: not for a stream that may be capturing.)
+uint64_t launch_number();
+bool may_be_capturing(hipStream_t stream);
 
 // Compute units of the current device, cached per device; 256 when no device can be asked.
 int device_compute_units();

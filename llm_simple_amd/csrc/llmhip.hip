@@ -127,9 +127,20 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
   // a chunk of few rows over a long cache is split over the key range: fp32 partials in the
   // per-stream scratch
   const size_t need = flash_prefill_workspace_bytes(m, n, offset, group_size, kv_head_num);
-  if (!need)
+  if (!need) {
+    // a prompt: its longest rows shared by two workgroups, if the scratch is there or can be had.  Not on hipStreamPerThread,
+    // where calls of several threads have one buffer and no order.
+    const size_t halves = flash_prefill_halves_bytes(m, n, offset, group_size, kv_head_num);
+    if (halves && as_stream(stream) != hipStreamPerThread && !may_be_capturing(as_stream(stream))) {
+      std::lock_guard<std::mutex> lk(g_scratch_mu);
+      StreamScratch *ws = nullptr;
+      (void)scratch_for_locked(stream, halves, [] { return (size_t)0; }, &ws);
+      if (ws->bytes >= halves)
+        return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt, as_stream(stream), ws->ptr, ws->bytes));
+    }
     return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
                                          as_stream(stream), nullptr, 0));
+  }
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   StreamScratch *ws = nullptr;
   int rc = scratch_for_locked(
