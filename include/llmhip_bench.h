@@ -38,6 +38,12 @@ int llmhip_bench_decode_step_gqa_alone(void *out, void *k_cache, void *v_cache, 
                                        int group_size, int kv_head_num, int head_dim, int is_neox_style, int num_splits, int dt,
                                        void *stream);
 
+/* llmhip_matmul_bias (bias_f32 null: llmhip_matmul) of a size that is computed in pieces of k, by a copy of that kernel whose adding workgroups
+ * do not wait for the other pieces' sums but make all of them by themselves, as they do after waiting in vain: the same bits.  LLMHIP_ERR_UNSUPPORTED for
+ * other sizes; workspace: 2 MiB are enough for any. */
+int llmhip_bench_matmul_alone(void *out, const void *lhs, const void *weight, const void *bias_f32, void *workspace, size_t workspace_bytes,
+                              int m, int n, int k, int dt, void *stream);
+
 /* Runs, for about target_ms (<= 2000), a loop of back-to-back bf16 32x32x16 MFMAs on N(0,1)
  * operands on every CU and returns the sustained TFLOP/s.  mix 0: the MFMAs alone (what the matrix
  * pipe sustains at the clock its own power draw allows); mix 1: the same MFMAs with the LDS

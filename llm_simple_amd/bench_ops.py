@@ -14,6 +14,7 @@ SYMBOLS = {
     "llmhip_bench_flash_attn_gqa_clocked": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp]),
     "llmhip_bench_flash_decode_gqa_alone": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, ctypes.c_int64, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_decode_step_gqa_alone": (_i, [_vp] * 8 + [_sz, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "llmhip_bench_matmul_alone": (_i, [_vp] * 5 + [_sz, _i, _i, _i, _i, _vp]),
     "llmhip_bench_mfma_ceiling": (_i, [_i, ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
     "llmhip_bench_stream_read": (_i, [_vp, _vp, _sz, _vp, _sz, _i, _vp]),
 }
@@ -66,6 +67,14 @@ def hip_decode_step_gqa_alone_layer(output_dev, k_dev, v_dev, freq_cis_dev, q_de
     _check(lib.llmhip_bench_decode_step_gqa_alone(p(output_dev), p(k_dev), p(v_dev), p(freq_cis_dev), p(q_dev), p(new_k_dev),
                                                   p(new_v_dev), p(ws_dev), ws_bytes, pos, group_size, kv_head_num, head_dim,
                                                   is_neox_style, num_splits, dt, stream), "hip_decode_step_gqa_alone_layer")
+
+
+def hip_matmul_alone_layer(output_dev, lhs_dev, weight_dev, bias_dev, ws_dev, ws_bytes, m, n, k, dt, stream=0):
+    """hip_matmul_bias_layer (bias_dev None: hip_matmul_layer) of a size computed in pieces of k, on the measurement library's copy, whose
+    adding workgroups make all sums by themselves."""
+    p = ops._ptr
+    _check(lib.llmhip_bench_matmul_alone(p(output_dev), p(lhs_dev), p(weight_dev), None if bias_dev is None else p(bias_dev), p(ws_dev),
+                                         ws_bytes, m, n, k, dt, stream), "hip_matmul_alone_layer")
 
 
 def probe_mfma_ceiling(mix, target_ms=60.0):

@@ -72,6 +72,20 @@ int llmhip_bench_decode_step_gqa_alone(void *out, void *k_cache, void *v_cache, 
                                            static_cast<hipStream_t>(stream)));
 }
 
+int llmhip_bench_matmul_alone(void *out, const void *lhs, const void *weight, const void *bias_f32, void *workspace, size_t workspace_bytes,
+                              int m, int n, int k, int dt, void *stream) {
+  if (!out || !lhs || !weight || !workspace || !aligned16(out) || !aligned16(lhs) || !aligned16(weight) || !aligned16(workspace))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (m < 1 || n < 1 || k < 1 || (dt != LLMHIP_DT_FLOAT16 && dt != LLMHIP_DT_BFLOAT16)) return LLMHIP_ERR_INVALID_ARG;
+  if (n % 16 != 0 || k % 16 != 0) return LLMHIP_ERR_UNSUPPORTED;
+  const int pieces = matmul_tile_pieces(m, n, k);
+  if (pieces < 2) return LLMHIP_ERR_UNSUPPORTED;
+  if (matmul_pieces_bytes(m, n, pieces) > workspace_bytes) return LLMHIP_ERR_WORKSPACE;
+  if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
+  return from_hip(launch_matmul_tile(out, lhs, weight, static_cast<const float *>(bias_f32), m, n, k, dt, static_cast<hipStream_t>(stream),
+                                     pieces, workspace));
+}
+
 int llmhip_bench_mfma_ceiling(int mix, double target_ms, double *tflops) {
   if (!tflops || (mix != 0 && mix != 1) || target_ms < 0.0 || target_ms > 2000.0) return LLMHIP_ERR_INVALID_ARG;
   if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;

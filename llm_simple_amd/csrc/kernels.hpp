@@ -95,13 +95,16 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
 
 // Projection out[m][n] = round(lhs[m][k] . weight[n][k]^T + bias), bias fp32 [n] or null; n and k multiples
 // of 16.  matmul_skinny: m <= 16, pointers 16-byte aligned.  matmul_tile: the sizes that matmul_tile_takes
-// accepts, pointers 16-byte aligned.  matmul_bias: hipBLASLt, whose handle and 64 MiB
+// accepts, pointers 16-byte aligned; with more than one of matmul_tile_pieces' pieces of k a workspace of matmul_pieces_bytes, and not on a
+// stream that may be capturing.  matmul_bias: hipBLASLt, whose handle and 64 MiB
 // workspace the first call creates.
 hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, const float *bias,
                                 int m, int n, int k, int dt, hipStream_t stream);
 bool matmul_tile_takes(int m, int n, int k);
+int matmul_tile_pieces(int m, int n, int k);
+size_t matmul_pieces_bytes(int m, int n, int pieces);
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias,
-                              int m, int n, int k, int dt, hipStream_t stream);
+                              int m, int n, int k, int dt, hipStream_t stream, int pieces = 1, void *workspace = nullptr);
 hipError_t launch_matmul_bias(void *out, const void *lhs, const void *weight, const float *bias,
                               int m, int n, int k, int dt, hipStream_t stream);
 void release_matmul_resources();

@@ -481,6 +481,15 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
   // base.
   if (all_aligned16(out, lhs, weight)) {
     const float *b = static_cast<const float *>(bias);
+    // Few tiles over a long k in pieces, if the scratch is there or can be had (not on hipStreamPerThread, see attn_common)
+    const int pieces = matmul_tile_pieces(m, n, k);
+    if (pieces > 1 && as_stream(stream) != hipStreamPerThread && !may_be_capturing(as_stream(stream))) {
+      const size_t need = matmul_pieces_bytes(m, n, pieces);
+      std::lock_guard<std::mutex> lk(g_scratch_mu);
+      StreamScratch *ws = nullptr;
+      (void)scratch_for_locked(stream, need, [] { return (size_t)0; }, &ws);
+      if (ws->bytes >= need) return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream), pieces, ws->ptr));
+    }
     const bool tiles = m > 8 && matmul_tile_takes(m, n, k);
     const long long per_cu = (n + device_compute_units() - 1) / device_compute_units();
     if (m <= 16 && !(tiles && (per_cu > 16 || m * per_cu > (k > 7168 ? 130 : 190))))

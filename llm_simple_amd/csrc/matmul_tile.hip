@@ -52,7 +52,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 
-namespace llmhip {
+namespace LLMHIP_NS {
 
 namespace {
 
@@ -61,6 +61,13 @@ constexpr int kLineK = 64;             // k of a 128-byte line of an operand row
 constexpr int kStageRow = 2 * kLineK;  // its bytes
 constexpr int kBiasBytes = 4 * 512;    // LDS: bias of each wave's features
 constexpr int kBandRows = 4;           // m tiles of a band
+constexpr int kMostPieces = 8;         // of k
+constexpr int kWordsBytes = 2 * 16 * kTileThreads;  // of a piece's sums
+#ifdef LLMHIP_BENCH
+constexpr uint32_t kLooks = 0;  // (the measurement library's copy: a workgroup that adds up makes all sums by itself)
+#else
+constexpr uint32_t kLooks = 2000;      // 0.7 us each or more: what a launch takes, many times over
+#endif
 
 // LDS offset of logical 16-byte granule g of a staged row
 __device__ __forceinline__ int stage_off(int row, int g) { return row * kStageRow + ((g ^ ((row >> 1) & 7)) << 4); }
@@ -76,13 +83,23 @@ template <int OFF> __device__ __forceinline__ void line_load(uint32_t voff, cons
   else asm volatile("global_load_lds_dwordx4 %0, %1 offset:%2" : : "v"(voff), "s"(base), "n"(OFF));
 }
 
-template <typename T, int MT, int NT, int KS, int STAGES>
-__global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_t a_, u32x4_t size, u32x2_t divisors) {
+// What the workgroups of a tile whose k is cut pass on (PIECES): fetched from memory while the first lines are under way.
+struct TilePieces {
+  char *words;   // [tile][piece][half of a lane's four][thread], 16 bytes each: two sums, beside either half of the launch's number
+  uint64_t number;
+  uint32_t looks;
+};
+struct NoPieces {};
+
+template <typename T, int MT, int NT, int KS, int STAGES, bool PIECES>
+__global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_t a_, u32x4_t size, u32x2_t divisors,
+                                                                      std::conditional_t<PIECES, TilePieces, NoPieces> late) {
   using E = Elem<T>;
+  static_assert(!PIECES || MT * NT == 1);
   const char *x = at_address<const char>(a_[0]), *w = at_address<const char>(a_[1]);
   const float *bias = at_address<const float>(a_[2]);
   uint16_t *out = at_address<uint16_t>(a_[3]);
-  const int m = size[0], n = size[1], k = size[2];
+  const int m = size[0], n = size[1], k = size[2] & 0x1fffffu, pieces = PIECES ? (int)(size[2] >> 21) : 1;
   constexpr int BM = 32 * MT, BN = 32 * NT;
   constexpr int kLineBytes = (BM + BN) * kStageRow, kStageBytes = KS * kLineBytes;
   constexpr int L = MT + NT;
@@ -92,11 +109,16 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
 
   // Workgroups are dealt round-robin to the 8 XCDs: each takes a run of tiles, and runs go through bands of up to four
   // m tiles, so that the tiles of an XCD share rows of both operands in its L2.
-  // (divisors and size[3]: factors and shifts of the divisions by the tiles of a band and by the m tiles of a full band)
+  // (divisors and size[3]: factors and shifts of the divisions by the tiles of a band and by the m tiles of a full band; with pieces, from bit 10
+  // on, 2^16 over the tiles, rounded up)
   const int m_tiles = (m + BM - 1) / BM, n_tiles = (n + BN - 1) / BN, gm = min(m_tiles, kBandRows);
-  const FastDiv by_band = {(uint32_t)(gm * n_tiles), divisors[0], size[3] & 0xffffu}, by_rows = {(uint32_t)gm, divisors[1], size[3] >> 16};
-  const int total = m_tiles * n_tiles, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
-  const int t = xcd * each + min(xcd, rest) + (int)(blockIdx.x >> 3);
+  const FastDiv by_band = {(uint32_t)(gm * n_tiles), divisors[0], size[3] & 31u}, by_rows = {(uint32_t)gm, divisors[1], size[3] >> 5 & 31u};
+  const int tiles = m_tiles * n_tiles, total = tiles * pieces, xcd = blockIdx.x & 7, each = total >> 3, rest = total & 7;
+  int t = xcd * each + min(xcd, rest) + (int)(blockIdx.x >> 3), piece = 0;
+  if (PIECES) {  // the slow index: an XCD reads one or two of them, and those of the last piece, which wait, come behind the others of their XCD
+    piece = (int)((uint32_t)t * (size[3] >> 10) >> 16);
+    t -= piece * tiles;
+  }
   const int band = (int)fast_div(t, by_band), rem = t - band * gm * n_tiles;
   const int rows_here = min(gm, m_tiles - band * gm);
   const int tn = rows_here == gm ? (int)fast_div(rem, by_rows) : rem / rows_here;
@@ -141,25 +163,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
       asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0" : : "s"(slot + (is_w ? wdst : xdst)), "n"(nth * 1024) : "m0", "scc");
     line_load<1024 * (nth % 4)>(voff[s], is_w ? wk : xk);
   };
-  const int lines = k / kLineK, stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
-  // The order of the lines: each XCD begins at another eighth, and in every group of 8 (4, 2: what divides k) each tile of those that share
-  // W rows at another place.  Not where a quarter of the last one is padding: begun ahead of the others it stays there, and fetches for them.
-  const bool padded = m_tiles <= kBandRows && 4 * (m - (m_tiles - 1) * BM) <= 3 * BM;
-  uint32_t pos = (((uint32_t)(xcd * lines) >> 3) + ((padded ? t : tn) & 3)) * kStageRow;
-  if (pos >= row_bytes) pos = 0;
-  const int group = lines % 8 == 0 ? 8 : lines % 4 == 0 ? 4 : lines % 2 == 0 ? 2 : 1;
-  const uint32_t turn = padded ? 0u : (uint32_t)(in_band * group >> (rows_here == 2 ? 1 : 2)) * kStageRow;
-  uint32_t kpos = pos ^ turn;
-  auto advance = [&]() {
-    pos = pos + kStageRow == row_bytes ? 0 : pos + kStageRow;
-    kpos = pos ^ turn;
-  };
-#pragma unroll
-  for (int s = 0; s < STAGES * KS; ++s) {
-    static_for<0, L>([&](auto l) { issue(l, wbase + kpos, xbase + kpos, s * kLineBytes); });
-    advance();
-  }
-
+  const int all_lines = k / kLineK;
   int w_addr[2], x_addr[2];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -167,12 +171,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
     x_addr[h] = stage_off(BN + wm * (BM / 2) + i, 4 * h + cg);
   }
   f32x4_t acc[MT][NT];
-#pragma unroll
-  for (int a = 0; a < MT; ++a)
-#pragma unroll
-    for (int b = 0; b < NT; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  uint32_t slot = 0;
   u32x4_t wf[2][NT], xf[2][MT];
   constexpr int NR = MT + NT, NM = MT * NT;
   auto read = [&](auto r_, int h, uint32_t at) {  // in the order of use
@@ -181,53 +179,147 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
     else if constexpr (r <= MT) xf[h][r - 1] = lds_read_b128(lds, x_addr[h] + at + (r - 1) * 16 * kStageRow);
     else wf[h][r - MT] = lds_read_b128(lds, w_addr[h] + at + (r - MT) * 16 * kStageRow);
   };
-  // Fragments of 32 k (half a line) are read while the MFMAs of the 32 before run.
-  wait_loads<L * KS * (STAGES - 1)>();
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  static_for<0, NR>([&](auto r) { read(r, 0, 0); });
   constexpr int R1 = NR + 4 > NM ? 2 : 1;               // fragment reads of a slot
   constexpr int READ = (NR + R1 - 1) / R1 + 5;          // by this slot the reads of a phase have come back
   constexpr int PH = 2 * KS, BS = (PH - 2) * NM + (READ < NM ? READ : NM), DS = PH * NM - BS, NL = KS * L;
-  // One stage.  LEFT: stages under way beyond the next one; LOAD: fetch another; NEXT: there is a next one.
-  auto stage = [&](auto left, auto load, auto next_) {
-    constexpr int LEFT = decltype(left)::value;
-    constexpr bool LOAD = decltype(load)::value, NEXT = decltype(next_)::value;
-    const uint32_t fetch = slot, next = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
-    static_for<0, PH * NM>([&](auto j_) {
-      constexpr int j = decltype(j_)::value, h = j / NM, q = j % NM;
-      if (KS > 1 && !NEXT && h >= 2 && h / 2 >= last_lines) return;  // (the last stage may hold surplus lines)
-      if constexpr (j == BS && NEXT) {
-        wait_loads<L * KS * LEFT>();
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      }
-      static_for<0, R1>([&](auto r_) {
-        constexpr int r = q * R1 + decltype(r_)::value;
-        if constexpr (r < NR && (h < PH - 1 || NEXT))
-          read(std::integral_constant<int, r>(), (h + 1) & 1, h == PH - 1 ? next : slot + (h + 1) / 2 * kLineBytes);
-      });
-      if constexpr (LOAD && j >= BS) {  // load l in slot BS + l * DS / NL
-        constexpr int first = ((j - BS) * NL + DS - 1) / DS, end = ((j + 1 - BS) * NL + DS - 1) / DS;
-        static_for<first, end>([&](auto l_) {
-          constexpr int l = decltype(l_)::value;
-          issue(std::integral_constant<int, l % L>(), wbase + kpos, xbase + kpos, fetch + l / L * kLineBytes);
-          if (l % L == L - 1) advance();
-        });
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      acc[q % MT][q / MT] = E::mfma16(wf[h & 1][q / MT], xf[h & 1][q % MT], acc[q % MT][q / MT]);
-      __builtin_amdgcn_sched_barrier(0);
-    });
-    slot = next;
-  };
   using True = std::true_type;
   using False = std::false_type;
-  for (int s = STAGES; s < stages; ++s) stage(std::integral_constant<int, STAGES - 2>(), True(), True());
-  static_for<0, STAGES>([&](auto u_) {
-    constexpr int u = decltype(u_)::value, left = STAGES - 2 - u;
-    if (stages - STAGES + u < 0) return;  // k of fewer stages than are kept
-    stage(std::integral_constant<int, (left > 0 ? left : 0)>(), False(), std::integral_constant<bool, (u < STAGES - 1)>());
-  });
-  wait_loads<0>();  // (k of one stage: the surplus ones are still under way, and LDS is given up at the end)
+  [[maybe_unused]] bool alone = false;
+  for (;;) {  // (once, unless a workgroup that has waited in vain for the sums of others makes them itself)
+    // The order of the lines: each XCD begins at another eighth, and in every group of 8 (4, 2: what divides k) each tile of those that share
+    // W rows at another place.  Not where a quarter of the last one is padding: begun ahead of the others it stays there, and fetches for them.
+    // Of a piece each tile begins elsewhere.
+    int lines = all_lines;
+    uint32_t from = 0, end = row_bytes, pos, turn = 0;
+    if constexpr (PIECES) {
+      const int first = piece * all_lines / pieces;
+      lines = (piece + 1) * all_lines / pieces - first;
+      from = (uint32_t)first * kStageRow;
+      end = from + (uint32_t)lines * kStageRow;
+      pos = from + ((uint32_t)t * (size[3] >> 10) * (uint32_t)lines >> 16) * kStageRow;
+    } else {
+      const bool padded = m_tiles <= kBandRows && 4 * (m - (m_tiles - 1) * BM) <= 3 * BM;
+      pos = (((uint32_t)(xcd * lines) >> 3) + ((padded ? t : tn) & 3)) * kStageRow;
+      if (pos >= row_bytes) pos = 0;
+      const int group = lines % 8 == 0 ? 8 : lines % 4 == 0 ? 4 : lines % 2 == 0 ? 2 : 1;
+      turn = padded ? 0u : (uint32_t)(in_band * group >> (rows_here == 2 ? 1 : 2)) * kStageRow;
+    }
+    const int stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
+    uint32_t kpos = pos ^ turn;
+    auto advance = [&]() {
+      pos = pos + kStageRow == end ? from : pos + kStageRow;
+      kpos = pos ^ turn;
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES * KS; ++s) {
+      static_for<0, L>([&](auto l) { issue(l, wbase + kpos, xbase + kpos, s * kLineBytes); });
+      advance();
+    }
+
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+      for (int b = 0; b < NT; ++b) acc[a][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+    uint32_t slot = 0;
+    // Fragments of 32 k (half a line) are read while the MFMAs of the 32 before run.
+    wait_loads<L * KS * (STAGES - 1)>();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    static_for<0, NR>([&](auto r) { read(r, 0, 0); });
+    // One stage.  LEFT: stages under way beyond the next one; LOAD: fetch another; NEXT: there is a next one.
+    auto stage = [&](auto left, auto load, auto next_) {
+      constexpr int LEFT = decltype(left)::value;
+      constexpr bool LOAD = decltype(load)::value, NEXT = decltype(next_)::value;
+      const uint32_t fetch = slot, next = slot + kStageBytes == STAGES * kStageBytes ? 0 : slot + kStageBytes;
+      static_for<0, PH * NM>([&](auto j_) {
+        constexpr int j = decltype(j_)::value, h = j / NM, q = j % NM;
+        if (KS > 1 && !NEXT && h >= 2 && h / 2 >= last_lines) return;  // (the last stage may hold surplus lines)
+        if constexpr (j == BS && NEXT) {
+          wait_loads<L * KS * LEFT>();
+          asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        static_for<0, R1>([&](auto r_) {
+          constexpr int r = q * R1 + decltype(r_)::value;
+          if constexpr (r < NR && (h < PH - 1 || NEXT))
+            read(std::integral_constant<int, r>(), (h + 1) & 1, h == PH - 1 ? next : slot + (h + 1) / 2 * kLineBytes);
+        });
+        if constexpr (LOAD && j >= BS) {  // load l in slot BS + l * DS / NL
+          constexpr int first = ((j - BS) * NL + DS - 1) / DS, end = ((j + 1 - BS) * NL + DS - 1) / DS;
+          static_for<first, end>([&](auto l_) {
+            constexpr int l = decltype(l_)::value;
+            issue(std::integral_constant<int, l % L>(), wbase + kpos, xbase + kpos, fetch + l / L * kLineBytes);
+            if (l % L == L - 1) advance();
+          });
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        acc[q % MT][q / MT] = E::mfma16(wf[h & 1][q / MT], xf[h & 1][q % MT], acc[q % MT][q / MT]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      slot = next;
+    };
+    for (int s = STAGES; s < stages; ++s) stage(std::integral_constant<int, STAGES - 2>(), True(), True());
+    static_for<0, STAGES>([&](auto u_) {
+      constexpr int u = decltype(u_)::value, left = STAGES - 2 - u;
+      if (stages - STAGES + u < 0) return;  // k of fewer stages than are kept
+      stage(std::integral_constant<int, (left > 0 ? left : 0)>(), False(), std::integral_constant<bool, (u < STAGES - 1)>());
+    });
+    wait_loads<0>();  // (k of one stage: the surplus ones are still under way, and LDS is given up at the end)
+    if constexpr (!PIECES) {
+      break;
+    } else {
+      // The last piece's workgroup adds up: its own sums, then those of pieces 0, 1, ...  Every word of theirs goes past the XCD's L2 beside half
+      // of the launch's number, and is looked at until the number is there.  They wait for nothing, and come before it in the order of
+      // their XCD; launches of two streams can hold each other's workgroups up all the same, and so a look in vain has an end.
+      f32x4_t &own = acc[0][0];
+      const __amdgpu_buffer_rsrc_t words = byte_buffer(late.words + (size_t)t * pieces * kWordsBytes, (uint32_t)pieces * kWordsBytes);
+      const uint32_t tag0 = (uint32_t)late.number, tag1 = (uint32_t)(late.number >> 32);
+      if (!alone) {
+        if (piece < pieces - 1) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            store_device(words, piece * kWordsBytes + h * (kWordsBytes / 2) + tid * 16,
+                         __builtin_bit_cast(f32x4_t, u32x4_t{__builtin_bit_cast(uint32_t, (float)own[2 * h]), tag0,
+                                                             __builtin_bit_cast(uint32_t, (float)own[2 * h + 1]), tag1}));
+          return;
+        }
+        u32x4_t v[kMostPieces - 1][2];
+        bool there;
+        int looks = (int)late.looks;
+        do {
+          asm volatile("" ::: "memory");  // (the loads are made again)
+          uint32_t differs = 0;
+#pragma unroll
+          for (int o = 0; o < kMostPieces - 1; ++o)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)  // (past the others: past the buffer, and zero)
+              v[o][h] = __builtin_bit_cast(u32x4_t, load_device(words, o < pieces - 1 ? o * kWordsBytes + h * (kWordsBytes / 2) + tid * 16 : 0x7fffff00));
+#pragma unroll
+          for (int o = 0; o < kMostPieces - 1; ++o)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) differs |= o < pieces - 1 ? (v[o][h][1] ^ tag0) | (v[o][h][3] ^ tag1) : 0u;
+          there = __builtin_amdgcn_ballot_w64(differs != 0) == 0;
+        } while (!there && --looks > 0);
+#pragma unroll
+        for (int o = 0; o < kMostPieces - 1; ++o)
+          if (o < pieces - 1)
+            own += f32x4_t{__builtin_bit_cast(float, (uint32_t)v[o][0][0]), __builtin_bit_cast(float, (uint32_t)v[o][0][2]),
+                           __builtin_bit_cast(float, (uint32_t)v[o][1][0]), __builtin_bit_cast(float, (uint32_t)v[o][1][2])};
+        volatile uint32_t *gave_up = reinterpret_cast<volatile uint32_t *>(lds + STAGES * kStageBytes + kBiasBytes);
+        if (lane == 0) gave_up[wave] = !there;
+        __syncthreads();
+        if (__builtin_amdgcn_readfirstlane(gave_up[0] | gave_up[1] | gave_up[2] | gave_up[3]) == 0) break;
+        alone = true;  // all pieces in the same order, the sum so far in the last one's place among the words
+      } else {
+        const int place = (pieces - 1) * kWordsBytes + tid * 16;
+        if (piece != pieces - 1) own = load_device(words, place) + own;
+        if (piece == pieces - 2) break;
+        store_device(words, place, own);
+        piece = piece == pieces - 1 ? 0 : piece + 1;
+      }
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();  // (nobody reads the lines of the piece before any more)
+    }
+  }
   const int row0 = m0 + wm * (BM / 2);
 #pragma unroll
   for (int b = 0; b < NT; b += 2) {
@@ -257,15 +349,19 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
 struct TileCall {
   addresses_t a;  // lhs, W, bias, out
   int m, n, k;
+  int pieces = 1;
+  TilePieces late = {};
 };
 
-template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile(const TileCall &c, hipStream_t stream) {
+template <typename T, int MT, int NT, int KS, int STAGES, bool PIECES = false> hipError_t launch_tile(const TileCall &c, hipStream_t stream) {
   const int m_tiles = (c.m + 32 * MT - 1) / (32 * MT), n_tiles = (c.n + 32 * NT - 1) / (32 * NT);
   const int gm = m_tiles < kBandRows ? m_tiles : kBandRows;
   const FastDiv band = make_fast_div((uint32_t)(gm * n_tiles)), band_rows = make_fast_div((uint32_t)gm);
-  constexpr int lds_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow + kBiasBytes;
+  constexpr int lds_bytes = STAGES * KS * 32 * (MT + NT) * kStageRow + kBiasBytes + (PIECES ? 16 : 0);
   static_assert(lds_bytes > 64 * 1024 && lds_bytes <= 160 * 1024, "");
-  const auto kern = matmul_tile_kernel<T, MT, NT, KS, STAGES>;
+  const auto kern = matmul_tile_kernel<T, MT, NT, KS, STAGES, PIECES>;
+  std::conditional_t<PIECES, TilePieces, NoPieces> late;
+  if constexpr (PIECES) late = c.late;
   static std::atomic<uint64_t> attr_done{0};  // more than 64 KiB of dynamic LDS is an opt-in per device and kernel
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -276,8 +372,11 @@ template <typename T, int MT, int NT, int KS, int STAGES> hipError_t launch_tile
     if (e != hipSuccess) return e;
     attr_done.fetch_or(bit, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3(m_tiles * n_tiles), dim3(kTileThreads), lds_bytes, stream, c.a,
-                     u32x4_t{(uint32_t)c.m, (uint32_t)c.n, (uint32_t)c.k, band.l | band_rows.l << 16}, u32x2_t{band.m, band_rows.m});
+  const uint32_t tiles = (uint32_t)(m_tiles * n_tiles);
+  hipLaunchKernelGGL(kern, dim3(tiles * c.pieces), dim3(kTileThreads), lds_bytes, stream, c.a,
+                     u32x4_t{(uint32_t)c.m, (uint32_t)c.n, (uint32_t)c.k | (uint32_t)c.pieces << 21,
+                             band.l | band_rows.l << 5 | (65536u / tiles + 1) << 10},
+                     u32x2_t{band.m, band_rows.m}, late);
   return hipGetLastError();
 }
 
@@ -297,6 +396,7 @@ constexpr Tile kTiles[] = {
 constexpr int kTileKinds = sizeof(kTiles) / sizeof(kTiles[0]), kDeep = 1, kTall = 2, kWide = 3;  // 32 x 32 with more stages, 64 x 32, 32 x 64
 static_assert(kTiles[kTall].m == 2 * kTiles[kTall].n && kTiles[kWide].n == 2 * kTiles[kWide].m, "");
 
+#ifndef LLMHIP_BENCH
 template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStream_t stream) {
   using Launch = hipError_t (*)(const TileCall &, hipStream_t);
   static constexpr Launch launch[] = {
@@ -306,6 +406,7 @@ template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStr
   };
   return launch[kind](c, stream);
 }
+#endif
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
 // Over 270 sizes (16 weights of 256-11008 rows and k of 1536-18944, 17-4096 lhs rows, W from HBM) it takes 0.80 of hipBLASLt's
@@ -340,11 +441,38 @@ bool matmul_tile_takes(int m, int n, int k) {
   return k % kLineK == 0 && k <= 1 << 20 && tile_kind(m, n, k) >= 0;
 }
 
+// Few tiles of 32 x 32 over k of some thousands wait for a chain of 48 or more lines, and for the 30 to 45 GB/s that a CU gets from beyond its L2,
+// while most CUs have nothing to do: k is cut into as many pieces as give every CU a workgroup, of at least 12 lines.  A piece's sums
+// go past the L2 with tags and are added up by the workgroup of the last one: 2.2 us, a third of it the way there (us, whole / in
+// pieces, W from HBM, then in the last-level cache: 1024 x 5120, 16 rows 9.5 / 6.6, 8.2 / 5.9, 32 14.2 / 7.0, 8.3 / 6.0, 64 12.05 / 7.8,
+// 8.45 / 6.5, 128 10.9 / 9.8, 8.5 / 7.4; 512 x 3584, 9 rows 5.05 / 4.95, 4.8 / 4.9, 32 6.5 / 5.1, 64 6.3 / 5.4, 128 6.3 / 6.0; 3584 x 3584, 32 rows
+// 10.9 / 9.0, 6.75 / 6.4; 4096 x 4096, 32 rows 11.45 / 9.4; but 8 rows, for which W is read in shares, 1024 x 5120 5.9 / 6.35, 9 of two pieces, 3584 x 3584 7.8 / 8.0, and k below
+// 3072, 512 x 2048 4.4 / 4.6, 1536 x 1536 5.2 / 5.15, 3.75 / 4.7).  One line to a stage less and five stages: 3 to 10 % ahead of two or three of four
+// lines.  Tiles that are larger have too much to pass on (64 x 128 over half of 3584: 18.5 us, of them 3.5).  Not from k = 6144 on, where a call
+// gives the same bits under capture.
+int matmul_tile_pieces(int m, int n, int k) {
+  const long long cus = device_compute_units(), tiles = (long long)((m + 31) / 32) * ((n + 31) / 32);
+  if (m <= 8 || k % kLineK != 0 || k < 3072 || k >= 6144 || 2 * tiles > cus || tiles * cus >= 65536) return 1;
+  const long long by_cus = cus / tiles, by_lines = k / kLineK / 12, pieces = by_cus < by_lines ? by_cus : by_lines;
+  if (pieces == 2 && m < 12) return 1;
+  return (int)(pieces < kMostPieces ? pieces : kMostPieces);
+}
+size_t matmul_pieces_bytes(int m, int n, int pieces) { return (size_t)((m + 31) / 32) * ((n + 31) / 32) * pieces * kWordsBytes; }
+
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias, int m, int n, int k,
-                              int dt, hipStream_t stream) {
-  const TileCall c = {{address(lhs), address(weight), address(bias), address(out)}, m, n, k};
+                              int dt, hipStream_t stream, int pieces, void *workspace) {
+  TileCall c = {{address(lhs), address(weight), address(bias), address(out)}, m, n, k};
+  if (pieces > 1) {
+    c.pieces = pieces;
+    c.late = {static_cast<char *>(workspace), launch_number(), kLooks};
+    return dt == kDtFloat16 ? launch_tile<_Float16, 1, 1, 2, 5, true>(c, stream) : launch_tile<__bf16, 1, 1, 2, 5, true>(c, stream);
+  }
+#ifdef LLMHIP_BENCH
+  return hipErrorInvalidValue;
+#else
   const int kind = tile_kind(m, n, k);
   return dt == kDtFloat16 ? launch_kind<_Float16>(c, kind, stream) : launch_kind<__bf16>(c, kind, stream);
+#endif
 }
 
-}  // namespace llmhip
+}  // namespace LLMHIP_NS
