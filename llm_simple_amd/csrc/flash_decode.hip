@@ -1084,14 +1084,12 @@ static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
     const int pairs = p.batch * p.Hkv;
     grid = dim3(p.num_splits, pairs + (pairs * p.folders + p.num_splits - 1) / p.num_splits);
   }
-  hipLaunchKernelGGL(kern, grid, dim3(64 * NW), pad, stream, early.a, early.b, early.c, static_cast<const DecodeLate &>(p));
-  hipError_t e = hipGetLastError();
+  const hipError_t e = launch(kern, grid, 64 * NW, pad, stream, early.a, early.b, early.c, static_cast<const DecodeLate &>(p));
   if (e != hipSuccess || p.num_splits == 1 || FOLD != kNoFold) return e;
-  hipLaunchKernelGGL(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), dim3(256), 0, stream,
-                     addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), (uint64_t)p.tokens},
-                     u32x4_t{(uint32_t)p.num_splits, (uint32_t)p.cols, (uint32_t)p.Hkv, (uint32_t)p.m},
-                     u32x2_t{(uint32_t)p.g, 65536u / p.g + 1});
-  return hipGetLastError();
+  return launch(flash_decode_combine_kernel<T>, dim3(p.rows, p.Hkv, p.batch), 256, 0, stream,
+                addresses_t{address(p.ws_o), address(p.ws_ml), address(p.out), (uint64_t)p.tokens},
+                u32x4_t{(uint32_t)p.num_splits, (uint32_t)p.cols, (uint32_t)p.Hkv, (uint32_t)p.m},
+                u32x2_t{(uint32_t)p.g, 65536u / p.g + 1});
 }
 
 template <typename T, bool FUSED, FoldMode FOLD>

@@ -1208,32 +1208,29 @@ static hipError_t launch_prefill_t(const PrefillParams &p0, hipStream_t stream) 
   }
   const PrefillEarly early(p);
   if (cut) {
-    hipLaunchKernelGGL(ranges, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
+    e = launch(ranges, dim3(grid), NT, lds_bytes, stream, early.a, early.b, early.c, static_cast<const PrefillLate &>(p));
   } else if (p.cut) {
     PrefillHalves late = {};
     late.out = p.out;
     late.halves = p.halves;
     late.number = p.number;
     late.pairs = p.cut * p.H;
-    hipLaunchKernelGGL(halves, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, late);
+    e = launch(halves, dim3(grid), NT, lds_bytes, stream, early.a, early.b, early.c, late);
   } else {
     PrefillBrief brief;
     brief.out = p.out;
 #ifdef LLMHIP_BENCH
     brief.clock_probe = p.clock_probe;
 #endif
-    hipLaunchKernelGGL(whole, dim3(grid), dim3(NT), lds_bytes, stream, early.a, early.b, early.c, brief);
+    e = launch(whole, dim3(grid), NT, lds_bytes, stream, early.a, early.b, early.c, brief);
   }
-  e = hipGetLastError();
   if (e != hipSuccess || p.num_splits == 1) return e;
   const size_t slots = (size_t)p.m * p.H;
   const addresses_t a = {address(p.ws_o), address(p.ws_o + (size_t)p.num_splits * slots * kHeadDim), address(p.out), slots};
   const u32x2_t c = {(uint32_t)p.num_splits, __builtin_bit_cast(uint32_t, kScaleLog2e)};
   if (slots <= 2048 && p.num_splits >= 8)
-    hipLaunchKernelGGL(prefill_combine_wide_kernel<T>, dim3((unsigned)slots), dim3(256), 0, stream, a, c);
-  else
-    hipLaunchKernelGGL(prefill_combine_kernel<T>, dim3((unsigned)((slots + 7) / 8)), dim3(256), 0, stream, a, c);
-  return hipGetLastError();
+    return launch(prefill_combine_wide_kernel<T>, dim3((unsigned)slots), 256, 0, stream, a, c);
+  return launch(prefill_combine_kernel<T>, dim3((unsigned)((slots + 7) / 8)), 256, 0, stream, a, c);
 }
 
 // Compute units of the current device (the kernel choice and the split counts aim at them); 256 when

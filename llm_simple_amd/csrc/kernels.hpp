@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "common.hpp"
+#include "launch.hpp"
 
 namespace LLMHIP_NS {
 

@@ -190,12 +190,10 @@ hipError_t launch_add(void *out, const void *lhs, const void *rhs, size_t total,
   const size_t threads = (total + 7) / 8;
   const dim3 grid((unsigned)((threads + 255) / 256));
   if (dt == kDtFloat16)
-    hipLaunchKernelGGL(add_kernel<_Float16>, grid, dim3(256), 0, stream, (uint16_t *)out,
-                       (const uint16_t *)lhs, (const uint16_t *)rhs, total);
-  else
-    hipLaunchKernelGGL(add_kernel<__bf16>, grid, dim3(256), 0, stream, (uint16_t *)out,
-                       (const uint16_t *)lhs, (const uint16_t *)rhs, total);
-  return hipGetLastError();
+    return launch(add_kernel<_Float16>, grid, 256, 0, stream, (uint16_t *)out,
+                  (const uint16_t *)lhs, (const uint16_t *)rhs, total);
+  return launch(add_kernel<__bf16>, grid, 256, 0, stream, (uint16_t *)out,
+                (const uint16_t *)lhs, (const uint16_t *)rhs, total);
 }
 
 // Byte fill, the kernel behind llmhip_memset_async: a memset node recorded into a HIP graph has given wrong
@@ -220,9 +218,8 @@ hipError_t launch_fill(void *dst, int value, size_t bytes, hipStream_t stream) {
   size_t blocks = (bytes / 16 + 255) / 256;
   if (blocks < 1) blocks = 1;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(fill_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<unsigned char *>(dst),
-                     (unsigned char)value, bytes);
-  return hipGetLastError();
+  return launch(fill_kernel, dim3((unsigned)blocks), 256, 0, stream, static_cast<unsigned char *>(dst),
+                (unsigned char)value, bytes);
 }
 
 }  // namespace llmhip

@@ -170,10 +170,9 @@ hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, 
   const int rounds = (n + 16 * cus - 1) / (16 * cus);
   const int rows = (n + rounds * cus - 1) / (rounds * cus);
   const SkinnyKernel kern = dt == kDtFloat16 ? kernel_of<_Float16>(m, k, rows) : kernel_of<__bf16>(m, k, rows);
-  hipLaunchKernelGGL(kern, dim3((n + rows - 1) / rows), dim3(64 * kSkinnyWaves), 0, stream,
-                     addresses_t{address(lhs), address(weight), address(bias), address(out)},
-                     u32x4_t{(uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)rows});
-  return hipGetLastError();
+  return launch(kern, dim3((n + rows - 1) / rows), 64 * kSkinnyWaves, 0, stream,
+                addresses_t{address(lhs), address(weight), address(bias), address(out)},
+                u32x4_t{(uint32_t)m, (uint32_t)n, (uint32_t)k, (uint32_t)rows});
 }
 
 }  // namespace llmhip

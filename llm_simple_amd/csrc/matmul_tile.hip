@@ -373,11 +373,10 @@ template <typename T, int MT, int NT, int KS, int STAGES, bool PIECES = false> h
     attr_done.fetch_or(bit, std::memory_order_release);
   }
   const uint32_t tiles = (uint32_t)(m_tiles * n_tiles);
-  hipLaunchKernelGGL(kern, dim3(tiles * c.pieces), dim3(kTileThreads), lds_bytes, stream, c.a,
-                     u32x4_t{(uint32_t)c.m, (uint32_t)c.n, (uint32_t)c.k | (uint32_t)c.pieces << 21,
-                             band.l | band_rows.l << 5 | (65536u / tiles + 1) << 10},
-                     u32x2_t{band.m, band_rows.m}, late);
-  return hipGetLastError();
+  return launch(kern, dim3(tiles * c.pieces), kTileThreads, lds_bytes, stream, c.a,
+                u32x4_t{(uint32_t)c.m, (uint32_t)c.n, (uint32_t)c.k | (uint32_t)c.pieces << 21,
+                        band.l | band_rows.l << 5 | (65536u / tiles + 1) << 10},
+                u32x2_t{band.m, band_rows.m}, late);
 }
 
 // Lhs rows, features, lines of a stage and stages of the tiles; see tile_kind for their order

@@ -165,11 +165,10 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
   const long long threads = placed ? (long long)((cur_size + (1 << share) - 1) >> share) * list_rows * 8 : total;
   const int grid = (int)((threads + 255) / 256) * (placed ? 8 : 1);
   const auto kern = (dt == kDtFloat16) ? kernel_of<_Float16>(is_neox, way) : kernel_of<__bf16>(is_neox, way);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, stream, addresses_t{address(in_q), address(in_k), address(in_v), address(freq_cis)},
-                     u32x4_t{(uint32_t)(placed ? cur_size : total), div.m,
-                             div.l | (in_v != nullptr ? 256u : 0u) | (placed ? (uint32_t)share << 9 : 0u), (uint32_t)start_pos},
-                     u32x2_t{(uint32_t)q_heads, (uint32_t)k_heads}, to);
-  return hipGetLastError();
+  return launch(kern, dim3(grid), 256, 0, stream, addresses_t{address(in_q), address(in_k), address(in_v), address(freq_cis)},
+                u32x4_t{(uint32_t)(placed ? cur_size : total), div.m,
+                        div.l | (in_v != nullptr ? 256u : 0u) | (placed ? (uint32_t)share << 9 : 0u), (uint32_t)start_pos},
+                u32x2_t{(uint32_t)q_heads, (uint32_t)k_heads}, to);
 }
 
 }  // namespace llmhip
