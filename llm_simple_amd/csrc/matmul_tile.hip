@@ -445,7 +445,9 @@ bool matmul_tile_takes(int m, int n, int k) {
 // go past the L2 with tags and are added up by the workgroup of the last one: 2.2 us, a third of it the way there (us, whole / in
 // pieces, W from HBM, then in the last-level cache: 1024 x 5120, 16 rows 9.5 / 6.6, 8.2 / 5.9, 32 14.2 / 7.0, 8.3 / 6.0, 64 12.05 / 7.8,
 // 8.45 / 6.5, 128 10.9 / 9.8, 8.5 / 7.4; 512 x 3584, 9 rows 5.05 / 4.95, 4.8 / 4.9, 32 6.5 / 5.1, 64 6.3 / 5.4, 128 6.3 / 6.0; 3584 x 3584, 32 rows
-// 10.9 / 9.0, 6.75 / 6.4; 4096 x 4096, 32 rows 11.45 / 9.4; but 8 rows, for which W is read in shares, 1024 x 5120 5.9 / 6.35, 9 of two pieces, 3584 x 3584 7.8 / 8.0, and k below
+// 10.9 / 9.0, 6.75 / 6.4; 4096 x 4096, 32 rows 11.45 / 9.4; but 8 rows, for which W is read in shares, 1024 x 5120 5.9 / 6.35, two pieces of
+// fewer than 24 rows, where a part whose way past the L2s is 1 us longer gains nothing from HBM and loses from the cache, 3584 x 3584,
+// 17 rows 9.25 / 9.25, 6.65 / 8.5 (32 there 10.8 / 9.7, 7.0 / 8.5; blocks of 30 and 32 rows gain 6 and 18 %), and k below
 // 3072, 512 x 2048 4.4 / 4.6, 1536 x 1536 5.2 / 5.15, 3.75 / 4.7).  One line to a stage less and five stages: 3 to 10 % ahead of two or three of four
 // lines.  Tiles that are larger have too much to pass on (64 x 128 over half of 3584: 18.5 us, of them 3.5).  Not from k = 6144 on, where a call
 // gives the same bits under capture.
@@ -453,7 +455,7 @@ int matmul_tile_pieces(int m, int n, int k) {
   const long long cus = device_compute_units(), tiles = (long long)((m + 31) / 32) * ((n + 31) / 32);
   if (m <= 8 || k % kLineK != 0 || k < 3072 || k >= 6144 || 2 * tiles > cus || tiles * cus >= 65536) return 1;
   const long long by_cus = cus / tiles, by_lines = k / kLineK / 12, pieces = by_cus < by_lines ? by_cus : by_lines;
-  if (pieces == 2 && m < 12) return 1;
+  if (pieces == 2 && m < 24) return 1;
   return (int)(pieces < kMostPieces ? pieces : kMostPieces);
 }
 size_t matmul_pieces_bytes(int m, int n, int pieces) { return (size_t)((m + 31) / 32) * ((n + 31) / 32) * pieces * kWordsBytes; }

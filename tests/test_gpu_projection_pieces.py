@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 CUT = [(9, 1024, 5120), (16, 512, 3584), (17, 16, 3072), (31, 1008, 4160), (32, 4096, 3072), (33, 1024, 6080), (64, 2032, 3648), (65, 496, 5120),
        (97, 1024, 5056), (128, 1024, 3136), (40, 528, 6016)]
-WHOLE = [(8, 1024, 5120), (11, 3584, 3584), (9, 1024, 3008), (33, 2064, 3584), (17, 4112, 3072), (16, 1024, 6144), (24, 1024, 4000)]
+WHOLE = [(8, 1024, 5120), (23, 3584, 3584), (9, 1024, 3008), (33, 2064, 3584), (17, 4112, 3072), (16, 1024, 6144), (24, 1024, 4000)]
 
 
 def inputs(m, n, k, dt):
