@@ -32,12 +32,13 @@
 // (4096 x 4096, 1024 rows: 40 -> 36.6 us; 3584 x 3584, 2048 rows, W from HBM: 51.8 -> 49.5, kernel of eight waves).
 //   A CU draws no more than 30 to 45 GB/s from beyond its XCD's L2, however much it has under way.  Tiles of the same W rows that
 // take the lines in one order leave all of that to the one that is ahead, and the others wait with it (3584 x 3584, 256 rows: 31 GB/s of
-// W to a tile of 64 rows, and as long with 112 workgroups as with 224).  So lines go in groups of 8, and each of up to 4 such tiles
+// W to a tile of 64 rows, and as long with 112 workgroups as with 224).  So lines go in groups, and each of up to 4 such tiles
 // begins at another place of a group: the first to ask for a line is a different one each time, and the rest find it in the L2 a moment later
-// (us, one order / so, W from HBM: 3584 x 3584, 64 rows 10.7 / 9.5, 256 18.5 / 14.6, 512 24.2 / 20.8, 1024 30.9 / 28.3, 2048 48.0 /
-// 46.5; 4096 x 4096, 256 rows 20.3 / 16.5; 5120 x 5120, 384 rows 36.9 / 31.0; 1024 x 5120, 128 rows 13.3 / 11.1).  Half or a quarter of k apart
-// instead, the small ones are as fast, but what the L2 has to keep in between outgrows it (3584 x 3584, 1024 rows 36.0); groups of 4 or 16 lose 1-3 %
-// either at the small or at the large sizes; turns by the tile's W rows too, for those that share lhs rows, change nothing.
+// (us, one order / so, W from HBM: 3584 x 3584, 64 rows 10.4 / 9.0, 256 18.2 / 13.9, 512 24.1 / 20.2, 1024 30.2 / 27.2, 2048 44.0 / 43.0;
+// 4096 x 4096, 256 rows 20.2 / 15.3; 5120 x 5120, 768 rows 47.9 / 43.7).  With W in the last-level cache it costs 1-3 % (3584 x 3584, 256
+// rows 11.5 / 12.2, 1024 24.5 / 25.0), and more the larger group and tile are, the lines of a group being in the L2 longer: hence groups of 8, 4 and 2
+// (2048 rows by groups of 8 43.8).  Where lhs is the larger operand there is nothing to gain (512 x 3584, 2048 rows 11.6 / 12.6 by groups of 8).  Half
+// or a quarter of k apart instead, the small ones are as fast, but what the L2 has to keep outgrows it (1024 rows 36.0).
 //   Stages under way: as few as hold 64 to 100 KiB, but for 96 x 64.  More of them are no faster anywhere, and begin with a longer burst (5 / 9 stages of a
 // 64 x 64 tile, us: 512 x 3584, 2048 rows 12.6 / 13.1, 3584 x 3584, 256 rows 14.15 / 14.55; 3 / 4 of 32 x 32, 512 x 3584, 512 rows 7.1 / 7.35;
 // 3 / 5 of 96 x 128, 3584 x 3584, 768 rows 24.0 / 24.9; one line to a stage less and four stages of 64 x 32: 256 x 1536, 2048 rows 5.65 / 5.45).
@@ -186,9 +187,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
   using False = std::false_type;
   [[maybe_unused]] bool alone = false;
   for (;;) {  // (once, unless a workgroup that has waited in vain for the sums of others makes them itself)
-    // The order of the lines: each XCD begins at another eighth, and in every group of 8 (4, 2: what divides k) each tile of those that share
-    // W rows at another place.  Not where a quarter of the last one is padding: begun ahead of the others it stays there, and fetches for them.
-    // Of a piece each tile begins elsewhere.
+    // The order of the lines: each XCD begins at another eighth, and where W is the larger operand, in every group of 8, of 4 (tiles from 96 x 64 on) or
+    // of 2 (from 128 x 160 on, and what divides k) each tile of those that share W rows at another place.  Not where a quarter of the last one is padding:
+    // begun ahead of the others it stays there, and fetches for them.  Of a piece each tile begins elsewhere.
     int lines = all_lines;
     uint32_t from = 0, end = row_bytes, pos, turn = 0;
     if constexpr (PIECES) {
@@ -201,8 +202,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
       const bool padded = m_tiles <= kBandRows && 4 * (m - (m_tiles - 1) * BM) <= 3 * BM;
       pos = (((uint32_t)(xcd * lines) >> 3) + ((padded ? t : tn) & 3)) * kStageRow;
       if (pos >= row_bytes) pos = 0;
-      const int group = lines % 8 == 0 ? 8 : lines % 4 == 0 ? 4 : lines % 2 == 0 ? 2 : 1;
-      turn = padded ? 0u : (uint32_t)(in_band * group >> (rows_here == 2 ? 1 : 2)) * kStageRow;
+      constexpr int kGroup = L <= 4 ? 8 : L <= 8 ? 4 : 2;
+      const int group = min(lines & -lines, kGroup);
+      turn = padded || n < m ? 0u : (uint32_t)(group == 2 ? in_band & 1 : in_band * group >> (rows_here == 2 ? 1 : 2)) * kStageRow;
     }
     const int stages = (lines + KS - 1) / KS, last_lines = lines - (stages - 1) * KS;
     uint32_t kpos = pos ^ turn;
@@ -320,11 +322,43 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
       __syncthreads();  // (nobody reads the lines of the piece before any more)
     }
   }
-  const int row0 = m0 + wm * (BM / 2);
+  if constexpr (MT * NT <= 2) {  // (two barriers and a way through LDS take longer there: 512 x 2048, 24 rows 4.56 / 4.70)
+    const int row0 = m0 + wm * (BM / 2);
+#pragma unroll
+    for (int b = 0; b < NT; b += 2) {
+      const bool two = b + 1 < NT;
+      const int c = 16 * b + (two ? 8 : 4) * cg, col = col0 + c;
+      f32x4_t b0 = {0.f, 0.f, 0.f, 0.f}, b1 = b0;
+      if (bias) {
+        b0 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c);
+        if (two) b1 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c + 16);
+      }
+#pragma unroll
+      for (int a = 0; a < MT; ++a) {
+        const int row = row0 + 16 * a + i;
+        const f32x4_t u = acc[a][b] + b0;
+        uint16_t *o = out + (size_t)row * n + col;
+        if (two) {
+          const f32x4_t v = acc[a][b + 1 < NT ? b + 1 : b] + b1;
+          if (row < m && col < n)
+            *reinterpret_cast<u32x4_t *>(o) = u32x4_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3]), E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+        } else if (row < m && col < n) {
+          *reinterpret_cast<u32x2_t *>(o) = u32x2_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3])};
+        }
+      }
+    }
+    return;
+  }
+  // The tile leaves as whole rows, by way of the lines' place (rows 16 bytes apart from a multiple of the banks), and past the L2, where they are whole
+  // sectors: lines that are left there are written back at the end of the launch.  (Block of Qwen2.5-7B, 2048 tokens, us, pieces of 64 bytes and
+  // ordinary stores / rows / rows past the L2: 174.5 / 173.8 / 170.6; 3584 x 3584, 2048 rows 43.05 / 42.65 / 41.9, 1536 x 1536 12.05 / 12.0 / 11.6.)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  constexpr int kRow = 2 * BN + 16;
+  static_assert(BM * kRow <= STAGES * kStageBytes, "");
 #pragma unroll
   for (int b = 0; b < NT; b += 2) {
     const bool two = b + 1 < NT;
-    const int c = 16 * b + (two ? 8 : 4) * cg, col = col0 + c;
+    const int c = 16 * b + (two ? 8 : 4) * cg;
     f32x4_t b0 = {0.f, 0.f, 0.f, 0.f}, b1 = b0;
     if (bias) {
       b0 = *reinterpret_cast<const f32x4_t *>(lds + bias_at + 4 * c);
@@ -332,16 +366,27 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
     }
 #pragma unroll
     for (int a = 0; a < MT; ++a) {
-      const int row = row0 + 16 * a + i;
+      char *at = lds + (wm * (BM / 2) + 16 * a + i) * kRow + (wn * (BN / 2) + c) * 2;
       const f32x4_t u = acc[a][b] + b0;
-      uint16_t *o = out + (size_t)row * n + col;
       if (two) {
         const f32x4_t v = acc[a][b + 1 < NT ? b + 1 : b] + b1;
-        if (row < m && col < n)
-          *reinterpret_cast<u32x4_t *>(o) = u32x4_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3]), E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
-      } else if (row < m && col < n) {
-        *reinterpret_cast<u32x2_t *>(o) = u32x2_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3])};
+        *reinterpret_cast<u32x4_t *>(at) = u32x4_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3]), E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+      } else {
+        *reinterpret_cast<u32x2_t *>(at) = u32x2_t{E::pack2(u[0], u[1]), E::pack2(u[2], u[3])};
       }
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  constexpr int kPieces = BN / 8;  // of a row
+  const bool sectors = (a_[3] & 63) == 0 && n % 32 == 0;
+#pragma unroll
+  for (int j = 0; j < (BM * kPieces + kTileThreads - 1) / kTileThreads; ++j) {
+    const int piece = tid + j * kTileThreads, r = piece / kPieces, c = piece - r * kPieces;
+    if (r < BM && m0 + r < m && n0 + 8 * c < n) {
+      const u32x4_t v = lds_read_b128(lds, r * kRow + 16 * c);
+      uint16_t *o = out + (size_t)(m0 + r) * n + n0 + 8 * c;
+      if (sectors) store_device_b128(o, v);
+      else *reinterpret_cast<u32x4_t *>(o) = v;
     }
   }
 }
