@@ -99,6 +99,7 @@ struct DecodeParams : DecodeLate {
   int g, Hkv, rows;
   int is_neox;
   bool fused;
+  bool two;  // workgroups to a CU
   int cols;  // columns of a partial's slot: 16, or 8 of workgroups of two waves
 };
 // a: q, K, V, then freq_row or kv_seq_stride; b: new_k and new_v, or rows | m << 8 | tokens << 16, 2^16 / g + 1, offset, pairs | 2^20 / Hkv (rounded
@@ -914,7 +915,7 @@ int flash_decode_max_default_splits(long long pairs) {
   return (int)base;
 }
 
-// Split count that a simple model of the launch makes fastest.  Workgroups run one per CU.  While each has a CU of its own, a CU
+// Split count that a simple model of the launch makes fastest.  One workgroup to a CU (two: the next model).  While each has a CU of its own, a CU
 // streams the more the fewer they are (32 KiB in flight, over a latency that grows with the load); beyond that a CU streams 27.9
 // GB/s (all 256 of an MI355X together 7.1 TB/s, what its memory system gives a kernel that only reads) and the launch takes
 // something between the rounds that the fullest CU runs and the mean of all.  A fold by folders costs 0.9 us in blocks of 64
@@ -938,6 +939,23 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus, int r
   if (s == nblocks && 2 * s <= kFoldDepth && pairs * (s == 2 ? 6 : 2 * s) <= cus && rows < kDecCols / 2) return t + 0.9;
   return t + (s <= kFoldDepth ? 2.0 : s <= 16 ? 1.8 : 1.4);
 }
+// Two workgroups to a CU, where there are more of them than CUs: what one does not stream while it begins, merges its waves and stores, the other one
+// does, and it is that which short rounds lose most to; 64 KiB are in flight then, with which a stream is slower (us, one to a CU / two, each with
+// its best count: 10 sequences of 32 kv heads, 300 keys 14.2 / 12.2, 700 25.8 / 21.9, 1024 32.6 / 29.3, 1500 43.0 / 40.5, 3000 78.5 / 76.8; 2 blocks,
+// 480 pairs 11.85 / 9.0; but 16 x 1500 of 32 kv heads, two even rounds, 58.2 / 61.6, 16 x 32768 of 8 295 / 325).  A workgroup's number within its XCD's
+// share repeats with the split, so that the XCD of the longer ones counts.  Fitted over 1261 shapes of 1-16 sequences, 2-32 kv heads, 64-32768 keys, up to 1.1 GB
+// and 17 counts each.  Two are taken where the model has them 4 % ahead, 160 of the shapes: 0.865 of the time there on average, none of all slower
+// by 2 %.
+static double two_model_us(long long pairs, int nblocks, int s, int cus) {
+  const long long wgs = pairs * s;
+  if (wgs <= cus || (s > 1 && nblocks < 2 * s)) return 1e30;  // (one block each: the fold is the larger part)
+  constexpr double kBlockKb = 2.0 * kRowBytes * kDecStepKeys * 1e-3;
+  const int classes = s % 8 == 0 ? 8 : s % 4 == 0 ? 4 : s % 2 == 0 ? 2 : 1;  // of splits, an XCD's each
+  const double mean = nblocks / s + (double)((nblocks % s + classes - 1) / classes * classes) / s;
+  const double rounds = 0.28 * 2 * (double)((wgs + 2 * cus - 1) / (2 * cus)) + 0.72 * (double)wgs / cus;
+  return rounds * kBlockKb * (0.05 * ((nblocks + s - 1) / s) + 0.95 * mean) / 27.1 + 1.92 + (s > 1 ? 2.46 : 0.0);
+}
+constexpr double kTwoMargin = 0.96;
 // The smallest count within `tolerance` of the best, or one that fills up to full_rounds rounds exactly.
 template <typename Model>
 static int best_splits(long long pairs, int smax, int cus, double tolerance, long long full_rounds, Model model) {
@@ -954,11 +972,24 @@ static int best_splits(long long pairs, int smax, int cus, double tolerance, lon
   }
   return first;
 }
-static int default_splits_model(long long pairs, int nblocks, int cus, int most, int rows) {
+static int default_splits_model(long long pairs, int nblocks, int cus, int most, int rows, bool may_two = true) {
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
   if (smax > most) smax = most;
-  return best_splits(pairs, smax, cus, 1.005, 1, [&](int s) { return split_model_us(pairs, nblocks, s, cus, rows); });
+  const int one = best_splits(pairs, smax, cus, 1.005, 1, [&](int s) { return split_model_us(pairs, nblocks, s, cus, rows); });
+  double least = kTwoMargin * split_model_us(pairs, nblocks, one, cus, rows);
+  int best = one;
+  for (int s = 1; may_two && s <= smax; ++s) {
+    const double t = two_model_us(pairs, nblocks, s, cus);
+    if (t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  return best;
+}
+static bool two_to_a_cu(long long pairs, int nblocks, int s, int cus, int rows) {
+  return two_model_us(pairs, nblocks, s, cus) < kTwoMargin * split_model_us(pairs, nblocks, s, cus, rows);
 }
 
 // The model is evaluated a few hundred times per call; a decode loop asks for the same (pairs, key
@@ -996,8 +1027,8 @@ int flash_decode_splits_within(int batch, int n, int kv_head_num, int rows, size
 // What a call may insist on is counted with coarser figures than the default: 27.7 GB/s per CU in a full round and at most
 // 32 in a thin one, 3 us per workgroup, 5 for a fold.  Callers were promised that calls which are not worth a split by
 // these need no room; the promise does not move with the model above.  Nor does it move for callers whose workspace was sized by the default
-// count of the model before (whole rounds, folds of 1.2 to 2.6 us): the smaller of the two is enough (3 x 3584 keys of 8 kv heads: 10 of
-// now, 7 before, 10 by the coarser figures).
+// count of a model before (whole rounds, folds of 1.2 to 2.6 us, or one workgroup to a CU only): the smallest of the three is enough (3 x 3584 keys of 8
+// kv heads: 10 of the second, 7 of the first, 10 by the coarser figures).
 size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
   const long long pairs = (long long)batch * kv_head_num;
   const int nblocks = (n + kDecStepKeys - 1) / kDecStepKeys, cus = device_compute_units();
@@ -1022,7 +1053,10 @@ size_t flash_decode_least_workspace_bytes(int batch, int n, int kv_head_num) {
     if (splits == nblocks && 2 * splits <= kFoldDepth && 2 * pairs * splits <= cus) return t + 1.2;
     return t + (splits <= kFoldDepth ? 2.0 : splits <= 16 ? 2.6 : 2.1);
   });
-  return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, coarse < before ? coarse : before);
+  int least = default_splits_model(pairs, nblocks, cus, kMaxSplits, 1, false);
+  for (const int s : {default_splits_model(pairs, nblocks, cus, kMaxSplits, kDecCols, false), coarse, before})
+    if (s < least) least = s;
+  return flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, least);
 }
 
 int flash_decode_effective_splits(int num_splits, int n) {
@@ -1061,10 +1095,10 @@ bool may_be_capturing(hipStream_t stream) {
 
 template <typename T, bool FUSED, int NW, bool LONG, FoldMode FOLD>
 static hipError_t launch_decode_t(const DecodeParams &p, hipStream_t stream) {
-  // kDecLdsPad bytes of dynamic LDS that nobody touches keep a second workgroup off the CU (two of
-  // them would put 64 KiB of loads in flight again).  More than 64 KiB of LDS in total is an opt-in
+  // kDecLdsPad bytes of dynamic LDS that nobody touches keep a second workgroup off the CU where it is not wanted (two of
+  // them put 64 KiB of loads in flight again, see two_model_us).  More than 64 KiB of LDS in total is an opt-in
   // per device and kernel.
-  constexpr int pad = NW == 4 ? kDecLdsPad : 0;
+  const int pad = NW == 4 && !p.two ? kDecLdsPad : 0;
   const auto kern = flash_decode_kernel<T, FUSED, NW, LONG, FOLD>;
   if (pad) {
     static std::atomic<uint64_t> attr_done{0};
@@ -1155,6 +1189,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
   p.ws_o = static_cast<float *>(workspace);
   p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;
+  p.two = !half && two_to_a_cu(pairs, nblocks, p.num_splits, cus, p.rows);
   const bool many = p.iters_each >= 8;  // long enough to be bound by the stream, see the kernel
   if (dt == kDtFloat16)
     return fused ? launch_decode<_Float16, true>(p, how, half, many, stream) : launch_decode<_Float16, false>(p, how, half, many, stream);
