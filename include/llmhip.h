@@ -229,7 +229,8 @@ int llmhip_release_internal_workspace(void);
  * reference's Ascend "nz" repacking [n/16][k][16] (tests/gemm_test.cpp:95-101).  n and k
  * must be multiples of 16 (src/llama2_layer_npu.cpp:1211-1218).  Runs on kernels of this library up to 16 rows, and where its
  * tiles fit the chip in one round (16-byte aligned pointers; k a multiple of 64 beyond 16 rows); other calls run on
- * hipBLASLt, the first of which allocates its handle and a 64 MiB workspace. */
+ * hipBLASLt, the first of which allocates its handle and a 64 MiB workspace.  Few tiles over a k of 3072 to 6143 sum pieces of k
+ * in the stream's scratch, as far as it can be had outside of capture: a captured call may differ in the last bit. */
 int llmhip_matmul(void *out, const void *lhs, const void *weight, int m, int n, int k, int dt,
                   void *stream);
 
