@@ -44,9 +44,9 @@
 // 3 / 5 of 96 x 128, 3584 x 3584, 768 rows 24.0 / 24.9; one line to a stage less and four stages of 64 x 32: 256 x 1536, 2048 rows 5.65 / 5.45).
 //
 // bf16, us, hipBLASLt / here, back-to-back calls, W walked through 800 MB (hipBLASLt takes the host 10-13 us a call, which is
-// what its small sizes show): 3584 x 3584: 64 rows 13.7 / 11.1, 128 rows 22.5 / 14.5, 256 rows 20.1 / 18.8, 768 rows 32.2 / 26.8,
-// 2048 rows 55.9 / 47.0; 512 x 3584: 100 rows 13.4 / 7.1, 2048 rows 19.3 / 13.2; 1536 x 1536: 128 rows 9.7 / 5.7; 5120 x 5120: 100
-// rows 27.6 / 25.2, 1280 rows 76.1 / 59.8 (before the order of lines above).
+// what its small sizes show): 3584 x 3584: 64 rows 13.7 / 9.4, 128 rows 22.5 / 11.5, 256 rows 20.1 / 14.1, 768 rows 32.2 / 23.9,
+// 2048 rows 55.9 / 44.1; 512 x 3584: 100 rows 13.4 / 6.7, 2048 rows 19.3 / 12.4; 1536 x 1536: 128 rows 9.7 / 4.8; 5120 x 5120: 100
+// rows 27.6 / 24.7, 1280 rows 76.1 / 55.3.
 #include <atomic>
 #include <type_traits>
 
@@ -454,11 +454,11 @@ template <typename T> hipError_t launch_kind(const TileCall &c, int kind, hipStr
 
 // The smallest tile that needs no more workgroups than there are CUs: the chain of a workgroup is the shortest then.
 // Over 270 sizes (16 weights of 256-11008 rows and k of 1536-18944, 17-4096 lhs rows, W from HBM) it takes 0.80 of hipBLASLt's
-// time on average.  Taken though slower, so that no such call needs hipBLASLt's handle and 64 MiB workspace (which a stream under
+// time on average, before the lines went in turns.  Taken though slower, so that no such call needs hipBLASLt's handle and 64 MiB workspace (which a stream under
 // capture cannot create): few rows over k = 8192, which hipBLASLt cuts (us, hipBLASLt / here: 1024 x 8192, 17 rows 11.8 / 15.4,
 // 64 rows 13.8 / 17.5; 2048 x 8192, 24 rows 14.0 / 18.3; 4096 x 8192, 17 rows 17.2 / 17.2, 32 rows 18.3 / 20.3; not so 1536 x
-// 8960, 17 rows 28.2 / 19.0, 3584 x 18944, 32 rows 109.6 / 48.4); 5120 x 5120, 64 rows 21.5 / 22.9; 4096 x 11008, 680 rows 80.5 /
-// 85.0.  More than one round is not: 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 /
+// 8960, 17 rows 28.2 / 19.0, 3584 x 18944, 32 rows 109.6 / 48.4; 64 rows of 1024 x 8192 15.1 by now; 5120 x 5120, 64 rows 21.5 / 18.9, 4096 x 11008, 680 rows
+// 80.5 / 71.3).  More than one round is not: 5120 x 5120, 2048 rows 100.5 / 101.4 with 128 x 160 tiles, 3584 x 3584, 2048 rows 54.4 /
 // 54.5 with 128 x 128.
 //   Of 64 x 32 and 32 x 64 the second where W is much the larger operand and next to nothing is padding: up to 4 tiles then share its rows,
 // and not two (us, 64 x 32 / 32 x 64: 3584 x 3584, 128 rows 12.5 / 11.7, 5120 x 5120, 64 rows 23.1 / 19.0, with 320 workgroups; but
