@@ -26,6 +26,13 @@ int llmhip_bench_flash_attn_gqa_clocked(void *out, const void *q, const void *k,
                                         int n, int offset, int group_size, int kv_head_num, int head_dim,
                                         int dt, void *clock_probe, void *stream);
 
+/* llmhip_flash_attn_gqa of a prompt whose longest rows two workgroups share, on this library's own copy of the kernel, in which the second one of a
+ * pair to begin does not wait for the first one's half of the keys but goes over both by itself, as the product's does when it has looked for it in
+ * vain for some 0.1 s: the results are those of whole rows.  LLMHIP_ERR_UNSUPPORTED for other sizes; LLMHIP_ERR_WORKSPACE if workspace is too small (16 MiB
+ * are enough for any on 256 compute units).  On a capturing stream no rows are shared. */
+int llmhip_bench_flash_attn_gqa_alone(void *out, const void *q, const void *k, const void *v, void *workspace, size_t workspace_bytes,
+                                      int m, int n, int offset, int group_size, int kv_head_num, int head_dim, int dt, void *stream);
+
 /* llmhip_flash_decode_gqa and llmhip_decode_step_gqa (llmhip.h) on this library's own copy of the decode kernel, in which the
  * workgroups that fold partials do not wait for them: each computes its rows from the caches by itself, as the product's do
  * when they have looked for partials in vain for some 50 ms.  num_splits >= 1 and a workspace of

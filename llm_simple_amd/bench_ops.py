@@ -12,6 +12,7 @@ LIB_PATH = os.path.join(_HERE, "libllmhip_bench.so")
 _vp, _i, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
 SYMBOLS = {
     "llmhip_bench_flash_attn_gqa_clocked": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _vp]),
+    "llmhip_bench_flash_attn_gqa_alone": (_i, [_vp] * 5 + [_sz] + [_i] * 7 + [_vp]),
     "llmhip_bench_flash_decode_gqa_alone": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, ctypes.c_int64, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_decode_step_gqa_alone": (_i, [_vp] * 8 + [_sz, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_matmul_alone": (_i, [_vp] * 5 + [_sz, _i, _i, _i, _i, _vp]),
@@ -48,6 +49,15 @@ def hip_flash_attn_gqa_clocked_layer(output_dev, q_dev, k_dev, v_dev, m, n, offs
     _check(lib.llmhip_bench_flash_attn_gqa_clocked(p(output_dev), p(q_dev), p(k_dev), p(v_dev), m, n, offset,
                                                    group_size, kv_head_num, head_dim, dt, p(clock_probe_dev),
                                                    stream), "hip_flash_attn_gqa_clocked_layer")
+
+
+def hip_flash_attn_gqa_alone_layer(output_dev, q_dev, k_dev, v_dev, ws_dev, ws_bytes, m, n, offset, group_size, kv_head_num, head_dim, dt,
+                                   stream=0):
+    """hip_flash_attn_gqa_layer of a prompt whose longest rows two workgroups share, on the measurement library's copy, in which the second
+    of a pair goes over both halves of the keys by itself."""
+    p = ops._ptr
+    _check(lib.llmhip_bench_flash_attn_gqa_alone(p(output_dev), p(q_dev), p(k_dev), p(v_dev), p(ws_dev), ws_bytes, m, n, offset, group_size,
+                                                 kv_head_num, head_dim, dt, stream), "hip_flash_attn_gqa_alone_layer")
 
 
 def hip_flash_decode_gqa_alone_layer(output_dev, q_dev, k_dev, v_dev, ws_dev, ws_bytes, batch, n, kv_seq_stride, group_size,

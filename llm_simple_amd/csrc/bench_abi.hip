@@ -35,7 +35,24 @@ int llmhip_bench_flash_attn_gqa_clocked(void *out, const void *q, const void *k,
   if ((long long)m * group_size <= 16) return LLMHIP_ERR_UNSUPPORTED;  // prefill kernel only
   if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
   return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
-                                       static_cast<hipStream_t>(stream), clock_probe));
+                                       static_cast<hipStream_t>(stream), nullptr, 0, clock_probe));
+}
+
+int llmhip_bench_flash_attn_gqa_alone(void *out, const void *q, const void *k, const void *v, void *workspace, size_t workspace_bytes,
+                                      int m, int n, int offset, int group_size, int kv_head_num, int head_dim, int dt, void *stream) {
+  if (!out || !q || !k || !v || !workspace || !aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(workspace))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (m < 1 || n < 1 || offset < 0 || group_size < 1 || kv_head_num < 1 ||
+      (dt != LLMHIP_DT_FLOAT16 && dt != LLMHIP_DT_BFLOAT16))
+    return LLMHIP_ERR_INVALID_ARG;
+  if (head_dim != 128 || kv_head_num > 65535 || (long long)group_size * kv_head_num > 65535 || (long long)m * group_size <= 16)
+    return LLMHIP_ERR_UNSUPPORTED;
+  const size_t need = flash_prefill_halves_bytes(m, n, offset, group_size, kv_head_num);
+  if (!need) return LLMHIP_ERR_UNSUPPORTED;
+  if (need > workspace_bytes) return LLMHIP_ERR_WORKSPACE;
+  if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;
+  return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt, static_cast<hipStream_t>(stream),
+                                       workspace, workspace_bytes, nullptr));
 }
 
 int llmhip_bench_flash_decode_gqa_alone(void *out, const void *q, const void *k_cache, const void *v_cache, void *workspace,

@@ -66,7 +66,7 @@ constexpr int kWholeRange = 0x7fffffc0;          // keys of a range without an e
 constexpr int kFewRows = 64;                     // rows up to which partials are stored straight from registers
 
 // Keys of a workgroup: all that its rows see; a range of them, its partial to be folded by a launch of its own; all, but a half where
-// two workgroups have the longest rows (see fold_halves)
+// two workgroups have the longest rows (see pass_half)
 enum PrefillKeys { kAllKeys, kRanges, kHalves };
 
 // What a launch is told beyond what its first loads need (PrefillEarly): fetched while those are under way -- except with SPLIT, where
@@ -572,7 +572,13 @@ __device__ __forceinline__ void store_partial_rows(const WaveAttn<T, KB> &w, cha
 // The longest rows of a prompt, dealt to two workgroups: each has half of the keys, and the one that began first passes what it has to
 // the other, lane by lane as it lies in registers, every word beside half of the launch's number, past the XCD's L2.  No fence, no flag;
 // the other looks at what is stored last until it finds the number, then at all.  Both in the order of the halves, whoever folds.
+//   The wait has an end, 0.1 s (the other one is under way): who has looked in vain goes over all keys by itself, as where no rows are shared.
 constexpr int kHalfBytes = 4 * 17 * 1024;  // 4 waves of 32 floats, a maximum and a sum to a lane
+#ifdef LLMHIP_BENCH
+constexpr int kHalfLooks = 0;  // (the measurement library's copy: who began second goes over all keys by itself)
+#else
+constexpr int kHalfLooks = 1 << 17;
+#endif
 template <int D0, int ND, typename T, int KB>
 __device__ __forceinline__ void pass_half(const WaveAttn<T, KB> &w, __amdgpu_buffer_rsrc_t words, int wave, uint64_t number) {
   const uint32_t tag0 = (uint32_t)number, tag1 = (uint32_t)(number >> 32);
@@ -584,29 +590,29 @@ __device__ __forceinline__ void pass_half(const WaveAttn<T, KB> &w, __amdgpu_buf
   for (int i = 0; i < 8 * ND; ++i) word(i, w.o[D0 + i / 8][2 * (i % 8)], w.o[D0 + i / 8][2 * (i % 8) + 1]);
   word(8 * ND, w.m_run, w.l_run);
 }
+// Whether the other half was there, and is folded in
 template <int D0, int ND, typename T, int KB>
-__device__ __forceinline__ void fold_halves(WaveAttn<T, KB> &w, __amdgpu_buffer_rsrc_t words, int wave, uint64_t number, bool first, float scale_log2e) {
+__device__ __forceinline__ bool fold_halves(WaveAttn<T, KB> &w, __amdgpu_buffer_rsrc_t words, int wave, uint64_t number, bool first, float scale_log2e) {
   const uint32_t tag0 = (uint32_t)number, tag1 = (uint32_t)(number >> 32);
   const int at = wave * 17 * 1024 + w.lane * 16;
   u32x4_t v[8 * ND + 1];
-  bool there;
-  int looks = 1 << 17;  // (0.1 s: the other one is under way.  Rows of NaN where the buffer was another launch's too)
-  do {
-    do {
-      asm volatile("" ::: "memory");  // (the load is made again)
-      v[8 * ND] = __builtin_bit_cast(u32x4_t, load_device(words, at + 8 * ND * 1024));
-      there = __builtin_amdgcn_ballot_w64(((v[8 * ND][1] ^ tag0) | (v[8 * ND][3] ^ tag1)) != 0) == 0;
-      if (!there) __builtin_amdgcn_s_sleep(1);
-    } while (!there && --looks > 0);
+  bool there = false;
+  for (int looks = kHalfLooks; looks > 0 && !there; --looks) {
+    asm volatile("" ::: "memory");  // (the load is made again)
+    v[8 * ND] = __builtin_bit_cast(u32x4_t, load_device(words, at + 8 * ND * 1024));
+    if (__builtin_amdgcn_ballot_w64(((v[8 * ND][1] ^ tag0) | (v[8 * ND][3] ^ tag1)) != 0) != 0) {
+      __builtin_amdgcn_s_sleep(1);
+      continue;
+    }
     asm volatile("" ::: "memory");
     uint32_t differs = 0;
 #pragma unroll
     for (int i = 0; i < 8 * ND; ++i) v[i] = __builtin_bit_cast(u32x4_t, load_device(words, at + i * 1024));
 #pragma unroll
     for (int i = 0; i < 8 * ND; ++i) differs |= (v[i][1] ^ tag0) | (v[i][3] ^ tag1);
-    there = there && __builtin_amdgcn_ballot_w64(differs != 0) == 0;
-  } while (!there && --looks > 0);
-  if (!there) w.l_run = NAN;
+    there = __builtin_amdgcn_ballot_w64(differs != 0) == 0;
+  }
+  if (!there) return false;
   const float m = __builtin_bit_cast(float, (uint32_t)v[8 * ND][0]), l = __builtin_bit_cast(float, (uint32_t)v[8 * ND][2]);
   const float m_new = fmaxf(w.m_run, m), m_use = (m_new == -INFINITY) ? 0.0f : m_new;
   const float own = fast_exp2((w.m_run - m_use) * scale_log2e), other = fast_exp2((m - m_use) * scale_log2e);
@@ -621,6 +627,7 @@ __device__ __forceinline__ void fold_halves(WaveAttn<T, KB> &w, __amdgpu_buffer_
     for (int j = 0; j < 2; ++j)
       w.o[D0 + i / 8][2 * (i % 8) + j] = sum(w.o[D0 + i / 8][2 * (i % 8) + j], __builtin_bit_cast(float, (uint32_t)v[i][2 * j]));
   w.m_run = m_new;
+  return true;
 }
 
 // One global_load_lds_dwordx4: lane l's 16 bytes at `src` land at the wave-uniform LDS address lds_addr + 16*l.
@@ -716,9 +723,9 @@ template <PrefillKeys KEYS> struct LateOf { using type = PrefillBrief; };
 template <> struct LateOf<kRanges> { using type = PrefillLate; };
 template <> struct LateOf<kHalves> { using type = PrefillHalves; };
 
-template <typename T, int NW, int KP, bool NT, PrefillKeys KEYS>
-__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec,
-                                                                                  typename LateOf<KEYS>::type late) {
+// The rows of a workgroup.  AGAIN: after it has looked for the other half of their keys in vain, over all of them.  True if they are still to be made.
+template <typename T, int NW, int KP, bool NT, PrefillKeys KEYS, bool AGAIN = false>
+__device__ __forceinline__ bool prefill_rows(addresses_t ea, u32x4_t eb, u32x2_t ec, typename LateOf<KEYS>::type late) {
   constexpr bool SPLIT = KEYS == kRanges;
   const PrefillLate p = late;
   // SUB tiles of 64 keys per stage and per barrier: with one workgroup per CU (NW = 8) a stage
@@ -732,11 +739,11 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   constexpr int kWaveKeys = 32 * KB;  // keys of a tile per wave
   constexpr int kSplitKK = 3;  // k-steps of S(j+1) issued beside the row-maximum chain
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const PrefillShared e(ea, eb, ec, KEYS == kHalves);
+  const PrefillShared e(ea, eb, ec, AGAIN || KEYS == kHalves);
   const bool pack = SPLIT && e.pack;  // (packed rows exist in split mode only)
   const int rows = pack ? e.m * e.g : e.m;
   int tile, head, split;
-  if (!prefill_schedule<KEYS>(e, p, blockIdx.x, (rows + BM - 1) / BM, tile, head, split)) return;
+  if (!prefill_schedule<AGAIN ? kHalves : KEYS>(e, p, blockIdx.x, (rows + BM - 1) / BM, tile, head, split)) return false;
 #ifdef LLMHIP_BENCH
   unsigned long long clk0 = 0, ref0 = 0;
   if (p.clock_probe) {
@@ -796,9 +803,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     find_partial();
     w.init(lds, lane, kVRegion);
     store_partial(w, part_o, part_ml, row_valid);
-    return;
+    return false;
   }
-  // Which of a pair begins first passes its half on: it is under way, and so the other one never waits for a workgroup that is not.
+  // Which of a pair begins first passes its half on: it is under way, and so the other one does not wait for a workgroup that is not.
   [[maybe_unused]] unsigned long long began = 0;
   [[maybe_unused]] int pair = 0;
   if constexpr (KEYS == kHalves) {
@@ -815,7 +822,7 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
   // and V tiles, or, where every row has one wave, begins with the V slots that the first stage fills.
   constexpr int kQRegion = KP > 1 ? 2 * NSLOT * TB : kVRegion + SUB * TB;
 #pragma unroll
-  for (int sl = 0; sl < 8 / KP; ++sl) {
+  for (int sl = 0; sl < 8 / KP && !AGAIN; ++sl) {  // (they are still there)
     const int r = 4 * (sl * NW + wave) + (lane >> 4);
     const int idx = min(row0 + r, rows - 1);
     const char *src = e.q + ((lane & 15) ^ (r & 15)) * 16;
@@ -944,23 +951,29 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     constexpr int kTrade = WaveAttn<T, KB>::trade_bytes(KP), ND = 4 / KP;
     char *rows_lds = lds + rb * kTrade;
     w.template give<KP>(rows_lds, kpar);
-    volatile uint32_t *second = reinterpret_cast<volatile uint32_t *>(lds + 2 * NSLOT * TB);  // (Q's place)
+    constexpr int kNotes = 2 * NSLOT * TB - 32;
+    static_assert(KEYS != kHalves || RB * kTrade + NW * 32 * 64 * ND <= kNotes, "");
+    // (told to be in LDS: a read through a generic pointer would wait for the stores of the rows too)
+    auto *notes = (volatile __attribute__((address_space(3))) uint32_t *)(lds + kNotes);
     if constexpr (KEYS == kHalves) {
-      if (split && tid == 0) *second = began == late.number;
+      if (split && tid == 0) notes[0] = began == late.number;  // (the second to begin)
     }
     __syncthreads();
-    bool there = true;  // (all that the rows see)
+    [[maybe_unused]] bool in_vain = false;
     auto finish = [&](auto part) {
       constexpr int PART = decltype(part)::value;
       w.template take<KP, PART>(rows_lds, scale);
       if constexpr (KEYS == kHalves) {
         if (split) {
           const __amdgpu_buffer_rsrc_t words = byte_buffer(late.halves + (size_t)pair * kHalfBytes, kHalfBytes);
-          if (__builtin_amdgcn_readfirstlane(*second)) fold_halves<PART * ND, ND>(w, words, wave, late.number, split == 1, scale);
-          else pass_half<PART * ND, ND>(w, words, wave, late.number), there = false;
+          if (!__builtin_amdgcn_readfirstlane(notes[0])) {
+            pass_half<PART * ND, ND>(w, words, wave, late.number);
+            return;
+          }
+          in_vain = !fold_halves<PART * ND, ND>(w, words, wave, late.number, split == 1, scale);
+          if (in_vain) return;
         }
       }
-      if (!there) return;
       if (SPLIT && rows > kFewRows)
         store_partial_rows<PART * ND, ND>(w, lds + RB * kTrade + wave * (32 * 128 * ND), part_row, part_ml, row_valid, rows - qblk0);
       else if (SPLIT)
@@ -973,6 +986,13 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     if constexpr (KP == 4) {
       if (kpar == 2) finish(std::integral_constant<int, 2>());
       if (kpar == 3) finish(std::integral_constant<int, 3>());
+    }
+    if constexpr (KEYS == kHalves) {
+      if (split && __builtin_amdgcn_readfirstlane(notes[0])) {  // all waves or none
+        if (lane == 0) notes[1 + wave] = in_vain;
+        lds_barrier();
+        return __builtin_amdgcn_readfirstlane(notes[1] | notes[2] | notes[3] | notes[4]) != 0;
+      }
     }
   } else if (SPLIT) {
     if (rows > kFewRows)
@@ -988,6 +1008,19 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel
     p.clock_probe[1] = __builtin_amdgcn_s_memrealtime() - ref0;
   }
 #endif
+  return false;
+}
+
+template <typename T, int NW, int KP, bool NT, PrefillKeys KEYS>
+__global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void flash_prefill_kernel(addresses_t ea, u32x4_t eb, u32x2_t ec,
+                                                                                  typename LateOf<KEYS>::type late) {
+  const bool in_vain = prefill_rows<T, NW, KP, NT, KEYS>(ea, eb, ec, late);
+  if constexpr (KEYS == kHalves) {
+    if (!in_vain) return;
+    lds_barrier();  // (tiles come where the notes are)
+    asm volatile("" : "+s"(ea), "+s"(eb), "+s"(ec));  // (nothing is kept for this beside the first way)
+    prefill_rows<T, NW, KP, NT, kAllKeys, true>(ea, eb, ec, late);
+  }
 }
 
 // Folds the key-range partials of the output rows with the log-sum-exp rule.  256 threads handle 8
@@ -1310,7 +1343,7 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 }
 
 // Where two waves share 64 rows and not every CU has two workgroups, the launch waits for those with the most keys, while others have long
-// ended: the longest rows are dealt to two workgroups each (see fold_halves), as many as leave places for all workgroups at once, and as many
+// ended: the longest rows are dealt to two workgroups each (see pass_half), as many as leave places for all workgroups at once, and as many
 // as leave those that are not cut longer than a half and what it is passed on in, which takes as long as 6 steps.  Cut ones come behind those that
 // are longer than a half and 4 steps (by 2 to 6 the same; before all others 1.05 to 1.15 times as long: the longest rows then begin later and
 // beside longer ones).  Attention, us, whole / so: 1019 tokens of 28 + 4 heads (of 16 steps 14) 14.9 / 14.1, 930 13.2 / 12.75, 1088 15.9 / 15.4, 930 of 32
@@ -1466,9 +1499,7 @@ template <typename T> static hipError_t launch_prefill(const PrefillParams &p, P
 #ifdef LLMHIP_BENCH
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *clock_probe) {
-  void *const workspace = nullptr;
-  size_t workspace_bytes = 0;
+                                hipStream_t stream, void *workspace, size_t workspace_bytes, void *clock_probe) {
   PrefillParams p;
   p.clock_probe = static_cast<unsigned long long *>(clock_probe);
 #else

@@ -19,11 +19,12 @@ size_t flash_prefill_least_workspace_bytes(int m, int n, int offset, int group_s
 // shared; nor are they on a stream that may be capturing.
 size_t flash_prefill_halves_bytes(int m, int n, int offset, int group_size, int kv_head_num);
 #ifdef LLMHIP_BENCH
-// The measurement library's copy, never split: clock_probe is a device pointer to two 64-bit counters that
-// workgroup 0 fills with the shader-clock ticks and the reference-clock ticks of its lifetime.
+// The measurement library's copy: clock_probe is null or a device pointer to two 64-bit counters that
+// workgroup 0 fills with the shader-clock ticks and the reference-clock ticks of its lifetime; where rows are shared,
+// who began second of a pair does not wait for the other one's half.
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
-                                hipStream_t stream, void *clock_probe);
+                                hipStream_t stream, void *workspace, size_t workspace_bytes, void *clock_probe);
 #else
 hipError_t launch_flash_prefill(void *out, const void *q, const void *k, const void *v, int m,
                                 int n, int offset, int group_size, int kv_head_num, int dt,
