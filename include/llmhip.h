@@ -74,7 +74,7 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
  * ordinary prefill shapes, which need none (prompts of some 900 to 1500 tokens, by the number of
  * heads, use some MiB of the buffer where it can be had and the stream is not capturing: the longest
  * rows are then shared by two workgroups each).  The buffer is allocated on the first call that
- * needs it on a stream (a power of two, at least 4 MiB) and replaced by a larger one when a later
+ * needs it on a stream (of a device: the null stream has one on each; a power of two, at least 4 MiB) and replaced by a larger one when a later
  * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
  * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or
  * llmhip_release_internal_workspace.  HIP graphs: a call made while its stream is capturing cannot

@@ -5,11 +5,10 @@
 
 #include <hip/hip_runtime.h>
 
-#include <map>
 #include <mutex>
-#include <vector>
 
 #include "kernels.hpp"
+#include "stream_scratch.hpp"
 
 using namespace llmhip;
 
@@ -26,62 +25,60 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 template <typename... P> inline bool all_aligned16(P... ptrs) { return (aligned16(ptrs) && ...); }
 
 // Split-KV scratch for the entry points that mirror the reference signatures
-// and therefore have no workspace argument: one buffer per stream that only grows.
-// A buffer that has become too small is not freed when a larger one replaces it: launches already
-// queued, and HIP graphs captured earlier, keep their pointer valid.  Retired buffers go with
+// and therefore have no workspace argument: see stream_scratch.hpp.  It goes with
 // llmhip_stream_destroy / llmhip_release_internal_workspace.
-struct StreamScratch {
-  void *ptr = nullptr;
-  size_t bytes = 0;
-  std::vector<void *> retired;
+class OnDevice {  // makes a device the current one for a while
+ public:
+  explicit OnDevice(int device) {
+    if (hipGetDevice(&before_) == hipSuccess && before_ != device && hipSetDevice(device) == hipSuccess) moved_ = true;
+  }
+  ~OnDevice() {
+    if (moved_) (void)hipSetDevice(before_);
+  }
+
+ private:
+  int before_ = 0;
+  bool moved_ = false;
+};
+struct HipScratch {
+  // (of the null stream and its likes: the current device)
+  static int device_of(void *stream) {
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) (void)hipGetLastError();
+    const hipStream_t s = as_stream(stream);
+    hipDevice_t of_stream;
+    if (s == nullptr || s == hipStreamLegacy || s == hipStreamPerThread) return device;
+    if (hipStreamGetDevice(s, &of_stream) == hipSuccess) return of_stream;
+    (void)hipGetLastError();
+    return device;
+  }
+  // hipMalloc that another stream's capture does not forbid.
+  static int allocate(int device, void **ptr, size_t bytes) {
+    const OnDevice on(device);
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t e = hipMalloc(ptr, bytes);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) (void)hipGetLastError();  // handled here: not for the next launch to report
+    return (int)e;
+  }
+  static int release(void *ptr) { return (int)hipFree(ptr); }
+  static bool capturing(void *stream) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess) (void)hipGetLastError();
+    return cap != hipStreamCaptureStatusNone;
+  }
+  static void wait_stream(int device, void *stream) {
+    const OnDevice on(device);
+    (void)hipStreamSynchronize(as_stream(stream));
+  }
+  static int wait_device(int device) {
+    const OnDevice on(device);
+    return (int)hipDeviceSynchronize();
+  }
 };
 std::mutex g_scratch_mu;
-std::map<void *, StreamScratch> g_scratch;
-
-// hipMalloc that another stream's capture does not forbid.
-hipError_t scratch_malloc(void **ptr, size_t bytes) {
-  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-  const hipError_t e = hipMalloc(ptr, bytes);
-  if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-  if (e != hipSuccess) (void)hipGetLastError();  // handled here: not for the next launch to report
-  return e;
-}
-
-// The stream's scratch for a call whose fastest form takes `need` bytes and that is to run with no less than least().
-// Where the buffer cannot grow -- its stream is under capture, which must not allocate, or the device is full -- the
-// call gets what there is; only if that is less than least() is it refused (LLMHIP_ERR_WORKSPACE under capture:
-// warm the stream up with its largest shape first).  Sizes are powers of two from 4 MiB on (the exact size where the
-// device has no room for that), so that the replaced buffers together are smaller than the one in use.
-// Caller holds g_scratch_mu.
-template <typename Least> int scratch_for_locked(void *stream, size_t need, Least least, StreamScratch **out) {
-  StreamScratch &s = g_scratch[stream];
-  *out = &s;
-  if (s.bytes >= need) return LLMHIP_OK;
-  const size_t fewest = least();
-  int refused = LLMHIP_ERR_WORKSPACE;
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(as_stream(stream), &cap) != hipSuccess) (void)hipGetLastError();
-  if (cap == hipStreamCaptureStatusNone) {
-    size_t grown = (size_t)4 << 20;
-    while (grown < need) grown *= 2;
-    const size_t wanted[] = {grown, need, fewest};
-    for (size_t want : wanted) {
-      if (want <= s.bytes) continue;
-      void *fresh = nullptr;
-      const hipError_t e = scratch_malloc(&fresh, want);
-      if (e != hipSuccess) {
-        refused = (int)e;
-        continue;
-      }
-      if (s.ptr) s.retired.push_back(s.ptr);
-      s.ptr = fresh;
-      s.bytes = want;
-      return LLMHIP_OK;
-    }
-  }
-  return s.bytes >= fewest ? LLMHIP_OK : refused;
-}
+ScratchTable<HipScratch> g_scratch;
 
 int attn_common(void *out, const void *q, const void *k, const void *v, int m, int n,
                 int offset, int group_size, int kv_head_num, int head_dim, int dt,
@@ -103,7 +100,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
                                           kv_head_num, splits, dt, as_stream(stream)));
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     StreamScratch *ws = nullptr;
-    int rc = scratch_for_locked(
+    int rc = g_scratch.get(
         stream, need, [&] { return flash_decode_least_workspace_bytes(1, n_vis, kv_head_num); }, &ws);
     if (rc != LLMHIP_OK) return rc;
     if (ws->bytes < need) splits = flash_decode_splits_within(1, n_vis, kv_head_num, m * group_size, ws->bytes);
@@ -119,7 +116,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     const size_t need = flash_decode_workspace_bytes(tiles, m, group_size, kv_head_num, splits);
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     StreamScratch *ws = nullptr;
-    if (need) (void)scratch_for_locked(stream, need, [] { return (size_t)0; }, &ws);
+    if (need) (void)g_scratch.get(stream, need, [] { return (size_t)0; }, &ws);
     if (!need || ws->bytes >= need)
       return from_hip(launch_flash_decode_tiles(out, q, k, v, need ? ws->ptr : nullptr, need ? ws->bytes : 0, m, n_vis, offset,
                                                 group_size, kv_head_num, splits, dt, as_stream(stream)));
@@ -134,7 +131,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     if (halves && as_stream(stream) != hipStreamPerThread && !may_be_capturing(as_stream(stream))) {
       std::lock_guard<std::mutex> lk(g_scratch_mu);
       StreamScratch *ws = nullptr;
-      (void)scratch_for_locked(stream, halves, [] { return (size_t)0; }, &ws);
+      (void)g_scratch.get(stream, halves, [] { return (size_t)0; }, &ws);
       if (ws->bytes >= halves)
         return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt, as_stream(stream), ws->ptr, ws->bytes));
     }
@@ -143,7 +140,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
   }
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   StreamScratch *ws = nullptr;
-  int rc = scratch_for_locked(
+  int rc = g_scratch.get(
       stream, need, [&] { return flash_prefill_least_workspace_bytes(m, n, offset, group_size, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
   return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt,
@@ -278,7 +275,7 @@ int llmhip_decode_step_gqa(void *out, void *k_cache, void *v_cache, const void *
                                              as_stream(stream)));
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   StreamScratch *ws = nullptr;
-  int rc = scratch_for_locked(
+  int rc = g_scratch.get(
       stream, need, [&] { return flash_decode_least_workspace_bytes(1, n, kv_head_num); }, &ws);
   if (rc != LLMHIP_OK) return rc;
   if (ws->bytes < need) splits = flash_decode_splits_within(1, n, kv_head_num, group_size, ws->bytes);
@@ -383,15 +380,7 @@ int llmhip_stream_destroy(void *stream) {
   {
     // the split-KV scratch kept for this stream goes with it
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    auto it = g_scratch.find(stream);
-    if (it != g_scratch.end()) {
-      if (it->second.ptr) {
-        (void)hipStreamSynchronize(as_stream(stream));
-        (void)hipFree(it->second.ptr);
-      }
-      for (void *old : it->second.retired) (void)hipFree(old);
-      g_scratch.erase(it);
-    }
+    g_scratch.drop(stream);
   }
   return from_hip(hipStreamDestroy(as_stream(stream)));
 }
@@ -445,20 +434,7 @@ const char *llmhip_error_string(int status) {
 }
 int llmhip_release_internal_workspace(void) {
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  int rc = LLMHIP_OK;
-  if (!g_scratch.empty()) {
-    // queued launches may still use the buffers
-    hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess) rc = (int)e;
-  }
-  for (auto &kv : g_scratch) {
-    if (kv.second.ptr) {
-      hipError_t e = hipFree(kv.second.ptr);
-      if (e != hipSuccess) rc = (int)e;
-    }
-    for (void *old : kv.second.retired) (void)hipFree(old);
-  }
-  g_scratch.clear();
+  const int rc = g_scratch.release();
   release_matmul_resources();
   return rc;
 }
@@ -487,7 +463,7 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
       const size_t need = matmul_pieces_bytes(m, n, pieces);
       std::lock_guard<std::mutex> lk(g_scratch_mu);
       StreamScratch *ws = nullptr;
-      (void)scratch_for_locked(stream, need, [] { return (size_t)0; }, &ws);
+      (void)g_scratch.get(stream, need, [] { return (size_t)0; }, &ws);
       if (ws->bytes >= need) return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream), pieces, ws->ptr));
     }
     const bool tiles = m > 8 && matmul_tile_takes(m, n, k);

@@ -12,6 +12,7 @@
 
 #include "../../llm_simple_amd/csrc/device_hip.hpp"
 #include "../../llm_simple_amd/csrc/launch_number.hpp"
+#include "../../llm_simple_amd/csrc/stream_scratch.hpp"
 
 using namespace llm_simple_amd;
 
@@ -418,7 +419,77 @@ static void test_launch_numbers() {
   EXPECT(llmhip::next_launch_number(7 - step) == 7 + step);
 }
 
+// Two devices of the host's memory, of which the null stream and its likes mean the current one
+struct TwoDevices {
+  static int current, waits[2];
+  static size_t held[2], room;
+  static std::vector<std::pair<void *, std::pair<int, size_t>>> blocks;
+  static int device_of(void *stream) { return stream ? (int)((uintptr_t)stream & 1) : current; }
+  static int allocate(int device, void **ptr, size_t bytes) {
+    if (held[device] + bytes > room) return 2;
+    *ptr = std::malloc(1);
+    held[device] += bytes;
+    blocks.push_back({*ptr, {device, bytes}});
+    return 0;
+  }
+  static int release(void *ptr) {
+    for (size_t i = 0; i < blocks.size(); ++i)
+      if (blocks[i].first == ptr) {
+        held[blocks[i].second.first] -= blocks[i].second.second;
+        blocks.erase(blocks.begin() + (long)i);
+        std::free(ptr);
+        return 0;
+      }
+    return 1;
+  }
+  static bool capturing(void *stream) { return (uintptr_t)stream >= 0x1000; }
+  static void wait_stream(int device, void *) { ++waits[device]; }
+  static int wait_device(int device) { return ++waits[device], 0; }
+  static int device_holding(void *ptr) {
+    for (const auto &b : blocks)
+      if (b.first == ptr) return b.second.first;
+    return -1;
+  }
+};
+int TwoDevices::current = 0, TwoDevices::waits[2] = {};
+size_t TwoDevices::held[2] = {}, TwoDevices::room = (size_t)64 << 20;
+std::vector<std::pair<void *, std::pair<int, size_t>>> TwoDevices::blocks;
+
+// Scratch of a stream lies on the stream's device, that of the null stream on the current one's
+static void test_stream_scratch() {
+  using D = TwoDevices;
+  llmhip::ScratchTable<D> table;
+  llmhip::StreamScratch *s = nullptr;
+  auto none = [] { return (size_t)0; };
+  auto handle = [](uintptr_t h) { return reinterpret_cast<void *>(h); };
+  void *first[2];
+  for (int device = 0; device < 2; ++device) {
+    D::current = device;
+    EXPECT(table.get(nullptr, 1000, none, &s) == 0 && s->bytes == (size_t)4 << 20);
+    first[device] = s->ptr;
+    EXPECT(D::device_holding(s->ptr) == device);
+    EXPECT(table.get(handle(0x10 + (device ^ 1)), 1000, none, &s) == 0 && D::device_holding(s->ptr) == (device ^ 1));  // the other device's stream
+  }
+  EXPECT(first[0] != first[1] && D::held[0] == (size_t)8 << 20 && D::held[1] == D::held[0]);
+  D::current = 0;
+  EXPECT(table.get(nullptr, 500, none, &s) == 0 && s->ptr == first[0]);
+  // growth keeps the one before, on its device alone
+  EXPECT(table.get(nullptr, (size_t)5 << 20, none, &s) == 0 && s->bytes == (size_t)8 << 20 && s->retired.size() == 1 && s->retired[0] == first[0]);
+  D::current = 1;
+  EXPECT(table.get(nullptr, 500, none, &s) == 0 && s->ptr == first[1] && s->retired.empty());
+  // no room, and a stream under capture: what there is, or a refusal
+  EXPECT(table.get(nullptr, (size_t)100 << 20, none, &s) == 0 && s->ptr == first[1]);
+  EXPECT(table.get(nullptr, (size_t)100 << 20, [] { return (size_t)90 << 20; }, &s) == 2);
+  EXPECT(table.get(handle(0x1000), 16, none, &s) == 0 && s->bytes == 0);
+  EXPECT(table.get(handle(0x1000), 16, [] { return (size_t)16; }, &s) == LLMHIP_ERR_WORKSPACE);
+  // a destroyed stream's go, and nobody else's
+  table.drop(handle(0x11));
+  EXPECT(D::waits[0] == 0 && D::waits[1] == 1 && D::held[1] == (size_t)4 << 20 && D::held[0] == (size_t)16 << 20);
+  EXPECT(table.release() == 0 && D::waits[0] == 1 && D::waits[1] == 2 && D::held[0] + D::held[1] == 0 && D::blocks.empty());
+}
+
 int main() {
+  test_stream_scratch();
   test_launch_numbers();
   test_profiler_file();
   test_sizes();
