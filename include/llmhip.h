@@ -71,12 +71,15 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
  * partials of the split-KV decode kernel (m * group_size <= 16, and a few tokens more over a short
  * cache, which it takes in tiles of up to 16 rows) or of a key-range split of the prefill kernel (a
  * chunk behind at least as many cached tokens, wherever the split is faster; at most 256 MiB); 0 for
- * ordinary prefill shapes, which need none (prompts of some 900 to 1500 tokens, by the number of
- * heads, use some MiB of the buffer where it can be had and the stream is not capturing: the longest
- * rows are then shared by two workgroups each).  The buffer is allocated on the first call that
- * needs it on a stream (of a device: the null stream has one on each; a power of two, at least 4 MiB) and replaced by a larger one when a later
+ * ordinary prefill shapes, which need none.  (Prompts of some 600 to 1500 tokens, by the
+ * heads and the tokens cached before, use up to 16 MiB of another buffer of the stream where it can be
+ * had and the stream is not capturing: the longest rows are then shared by two workgroups each.  It is
+ * not counted here and needs no warming up: without it, as under capture, the rows stay whole, and the
+ * result may differ in the last bit.)  The buffer is allocated on the first call that needs it on a
+ * stream (of a device: the null stream has one on each; a power of two, at least 4 MiB) and replaced by a larger one when a later
  * call needs more; a replaced buffer is kept, not freed, so launches already queued and HIP graphs
- * captured earlier keep a valid pointer.  All of them go with llmhip_stream_destroy or
+ * captured earlier keep a valid pointer.  (A graph that uses the buffer is not to be replayed on another
+ * stream while calls that use it run on its own.)  All of them go with llmhip_stream_destroy or
  * llmhip_release_internal_workspace.  HIP graphs: a call made while its stream is capturing cannot
  * allocate; where the buffer would have to grow it runs with what there is, unsplit if need be, which can
  * be slower -- warm the stream up with its largest shape before capturing.  Where that would be
@@ -230,7 +233,7 @@ int llmhip_release_internal_workspace(void);
  * must be multiples of 16 (src/llama2_layer_npu.cpp:1211-1218).  Runs on kernels of this library up to 16 rows, and where its
  * tiles fit the chip in one round (16-byte aligned pointers; k a multiple of 64 beyond 16 rows); other calls run on
  * hipBLASLt, the first of which allocates its handle and a 64 MiB workspace.  Few tiles over a k of 3072 to 6143 sum pieces of k
- * in the stream's scratch, as far as it can be had outside of capture: a captured call may differ in the last bit. */
+ * in a buffer of the stream's, 4 MiB, as far as it can be had outside of capture: a captured call may differ in the last bit. */
 int llmhip_matmul(void *out, const void *lhs, const void *weight, int m, int n, int k, int dt,
                   void *stream);
 

@@ -78,7 +78,9 @@ struct HipScratch {
   }
 };
 std::mutex g_scratch_mu;
-ScratchTable<HipScratch> g_scratch;
+// Partials; and what workgroups of an eager launch pass each other, which captured launches do not.  A captured graph keeps its stream's partials
+// buffer and may be replayed on any other stream: calls that need no partials stay safe beside it.
+ScratchTable<HipScratch> g_scratch, g_exchange;
 
 int attn_common(void *out, const void *q, const void *k, const void *v, int m, int n,
                 int offset, int group_size, int kv_head_num, int head_dim, int dt,
@@ -131,7 +133,7 @@ int attn_common(void *out, const void *q, const void *k, const void *v, int m, i
     if (halves && as_stream(stream) != hipStreamPerThread && !may_be_capturing(as_stream(stream))) {
       std::lock_guard<std::mutex> lk(g_scratch_mu);
       StreamScratch *ws = nullptr;
-      (void)g_scratch.get(stream, halves, [] { return (size_t)0; }, &ws);
+      (void)g_exchange.get(stream, halves, [] { return (size_t)0; }, &ws);
       if (ws->bytes >= halves)
         return from_hip(launch_flash_prefill(out, q, k, v, m, n, offset, group_size, kv_head_num, dt, as_stream(stream), ws->ptr, ws->bytes));
     }
@@ -378,9 +380,10 @@ int llmhip_stream_create(void **stream) {
 }
 int llmhip_stream_destroy(void *stream) {
   {
-    // the split-KV scratch kept for this stream goes with it
+    // the scratch kept for this stream goes with it
     std::lock_guard<std::mutex> lk(g_scratch_mu);
     g_scratch.drop(stream);
+    g_exchange.drop(stream);
   }
   return from_hip(hipStreamDestroy(as_stream(stream)));
 }
@@ -434,7 +437,7 @@ const char *llmhip_error_string(int status) {
 }
 int llmhip_release_internal_workspace(void) {
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  const int rc = g_scratch.release();
+  const int kept = g_scratch.release(), passed = g_exchange.release(), rc = kept ? kept : passed;
   release_matmul_resources();
   return rc;
 }
@@ -463,7 +466,7 @@ static int matmul_common(void *out, const void *lhs, const void *weight, const v
       const size_t need = matmul_pieces_bytes(m, n, pieces);
       std::lock_guard<std::mutex> lk(g_scratch_mu);
       StreamScratch *ws = nullptr;
-      (void)g_scratch.get(stream, need, [] { return (size_t)0; }, &ws);
+      (void)g_exchange.get(stream, need, [] { return (size_t)0; }, &ws);
       if (ws->bytes >= need) return from_hip(launch_matmul_tile(out, lhs, weight, b, m, n, k, dt, as_stream(stream), pieces, ws->ptr));
     }
     const bool tiles = m > 8 && matmul_tile_takes(m, n, k);

@@ -1,6 +1,6 @@
 """Prompts whose longest rows two workgroups share: head counts that are dealt to XCDs and not, a ragged last tile, tokens cached before,
 keys past those that are seen, one and several cut tiles, and the sizes on either side.  Against the oracle on rows of every tile; every call gives
-the same bits, with decode calls between, and under capture, where no rows are shared, the same within the tolerance.  Workgroups that do not wait for
+the same bits, with projections between that use the same buffer, and under capture, where no rows are shared, the same within the tolerance.  Workgroups that do not wait for
 the other half give what the captured call gives."""
 import ctypes
 
@@ -28,7 +28,7 @@ def test_halves(dt, m, past, H, Hkv):
     q, k, v = normal_bits(m, (m, H, 128), dt), normal_bits(n + 1, (n + 64, Hkv, 128), dt), normal_bits(n + 2, (n + 64, Hkv, 128), dt)
     k[n:], v[n:] = 0x7FFF, 0x7FFF  # (not to be read)
     dq, dk, dv = to_dev(q), to_dev(k), to_dev(v)
-    one = dev_empty((1, H, 128))
+    x, weight, y = (dev_empty(s).fill_(0x3c00) for s in ((32, 5120), (1024, 5120), (32, 1024)))
 
     def call(out, stream=None):
         ops.hip_flash_attn_gqa_layer(out, dq, dk, dv, m, n, past, g, Hkv, 128, dt, *([] if stream is None else [stream]))
@@ -36,7 +36,7 @@ def test_halves(dt, m, past, H, Hkv):
     outs = [dev_empty(q.shape).fill_(0x7FFF) for _ in range(12)]
     for o in outs:
         call(o)
-        ops.hip_flash_attn_gqa_layer(one, dq, dk, dv, 1, n, n - 1, g, Hkv, 128, dt)
+        ops.hip_matmul_layer(y, x, weight, 32, 1024, 5120, dt)  # (pieces of k)
     got = to_host(outs[0])
     wide = orc.widen(got, dt)
     assert np.isfinite(wide).all()

@@ -1,7 +1,7 @@
 """Calls that take split-KV scratch when there is none to be had: on a stream under capture whose buffer would have to
 grow they run with what there is, except those that insist on theirs (a short chunk or a token over a long cache:
 LLMHIP_ERR_WORKSPACE); the batched decode does the same with a workspace smaller than its default count takes; and a
-buffer grows on one stream while another is being captured."""
+buffer grows on one stream while another is being captured; and a graph is replayed on another stream than its own."""
 import contextlib
 import ctypes
 
@@ -144,6 +144,39 @@ def test_buffer_grows_while_another_stream_is_captured():
         s.synchronize()
         check_attention(to_host(out), *bits, n, past, DT)
         replays_match(graph, small, (bits[0][:1],) + bits[1:], 64, 63)
+
+
+def test_replay_elsewhere_beside_calls_that_need_no_partials():
+    """A graph keeps its stream's partials and is replayed on another stream, while prompts and projections run on its own: what workgroups of
+    those pass each other lies elsewhere."""
+    import torch
+    import llm_simple_amd.ops as ops
+    (n, H, Hkv), m, (rows, width, k_dim) = (32768, 40, 8), 1019, (32, 1024, 5120)
+    bits, (q, k, v) = inputs(1, n, H, Hkv)
+    _, (pq, pk, pv) = inputs(m, m, 28, 4)
+    x, w = to_dev(normal_bits(4, (rows, k_dim), DT)), to_dev(normal_bits(5, (width, k_dim), DT))
+    out, prompts, sums = dev_empty(q.shape), [dev_empty(pq.shape) for _ in range(30)], [dev_empty((rows, width)) for _ in range(30)]
+    with fresh_stream() as s, fresh_stream() as other:
+        one = lambda: ops.hip_flash_attn_gqa_layer(out, q, k, v, 1, n, n - 1, H // Hkv, Hkv, 128, DT, s.cuda_stream)
+        one()  # (the buffer)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            one()
+        replays_match(graph, out, bits, n, n - 1)
+        want = to_host(out).copy()
+        for i, (p, y) in enumerate(zip(prompts, sums)):  # (the first ones by themselves)
+            if i:
+                with torch.cuda.stream(other):
+                    graph.replay()
+            ops.hip_flash_attn_gqa_layer(p, pq, pk, pv, m, m, 0, 7, 4, 128, DT, s.cuda_stream)
+            ops.hip_matmul_layer(y, x, w, rows, width, k_dim, DT, s.cuda_stream)
+            if not i:
+                torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        assert np.array_equal(to_host(out), want)
+        for o in prompts[1:] + sums[1:]:
+            assert torch.equal(o, prompts[0] if o.dim() == 3 else sums[0])
 
 
 def test_batched_decode_with_less_workspace_than_the_default_count_takes():
