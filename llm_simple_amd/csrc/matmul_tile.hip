@@ -65,7 +65,7 @@ constexpr int kBandRows = 4;           // m tiles of a band
 constexpr int kMostPieces = 8;         // of k
 constexpr int kWordsBytes = 2 * 16 * kTileThreads;  // of a piece's sums
 #ifdef LLMHIP_BENCH
-constexpr uint32_t kLooks = 0;  // (the measurement library's copy: a workgroup that adds up makes all sums by itself)
+constexpr uint32_t kLooks = 0;  // (the measurement library's copy: a workgroup that adds up takes no words for new, and makes all sums by itself)
 #else
 constexpr uint32_t kLooks = 2000;      // 0.7 us each or more: what a launch takes, many times over
 #endif
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void matmul_tile_kernel(addresses_
           for (int o = 0; o < kMostPieces - 1; ++o)
 #pragma unroll
             for (int h = 0; h < 2; ++h) differs |= o < pieces - 1 ? (v[o][h][1] ^ tag0) | (v[o][h][3] ^ tag1) : 0u;
-          there = __builtin_amdgcn_ballot_w64(differs != 0) == 0;
+          there = kLooks != 0 && __builtin_amdgcn_ballot_w64(differs != 0) == 0;
         } while (!there && --looks > 0);
 #pragma unroll
         for (int o = 0; o < kMostPieces - 1; ++o)

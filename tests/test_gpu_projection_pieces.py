@@ -53,6 +53,11 @@ def test_pieces(m, n, k, dt):
     if (m, n, k) in CUT:
         call()
         assert torch.equal(alone, out)
+        # who makes all sums itself keeps those so far in the last piece's place among the words (per tile of 32 x 32 and piece 8192 bytes, 4096 of sums)
+        tiles = -(-m // 32) * -(-n // 32)
+        pieces = min(256 // tiles, k // 64 // 12, 8)
+        kept = ws[:tiles * pieces * 8192].view(torch.int32).view(tiles, pieces, 2048)[:, -1, :1024]
+        assert (kept != 0).any(1).all()
     else:
         with pytest.raises(ops.LlmHipError):
             call()
