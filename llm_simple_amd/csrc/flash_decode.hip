@@ -945,7 +945,9 @@ static double split_model_us(long long pairs, int nblocks, int s, int cus, int r
 // 480 pairs 11.85 / 9.0; but 16 x 1500 of 32 kv heads, two even rounds, 58.2 / 61.6, 16 x 32768 of 8 295 / 325).  A workgroup's number within its XCD's
 // share repeats with the split, so that the XCD of the longer ones counts.  Fitted over 1261 shapes of 1-16 sequences, 2-32 kv heads, 64-32768 keys, up to 1.1 GB
 // and 17 counts each.  Two are taken where the model has them 4 % ahead, 160 of the shapes: 0.865 of the time there on average, none of all slower
-// by 2 %.
+// by 2 %.  Not for one sequence: the fused step's kernels take more than half of a CU's registers, and its unfused equal, which gives the same bits, has the same
+// count (fused / unfused, us, count for one / for two: 2000 keys of 100 kv heads 21.1 / 22.1, 20.25 / 20.35, 3072 of 66 21.05 / 22.15, 20.2 / 19.3; but 2000
+// of 88 22.8 / 20.75, 21.6 / 18.65; below 65 kv heads the counts are the same).
 static double two_model_us(long long pairs, int nblocks, int s, int cus) {
   const long long wgs = pairs * s;
   if (wgs <= cus || (s > 1 && nblocks < 2 * s)) return 1e30;  // (one block each: the fold is the larger part)
@@ -972,7 +974,7 @@ static int best_splits(long long pairs, int smax, int cus, double tolerance, lon
   }
   return first;
 }
-static int default_splits_model(long long pairs, int nblocks, int cus, int most, int rows, bool may_two = true) {
+static int default_splits_model(long long pairs, int nblocks, int cus, int most, int rows, bool may_two) {
   int smax = flash_decode_max_default_splits(pairs);
   if (smax > nblocks) smax = nblocks;
   if (smax > most) smax = most;
@@ -988,8 +990,8 @@ static int default_splits_model(long long pairs, int nblocks, int cus, int most,
   }
   return best;
 }
-static bool two_to_a_cu(long long pairs, int nblocks, int s, int cus, int rows) {
-  return two_model_us(pairs, nblocks, s, cus) < kTwoMargin * split_model_us(pairs, nblocks, s, cus, rows);
+static bool two_to_a_cu(int batch, long long pairs, int nblocks, int s, int cus, int rows) {
+  return batch > 1 && two_model_us(pairs, nblocks, s, cus) < kTwoMargin * split_model_us(pairs, nblocks, s, cus, rows);
 }
 
 // The model is evaluated a few hundred times per call; a decode loop asks for the same (pairs, key
@@ -1004,14 +1006,15 @@ int flash_decode_default_splits(int batch, int n, int kv_head_num, int rows) {
     long long pairs;
     int nblocks, cus, splits;
     int rows;
+    bool one;  // sequence
   };
   constexpr int kMemo = 8;
   static thread_local Memo memo[kMemo] = {};
   static thread_local unsigned next = 0;
   for (const Memo &e : memo)
-    if (e.splits > 0 && e.pairs == pairs && e.nblocks == nblocks && e.cus == cus && e.rows == rows) return e.splits;
-  const int s = default_splits_model(pairs, nblocks, cus, kMaxSplits, rows);
-  memo[next++ % kMemo] = Memo{pairs, nblocks, cus, s, rows};
+    if (e.splits > 0 && e.pairs == pairs && e.nblocks == nblocks && e.cus == cus && e.rows == rows && e.one == (batch == 1)) return e.splits;
+  const int s = default_splits_model(pairs, nblocks, cus, kMaxSplits, rows, batch > 1);
+  memo[next++ % kMemo] = Memo{pairs, nblocks, cus, s, rows, batch == 1};
   return s;
 }
 
@@ -1021,7 +1024,7 @@ int flash_decode_splits_within(int batch, int n, int kv_head_num, int rows, size
   int fits = s - 1;
   while (fits > 1 && flash_decode_workspace_bytes(batch, 1, 1, kv_head_num, fits) > bytes) --fits;
   return default_splits_model((long long)batch * kv_head_num, (n + kDecStepKeys - 1) / kDecStepKeys,
-                              device_compute_units(), fits, rows);
+                              device_compute_units(), fits, rows, batch > 1);
 }
 
 // What a call may insist on is counted with coarser figures than the default: 27.7 GB/s per CU in a full round and at most
@@ -1189,7 +1192,7 @@ static hipError_t launch_decode_impl(DecodeParams &p, void *workspace, size_t wo
   const size_t slots = (size_t)p.batch * p.Hkv * p.num_splits * p.cols;
   p.ws_o = static_cast<float *>(workspace);
   p.ws_ml = p.ws_o ? p.ws_o + slots * kHeadDim : nullptr;
-  p.two = !half && two_to_a_cu(pairs, nblocks, p.num_splits, cus, p.rows);
+  p.two = !half && two_to_a_cu(p.batch, pairs, nblocks, p.num_splits, cus, p.rows);
   const bool many = p.iters_each >= 8;  // long enough to be bound by the stream, see the kernel
   if (dt == kDtFloat16)
     return fused ? launch_decode<_Float16, true>(p, how, half, many, stream) : launch_decode<_Float16, false>(p, how, half, many, stream);

@@ -1,4 +1,4 @@
-"""How much per-stream scratch a chunk may ask for (no GPU: the sizes for 256 compute units)."""
+"""How much per-stream scratch a chunk may ask for, and the default counts of decode (no GPU: those for 256 compute units)."""
 import pytest
 
 
@@ -21,3 +21,12 @@ def test_cut_of_a_chunk(m, past, H, Hkv, ranges):
     import llm_simple_amd.ops as ops
     need = ops.lib.llmhip_flash_attn_scratch_bytes(m, m + past, past, H // Hkv, Hkv)
     assert need == (0 if ranges == 1 else ranges * m * H * 130 * 4)
+
+
+# (us of the fused step, which runs one workgroup to a CU, with the count for one / for two: 3072 keys of 66 kv heads 21.05 / 22.15, 2000 of 100 21.1 / 22.1)
+@pytest.mark.parametrize("batch,n,Hkv,count", [(1, 3072, 66, 3), (1, 2000, 100, 2), (1, 2000, 88, 8), (2, 2000, 50, 5), (2, 3072, 33, 7)])
+def test_counts_for_two_workgroups_to_a_cu_are_for_batches(batch, n, Hkv, count):
+    import llm_simple_amd.ops as ops
+    for other in (1, 2, batch):  # (as many pairs as before in one sequence or several)
+        assert ops.flash_decode_default_splits(other, n, Hkv * batch // other) > 0
+    assert ops.flash_decode_default_splits(batch, n, Hkv) == count
