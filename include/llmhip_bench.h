@@ -51,6 +51,9 @@ int llmhip_bench_decode_step_gqa_alone(void *out, void *k_cache, void *v_cache, 
 int llmhip_bench_matmul_alone(void *out, const void *lhs, const void *weight, const void *bias_f32, void *workspace, size_t workspace_bytes,
                               int m, int n, int k, int dt, void *stream);
 
+/* The tile by which llmhip_matmul(_bias) of 17 rows or more goes where k is not cut, lhs rows << 16 | features; 0: not by tiles. */
+int llmhip_bench_matmul_tile(int m, int n, int k);
+
 /* Runs, for about target_ms (<= 2000), a loop of back-to-back bf16 32x32x16 MFMAs on N(0,1)
  * operands on every CU and returns the sustained TFLOP/s.  mix 0: the MFMAs alone (what the matrix
  * pipe sustains at the clock its own power draw allows); mix 1: the same MFMAs with the LDS

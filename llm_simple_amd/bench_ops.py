@@ -16,6 +16,7 @@ SYMBOLS = {
     "llmhip_bench_flash_decode_gqa_alone": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, ctypes.c_int64, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_decode_step_gqa_alone": (_i, [_vp] * 8 + [_sz, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "llmhip_bench_matmul_alone": (_i, [_vp] * 5 + [_sz, _i, _i, _i, _i, _vp]),
+    "llmhip_bench_matmul_tile": (_i, [_i, _i, _i]),
     "llmhip_bench_mfma_ceiling": (_i, [_i, ctypes.c_double, ctypes.POINTER(ctypes.c_double)]),
     "llmhip_bench_stream_read": (_i, [_vp, _vp, _sz, _vp, _sz, _i, _vp]),
 }

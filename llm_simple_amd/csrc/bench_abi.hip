@@ -103,6 +103,8 @@ int llmhip_bench_matmul_alone(void *out, const void *lhs, const void *weight, co
                                      pieces, workspace));
 }
 
+int llmhip_bench_matmul_tile(int m, int n, int k) { return m < 1 || n < 1 || k < 1 ? LLMHIP_ERR_INVALID_ARG : matmul_tile_size(m, n, k); }
+
 int llmhip_bench_mfma_ceiling(int mix, double target_ms, double *tflops) {
   if (!tflops || (mix != 0 && mix != 1) || target_ms < 0.0 || target_ms > 2000.0) return LLMHIP_ERR_INVALID_ARG;
   if (device_count() < 1) return LLMHIP_ERR_NO_DEVICE;

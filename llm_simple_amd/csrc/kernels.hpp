@@ -103,6 +103,7 @@ hipError_t launch_rope_kv_append(void *out_q, void *out_k, void *out_v, const vo
 hipError_t launch_matmul_skinny(void *out, const void *lhs, const void *weight, const float *bias,
                                 int m, int n, int k, int dt, hipStream_t stream);
 bool matmul_tile_takes(int m, int n, int k);
+int matmul_tile_size(int m, int n, int k);  // lhs rows << 16 | features; 0: not taken
 int matmul_tile_pieces(int m, int n, int k);
 size_t matmul_pieces_bytes(int m, int n, int pieces);
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias,

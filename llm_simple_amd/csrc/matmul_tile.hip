@@ -503,6 +503,9 @@ int matmul_tile_pieces(int m, int n, int k) {
   if (pieces == 2 && m < 24) return 1;
   return (int)(pieces < kMostPieces ? pieces : kMostPieces);
 }
+int matmul_tile_size(int m, int n, int k) {
+  return matmul_tile_takes(m, n, k) ? kTiles[tile_kind(m, n, k)].m << 16 | kTiles[tile_kind(m, n, k)].n : 0;
+}
 size_t matmul_pieces_bytes(int m, int n, int pieces) { return (size_t)((m + 31) / 32) * ((n + 31) / 32) * pieces * kWordsBytes; }
 
 hipError_t launch_matmul_tile(void *out, const void *lhs, const void *weight, const float *bias, int m, int n, int k,
