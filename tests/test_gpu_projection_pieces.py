@@ -42,9 +42,9 @@ def test_pieces(m, n, k, dt):
     ops.hip_matmul_bias_layer(out, x, w, b, m, n, k, dt)
     got = to_host(out).copy()
     assert near(got, ref, dt)
-    q, kv, o = (to_dev(normal_bits(s, (1019, h, 128), dt)) for s, h in ((1, 28), (2, 4), (3, 28)))
+    q, kv, o = (to_dev(normal_bits(s, (r, h, 128), dt)) for s, r, h in ((1, 1, 40), (2, 3000, 8), (3, 1, 40)))
     for _ in range(5):
-        ops.hip_flash_attn_gqa_layer(o, q, kv, kv, 1019, 1019, 0, 7, 4, 128, dt)  # halves in the same buffer
+        ops.hip_flash_attn_gqa_layer(o, q, kv, kv, 1, 3000, 2999, 5, 8, 128, dt)  # partials in the same buffer
         again = nan(m, n, dt)
         ops.hip_matmul_bias_layer(again, x, w, b, m, n, k, dt)
         assert torch.equal(again, out)
@@ -53,11 +53,6 @@ def test_pieces(m, n, k, dt):
     if (m, n, k) in CUT:
         call()
         assert torch.equal(alone, out)
-        # who makes all sums itself keeps those so far in the last piece's place among the words (per tile of 32 x 32 and piece 8192 bytes, 4096 of sums)
-        tiles = -(-m // 32) * -(-n // 32)
-        pieces = min(256 // tiles, k // 64 // 12, 8)
-        kept = ws[:tiles * pieces * 8192].view(torch.int32).view(tiles, pieces, 2048)[:, -1, :1024]
-        assert (kept != 0).any(1).all()
     else:
         with pytest.raises(ops.LlmHipError):
             call()
