@@ -71,7 +71,7 @@ int llmhip_flash_attn_opt_prefill(void *out, const void *q, const void *k, const
  * partials of the split-KV decode kernel (m * group_size <= 16, and a few tokens more over a short
  * cache, which it takes in tiles of up to 16 rows) or of a key-range split of the prefill kernel (a
  * chunk behind at least as many cached tokens, wherever the split is faster; at most 256 MiB); 0 for
- * ordinary prefill shapes, which need none.  (Prompts of some 600 to 1500 tokens, by the
+ * ordinary prefill shapes, which need none.  (Prompts of some 400 to 1500 tokens, by the
  * heads and the tokens cached before, use up to 16 MiB of another buffer of the stream where it can be
  * had and the stream is not capturing: the longest rows are then shared by two workgroups each.  It is
  * not counted here and needs no warming up: without it, as under capture, the rows stay whole, and the

@@ -1346,8 +1346,9 @@ static PrefillKind prompt_kind(int m, long long n_vis, int H, int cus) {
 // ended: the longest rows are dealt to two workgroups each (see pass_half), as many as leave places for all workgroups at once, and as many
 // as leave those that are not cut longer than a half and what it is passed on in, which takes as long as 6 steps.  Cut ones come behind those that
 // are longer than a half and 4 steps (by 2 to 6 the same; before all others 1.05 to 1.15 times as long: the longest rows then begin later and
-// beside longer ones).  Attention, us, whole / so: 1019 tokens of 28 + 4 heads (of 16 steps 14) 14.9 / 14.1, 930 13.2 / 12.75, 1088 15.9 / 15.4, 930 of 32
-// + 32 15.2 / 13.8, 1480 of 12 + 2 17.2 / 15.0; with 3 steps for passing a half on 700 of 28 + 4 10.35 / 11.1.
+// beside longer ones).  Attention, us, whole / so: 1019 tokens of 28 + 4 heads (of 16 steps 14) 14.15 / 13.8, 930 13.35 / 13.05, 1088 15.1 / 15.05, 930 of 32
+// + 32 13.75 / 13.6, 1480 of 12 + 2 17.1 / 15.35 (another box 14.9 / 14.1, 13.2 / 12.75, 15.9 / 15.4, 15.2 / 13.8, 17.2 / 15.0, before those who look in vain made
+// their rows themselves, which costs up to 0.1); with 3 steps for passing a half on 700 of 28 + 4 10.35 / 11.1.
 static void prompt_cut(int m, long long n_vis, int g, int Hkv, int cus, int &cut, int &cut_at) {
   constexpr int kPassSteps = 6, kOrderSteps = 4;
   const int share = prefill_xcd_share_log2(Hkv), H = g * Hkv;

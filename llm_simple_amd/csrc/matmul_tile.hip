@@ -20,8 +20,8 @@
 // lines instead of two: 512 x 3584, 400 rows 8.5 -> 7.8 us; 1536 x 1536, 100 rows 5.4 -> 4.9).  There the barrier comes so late that
 // the loads go out in a burst behind it: 32 x 32 all eight in the last of 8 slots, 64 x 32 (two lines) six in the last two of 8.
 // Where the time of a launch goes, by clock stamps in a copy of the kernel, us: 128 x 224 tile, k = 3584: 2.6 until the first
-// lines are in, 56 stages of 0.67, 2.3 for the store (14.7 MB at once), the rest launch.  A stage takes 1120 cycles at
-// 1.68 GHz: the clock is what the power leaves (half of the chip: 1090 cycles at 2.2 GHz; without the line loads 1.9 GHz).
+// lines are in, 56 stages of 0.67, 2.3 for the store (of pieces of 64 bytes into the L2s, before rows past them), the rest launch.
+// A stage takes 1120 cycles at 1.68 GHz: the clock is what the power leaves (half of the chip: 1090 cycles at 2.2 GHz; without the line loads 1.9 GHz).
 //
 // A lane's accumulators are four features of one lhs row; W rows are dealt to LDS so that two neighbouring blocks make
 // them eight, and a store 16 bytes.  The bias goes to LDS ahead of the first lines: read from memory at the end it
@@ -35,10 +35,11 @@
 // W to a tile of 64 rows, and as long with 112 workgroups as with 224).  So lines go in groups, and each of up to 4 such tiles
 // begins at another place of a group: the first to ask for a line is a different one each time, and the rest find it in the L2 a moment later
 // (us, one order / so, W from HBM: 3584 x 3584, 64 rows 10.4 / 9.0, 256 18.2 / 13.9, 512 24.1 / 20.2, 1024 30.2 / 27.2, 2048 44.0 / 43.0;
-// 4096 x 4096, 256 rows 20.2 / 15.3; 5120 x 5120, 768 rows 47.9 / 43.7).  With W in the last-level cache it costs 1-3 % (3584 x 3584, 256
-// rows 11.5 / 12.2, 1024 24.5 / 25.0), and more the larger group and tile are, the lines of a group being in the L2 longer: hence groups of 8, 4 and 2
-// (2048 rows by groups of 8 43.8).  Where lhs is the larger operand there is nothing to gain (512 x 3584, 2048 rows 11.6 / 12.6 by groups of 8).  Half
-// or a quarter of k apart instead, the small ones are as fast, but what the L2 has to keep outgrows it (1024 rows 36.0).
+// 4096 x 4096, 256 rows 20.2 / 15.3; 5120 x 5120, 768 rows 47.9 / 43.7; what leaves the L2s downwards stays within
+// 5 %: 256 rows 39.9 / 41.8 MiB, 2048 131.4 / 129.4).
+// With W in the last-level cache it costs 2 to 6 % (3584 x 3584, 256 rows 11.5 / 12.2, 1024 24.5 / 25.0), and more the larger group and tile are, the lines of
+// a group being in the L2 longer: hence groups of 8, 4 and 2 (2048 rows by groups of 8 43.8).  Where lhs is the larger operand there is nothing to gain (512 x 3584,
+// 2048 rows 11.6 / 12.6 by groups of 8).  Half or a quarter of k apart instead, the small ones are as fast, but what the L2 has to keep outgrows it (1024 rows 36.0).
 //   Stages under way: as few as hold 64 to 100 KiB, but for 96 x 64.  More of them are no faster anywhere, and begin with a longer burst (5 / 9 stages of a
 // 64 x 64 tile, us: 512 x 3584, 2048 rows 12.6 / 13.1, 3584 x 3584, 256 rows 14.15 / 14.55; 3 / 4 of 32 x 32, 512 x 3584, 512 rows 7.1 / 7.35;
 // 3 / 5 of 96 x 128, 3584 x 3584, 768 rows 24.0 / 24.9; one line to a stage less and four stages of 64 x 32: 256 x 1536, 2048 rows 5.65 / 5.45).
@@ -494,8 +495,8 @@ bool matmul_tile_takes(int m, int n, int k) {
 // fewer than 24 rows, where a part whose way past the L2s is 1 us longer gains nothing from HBM and loses from the cache, 3584 x 3584,
 // 17 rows 9.25 / 9.25, 6.65 / 8.5 (32 there 10.8 / 9.7, 7.0 / 8.5; blocks of 30 and 32 rows gain 6 and 18 %), and k below
 // 3072, 512 x 2048 4.4 / 4.6, 1536 x 1536 5.2 / 5.15, 3.75 / 4.7).  One line to a stage less and five stages: 3 to 10 % ahead of two or three of four
-// lines.  Tiles that are larger have too much to pass on (64 x 128 over half of 3584: 18.5 us, of them 3.5).  Not from k = 6144 on, where a call
-// gives the same bits under capture.
+// lines.  Tiles that are larger have too much to pass on (64 x 128 over half of 3584: 18.5 us, of them 3.5).  The line at k = 6144 is not a
+// measured one (whole, 1024 x 8192, 17 rows 15.4 us, hipBLASLt 11.8): from there on a call gives the same bits eager and captured, which below it does not.
 int matmul_tile_pieces(int m, int n, int k) {
   const long long cus = device_compute_units(), tiles = (long long)((m + 31) / 32) * ((n + 31) / 32);
   if (m <= 8 || k % kLineK != 0 || k < 3072 || k >= 6144 || 2 * tiles > cus || tiles * cus >= 65536) return 1;
